@@ -76,6 +76,7 @@ struct mis_tts {
     // batched prefill (lm_prefill.hip): one chunk of positions x rows
     DevBuf<bf16_t> pf_h, pf_x, pf_attn, pf_act, pf_xpk, pf_actpk;
     DevBuf<float> pf_qkv, pf_tmp;
+    DevBuf<bf16_t> pf_qkv16, pf_q;               // the chunk's q|k|v and its roped queries
     DevBuf<int32_t> pf_pos;
     DevBuf<uint8_t> pf_on;
     DevBuf<SamplerScratch> samp_scratch;
@@ -852,20 +853,12 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     hipStream_t s = c->stream;
     const int d = c->d, HD = c->H * c->D, Mpad = c->Mpad, batch = c->batch;
     const float eps = c->cfg.rms_norm_eps;
-    // Causal attention of a chunk, two arrangements: one launch per position (rows = sequences) - fills the chip on its own once
-    // batch x kv heads reaches about half the CUs - or every (position, sequence) pair as a row of ONE launch: an append-only launch
-    // puts the roped keys and the values of all the chunk's positions into the caches, then the attention launch reads them like any
-    // earlier key (its own key is patched in registers as in the decode step).  Measured: batch 32 x 8 heads, 32 positions: 14.3 ms
-    // per position against 15.8 ms as pairs; batch 1, 350 positions: 90 -> 32 ms the other way.  MIS_PF_ATTN_LOOP=1 / 0 forces one.
-    const char* loop_env = getenv("MIS_PF_ATTN_LOOP");
-    const bool attn_loop = loop_env ? atoi(loop_env) != 0 : batch * c->Hkv >= 128;
-    // rows of the chunk: position-major, `rs` rows per position.  The pair arrangement needs no padding between positions (a batch of 1
-    // would otherwise carry 15 padding rows per position through every GEMM); the per-position one keeps Mpad (its flag words are aligned)
-    const int rs = attn_loop ? Mpad : batch;
+    // rows of the chunk: position-major, one row per sequence (no padding between positions)
+    const int rs = batch;
     const int Tc = std::min(Lmax, std::max(1, 4096 / rs));                   // positions per chunk: <= 4096 rows of activations
     const size_t Mc = round_up((size_t)Tc * rs, 16) + Mpad;                  // GEMM rows round up to 16; the last position is read Mpad rows wide
     c->pf_h.alloc(Mc * d); c->pf_x.alloc(Mc * d); c->pf_attn.alloc(Mc * HD);
-    c->pf_qkv.alloc(Mc * c->Nqkv); c->pf_pos.alloc(Mc); c->pf_on.alloc(Mc);
+    c->pf_q.alloc(Mc * HD); c->pf_pos.alloc(Mc); c->pf_on.alloc(Mc);
     HIP_CHECK(hipMemsetAsync(c->pf_attn.p, 0, Mc * HD * 2, s));             // rows of padded positions are never written by the attention
     HIP_CHECK(hipMemsetAsync(c->pf_x.p, 0, Mc * d * 2, s));                 // rows past the chunk (rounding, slack) hold zeros, not stale bits
     HIP_CHECK(hipMemsetAsync(c->pf_h.p, 0, Mc * d * 2, s));
@@ -873,6 +866,7 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     // slices - rows packed into MFMA fragments first, float32 sums out, the residual add as its own small kernel; gate|up writes the
     // packed activation its down projection reads.  The weights are streamed once per 64 rows instead of once per position.
     const bool coded = c->q_qkv.on;
+    if (coded) c->pf_qkv.alloc(Mc * c->Nqkv); else c->pf_qkv16.alloc(Mc * c->Nqkv);
     if (coded) { c->pf_xpk.alloc((size_t)64 * std::max(d, HD)); c->pf_actpk.alloc((size_t)64 * c->ff); c->pf_tmp.alloc((size_t)64 * d); }
     else c->pf_act.alloc(Mc * c->ff);
     auto q_rows = [&](int M, const std::function<void(int r0, int mp)>& body) {
@@ -900,34 +894,25 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
                 launch_pf_pack_rows(c->pf_x.p + (size_t)r0 * d, c->pf_xpk.p, mp, d, s);
                 q_partial(c->q_qkv, li, c->pf_xpk.p, c->pf_qkv.p + (size_t)r0 * c->Nqkv, c->Nqkv, d, mp);
             });
-            else launch_gemm_pf(PF_F32, c->pf_x.p, c->wqkv.p + layer_qkv_elems(c) * li, c->pf_qkv.p, M, c->Nqkv, d, s);
-            auto attn_params = [&](int tl0) {
-                AttnParams ap{};
-                ap.qkv_part = c->pf_qkv.p + (size_t)tl0 * rs * c->Nqkv; ap.S = 1; ap.Mpad = Mpad; ap.Nqkv = c->Nqkv;
-                ap.kcache = c->kcache.p + lkv * li; ap.vtcache = c->vtcache.p + lkv * li;
-                ap.pos = c->pf_pos.p + (size_t)tl0 * rs; ap.active = c->pf_on.p + (size_t)tl0 * rs;
-                ap.rope_cos = c->rope_cos.p; ap.rope_sin = c->rope_sin.p;
-                ap.out = c->pf_attn.p + (size_t)tl0 * rs * HD; ap.out_ld = HD;
-                ap.H = c->H; ap.Hkv = c->Hkv; ap.D = c->D; ap.Smax = c->Smax; ap.scale = 1.0f / sqrtf((float)c->D);
-                if (c->cfg.qk_norm) {
-                    ap.qnorm_w = c->qknorm.p + (size_t)(2 * li) * c->D;
-                    ap.knorm_w = c->qknorm.p + (size_t)(2 * li + 1) * c->D;
-                    ap.qk_eps = c->cfg.rms_norm_eps;
-                }
-                ap.rope_in_dtype = c->cfg.rope_ops_in_dtype;
-                ap.first_schedule = 1;          // one kernel for both arrangements: a row's logits do not depend on how many rows share the call
-                return ap;
-            };
-            if (attn_loop) {
-                for (int tl = 0; tl < tc; ++tl) launch_attn_decode(attn_params(tl), batch, s);
-            } else {
-                AttnParams ap = attn_params(0);
-                ap.cache_rows = rs;
-                ap.append_only = 1;
-                launch_attn_decode(ap, Mr, s);
-                ap.append_only = 0;
-                launch_attn_decode(ap, Mr, s);
+            else {
+                PfExtra ex;
+                ex.ldx = d; ex.ldc = c->Nqkv;
+                launch_gemm_pf(PF_ROWS_BF16, c->pf_x.p, c->wqkv.p + layer_qkv_elems(c) * li, c->pf_qkv16.p, M, c->Nqkv, d, s, ex);
             }
+            PfAttn pa{};
+            pa.qkv = coded ? (const void*)c->pf_qkv.p : (const void*)c->pf_qkv16.p; pa.qkv_f32 = coded;
+            pa.q = c->pf_q.p; pa.out = c->pf_attn.p;
+            pa.kcache = c->kcache.p + lkv * li; pa.vcache = c->vtcache.p + lkv * li;
+            pa.lens = lens_dev; pa.Lmax = Lmax; pa.t0 = t0; pa.tc = tc; pa.rs = rs; pa.batch = batch;
+            pa.Nqkv = c->Nqkv; pa.H = c->H; pa.Hkv = c->Hkv; pa.D = c->D; pa.Smax = c->Smax;
+            pa.rope_cos = c->rope_cos.p; pa.rope_sin = c->rope_sin.p; pa.scale = 1.0f / sqrtf((float)c->D);
+            if (c->cfg.qk_norm) {
+                pa.qnorm_w = c->qknorm.p + (size_t)(2 * li) * c->D;
+                pa.knorm_w = c->qknorm.p + (size_t)(2 * li + 1) * c->D;
+                pa.qk_eps = c->cfg.rms_norm_eps;
+            }
+            pa.rope_in_dtype = c->cfg.rope_ops_in_dtype;
+            launch_pf_attention(pa, s);
             if (coded) q_rows(M, [&](int r0, int mp) {
                 launch_pf_pack_rows(c->pf_attn.p + (size_t)r0 * HD, c->pf_xpk.p, mp, HD, s);
                 q_partial(c->q_o, li, c->pf_xpk.p, c->pf_tmp.p, d, HD, mp);

@@ -62,7 +62,7 @@ void launch_pack_qweight(int bits, const uint32_t* wq, const bf16_t* scales, con
 enum { PF_F32 = 0, PF_RESID = 1, PF_SILU = 2,
        PF_SPLIT_RELU2 = 3,       // tiles below PfExtra::split: float32 [M][ldc]; the others: T(relu(y)^2) bf16 row-major [M][ld2] at out2
        PF_SCALED_ADD = 4,        // float32 C[M][ldc] += ls[n] * y
-       PF_ROWS_BF16 = 5,         // bf16 row-major [M][ldc]; rows of X gathered: row m at X + xrow[m] * ldx
+       PF_ROWS_BF16 = 5,         // bf16 row-major [M][ldc]; row m of X at X + xrow[m] * ldx (xrow null: m * ldx)
        PF_SOFTCAP = 6,           // float32 [M][ldc]: cap tanh(scale y / cap)
        PF_SWIGLU = 7,            // PF_SILU in float32 up to one rounding
        PF_ACT_ROWS = 8 };        // bf16 row-major [M][ldc]: T(silu(y)) in the tiles below PfExtra::split, T(sigmoid(y)) in the others
@@ -75,6 +75,21 @@ void launch_pf_rows_rmsnorm(const bf16_t* rows, int src_rows, const int32_t* len
                             bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int d, float eps, hipStream_t s);
 void launch_pf_rmsnorm(const bf16_t* h, const bf16_t* wnorm, bf16_t* x, int rows, int d, float eps, hipStream_t s);
 void launch_pf_pack_rows(const bf16_t* rows, bf16_t* xpk, int Mpad, int d, hipStream_t s);
+
+// causal attention of the chunk of positions [t0, t0 + tc) of `batch` left-padded prompts (row (t - t0) * rs + b; lens: device): q|k|v -> norm, rotation,
+// cache append, attention over the caches.  q: scratch for the roped queries, out: bf16 [rows][H D] (rows of padded positions are not written)
+struct PfAttn {
+    const void* qkv; int qkv_f32;            // [rows][Nqkv] float32 or bf16
+    bf16_t *q, *out;
+    bf16_t *kcache, *vcache;                 // layer slices, tiled
+    const int32_t* lens;
+    int Lmax, t0, tc, rs, batch, Nqkv, H, Hkv, D, Smax;
+    const float *rope_cos, *rope_sin;
+    const bf16_t *qnorm_w, *knorm_w;         // null: no per-head norm
+    float qk_eps, scale;
+    int rope_in_dtype;
+};
+void launch_pf_attention(const PfAttn& a, hipStream_t s);
 
 // split-K factor of a weight-streaming GEMM (items = n-tile groups, KT = k-tiles, ksb = waves per item), see the definition
 int gemm_choose_split(int items, int KT, int ksb, int s_max);

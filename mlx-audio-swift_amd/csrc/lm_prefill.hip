@@ -13,14 +13,18 @@
 //                       a weight fragment is one 1 KiB global_load_lds piece and its LDS image IS the A fragment (lane-linear:
 //                       ds_read_b128 at lane*16, conflict free); X tiles as in k_gemm_big2 (whisper_kernels.hip: source-side
 //                       XOR swizzle).  128 x 128 x 64 tiles, two LDS buffers, one barrier per k-step.  Epilogues:
-//                         PF_F32    float32 [M][N]                       (q|k|v: the attention prologue reads it as a 1-slab split-K sum)
+//                         PF_ROWS_BF16  T(acc) [M][N]                    (q|k|v)
 //                         PF_RESID  h = T(h + T(acc)) in place, bf16      (o_proj, down_proj: LlamaTTS.swift:306-309)
 //                         PF_SILU   act = T(T(g T(sigmoid g)) u), gate / up tiles interleaved as packed (:283)
+//   k_pf_rope_append    q|k|v of the chunk -> roped queries (bf16 rows) and the tiled K / V caches of the decode step
+//   k_pf_attn           causal attention of the chunk's queries over the caches (MFMA, K / V tiles shared by 128 or 256 queries)
 //   k_pf_rmsnorm        x[r] = RMSNorm(h[r]) row-major
 //   k_pf_pack_rows      rows of the last position -> the packed x operand of the decode step (lm_head of the first new token)
 // Rounding points are those of the decode step (bf16 at every MLX primitive boundary); only float32 summation orders differ.
 #include "common.h"
 #include "lm_kernels.h"
+
+#include <type_traits>
 
 #define PF_BM 128
 #define PF_BN 128
@@ -138,7 +142,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf(PfGemmParams p) {
         const int r = (wave * 4 + q) * 8 + (lane >> 3);
         const int chunk = (lane & 7) ^ ((r >> 1) & 7);
         const int xm = min(m0 + r, p.M - 1);
-        if constexpr (EPI == PF_ROWS_BF16) xsrc[q] = p.X + (size_t)p.ex.xrow[xm] * p.ex.ldx + chunk * 8;
+        if constexpr (EPI == PF_ROWS_BF16) xsrc[q] = p.X + (size_t)(p.ex.xrow ? p.ex.xrow[xm] : xm) * p.ex.ldx + chunk * 8;
         else xsrc[q] = p.X + (size_t)xm * p.K + chunk * 8;
     }
     auto stage = [&](int buf, int ks) {                  // k-step ks covers k-tiles 2 ks, 2 ks + 1 = columns 64 ks .. +64
@@ -276,7 +280,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf(PfGemmParams p) {
 void launch_gemm_pf(int epi, const bf16_t* X, const bf16_t* Wp, void* C, int M, int N, int K, hipStream_t s, const PfExtra& ex) {
     MIS_REQUIRE(K % PF_BK == 0 && K >= 2 * PF_BK && N % 16 == 0 && M >= 1, MIS_ERR_GENERATION_FAILED, "prefill GEMM: K must be a multiple of 64");
     MIS_REQUIRE((epi != PF_SILU && epi != PF_SWIGLU) || N % 32 == 0, MIS_ERR_GENERATION_FAILED, "prefill GEMM: gate / up tiles come in pairs");
-    MIS_REQUIRE(epi < PF_SPLIT_RELU2 || epi == PF_SWIGLU || (ex.ldc % 4 == 0 && (epi != PF_ROWS_BF16 || (ex.xrow && ex.ldx % 8 == 0))), MIS_ERR_GENERATION_FAILED,
+    MIS_REQUIRE(epi < PF_SPLIT_RELU2 || epi == PF_SWIGLU || (ex.ldc % 4 == 0 && (epi != PF_ROWS_BF16 || ex.ldx % 8 == 0)), MIS_ERR_GENERATION_FAILED,
                 "prefill GEMM: bad row strides");
     PfGemmParams p{X, Wp, C, M, N, K, ex};
     // column tiles rounded up to the 8 XCDs: blocks are dealt to the XCDs by linear id, so that every row of tiles finds its weight tiles in the
@@ -317,4 +321,297 @@ void launch_pf_add_resid(bf16_t* h, const float* part, size_t n, hipStream_t s) 
 }
 void launch_pf_pack_rows(const bf16_t* rows, bf16_t* xpk, int Mpad, int d, hipStream_t s) {
     hipLaunchKernelGGL(k_pf_pack_rows, dim3(Mpad), dim3(256), 0, s, rows, xpk, d, Mpad / 16);
+}
+
+// ============================================================================ causal attention of a chunk of positions
+//
+// Two launches per layer.  k_pf_rope_append rounds q|k|v to bf16, applies the per-head norm (where the model has one) and the rotation, writes the
+// queries as bf16 rows and the keys / values into the decode step's tiled caches (whole 16-byte pieces; one block = the positions of one 32-key tile
+// of one kv head of one sequence).  k_pf_attn then walks the cache tiles: the G query heads of a kv head times its positions are ONE list of queries
+// (query n = position n / G, head n % G), a block takes 32 of them per wave, stages every 32-key tile's K and V images once through LDS (two buffers,
+// the next tile requested before this one is multiplied) and uses each fragment for both of a wave's groups of 16 queries.  A tile above a
+// wave's last position is skipped, only tiles that reach a wave's positions are masked, and the output is rescaled only when some maximum moved.
+// A query's sums run over the tiles 0, 1, 2, ... whatever block, chunk or batch it is part of: the same bits in every arrangement.
+// P enters P.V as bf16 hi + lo (probabilities keep float32 accuracy), like the decode step.
+// Measured (8 rows x 450 positions, 24 / 8 heads x 128): 59 us attention + 25 us rope / append per layer; the decode kernel with one block per (position,
+// kv head), which stood here before, streamed every query's whole cache for itself: 766 us.  Bound now: the softmax's VALU work and one barrier a tile.
+// float32 q|k|v rows would cost another 37 MB written and read per layer: the projection rounds them, which is the first thing the attention did.
+struct PfAttnDev {
+    const void* qkv; int Nqkv;
+    bf16_t *q, *kc, *vc, *out;
+    const int32_t* lens;
+    int Lmax, t0, tc, rs, H, Hkv, Smax;
+    const float *rope_cos, *rope_sin;
+    const bf16_t *qnorm_w, *knorm_w;
+    float qk_eps, scale;
+    int rope_in_dtype;
+};
+// positions of sequence b that the chunk holds: [lo, hi); position p is row (p + shift) * rs + b
+struct PfSpan { int lo, hi, shift; };
+__device__ __forceinline__ PfSpan pf_span(const PfAttnDev& p, int b) {
+    PfSpan r;
+    r.shift = p.Lmax - p.lens[b] - p.t0;
+    r.lo = max(0, -r.shift);
+    r.hi = p.tc - r.shift;
+    return r;
+}
+__device__ __forceinline__ void pf_load8(const float* src, float (&v)[8]) {
+    const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
+    v[0] = bf16_round_f32(a.x); v[1] = bf16_round_f32(a.y); v[2] = bf16_round_f32(a.z); v[3] = bf16_round_f32(a.w);
+    v[4] = bf16_round_f32(b.x); v[5] = bf16_round_f32(b.y); v[6] = bf16_round_f32(b.z); v[7] = bf16_round_f32(b.w);
+}
+__device__ __forceinline__ void pf_load8(const bf16_t* src, float (&v)[8]) {
+    const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(src);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = bf16_to_f32((bf16_t)a[e]);
+}
+template <int D, typename TIN>
+__global__ void __launch_bounds__(256) k_pf_rope_append(PfAttnDev p) {
+    constexpr int VT = D / 16;                                   // threads per head row: 8 dimensions and their 8 rotation partners each
+    __shared__ __attribute__((aligned(16))) bf16_t vs[32][D + 8];
+    const int b = blockIdx.z, kvh = blockIdx.y, tid = threadIdx.x;
+    const PfSpan sp = pf_span(p, b);
+    const int tile = (sp.lo >> 5) + blockIdx.x, p0 = max(tile * 32, sp.lo), p1 = min(tile * 32 + 32, sp.hi);
+    if (p0 >= p1) return;
+    const int G = p.H / p.Hkv;
+    const TIN* qkv = reinterpret_cast<const TIN*>(p.qkv);
+    bf16_t* kc = p.kc + ((size_t)(b * p.Hkv + kvh) * p.Smax) * D;
+    bf16_t* vc = p.vc + ((size_t)(b * p.Hkv + kvh) * p.Smax) * D;
+    for (int it = tid; it < (p1 - p0) * VT * 2; it += 256) {     // V rows -> LDS
+        const int i = it / (VT * 2), c = it - i * (VT * 2), pos = p0 + i;
+        const size_t row = (size_t)(pos + sp.shift) * p.rs + b;
+        float v[8];
+        pf_load8(qkv + row * p.Nqkv + (size_t)(p.H + p.Hkv + kvh) * D + c * 8, v);
+        bf16x8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (short)f32_to_bf16(v[e]);
+        *reinterpret_cast<bf16x8_t*>(&vs[pos & 31][c * 8]) = o;
+    }
+    for (int it = tid; it < (p1 - p0) * (G + 1) * VT; it += 256) {
+        const int j = it % VT, hr = it / VT, i = hr / (G + 1), hh = hr - i * (G + 1), pos = p0 + i;
+        const size_t row = (size_t)(pos + sp.shift) * p.rs + b;
+        const int col = (hh < G ? kvh * G + hh : p.H + kvh) * D + j * 8;
+        float x1[8], x2[8];
+        pf_load8(qkv + row * p.Nqkv + col, x1);
+        pf_load8(qkv + row * p.Nqkv + col + D / 2, x2);
+        if (p.qnorm_w) {                                         // n = T(x rsqrt(mean x^2 + eps)), T(w n)
+            float ss = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += x1[e] * x1[e] + x2[e] * x2[e];
+#pragma unroll
+            for (int o = 1; o < VT; o <<= 1) ss += __shfl_xor(ss, o, 64);
+            const float inv = 1.0f / sqrtf(ss / (float)D + p.qk_eps);
+            const bf16_t* w = hh < G ? p.qnorm_w : p.knorm_w;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                x1[e] = bf16_round_f32(bf16_to_f32(w[j * 8 + e]) * bf16_round_f32(x1[e] * inv));
+                x2[e] = bf16_round_f32(bf16_to_f32(w[D / 2 + j * 8 + e]) * bf16_round_f32(x2[e] * inv));
+            }
+        }
+        const float* ct = p.rope_cos + (size_t)pos * (D / 2) + j * 8;
+        const float* st = p.rope_sin + (size_t)pos * (D / 2) + j * 8;
+        bf16x8_t r1, r2;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float c = ct[e], s = st[e];
+            if (p.rope_in_dtype) {
+                c = bf16_round_f32(c); s = bf16_round_f32(s);
+                r1[e] = (short)f32_to_bf16(bf16_round_f32(x1[e] * c) + bf16_round_f32(-x2[e] * s));
+                r2[e] = (short)f32_to_bf16(bf16_round_f32(x2[e] * c) + bf16_round_f32(x1[e] * s));
+            } else {
+                r1[e] = (short)f32_to_bf16(x1[e] * c - x2[e] * s);
+                r2[e] = (short)f32_to_bf16(x1[e] * s + x2[e] * c);
+            }
+        }
+        if (hh < G) {
+            bf16_t* o = p.q + row * ((size_t)p.H * D) + col;
+            *reinterpret_cast<bf16x8_t*>(o) = r1;
+            *reinterpret_cast<bf16x8_t*>(o + D / 2) = r2;
+        } else {                                                 // K tiling: fragment row `prow` of half `half` (lm_kernels.hip), 8 dimensions = one piece
+            const int pr = pos & 31, prow = ((pr >> 3) << 2) | (pr & 3), half = (pr >> 2) & 1;
+            bf16_t* o = kc + ((size_t)tile * 2 + half) * (D / 32) * 512 + prow * 8;
+            const int d2 = D / 2 + j * 8;
+            *reinterpret_cast<bf16x8_t*>(o + ((j >> 2) * 64 + ((j & 3) << 4)) * 8) = r1;
+            *reinterpret_cast<bf16x8_t*>(o + ((d2 >> 5) * 64 + (((d2 & 31) >> 3) << 4)) * 8) = r2;
+        }
+    }
+    __syncthreads();
+    const int a0 = p0 & 31, a1 = a0 + (p1 - p0);                 // slots of the tile that this chunk fills
+    for (int it = tid; it < 4 * D; it += 256) {                  // V tiling: piece (d, octet of keys)
+        const int d = it & (D - 1), o = it / D;
+        bf16_t* dst = vc + (((size_t)tile * (D / 16) + (d >> 4)) * 64 + (o << 4) + (d & 15)) * 8;
+        if (o * 8 >= a0 && o * 8 + 8 <= a1) {
+            bf16x8_t v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = (short)vs[o * 8 + e][d];
+            *reinterpret_cast<bf16x8_t*>(dst) = v;
+        } else {
+            for (int e = 0; e < 8; ++e)
+                if (o * 8 + e >= a0 && o * 8 + e < a1) dst[e] = vs[o * 8 + e][d];
+        }
+    }
+}
+
+template <int D, int NW>
+__global__ void __launch_bounds__(NW * 64) k_pf_attn(PfAttnDev p) {
+    constexpr int IMG = 32 * D, PIECES = 2 * IMG / 8 / (NW * 64);    // bf16 elements of one K (or V) tile image; 16-byte pieces per thread
+    static_assert(PIECES * NW * 64 * 8 == 2 * IMG, "whole pieces");
+    __shared__ __attribute__((aligned(16))) bf16_t kv[2][2 * IMG];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kvh = blockIdx.y, b = blockIdx.z, G = p.H / p.Hkv;
+    const PfSpan sp = pf_span(p, b);
+    const int nq = (sp.hi - sp.lo) * G;
+    const int nb = (nq + 32 * NW - 1) / (32 * NW), blk = nb - 1 - (int)blockIdx.x;   // the longest blocks first
+    if (blk < 0) return;
+    const int n0 = blk * 32 * NW, w0 = n0 + wave * 32;
+    const int j = lane & 15, g4 = lane >> 4;
+    const int HD = p.H * D;
+    bf16x8_t qf[2][D / 32];
+    int qpos[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        const int n = min(w0 + 16 * g + j, nq - 1);                  // (queries past the list repeat the last one; never written)
+        const int pos = sp.lo + n / G;
+        qpos[g] = pos;
+        const bf16_t* src = p.q + ((size_t)(pos + sp.shift) * p.rs + b) * HD + (size_t)(kvh * G + n % G) * D + g4 * 8;
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c) qf[g][c] = *reinterpret_cast<const bf16x8_t*>(src + c * 32);
+    }
+    const int wlo = sp.lo + min(w0, nq - 1) / G, whi = w0 < nq ? sp.lo + min(w0 + 31, nq - 1) / G : -1;       // positions of the wave's queries
+    const int n_tiles = (sp.lo + min(n0 + 32 * NW - 1, nq - 1) / G) / 32 + 1;
+    const size_t base = ((size_t)(b * p.Hkv + kvh) * p.Smax) * D;
+    const uint4* ksrc = reinterpret_cast<const uint4*>(p.kc + base);
+    const uint4* vsrc = reinterpret_cast<const uint4*>(p.vc + base);
+    uint4 st[PIECES];
+    auto fetch = [&](int tile) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int pc = tid + i * NW * 64;                        // K image first, V image behind it
+            st[i] = pc < IMG / 8 ? ksrc[(size_t)tile * (IMG / 8) + pc] : vsrc[(size_t)tile * (IMG / 8) + pc - IMG / 8];
+        }
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) *(reinterpret_cast<uint4*>(kv[buf]) + tid + i * NW * 64) = st[i];
+    };
+    fetch(0);
+    put(0);
+    __syncthreads();
+    f32x4_t O[2][D / 16];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) O[g][dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f};
+    auto tile_math = [&](int tile, const bf16_t* img, auto masked_tag) {
+        constexpr bool MASKED = decltype(masked_tag)::value;
+        const int kb = tile * 32 + g4 * 8;
+        const bf16x8_t* kf = reinterpret_cast<const bf16x8_t*>(img) + lane;
+        const bf16x8_t* vf = reinterpret_cast<const bf16x8_t*>(img + IMG) + lane;
+        f32x4_t S[2][2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) S[g][0] = S[g][1] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c) {
+            const bf16x8_t a0 = kf[c * 64], a1 = kf[((D / 32) + c) * 64];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                S[g][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[g][c], S[g][0], 0, 0, 0);
+                S[g][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qf[g][c], S[g][1], 0, 0, 0);
+            }
+        }
+        bf16x8_t ph[2], pl[2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {                                // lane (query j, group g4): scores of keys kb .. kb + 7
+            float sc[8], mx = -INFINITY;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                float v = S[g][e >> 2][e & 3] * p.scale;
+                if constexpr (MASKED) v = kb + e <= qpos[g] ? v : -INFINITY;
+                sc[e] = v;
+                mx = fmaxf(mx, v);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float m_new = fmaxf(m_run[g], mx);                 // (tile 0 holds key 0, which every query sees: finite from there on)
+            const float alpha = __expf(m_run[g] - m_new);
+            float psum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pe = __expf(sc[e] - m_new);
+                psum += pe;
+                const bf16_t hi = f32_to_bf16(pe);
+                ph[g][e] = (short)hi;
+                pl[g][e] = (short)f32_to_bf16(pe - bf16_to_f32(hi));
+            }
+            l_run[g] = l_run[g] * alpha + psum;
+            const bool moved = m_new != m_run[g];
+            m_run[g] = m_new;
+            if (__any(moved)) {                                      // (alpha = 1 for every query otherwise)
+                float ar[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, g4 * 4 + r, 64);
+#pragma unroll
+                for (int dt = 0; dt < D / 16; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) O[g][dt][r] *= ar[r];
+            }
+        }
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) {
+            const bf16x8_t vb = vf[dt * 64];
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                O[g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph[g], vb, O[g][dt], 0, 0, 0);
+                O[g][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl[g], vb, O[g][dt], 0, 0, 0);
+            }
+        }
+    };
+    for (int tile = 0; tile < n_tiles; ++tile) {
+        const bool more = tile + 1 < n_tiles;
+        if (more) fetch(tile + 1);
+        if (tile * 32 + 31 <= wlo) tile_math(tile, kv[tile & 1], std::false_type{});
+        else if (tile * 32 <= whi) tile_math(tile, kv[tile & 1], std::true_type{});
+        if (more) put((tile + 1) & 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+        float l = l_run[g];
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {                                // O[g][dt][r]: query g4 * 4 + r, dimension dt * 16 + j
+            const float lr = __shfl(l, g4 * 4 + r, 64);
+            const int n = w0 + 16 * g + g4 * 4 + r;
+            if (n < nq) {
+                bf16_t* o = p.out + ((size_t)(sp.lo + n / G + sp.shift) * p.rs + b) * HD + (size_t)(kvh * G + n % G) * D + j;
+#pragma unroll
+                for (int dt = 0; dt < D / 16; ++dt) o[dt * 16] = f32_to_bf16(O[g][dt][r] / lr);
+            }
+        }
+    }
+}
+
+void launch_pf_attention(const PfAttn& a, hipStream_t s) {
+    MIS_REQUIRE(a.D == 64 || a.D == 128, MIS_ERR_INVALID_INPUT, "head_dim must be 64 or 128");
+    MIS_REQUIRE(a.H % a.Hkv == 0 && a.Smax % 32 == 0 && a.t0 + a.tc <= a.Smax && a.Nqkv == (a.H + 2 * a.Hkv) * a.D && a.rs >= a.batch, MIS_ERR_GENERATION_FAILED,
+                "prompt attention: bad dimensions");
+    MIS_REQUIRE((((uintptr_t)a.qkv | (uintptr_t)a.q | (uintptr_t)a.kcache | (uintptr_t)a.vcache) & 15) == 0, MIS_ERR_GENERATION_FAILED, "prompt attention: misaligned buffers");
+    PfAttnDev p{a.qkv, a.Nqkv, a.q, a.kcache, a.vcache, a.out, a.lens, a.Lmax, a.t0, a.tc, a.rs, a.H, a.Hkv, a.Smax, a.rope_cos, a.rope_sin, a.qnorm_w, a.knorm_w,
+                a.qk_eps, a.scale, a.rope_in_dtype};
+    const dim3 ga(a.tc / 32 + 2, a.Hkv, a.batch);                    // 32-key tiles that tc consecutive positions can touch
+    const int nq = a.tc * (a.H / a.Hkv);
+    // 256 queries a block share each staged tile where that still gives every compute unit a block; 128 otherwise
+    const bool wide = (long)cdiv(nq, 256) * a.Hkv * a.batch >= 256;
+    const dim3 gt(cdiv(nq, wide ? 256 : 128), a.Hkv, a.batch);
+    auto go = [&](auto tag) {
+        constexpr int D = decltype(tag)::value;
+        if (a.qkv_f32) hipLaunchKernelGGL((k_pf_rope_append<D, float>), ga, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((k_pf_rope_append<D, bf16_t>), ga, dim3(256), 0, s, p);
+        if (wide) hipLaunchKernelGGL((k_pf_attn<D, 8>), gt, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL((k_pf_attn<D, 4>), gt, dim3(256), 0, s, p);
+    };
+    if (a.D == 128) go(std::integral_constant<int, 128>{});
+    else go(std::integral_constant<int, 64>{});
 }
