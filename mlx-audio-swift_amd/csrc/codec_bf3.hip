@@ -273,7 +273,7 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
             }
         }
 
-        // ---- epilogue (the modes of k_snac_gemm / k_conv_taps).  C/D layout: col = lane & 31, row = (r & 3) + 8 (r >> 2) + 4 (lane >> 5)
+        // ---- epilogue (the modes of k_codec_gemm / k_conv_taps / k_snac_convt).  C/D layout: col = lane & 31, row = (r & 3) + 8 (r >> 2) + 4 (lane >> 5)
         // opaque: left visible, the 32 rows' 64-bit offsets are computed ahead of the main loop and spilled (860 B of scratch per
         // lane in the multi-tile experiment: 1.9x slower)
         int lane_hi = lane >> 5;
@@ -301,13 +301,7 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
             float nz = 0.0f;
             if (noise) {
                 if (pnoise) nz = pnoise[(size_t)b * p.N + n];
-                else if (p.noise_rng) {
-                    uint64_t row = (uint64_t)(p.row_offset + (p.row_ids ? p.row_ids[b] : b));
-                    uint64_t u = mis_splitmix64((p.noise_key ^ (row * 0xD1B54A32D192ED03ull)) + (uint64_t)n);
-                    float u1 = ((float)(uint32_t)(u >> 40) + 0.5f) * 5.9604644775390625e-08f;
-                    float u2 = ((float)(uint32_t)((u >> 16) & 0xFFFFFF) + 0.5f) * 5.9604644775390625e-08f;
-                    nz = sqrtf(-2.0f * logf(u1)) * cosf(6.283185307179586f * u2);
-                }
+                else if (p.noise_rng) nz = codec_noise_value(p.noise_key, (uint64_t)(p.row_offset + (p.row_ids ? p.row_ids[b] : b)), n);
             }
             const int o = convt ? p.s * n + phase : n;
             if (o >= p.Tout) continue;

@@ -23,6 +23,14 @@ __device__ __forceinline__ float mis_sin_sq(float y) {
     return p * p;
 }
 
+// NoiseBlock noise (MLXRandom.normal([B,1,T]), Layers.swift:274): Box-Muller on mis-synth-v1 uniforms keyed by (seed, block, GLOBAL row, t)
+__device__ __forceinline__ float codec_noise_value(uint64_t key, uint64_t row, int n) {
+    const uint64_t u = mis_splitmix64((key ^ (row * 0xD1B54A32D192ED03ull)) + (uint64_t)n);
+    const float u1 = ((float)(uint32_t)(u >> 40) + 0.5f) * 5.9604644775390625e-08f;
+    const float u2 = ((float)(uint32_t)((u >> 16) & 0xFFFFFF) + 0.5f) * 5.9604644775390625e-08f;
+    return sqrtf(-2.0f * logf(u1)) * cosf(6.283185307179586f * u2);
+}
+
 // Per-model state of the split-bf16 path (codec_bf3.hip): packed hi/lo weight fragments keyed by the A^T pointer (packed on first use,
 // on the calling stream) and the split-activation scratch planes.  One in-flight call per model handle, as for the rest of the engine.
 struct CodecPack {
@@ -75,6 +83,8 @@ struct GemmParams {
 };
 // snake: Snake prologue on the X rows (CONVT always runs it: pass alpha = ralpha = zeros for identity)
 void launch_gemm(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
+// exact-f32 kernels (codec_f32.hip): every mode but CONVT, TAPS without Snake; p must have ldx / ldy resolved
+void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // split-bf16 path; false = shape not eligible (or MIS_CODEC_EXACT_F32=1), nothing launched.  p must have ldx / ldy resolved
 bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // depthwise 7-tap conv (zero padded, dilation dil): shorter odd kernels ride in centred 7-tap weights

@@ -17,7 +17,7 @@
 //    to the whole-sequence decode - except where the reference itself differs: its overlap-add sums two biased transposed-conv
 //    outputs, so the first `stride` samples after every chunk boundary carry the bias twice (`dup_bias`, on by default).
 // Activations are NCT ([B][C][T], time contiguous); dense convs are exact-f32 MFMA contractions over (tap, channel)
-// (k_snac_gemm modes TAPS / CONVT of snac.hip) with the SnakeBeta activation fused into the operand load.
+// (modes TAPS / CONVT of launch_gemm) with the SnakeBeta activation fused into the operand load.
 #include "common.h"
 #include "kernels.h"
 #include "codec_kernels.h"

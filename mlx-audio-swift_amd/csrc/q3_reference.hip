@@ -12,7 +12,7 @@
 //
 // Both run once per reference recording (the model caches the result, Qwen3TTS.swift:268-300), so the design goal is exactness and
 // few moving parts, not the last microsecond: activations are [C][T] (time contiguous), every contraction is an exact-f32 MFMA GEMM of
-// snac.hip (k_snac_gemm / k_conv_taps: the codebook decisions of the VQ do not survive reduced precision), strided convs become
+// the exact-f32 kernels (codec_f32.hip: the codebook decisions of the VQ do not survive reduced precision), strided convs become
 // two-tap convs over a phase-split copy of their input, the transformer reuses the decoder's attention and normalisation kernels
 // (q3_codec.hip; interleaved RoPE = rotate-half RoPE after permuting the q / k rows of every head to evens-then-odds, which leaves
 // q.k unchanged), and the residual VQ of a frame runs in one block that keeps the residual in LDS across all quantizer layers.

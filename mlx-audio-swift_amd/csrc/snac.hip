@@ -9,8 +9,7 @@
 // Kernels (activations f32 [B][C][T], T contiguous):
 //   k_snac_embed   z_q = sum_i table_i[codes_i[b, t/stride_i]]       (table_i = codebook_i x out_proj_i + b_i)
 //   k_snac_dw      depthwise k=7 dilated conv with optional Snake before/after, LDS halo tile
-//   k_snac_gemm    Y = A x X on v_mfma_f32_32x32x2_f32 with fused Snake prologue and
-//                  bias / residual / NoiseBlock / transposed-conv-phase epilogues
+//   k_snac_convt   Snake -> transposed conv on v_mfma_f32_32x32x2_f32 (1x1 convs, NoiseBlock, strided convs: codec_f32.hip)
 //   k_snac_final   Snake -> conv k7 (C -> 1) -> tanh
 #include "common.h"
 #include "kernels.h"
@@ -207,7 +206,7 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
     __shared__ float As[RU_KC][C];
     constexpr bool SQ = C == 128;                         // 2 x 2 waves of 64 x 64; else every wave: all C rows x 32 columns
     constexpr int MTW = SQ ? 2 : C / 32, NTW = SQ ? 2 : 1;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // (scalar: the channels' parameters come by s_load)
     const int n0 = blockIdx.x * RU_NT, b = blockIdx.y;
     const int wr = SQ ? (wave >> 1) * 64 : 0;             // first row / first column of the wave's tile
     const int wc = SQ ? (wave & 1) * 64 : wave * 32;
@@ -337,35 +336,27 @@ __global__ void __launch_bounds__(256, 2) k_pw_fused(PwFusedParams p) {
 #define G_AH (G_BK / 16)              // staged A float4 per thread: rows ar + 16 h
 #define G_XH (G_BK / 8)               // staged X float4 per thread: rows xr + 8 h
 
+// transposed conv (the other modes: codec_f32.hip): phase = output index mod s; output o = s*n + phase takes taps j = 0, 1 from x[:, n + q - j]
 // (body behind restrict-qualified parameters for the arrays the epilogue touches: see k_pw_fused)
-template <int MODE, bool SNAKE>
-__device__ __forceinline__ void snac_gemm_body(const GemmParams& p, const float* __restrict__ pX, const float* __restrict__ pR,
-                                               float* __restrict__ pY, const float* __restrict__ pbias, const float* __restrict__ pscale) {
+__device__ __forceinline__ void snac_convt_body(const GemmParams& p, const float* __restrict__ pX, float* __restrict__ pY, const float* __restrict__ pbias) {
     __shared__ float As[G_BK][G_BM];
     __shared__ float Xs[G_BK][G_BN];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int n0 = blockIdx.x * G_BN, m0 = blockIdx.y * G_BM;
-    int b, phase = 0;
-    if (MODE == GEMM_CONVT) { b = blockIdx.z / p.s; phase = blockIdx.z % p.s; }
-    else b = blockIdx.z;
-    const int Kx = (MODE == GEMM_CONVT || MODE == GEMM_TAPS) ? p.Cin : p.K;
+    const int b = blockIdx.z / p.s, phase = blockIdx.z % p.s;
     const float* AT = p.AT + (size_t)phase * p.K * p.M;
-    const float* Xb = pX + (size_t)b * Kx * p.ldx;
-    // transposed conv phase: out o = s*n + phase takes taps j=0,1 from x[:, n + q - j]
-    const int q = (MODE == GEMM_CONVT) ? (phase + p.pad) / p.s : 0;
-
+    const float* Xb = pX + (size_t)b * p.Cin * p.ldx;
+    const int q = (phase + p.pad) / p.s;
     f32x16_t acc[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
-
     // staging registers: A: G_AH float4 / thread, X: G_XH float4 / thread
     const int ar = tid >> 4, ac = (tid & 15) * 4;          // A tile rows ar + 16 h (k), col (m)
     const int xr = tid >> 5, xc = (tid & 31) * 4;          // X tile rows xr + 8 h, col (n)
     float ra[G_AH][4], rx[G_XH][4];
-
     auto load_chunk = [&](int k0) {
 #pragma unroll
         for (int h = 0; h < G_AH; ++h) {   // A^T tile
@@ -380,31 +371,21 @@ __device__ __forceinline__ void snac_gemm_body(const GemmParams& p, const float*
         }
 #pragma unroll
         for (int h = 0; h < G_XH; ++h) {   // X tile
-            int k = k0 + xr + 8 * h;
-            int row = k, shift = 0;
-            if (MODE == GEMM_CONVT) { int j = k / p.Cin; row = k - j * p.Cin; shift = q - j; }
-            if (MODE == GEMM_TAPS) { int j = k / p.Cin; row = k - j * p.Cin; shift = (j - (p.taps - 1)) * p.dil; }
-            int n = n0 + xc + shift;
-            bool kin = k < p.K;
+            const int k = k0 + xr + 8 * h, j = k / p.Cin, row = k - j * p.Cin, n = n0 + xc + q - j;
+            const bool kin = k < p.K;
             const float* src = Xb + (size_t)row * p.ldx;
-            if (MODE != GEMM_CONVT && MODE != GEMM_TAPS && kin && (p.ldx & 3) == 0 && n + 3 < p.Tin) {
-                float4 v = *reinterpret_cast<const float4*>(src + n);
-                rx[h][0] = v.x; rx[h][1] = v.y; rx[h][2] = v.z; rx[h][3] = v.w;
-            } else {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    int nn = n + e;
-                    rx[h][e] = (kin && nn >= p.x_lo && nn < p.Tin) ? src[nn] : 0.0f;
-                }
+            for (int e = 0; e < 4; ++e) {
+                const int nn = n + e;
+                rx[h][e] = (kin && nn >= p.x_lo && nn < p.Tin) ? src[nn] : 0.0f;
             }
-            if (SNAKE && kin) {
+            if (kin) {
                 float a = p.alpha[row], r = p.ralpha[row];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) rx[h][e] = snake_f(rx[h][e], a, r);   // snake(0)=0 keeps the zero pad
             }
         }
     };
-
     const int nchunks = (p.K + G_BK - 1) / G_BK;
     load_chunk(0);
     for (int kc = 0; kc < nchunks; ++kc) {
@@ -428,57 +409,23 @@ __device__ __forceinline__ void snac_gemm_body(const GemmParams& p, const float*
             }
         }
     }
-
-    // NoiseBlock noise for this lane's two columns (MLXRandom.normal([B,1,T]), Layers.swift:274):
-    // explicit tensor, or Box-Muller on mis-synth-v1 uniforms keyed by (seed, block, GLOBAL row, t)
-    float nzv[2] = {0.0f, 0.0f};
-    if (MODE == GEMM_NOISE) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            int n = n0 + wn * 64 + t * 32 + (lane & 31);
-            if (n >= p.N) continue;
-            if (p.noise) nzv[t] = p.noise[(size_t)b * p.N + n];
-            else if (p.noise_rng) {
-                uint64_t row = (uint64_t)(p.row_offset + (p.row_ids ? p.row_ids[b] : b));
-                uint64_t u = mis_splitmix64((p.noise_key ^ (row * 0xD1B54A32D192ED03ull)) + (uint64_t)n);
-                float u1 = ((float)(uint32_t)(u >> 40) + 0.5f) * 5.9604644775390625e-08f;
-                float u2 = ((float)(uint32_t)((u >> 16) & 0xFFFFFF) + 0.5f) * 5.9604644775390625e-08f;
-                nzv[t] = sqrtf(-2.0f * logf(u1)) * cosf(6.283185307179586f * u2);
-            }
-        }
-    }
     // epilogue: C/D layout col = lane&31, row = (r&3) + 8*(r>>2) + 4*(lane>>5)
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        int n = n0 + wn * 64 + t * 32 + (lane & 31);
-        if (n >= p.N) continue;
+        const int n = n0 + wn * 64 + t * 32 + (lane & 31), o = p.s * n + phase;
+        if (n >= p.N || o >= p.Tout) continue;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            int m = m0 + wm * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
+            const int m = m0 + wm * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
             if (m >= p.M) continue;
             float v = acc[t][r];
             if (pbias) v += pbias[m];
-            if (MODE == GEMM_PLAIN || MODE == GEMM_TAPS) {
-                pY[((size_t)b * p.M + m) * p.ldy + n] = v;
-            } else if (MODE == GEMM_GELU) {                            // exact-erf GELU (VocosBackbone.swift:89)
-                pY[((size_t)b * p.M + m) * p.ldy + n] = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
-            } else if (MODE == GEMM_RESID) {
-                size_t o = ((size_t)b * p.M + m) * p.ldy + n;
-                if (pscale) v *= pscale[m];                          // ConvNeXt layer scale gamma (VocosBackbone.swift:92-95)
-                pY[o] = pR[o] + v;                                   // Layers.swift:230
-            } else if (MODE == GEMM_NOISE) {
-                size_t o = ((size_t)b * p.M + m) * p.ldy + n;
-                pY[o] = Xb[(size_t)m * p.ldx + n] + nzv[t] * v;       // Layers.swift:276-277
-            } else {
-                int o = p.s * n + phase;
-                if (n == 0 && p.dup_bias_n0 && pbias) v += pbias[m];   // streaming overlap-add counts the bias twice (GemmParams)
-                if (o < p.Tout) pY[((size_t)b * p.M + m) * p.ldy + o] = v;
-            }
+            if (n == 0 && p.dup_bias_n0 && pbias) v += pbias[m];       // streaming overlap-add counts the bias twice (GemmParams)
+            pY[((size_t)b * p.M + m) * p.ldy + o] = v;
         }
     }
 }
-template <int MODE, bool SNAKE>
-__global__ void __launch_bounds__(256) k_snac_gemm(GemmParams p) { snac_gemm_body<MODE, SNAKE>(p, p.X, p.R, p.Y, p.bias, p.scale); }
+__global__ void __launch_bounds__(256) k_snac_convt(GemmParams p) { snac_convt_body(p, p.X, p.Y, p.bias); }
 
 // ---- encoder kernels (Layers.swift:319-360, VQ.swift:47-120) ---------------------------------------------------------
 // first layer: conv k7 "same", 1 -> C
@@ -1229,22 +1176,16 @@ void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
         return;
     }
     if (launch_gemm_bf3(mode, snake, p, batch, s)) return;
-    int phases = (mode == GEMM_CONVT) ? p.s : 1;
+    MIS_REQUIRE(mode != GEMM_TAPS || (p.taps >= 1 && p.taps <= CT_MAXT && (p.taps - 1) * p.dil + 3 + G_BN <= CT_XS), MIS_ERR_INVALID_INPUT,
+                "dense conv: %d taps with dilation %d exceed the staged halo", p.taps, p.dil);
+    if (mode != GEMM_CONVT && (mode != GEMM_TAPS || !snake)) { launch_gemm_f32(mode, snake, p, batch, s); return; }
+    const int phases = mode == GEMM_CONVT ? p.s : 1;
     dim3 grid(cdiv(p.N, G_BN), cdiv(p.M, G_BM), batch * phases), block(256);
-    if (mode == GEMM_PLAIN) hipLaunchKernelGGL((k_snac_gemm<GEMM_PLAIN, false>), grid, block, 0, s, p);
-    else if (mode == GEMM_GELU) hipLaunchKernelGGL((k_snac_gemm<GEMM_GELU, false>), grid, block, 0, s, p);
-    else if (mode == GEMM_RESID && snake) hipLaunchKernelGGL((k_snac_gemm<GEMM_RESID, true>), grid, block, 0, s, p);
-    else if (mode == GEMM_RESID) hipLaunchKernelGGL((k_snac_gemm<GEMM_RESID, false>), grid, block, 0, s, p);
-    else if (mode == GEMM_TAPS) {
-        MIS_REQUIRE(p.taps >= 1 && p.taps <= CT_MAXT && (p.taps - 1) * p.dil + 3 + G_BN <= CT_XS, MIS_ERR_INVALID_INPUT,
-                    "dense conv: %d taps with dilation %d exceed the staged halo", p.taps, p.dil);
-        GemmParams q = p;
-        if (!snake) { q.alpha = nullptr; q.ralpha = nullptr; }
-        if (q.R) hipLaunchKernelGGL((k_conv_taps<true>), grid, block, 0, s, q);
-        else hipLaunchKernelGGL((k_conv_taps<false>), grid, block, 0, s, q);
+    if (mode == GEMM_TAPS) {             // dense conv with Snake in front: the activation runs once per staged element
+        if (p.R) hipLaunchKernelGGL((k_conv_taps<true>), grid, block, 0, s, p);
+        else hipLaunchKernelGGL((k_conv_taps<false>), grid, block, 0, s, p);
     }
-    else if (mode == GEMM_NOISE) hipLaunchKernelGGL((k_snac_gemm<GEMM_NOISE, false>), grid, block, 0, s, p);
-    else { MIS_REQUIRE(snake, MIS_ERR_GENERATION_FAILED, "convT without snake"); hipLaunchKernelGGL((k_snac_gemm<GEMM_CONVT, true>), grid, block, 0, s, p); }
+    else { MIS_REQUIRE(snake, MIS_ERR_GENERATION_FAILED, "convT without snake"); hipLaunchKernelGGL(k_snac_convt, grid, block, 0, s, p); }
 }
 
 static int64_t mis_snac_hop_for_encoder(const mis_snac* c) {

@@ -1,5 +1,5 @@
-"""Workload for a rocprofv3 --pmc pass over the MFMA-bound kernels: Qwen3-TTS speech-tokenizer decode (k_conv_taps, k_snac_gemm),
-SNAC decode (k_snac_gemm), Whisper-large-v3 encoder (k_gemm_big, k_attn_prefill), log-mel (k_mel_tile).  Synthetic weights."""
+"""Workload for a rocprofv3 --pmc pass over the MFMA-bound kernels: Qwen3-TTS speech-tokenizer decode (k_conv_taps, k_codec_gemm),
+SNAC decode (k_codec_gemm), Whisper-large-v3 encoder (k_gemm_big, k_attn_prefill), log-mel (k_mel_tile).  Synthetic weights."""
 import os, sys
 import numpy as np
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
