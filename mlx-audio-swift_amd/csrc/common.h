@@ -96,6 +96,25 @@ static inline hipError_t copy_now(void* dst, const void* src, size_t n, hipMemcp
     return e != hipSuccess ? e : hipStreamSynchronize(hipStreamPerThread);
 }
 
+// Large copies between device memory and the caller's pageable memory, through a pinned ring with the host side spread over threads: one thread alone
+// writes fresh pages (allocated and cleared as they are touched) at a fifth of the link's rate.  Belongs to a handle (one call in flight); reserve()
+// where the handle is finalized.  Without a ring, for small copies and for device or pinned memory: one plain asynchronous copy.  Both wait for the copy.
+struct HostRing {
+    static constexpr int SLOTS = 8;
+    static constexpr size_t SLOT = (size_t)2 << 20, MIN = (size_t)4 << 20;
+    PinnedBuf<uint8_t> buf;
+    hipEvent_t ev[SLOTS] = {};
+    HostRing() {}
+    HostRing(const HostRing&) = delete;
+    HostRing& operator=(const HostRing&) = delete;
+    ~HostRing();
+    void reserve();
+    void out(void* host, const void* dev, size_t n, hipStream_t s);
+    void in(void* dev, const void* host, size_t n, hipStream_t s);
+private:
+    void run(uint8_t* host, uint8_t* dev, size_t n, bool to_host, hipStream_t s);
+};
+
 static inline size_t round_up(size_t a, size_t b) { return (a + b - 1) / b * b; }
 static inline int cdiv(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 

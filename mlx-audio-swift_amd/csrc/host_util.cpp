@@ -11,8 +11,10 @@
 #include <sys/stat.h>
 #include <unistd.h>
 #include <algorithm>
+#include <atomic>
 #include <fstream>
 #include <sstream>
+#include <thread>
 
 static thread_local std::string g_last_error;
 
@@ -204,4 +206,91 @@ mis_dtype dtype_from_safetensors(const std::string& s) {
     if (s == "BF16") return MIS_BF16;
     if (s == "I32") return MIS_I32;
     throw MisError(MIS_ERR_INVALID_INPUT, "unsupported safetensors dtype " + s);
+}
+
+// ---------------------------------------------------------------------------- large host copies
+HostRing::~HostRing() {
+    for (auto& e : ev) if (e) (void)hipEventDestroy(e);
+}
+void HostRing::reserve() {
+    if (buf.p) return;
+    for (auto& e : ev) if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    buf.alloc(SLOTS * SLOT);
+}
+static bool is_pageable(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) { (void)hipGetLastError(); return true; }
+    return a.type == hipMemoryTypeUnregistered;
+}
+void HostRing::out(void* host, const void* dev, size_t n, hipStream_t s) {
+    if (n == 0) { HIP_CHECK(hipStreamSynchronize(s)); return; }
+    if (buf.p && n >= MIN && is_pageable(host)) { run((uint8_t*)host, (uint8_t*)const_cast<void*>(dev), n, true, s); return; }
+    HIP_CHECK(hipMemcpyAsync(host, dev, n, hipMemcpyDefault, s));
+    HIP_CHECK(hipStreamSynchronize(s));
+}
+void HostRing::in(void* dev, const void* host, size_t n, hipStream_t s) {
+    if (n == 0) return;
+    if (buf.p && n >= MIN && is_pageable(host)) { run((uint8_t*)const_cast<void*>(host), (uint8_t*)dev, n, false, s); return; }
+    HIP_CHECK(hipMemcpyAsync(dev, host, n, hipMemcpyDefault, s));
+    HIP_CHECK(hipStreamSynchronize(s));
+}
+// Chunk i uses slot i % SLOTS.  The calling thread queues the copies in order; worker w moves chunks w, w + SLOTS, ... between slot w and the caller's
+// memory.  turn[w] counts the hand-overs of slot w: even - the worker's, odd - the queue's (to the device), the other way round from it.
+void HostRing::run(uint8_t* host, uint8_t* dev, size_t n, bool to_host, hipStream_t s) {
+    const size_t chunks = (n + SLOT - 1) / SLOT;
+    const int workers = (int)std::min<size_t>(SLOTS, chunks);
+    int device = 0;
+    HIP_CHECK(hipGetDevice(&device));
+    std::atomic<size_t> turn[SLOTS];
+    std::atomic<int> bad{(int)hipSuccess};
+    for (auto& t : turn) t.store(0);
+    auto bytes = [&](size_t i) { return std::min(SLOT, n - i * SLOT); };
+    auto wait_turn = [&](int w, size_t t) {
+        while (turn[w].load(std::memory_order_acquire) < t) {
+            if (bad.load(std::memory_order_relaxed) != (int)hipSuccess) return false;
+            std::this_thread::yield();
+        }
+        return true;
+    };
+    auto worker = [&](int w) {
+        hipError_t e = hipSetDevice(device);
+        for (size_t i = w, k = 0; i < chunks && e == hipSuccess; i += SLOTS, ++k) {
+            if (to_host) {
+                if (!wait_turn(w, 2 * k + 1)) return;                 // the copy of this chunk is queued
+                if ((e = hipEventSynchronize(ev[w])) != hipSuccess) break;
+                memcpy(host + i * SLOT, buf.p + w * SLOT, bytes(i));
+            } else {
+                if (!wait_turn(w, 2 * k)) return;
+                if (k > 0 && (e = hipEventSynchronize(ev[w])) != hipSuccess) break;      // the slot's last copy has left it
+                memcpy(buf.p + w * SLOT, host + i * SLOT, bytes(i));
+            }
+            turn[w].fetch_add(1, std::memory_order_release);
+        }
+        if (e != hipSuccess) bad.store((int)e);
+    };
+    std::vector<std::thread> th;
+    auto join = [&] { for (auto& t : th) t.join(); th.clear(); };
+    try {
+        for (int w = 0; w < workers; ++w) th.emplace_back(worker, w);
+    } catch (...) {                                                   // no threads to be had: the plain copy
+        bad.store((int)hipErrorUnknown);
+        join();
+        HIP_CHECK(hipMemcpyAsync(to_host ? host : dev, to_host ? dev : host, n, hipMemcpyDefault, s));
+        HIP_CHECK(hipStreamSynchronize(s));
+        return;
+    }
+    for (size_t i = 0; i < chunks; ++i) {
+        const int w = (int)(i % SLOTS);
+        const size_t k = i / SLOTS;
+        if (!wait_turn(w, to_host ? 2 * k : 2 * k + 1)) break;
+        hipError_t e = to_host ? hipMemcpyAsync(buf.p + w * SLOT, dev + i * SLOT, bytes(i), hipMemcpyDeviceToHost, s)
+                               : hipMemcpyAsync(dev + i * SLOT, buf.p + w * SLOT, bytes(i), hipMemcpyHostToDevice, s);
+        if (e == hipSuccess) e = hipEventRecord(ev[w], s);
+        if (e != hipSuccess) { bad.store((int)e); break; }
+        turn[w].fetch_add(1, std::memory_order_release);
+    }
+    join();
+    const hipError_t e = hipStreamSynchronize(s);
+    if (bad.load() != (int)hipSuccess) HIP_CHECK((hipError_t)bad.load());
+    HIP_CHECK(e);
 }

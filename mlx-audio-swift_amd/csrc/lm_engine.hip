@@ -80,6 +80,7 @@ struct mis_tts {
     DevBuf<int32_t> pf_pos;
     DevBuf<uint8_t> pf_on;
     DevBuf<SamplerScratch> samp_scratch;
+    HostRing ring;
     hipGraphExec_t g_prefill = nullptr, g_decode = nullptr;
     bool shared_device = false;      // another replica's streams run on this device (group.hip): never a kernel that waits for co-resident blocks
     uint64_t graph_key = 0;
@@ -521,6 +522,7 @@ extern "C" mis_status mis_tts_finalize(mis_tts* c) {
     }
     c->staging.release();
     c->raw_staging.release();
+    c->ring.reserve();
     c->finalized = true;
     MIS_API_END
 }
@@ -1098,7 +1100,8 @@ extern "C" mis_status mis_lm_forward_hidden(mis_tts* c, const int32_t* ids, cons
         size_t n = (size_t)c->batch * c->V;
         hipLaunchKernelGGL(k_bf16_rows_to_f32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, c->logits.p, c->Vpad,
                            c->logits_f32.p, c->V, c->batch);
-        HIP_CHECK(hipMemcpyAsync(logits_out, c->logits_f32.p, n * 4, hipMemcpyDefault, s));
+        HIP_CHECK(hipGetLastError());
+        c->ring.out(logits_out, c->logits_f32.p, n * 4, s);
     }
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(s));
@@ -1174,7 +1177,8 @@ extern "C" mis_status mis_lm_prefill(mis_tts* c, const int32_t* prompt_ids, cons
         const size_t n = (size_t)batch * c->V;
         c->logits_f32.alloc(n);
         hipLaunchKernelGGL(k_bf16_rows_to_f32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, c->logits.p, c->Vpad, c->logits_f32.p, c->V, batch);
-        HIP_CHECK(hipMemcpyAsync(logits_out, c->logits_f32.p, n * 4, hipMemcpyDefault, s));
+        HIP_CHECK(hipGetLastError());
+        c->ring.out(logits_out, c->logits_f32.p, n * 4, s);
     }
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(s));

@@ -704,7 +704,8 @@ struct mis_snac {
     DevBuf<float> buf[3];
     CodecPack pack;                      // split-bf16 weight fragments + activation scratch (codec_bf3.hip)
     DevBuf<int32_t> codes_ws;
-    DevBuf<float> noise_ws;
+    DevBuf<float> noise_ws, pcm_ws;
+    HostRing ring;
     size_t act_capacity = 0;
     // noise == NULL policy: 0 = draw N(0,1) internally (the reference's behaviour), 1 = add nothing
     int null_noise_zero = 0;
@@ -1012,6 +1013,7 @@ extern "C" mis_status mis_snac_finalize(mis_snac* c) {
     c->arena.alloc(arena.size());
     HIP_CHECK(hipMemcpy(c->arena.p, arena.data(), arena.size() * sizeof(float), hipMemcpyHostToDevice));
     c->raw.clear();
+    c->ring.reserve();
     c->finalized = true;
     MIS_API_END
 }
@@ -1379,15 +1381,13 @@ extern "C" mis_status mis_snac_decode(mis_snac* c, const int32_t* const* codes, 
     std::vector<const float*> dnoise;
     snac_stage_inputs(c, codes, batch, t_coarse, noise, dcodes, dnoise);
     int64_t N = mis_snac_num_samples(c, t_coarse);
-    DevBuf<float> pcm;
-    pcm.alloc((size_t)batch * N);
+    c->pcm_ws.alloc((size_t)batch * N);
     int C; int64_t T;
     NoiseRng rng;
     rng.enabled = c->null_noise_zero ? 0 : 1; rng.seed = c->noise_seed;
-    snac_run(c, dcodes.data(), batch, t_coarse, dnoise.empty() ? nullptr : dnoise.data(), rng, pcm.p, N, -1, &C, &T, c->stream);
+    snac_run(c, dcodes.data(), batch, t_coarse, dnoise.empty() ? nullptr : dnoise.data(), rng, c->pcm_ws.p, N, -1, &C, &T, c->stream);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(pcm_out, pcm.p, (size_t)batch * N * sizeof(float), hipMemcpyDefault, c->stream));
-    HIP_CHECK(hipStreamSynchronize(c->stream));
+    c->ring.out(pcm_out, c->pcm_ws.p, (size_t)batch * N * sizeof(float), c->stream);
     c->last_batch = batch; c->last_t = t_coarse;
     c->last_codes = dcodes; c->last_noise_ptrs = dnoise; c->last_noise = !dnoise.empty();
     MIS_API_END

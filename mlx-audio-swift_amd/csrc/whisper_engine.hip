@@ -46,6 +46,10 @@ struct mis_whisper {
     DevBuf<bf16_t> h, h2, x, attn_out, act, logits;      // h2: the other residual buffer of the folded glue (enqueue_decoder_step)
     DevBuf<float> qkv_part, part, e_buf, logits_f32;
     DevBuf<SamplerScratch> scratch;
+    // encoder workspace (a sub-batch of up to 8 windows), audio and features of a call: kept, they are the same size call after call
+    DevBuf<bf16_t> e_col1, e_tight, e_h1, e_col2, e_h, e_x, e_qkv, e_att, e_ff, e_kc, e_vc, e_ckv;
+    DevBuf<float> pcm, padded, feats, enc_f32;
+    HostRing ring;
     bool shared_device = false;      // another replica's streams run on this device (group.hip): never a kernel that waits for co-resident blocks
 };
 
@@ -297,6 +301,7 @@ extern "C" mis_status mis_whisper_finalize(mis_whisper* c) {
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(s));
     c->raw.clear();
+    c->ring.reserve();
     c->finalized = true;
     MIS_API_END
 }
@@ -403,12 +408,14 @@ static void whisper_encode_device(mis_whisper* c, const float* features_dev, int
     // the encoder runs in sub-batches of <= 8 utterances to bound the activation buffers
     const int SB = std::min(batch, 8);
     const size_t M1 = (size_t)SB * 3000, M = (size_t)SB * 1500;
-    DevBuf<bf16_t> col1, h1, col2, h, x, qkv, att, ff, kc, vc, ckv;
+    DevBuf<bf16_t> &col1 = c->e_col1, &h1 = c->e_h1, &col2 = c->e_col2, &h = c->e_h, &x = c->e_x, &qkv = c->e_qkv, &att = c->e_att, &ff = c->e_ff, &kc = c->e_kc,
+                   &vc = c->e_vc, &ckv = c->e_ckv;
     col1.alloc(M1 * c->K1); h1.alloc(M1 * d); col2.alloc(M * 3 * d); h.alloc(M * d); x.alloc(M * d); qkv.alloc(M * 3 * d);
     att.alloc(M * d); ff.alloc(M * fe); ckv.alloc(M * 2 * d);
+    c->e_tight.alloc(M1 * 3 * c->nmel);
     size_t kvn = (size_t)SB * H * c->Spad * D;
     kc.alloc(kvn); vc.alloc(kvn);
-    HIP_CHECK(hipMemsetAsync(col1.p, 0, col1.bytes(), s));
+    HIP_CHECK(hipMemsetAsync(col1.p, 0, M1 * c->K1 * 2, s));
     HIP_CHECK(hipMemsetAsync(kc.p, 0, kvn * 2, s));
     HIP_CHECK(hipMemsetAsync(vc.p, 0, kvn * 2, s));
     for (int b0 = 0; b0 < batch; b0 += SB) {
@@ -417,12 +424,9 @@ static void whisper_encode_device(mis_whisper* c, const float* features_dev, int
         BigGemmParams g{};
         // gelu(conv1), gelu(conv2) + positions     (WhisperLayers.swift:147-151)
         {   // conv1 patches with row stride K1 (zero padded columns)
-            DevBuf<bf16_t> tight;
-            tight.alloc((size_t)m1 * 3 * c->nmel);
-            launch_im2col3_f32(features_dev + (size_t)b0 * 3000 * c->nmel, tight.p, nb, 3000, c->nmel, 3000, 1, s);
-            HIP_CHECK(hipMemcpy2DAsync(col1.p, (size_t)c->K1 * 2, tight.p, (size_t)3 * c->nmel * 2, (size_t)3 * c->nmel * 2, m1,
+            launch_im2col3_f32(features_dev + (size_t)b0 * 3000 * c->nmel, c->e_tight.p, nb, 3000, c->nmel, 3000, 1, s);
+            HIP_CHECK(hipMemcpy2DAsync(col1.p, (size_t)c->K1 * 2, c->e_tight.p, (size_t)3 * c->nmel * 2, (size_t)3 * c->nmel * 2, m1,
                                        hipMemcpyDeviceToDevice, s));
-            HIP_CHECK(hipStreamSynchronize(s));
         }
         g = BigGemmParams{col1.p, c->conv1w, c->conv1b, nullptr, h1.p, m1, d, c->K1, c->K1, 0};
         launch_gemm_big(BG_GELU, g, s);
@@ -457,7 +461,6 @@ static void whisper_encode_device(mis_whisper* c, const float* features_dev, int
                               c->Hd, D, c->Spad, s);
         }
         HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipStreamSynchronize(s));
     }
     whisper_decoder_reset(c);
 }
@@ -472,18 +475,16 @@ extern "C" mis_status mis_whisper_encode(mis_whisper* c, const float* features, 
     MIS_REQUIRE(c && features, MIS_ERR_INVALID_INPUT, "null argument");
     MIS_REQUIRE(batch >= 1 && batch <= 64, MIS_ERR_INVALID_INPUT, "batch per GPU must be 1..64");
     HIP_CHECK(hipSetDevice(c->device));
-    DevBuf<float> f;
     size_t n = (size_t)batch * 3000 * c->nmel;
-    f.alloc(n);
-    HIP_CHECK(copy_now(f.p, features, n * 4, hipMemcpyDefault));
-    whisper_encode_device(c, f.p, batch);
+    c->feats.alloc(n);
+    c->ring.in(c->feats.p, features, n * 4, c->stream);
+    whisper_encode_device(c, c->feats.p, batch);
     if (enc_out) {
         size_t ne = (size_t)batch * 1500 * c->d;
-        DevBuf<float> o;
-        o.alloc(ne);
-        hipLaunchKernelGGL(k_bf16_to_f32_flat, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, c->stream, c->enc_out.p, o.p, ne);
-        HIP_CHECK(hipStreamSynchronize(c->stream));
-        HIP_CHECK(copy_now(enc_out, o.p, ne * 4, hipMemcpyDefault));
+        c->enc_f32.alloc(ne);
+        hipLaunchKernelGGL(k_bf16_to_f32_flat, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, c->stream, c->enc_out.p, c->enc_f32.p, ne);
+        HIP_CHECK(hipGetLastError());
+        c->ring.out(enc_out, c->enc_f32.p, ne * 4, c->stream);
     }
     MIS_API_END
 }
@@ -627,17 +628,18 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     const int64_t W = 480000;
     std::vector<int64_t> hl(batch, stride);
     if (lens) HIP_CHECK(copy_now(hl.data(), lens, batch * sizeof(int64_t), hipMemcpyDefault));
-    DevBuf<float> padded, feats;
-    padded.alloc((size_t)batch * W);
-    feats.alloc((size_t)batch * 3000 * c->nmel);
-    HIP_CHECK(hipMemsetAsync(padded.p, 0, (size_t)batch * W * 4, hipStreamPerThread));
+    c->padded.alloc((size_t)batch * W);
+    c->feats.alloc((size_t)batch * 3000 * c->nmel);
+    c->pcm.alloc((size_t)batch * stride);
+    const int64_t last = std::max<int64_t>(0, std::min(hl[batch - 1], stride));         // (the last row need not be as long as the others)
+    c->ring.in(c->pcm.p, pcm, ((size_t)(batch - 1) * stride + last) * 4, s);
+    HIP_CHECK(hipMemsetAsync(c->padded.p, 0, (size_t)batch * W * 4, s));
     for (int b = 0; b < batch; ++b) {
-        int64_t n = std::min<int64_t>(std::min<int64_t>(hl[b], stride), W);
-        if (n > 0) HIP_CHECK(copy_now(padded.p + (size_t)b * W, pcm + (size_t)b * stride, (size_t)n * 4, hipMemcpyDefault));
+        const int64_t n = std::min<int64_t>(std::min<int64_t>(hl[b], stride), W);
+        if (n > 0) HIP_CHECK(hipMemcpyAsync(c->padded.p + (size_t)b * W, c->pcm.p + (size_t)b * stride, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
     }
-    HIP_CHECK(hipStreamSynchronize(hipStreamPerThread));
-    whisper_features_device(c->device, padded.p, batch, c->nmel, feats.p, s);
-    whisper_encode_device(c, feats.p, batch);
+    whisper_features_device(c->device, c->padded.p, batch, c->nmel, c->feats.p, s);
+    whisper_encode_device(c, c->feats.p, batch);
     // ---- prompt prefill, one token per step (same prompt for every row)
     std::vector<int32_t> prompt(n_prompt);
     HIP_CHECK(copy_now(prompt.data(), prompt_ids, n_prompt * 4, hipMemcpyDefault));
