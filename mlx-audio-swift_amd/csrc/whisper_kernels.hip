@@ -24,7 +24,7 @@
 // that follows: max |diff| 1.0e-6 of full scale, fewer mismatching roundings than the float32 0.5 x (1 + erf) form itself has.
 __device__ __forceinline__ float gelu_erf_w(float x) {
     const float z = fabsf(x) * 0.70710678118654752f;
-    const float t = __frcp_rn(1.0f + 0.3275911f * z);
+    const float t = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * z);      // (1 ulp: 6e-8 of a value good to 1.5e-7; the rounded division is ten instructions)
     float p = 1.061405429f;
     p = p * t - 1.453152027f;
     p = p * t + 1.421413741f;
@@ -261,7 +261,17 @@ __global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
     bf16_t* Ws = bg3_lds;                                        // [2][BN * 64]
     bf16_t* Xs = bg3_lds + (size_t)2 * BG3_BN * BG2_BK;          // [2][BM * 64]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * BG3_BN, m0 = blockIdx.y * BG3_BM;
+    // Blocks are dealt to the XCDs by id mod 8.  Up to 8 column tiles an XCD takes a contiguous range of row tiles and walks it column tile by column tile:
+    // the blocks it runs together share 6 tiles of X and 5 of W in one L2 (fc2 169 -> 158 us, out_proj 62 -> 58); with more column tiles the row-major
+    // order is the faster one (q|k|v 135 against 143 us).
+    const int nt = (p.N + BG3_BN - 1) / BG3_BN, mt = (p.M + BG3_BM - 1) / BG3_BM;
+    int ni = blockIdx.x % nt, mi = blockIdx.x / nt;
+    if (nt <= 8) {
+        const int xcd = blockIdx.x & 7, j0 = blockIdx.x >> 3, mlo = mt * xcd / 8, mcnt = mt * (xcd + 1) / 8 - mlo;
+        if (j0 >= mcnt * nt) return;
+        ni = j0 / mcnt; mi = mlo + j0 % mcnt;
+    }
+    const int n0 = ni * BG3_BN, m0 = mi * BG3_BM;
     const int wn = wave / WM, wm = wave % WM;
     f32x4_t acc[TN][TM];
 #pragma unroll
@@ -315,8 +325,11 @@ __global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
         if (kt + 1 < KT) stage((kt + 1) & 1, (kt + 1) * BG2_BK);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
+            // one wait, naming every fragment of this half; the other half's reads (LDS returns in order) run under its MFMAs
+            if (ks == 0) asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(a[0][0]) : "n"(TN + TM));
+            else asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a[1][0]));
 #pragma unroll
-            for (int i = 0; i < TN; ++i) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a[ks][i]));      // one wait, naming every fragment
+            for (int i = 0; i < TN; ++i) asm volatile("" : "+v"(a[ks][i]));
 #pragma unroll
             for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(b[ks][j]));
 #pragma unroll
@@ -367,7 +380,8 @@ static bool launch_big3_one(const BigGemmParams& p, hipStream_t s) {
     constexpr int lds_bytes = 2 * (BG3_BM + BG3_BN) * BG2_BK * 2;            // 128 KB
     static const bool ok = hipFuncSetAttribute((const void*)k_gemm_big3<EPI, WM, WN>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
     if (!ok) { (void)hipGetLastError(); return false; }
-    hipLaunchKernelGGL((k_gemm_big3<EPI, WM, WN>), dim3(cdiv(p.N, BG3_BN), cdiv(p.M, BG3_BM)), dim3(512), lds_bytes, s, p);
+    const int nt = cdiv(p.N, BG3_BN), mt = cdiv(p.M, BG3_BM);
+    hipLaunchKernelGGL((k_gemm_big3<EPI, WM, WN>), dim3(nt <= 8 ? 8 * nt * cdiv(mt, 8) : nt * mt), dim3(512), lds_bytes, s, p);
     return true;
 }
 template <int EPI>
@@ -570,6 +584,50 @@ void launch_scatter_kv(const bf16_t* src, int ld, int kcol0, int vcol0, bf16_t* 
 }
 
 // ============================================================================ encoder self attention (non causal)
+//
+// One 32-key tile of 16 queries: raw scores (lane = query j, key group g4: keys g4*8 + e) -> P as bf16 hi + lo in the P.V operand layout.  The softmax is
+// bound by VALU issue (360 M scores per layer of 8 windows), so: scores stay raw, p = 2^(S c - m) with c = scale log2 e in one fma; the maximum that p is
+// taken against moves only when some score passes it by more than 2^8 (`lim`: one compare per lane, no cross-lane traffic on the usual tile) - the ratio
+// numerator / denominator does not depend on it, and sums of at most 256 T stay far inside float32; hi / lo are converted two at a time.
+// Returns true where the maximum moved (wave-uniform): the output so far must be scaled by alpha.
+struct AttnRow { float m = -INFINITY, lim = -INFINITY, l = 0.0f; };
+template <bool MASKED>
+__device__ __forceinline__ bool attn_softmax_tile(const f32x4_t& S0, const f32x4_t& S1, int key0, int T, float c, AttnRow& r, bf16x8_t& ph, bf16x8_t& pl, float& alpha) {
+    typedef float f2_t __attribute__((ext_vector_type(2)));
+    typedef __bf16 h2_t __attribute__((ext_vector_type(2)));
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        s[e] = e < 4 ? S0[e] : S1[e - 4];
+        if constexpr (MASKED) s[e] = key0 + e < T ? s[e] : -INFINITY;
+    }
+    float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+    const bool moved = __any(mx > r.lim);
+    if (moved) {
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(r.m, mx * c);
+        alpha = __builtin_amdgcn_exp2f(r.m - m_new);                // (first tile: 2^-inf = 0)
+        r.m = m_new;
+        r.lim = (m_new + 8.0f) / c;
+        r.l *= alpha;
+    }
+    float psum = 0.0f;
+    uint32_t hw[4], lw[4];
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[e], c, -r.m)), p1 = __builtin_amdgcn_exp2f(fmaf(s[e + 1], c, -r.m));
+        psum += p0;
+        psum += p1;
+        const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){p0, p1}, h2_t));
+        hw[e >> 1] = h;
+        lw[e >> 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){p0 - __uint_as_float(h << 16), p1 - __uint_as_float(h & 0xffff0000u)}, h2_t));
+    }
+    r.l += psum;
+    ph = __builtin_bit_cast(bf16x8_t, make_uint4(hw[0], hw[1], hw[2], hw[3]));
+    pl = __builtin_bit_cast(bf16x8_t, make_uint4(lw[0], lw[1], lw[2], lw[3]));
+    return moved;
+}
 // grid (ceil(T/64), H, B), 4 waves x 16 query rows.  S^T = K Q^T (A = K fragment, B = Q^T): lane (q row j, group g4)
 // holds the scores of keys base + g4*8 + e; online softmax per query row; O += P V with P split into bf16 hi + lo.
 template <int D>
@@ -593,7 +651,8 @@ __global__ void __launch_bounds__(256) k_attn_prefill(const bf16_t* __restrict__
     f32x4_t O[D / 16];
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) O[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.0f;
+    AttnRow row;
+    const float sc2 = scale * 1.4426950408889634f;
     const int n_tiles = (T + 31) >> 5;
     for (int tile = 0; tile < n_tiles; ++tile) {
         const int kb = tile * 32;
@@ -605,45 +664,27 @@ __global__ void __launch_bounds__(256) k_attn_prefill(const bf16_t* __restrict__
             S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, qf[c], S0, 0, 0, 0);
             S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qf[c], S1, 0, 0, 0);
         }
-        float sc[8], mx = -INFINITY;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            float v = (e < 4 ? S0[e] : S1[e - 4]) * scale;
-            v = (kb + g4 * 8 + e < T) ? v : -INFINITY;
-            sc[e] = v;
-            mx = fmaxf(mx, v);
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        float m_new = fmaxf(m_run, mx);
-        float alpha = __expf(m_run - m_new);
-        float psum = 0.0f;
         bf16x8_t ph, pl;
+        float alpha = 1.0f;
+        if (attn_softmax_tile<true>(S0, S1, kb + g4 * 8, T, sc2, row, ph, pl, alpha)) {
+            float ar[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            float pe = __expf(sc[e] - m_new);
-            psum += pe;
-            bf16_t hi = f32_to_bf16(pe);
-            bf16_t lo = f32_to_bf16(pe - bf16_to_f32(hi));
-            ph[e] = (short)hi;
-            pl[e] = (short)lo;
+            for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, g4 * 4 + r, 64);
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) O[dt][r] *= ar[r];
         }
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        float ar[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, g4 * 4 + r, 64);
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) {
             bf16x8_t vb = vbase[((size_t)tile * (D / 16) + dt) * 64];
             f32x4_t o = O[dt];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] *= ar[r];
             o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, vb, o, 0, 0, 0);
             o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, vb, o, 0, 0, 0);
             O[dt] = o;
         }
     }
+    float l_run = row.l;
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
     // O[dt][r]: row = query (g4*4 + r), col = d (dt*16 + j); the row's normaliser lives in lane (g4*4 + r)
@@ -658,16 +699,14 @@ __global__ void __launch_bounds__(256) k_attn_prefill(const bf16_t* __restrict__
         }
     }
 }
-// ---- the same attention, tiled for the matrix core's appetite (round 6: k_attn_prefill<64> at MfmaUtil 0.21 was the worst
-// MFMA kernel of the tree).  What the kernel above costs per 32-key tile and wave: 16 fragment loads straight from global memory, waited
-// for where they are used (no tile in flight while another is multiplied), for 12 MFMAs on 16 query rows - and every one of the 94
-// waves of a head streams the head's whole 393 KB of K/V for itself.  Here a block is 256 query rows (8 waves x 2 groups of 16): the
-// tile's K and V images (8 KB, already in fragment order - lm_kernels.hip's cache tiling) are staged ONCE per block through LDS, one
-// 16-byte piece per thread, tile t + 1 requested before tile t is multiplied (two LDS buffers, one barrier per tile); a wave reads each
-// fragment once (lane-linear ds_read_b128, conflict-free) and uses it for both of its row groups: 24 MFMAs per 8 LDS reads.  The key
-// mask is applied on the last tile only, and the running output is rescaled only when some row's maximum moved (alpha = 1 otherwise:
-// skipping the multiply is exact).  Same operations per query row in the same order as k_attn_prefill: results are bit-identical
-// (tests/test_gpu_whisper.py).  Bound after this: the softmax's VALU work (exp, the bf16 hi/lo split of P), not the matrix core.
+// ---- the same attention on 256-row blocks.  What the kernel above costs per 32-key tile and wave: 16 fragment loads straight from global memory, waited
+// for where they are used, for 12 MFMAs on 16 query rows - and every one of the 94 waves of a head streams the head's whole 393 KB of K/V for itself.
+// Here a block is 256 query rows (8 waves x 2 groups of 16): the tile's K and V images (8 KB, already in fragment order - lm_kernels.hip's cache
+// tiling) are staged ONCE per block through LDS, one 16-byte piece per thread, tile t + 1 requested before tile t is multiplied (two LDS buffers, one
+// barrier per tile); a wave reads each fragment once (lane-linear ds_read_b128, conflict-free) and uses it for both of its row groups: 24 MFMAs per 8 LDS
+// reads.  The key mask is applied on the last tile only.  Same operations per query row in the same order as k_attn_prefill: results are bit-identical
+// (tests/test_gpu_whisper.py).  Bound: the softmax's VALU work, not the matrix core: 228 us per layer of 8 windows x 20 heads (260 us with the score's scale,
+// its logarithm base and a cross-lane maximum per tile in the loop; two tiles per barrier: 251).
 template <int D>
 __global__ void __launch_bounds__(512, 1) k_attn_prefill2(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kc,
                                                           const bf16_t* __restrict__ vc, bf16_t* __restrict__ out, int ldo,
@@ -701,7 +740,8 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill2(const bf16_t* __restri
     for (int g = 0; g < 2; ++g)
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) O[g][dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f};
+    AttnRow row[2];
+    const float sc2 = scale * 1.4426950408889634f;
     auto tile_math = [&](int tile, const bf16_t* img, auto masked_tag) {
         constexpr bool MASKED = decltype(masked_tag)::value;
         const int kb = tile * 32;
@@ -720,33 +760,9 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill2(const bf16_t* __restri
                 S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[c], qf[g][c], S0, 0, 0, 0);
                 S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[c], qf[g][c], S1, 0, 0, 0);
             }
-            float sc[8], mx = -INFINITY;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float v = (e < 4 ? S0[e] : S1[e - 4]) * scale;
-                if constexpr (MASKED) v = (kb + g4 * 8 + e < T) ? v : -INFINITY;
-                sc[e] = v;
-                mx = fmaxf(mx, v);
-            }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(m_run[g], mx);
-            const float alpha = __expf(m_run[g] - m_new);
-            float psum = 0.0f;
             bf16x8_t ph, pl;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float pe = __expf(sc[e] - m_new);
-                psum += pe;
-                const bf16_t hi = f32_to_bf16(pe);
-                const bf16_t lo = f32_to_bf16(pe - bf16_to_f32(hi));
-                ph[e] = (short)hi;
-                pl[e] = (short)lo;
-            }
-            l_run[g] = l_run[g] * alpha + psum;
-            const bool moved = m_new != m_run[g];
-            m_run[g] = m_new;
-            if (__any(moved)) {                              // (wave-uniform; alpha = exp(0) = 1 for every row otherwise)
+            float alpha = 1.0f;
+            if (attn_softmax_tile<MASKED>(S0, S1, kb + g4 * 8, T, sc2, row[g], ph, pl, alpha)) {
                 float ar[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, g4 * 4 + r, 64);
@@ -774,7 +790,7 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill2(const bf16_t* __restri
     }
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
-        float lr_all = l_run[g];
+        float lr_all = row[g].l;
         lr_all += __shfl_xor(lr_all, 16, 64);
         lr_all += __shfl_xor(lr_all, 32, 64);
         // O[g][dt][r]: row = query (g4*4 + r), col = d (dt*16 + j); the row's normaliser lives in lane (g4*4 + r)

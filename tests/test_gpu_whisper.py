@@ -435,3 +435,23 @@ def test_glue_folded_into_its_consumers_matches_the_separate_launches_and_the_or
             assert d_max <= 0.022 and d_rms <= 0.012, (name, d_max, d_rms)
     if strict:
         assert np.array_equal(got["default"], got["both"])                                        # (the default IS bits 2 and 4)
+
+
+def test_encoder_attention_when_the_maximum_moves_from_tile_to_tile():
+    """The softmax's reference maximum follows only scores that pass it by more than 2^8: query and key projections three times as large (scores
+    spread over +-40, the maximum of a row found late in the keys) against the oracle.  bf16 rounding of q and k moves a score s by up to
+    |s| 2^-8 <= 0.16, i.e. a probability by that share of itself: rms 0.05 instead of the 0.012 of flat scores."""
+    cfg = ow.WhisperConfig(vocab_size=700, num_mel_bins=80, d_model=128, encoder_layers=1, encoder_attention_heads=2, encoder_ffn_dim=256, decoder_layers=1,
+                           decoder_attention_heads=2, decoder_ffn_dim=256)
+    W = ow.make_synthetic_weights(cfg, seed=91)
+    for n in ("q_proj", "k_proj"):
+        k = f"model.encoder.layers.0.self_attn.{n}.weight"
+        W[k] = (W[k].float() * 3.0).to(W[k].dtype)
+    oracle, dev = ow.WhisperOracle(cfg, W, round="bf16"), mas.WhisperModel.from_weights(_host_cfg(cfg), W)
+    feats = _feats(2, cfg.num_mel_bins, 3)
+    feats *= np.linspace(0.2, 2.0, feats.shape[1], dtype=np.float32)[None, :, None]       # later frames are louder: larger scores at later keys
+    got = dev.encode(feats)
+    oracle.reset(2)
+    for g, r in zip(got, oracle.encode(feats)):
+        r = r.numpy()
+        assert np.isfinite(g).all() and np.sqrt(np.mean((g - r) ** 2)) <= 0.05 * np.sqrt(np.mean(r ** 2))
