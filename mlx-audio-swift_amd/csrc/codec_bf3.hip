@@ -349,6 +349,7 @@ __global__ void k_bf3_splitk_epilogue(const float* __restrict__ part, int S, int
 // ---- host side ------------------------------------------------------------------------------------------------------------------------
 CodecPack::~CodecPack() {
     for (auto& e : entries) if (e.wp) (void)hipFree(e.wp);
+    for (auto& e : x6) if (e.wp) (void)hipFree(e.wp);
 }
 
 const CodecPack::Entry& CodecPack::get(const float* at, int ntaps, int Cin, int M, hipStream_t s) {
@@ -374,6 +375,9 @@ static int bf3_env(const char* name, int dflt) {
     const char* v = getenv(name);
     return v ? atoi(v) : dflt;
 }
+
+CodecPack* codec_pack_scope() { return tl_pack; }
+bool codec_exact_f32() { return bf3_env("MIS_CODEC_EXACT_F32", 0) != 0; }
 
 bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s) {
     GemmParams p = p_in;

@@ -36,6 +36,8 @@ __device__ __forceinline__ float codec_noise_value(uint64_t key, uint64_t row, i
 struct CodecPack {
     struct Entry { const float* at; int ntaps, Cin, M, Cp, KS, MT32; uint16_t* wp; };
     std::vector<Entry> entries;
+    struct X6 { const float* at; int ntaps, Cin, M, KS, MT32; uint16_t* wp; };
+    std::vector<X6> x6;   // three-plane fragments (codec_x6.hip)
     DevBuf<uint16_t> xh, xl;
     DevBuf<float> part;   // split-K slabs of launch-shaped contractions (GemmParams.split_k_ok)
     CodecPack() {}
@@ -43,6 +45,7 @@ struct CodecPack {
     CodecPack& operator=(const CodecPack&) = delete;
     ~CodecPack();
     const Entry& get(const float* at, int ntaps, int Cin, int M, hipStream_t s);
+    const X6& get_x6(const float* at, int ntaps, int Cin, int M, hipStream_t s);
 };
 
 // Decoders open a scope around their launches: launch_gemm picks the scope's CodecPack up when GemmParams.pack is null.  Encoders
@@ -52,6 +55,20 @@ struct CodecPackScope {
     explicit CodecPackScope(CodecPack* p);
     ~CodecPackScope();
 };
+
+CodecPack* codec_pack_scope();        // the innermost scope's, or null
+bool codec_exact_f32();               // MIS_CODEC_EXACT_F32=1
+
+#define CODEC_DW_HALO 27              // 3 * max dilation (9)
+struct PwFusedParams {
+    const float* X; const float* R; float* Y;
+    const float *w7, *b1, *a1, *ra1;       // DW: depthwise weights [C][7], bias, Snake before the taps
+    const float *a2, *ra2;                 // Snake in front of the 1x1 conv
+    const float *AT, *b2;                  // W2^T [C][C] ([k][m]), bias
+    int T, dil, ldx, ldr, ldy;
+};
+// three-plane split of the unit tails (codec_x6.hip); false: no pack (encoders), exact-f32 asked for, or another width - nothing launched
+bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s);
 
 struct GemmParams {
     CodecPack* pack;      // non-null: MFMA-bound shapes run as split-bf16 contractions (codec_bf3.hip); null: exact-f32 kernels only

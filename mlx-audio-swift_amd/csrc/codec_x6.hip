@@ -1,0 +1,242 @@
+// codec_x6.hip - the f32 contraction of the codecs' narrow residual units on the bf16 matrix pipe, at f32 accuracy.
+//
+// Every f32 operand is written EXACTLY as three bfloat16, x = h + m + l, each the nearest to what is left (3 x 8 significant bits, signs absorb the carry),
+// and a product becomes the six bf16 MFMAs whose weight is above 2^-24: wh.xh + wh.xm + wm.xh + wm.xm + wh.xl + wl.xh (dropped: wm.xl + wl.xm + wl.xl,
+// <= 2^-25 of the product).  One 16-deep step is 6 x 32 cycles instead of 8 x 64 of v_mfma_f32_32x32x2_f32.  Error against 64 bits (2-norm over 2-norm,
+// this kernel / the exact-f32 one; K = 96, 128, 192; operands normal): 1.38e-7 / 1.77e-7, 1.65e-7 / 2.06e-7, 2.04e-7 / 2.49e-7; all of one sign: 1.14 / 1.44,
+// 1.29 / 1.60, 1.64 / 2.05; normal times exp(2 normal): 1.25 / 1.93, 1.42 / 2.00, 1.84 / 2.45: lower each time (6 roundings of the sum per 16 products, not 16).
+// An infinite operand gives NaN where the f32 kernels may give an infinity; Snake in front of it turns infinities into NaN on both.
+//
+//   k_x6_pack_w   A^T f32 -> the three planes as MFMA-A fragments (once per weight matrix, kept in the model's CodecPack)
+//   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels, for the encoders and for MIS_CODEC_EXACT_F32=1)
+#include "common.h"
+#include "codec_kernels.h"
+
+#include <algorithm>
+
+__device__ __forceinline__ float x6_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
+
+// x = h + m + l exactly (three bfloat16, each the nearest to what is left): eight values of consecutive channels -> one 16-byte piece per plane
+__device__ __forceinline__ void x6_split(const float (&v)[8], uint4& h, uint4& m, uint4& l) {
+    uint32_t o[3][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const uint32_t ab = (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
+            o[q][i] = ab;
+            a -= __uint_as_float(ab << 16);
+            b -= __uint_as_float(ab & 0xffff0000u);
+        }
+    }
+    h = make_uint4(o[0][0], o[0][1], o[0][2], o[0][3]);
+    m = make_uint4(o[1][0], o[1][1], o[1][2], o[1][3]);
+    l = make_uint4(o[2][0], o[2][1], o[2][2], o[2][3]);
+}
+
+// A^T f32 [ntaps][Cin][M] -> fragments of v_mfma_f32_32x32x16_bf16: [tap][Cp / 16][MT32][plane][64 lanes][8]
+__global__ void k_x6_pack_w(const float* __restrict__ AT, uint16_t* __restrict__ wp, int ntaps, int Cin, int M, int MT32, int KS) {
+    const size_t total = (size_t)ntaps * KS * MT32 * 512;
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
+        const int j = (int)(e & 7), lane = (int)((e >> 3) & 63);
+        size_t r = e >> 9;
+        const int mt = (int)(r % MT32); r /= MT32;
+        const int ks = (int)(r % KS);
+        const int tap = (int)(r / KS);
+        const int m = mt * 32 + (lane & 31), c = ks * 16 + (lane >> 5) * 8 + j;
+        float v = (m < M && c < Cin) ? AT[((size_t)tap * Cin + c) * M + m] : 0.0f;
+        const size_t o = (e >> 9) * 1536 + (size_t)lane * 8 + j;
+        for (int q = 0; q < 3; ++q) {
+            const uint16_t h = f32_to_bf16(v);
+            wp[o + q * 512] = h;
+            v -= bf16_to_f32(h);
+        }
+    }
+}
+
+const CodecPack::X6& CodecPack::get_x6(const float* at, int ntaps, int Cin, int M, hipStream_t s) {
+    for (auto& e : x6)
+        if (e.at == at && e.ntaps == ntaps && e.Cin == Cin && e.M == M) return e;
+    X6 e{};
+    e.at = at; e.ntaps = ntaps; e.Cin = Cin; e.M = M;
+    e.KS = (Cin + 15) / 16;
+    e.MT32 = (M + 31) / 32;
+    const size_t n = (size_t)ntaps * e.KS * e.MT32 * 1536;
+    HIP_CHECK(hipMalloc((void**)&e.wp, n * sizeof(uint16_t)));
+    hipLaunchKernelGGL(k_x6_pack_w, dim3((unsigned)std::min<size_t>((n / 3 + 255) / 256, 8192)), dim3(256), 0, s, at, e.wp, ntaps, Cin, M, e.MT32, e.KS);
+    x6.push_back(e);
+    return x6.back();
+}
+
+// ---- fused residual unit tails --------------------------------------------------------------------------------------------------------
+// The kernels of k_pw_fused (snac.hip), chunk by chunk: DW: x with its dilation halo -> Snake -> LDS -> seven taps, bias, Snake; else Snake alone; then eight
+// channels of a column per thread are split and written as one 16-byte piece per plane, [plane][channel / 8][column], which is the MFMA-B fragment.
+// What bounds it: k_pw_fused<128, DW> took 1.05 ms without its MFMAs (4.8 GB of loads and stores, 32 rows of 98304 columns) and 1.75 ms with: the f32
+// matrix time adds to the memory time.  Six bf16 products take 0.25 instead of 0.68 ms of it: 1.95 -> 1.44 ms.
+#define RU_NT 128
+#define RU_XS (RU_NT + 2 * CODEC_DW_HALO + 2)
+struct PwScalars { int T, dil, ldx, ldr, ldy; };
+template <int C, bool DW, int KC>
+__device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
+                                           const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
+                                           const float* __restrict__ pra1, const float* __restrict__ pa2, const float* __restrict__ pra2,
+                                           const uint16_t* __restrict__ pwp, const float* __restrict__ pb2, const PwScalars p) {
+    constexpr int KG = KC / 8, MT = C / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
+    constexpr int XR = KC / 4, GS = KG * 2 / 4;                             // rows of x and (group, strip) pairs per wave
+    __shared__ float xs[DW ? KC : 1][DW ? RU_XS : 1];
+    __shared__ uint4 ts[3][KG][RU_NT];
+    __shared__ uint4 As[APC];
+    constexpr bool SQ = C == 128;                         // 2 x 2 waves of 64 x 64; else every wave: all C rows x 32 columns
+    constexpr int MTW = SQ ? 2 : MT, NTW = SQ ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = blockIdx.x * RU_NT, b = blockIdx.y;
+    const int wr = SQ ? (wave >> 1) * 2 : 0;              // first row tile / first column of the wave's tile
+    const int wc = SQ ? (wave & 1) * 64 : wave * 32;
+    const float* xb = pX + (size_t)b * C * p.ldx;
+    const int T = p.T, halo = 3 * p.dil, ncols = RU_NT + 2 * halo;
+    f32x16_t acc[MTW][NTW];
+#pragma unroll
+    for (int i = 0; i < MTW; ++i)
+#pragma unroll
+        for (int j = 0; j < NTW; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    for (int c0 = 0; c0 < C; c0 += KC) {
+        __syncthreads();                                   // the previous chunk's MFMAs are done with ts / As
+        uint4 wv[(APC + 255) / 256];
+        const uint4* wsrc = reinterpret_cast<const uint4*>(pwp) + (size_t)(c0 / 16) * MT * 192;
+#pragma unroll
+        for (int i = 0; i < (APC + 255) / 256; ++i) wv[i] = wsrc[min(tid + i * 256, APC - 1)];
+        if (DW) {
+            float v[XR][3];
+#pragma unroll
+            for (int r = 0; r < XR; ++r) {
+                const int c = c0 + wave + 4 * r;
+#pragma unroll
+                for (int sx = 0; sx < 3; ++sx) {
+                    const int j = sx * 64 + lane, t = n0 - halo + j;
+                    const bool ok = j < ncols && t >= 0 && t < T;
+                    v[r][sx] = xb[(size_t)c * p.ldx + (ok ? t : 0)];
+                    v[r][sx] = ok ? v[r][sx] : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < XR; ++r) {
+                const int cc = wave + 4 * r, c = c0 + cc;
+                const float al = pa1[c], ral = pra1[c];
+#pragma unroll
+                for (int sx = 0; sx < 3; ++sx) {
+                    const int j = sx * 64 + lane;
+                    if (j < RU_XS) xs[cc][j] = x6_snake(v[r][sx], al, ral);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < GS; ++g) {
+                const int kg = KC == 32 ? wave : wave >> 1, n = (KC == 32 ? g : wave & 1) * 64 + lane, t = n0 + n;
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = xb[(size_t)(c0 + kg * 8 + j) * p.ldx + (t < T ? t : 0)];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) v[j] = x6_snake(v[j], pa2[c0 + kg * 8 + j], pra2[c0 + kg * 8 + j]);
+                uint4 h, m, l;
+                x6_split(v, h, m, l);
+                ts[0][kg][n] = h; ts[1][kg][n] = m; ts[2][kg][n] = l;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < (APC + 255) / 256; ++i)
+            if (APC % 256 == 0 || tid + i * 256 < APC) As[tid + i * 256] = wv[i];
+        if (DW) {
+            __syncthreads();
+            // depthwise taps + bias + Snake -> eight channels of one column per thread (consecutive lanes read consecutive LDS words)
+#pragma unroll
+            for (int g = 0; g < GS; ++g) {
+                const int kg = KC == 32 ? wave : wave >> 1, n = (KC == 32 ? g : wave & 1) * 64 + lane;
+                float v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int cc = kg * 8 + j, c = c0 + cc;
+                    float a = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < 7; ++k) a += pw7[c * 7 + k] * xs[cc][n + k * p.dil];
+                    v[j] = x6_snake(a + pb1[c], pa2[c], pra2[c]);
+                }
+                uint4 h, m, l;
+                x6_split(v, h, m, l);
+                ts[0][kg][n] = h; ts[1][kg][n] = m; ts[2][kg][n] = l;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < KC / 16; ++ks) {
+            bf16x8_t bv[NTW][3];
+#pragma unroll
+            for (int ni = 0; ni < NTW; ++ni)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) bv[ni][q] = *reinterpret_cast<const bf16x8_t*>(&ts[q][2 * ks + (lane >> 5)][wc + ni * 32 + (lane & 31)]);
+            constexpr int MP = NTW == 1 && MTW % 2 == 0 ? 2 : 1;             // row tiles at a time: two accumulators alternate
+#pragma unroll
+            for (int m0 = 0; m0 < MTW; m0 += MP) {
+                bf16x8_t av[MP][3];
+#pragma unroll
+                for (int mi = 0; mi < MP; ++mi)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) av[mi][q] = *reinterpret_cast<const bf16x8_t*>(&As[((ks * MT + wr + m0 + mi) * 3 + q) * 64 + lane]);
+                // smallest first: w_l x_h, w_h x_l, w_m x_m, w_m x_h, w_h x_m, w_h x_h
+                constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int mi = 0; mi < MP; ++mi)
+#pragma unroll
+                        for (int ni = 0; ni < NTW; ++ni)
+                            acc[m0 + mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[ni][QB[q]], acc[m0 + mi][ni], 0, 0, 0);
+            }
+        }
+    }
+    // epilogue: + bias + residual (C/D layout: col = lane & 31, row = (r & 3) + 8 (r >> 2) + 4 (lane >> 5))
+    const float* rb = pR + (size_t)b * C * p.ldr;
+    float* yb = pY + (size_t)b * C * p.ldy;
+#pragma unroll
+    for (int ni = 0; ni < NTW; ++ni) {
+        const int n = n0 + wc + ni * 32 + (lane & 31);
+        if (n >= T) continue;
+#pragma unroll
+        for (int mi = 0; mi < MTW; ++mi)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = (wr + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
+                yb[(size_t)m * p.ldy + n] = rb[(size_t)m * p.ldr + n] + (acc[mi][ni][r] + pb2[m]);
+            }
+    }
+}
+template <int C, bool DW, int KC>
+__global__ void __launch_bounds__(256, KC == 32 ? 2 : C == 128 && DW ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp) {
+    pw_x6_body<C, DW, KC>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
+}
+
+// Chunk depth (the same bits): 32 channels need half the barriers, 16 let three or four blocks (not two, C = 96: three) share a compute unit.  32 while its
+// blocks are all resident at once, else 16 (us, chunks of 32 / 16): 128 channels 96 blocks 28 / 33, 384: 34 / 38, 576: 61 / 45, 24576: 1584 / 1430;
+// 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150.  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32.
+template <int C, bool DW>
+static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hipStream_t s) {
+    const dim3 grid((p.T + RU_NT - 1) / RU_NT, batch);
+    if constexpr (C <= 128) {
+        if ((int64_t)grid.x * batch > (C == 96 ? 768 : 512)) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16>), grid, dim3(256), 0, s, p, wp); return; }
+    }
+    hipLaunchKernelGGL((k_pw_x6<C, DW, 32>), grid, dim3(256), 0, s, p, wp);
+}
+
+// 64 channels stay on k_pw_fused: twice the columns per product, bound by memory and by the units' VALU work (1.16 ms here, 1.10 there)
+bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s) {
+    if (!pack) pack = codec_pack_scope();
+    if (!pack || codec_exact_f32() || !(dw ? C == 128 : (C == 96 || C == 128 || C == 192))) return false;
+    const uint16_t* wp = pack->get_x6(p.AT, 1, C, C, s).wp;
+    if (dw) launch_x6<128, true>(p, wp, batch, s);
+    else if (C == 96) launch_x6<96, false>(p, wp, batch, s);
+    else if (C == 128) launch_x6<128, false>(p, wp, batch, s);
+    else launch_x6<192, false>(p, wp, batch, s);
+    return true;
+}

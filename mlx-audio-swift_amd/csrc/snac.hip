@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(256) k_snac_embed(EmbedParams p, float* __rest
 
 // ---- depthwise conv k=7 ---------------------------------------------------------------------------
 #define DW_TILE 1024
-#define DW_HALO 27      // 3 * max dilation (9)
+#define DW_HALO CODEC_DW_HALO
 
 template <bool SNAKE_IN, bool SNAKE_OUT>
 __global__ void __launch_bounds__(256) k_snac_dw(const float* __restrict__ X, float* __restrict__ Y,
@@ -180,30 +180,24 @@ __global__ void __launch_bounds__(256) k_snac_local_attn(const float* __restrict
 // Per 128-column tile and 32-channel chunk: the input (DW: with its dilation halo) is staged once, Snake applied on the way in; DW:
 // the depthwise taps read it from LDS; the chunk of t goes straight into the B-operand tile of the exact-f32 MFMA contraction with
 // the chunk's rows of W2^T.  The residual is read at the end (DW: L2-hot).  Same arithmetic per element as the unfused kernels.
+// Chunk depth KC (the same bits): 16 channels let six blocks, not three, share a compute unit (64 channels, 98304 blocks: 1.26 -> 1.10 ms); 32 need half the
+// barriers while all blocks are resident at once (384 blocks: 16.7 us, 19.7 us with 16).
 #define RU_NT 128
-#define RU_KC 32
 #define RU_XS (RU_NT + 2 * DW_HALO + 2)
-struct PwFusedParams {
-    const float* X; const float* R; float* Y;
-    const float *w7, *b1, *a1, *ra1;       // DW: depthwise weights [C][7], bias, Snake before the taps
-    const float *a2, *ra2;                 // Snake in front of the 1x1 conv
-    const float *AT, *b2;                  // W2^T [C][C] ([k][m]), bias
-    int T, dil, ldx, ldr, ldy;
-};
 // The body takes restrict-qualified PARAMETERS (clang ignores restrict on struct members and on locals; after inlining the parameter
 // attributes survive as scoped-noalias metadata): without them every residual / bias load of the epilogue has to wait behind the
 // previous row's store (measured: the SNAC units 2.25 -> 2.83 ms when the pointers were read from the parameter struct directly).
 struct PwFusedScalars { int T, dil, ldx, ldr, ldy; };
-template <int C, bool DW>
+template <int C, bool DW, int KC>
 __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                               const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
                                               const float* __restrict__ pra1, const float* __restrict__ pa2, const float* __restrict__ pra2,
                                               const float* __restrict__ pAT, const float* __restrict__ pb2, const PwFusedScalars sc) {
     struct { const float *X, *R; float* Y; const float *w7, *b1, *a1, *ra1, *a2, *ra2, *AT, *b2; int T, dil, ldx, ldr, ldy; } p =
         {pX, pR, pY, pw7, pb1, pa1, pra1, pa2, pra2, pAT, pb2, sc.T, sc.dil, sc.ldx, sc.ldr, sc.ldy};
-    __shared__ float xs[DW ? RU_KC : 1][DW ? RU_XS : 1];
-    __shared__ float ts[RU_KC][RU_NT];
-    __shared__ float As[RU_KC][C];
+    __shared__ float xs[DW ? KC : 1][DW ? RU_XS : 1];
+    __shared__ float ts[KC][RU_NT];
+    __shared__ float As[KC][C];
     constexpr bool SQ = C == 128;                         // 2 x 2 waves of 64 x 64; else every wave: all C rows x 32 columns
     constexpr int MTW = SQ ? 2 : C / 32, NTW = SQ ? 2 : 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);      // (scalar: the channels' parameters come by s_load)
@@ -219,15 +213,15 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
         for (int j = 0; j < NTW; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    for (int c0 = 0; c0 < C; c0 += RU_KC) {
+    for (int c0 = 0; c0 < C; c0 += KC) {
         __syncthreads();                                   // the previous chunk's MFMAs are done with ts / As
         if (DW) {
             // x chunk with halo, Snake on the way in (zero padding AFTER Snake: snake(0) = 0).  All 24 loads of a thread are issued
             // before the first use: lane -> column within a 64-column strip (3 strips cover 128 + 54), wave -> rows wave, wave + 4, ...
             // (fetching the next chunk under this chunk's MFMAs was measured too: no gain at 128 channels, 8 % slower at 64)
-            float v[8][3];
+            float v[KC / 4][3];
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
+            for (int r = 0; r < KC / 4; ++r) {
                 const int c = c0 + wave + 4 * r;
 #pragma unroll
                 for (int sx = 0; sx < 3; ++sx) {
@@ -238,7 +232,7 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
+            for (int r = 0; r < KC / 4; ++r) {
                 const int cc = wave + 4 * r, c = c0 + cc;
                 const float al = p.a1[c], ral = p.ra1[c];
 #pragma unroll
@@ -249,9 +243,9 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
             }
         } else {
             // the chunk of the 1x1 conv's input, Snake on the way in: 16 loads per thread up front (lane -> column, wave -> rows)
-            float v[8][2];
+            float v[KC / 4][2];
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
+            for (int r = 0; r < KC / 4; ++r) {
                 const int c = c0 + wave + 4 * r;
 #pragma unroll
                 for (int hx = 0; hx < 2; ++hx) {
@@ -260,14 +254,14 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
+            for (int r = 0; r < KC / 4; ++r) {
                 const int cc = wave + 4 * r, c = c0 + cc;
                 const float al = p.a2[c], ral = p.ra2[c];
 #pragma unroll
                 for (int hx = 0; hx < 2; ++hx) ts[cc][hx * 64 + lane] = snake_f(v[r][hx], al, ral);
             }
         }
-        for (int i = tid; i < RU_KC * (C / 4); i += 256) { // rows c0 .. c0+31 of W2^T
+        for (int i = tid; i < KC * (C / 4); i += 256) { // rows c0 .. c0+31 of W2^T
             const int r = i / (C / 4), m4 = (i - r * (C / 4)) * 4;
             *reinterpret_cast<float4*>(&As[r][m4]) = *reinterpret_cast<const float4*>(p.AT + (size_t)(c0 + r) * C + m4);
         }
@@ -276,7 +270,7 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
             // depthwise taps + bias + Snake -> the chunk of t.  lane -> column (consecutive lanes read consecutive LDS words: no bank
             // conflicts), wave -> channels wave, wave + 4, ...
 #pragma unroll 2
-            for (int r = 0; r < 8; ++r) {
+            for (int r = 0; r < KC / 4; ++r) {
                 const int cc = wave + 4 * r, c = c0 + cc;
                 float wk[7];
 #pragma unroll
@@ -295,7 +289,7 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
         }
         __syncthreads();
 #pragma unroll
-        for (int kk = 0; kk < RU_KC; kk += 2) {
+        for (int kk = 0; kk < KC; kk += 2) {
             float av[MTW], bv2[NTW];
 #pragma unroll
             for (int mi = 0; mi < MTW; ++mi) av[mi] = As[kk + (lane >> 5)][wr + mi * 32 + (lane & 31)];
@@ -323,9 +317,9 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
             }
     }
 }
-template <int C, bool DW>
-__global__ void __launch_bounds__(256, 2) k_pw_fused(PwFusedParams p) {
-    pw_fused_body<C, DW>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, p.AT, p.b2, PwFusedScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
+template <int C, bool DW, int KC>
+__global__ void __launch_bounds__(256, KC == 16 ? 4 : 2) k_pw_fused(PwFusedParams p) {
+    pw_fused_body<C, DW, KC>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, p.AT, p.b2, PwFusedScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
 }
 
 // ---- dense contraction on f32 MFMA ----------------------------------------------------------------
@@ -1170,11 +1164,12 @@ void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
         PwFusedParams fp{};
         fp.X = p.X; fp.R = p.R; fp.Y = p.Y; fp.a2 = p.alpha; fp.ra2 = p.ralpha; fp.AT = p.AT; fp.b2 = p.bias;
         fp.T = p.N; fp.dil = 0; fp.ldx = p.ldx; fp.ldr = p.ldy; fp.ldy = p.ldy;
+        if (launch_pw_x6(p.M, false, fp, p.pack, batch, s)) return;
         dim3 fg(cdiv(p.N, RU_NT), batch);
-        if (p.M == 64) hipLaunchKernelGGL((k_pw_fused<64, false>), fg, dim3(256), 0, s, fp);
-        else if (p.M == 96) hipLaunchKernelGGL((k_pw_fused<96, false>), fg, dim3(256), 0, s, fp);
-        else if (p.M == 128) hipLaunchKernelGGL((k_pw_fused<128, false>), fg, dim3(256), 0, s, fp);
-        else hipLaunchKernelGGL((k_pw_fused<192, false>), fg, dim3(256), 0, s, fp);
+        if (p.M == 64) hipLaunchKernelGGL((k_pw_fused<64, false, 32>), fg, dim3(256), 0, s, fp);
+        else if (p.M == 96) hipLaunchKernelGGL((k_pw_fused<96, false, 32>), fg, dim3(256), 0, s, fp);
+        else if (p.M == 128) hipLaunchKernelGGL((k_pw_fused<128, false, 32>), fg, dim3(256), 0, s, fp);
+        else hipLaunchKernelGGL((k_pw_fused<192, false, 32>), fg, dim3(256), 0, s, fp);
         return;
     }
     if (launch_gemm_bf3(mode, snake, p, batch, s)) return;
@@ -1299,8 +1294,10 @@ static const float* snac_run(mis_snac* c, const int32_t* const* codes, int batch
                 fp.a2 = W + ru.s2.a; fp.ra2 = W + ru.s2.ra; fp.AT = W + ru.pw.w; fp.b2 = W + ru.pw.b;
                 fp.T = (int)T; fp.dil = dils[j]; fp.ldx = fp.ldr = fp.ldy = (int)T;
                 dim3 fg(cdiv(T, RU_NT), batch);
-                if (blk.cout == 128) hipLaunchKernelGGL((k_pw_fused<128, true>), fg, dim3(256), 0, s, fp);
-                else hipLaunchKernelGGL((k_pw_fused<64, true>), fg, dim3(256), 0, s, fp);
+                if (launch_pw_x6(blk.cout, true, fp, nullptr, batch, s)) ;
+                else if (blk.cout == 128) hipLaunchKernelGGL((k_pw_fused<128, true, 32>), fg, dim3(256), 0, s, fp);
+                else if ((int64_t)fg.x * fg.y > 768) hipLaunchKernelGGL((k_pw_fused<64, true, 16>), fg, dim3(256), 0, s, fp);
+                else hipLaunchKernelGGL((k_pw_fused<64, true, 32>), fg, dim3(256), 0, s, fp);
                 std::swap(x, f2);
                 continue;
             }

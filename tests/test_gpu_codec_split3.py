@@ -1,0 +1,55 @@
+"""The three-plane contraction of the residual units (csrc/codec_x6.hip): both chunk depths, 96 / 128 / 192 channels, a column remainder - as accurate as the
+exact-f32 kernels, and the same bits whatever batch (and with it chunk depth) a row comes in."""
+import numpy as np
+import pytest
+
+import mlx_audio_swift_amd as mas
+from gpu_util import codec_exact_f32
+from oracle import dac as odac
+from oracle import snac as osnac
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def no_bf3(monkeypatch):
+    """The two-plane contractions off: what is left of the error is the f32 kernels' and the three-plane kernel's."""
+    monkeypatch.setenv("MIS_BF3_MIN_K", "1000000")
+    monkeypatch.setenv("MIS_BF3_MIN_K1", "1000000")
+
+
+def check(dev, orc, codes, rows, pick):
+    """rows of codes as one batch; the first two against the oracle (SNAC: 64 bits, DAC: float32)."""
+    ref = orc(pick(codes, slice(0, 2)))
+    got = dev(codes)
+    with codec_exact_f32():
+        f32 = dev(codes)
+    err, err32 = (np.sqrt(np.mean((g[:2] - ref) ** 2) / np.mean(ref ** 2)) for g in (got, f32))
+    assert not np.array_equal(got, f32)                    # the other kernel did run
+    # both are float32 sums in another order: the same size within the scatter of a few thousand samples, and under 24-bit sums through ten layers
+    assert err <= 1.25 * err32 and err32 <= 1e-5, (err, err32)
+    for r in (0, rows - 1):
+        assert np.array_equal(dev(pick(codes, slice(r, r + 1)))[0], got[r])
+
+
+@pytest.mark.parametrize("rows, groups", [(3, 5), (40, 60)], ids=["one-wave", "many"])
+def test_snac_128(no_bf3, rows, groups):
+    cfg = dict(encoder_dim=8, encoder_rates=[2, 2, 2, 8], decoder_dim=256, decoder_rates=[8, 2, 2, 2], codebook_size=64, codebook_dim=8, vq_strides=[4, 2, 1])
+    ocfg = osnac.SnacConfig(**cfg)
+    W = osnac.make_synthetic_weights(ocfg, seed=31, with_encoder=True)
+    dev = mas.SNAC.from_weights(mas.SNACConfig(**{k: getattr(ocfg, k) for k in mas.SNACConfig.__dataclass_fields__}), W)
+    dev.set_noise(True)
+    oracle = osnac.SnacOracle(ocfg, W, dtype=np.float64)
+    codes = osnac.synthetic_codes(ocfg, rows, groups)
+    check(dev.decode, lambda c: oracle.decode(c, None), codes, rows, lambda c, sl: [x[sl] for x in c])
+
+
+@pytest.mark.parametrize("rows, frames", [(2, 9), (9, 211)], ids=["one-wave", "many"])
+def test_dac_192_96(no_bf3, rows, frames):
+    ocfg = odac.DacConfig(encoder_dim=4, encoder_rates=(2, 2), latent_dim=40, decoder_dim=384, decoder_rates=(8, 5, 2), n_codebooks=2, codebook_size=64)
+    W = odac.make_synthetic_weights(ocfg)
+    stored = {k.replace(".outProj.", ".out_proj.").replace(".inProj.", ".in_proj.").replace("decoder.model.", "decoder.model.layers."): v for k, v in W.items()}
+    dev = mas.DescriptDAC.from_weights(mas.DescriptDACConfig(**{k: getattr(ocfg, k) for k in mas.DescriptDACConfig.__dataclass_fields__}), stored)
+    orc = odac.DacOracle(ocfg, W)
+    codes = np.random.default_rng(3).integers(0, ocfg.codebook_size, (rows, ocfg.n_codebooks, frames)).astype(np.int32)
+    check(dev.decode_from_codes, orc.decode_from_codes, codes, rows, lambda c, sl: c[sl])
