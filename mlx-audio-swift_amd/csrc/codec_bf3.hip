@@ -64,30 +64,48 @@ __global__ void k_bf3_pack_w(const float* __restrict__ AT, uint16_t* __restrict_
 }
 
 // ---- activations: x f32 [B][C][ldx] -> planes [B][Tp][Cp] (column t' holds input column t' + t_org; zero outside [x_lo, Tin)) ---------
-// Block: 64 columns x SP_CB channels.  Loads are coalesced along time (a wave reads 64 consecutive columns of one channel), the split
-// halves go through an LDS transpose, stores are coalesced along channels (16-byte pieces, a full SP_CB-channel row per 16 threads)
+// Block: 64 columns x SP_CB channels.  A wave reads 64 consecutive columns of eight channels at a time (all its 32 loads are requested before the first use:
+// one memory round trip), splits them and writes one 16-byte piece per plane to LDS; stores are coalesced along channels (16-byte pieces, a full
+// SP_CB-channel row per 16 threads).  Channel by channel under its guard it was 32 round trips of latency: 663 -> 297 us for 32 x 98304 columns of 256 channels
+// (1.6 GB: 5.4 TB/s), 17.9 -> 9.2 us for 2080 columns of 768
 #define SP_CB 128
-#define SP_LD (SP_CB + 8)             // LDS row stride in bf16 (272 B: 16-byte aligned rows; the 2-byte transposing writes of a wave hit
-                                      // rows 68 dwords apart: 4 | 68 only by 4, so the 64 lanes spread over 16 banks x 2 ways at worst)
+#define SP_LD (SP_CB + 8)             // LDS row stride in bf16 (272 B: 16-byte aligned rows, 4 banks apart: eight lanes' 16-byte writes cover 32 banks)
 __global__ void __launch_bounds__(256) k_bf3_split(const float* __restrict__ X, uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
                                                    const float* __restrict__ alpha, const float* __restrict__ ralpha,
                                                    int C, int ldx, int x_lo, int Tin, int Cp, int Tp, int t_org) {
     __shared__ __attribute__((aligned(16))) uint16_t sh[64 * SP_LD], sl[64 * SP_LD];
-    const int tl = threadIdx.x & 63, cg = threadIdx.x >> 6;
+    const int tl = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);       // (scalar: the channels' parameters come by s_load)
     const int tp0 = blockIdx.x * 64, c0 = blockIdx.y * SP_CB, b = blockIdx.z;
     const int cw = min(SP_CB, Cp - c0);                         // channels of this block (multiple of 32)
     const int t = tp0 + tl + t_org;
     const bool tin = tp0 + tl < Tp && t >= x_lo && t < Tin;
-    for (int cc = cg; cc < cw; cc += 4) {
-        const int c = c0 + cc;
-        float x = 0.0f;
-        if (tin && c < C) {
-            x = X[((int64_t)b * C + c) * ldx + t];
-            if (alpha) x = bf3_snake(x, alpha[c], ralpha[c]);
+    const float* xb = X + (int64_t)b * C * ldx + (tin ? t : 0);
+    constexpr int NO = SP_CB / 32;                              // octets of channels per wave
+    float v[NO][8];
+#pragma unroll
+    for (int o = 0; o < NO; ++o)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[o][j] = xb[(int64_t)min(c0 + (wave + 4 * o) * 8 + j, C - 1) * ldx];
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+        const int cc = (wave + 4 * o) * 8;
+        if (cc >= cw) continue;
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            float x[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int c = c0 + cc + j + i;
+                x[i] = v[o][j + i];
+                if (alpha) x[i] = bf3_snake(x[i], alpha[min(c, C - 1)], ralpha[min(c, C - 1)]);
+                x[i] = tin && c < C ? x[i] : 0.0f;
+            }
+            h[j / 2] = (uint32_t)f32_to_bf16(x[0]) | ((uint32_t)f32_to_bf16(x[1]) << 16);
+            l[j / 2] = (uint32_t)f32_to_bf16(x[0] - __uint_as_float(h[j / 2] << 16)) | ((uint32_t)f32_to_bf16(x[1] - __uint_as_float(h[j / 2] & 0xffff0000u)) << 16);
         }
-        const uint16_t h = f32_to_bf16(x);
-        sh[tl * SP_LD + cc] = h;
-        sl[tl * SP_LD + cc] = f32_to_bf16(x - bf16_to_f32(h));
+        *reinterpret_cast<uint4*>(sh + tl * SP_LD + cc) = make_uint4(h[0], h[1], h[2], h[3]);
+        *reinterpret_cast<uint4*>(sl + tl * SP_LD + cc) = make_uint4(l[0], l[1], l[2], l[3]);
     }
     __syncthreads();
     const int pieces = cw / 8;                                  // 16-byte pieces per row
