@@ -54,36 +54,10 @@ struct mis_dac {
     DevBuf<int32_t> enc_codes;
 };
 
-__global__ void k_dac_embed(const int32_t* __restrict__ codes, const float* __restrict__ tables, float* __restrict__ z, int ncb, int bins,
-                            int C, int T) {
-    const int t = blockIdx.x, b = blockIdx.y;
-    for (int c = threadIdx.x; c < C; c += blockDim.x) {
-        float acc = 0.0f;
-        for (int q = 0; q < ncb; ++q) {
-            int code = min(max(codes[((size_t)b * ncb + q) * T + t], 0), bins - 1);
-            acc += tables[((size_t)q * bins + code) * C + c];
-        }
-        z[((size_t)b * C + c) * T + t] = acc;
-    }
-}
-
-// Snake -> conv k7 "same" (C -> 1) -> tanh   (DescriptDAC.swift:146-148)
-__global__ void k_dac_final(const float* __restrict__ x, float* __restrict__ out, int64_t out_stride, const float* __restrict__ w /*[7][C]*/,
-                            float bias, const float* __restrict__ a, const float* __restrict__ ra, int C, int T) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
-    if (t >= T) return;
-    float acc = bias;
-    for (int c = 0; c < C; ++c) {
-        const float* xr = x + ((size_t)b * C + c) * T;
-        const float ac = a[c], rc = ra[c];
-        for (int j = 0; j < 7; ++j) {
-            int ts = t + j - 3;
-            if (ts < 0 || ts >= T) continue;
-            const float v = xr[ts];
-            acc += w[j * C + c] * fmaf(rc, mis_sin_sq(ac * v), v);
-        }
-    }
-    out[(size_t)b * out_stride + t] = tanhf(acc);
+__global__ void __launch_bounds__(256) k_dac_embed(const int32_t* __restrict__ codes, const float* __restrict__ tables, float* __restrict__ z, int ncb, int bins,
+                                                   int C, int T) {
+    const int b = blockIdx.z;
+    codec_embed(tables, ncb, bins, C, T, z + (size_t)b * C * T, [&](int q, int t) { return codes[((size_t)b * ncb + q) * T + t]; });
 }
 
 extern "C" mis_status mis_dac_create(const mis_dac_config* cfg, int device, mis_dac** out) {
@@ -419,7 +393,7 @@ static const float* dac_run(mis_dac* c, const int32_t* codes_dev, int batch, int
         g.AT = W + L.w; g.bias = W + L.b; g.X = X; g.Y = Y; g.M = L.M; g.K = L.K; g.N = N; g.Tin = Tin; g.Tout = Tout;
         return g;
     };
-    hipLaunchKernelGGL(k_dac_embed, dim3(T, batch), dim3(256), 0, s, codes_dev, W + c->tables, x, cf.n_codebooks, cf.codebook_size, c->latent, T);
+    hipLaunchKernelGGL(k_dac_embed, dim3(cdiv(T, 32), cdiv(c->latent, 32), batch), dim3(256), 0, s, codes_dev, W + c->tables, x, cf.n_codebooks, cf.codebook_size, c->latent, T);
     {
         GemmParams g = gp(c->first, x, y, T, T, T);
         g.Cin = c->latent; g.taps = 7; g.dil = 1; g.pad = 3;
@@ -448,8 +422,8 @@ static const float* dac_run(mis_dac* c, const int32_t* codes_dev, int batch, int
         if (stage == 1 + bi) { *outC = B.cout; *outT = Tc; return x; }
         ++bi;
     }
-    hipLaunchKernelGGL(k_dac_final, dim3(cdiv(Tc, 128), batch), dim3(128), 0, s, x, wav_dev, wav_stride, W + c->fin_w, c->fin_b, W + c->fin_a,
-                       W + c->fin_ra, c->fin_c, (int)Tc);
+    // DescriptDAC.swift:146-148
+    launch_codec_final(x, wav_dev, wav_stride, W + c->fin_w, 1, c->fin_c, c->fin_b, W + c->fin_a, W + c->fin_ra, batch, c->fin_c, (int)Tc, s);
     HIP_CHECK(hipGetLastError());
     *outC = 1; *outT = Tc;
     return wav_dev;

@@ -10,7 +10,7 @@
 //   k_snac_embed   z_q = sum_i table_i[codes_i[b, t/stride_i]]       (table_i = codebook_i x out_proj_i + b_i)
 //   k_snac_dw      depthwise k=7 dilated conv with optional Snake before/after, LDS halo tile
 //   k_snac_convt   Snake -> transposed conv on v_mfma_f32_32x32x2_f32 (1x1 convs, NoiseBlock, strided convs: codec_f32.hip)
-//   k_snac_final   Snake -> conv k7 (C -> 1) -> tanh
+//   k_codec_final  Snake -> conv k7 (C -> 1) -> tanh
 #include "common.h"
 #include "kernels.h"
 #include "codec_kernels.h"
@@ -33,32 +33,12 @@ struct EmbedParams {
     int n_q, codebook_size, C, T0;
 };
 
-// block: 32 channels x 32 frames, 256 threads; LDS transpose so that table reads are coalesced over
-// c and z_q writes are coalesced over t.
+// (0 + z0) + z1 + z2 : VQ.swift:186 order
 __global__ void __launch_bounds__(256) k_snac_embed(EmbedParams p, float* __restrict__ zq) {
-    __shared__ float tile[32][33];
-    int b = blockIdx.z, c0 = blockIdx.y * 32, t0 = blockIdx.x * 32;
-    int tid = threadIdx.x;
-    int cc = tid & 31;
-    for (int tt = tid >> 5; tt < 32; tt += 8) {
-        int t = t0 + tt, c = c0 + cc;
-        float acc = 0.0f;
-        if (t < p.T0 && c < p.C) {
-            for (int i = 0; i < p.n_q; ++i) {          // (0 + z0) + z1 + z2 : VQ.swift:186 order
-                int Ti = p.T0 / p.strides[i];
-                int code = p.codes[i][(size_t)b * Ti + t / p.strides[i]];
-                code = code < 0 ? 0 : (code >= p.codebook_size ? p.codebook_size - 1 : code);
-                acc += p.tables[((size_t)i * p.codebook_size + code) * p.C + c];
-            }
-        }
-        tile[cc][tt] = acc;
-    }
-    __syncthreads();
-    int tt = tid & 31;
-    for (int c2 = tid >> 5; c2 < 32; c2 += 8) {
-        int t = t0 + tt, c = c0 + c2;
-        if (t < p.T0 && c < p.C) zq[((size_t)b * p.C + c) * p.T0 + t] = tile[c2][tt];
-    }
+    const int b = blockIdx.z;
+    codec_embed(p.tables, p.n_q, p.codebook_size, p.C, p.T0, zq + (size_t)b * p.C * p.T0, [&](int q, int t) {
+        return p.codes[q][(size_t)b * (p.T0 / p.strides[q]) + t / p.strides[q]];
+    });
 }
 
 // ---- depthwise conv k=7 ---------------------------------------------------------------------------
@@ -616,34 +596,65 @@ template <bool RESID>
 __global__ void __launch_bounds__(256) k_conv_taps(GemmParams p) { conv_taps_body<RESID>(p, p.X, p.R, p.Y, p.bias, p.scale); }
 
 // ---- final Snake -> conv k7 (C -> 1) -> tanh ----------------------------------------------------------
-#define FIN_TILE 256
-#define FIN_CH 16
-__global__ void __launch_bounds__(256) k_snac_final(const float* __restrict__ X, float* __restrict__ out,
-                                                    int64_t out_stride, const float* __restrict__ w /*[C][7]*/,
-                                                    float bias, const float* __restrict__ alpha,
-                                                    const float* __restrict__ ralpha, int C, int T) {
-    __shared__ float s[FIN_CH][FIN_TILE + 8];
-    int b = blockIdx.y, t0 = blockIdx.x * FIN_TILE, tid = threadIdx.x;
-    float acc = 0.0f;
-    for (int c0 = 0; c0 < C; c0 += FIN_CH) {
-        __syncthreads();
-        for (int i = tid; i < FIN_CH * (FIN_TILE + 6); i += 256) {
-            int cc = i / (FIN_TILE + 6), j = i % (FIN_TILE + 6);
-            int c = c0 + cc, t = t0 - 3 + j;
-            float v = 0.0f;
-            if (c < C && t >= 0 && t < T) v = snake_f(X[((size_t)b * C + c) * T + t], alpha[c], ralpha[c]);
-            s[cc][j] = v;
-        }
-        __syncthreads();
-        int cmax = min(FIN_CH, C - c0);
-        for (int cc = 0; cc < cmax; ++cc) {
-            const float* wc = w + (size_t)(c0 + cc) * 7;
+// Wave w takes channels w, w + 4, ..., eight at a time with their loads in one round trip, for 122 outputs: two strips of 64 columns, three of them halo on
+// each side; Snake once per element into LDS of its own (no barrier), taps from there; the four waves' sums are added at the end.  Bound: one pass over X
+// (1.6 GB for 32 rows of 196608 columns of 64 channels: 700 -> 457 us) and 21 VALU instructions per element; one row of 24576: 36.7 -> 11.5 us, 80043 columns
+// of 96 channels (DAC, Snake seven times per element before): 143 -> 19.5 us.  Weights at w[c cs + k ks].
+#define FIN_OUT 122
+#define FIN_CH 8
+__global__ void __launch_bounds__(256) k_codec_final(const float* __restrict__ X, float* __restrict__ out, int64_t out_stride, const float* __restrict__ w, int cs, int ks,
+                                                     float bias, const float* __restrict__ alpha, const float* __restrict__ ralpha, int C, int T) {
+    __shared__ float s[4][FIN_CH][128];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.y, t0 = blockIdx.x * FIN_OUT;
+    const float* xb = X + (size_t)b * C * T;
+    int tc[2];
+    bool ok[2];
 #pragma unroll
-            for (int k = 0; k < 7; ++k) acc += wc[k] * s[cc][tid + k];
-        }
+    for (int h = 0; h < 2; ++h) {
+        const int t = t0 - 3 + h * 64 + lane;
+        ok[h] = t >= 0 && t < T;
+        tc[h] = min(max(t, 0), T - 1);
     }
-    int t = t0 + tid;
-    if (t < T) out[(size_t)b * out_stride + t] = tanhf(acc + bias);
+    float v[FIN_CH][2], acc[2] = {0.0f, 0.0f};
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int i = 0; i < FIN_CH; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[i][h] = xb[(size_t)min(c0 + 4 * i, C - 1) * T + tc[h]];
+    };
+    load(wave);
+    for (int c0 = wave; c0 < C; c0 += 4 * FIN_CH) {
+#pragma unroll
+        for (int i = 0; i < FIN_CH; ++i) {
+            const int c = min(c0 + 4 * i, C - 1);
+            const float a = alpha[c], ra = ralpha[c];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) s[wave][i][h * 64 + lane] = ok[h] ? snake_f(v[i][h], a, ra) : 0.0f;
+        }
+        if (c0 + 4 * FIN_CH < C) load(c0 + 4 * FIN_CH);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < FIN_CH; ++i) {
+            if (c0 + 4 * i >= C) break;
+#pragma unroll
+            for (int k = 0; k < 7; ++k) {
+                const float wk = w[(size_t)(c0 + 4 * i) * cs + k * ks];
+                acc[0] += wk * s[wave][i][lane + k];
+                acc[1] += wk * s[wave][i][min(64 + lane + k, 127)];                  // (lanes 58 .. 63 of the second strip are halo)
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    s[wave][0][lane] = acc[0];
+    s[wave][0][64 + lane] = acc[1];
+    __syncthreads();
+    const int j = threadIdx.x, t = t0 + j;
+    if (j < FIN_OUT && t < T) out[(size_t)b * out_stride + t] = tanhf(((s[0][0][j] + s[1][0][j]) + (s[2][0][j] + s[3][0][j])) + bias);
+}
+void launch_codec_final(const float* X, float* out, int64_t out_stride, const float* w, int cs, int ks, float bias, const float* alpha, const float* ralpha, int batch, int C, int T,
+                        hipStream_t s) {
+    hipLaunchKernelGGL(k_codec_final, dim3((T + FIN_OUT - 1) / FIN_OUT, batch), dim3(256), 0, s, X, out, out_stride, w, cs, ks, bias, alpha, ralpha, C, T);
 }
 
 // ============================================================================ host side
@@ -1314,8 +1325,7 @@ static const float* snac_run(mis_snac* c, const int32_t* const* codes, int batch
     }
     MIS_REQUIRE(T == Tfinal, MIS_ERR_AUDIO_DECODE, "internal length mismatch");
     int cl = cf.decoder_dim >> cf.n_decoder_rates;
-    hipLaunchKernelGGL(k_snac_final, dim3(cdiv(T, FIN_TILE), batch), dim3(256), 0, s, x, pcm, pcm_stride,
-                       W + c->fin.w, c->fin_bias, W + c->fin_snake.a, W + c->fin_snake.ra, cl, (int)T);
+    launch_codec_final(x, pcm, pcm_stride, W + c->fin.w, 7, 1, c->fin_bias, W + c->fin_snake.a, W + c->fin_snake.ra, batch, cl, (int)T, s);
     *outC = 1; *outT = T;
     return pcm;
 }
