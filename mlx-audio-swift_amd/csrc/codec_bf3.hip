@@ -14,17 +14,16 @@
 //   k_bf3_split    activation pre-pass: (Snake) -> split -> transpose to time-major planes xh, xl [B][Tp][Cp] with zero pads, so that a
 //                  B fragment (8 consecutive channels of one time column) is one aligned 16-byte piece; Snake runs ONCE per element
 //                  (the staged f32 kernels re-run it per 64-row block and per transposed-conv phase)
-//   k_bf3_gemm     128 x 128 output tile per block: 4 MFMA waves (64 x 64 each) + 1 loader wave.  The loader streams the activation
+//   k_bf3_gemm     128 x 128 output tile per block (64 x 128 or 64 x 64 where that gives few blocks): 4 MFMA waves (64 x 64 each) + 1 loader wave.  The loader streams the activation
 //                  tile (with its tap halo) by LDS-DMA into an NBUF-deep ring, chunk = 32 channels, running NBUF-1 chunks ahead on its
 //                  OWN vmcnt counter; the MFMA waves take the packed weight fragments straight from L2 into registers (prefetched two
-//                  steps ahead) and the activation fragments from LDS (XOR-swizzled at the DMA source, conflict-free ds_read_b128).
+//                  to seven steps ahead) and the activation fragments from LDS (XOR-swizzled at the DMA source, conflict-free ds_read_b128).
 //                  One s_barrier per chunk.  Taps (dense k-tap convs), transposed-conv phases and 1x1 convs share the tile code:
 //                  tap j reads the staged tile at a column offset.
 #include "common.h"
 #include "codec_kernels.h"
 
 #define B3_BM 128
-#define B3_BN 128
 #define B3_KC 32
 #define B3_THREADS 320
 
@@ -37,9 +36,10 @@ struct Bf3Params {
     const uint16_t* xh;
     const uint16_t* xl;
     int mode, ntaps, MT32, KS, Cp, Tp, t_org;
-    int ksplit;           // > 1: blockIdx.z = batch row x slice; the block contracts chunks [nchunks slice / ksplit, nchunks (slice + 1) / ksplit)
+    int ksplit;           // > 1: a tile has that many blocks; a block contracts chunks [nchunks slice / ksplit, nchunks (slice + 1) / ksplit)
     float* part;          //      and writes its raw float32 sums to part[slice][b][M][ldy] (k_bf3_splitk_epilogue finishes)
     int batch;
+    int nbx, my, inner, per, tiles;       // column tiles, row tiles, phases or K slices of a tile, tiles per XCD, all tiles
 };
 
 __device__ __forceinline__ float bf3_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
@@ -119,36 +119,47 @@ __global__ void __launch_bounds__(256) k_bf3_split(const float* __restrict__ X, 
 }
 
 // ---- the contraction -----------------------------------------------------------------------------------------------------------------
-struct Bf3A { bf16x8_t v[2][2]; };     // [m tile][hi, lo]
-struct Bf3B { bf16x8_t v[2][2]; };     // [n tile][hi, lo]
+template <int MI> struct Bf3A { bf16x8_t v[MI][2]; };     // [m tile][hi, lo]
+template <int NI> struct Bf3B { bf16x8_t v[NI][2]; };     // [n tile][hi, lo]
 
 // sched_group_barrier masks: 0x008 MFMA, 0x002 VALU, 0x020 VMEM read, 0x100 DS read
 #define B3_IL_V __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x002, 3, 0); __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
 #define B3_IL_D __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x002, 3, 0); __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
 #define B3_IL_M __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-#define B3_INTERLEAVE B3_IL_V B3_IL_V B3_IL_V B3_IL_V B3_IL_D B3_IL_D B3_IL_D B3_IL_D B3_IL_M B3_IL_M B3_IL_M B3_IL_M
+#define B3_INTERLEAVE_22 B3_IL_V B3_IL_V B3_IL_V B3_IL_V B3_IL_D B3_IL_D B3_IL_D B3_IL_D B3_IL_M B3_IL_M B3_IL_M B3_IL_M
+#define B3_INTERLEAVE_12 B3_IL_V B3_IL_V B3_IL_D B3_IL_D B3_IL_D B3_IL_D
+#define B3_INTERLEAVE_11 B3_IL_V B3_IL_V B3_IL_D
 
 // The body takes the arrays the epilogue touches as restrict-qualified PARAMETERS: GemmParams is a struct, clang ignores restrict on
 // struct members, and without it every bias / residual load of the epilogue waits behind the previous row's store (the same effect
 // cost the fused unit kernel of snac.hip 25 %).
-template <int NQ, int NBUF, int NTAPS>
+template <int MI, int NI, int NQ, int NBUF, int NTAPS, int AR>
 __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                          const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise) {
     constexpr int PLANE = NQ * 512;                       // bf16 per plane: NQ DMA instructions of 1 KiB (16 columns x 32 channels)
     constexpr int BUF = 2 * PLANE;
     constexpr int NST = 2 * NTAPS;                        // MFMA steps (16 channels of one tap) per chunk
+    constexpr int CG = NST % AR == 0 ? 1 : (2 * NST) % AR == 0 ? 2 : (3 * NST) % AR == 0 ? 3 : 4;      // chunks per straight-line group: whole turns of the weight ring
+    static_assert(CG * NST % AR == 0 && CG * NST % 2 == 0, "registers rotate in whole turns");
+    constexpr int BN = 64 * NI;
     __shared__ __attribute__((aligned(1024))) uint16_t lds[NBUF * BUF];
     const GemmParams& p = P.g;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int b = blockIdx.z, phase = 0, sh0 = 0, dsh = 0, tapbase = 0, slice = 0;
-    if (P.mode == GEMM_CONVT) { b = blockIdx.z / p.s; phase = blockIdx.z - b * p.s; sh0 = (phase + p.pad) / p.s; dsh = -1; tapbase = phase * NTAPS; }
+    // blocks are dealt to the XCDs by id mod 8: an XCD takes a contiguous range of tiles, all row tiles of a column tile in a row and all phases of a tile in
+    // a row, so that its L2 holds their activation tile and merges the phases' interleaved stores (M = 128, K = 2 x 256, 4 phases, 32 x 24576 columns: 2.03 ->
+    // 1.68 ms; where the phases' weights, 34 MB for M = 512, K = 2 x 1024, 8 phases, are more than it holds: 0.57 -> 0.60, 0.80 with the phases outside)
+    const int xi = blockIdx.x >> 3, in = xi % P.inner, tileid = (blockIdx.x & 7) * P.per + xi / P.inner;
+    if (tileid >= P.tiles) return;
+    const int by = tileid % P.my, bxb = tileid / P.my, bx = bxb % P.nbx, b = bxb / P.nbx;
+    int phase = 0, sh0 = 0, dsh = 0, tapbase = 0, slice = 0;
+    if (P.mode == GEMM_CONVT) { phase = in; sh0 = (phase + p.pad) / p.s; dsh = -1; tapbase = phase * NTAPS; }
     else if (P.mode == GEMM_TAPS) { sh0 = -p.pad; dsh = p.dil; }
-    else if (P.ksplit > 1) { b = blockIdx.z / P.ksplit; slice = blockIdx.z - b * P.ksplit; }
+    else if (P.ksplit > 1) slice = in;
     const int shmin = min(sh0, sh0 + (NTAPS - 1) * dsh);
     const int nchunks_all = P.Cp / B3_KC;
     const int c_lo = P.ksplit > 1 ? nchunks_all * slice / P.ksplit : 0;                        // this block's chunks (split-K: a slice of them)
     const int nchunks = (P.ksplit > 1 ? nchunks_all * (slice + 1) / P.ksplit : nchunks_all) - c_lo;
-    const int n0 = blockIdx.x * B3_BN;
+    const int n0 = bx * BN;
 
     if (wave == 4) {
         // ---- loader: tile column i = input column n0 + shmin + i.  DMA instruction q moves columns 16q .. 16q+15, four lanes per column;
@@ -179,58 +190,59 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
         return;
     }
 
-    // ---- MFMA waves: 2 x 2, wave tile 64 rows x 64 columns = 2 x 2 tiles of 32 x 32
+    // ---- MFMA waves: 2 x 2, wave tile MI x NI tiles of 32 x 32
     const int wm = wave >> 1, wn = wave & 1;
-    const int mt0 = blockIdx.y * 4 + wm * 2;
+    const int mt0 = (by * 2 + wm) * MI;
     if (mt0 >= P.MT32) {                                   // no rows for this wave (M <= 64 in this block row): keep the barrier count
         for (int cc = 0; cc < nchunks; ++cc) __builtin_amdgcn_s_barrier();
         return;
     }
-    f32x16_t acc[2][2];
+    f32x16_t acc[MI][NI];
 
-    // weight stream: step (chunk, tap, ks) -> fragments of both row tiles, hi and lo.  It runs two steps ahead of the MFMAs, across
+    // weight stream: step (chunk, tap, ks) -> fragments of the row tiles, hi and lo.  It runs AR - 1 steps ahead of the MFMAs, across
     // chunk boundaries (it does not depend on the staged tile).  A second row tile past M re-reads the first (its rows are
-    // never stored).  The body below is three chunks (3 * NST steps) of straight-line code: the weight registers rotate with period 3,
+    // never stored).  The body below is CG chunks (CG * NST steps) of straight-line code: the weight registers rotate with period AR,
     // the tile-fragment registers with period 2, every index is a compile-time constant and there is no branch between the MFMAs,
-    // so the waitcnt pass keeps exactly the two younger weight loads in flight (with branches in the body it fell back to vmcnt(0)).
+    // so the waitcnt pass keeps exactly the AR - 2 younger weight loads in flight (with branches in the body it fell back to vmcnt(0)).
     const size_t tap_stride = (size_t)P.MT32 * P.KS * 1024, mt_stride = (size_t)P.KS * 1024;
     const uint16_t* wbase = P.wp + (size_t)lane * 8 + (size_t)tapbase * tap_stride + (size_t)mt0 * mt_stride + (size_t)c_lo * 2 * 1024;
     const size_t mt1 = (mt0 + 1 < P.MT32) ? mt_stride : 0;
-    const int ncol = wn * 64 + (lane & 31), kgrp = lane >> 5;
-    Bf3A aq[3];
-    Bf3B bq[2];
-    auto loadA = [&](Bf3A& f, int chunk, int tap, int ks) {
+    const int ncol = wn * 32 * NI + (lane & 31), kgrp = lane >> 5;
+    Bf3A<MI> aq[AR];
+    Bf3B<NI> bq[2];
+    auto loadA = [&](Bf3A<MI>& f, int chunk, int tap, int ks) {
         chunk = min(chunk, nchunks - 1);                     // the last steps prefetch past the end: re-read the last chunk
         const uint16_t* q = wbase + (size_t)tap * tap_stride + (size_t)(chunk * 2 + ks) * 1024;
-        f.v[0][0] = *reinterpret_cast<const bf16x8_t*>(q);
-        f.v[0][1] = *reinterpret_cast<const bf16x8_t*>(q + 512);
-        f.v[1][0] = *reinterpret_cast<const bf16x8_t*>(q + mt1);
-        f.v[1][1] = *reinterpret_cast<const bf16x8_t*>(q + mt1 + 512);
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) {
+            f.v[mi][0] = *reinterpret_cast<const bf16x8_t*>(q + (mi ? mt1 : 0));
+            f.v[mi][1] = *reinterpret_cast<const bf16x8_t*>(q + (mi ? mt1 : 0) + 512);
+        }
     };
-    auto readB = [&](Bf3B& f, const uint16_t* tile, int tap, int ks) {
+    auto readB = [&](Bf3B<NI>& f, const uint16_t* tile, int tap, int ks) {
         const int toff = sh0 + tap * dsh - shmin;
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
+        for (int ni = 0; ni < NI; ++ni) {
             const int i = ncol + ni * 32 + toff;
             const uint16_t* q = tile + i * 32 + (((ks * 2 + kgrp) ^ ((i >> 2) & 3)) * 8);
             f.v[ni][0] = *reinterpret_cast<const bf16x8_t*>(q);
             f.v[ni][1] = *reinterpret_cast<const bf16x8_t*>(q + PLANE);
         }
     };
-    // three products per tile pair: hi.hi, hi.lo, lo.hi; four independent accumulators between dependent MFMAs
-    auto mfma12 = [&](const Bf3A& A, const Bf3B& B) {
+    // three products per tile pair: hi.hi, hi.lo, lo.hi; MI * NI independent accumulators between dependent MFMAs
+    auto products = [&](const Bf3A<MI>& A, const Bf3B<NI>& B) {
 #pragma unroll
         for (int term = 0; term < 3; ++term) {
             const int ta = term == 2 ? 1 : 0, tb = term == 1 ? 1 : 0;
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi)
+            for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
-                for (int ni = 0; ni < 2; ++ni)
+                for (int ni = 0; ni < NI; ++ni)
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v[mi][ta], B.v[ni][tb], acc[mi][ni], 0, 0, 0);
         }
     };
-    loadA(aq[0], 0, 0, 0);
-    loadA(aq[1], 0, 0, 1);
+#pragma unroll
+    for (int J = 0; J < AR - 1; ++J) loadA(aq[J], J / NST, (J % NST) >> 1, J & 1);
     const uint16_t* tile = lds;
     int gbuf = 0;                                           // ring slot of the next chunk
     const float* Xb = pX + (size_t)b * p.Cin * p.ldx;
@@ -239,15 +251,15 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
 
     {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < NI; ++j)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
         int cc = 0;
-        for (; cc + 3 <= nchunks; cc += 3) {
+        for (; cc + CG <= nchunks; cc += CG) {
 #pragma unroll
-            for (int I = 0; I < 3 * NST; ++I) {
+            for (int I = 0; I < CG * NST; ++I) {
                 const int t = I % NST;
                 if (t == 0) {
                     __builtin_amdgcn_s_barrier();
@@ -256,22 +268,22 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                     readB(bq[I & 1], tile, 0, 0);
                 }
                 // one scheduling region per step: the prefetches of later steps cannot sink out of it (left alone the scheduler moves
-                // them next to their use), and inside it they are spread over the shadows of the 12 MFMAs instead of running ahead
+                // them next to their use), and inside it they are spread over the shadows of the MFMAs instead of running ahead
                 // of them with the matrix pipe idle: MFMA, then a weight load or a tile read with its address arithmetic
                 __builtin_amdgcn_sched_barrier(0);
                 if (t + 1 < NST) readB(bq[(I + 1) & 1], tile, (t + 1) >> 1, (t + 1) & 1);
-                const int J = I + 2;
-                loadA(aq[J % 3], cc + J / NST, (J % NST) >> 1, J & 1);
-                mfma12(aq[I % 3], bq[I & 1]);
-                B3_INTERLEAVE
+                const int J = I + AR - 1;
+                loadA(aq[J % AR], cc + J / NST, (J % NST) >> 1, J & 1);
+                products(aq[I % AR], bq[I & 1]);
+                if constexpr (MI == 2) { B3_INTERLEAVE_22 } else if constexpr (NI == 2) { B3_INTERLEAVE_12 } else { B3_INTERLEAVE_11 }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        // tail: one or two chunks, same schedule with a runtime bound (rotation phase 0 here: 3 * NST steps per group)
-        if (cc < nchunks) {
+        // tail: up to CG - 1 chunks, same schedule with a runtime bound (rotation phase 0 here)
+        if (CG > 1 && cc < nchunks) {
             const int rem = (nchunks - cc) * NST;
 #pragma unroll
-            for (int I = 0; I < 2 * NST; ++I) {
+            for (int I = 0; I < (CG - 1) * NST; ++I) {
                 if (I < rem) {
                     const int t = I % NST;
                     if (t == 0) {
@@ -282,10 +294,10 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                     }
                     __builtin_amdgcn_sched_barrier(0);
                     if (t + 1 < NST) readB(bq[(I + 1) & 1], tile, (t + 1) >> 1, (t + 1) & 1);
-                    const int J = I + 2;
-                    loadA(aq[J % 3], cc + J / NST, (J % NST) >> 1, J & 1);
-                    mfma12(aq[I % 3], bq[I & 1]);
-                    B3_INTERLEAVE
+                    const int J = I + AR - 1;
+                    loadA(aq[J % AR], cc + J / NST, (J % NST) >> 1, J & 1);
+                    products(aq[I % AR], bq[I & 1]);
+                    if constexpr (MI == 2) { B3_INTERLEAVE_22 } else if constexpr (NI == 2) { B3_INTERLEAVE_12 } else { B3_INTERLEAVE_11 }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -298,11 +310,11 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
         asm volatile("" : "+v"(lane_hi));
         if (P.ksplit > 1) {                                  // split-K: the raw sums of this slice; k_bf3_splitk_epilogue adds the slices up
 #pragma unroll
-            for (int ni = 0; ni < 2; ++ni) {
-                const int n = n0 + wn * 64 + ni * 32 + (lane & 31);
+            for (int ni = 0; ni < NI; ++ni) {
+                const int n = n0 + (wn * NI + ni) * 32 + (lane & 31);
                 if (n >= p.N) continue;
 #pragma unroll
-                for (int mi = 0; mi < 2; ++mi) {
+                for (int mi = 0; mi < MI; ++mi) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int m = (mt0 + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * lane_hi;
@@ -312,42 +324,53 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
             }
             return;
         }
+        // a tile's bias and residual (or NoiseBlock input) values are requested together, clamped; one by one under their guards each was a round trip
+        const float* eb = noise ? Xb : Rr ? Rr + (size_t)b * p.M * p.ldy : nullptr;
+        const int lde = noise ? p.ldx : p.ldy;
 #pragma unroll
-        for (int ni = 0; ni < 2; ++ni) {
-            const int n = n0 + wn * 64 + ni * 32 + (lane & 31);
-            if (n >= p.N) continue;
-            float nz = 0.0f;
-            if (noise) {
-                if (pnoise) nz = pnoise[(size_t)b * p.N + n];
-                else if (p.noise_rng) nz = codec_noise_value(p.noise_key, (uint64_t)(p.row_offset + (p.row_ids ? p.row_ids[b] : b)), n);
+        for (int mi = 0; mi < MI; ++mi) {
+            const int m0 = (mt0 + mi) * 32 + 4 * lane_hi;
+            float bm[16], sc[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) bm[r] = pbias ? pbias[min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1)] : 0.0f;
+            if (Rr && pscale) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sc[r] = pscale[min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1)];
             }
-            const int o = convt ? p.s * n + phase : n;
-            if (o >= p.Tout) continue;
-            const bool dupb = convt && n == 0 && p.dup_bias_n0;
 #pragma unroll
-            for (int mi = 0; mi < 2; ++mi) {
+            for (int ni = 0; ni < NI; ++ni) {
+                const int n = n0 + (wn * NI + ni) * 32 + (lane & 31);
+                float e[16];
+                if (eb) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) e[r] = eb[(size_t)min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1) * lde + min(n, p.N - 1)];
+                }
+                float nz = 0.0f;
+                if (noise && n < p.N) {
+                    if (pnoise) nz = pnoise[(size_t)b * p.N + n];
+                    else if (p.noise_rng) nz = codec_noise_value(p.noise_key, (uint64_t)(p.row_offset + (p.row_ids ? p.row_ids[b] : b)), n);
+                }
+                const int o = convt ? p.s * n + phase : n;
+                if (n >= p.N || o >= p.Tout) continue;
+                const bool dupb = convt && n == 0 && p.dup_bias_n0;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int m = (mt0 + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * lane_hi;
-                    if (m >= p.M) continue;
-                    float v = acc[mi][ni][r];
-                    const float bm = pbias ? pbias[m] : 0.0f;
-                    v += bm;
-                    if (dupb) v += bm;
-                    const size_t rowo = ((size_t)b * p.M + m) * p.ldy;
+                    const int m = m0 + (r & 3) + 8 * (r >> 2);
+                    float v = acc[mi][ni][r] + bm[r];
+                    if (dupb) v += bm[r];
                     if (gelu) v = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
-                    if (Rr) { if (pscale) v *= pscale[m]; v += Rr[rowo + n]; }
-                    if (noise) v = Xb[(size_t)m * p.ldx + n] + nz * v;
-                    pY[rowo + o] = v;
+                    if (Rr) { if (pscale) v *= sc[r]; v += e[r]; }
+                    if (noise) v = e[r] + nz * v;
+                    if (m < p.M) pY[((size_t)b * p.M + m) * p.ldy + o] = v;
                 }
             }
         }
     }
 }
 
-template <int NQ, int NBUF, int NTAPS, int MINW>
+template <int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, int MINW>
 __global__ void __launch_bounds__(B3_THREADS, MINW) k_bf3_gemm(Bf3Params P) {
-    bf3_body<NQ, NBUF, NTAPS>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise);
+    bf3_body<MI, NI, NQ, NBUF, NTAPS, AR>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise);
 }
 
 // split-K: Y = epilogue(sum over slices in slice order + bias) - the 1x1 modes' epilogues of bf3_body (plain / GELU / residual with scale)
@@ -420,11 +443,19 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
     if (p.M < 32 || span > 64 || (ntaps != 1 && ntaps != 2 && ntaps != 7)) return false;
     const CodecPack::Entry& e = p.pack->get(p.AT, wtaps, Cin, p.M, s);
 
-    const int nbx = (p.N + B3_BN - 1) / B3_BN;
-    const int nq = span <= 16 ? 9 : 12;
+    // Tile: 128 x 128 (64 x 64 per wave); 64 x 128 while those are at most 128 blocks - half of the chip idle, each block one serial chain of chunks -
+    // and 64 x 64 while 64 x 128 still are (or no more than 64 columns exist).  The same bits: the order of the products of an output does not change.
+    // The small tiles run alone on a compute unit, with registers to spare: weights seven (not two) steps ahead, which covers a trip to HBM.
+    // us, 128 x 128 / 64 x 128 / 64 x 64: 768 rows, 7 taps of 768, 2080 columns: 102 / 60 / 79; 768 rows, K = 768: 51 / 24 / 26;
+    // 1536 rows, 7 taps of 1024, 250 columns: 140 / 70 / 55; SNAC, one row of 12 groups: 48 / - / 19, 41 / 22 / 15, 33 / - / 14, 29 / 17 / 16.
+    const int phases = mode == GEMM_CONVT ? p.s : 1;
+    const int nb128 = (p.N + 127) / 128;
+    const bool few = (int64_t)nb128 * ((p.M + B3_BM - 1) / B3_BM) * batch * phases <= 128;
+    const int NI = few && (p.N <= 64 || (int64_t)nb128 * ((p.M + 63) / 64) * batch * phases <= 128) ? 1 : 2, bn = 64 * NI, nbx = (p.N + bn - 1) / bn;
+    const int nq = span <= 16 ? 4 * NI + 1 : 4 * NI + 4;
     // the transposed conv's phases share one pre-pass: columns from the smallest shift of any phase to the largest
     const int extra = mode == GEMM_CONVT ? ((p.s - 1 + p.pad) / p.s - p.pad / p.s) : 0;
-    const int Tp = (nbx - 1) * B3_BN + nq * 16 + extra;
+    const int Tp = (nbx - 1) * bn + nq * 16 + extra;
     p.pack->xh.alloc((size_t)batch * Tp * e.Cp);
     p.pack->xl.alloc((size_t)batch * Tp * e.Cp);
     const bool sn = snake && p.alpha;
@@ -434,11 +465,10 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
     P.g = p; P.g.Cin = Cin;
     P.wp = e.wp; P.xh = p.pack->xh.p; P.xl = p.pack->xl.p;
     P.mode = mode; P.ntaps = ntaps; P.MT32 = e.MT32; P.KS = e.KS; P.Cp = e.Cp; P.Tp = Tp; P.t_org = t_org;
-    const int phases = mode == GEMM_CONVT ? p.s : 1;
     // launch-shaped 1x1 contractions (Soprano's ConvNeXt GEMMs at 257 frames: 18 or 54 blocks per row of a 256-CU part, 60 us per launch):
     // the K range split over blocks.  The factor is a function of the SHAPE of one batch row only (a row's bits do not depend on the batch
     // it shares); float32 slabs, summed in slice order by k_bf3_splitk_epilogue
-    const int nchunks = e.Cp / B3_KC, per_row = nbx * ((p.M + B3_BM - 1) / B3_BM);
+    const int nchunks = e.Cp / B3_KC, per_row = nb128 * ((p.M + B3_BM - 1) / B3_BM);
     int ksplit = 1;
     if (p.split_k_ok && ntaps == 1 && (mode == GEMM_PLAIN || mode == GEMM_GELU || mode == GEMM_RESID) && !bf3_env("MIS_BF3_NO_SPLITK", 0)) {
         if (per_row <= 32 && nchunks >= 32) ksplit = 4;
@@ -448,18 +478,31 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
         p.pack->part.alloc((size_t)ksplit * batch * p.M * p.ldy);
         P.ksplit = ksplit; P.part = p.pack->part.p; P.batch = batch;
     }
-    dim3 grid(nbx, (p.M + B3_BM - 1) / B3_BM, batch * phases * ksplit), block(B3_THREADS);
-    // MINW 3 = two blocks (ten waves) per CU: 168 registers; the 7-tap body then spills a few address temporaries (A/B by MIS_BF3_MINW)
+    const int bm = few ? 64 : B3_BM;
+    P.nbx = nbx; P.my = (p.M + bm - 1) / bm; P.inner = phases * ksplit;
+    P.tiles = nbx * P.my * batch; P.per = (P.tiles + 7) / 8;
+    dim3 grid(8 * P.per * P.inner), block(B3_THREADS);
+#define B3_GO(...) hipLaunchKernelGGL((k_bf3_gemm<__VA_ARGS__>), grid, block, 0, s, P)
+    if (few && NI == 1) {
+        if (ntaps == 1) B3_GO(1, 1, 5, 8, 1, 8, 2);
+        else if (ntaps == 2) B3_GO(1, 1, 5, 8, 2, 8, 2);
+        else if (span <= 16) B3_GO(1, 1, 5, 4, 7, 7, 2);
+        else B3_GO(1, 1, 8, 4, 7, 7, 2);
+    } else if (few) {
+        if (ntaps == 1) B3_GO(1, 2, 9, 5, 1, 8, 2);
+        else if (ntaps == 2) B3_GO(1, 2, 9, 5, 2, 8, 2);
+        else if (span <= 16) B3_GO(1, 2, 9, 4, 7, 7, 2);
+        else B3_GO(1, 2, 12, 4, 7, 7, 2);
+    }
     // MINW 3 = two blocks (ten waves) per CU, 168 registers: fits 1 and 2 taps; the 7-tap body would spill (measured 2.3x slower), so it
     // runs one block per CU (a persistent loop over column tiles was measured too: no gain, profiles/r02_codec/ab_record.json)
-    if (ntaps == 1) {
-        hipLaunchKernelGGL((k_bf3_gemm<9, 4, 1, 3>), grid, block, 0, s, P);
-        if (ksplit > 1)
-            hipLaunchKernelGGL(k_bf3_splitk_epilogue, dim3((p.N + 255) / 256, p.M, batch), dim3(256), 0, s, P.part, ksplit, batch, mode, p.bias, p.scale, p.R, p.Y, p.M,
-                               p.N, p.ldy);
-    }
-    else if (ntaps == 2) hipLaunchKernelGGL((k_bf3_gemm<9, 4, 2, 3>), grid, block, 0, s, P);
-    else if (nq == 9) hipLaunchKernelGGL((k_bf3_gemm<9, 4, 7, 2>), grid, block, 0, s, P);
-    else hipLaunchKernelGGL((k_bf3_gemm<12, 4, 7, 2>), grid, block, 0, s, P);
+    else if (ntaps == 1) B3_GO(2, 2, 9, 4, 1, 3, 3);
+    else if (ntaps == 2) B3_GO(2, 2, 9, 4, 2, 3, 3);
+    else if (span <= 16) B3_GO(2, 2, 9, 4, 7, 4, 2);
+    else B3_GO(2, 2, 12, 4, 7, 4, 2);
+#undef B3_GO
+    if (ksplit > 1)
+        hipLaunchKernelGGL(k_bf3_splitk_epilogue, dim3((p.N + 255) / 256, p.M, batch), dim3(256), 0, s, P.part, ksplit, batch, mode, p.bias, p.scale, p.R, p.Y, p.M,
+                           p.N, p.ldy);
     return true;
 }
