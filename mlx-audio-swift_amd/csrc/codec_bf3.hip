@@ -408,16 +408,16 @@ const CodecPack::Entry& CodecPack::get(const float* at, int ntaps, int Cin, int 
     return entries.back();
 }
 
-static thread_local CodecPack* tl_pack = nullptr;
-CodecPackScope::CodecPackScope(CodecPack* p) : prev(tl_pack) { tl_pack = p; }
-CodecPackScope::~CodecPackScope() { tl_pack = prev; }
+static thread_local CodecPack *tl_pack = nullptr, *tl_x6 = nullptr;
+CodecPackScope::CodecPackScope(CodecPack* p, bool bf3) : prev(tl_pack), prev_x6(tl_x6) { tl_pack = bf3 ? p : nullptr; tl_x6 = p; }
+CodecPackScope::~CodecPackScope() { tl_pack = prev; tl_x6 = prev_x6; }
 
 static int bf3_env(const char* name, int dflt) {
     const char* v = getenv(name);
     return v ? atoi(v) : dflt;
 }
 
-CodecPack* codec_pack_scope() { return tl_pack; }
+CodecPack* codec_x6_scope() { return tl_x6; }
 bool codec_exact_f32() { return bf3_env("MIS_CODEC_EXACT_F32", 0) != 0; }
 
 bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s) {

@@ -318,9 +318,11 @@ __device__ __forceinline__ void codec_gemm_split_body(const GemmParams& p, const
 }
 __global__ void __launch_bounds__(256) k_codec_gemm_split(GemmParams p) { codec_gemm_split_body(p, p.X, p.R, p.Y, p.bias, p.scale, p.AT); }
 
+bool codec_taps_split(const GemmParams& p) { return (long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 64 && p.K >= 1024 && cdiv(p.N, 16) <= 65535; }
+
 template <int MODE, bool SNAKE>
 static void launch_f32(const GemmParams& p, int batch, hipStream_t s) {
-    if (MODE == GEMM_TAPS && (long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 64 && p.K >= 1024 && cdiv(p.N, 16) <= 65535) {
+    if (MODE == GEMM_TAPS && codec_taps_split(p)) {
         hipLaunchKernelGGL(k_codec_gemm_split, dim3(cdiv(p.M, 32), cdiv(p.N, 16), batch), dim3(256), 0, s, p);
         return;
     }

@@ -82,15 +82,14 @@ struct CodecPack {
     const X6& get_x6(const float* at, int ntaps, int Cin, int M, hipStream_t s);
 };
 
-// Decoders open a scope around their launches: launch_gemm picks the scope's CodecPack up when GemmParams.pack is null.  Encoders
-// (codebook decisions) do not, and stay on the exact-f32 kernels.
+// Decoders open a scope around their launches: launch_gemm picks the scope's CodecPack up when GemmParams.pack is null.  Encoders (codebook decisions) open
+// one with bf3 = false: the three-plane contractions, which are as accurate as the f32 kernels, and none of two planes.  null: exact-f32 kernels only.
 struct CodecPackScope {
-    CodecPack* prev;
-    explicit CodecPackScope(CodecPack* p);
+    CodecPack *prev, *prev_x6;
+    explicit CodecPackScope(CodecPack* p, bool bf3 = true);
     ~CodecPackScope();
 };
-
-CodecPack* codec_pack_scope();        // the innermost scope's, or null
+CodecPack* codec_x6_scope();          // the innermost scope's, or null
 bool codec_exact_f32();               // MIS_CODEC_EXACT_F32=1
 
 #define CODEC_DW_HALO 27              // 3 * max dilation (9)
@@ -136,6 +135,9 @@ struct GemmParams {
 void launch_gemm(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // exact-f32 kernels (codec_f32.hip): every mode but CONVT, TAPS without Snake; p must have ldx / ldy resolved
 void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
+bool codec_taps_split(const GemmParams& p);      // k-tap contraction of few tiles and a long K: the k-split form of codec_f32.hip
+// three-plane split (codec_x6.hip): 1x1 and k-tap contractions of at least 32 rows and a multiple of 16 channels; false: not eligible, nothing launched
+bool launch_gemm_x6(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // split-bf16 path; false = shape not eligible (or MIS_CODEC_EXACT_F32=1), nothing launched.  p must have ldx / ldy resolved
 bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // depthwise 7-tap conv (zero padded, dilation dil): shorter odd kernels ride in centred 7-tap weights

@@ -13,6 +13,7 @@
 #include "codec_kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 __device__ __forceinline__ float x6_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
 
@@ -35,15 +36,15 @@ __device__ __forceinline__ void x6_split(const float (&v)[8], uint4& h, uint4& m
     l = make_uint4(o[2][0], o[2][1], o[2][2], o[2][3]);
 }
 
-// A^T f32 [ntaps][Cin][M] -> fragments of v_mfma_f32_32x32x16_bf16: [tap][Cp / 16][MT32][plane][64 lanes][8]
+// A^T f32 [ntaps][Cin][M] -> fragments of v_mfma_f32_32x32x16_bf16: [Cin / 16][tap][MT32][plane][64 lanes][8]
 __global__ void k_x6_pack_w(const float* __restrict__ AT, uint16_t* __restrict__ wp, int ntaps, int Cin, int M, int MT32, int KS) {
     const size_t total = (size_t)ntaps * KS * MT32 * 512;
     for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
         const int j = (int)(e & 7), lane = (int)((e >> 3) & 63);
         size_t r = e >> 9;
         const int mt = (int)(r % MT32); r /= MT32;
-        const int ks = (int)(r % KS);
-        const int tap = (int)(r / KS);
+        const int tap = (int)(r % ntaps);
+        const int ks = (int)(r / ntaps);
         const int m = mt * 32 + (lane & 31), c = ks * 16 + (lane >> 5) * 8 + j;
         float v = (m < M && c < Cin) ? AT[((size_t)tap * Cin + c) * M + m] : 0.0f;
         const size_t o = (e >> 9) * 1536 + (size_t)lane * 8 + j;
@@ -231,12 +232,267 @@ static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hip
 
 // 64 channels stay on k_pw_fused: twice the columns per product, bound by memory and by the units' VALU work (1.16 ms here, 1.10 there)
 bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s) {
-    if (!pack) pack = codec_pack_scope();
+    if (!pack) pack = codec_x6_scope();
     if (!pack || codec_exact_f32() || !(dw ? C == 128 : (C == 96 || C == 128 || C == 192))) return false;
     const uint16_t* wp = pack->get_x6(p.AT, 1, C, C, s).wp;
     if (dw) launch_x6<128, true>(p, wp, batch, s);
     else if (C == 96) launch_x6<96, false>(p, wp, batch, s);
     else if (C == 128) launch_x6<128, false>(p, wp, batch, s);
     else launch_x6<192, false>(p, wp, batch, s);
+    return true;
+}
+
+// ---- 1x1 and k-tap contractions -----------------------------------------------------------------------------------------------------------
+// A wave owns 32 columns and MTW row tiles: it reads its eight channels of a column per lane straight from memory, converts them once and multiplies them
+// with all its rows, so the activations need neither LDS nor a barrier.  WIDE: the four waves of a block share the weights, staged in LDS two chunks deep;
+// else (few blocks) one row tile per block, weights straight into registers.  k order: 16 channels, within them the taps, six products each.
+// Bound (256 x 256 with residual, 32 x 24576 columns): 2.4 GB = 0.49 ms of the 0.85; the products' 0.53 ms run half behind it.
+typedef uint32_t x6_u4 __attribute__((ext_vector_type(4)));
+struct X6Gemm {
+    GemmParams g;
+    int mode, ntaps, nsteps, MT32;        // steps of 16 channels of one tap
+    int nbx, my, per, tiles;              // column tiles, row tiles, tiles per XCD, all tiles
+};
+template <int MTW, bool SNAKE, bool TAPS, bool WIDE>
+__device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
+                                             const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise,
+                                             const float* __restrict__ pa, const float* __restrict__ pra, const uint16_t* __restrict__ pwp) {
+    constexpr int PF = MTW == 8 ? 2 : 4, SPB = MTW == 8 ? 1 : 2;            // steps of X (narrow: of weights too) in flight; steps per staged chunk of weights
+    constexpr int NA = (SPB * MTW * 192 + 255) / 256, APC = SPB * MTW * 192;
+    __shared__ x6_u4 As[WIDE ? 2 : 1][WIDE ? APC : 1];
+    extern __shared__ float x6_ab[];                                        // SNAKE: alpha [K], 1 / alpha [K]
+    const GemmParams& p = P.g;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kh = lane >> 5;
+    const int tileid = (blockIdx.x & 7) * P.per + (blockIdx.x >> 3);
+    if (tileid >= P.tiles) return;
+    const int by = tileid % P.my, bxb = tileid / P.my, bx = bxb % P.nbx, b = bxb / P.nbx;
+    const int n = bx * 128 + wave * 32 + (lane & 31), nc = min(n, p.N - 1);
+    const int mt0 = by * MTW, Kx = TAPS ? p.Cin : p.K;
+    if constexpr (SNAKE) {
+        for (int i = tid; i < Kx; i += 256) { x6_ab[i] = pa[i]; x6_ab[Kx + i] = pra[i]; }
+        __syncthreads();
+    }
+    if (!WIDE && bx * 128 + wave * 32 >= p.N) return;                       // (no barrier below)
+    const float* xb = pX + ((size_t)b * Kx + kh * 8) * p.ldx;
+    const x6_u4* wsrc = reinterpret_cast<const x6_u4*>(pwp) + (size_t)mt0 * 192;
+    const size_t wstep = (size_t)P.MT32 * 192;
+    const int mtop = (P.MT32 - mt0) * 192 - 1;                              // last piece of this block's rows within a step
+    float v[PF][8];
+    bool ok[PF];
+    x6_u4 aw[WIDE ? 1 : PF][MTW][3];
+    int fs = 0, ftap = 0;                                                   // next step to request
+    const float* fx = xb;
+    auto fetch = [&](int slot) {
+        const int t = TAPS ? nc - p.pad + ftap * p.dil : nc;
+        ok[slot] = !TAPS || (t >= p.x_lo && t < p.Tin);
+        const float* r = fx + (TAPS ? min(max(t, p.x_lo), p.Tin - 1) : t);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[slot][j] = r[(size_t)j * p.ldx];
+        if constexpr (!WIDE) {
+#pragma unroll
+            for (int mi = 0; mi < MTW; ++mi)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) aw[slot][mi][q] = wsrc[(size_t)fs * wstep + min((mi * 3 + q) * 64 + lane, mtop)];
+        }
+        if (fs + 1 < P.nsteps) {                                            // (past the end: the last step again)
+            ++fs;
+            if (!TAPS || ++ftap == P.ntaps) { ftap = 0; fx += (size_t)16 * p.ldx; }
+        }
+    };
+    x6_u4 wv[NA];
+    auto loadA = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int e = min(tid + i * 256, APC - 1), st = e / (MTW * 192), o = e - st * (MTW * 192);
+            wv[i] = wsrc[(size_t)min(c * SPB + st, P.nsteps - 1) * wstep + min(o, mtop)];
+        }
+    };
+    auto putA = [&](int h) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+            if (APC % 256 == 0 || tid + i * 256 < APC) As[h][tid + i * 256] = wv[i];
+    };
+        // Epilogue values (the modes of k_codec_gemm; C/D layout: col = lane & 31, row = (r & 3) + 8 (r >> 2) + 4 (lane >> 5)): a tile's bias, scale and residual or
+    // NoiseBlock input, requested together - the narrow form's before its contraction.
+    const bool noise = P.mode == GEMM_NOISE, gelu = P.mode == GEMM_GELU;
+    const float* eb = noise ? pX + (size_t)b * p.K * p.ldx : (!gelu && pR) ? pR + (size_t)b * p.M * p.ldy : nullptr;
+    const int lde = noise ? p.ldx : p.ldy;
+    const float* bp = pbias ? pbias : pX;                                   // (loaded either way: a guard per value would be a round trip per value)
+    const int btop = pbias ? p.M - 1 : 0;
+    float nz = 0.0f;
+    if (noise && n < p.N) {
+        if (pnoise) nz = pnoise[(size_t)b * p.N + n];
+        else if (p.noise_rng) nz = codec_noise_value(p.noise_key, (uint64_t)(p.row_offset + (p.row_ids ? p.row_ids[b] : b)), n);
+    }
+    float bm[16], sc[16], e[16];
+    auto want = [&](int mi, int lane_hi) {
+        const int m0 = (mt0 + mi) * 32 + 4 * lane_hi;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bm[r] = bp[min(m0 + (r & 3) + 8 * (r >> 2), btop)];
+        if (pscale) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = pscale[min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1)];
+        }
+        if (eb) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) e[r] = eb[(size_t)min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1) * lde + nc];
+        }
+    };
+    if constexpr (!WIDE) want(0, kh);
+    f32x16_t acc[MTW];
+#pragma unroll
+    for (int i = 0; i < MTW; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+    int ks = 0, tap = 0;                                                    // step being multiplied (SNAKE: its channels)
+    bf16x8_t bv[2][3];
+    auto convert = [&](int slot, int h2) {
+        float x[8];
+        [[maybe_unused]] const int kc = min(ks * 16, Kx - 16) + kh * 8;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            x[j] = v[slot][j];
+            if constexpr (SNAKE) x[j] = x6_snake(x[j], x6_ab[kc + j], x6_ab[Kx + kc + j]);
+            if constexpr (TAPS) x[j] = ok[slot] ? x[j] : 0.0f;
+        }
+        uint4 h, m, l;
+        x6_split(x, h, m, l);
+        bv[h2][0] = __builtin_bit_cast(bf16x8_t, h); bv[h2][1] = __builtin_bit_cast(bf16x8_t, m); bv[h2][2] = __builtin_bit_cast(bf16x8_t, l);
+        if (!TAPS || ++tap == P.ntaps) { tap = 0; ++ks; }
+    };
+    constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};   // as pw_x6_body
+    auto products = [&](int h2, auto frag) {
+        constexpr int MP = MTW >= 2 ? 2 : 1;
+#pragma unroll
+        for (int m0 = 0; m0 < MTW; m0 += MP) {
+            bf16x8_t av[MP][3];
+#pragma unroll
+            for (int mi = 0; mi < MP; ++mi)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, frag(m0 + mi, q));
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int mi = 0; mi < MP; ++mi) acc[m0 + mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[h2][QB[q]], acc[m0 + mi], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < PF; ++i) fetch(i);
+    // One scheduling region per step: this step's products, the next one's conversion, the request of the step PF ahead.  (With guards between them the
+    // conversion waits for the products; without the barrier the scheduler moves the requests to their use.)
+    convert(0, 0);
+    if constexpr (WIDE) {
+        constexpr int CG = PF / SPB;                                        // chunks per straight-line group: PF steps, an even number of chunks
+        static_assert(CG % 2 == 0, "the LDS buffer of a chunk is its parity inside the group");
+        const int nchunks = (P.nsteps + SPB - 1) / SPB;
+        loadA(0);
+        putA(0);
+        loadA(1);
+        __syncthreads();
+        auto group = [&](int c0, auto whole) {
+#pragma unroll
+            for (int u = 0; u < CG; ++u) {
+                putA((u + 1) & 1);
+                loadA(c0 + u + 2);
+#pragma unroll
+                for (int st = 0; st < SPB; ++st) {
+                    const int slot = u * SPB + st;
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch(slot);
+                    if (decltype(whole)::value || c0 * SPB + slot < P.nsteps) products(slot & 1, [&](int mi, int q) { return As[u & 1][(st * MTW + mi) * 192 + q * 64 + lane]; });
+                    convert((slot + 1) % PF, (slot + 1) & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                __syncthreads();
+            }
+        };
+        int c0 = 0;
+        for (; (c0 + CG) * SPB <= P.nsteps; c0 += CG) group(c0, std::true_type{});
+        if (c0 < nchunks) group(c0, std::false_type{});
+    } else {
+        auto group = [&](int s0, auto whole) {
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                x6_u4 a[MTW][3];
+#pragma unroll
+                for (int mi = 0; mi < MTW; ++mi)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) a[mi][q] = aw[u][mi][q];
+                __builtin_amdgcn_sched_barrier(0);
+                fetch(u);
+                if (decltype(whole)::value || s0 + u < P.nsteps) products(u & 1, [&](int mi, int q) { return a[mi][q]; });
+                convert((u + 1) % PF, (u + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        int s0 = 0;
+        for (; s0 + PF <= P.nsteps; s0 += PF) group(s0, std::true_type{});
+        if (s0 < P.nsteps) group(s0, std::false_type{});
+    }
+    int lane_hi = kh;                                                       // (opaque: the rows' addresses are not to be computed ahead of the contraction)
+    asm volatile("" : "+v"(lane_hi));
+#pragma unroll
+    for (int mi = 0; mi < MTW; ++mi) {
+        if ((mt0 + mi) * 32 >= p.M) break;
+        const int m0 = (mt0 + mi) * 32 + 4 * lane_hi;
+        if constexpr (WIDE) want(mi, lane_hi);
+        if (n < p.N) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + (r & 3) + 8 * (r >> 2);
+                float y = acc[mi][r] + (pbias ? bm[r] : 0.0f);
+                if (gelu) y = 0.5f * y * (1.0f + erff(y * 0.70710678118654752f));
+                else if (noise) y = e[r] + nz * y;
+                else if (eb) { if (pscale) y *= sc[r]; y = e[r] + y; }
+                if (m < p.M) pY[((size_t)b * p.M + m) * p.ldy + n] = y;
+            }
+        }
+    }
+}
+template <int MTW, bool SNAKE, bool TAPS, bool WIDE>
+__global__ void __launch_bounds__(256, 2) k_x6_gemm(X6Gemm P, const uint16_t* wp) {
+    x6_gemm_body<MTW, SNAKE, TAPS, WIDE>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.g.alpha, P.g.ralpha, wp);
+}
+
+template <bool SNAKE, bool TAPS>
+static void launch_x6_gemm(X6Gemm P, const uint16_t* wp, int batch, hipStream_t s) {
+    const GemmParams& p = P.g;
+    P.nbx = (p.N + 127) / 128;
+    const size_t sm = SNAKE ? (size_t)2 * p.K * sizeof(float) : 0;
+    auto go = [&](auto kernel, int mtw) {
+        P.my = (P.MT32 + mtw - 1) / mtw;
+        P.tiles = P.nbx * P.my * batch;
+        P.per = (P.tiles + 7) / 8;
+        hipLaunchKernelGGL(kernel, dim3(8 * P.per), dim3(256), sm, s, P, wp);
+    };
+    // The form with the most rows per block (each converts its columns once) that still gives blocks enough; the same bits in all of them.  us:
+    //   8 tiles / f32     256 x 256, 32 x 24576 columns 845 / 1133
+    //   4 / 2 / 1         192 x 192, 18888 columns (296, 592 blocks of 4 and 2): 29 / 20 / 24; the same rows, two taps of 192 (K = 768): 105 / 72 / 102
+    //   2 / 1 / f32       384 x 384 with Snake, 10160 columns: 41 / 56 / 71; 384 rows, K = 1536, 2361 columns (114 blocks of 2): 156 / 124 / 154
+    auto blocks = [&](int mtw) { return (int64_t)P.nbx * ((P.MT32 + mtw - 1) / mtw) * batch; };
+    if (P.MT32 > 4 && blocks(8) >= 512) go(k_x6_gemm<8, SNAKE, TAPS, true>, 8);
+    else if (P.MT32 > 2 && blocks(4) >= 512) go(k_x6_gemm<4, SNAKE, TAPS, true>, 4);
+    else if (blocks(2) >= 256) go(k_x6_gemm<2, SNAKE, TAPS, true>, 2);
+    else go(k_x6_gemm<1, SNAKE, TAPS, false>, 1);
+}
+
+bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s) {
+    GemmParams p = p_in;
+    CodecPack* pack = p.pack ? p.pack : codec_x6_scope();
+    const bool taps = mode == GEMM_TAPS;
+    if (!pack || codec_exact_f32() || mode == GEMM_CONVT || (snake && (mode != GEMM_RESID || !p.alpha))) return false;
+    const int Cin = taps ? p.Cin : p.K, ntaps = taps ? p.taps : 1;
+    // By the shape of the matrix alone: a row's result must not depend on its length or its batch.  512 channels at one short row are bound by latency,
+    // which the f32 kernel's four chunks of 64 channels in flight hide better (512 x 512, 96 columns: 15 us here, 8 there; 256 x 256, 768 columns: 11.3, 10.1);
+    // a NoiseBlock of 64 channels is bound by memory (32 x 196608 columns: 918 us here, 842 there; 48 channels with residual, 37776 columns: 23, 34).
+    if (p.M < (mode == GEMM_NOISE ? 96 : 48) || Cin < 32 || Cin % 16 || (!taps && Cin > 384)) return false;
+    if (taps && codec_taps_split(p)) return false;
+    if (mode != GEMM_RESID && mode != GEMM_TAPS) p.R = p.scale = nullptr;
+    const CodecPack::X6& e = pack->get_x6(p.AT, ntaps, Cin, p.M, s);
+    X6Gemm P{};
+    P.g = p; P.mode = mode; P.ntaps = ntaps; P.nsteps = e.KS * ntaps; P.MT32 = e.MT32;
+    if (taps) launch_x6_gemm<false, true>(P, e.wp, batch, s);
+    else if (snake) launch_x6_gemm<true, false>(P, e.wp, batch, s);
+    else launch_x6_gemm<false, false>(P, e.wp, batch, s);
     return true;
 }

@@ -1046,6 +1046,7 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
     MIS_REQUIRE(c->has_encoder, MIS_ERR_AUDIO_ENCODE, "this SNAC handle was loaded without encoder weights");
     HIP_CHECK(hipSetDevice(c->device));
     hipStream_t s = c->stream;
+    CodecPackScope pack_scope(&c->pack, false);                           // three-plane contractions (f32 accuracy), none of two planes
     const mis_snac_config& cf = c->cfg;
     const float* W = c->arena.p;
     const int64_t Tp = mis_snac_padded_length(c, n_samples);
@@ -1186,6 +1187,7 @@ void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
     if (launch_gemm_bf3(mode, snake, p, batch, s)) return;
     MIS_REQUIRE(mode != GEMM_TAPS || (p.taps >= 1 && p.taps <= CT_MAXT && (p.taps - 1) * p.dil + 3 + G_BN <= CT_XS), MIS_ERR_INVALID_INPUT,
                 "dense conv: %d taps with dilation %d exceed the staged halo", p.taps, p.dil);
+    if (launch_gemm_x6(mode, snake, p, batch, s)) return;
     if (mode != GEMM_CONVT && (mode != GEMM_TAPS || !snake)) { launch_gemm_f32(mode, snake, p, batch, s); return; }
     const int phases = mode == GEMM_CONVT ? p.s : 1;
     dim3 grid(cdiv(p.N, G_BN), cdiv(p.M, G_BM), batch * phases), block(256);

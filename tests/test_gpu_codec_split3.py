@@ -1,5 +1,6 @@
-"""The three-plane contraction of the residual units (csrc/codec_x6.hip): both chunk depths, 96 / 128 / 192 channels, a column remainder - as accurate as the
-exact-f32 kernels, and the same bits whatever batch (and with it chunk depth) a row comes in."""
+"""The three-plane contractions (csrc/codec_x6.hip) - the fused residual units: both chunk depths, 96 / 128 / 192 channels; the 1x1 and k-tap form: one to
+eight row tiles per block; column and row remainders in both - as accurate as the exact-f32 kernels, and the same bits whatever batch (and with it tile or
+chunk depth) a row comes in."""
 import numpy as np
 import pytest
 
@@ -32,9 +33,11 @@ def check(dev, orc, codes, rows, pick):
         assert np.array_equal(dev(pick(codes, slice(r, r + 1)))[0], got[r])
 
 
+# decoder channels 128 (units), 256 and 128 (NoiseBlock); 384, 192, 96, 48 (1x1 residuals, and rows past a tile of 32)
+@pytest.mark.parametrize("dim", [256, 512, 768])
 @pytest.mark.parametrize("rows, groups", [(3, 5), (40, 60)], ids=["one-wave", "many"])
-def test_snac_128(no_bf3, rows, groups):
-    cfg = dict(encoder_dim=8, encoder_rates=[2, 2, 2, 8], decoder_dim=256, decoder_rates=[8, 2, 2, 2], codebook_size=64, codebook_dim=8, vq_strides=[4, 2, 1])
+def test_snac(no_bf3, dim, rows, groups):
+    cfg = dict(encoder_dim=8, encoder_rates=[2, 2, 2, 8], decoder_dim=dim, decoder_rates=[8, 2, 2, 2], codebook_size=64, codebook_dim=8, vq_strides=[4, 2, 1])
     ocfg = osnac.SnacConfig(**cfg)
     W = osnac.make_synthetic_weights(ocfg, seed=31, with_encoder=True)
     dev = mas.SNAC.from_weights(mas.SNACConfig(**{k: getattr(ocfg, k) for k in mas.SNACConfig.__dataclass_fields__}), W)
@@ -53,3 +56,22 @@ def test_dac_192_96(no_bf3, rows, frames):
     orc = odac.DacOracle(ocfg, W)
     codes = np.random.default_rng(3).integers(0, ocfg.codebook_size, (rows, ocfg.n_codebooks, frames)).astype(np.int32)
     check(dev.decode_from_codes, orc.decode_from_codes, codes, rows, lambda c, sl: c[sl])
+
+
+# encoder channels 48 .. 768: strided convolutions of two taps over 2 - 8 phases of 48 - 384 channels, one short row to many
+@pytest.mark.parametrize("rows, samples", [(1, 4096 + 31), (12, 9 * 4096 - 5)], ids=["short", "many"])
+def test_snac_encode(rows, samples):
+    cfg = dict(encoder_dim=48, encoder_rates=[2, 2, 2, 8], decoder_dim=32, decoder_rates=[8, 2, 2, 2], codebook_size=64, codebook_dim=8, vq_strides=[4, 2, 1])
+    ocfg = osnac.SnacConfig(**cfg)
+    W = osnac.make_synthetic_weights(ocfg, seed=12, with_encoder=True)
+    dev = mas.SNAC.from_weights(mas.SNACConfig(**{k: getattr(ocfg, k) for k in mas.SNACConfig.__dataclass_fields__}), W)
+    oracle = osnac.SnacOracle(ocfg, W, dtype=np.float64)
+    audio = (0.3 * np.random.default_rng(8).standard_normal((rows, samples))).astype(np.float32)
+    codes, z = dev.encode(audio, return_latent=True)
+    with codec_exact_f32():
+        _, z32 = dev.encode(audio, return_latent=True)
+    ref = oracle.encoder(oracle.preprocess(audio[:1, None].astype(np.float64)))
+    err, err32 = (np.sqrt(np.mean((g[:1] - ref) ** 2) / np.mean(ref ** 2)) for g in (z, z32))
+    assert not np.array_equal(z, z32) and err <= 1.25 * err32 and err32 <= 1e-5, (err, err32)
+    one, z1 = dev.encode(audio[rows - 1:], return_latent=True)
+    assert np.array_equal(z1[0], z[rows - 1]) and all(np.array_equal(a[0], c[rows - 1]) for a, c in zip(one, codes))
