@@ -100,7 +100,7 @@ struct PwFusedParams {
     const float *AT, *b2;                  // W2^T [C][C] ([k][m]), bias
     int T, dil, ldx, ldr, ldy;
 };
-// three-plane split of the unit tails (codec_x6.hip); false: no pack (encoders), exact-f32 asked for, or another width - nothing launched
+// three-plane split of the unit tails (codec_x6.hip); false: no pack, exact-f32 asked for, or another width - nothing launched
 bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s);
 
 struct GemmParams {
@@ -136,8 +136,10 @@ void launch_gemm(int mode, bool snake, const GemmParams& p, int batch, hipStream
 // exact-f32 kernels (codec_f32.hip): every mode but CONVT, TAPS without Snake; p must have ldx / ldy resolved
 void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 bool codec_taps_split(const GemmParams& p);      // k-tap contraction of few tiles and a long K: the k-split form of codec_f32.hip
-// three-plane split (codec_x6.hip): 1x1 and k-tap contractions of at least 32 rows and a multiple of 16 channels; false: not eligible, nothing launched
+// three-plane split (codec_x6.hip): 1x1 and k-tap contractions of at least 48 rows and a multiple of 16 channels; false: not eligible, nothing launched
 bool launch_gemm_x6(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
+// three-plane split: transposed convolution of stride 2, two taps per phase, 32 .. 64 rows, behind Snake; false: another shape
+bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s);
 // split-bf16 path; false = shape not eligible (or MIS_CODEC_EXACT_F32=1), nothing launched.  p must have ldx / ldy resolved
 bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // depthwise 7-tap conv (zero padded, dilation dil): shorter odd kernels ride in centred 7-tap weights

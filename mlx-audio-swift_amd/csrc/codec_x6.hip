@@ -1,4 +1,4 @@
-// codec_x6.hip - the f32 contraction of the codecs' narrow residual units on the bf16 matrix pipe, at f32 accuracy.
+// codec_x6.hip - f32 contractions of the codecs on the bf16 matrix pipe, at f32 accuracy.
 //
 // Every f32 operand is written EXACTLY as three bfloat16, x = h + m + l, each the nearest to what is left (3 x 8 significant bits, signs absorb the carry),
 // and a product becomes the six bf16 MFMAs whose weight is above 2^-24: wh.xh + wh.xm + wm.xh + wm.xm + wh.xl + wl.xh (dropped: wm.xl + wl.xm + wl.xl,
@@ -9,6 +9,8 @@
 //
 //   k_x6_pack_w   A^T f32 -> the three planes as MFMA-A fragments (once per weight matrix, kept in the model's CodecPack)
 //   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels, for the encoders and for MIS_CODEC_EXACT_F32=1)
+//   k_x6_gemm     1x1 and k-tap contractions (codec_f32.hip keeps the rest)
+//   k_x6_convt    transposed convolutions of stride 2 and at most 64 rows
 #include "common.h"
 #include "codec_kernels.h"
 
@@ -494,5 +496,112 @@ bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hip
     if (taps) launch_x6_gemm<false, true>(P, e.wp, batch, s);
     else if (snake) launch_x6_gemm<true, false>(P, e.wp, batch, s);
     else launch_x6_gemm<false, false>(P, e.wp, batch, s);
+    return true;
+}
+
+// ---- transposed convolution of stride 2, kernel 4 (two taps per phase), at most 64 rows ----------------------------------------------------
+// Output 2 n + phase takes x[n + q] and x[n + q - 1], q = (phase + pad) / 2.  A block makes both phases of 126 columns n from 128 staged columns of x: Snake and
+// the split run once per element (k_snac_convt: per phase and tap), the taps read the planes at column offsets, and a lane stores its two phases as one
+// float2.  Chunks of 16 channels; weights of the four (phase, tap) pairs through LDS.  128 -> 64 channels, 32 x 98304 columns: 3.34 -> 1.44 ms (3.2 GB
+// are 0.65 ms, the products 1.05); one row of 12288: 43 -> 27 us.
+#define X6_CT 126
+template <int MT>
+__device__ __forceinline__ void x6_convt_body(const GemmParams& p, const float* __restrict__ pX, float* __restrict__ pY, const float* __restrict__ pbias,
+                                              const float* __restrict__ pa, const float* __restrict__ pra, const uint16_t* __restrict__ pwp) {
+    constexpr int APC = 4 * MT * 192, NA = APC / 256;
+    __shared__ x6_u4 As[APC];
+    __shared__ uint4 ts[3][2][128];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = blockIdx.x * X6_CT, b = blockIdx.y;
+    const int q0 = p.pad / 2, dq = (1 + p.pad) / 2 - q0;                    // phase 1 reads dq columns further
+    const int kg = wave >> 1, col = (wave & 1) * 64 + lane, t = n0 + q0 - 1 + col;
+    const bool ok = t >= p.x_lo && t < p.Tin;
+    const float* xb = pX + (size_t)b * p.Cin * p.ldx + min(max(t, p.x_lo), p.Tin - 1);
+    f32x16_t acc[2][MT];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    const x6_u4* wsrc = reinterpret_cast<const x6_u4*>(pwp) + tid;
+    float v[8];
+    x6_u4 wv[NA];
+    auto fetch = [&](int c0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = xb[(size_t)(c0 + kg * 8 + j) * p.ldx];
+#pragma unroll
+        for (int i = 0; i < NA; ++i) wv[i] = wsrc[(size_t)(c0 / 16) * APC + i * 256];
+    };
+    fetch(0);
+    for (int c0 = 0; c0 < p.Cin; c0 += 16) {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int c = c0 + kg * 8 + j;
+            x[j] = ok ? x6_snake(v[j], pa[c], pra[c]) : 0.0f;               // (the padding is zero behind Snake as well)
+        }
+        uint4 h, m, l;
+        x6_split(x, h, m, l);
+        __syncthreads();                                                    // the previous chunk's products are done
+        ts[0][kg][col] = h; ts[1][kg][col] = m; ts[2][kg][col] = l;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) As[tid + i * 256] = wv[i];
+        if (c0 + 16 < p.Cin) fetch(c0 + 16);
+        __syncthreads();
+        constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int ph = 0; ph < 2; ++ph)
+#pragma unroll
+            for (int tap = 0; tap < 2; ++tap) {
+                bf16x8_t bv[3];
+                const int i = min(wave * 32 + (lane & 31) + 1 - tap + (ph ? dq : 0), 127);      // (past the end only for columns that are not stored)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) bv[q] = *reinterpret_cast<const bf16x8_t*>(&ts[q][lane >> 5][i]);
+                bf16x8_t av[MT][3];
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, As[(((ph * 2 + tap) * MT + mi) * 3 + q) * 64 + lane]);
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int mi = 0; mi < MT; ++mi) acc[ph][mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[QB[q]], acc[ph][mi], 0, 0, 0);
+            }
+    }
+    const int nl = wave * 32 + (lane & 31), n = n0 + nl, o = 2 * n;
+    if (nl >= X6_CT || n >= p.N || o >= p.Tout) return;
+    const bool two = o + 1 < p.Tout, wide = two && !(p.ldy & 1) && !((uintptr_t)pY & 7), dup = n == 0 && p.dup_bias_n0;
+    const float* bp = pbias ? pbias : pX;                                   // (loaded either way: a guard per value would be a round trip per value)
+    const int btop = pbias ? p.M - 1 : 0;
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) {
+        const int m0 = mi * 32 + 4 * (lane >> 5);
+        float bm[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bm[r] = bp[min(m0 + (r & 3) + 8 * (r >> 2), btop)];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = m0 + (r & 3) + 8 * (r >> 2);
+            const float bv = pbias ? bm[r] : 0.0f;
+            float y0 = acc[0][mi][r] + bv, y1 = acc[1][mi][r] + bv;
+            if (dup) { y0 += bv; y1 += bv; }                                // streaming overlap-add counts the bias twice (GemmParams)
+            float* y = pY + ((size_t)b * p.M + m) * p.ldy + o;
+            if (m >= p.M) continue;
+            if (wide) *reinterpret_cast<float2*>(y) = make_float2(y0, y1);
+            else { y[0] = y0; if (two) y[1] = y1; }
+        }
+    }
+}
+template <int MT>
+__global__ void __launch_bounds__(256, 3) k_x6_convt(GemmParams p, const uint16_t* wp) { x6_convt_body<MT>(p, p.X, p.Y, p.bias, p.alpha, p.ralpha, wp); }
+
+bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s) {
+    CodecPack* pack = p.pack ? p.pack : codec_x6_scope();
+    if (!pack || codec_exact_f32() || p.s != 2 || p.K != 2 * p.Cin || p.M > 64 || p.M < 32 || p.Cin % 16 || !p.alpha) return false;
+    const uint16_t* wp = pack->get_x6(p.AT, 4, p.Cin, p.M, s).wp;           // [phase][tap][Cin][M]
+    const dim3 grid((p.N + X6_CT - 1) / X6_CT, batch);
+    if (p.M > 32) hipLaunchKernelGGL(k_x6_convt<2>, grid, dim3(256), 0, s, p, wp);
+    else hipLaunchKernelGGL(k_x6_convt<1>, grid, dim3(256), 0, s, p, wp);
     return true;
 }

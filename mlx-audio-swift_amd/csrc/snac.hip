@@ -9,7 +9,7 @@
 // Kernels (activations f32 [B][C][T], T contiguous):
 //   k_snac_embed   z_q = sum_i table_i[codes_i[b, t/stride_i]]       (table_i = codebook_i x out_proj_i + b_i)
 //   k_snac_dw      depthwise k=7 dilated conv with optional Snake before/after, LDS halo tile
-//   k_snac_convt   Snake -> transposed conv on v_mfma_f32_32x32x2_f32 (1x1 convs, NoiseBlock, strided convs: codec_f32.hip)
+//   k_snac_convt   Snake -> transposed conv on v_mfma_f32_32x32x2_f32 (stride 2: k_x6_convt; 1x1 convs, NoiseBlock, strided convs: codec_x6.hip, codec_f32.hip)
 //   k_codec_final  Snake -> conv k7 (C -> 1) -> tanh
 #include "common.h"
 #include "kernels.h"
@@ -1187,7 +1187,7 @@ void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
     if (launch_gemm_bf3(mode, snake, p, batch, s)) return;
     MIS_REQUIRE(mode != GEMM_TAPS || (p.taps >= 1 && p.taps <= CT_MAXT && (p.taps - 1) * p.dil + 3 + G_BN <= CT_XS), MIS_ERR_INVALID_INPUT,
                 "dense conv: %d taps with dilation %d exceed the staged halo", p.taps, p.dil);
-    if (launch_gemm_x6(mode, snake, p, batch, s)) return;
+    if (launch_gemm_x6(mode, snake, p, batch, s) || (mode == GEMM_CONVT && snake && launch_convt_x6(p, batch, s))) return;
     if (mode != GEMM_CONVT && (mode != GEMM_TAPS || !snake)) { launch_gemm_f32(mode, snake, p, batch, s); return; }
     const int phases = mode == GEMM_CONVT ? p.s : 1;
     dim3 grid(cdiv(p.N, G_BN), cdiv(p.M, G_BM), batch * phases), block(256);
