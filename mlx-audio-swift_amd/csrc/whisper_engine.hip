@@ -372,6 +372,9 @@ static void whisper_alloc_state(mis_whisper* c, int batch) {
     c->S_fc2 = split_for(d / 16 / 2, c->cfg.decoder_ffn_dim / 32);
     size_t ck = (size_t)Ld * batch * c->Hd * c->Spad * c->D;
     c->cross_k.alloc(ck); c->cross_v.alloc(ck);
+    // the keys past 1500 of every head stay zero; an encode overwrites all others, so they are cleared when the layout changes and not on each call
+    HIP_CHECK(hipMemsetAsync(c->cross_k.p, 0, c->cross_k.bytes(), c->stream));
+    HIP_CHECK(hipMemsetAsync(c->cross_v.p, 0, c->cross_v.bytes(), c->stream));
     size_t sk = (size_t)Ld * batch * c->Hd * Smax * c->D;
     c->self_k.alloc(sk); c->self_v.alloc(sk);
     c->enc_out.alloc((size_t)batch * 1500 * d);
@@ -403,21 +406,21 @@ static void whisper_encode_device(mis_whisper* c, const float* features_dev, int
     hipStream_t s = c->stream;
     const int d = c->d, fe = c->cfg.encoder_ffn_dim, H = c->He, D = c->D;
     if (batch != c->batch) whisper_alloc_state(c, batch);
-    HIP_CHECK(hipMemsetAsync(c->cross_k.p, 0, c->cross_k.bytes(), s));
-    HIP_CHECK(hipMemsetAsync(c->cross_v.p, 0, c->cross_v.bytes(), s));
     // the encoder runs in sub-batches of <= 8 utterances to bound the activation buffers
     const int SB = std::min(batch, 8);
     const size_t M1 = (size_t)SB * 3000, M = (size_t)SB * 1500;
     DevBuf<bf16_t> &col1 = c->e_col1, &h1 = c->e_h1, &col2 = c->e_col2, &h = c->e_h, &x = c->e_x, &qkv = c->e_qkv, &att = c->e_att, &ff = c->e_ff, &kc = c->e_kc,
                    &vc = c->e_vc, &ckv = c->e_ckv;
-    col1.alloc(M1 * c->K1); h1.alloc(M1 * d); col2.alloc(M * 3 * d); h.alloc(M * d); x.alloc(M * d); qkv.alloc(M * 3 * d);
+    if (col1.n < M1 * c->K1) { col1.alloc(M1 * c->K1); col1.zero(s); }
+    h1.alloc(M1 * d); col2.alloc(M * 3 * d); h.alloc(M * d); x.alloc(M * d); qkv.alloc(M * 3 * d);
     att.alloc(M * d); ff.alloc(M * fe); ckv.alloc(M * 2 * d);
     c->e_tight.alloc(M1 * 3 * c->nmel);
     size_t kvn = (size_t)SB * H * c->Spad * D;
-    kc.alloc(kvn); vc.alloc(kvn);
-    HIP_CHECK(hipMemsetAsync(col1.p, 0, M1 * c->K1 * 2, s));
-    HIP_CHECK(hipMemsetAsync(kc.p, 0, kvn * 2, s));
-    HIP_CHECK(hipMemsetAsync(vc.p, 0, kvn * 2, s));
+    // padded columns and keys are never written: cleared when the buffers grow
+    if (kc.n < kvn || vc.n < kvn) {
+        kc.alloc(kvn); vc.alloc(kvn);
+        kc.zero(s); vc.zero(s);
+    }
     for (int b0 = 0; b0 < batch; b0 += SB) {
         const int nb = std::min(SB, batch - b0);
         const int m1 = nb * 3000, m = nb * 1500;
@@ -437,8 +440,11 @@ static void whisper_encode_device(mis_whisper* c, const float* features_dev, int
             const EncLayer& L = c->enc[li];
             launch_layernorm(h.p, x.p, L.ln1w, L.ln1b, m, d, LN_EPS, s);
             g = BigGemmParams{x.p, L.wqkv, L.bqkv, nullptr, qkv.p, m, 3 * d, d, d, 0};
-            launch_gemm_big(BG_NONE, g, s);
-            launch_scatter_kv(qkv.p, 3 * d, d, 2 * d, kc.p, vc.p, nb, 1500, H, D, c->Spad, s);
+            g.kc = kc.p; g.vc = vc.p; g.kcol0 = d; g.vcol0 = 2 * d; g.T = 1500; g.H = H; g.Spad = c->Spad;
+            if (D != 64 || !launch_gemm_big_kv(g, s)) {
+                launch_gemm_big(BG_NONE, g, s);
+                launch_scatter_kv(qkv.p, 3 * d, d, 2 * d, kc.p, vc.p, nb, 1500, H, D, c->Spad, s);
+            }
             launch_attn_prefill(qkv.p, 3 * d, kc.p, vc.p, att.p, d, nb, 1500, H, D, c->Spad, s);
             g = BigGemmParams{att.p, L.wo, L.bo, h.p, h.p, m, d, d, d, 0};
             launch_gemm_big(BG_RESID, g, s);                                   // h = h + out_proj(attn)
@@ -454,11 +460,12 @@ static void whisper_encode_device(mis_whisper* c, const float* features_dev, int
         for (size_t li = 0; li < c->dec.size(); ++li) {
             const DecLayer& L = c->dec[li];
             g = BigGemmParams{eo, L.ckv, L.cbkv, nullptr, ckv.p, m, 2 * d, d, d, 0};
-            launch_gemm_big(BG_NONE, g, s);
-            size_t lstride = (size_t)c->batch * c->Hd * c->Spad * D;
-            size_t boff = (size_t)b0 * c->Hd * c->Spad * D;
-            launch_scatter_kv(ckv.p, 2 * d, 0, d, c->cross_k.p + li * lstride + boff, c->cross_v.p + li * lstride + boff, nb, 1500,
-                              c->Hd, D, c->Spad, s);
+            const size_t at = (li * c->batch + b0) * (size_t)c->Hd * c->Spad * D;
+            g.kc = c->cross_k.p + at; g.vc = c->cross_v.p + at; g.kcol0 = 0; g.vcol0 = d; g.T = 1500; g.H = c->Hd; g.Spad = c->Spad;
+            if (D != 64 || !launch_gemm_big_kv(g, s)) {
+                launch_gemm_big(BG_NONE, g, s);
+                launch_scatter_kv(ckv.p, 2 * d, 0, d, g.kc, g.vc, nb, 1500, c->Hd, D, c->Spad, s);
+            }
         }
         HIP_CHECK(hipGetLastError());
     }

@@ -273,6 +273,10 @@ __global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
     }
     const int n0 = ni * BG3_BN, m0 = mi * BG3_BM;
     const int wn = wave / WM, wm = wave % WM;
+    // Value tiles of BG_KV swap the operands: a lane then holds four consecutive KEYS of one dim, which are one 8-byte piece of the value image (two bytes each
+    // the other way round).  The tile is square, so only the sources and the epilogue differ; the products and their order do not.
+    // (8 windows: q|k|v 134 us, cross k|v 86 us, where GEMM and scatter kernel took 139 + 20 and 89 + 20)
+    const bool swp = EPI == BG_KV && n0 >= p.vcol0;
     f32x4_t acc[TN][TM];
 #pragma unroll
     for (int i = 0; i < TN; ++i)
@@ -284,13 +288,13 @@ __global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
     for (int q = 0; q < QW; ++q) {
         const int r = (wave * QW + q) * 8 + (lane >> 3);
         const int chunk = (lane & 7) ^ ((r >> 1) & 7);
-        wsrc[q] = p.W + (size_t)min(n0 + r, p.N - 1) * p.K + chunk * 8;
+        wsrc[q] = swp ? p.X + (size_t)min(m0 + r, p.M - 1) * p.ldx + chunk * 8 : p.W + (size_t)min(n0 + r, p.N - 1) * p.K + chunk * 8;
     }
 #pragma unroll
     for (int q = 0; q < QX; ++q) {
         const int r = (wave * QX + q) * 8 + (lane >> 3);
         const int chunk = (lane & 7) ^ ((r >> 1) & 7);
-        xsrc[q] = p.X + (size_t)min(m0 + r, p.M - 1) * p.ldx + chunk * 8;
+        xsrc[q] = swp ? p.W + (size_t)min(n0 + r, p.N - 1) * p.K + chunk * 8 : p.X + (size_t)min(m0 + r, p.M - 1) * p.ldx + chunk * 8;
     }
     auto stage = [&](int buf, int k0) {
 #pragma unroll
@@ -336,6 +340,50 @@ __global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
             for (int i = 0; i < TN; ++i)
 #pragma unroll
                 for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[ks][i], b[ks][j], acc[i][j], 0, 0, 0);
+        }
+    }
+    if constexpr (EPI == BG_KV) {
+        auto pack4 = [](const f32x4_t& v, float b0, float b1, float b2, float b3) {
+            uint2 o;
+            o.x = (uint32_t)f32_to_bf16(v[0] + b0) | ((uint32_t)f32_to_bf16(v[1] + b1) << 16);
+            o.y = (uint32_t)f32_to_bf16(v[2] + b2) | ((uint32_t)f32_to_bf16(v[3] + b3) << 16);
+            return o;
+        };
+        if (swp) {                                       // rows of the tile: keys; lane & 15: dim.  Image [D/16][64 lanes][8]: lane (key / 8) 16 + d & 15, key & 7
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const int m = m0 + wn * (BG3_BN / WN) + i * 16 + (lane >> 4) * 4;
+                if (m >= p.M) continue;                  // (M and T are multiples of 4: four keys share a batch row and a piece)
+                const int br = m / p.T, t = m - br * p.T, pr = t & 31;
+#pragma unroll
+                for (int j = 0; j < TM; ++j) {
+                    const int dd = n0 - p.vcol0 + wm * (BG3_BM / WM) + j * 16 + (lane & 15), hd = dd >> 6, d = dd & 63;
+                    const float bv = p.bias ? bf16_to_f32(p.bias[p.vcol0 + dd]) : 0.0f;
+                    bf16_t* o = p.vc + (((size_t)br * p.H + hd) * p.Spad + (t & ~31)) * 64 + (d >> 4) * 512 + ((pr >> 3) * 16 + (d & 15)) * 8 + (pr & 7);
+                    *reinterpret_cast<uint2*>(o) = pack4(acc[i][j], bv, bv, bv, bv);
+                }
+            }
+            return;
+        }
+        if (n0 >= p.kcol0) {                             // image [2][D/32][64 lanes][8]: the key permutation of k_scatter_kv
+#pragma unroll
+            for (int j = 0; j < TM; ++j) {
+                const int m = m0 + wm * (BG3_BM / WM) + j * 16 + (lane & 15);
+                if (m >= p.M) continue;
+                const int br = m / p.T, t = m - br * p.T, pr = t & 31, prow = ((pr >> 3) << 2) | (pr & 3), half = (pr >> 2) & 1;
+#pragma unroll
+                for (int i = 0; i < TN; ++i) {
+                    const int dd = n0 - p.kcol0 + wn * (BG3_BN / WN) + i * 16 + (lane >> 4) * 4, hd = dd >> 6, d = dd & 63;
+                    float bv[4] = {0.f, 0.f, 0.f, 0.f};
+                    if (p.bias) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) bv[e] = bf16_to_f32(p.bias[p.kcol0 + dd + e]);
+                    }
+                    bf16_t* o = p.kc + (((size_t)br * p.H + hd) * p.Spad + (t & ~31)) * 64 + (half * 2 + (d >> 5)) * 512 + (((d & 31) >> 3) * 16 + prow) * 8 + (d & 7);
+                    *reinterpret_cast<uint2*>(o) = pack4(acc[i][j], bv[0], bv[1], bv[2], bv[3]);
+                }
+            }
+            return;
         }
     }
     // epilogue: as k_gemm_big2 (C/D lane = column m (l & 15), rows n = 4 (l >> 4) + e)
@@ -388,6 +436,15 @@ template <int EPI>
 static bool launch_big3(const BigGemmParams& p, hipStream_t s) {
     // wave grid as measured: 2 (m) x 4 (n) for the wide / deep MLP shapes, 4 x 2 otherwise
     return (p.N >= 4096 || p.K >= 4096) ? launch_big3_one<EPI, 2, 4>(p, s) : launch_big3_one<EPI, 4, 2>(p, s);
+}
+
+bool launch_gemm_big_kv(const BigGemmParams& p, hipStream_t s) {
+    const char* e3 = getenv("MIS_GEMM_BIG3");
+    const int mode = e3 ? atoi(e3) : 1;
+    // key and value columns start at tile boundaries; pieces of four keys stay inside a batch row
+    if (mode == 0 || p.K % BG2_BK != 0 || p.K < 2 * BG2_BK || (mode != 2 && (long)cdiv(p.N, BG3_BN) * cdiv(p.M, BG3_BM) < 200)) return false;
+    if (p.ldx % 8 || p.kcol0 % BG3_BN || p.vcol0 % BG3_BN || p.N % BG3_BN || p.T % 4 || p.M % 4 || p.Spad % 32) return false;
+    return launch_big3<BG_KV>(p, s);
 }
 
 void launch_gemm_big(int epi, const BigGemmParams& p, hipStream_t s) {

@@ -455,3 +455,23 @@ def test_encoder_attention_when_the_maximum_moves_from_tile_to_tile():
     for g, r in zip(got, oracle.encode(feats)):
         r = r.numpy()
         assert np.isfinite(g).all() and np.sqrt(np.mean((g - r) ** 2)) <= 0.05 * np.sqrt(np.mean(r ** 2))
+
+
+def test_key_value_tiles_from_the_256x256_gemm_equal_the_scatter_kernel(monkeypatch):
+    """`launch_gemm_big_kv` writes keys and values straight as cache tiles (value tiles with swapped operands: the same products in the same order) where
+    `MIS_GEMM_BIG3=0` runs a plain GEMM and `k_scatter_kv`: encoder output and teacher-forced decoder logits equal bit for bit, with batches that change the
+    cache layout in between (padded keys are cleared with the layout, not on each encode)."""
+    cfg = ow.WhisperConfig(vocab_size=700, num_mel_bins=128, d_model=256, encoder_layers=2, encoder_attention_heads=4, encoder_ffn_dim=512,
+                           decoder_layers=2, decoder_attention_heads=4, decoder_ffn_dim=512)
+    dev = mas.WhisperModel.synthetic(_host_cfg(cfg), seed=17)
+    for B in (3, 1, 2, 2):
+        feats = _feats(B, cfg.num_mel_bins, 20 + B)
+        toks = np.random.default_rng(B).integers(0, cfg.vocab_size, (B, 4))
+        got = {}
+        for big in ("0", "2"):
+            monkeypatch.setenv("MIS_GEMM_BIG3", big)
+            enc = dev.encode(feats)
+            dev.decoder_reset()
+            got[big] = enc, np.stack([dev.decoder_forward(toks[:, t]) for t in range(toks.shape[1])])
+        for a, b in zip(got["0"], got["2"]):
+            assert np.isfinite(b).all() and np.abs(b).max() > 0 and np.array_equal(a, b), B
