@@ -116,6 +116,104 @@ struct PfGemmParams {
     PfExtra ex;           // the epilogues of layer-list models (lm_blocks.hip)
 };
 
+// epilogue of TN x TM MFMA tiles, the first at W rows 16 tile0 and X rows m0
+template <int EPI, int TN, int TM>
+__device__ __forceinline__ void pf_epilogue(const PfGemmParams& p, const f32x4_t (&acc)[TN][TM], int tile0, int m0, int lane) {
+    // epilogue.  C/D lane l, reg e: W row (n) = 16*tile + (l >> 4)*4 + e, X row (m) = l & 15
+    const int nl = (lane >> 4) * 4, NT = p.N >> 4;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+        const int m = m0 + j * 16 + (lane & 15);
+        if (m >= p.M) continue;
+        if (EPI == PF_SILU || EPI == PF_SWIGLU) {
+            bf16_t* act = reinterpret_cast<bf16_t*>(p.C);
+            const int ff = p.N >> 1;
+#pragma unroll
+            for (int i = 0; i + 1 < TN; i += 2) {             // tile pair (gate, up) -> feature tile
+                const int tile = tile0 + i;
+                if (tile + 1 >= NT) continue;             // (tile, tile + 1) = (gate, up) of feature tile `tile >> 1`
+                uint16_t res[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (EPI == PF_SWIGLU) {
+                        const float gf = acc[i][j][e];
+                        res[e] = f32_to_bf16(gf / (1.0f + __expf(-gf)) * acc[i + 1][j][e]);
+                        continue;
+                    }
+                    const float g = bf16_round_f32(acc[i][j][e]);
+                    const float u = bf16_round_f32(acc[i + 1][j][e]);
+                    const float sg = bf16_round_f32(1.0f / (1.0f + __expf(-g)));
+                    const float av = bf16_round_f32(g * sg);
+                    res[e] = f32_to_bf16(av * u);
+                }
+                uint2 v;
+                v.x = (uint32_t)res[0] | ((uint32_t)res[1] << 16);
+                v.y = (uint32_t)res[2] | ((uint32_t)res[3] << 16);
+                *reinterpret_cast<uint2*>(act + (size_t)m * ff + (tile >> 1) * 16 + nl) = v;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const int tile = tile0 + i;
+                if (tile >= NT) continue;
+                const int n = tile * 16 + nl;
+                if constexpr (EPI >= PF_SPLIT_RELU2 && EPI != PF_SWIGLU) {
+                    float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
+                    float* c32 = reinterpret_cast<float*>(p.C) + (size_t)m * p.ex.ldc + n;
+                    if (EPI == PF_ACT_ROWS) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float sg = 1.0f / (1.0f + __expf(-v[e]));
+                            v[e] = tile < p.ex.split ? v[e] * sg : sg;
+                        }
+                        *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.C) + (size_t)m * p.ex.ldc + n) =
+                            make_uint2((uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16), (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16));
+                    } else if (EPI == PF_ROWS_BF16 || (EPI == PF_SPLIT_RELU2 && tile >= p.ex.split)) {
+                        uint16_t res[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if (EPI == PF_SPLIT_RELU2) { const float t = fmaxf(v[e], 0.0f); v[e] = t * t; }
+                            res[e] = f32_to_bf16(v[e]);
+                        }
+                        bf16_t* o = EPI == PF_ROWS_BF16 ? reinterpret_cast<bf16_t*>(p.C) + (size_t)m * p.ex.ldc + n
+                                                        : reinterpret_cast<bf16_t*>(p.ex.out2) + (size_t)m * p.ex.ld2 + (n - p.ex.split * 16);
+                        *reinterpret_cast<uint2*>(o) = make_uint2((uint32_t)res[0] | ((uint32_t)res[1] << 16), (uint32_t)res[2] | ((uint32_t)res[3] << 16));
+                    } else if (EPI == PF_SCALED_ADD) {
+                        const uint2 lw = *reinterpret_cast<const uint2*>(p.ex.ls + n);
+                        const float l[4] = {bf16_to_f32((bf16_t)(lw.x & 0xffffu)), bf16_to_f32((bf16_t)(lw.x >> 16)), bf16_to_f32((bf16_t)(lw.y & 0xffffu)),
+                                            bf16_to_f32((bf16_t)(lw.y >> 16))};
+                        const float4 o = *reinterpret_cast<const float4*>(c32);
+                        *reinterpret_cast<float4*>(c32) = make_float4(o.x + l[0] * v[0], o.y + l[1] * v[1], o.z + l[2] * v[2], o.w + l[3] * v[3]);
+                    } else {
+                        if (EPI == PF_SOFTCAP) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) { const float t = v[e] * p.ex.scale; v[e] = p.ex.cap > 0.0f ? p.ex.cap * tanhf(t / p.ex.cap) : t; }
+                        }
+                        *reinterpret_cast<float4*>(c32) = make_float4(v[0], v[1], v[2], v[3]);
+                    }
+                } else if (EPI == PF_F32) {
+                    *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.C) + (size_t)m * p.N + n) =
+                        make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+                } else {
+                    bf16_t* h = reinterpret_cast<bf16_t*>(p.C) + (size_t)m * p.N + n;
+                    const uint2 old = *reinterpret_cast<const uint2*>(h);
+                    const uint32_t ow[2] = {old.x, old.y};
+                    uint16_t res[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float hv = bf16_to_f32((bf16_t)((ow[e >> 1] >> (16 * (e & 1))) & 0xffffu));
+                        res[e] = f32_to_bf16(hv + bf16_round_f32(acc[i][j][e]));                  // h = T(h + T(x W^T))
+                    }
+                    uint2 v;
+                    v.x = (uint32_t)res[0] | ((uint32_t)res[1] << 16);
+                    v.y = (uint32_t)res[2] | ((uint32_t)res[3] << 16);
+                    *reinterpret_cast<uint2*>(h) = v;
+                }
+            }
+        }
+    }
+}
+
 template <int EPI>
 __global__ void __launch_bounds__(256, 2) k_gemm_pf(PfGemmParams p) {
     __shared__ __attribute__((aligned(1024))) bf16_t Ws[2][PF_BN * PF_BK];
@@ -182,99 +280,84 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf(PfGemmParams p) {
                 for (int j = 0; j < 4; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
     }
-    // epilogue.  C/D lane l, reg e: W row (n) = 16*tile + (l >> 4)*4 + e, X row (m) = l & 15
-    const int nl = (lane >> 4) * 4;
+    pf_epilogue<EPI, 4, 4>(p, acc, (n0 >> 4) + wn * 4, m0 + wm * 64, lane);
+}
+
+// Few rows: k_gemm_pf waits 0.6 us for each of its 48 - 128 k-steps, and a short prompt's 24 - 128 tiles of 128 x 128 leave most of the chip idle meanwhile.
+// Tiles of 32 rows x 32 columns (gate | up: 64, the pairs of a wave) on two waves, with a ring of NBUF k-steps in LDS requested ahead under counted waits: bound
+// by the weights' way from memory.  The same MFMA instruction and k order: the bits of k_gemm_pf.  Orpheus-3B, us per launch, k_gemm_pf / here: 24 rows:
+// o and down 81 / 17, q|k|v 44 / 12, gate | up 48 / 20; 60 rows: 83 / 17, 45 / 18, 49 / 35; 120 rows: 88 / 30, 50 / 26, 54 / 64.
+// (The ring on 128 x 128 tiles: 79 for 83 us with o and down at 1024 rows, 83 for 51 with q|k|v.)
+template <int EPI, int TN, int NBUF>
+__global__ void __launch_bounds__(128) k_gemm_pf_ring(PfGemmParams p) {
+    constexpr int WN = 2, WM = 1, TM = 2, NW = WN * WM, BN = WN * TN * 16, BM = WM * TM * 16, QW = WN * TN * 2 / NW, QX = WM * TM * 2 / NW, NQ = QW + QX;   // DMA instructions per wave and k-step
+    constexpr int WB = WN * TN * 2048, STEP = WB + WM * TM * 2048;                                                        // bytes
+    static_assert((NBUF - 2) * NQ <= 63 && QW * NW == WN * TN * 2 && QX * NW == WM * TM * 2, "vmcnt; whole DMA instructions");
+    __shared__ __attribute__((aligned(1024))) unsigned char ring[NBUF * STEP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wave / WM, wm = wave % WM;
+    const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM, NT = p.N >> 4, KT = p.K >> 5, KS = p.K / PF_BK;
+    f32x4_t acc[TN][TM];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int m = m0 + wm * 64 + j * 16 + (lane & 15);
-        if (m >= p.M) continue;
-        if (EPI == PF_SILU || EPI == PF_SWIGLU) {
-            bf16_t* act = reinterpret_cast<bf16_t*>(p.C);
-            const int ff = p.N >> 1;
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
-            for (int i = 0; i < 4; i += 2) {             // tile pair (gate, up) -> feature tile
-                const int tile = (n0 >> 4) + wn * 4 + i;
-                if (tile + 1 >= NT) continue;             // (tile, tile + 1) = (gate, up) of feature tile `tile >> 1`
-                uint16_t res[4];
+        for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const bf16_t *wsrc[QW], *xsrc[QX];                  // the staging of k_gemm_pf: W fragments as they are, X rows with swizzled 16-byte pieces
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (EPI == PF_SWIGLU) {
-                        const float gf = acc[i][j][e];
-                        res[e] = f32_to_bf16(gf / (1.0f + __expf(-gf)) * acc[i + 1][j][e]);
-                        continue;
-                    }
-                    const float g = bf16_round_f32(acc[i][j][e]);
-                    const float u = bf16_round_f32(acc[i + 1][j][e]);
-                    const float sg = bf16_round_f32(1.0f / (1.0f + __expf(-g)));
-                    const float av = bf16_round_f32(g * sg);
-                    res[e] = f32_to_bf16(av * u);
-                }
-                uint2 v;
-                v.x = (uint32_t)res[0] | ((uint32_t)res[1] << 16);
-                v.y = (uint32_t)res[2] | ((uint32_t)res[3] << 16);
-                *reinterpret_cast<uint2*>(act + (size_t)m * ff + (tile >> 1) * 16 + nl) = v;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int tile = (n0 >> 4) + wn * 4 + i;
-                if (tile >= NT) continue;
-                const int n = tile * 16 + nl;
-                if constexpr (EPI >= PF_SPLIT_RELU2 && EPI != PF_SWIGLU) {
-                    float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-                    float* c32 = reinterpret_cast<float*>(p.C) + (size_t)m * p.ex.ldc + n;
-                    if (EPI == PF_ACT_ROWS) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float sg = 1.0f / (1.0f + __expf(-v[e]));
-                            v[e] = tile < p.ex.split ? v[e] * sg : sg;
-                        }
-                        *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.C) + (size_t)m * p.ex.ldc + n) =
-                            make_uint2((uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16), (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16));
-                    } else if (EPI == PF_ROWS_BF16 || (EPI == PF_SPLIT_RELU2 && tile >= p.ex.split)) {
-                        uint16_t res[4];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            if (EPI == PF_SPLIT_RELU2) { const float t = fmaxf(v[e], 0.0f); v[e] = t * t; }
-                            res[e] = f32_to_bf16(v[e]);
-                        }
-                        bf16_t* o = EPI == PF_ROWS_BF16 ? reinterpret_cast<bf16_t*>(p.C) + (size_t)m * p.ex.ldc + n
-                                                        : reinterpret_cast<bf16_t*>(p.ex.out2) + (size_t)m * p.ex.ld2 + (n - p.ex.split * 16);
-                        *reinterpret_cast<uint2*>(o) = make_uint2((uint32_t)res[0] | ((uint32_t)res[1] << 16), (uint32_t)res[2] | ((uint32_t)res[3] << 16));
-                    } else if (EPI == PF_SCALED_ADD) {
-                        const uint2 lw = *reinterpret_cast<const uint2*>(p.ex.ls + n);
-                        const float l[4] = {bf16_to_f32((bf16_t)(lw.x & 0xffffu)), bf16_to_f32((bf16_t)(lw.x >> 16)), bf16_to_f32((bf16_t)(lw.y & 0xffffu)),
-                                            bf16_to_f32((bf16_t)(lw.y >> 16))};
-                        const float4 o = *reinterpret_cast<const float4*>(c32);
-                        *reinterpret_cast<float4*>(c32) = make_float4(o.x + l[0] * v[0], o.y + l[1] * v[1], o.z + l[2] * v[2], o.w + l[3] * v[3]);
-                    } else {
-                        if (EPI == PF_SOFTCAP) {
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) { const float t = v[e] * p.ex.scale; v[e] = p.ex.cap > 0.0f ? p.ex.cap * tanhf(t / p.ex.cap) : t; }
-                        }
-                        *reinterpret_cast<float4*>(c32) = make_float4(v[0], v[1], v[2], v[3]);
-                    }
-                } else if (EPI == PF_F32) {
-                    *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.C) + (size_t)m * p.N + n) =
-                        make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
-                } else {
-                    bf16_t* h = reinterpret_cast<bf16_t*>(p.C) + (size_t)m * p.N + n;
-                    const uint2 old = *reinterpret_cast<const uint2*>(h);
-                    const uint32_t ow[2] = {old.x, old.y};
-                    uint16_t res[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float hv = bf16_to_f32((bf16_t)((ow[e >> 1] >> (16 * (e & 1))) & 0xffffu));
-                        res[e] = f32_to_bf16(hv + bf16_round_f32(acc[i][j][e]));                  // h = T(h + T(x W^T))
-                    }
-                    uint2 v;
-                    v.x = (uint32_t)res[0] | ((uint32_t)res[1] << 16);
-                    v.y = (uint32_t)res[2] | ((uint32_t)res[3] << 16);
-                    *reinterpret_cast<uint2*>(h) = v;
-                }
-            }
-        }
+    for (int q = 0; q < QW; ++q) {
+        const int f = wave * QW + q;
+        wsrc[q] = p.Wp + ((size_t)min((n0 >> 4) + (f >> 1), NT - 1) * KT + (f & 1)) * 512 + lane * 8;
     }
+#pragma unroll
+    for (int q = 0; q < QX; ++q) {
+        const int r = (wave * QX + q) * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7), xm = min(m0 + r, p.M - 1);
+        if constexpr (EPI == PF_ROWS_BF16) xsrc[q] = p.X + (size_t)(p.ex.xrow ? p.ex.xrow[xm] : xm) * p.ex.ldx + chunk * 8;
+        else xsrc[q] = p.X + (size_t)xm * p.K + chunk * 8;
+    }
+    auto stage = [&](int buf, int ks) {
+        unsigned char* l = ring + buf * STEP;
+#pragma unroll
+        for (int q = 0; q < QW; ++q)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wsrc[q] + (size_t)ks * 1024),
+                                             (__attribute__((address_space(3))) void*)(l + (wave * QW + q) * 1024), 16, 0, 0);
+#pragma unroll
+        for (int q = 0; q < QX; ++q)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xsrc[q] + ks * PF_BK),
+                                             (__attribute__((address_space(3))) void*)(l + WB + (wave * QX + q) * 1024), 16, 0, 0);
+    };
+    const int sw = (lane >> 1) & 7;
+    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)ring;
+    const uint32_t wa = base + wn * TN * 2048 + lane * 16, xa = base + WB + wm * TM * 2048 + (lane & 15) * 128;
+    const uint32_t x0 = xa + ((lane >> 4) ^ sw) * 16, x1 = xa + ((4 + (lane >> 4)) ^ sw) * 16;
+    for (int i = 0; i < NBUF - 1; ++i) stage(i, min(i, KS - 1));
+    int rd = 0, wr = NBUF - 1;
+    for (int ks = 0; ks < KS; ++ks) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * NQ) : "memory");      // this wave's part of k-step ks has landed
+        __builtin_amdgcn_s_barrier();                                               // everybody's; the slot read one step ago is free
+        const uint32_t o = rd * STEP;
+        bf16x8_t a[2][TN], b[2][TM];
+        // fragment reads and their wait in one block: behind an LDS-DMA the compiler would wait for every load in flight (see k_gemm_big3)
+        if constexpr (TN == 1)
+            asm volatile("ds_read_b128 %0, %6\n ds_read_b128 %1, %6 offset:1024\n ds_read_b128 %2, %7\n ds_read_b128 %3, %7 offset:2048\n"
+                         "ds_read_b128 %4, %8\n ds_read_b128 %5, %8 offset:2048\n s_waitcnt lgkmcnt(0)"
+                         : "=&v"(a[0][0]), "=&v"(a[1][0]), "=&v"(b[0][0]), "=&v"(b[0][1]), "=&v"(b[1][0]), "=&v"(b[1][1])
+                         : "v"(wa + o), "v"(x0 + o), "v"(x1 + o) : "memory");
+        else
+            asm volatile("ds_read_b128 %0, %8\n ds_read_b128 %1, %8 offset:1024\n ds_read_b128 %2, %8 offset:2048\n ds_read_b128 %3, %8 offset:3072\n"
+                         "ds_read_b128 %4, %9\n ds_read_b128 %5, %9 offset:2048\n ds_read_b128 %6, %10\n ds_read_b128 %7, %10 offset:2048\n s_waitcnt lgkmcnt(0)"
+                         : "=&v"(a[0][0]), "=&v"(a[1][0]), "=&v"(a[0][TN - 1]), "=&v"(a[1][TN - 1]), "=&v"(b[0][0]), "=&v"(b[0][1]), "=&v"(b[1][0]), "=&v"(b[1][1])
+                         : "v"(wa + o), "v"(x0 + o), "v"(x1 + o) : "memory");
+        stage(wr, min(ks + NBUF - 1, KS - 1));                                      // (past the end: the last step again, never read)
+        rd = rd + 1 == NBUF ? 0 : rd + 1;
+        wr = wr + 1 == NBUF ? 0 : wr + 1;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][i], b[kk][j], acc[i][j], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                // (no DMA into the LDS of a block that has ended)
+    pf_epilogue<EPI, TN, TM>(p, acc, (n0 >> 4) + wn * TN, m0 + wm * TM * 16, lane);
 }
 
 void launch_gemm_pf(int epi, const bf16_t* X, const bf16_t* Wp, void* C, int M, int N, int K, hipStream_t s, const PfExtra& ex) {
@@ -283,6 +366,18 @@ void launch_gemm_pf(int epi, const bf16_t* X, const bf16_t* Wp, void* C, int M, 
     MIS_REQUIRE(epi < PF_SPLIT_RELU2 || epi == PF_SWIGLU || (ex.ldc % 4 == 0 && (epi != PF_ROWS_BF16 || ex.ldx % 8 == 0)), MIS_ERR_GENERATION_FAILED,
                 "prefill GEMM: bad row strides");
     PfGemmParams p{X, Wp, C, M, N, K, ex};
+    // Few blocks of the small tile (the larger one reads a weight tile once per 128 rows, not per 32).  o and down at 240 / 400 rows (768 / 1248 blocks): 44 / 71
+    // against 85 / 82 us; q|k|v at 240 / 400 (1280 / 2080): 43 / 70 against 48 / 45; gate | up at 60 / 120 (512 / 1024): 35 / 64 against 49 / 54.
+    auto few = [&](auto e) {
+        constexpr int E = decltype(e)::value, TN = E == PF_SILU ? 2 : 1;
+        if ((int64_t)cdiv(N, 32 * TN) * cdiv(M, 32) > (TN == 2 ? 512 : 1280)) return false;
+        hipLaunchKernelGGL((k_gemm_pf_ring<E, TN, TN == 2 ? 12 : 16>), dim3(cdiv(N, 32 * TN), cdiv(M, 32)), dim3(128), 0, s, p);
+        return true;
+    };
+    if (epi == PF_F32 && few(std::integral_constant<int, PF_F32>{})) return;
+    if (epi == PF_RESID && few(std::integral_constant<int, PF_RESID>{})) return;
+    if (epi == PF_SILU && few(std::integral_constant<int, PF_SILU>{})) return;
+    if (epi == PF_ROWS_BF16 && few(std::integral_constant<int, PF_ROWS_BF16>{})) return;
     // column tiles rounded up to the 8 XCDs: blocks are dealt to the XCDs by linear id, so that every row of tiles finds its weight tiles in the
     // L2 that held them for the row before
     const int nx = cdiv(N, PF_BN);
