@@ -252,7 +252,7 @@ __device__ __forceinline__ bf16x8_t bg3_lds_read16(uint32_t addr) {
 #define BG3_BM 256
 #define BG3_BN 256
 template <int EPI, int WM, int WN>
-__global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
+__device__ __forceinline__ void gemm_big3_body(const BigGemmParams& p) {
     constexpr int NW = WM * WN;                                  // 8 waves
     constexpr int TM = BG3_BM / WM / 16, TN = BG3_BN / WN / 16;  // 16 x 16 MFMA tiles per wave (m, n)
     constexpr int QW = BG3_BN / 8 / NW, QX = BG3_BM / 8 / NW;    // LDS-DMA instructions per wave and tile (8 rows of 128 B each)
@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
     const int wn = wave / WM, wm = wave % WM;
     // Value tiles of BG_KV swap the operands: a lane then holds four consecutive KEYS of one dim, which are one 8-byte piece of the value image (two bytes each
     // the other way round).  The tile is square, so only the sources and the epilogue differ; the products and their order do not.
-    // (8 windows: q|k|v 134 us, cross k|v 86 us, where GEMM and scatter kernel took 139 + 20 and 89 + 20)
+    // (k_gemm_kv_tiles, 8 windows: q|k|v 134 us, cross k|v 86 us, where GEMM and scatter kernel took 139 + 20 and 89 + 20)
     const bool swp = EPI == BG_KV && n0 >= p.vcol0;
     f32x4_t acc[TN][TM];
 #pragma unroll
@@ -424,12 +424,19 @@ __global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) {
     }
 }
 template <int EPI, int WM, int WN>
+__global__ void __launch_bounds__(512, 1) k_gemm_big3(BigGemmParams p) { gemm_big3_body<EPI, WM, WN>(p); }
+template <int WM, int WN>
+__global__ void __launch_bounds__(512, 1) k_gemm_kv_tiles(BigGemmParams p) { gemm_big3_body<BG_KV, WM, WN>(p); }
+template <int EPI, int WM, int WN>
 static bool launch_big3_one(const BigGemmParams& p, hipStream_t s) {
     constexpr int lds_bytes = 2 * (BG3_BM + BG3_BN) * BG2_BK * 2;            // 128 KB
-    static const bool ok = hipFuncSetAttribute((const void*)k_gemm_big3<EPI, WM, WN>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
+    void (*kernel)(BigGemmParams);
+    if constexpr (EPI == BG_KV) kernel = k_gemm_kv_tiles<WM, WN>;
+    else kernel = k_gemm_big3<EPI, WM, WN>;
+    static const bool ok = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) == hipSuccess;
     if (!ok) { (void)hipGetLastError(); return false; }
     const int nt = cdiv(p.N, BG3_BN), mt = cdiv(p.M, BG3_BM);
-    hipLaunchKernelGGL((k_gemm_big3<EPI, WM, WN>), dim3(nt <= 8 ? 8 * nt * cdiv(mt, 8) : nt * mt), dim3(512), lds_bytes, s, p);
+    hipLaunchKernelGGL(kernel, dim3(nt <= 8 ? 8 * nt * cdiv(mt, 8) : nt * mt), dim3(512), lds_bytes, s, p);
     return true;
 }
 template <int EPI>
