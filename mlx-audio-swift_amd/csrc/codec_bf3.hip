@@ -5,8 +5,8 @@
 // xh = bf16(x), xl = bf16(x - xh) (relative error of the pair <= 2^-18), and a product becomes three bf16 MFMAs accumulated in f32:
 // xh.wh + xh.wl + xl.wh (the lo.lo term, <= 2^-16 of the product, is dropped).  Measured on the CPU emulation of exactly this
 // arithmetic inside the SNAC oracle (tools/bf16x3_emulation.py, profiles/r02_bf16x3_emulation.json): 1.06e-5 RMS on the 24 kHz decode
-// against the 1e-4 gate (plain bf16: 5.7e-3).  The exact-f32 kernels of snac.hip stay: encoders (codebook decisions), small or
-// memory-bound shapes, and MIS_CODEC_EXACT_F32=1.
+// against the 1e-4 gate (plain bf16: 5.7e-3).  The f32-accurate kernels (codec_x6.hip, codec_f32.hip, snac.hip) stay: encoders (codebook
+// decisions), small or memory-bound shapes, and MIS_CODEC_EXACT_F32=1.
 //
 // Three kernels:
 //   k_bf3_pack_w   A^T f32 [taps][Cin][M] -> MFMA-A fragments of v_mfma_f32_32x32x16_bf16, hi and lo, [tap][M/32][Cp/16][hl][64][8]

@@ -4,8 +4,8 @@
 // DescriptDecoder / DescriptDecoderBlock / DescriptResidualUnit (:7-32,103-160), DescriptResidualVectorQuantize.fromCodes
 // (DescriptQuantization.swift:150-163), weight-normalised convs (BigVGAN/BigVGANLayers.swift:113-225).  The reference keeps NLC
 // activations and recomputes the weight norm on every call; here weights are folded once (A^T per tap / per transposed-conv
-// phase, codebook x out_proj tables) and activations stay NCT.  Dense k7 dilated convs run on k_conv_taps, 1x1 convs and the
-// transposed convs on k_snac_convt (exact-f32 MFMA), Snake fused into the operand loads.
+// phase, codebook x out_proj tables) and activations stay NCT.  Dense k7 dilated convs and wide transposed convs run as
+// split-bf16 contractions (codec_bf3.hip), 1x1 convs and narrow transposed convs on codec_x6.hip / codec_f32.hip, Snake fused into the operand loads.
 // Encode (DescriptEncoder / DescriptEncoderBlock :40-95, preprocess + encode :216-233, DescriptVectorQuantize / residual loop
 // DescriptQuantization.swift:54-147): first conv k7, per block 3 residual units (the decoder's: dense dilated k7 on k_conv_taps + 1x1
 // with residual epilogue) then Snake + the stride-s conv (k = 2s, pad ceil(s/2)) as a 3-tap conv over the phase-split tensor, last
