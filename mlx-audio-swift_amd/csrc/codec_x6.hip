@@ -77,27 +77,27 @@ const CodecPack::X6& CodecPack::get_x6(const float* at, int ntaps, int Cin, int 
 // channels of a column per thread are split and written as one 16-byte piece per plane, [plane][channel / 8][column], which is the MFMA-B fragment.
 // What bounds it: k_pw_fused<128, DW> took 1.05 ms without its MFMAs (4.8 GB of loads and stores, 32 rows of 98304 columns) and 1.75 ms with: the f32
 // matrix time adds to the memory time.  Six bf16 products take 0.25 instead of 0.68 ms of it: 1.95 -> 1.44 ms.
-#define RU_NT 128
-#define RU_XS (RU_NT + 2 * CODEC_DW_HALO + 2)
 struct PwScalars { int T, dil, ldx, ldr, ldy; };
-template <int C, bool DW, int KC>
+template <int C, bool DW, int KC, int NT>
 __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                            const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
                                            const float* __restrict__ pra1, const float* __restrict__ pa2, const float* __restrict__ pra2,
                                            const uint16_t* __restrict__ pwp, const float* __restrict__ pb2, const PwScalars p) {
     constexpr int KG = KC / 8, MT = C / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
-    constexpr int XR = KC / 4, GS = KG * 2 / 4;                             // rows of x and (group, strip) pairs per wave
-    __shared__ float xs[DW ? KC : 1][DW ? RU_XS : 1];
-    __shared__ uint4 ts[3][KG][RU_NT];
+    constexpr int XR = KC / 4, GS = KG * (NT / 64) / 4, XS = NT + 2 * CODEC_DW_HALO + 2, NS = (XS + 61) / 64;      // (XS - 2 columns in strips of 64)
+                               // rows of x and (group, strip) pairs per wave
+    __shared__ float xs[DW ? KC : 1][DW ? XS : 1];
+    __shared__ uint4 ts[3][KG][NT];
     __shared__ uint4 As[APC];
     constexpr bool SQ = C == 128;                         // 2 x 2 waves of 64 x 64; else every wave: all C rows x 32 columns
-    constexpr int MTW = SQ ? 2 : MT, NTW = SQ ? 2 : 1;
+    constexpr int MTW = SQ ? 2 : MT, NTW = SQ ? NT / 64 : 1;
+    static_assert(SQ || NT == 128, "four waves of 32 columns");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * RU_NT, b = blockIdx.y;
+    const int n0 = blockIdx.x * NT, b = blockIdx.y;
     const int wr = SQ ? (wave >> 1) * 2 : 0;              // first row tile / first column of the wave's tile
-    const int wc = SQ ? (wave & 1) * 64 : wave * 32;
+    const int wc = SQ ? (wave & 1) * (NT / 2) : wave * 32;
     const float* xb = pX + (size_t)b * C * p.ldx;
-    const int T = p.T, halo = 3 * p.dil, ncols = RU_NT + 2 * halo;
+    const int T = p.T, halo = 3 * p.dil, ncols = NT + 2 * halo;
     f32x16_t acc[MTW][NTW];
 #pragma unroll
     for (int i = 0; i < MTW; ++i)
@@ -112,12 +112,12 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
         for (int i = 0; i < (APC + 255) / 256; ++i) wv[i] = wsrc[min(tid + i * 256, APC - 1)];
         if (DW) {
-            float v[XR][3];
+            float v[XR][NS];
 #pragma unroll
             for (int r = 0; r < XR; ++r) {
                 const int c = c0 + wave + 4 * r;
 #pragma unroll
-                for (int sx = 0; sx < 3; ++sx) {
+                for (int sx = 0; sx < NS; ++sx) {
                     const int j = sx * 64 + lane, t = n0 - halo + j;
                     const bool ok = j < ncols && t >= 0 && t < T;
                     v[r][sx] = xb[(size_t)c * p.ldx + (ok ? t : 0)];
@@ -129,9 +129,9 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                 const int cc = wave + 4 * r, c = c0 + cc;
                 const float al = pa1[c], ral = pra1[c];
 #pragma unroll
-                for (int sx = 0; sx < 3; ++sx) {
+                for (int sx = 0; sx < NS; ++sx) {
                     const int j = sx * 64 + lane;
-                    if (j < RU_XS) xs[cc][j] = x6_snake(v[r][sx], al, ral);
+                    if (j < XS) xs[cc][j] = x6_snake(v[r][sx], al, ral);
                 }
             }
         } else {
@@ -215,21 +215,26 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
             }
     }
 }
-template <int C, bool DW, int KC>
+template <int C, bool DW, int KC, int NT>
 __global__ void __launch_bounds__(256, KC == 32 ? 2 : C == 128 && DW ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp) {
-    pw_x6_body<C, DW, KC>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
+    pw_x6_body<C, DW, KC, NT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
 }
 
+// 128 channels, at most 256 blocks of 128 columns (a compute unit each, one serial chain of chunks): 64 columns per block.  96 blocks: 28 -> 22 us;
+// 192 and 248: 23 and 25 (384 of 128 columns: 34).  (The next chunk's loads ahead of this one's products instead: 31 us, no registers left.)
 // Chunk depth (the same bits): 32 channels need half the barriers, 16 let three or four blocks (not two, C = 96: three) share a compute unit.  32 while its
 // blocks are all resident at once, else 16 (us, chunks of 32 / 16): 128 channels 96 blocks 28 / 33, 384: 34 / 38, 576: 61 / 45, 24576: 1584 / 1430;
 // 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150.  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32.
 template <int C, bool DW>
 static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hipStream_t s) {
-    const dim3 grid((p.T + RU_NT - 1) / RU_NT, batch);
-    if constexpr (C <= 128) {
-        if ((int64_t)grid.x * batch > (C == 96 ? 768 : 512)) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16>), grid, dim3(256), 0, s, p, wp); return; }
+    const dim3 grid((p.T + 127) / 128, batch);
+    if constexpr (C == 128) {
+        if ((int64_t)grid.x * batch <= 256) { hipLaunchKernelGGL((k_pw_x6<C, DW, 32, 64>), dim3((p.T + 63) / 64, batch), dim3(256), 0, s, p, wp); return; }
     }
-    hipLaunchKernelGGL((k_pw_x6<C, DW, 32>), grid, dim3(256), 0, s, p, wp);
+    if constexpr (C <= 128) {
+        if ((int64_t)grid.x * batch > (C == 96 ? 768 : 512)) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16, 128>), grid, dim3(256), 0, s, p, wp); return; }
+    }
+    hipLaunchKernelGGL((k_pw_x6<C, DW, 32, 128>), grid, dim3(256), 0, s, p, wp);
 }
 
 // 64 channels stay on k_pw_fused: twice the columns per product, bound by memory and by the units' VALU work (1.16 ms here, 1.10 there)

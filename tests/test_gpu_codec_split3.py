@@ -1,4 +1,4 @@
-"""The three-plane contractions (csrc/codec_x6.hip) - the fused residual units: both chunk depths, 96 / 128 / 192 channels; the 1x1 and k-tap form: one to
+"""The three-plane contractions (csrc/codec_x6.hip) - the fused residual units: both column tiles and chunk depths, 96 / 128 / 192 channels; the 1x1 and k-tap form: one to
 eight row tiles per block; column and row remainders in both - as accurate as the exact-f32 kernels, and the same bits whatever batch (and with it tile or
 chunk depth) a row comes in."""
 import numpy as np
@@ -35,7 +35,7 @@ def check(dev, orc, codes, rows, pick):
 
 # decoder channels 128 (units), 256 and 128 (NoiseBlock); 384, 192, 96, 48 (1x1 residuals, and rows past a tile of 32)
 @pytest.mark.parametrize("dim", [256, 512, 768])
-@pytest.mark.parametrize("rows, groups", [(3, 5), (40, 60)], ids=["one-wave", "many"])
+@pytest.mark.parametrize("rows, groups", [(3, 5), (20, 60), (40, 60)], ids=["one-wave", "two-waves", "many"])
 def test_snac(no_bf3, dim, rows, groups):
     cfg = dict(encoder_dim=8, encoder_rates=[2, 2, 2, 8], decoder_dim=dim, decoder_rates=[8, 2, 2, 2], codebook_size=64, codebook_dim=8, vq_strides=[4, 2, 1])
     ocfg = osnac.SnacConfig(**cfg)
