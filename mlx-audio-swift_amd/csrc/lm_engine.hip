@@ -767,11 +767,12 @@ static bool prefill_batched_ok(const mis_tts* c, int Lmax) {
     return !off && Lmax >= 2 && (dense || coded) && c->d % 64 == 0 && HD % 64 == 0 && c->ff % 64 == 0 && c->d >= 128 && HD >= 128 && c->ff >= 128;
 }
 // ---- short prompts (positions x rows <= 64, dense weights): the DECODE STEP's kernels with (position, sequence) pairs as their rows.
-// k_gemm_pf works on 128 x 128 tiles: at 23 positions of one row its o_proj / down_proj grids are 4 blocks (21 us per launch on 256 CUs,
-// profiles/r05_final_soprano_engine_kernel_stats.csv: 1.4 ms to prefill 23 positions of Soprano-80M - 7 % of a batch-1 generate).  The
+// On the 128 x 128 tiles of k_gemm_pf the o_proj / down_proj grids of 23 positions are 4 blocks (21 us per launch on 256 CUs,
+// profiles/r05_final_soprano_engine_kernel_stats.csv: 1.4 ms to prefill 23 positions of Soprano-80M - 7 % of a batch-1 generate; k_gemm_pf_ring,
+// which such grids take now, was not there to compare).  The
 // weight-streaming GEMMs of the decode step take up to 64 rows, their glue does residual + RMSNorm and writes the packed operand, and the
 // attention kernel already has the pair arrangement (append-only launch, then every pair as a row; first schedule, like the chunked pass).
-// Same rounding points as both other prefill forms; float32 summation orders are the decode step's.  MIS_PREFILL_SMALL=0 keeps k_gemm_pf.
+// Same rounding points as both other prefill forms; float32 summation orders are the decode step's.  MIS_PREFILL_SMALL=0 keeps k_gemm_pf / k_gemm_pf_ring.
 __global__ void k_pf_repack_rows(const bf16_t* __restrict__ src, int MT_src, int row0, bf16_t* __restrict__ dst, int MT_dst, int d) {
     const int m = blockIdx.x;
     for (int k = threadIdx.x; k < d; k += blockDim.x) dst[xpk_index(m, k, MT_dst)] = src[xpk_index(row0 + m, k, MT_src)];
