@@ -28,7 +28,8 @@ typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));       //
 // One tile.  WM x WN waves; a wave holds TM x TN MFMA tiles of MS x MS (MS = 32 or 16); BK k per chunk; PF chunks requested ahead.
 // IN: the tile lies inside the output, its columns at every tap inside the input, M is a multiple of 4, the channels of 16 and the k units of the chunk -
 // nothing to clamp or mask.  Otherwise every element is clamped when it is loaded and masked when it is put into LDS.
-template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF, bool IN>
+// OFF: the type of an offset inside the tile's rows (see launch_f32).
+template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF, bool IN, typename OFF>
 __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int n0, int m0, int b, float* As, float* Xs, const float* __restrict__ pX, const float* __restrict__ pR,
                                                 float* __restrict__ pY, const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pAT) {
     constexpr int BM = WM * TM * MS, BN = WN * TN * MS, KS = MS == 32 ? 2 : 4;
@@ -56,8 +57,8 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
     };
     const std::integral_constant<int, BM / 4> pwa{};
     const std::integral_constant<int, BN / 4> pwx{};
-    // Addresses are a scalar base plus a 32-bit offset; loads are unconditional (a guarded load becomes a branch whose join waits for everything in flight)
-    auto at = [](const float* base, uint32_t off) { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off); };
+    // Addresses are a scalar base plus an offset (32 bits unless rows are very long); loads are unconditional (a guarded load becomes a branch whose join waits for everything in flight)
+    auto at = [](const float* base, OFF off) { return reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off); };
     float4 ra[PF][NA], rx[PF][NX];
     auto load = [&](int c, int slot) {
 #pragma unroll
@@ -79,7 +80,7 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
             unit(c, i, pwx, c16, tap);
             const int sh = taps ? tap * p.dil - p.pad : 0;
             if constexpr (IN) {
-                const f32x4u_t v = *reinterpret_cast<const f32x4u_t*>(at(Xb + (int64_t)c16 * p.ldx + n0 + sh, 4u * (uint32_t)(r * p.ldx + nl)));
+                const f32x4u_t v = *reinterpret_cast<const f32x4u_t*>(at(Xb + (int64_t)c16 * p.ldx + n0 + sh, 4 * ((OFF)r * p.ldx + nl)));
                 rx[slot][i] = make_float4(v[0], v[1], v[2], v[3]);
             } else {
                 const float* row = Xb + (int64_t)(c16 + min(r, Cin - 1 - c16)) * p.ldx;
@@ -175,7 +176,7 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
 #pragma unroll
                 for (int r = 0; r < NR; ++r) {
                     const int ml = i * MS + (MS == 32 ? (r & 3) + 8 * (r >> 2) : r) + row0;
-                    e[i][j][r] = add ? *at(eb, 4u * (uint32_t)((IN ? ml : min(ml, mtop)) * lde + (IN ? n : min(n, p.N - 1)))) : 0.0f;
+                    e[i][j][r] = add ? *at(eb, 4 * ((OFF)(IN ? ml : min(ml, mtop)) * lde + (IN ? n : min(n, p.N - 1)))) : 0.0f;
                 }
         }
     };
@@ -223,13 +224,13 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
                     if (add) v = e[i][j][r] + v;                                                    // Layers.swift:230
                 }
                 if (MODE == GEMM_NOISE) v = e[i][j][r] + nz * v;                                    // Layers.swift:276-277
-                if (IN || (nok && ml <= mtop && mw < p.M)) *const_cast<float*>(at(yb, 4u * (uint32_t)(ml * p.ldy + n))) = v;
+                if (IN || (nok && ml <= mtop && mw < p.M)) *const_cast<float*>(at(yb, 4 * ((OFF)ml * p.ldy + n))) = v;
             }
         }
     }
 }
-template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF>
-__global__ void __launch_bounds__(256, MS == 32 ? 3 : 1) k_codec_gemm(GemmParams p, F32Tiles q) {
+template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF, typename OFF>
+__global__ void __launch_bounds__(256, MS == 32 && sizeof(OFF) == 4 ? 3 : 1) k_codec_gemm(GemmParams p, F32Tiles q) {
     constexpr int BM = WM * TM * MS, BN = WN * TN * MS, LA = MS == 32 ? BM : BM + 16, LX = MS == 32 ? BN : BN + 16;
     __shared__ __attribute__((aligned(16))) float As[2 * BK * LA];
     __shared__ __attribute__((aligned(16))) float Xs[2 * BK * LX];
@@ -239,8 +240,8 @@ __global__ void __launch_bounds__(256, MS == 32 ? 3 : 1) k_codec_gemm(GemmParams
     const int lo = MODE == GEMM_TAPS ? n0 - p.pad : n0, hi = MODE == GEMM_TAPS ? n0 + BN + (q.taps - 1) * p.dil - p.pad : n0 + BN;
     const bool in = (p.M & 3) == 0 && (Cin & 15) == 0 && (Cin / 16 * q.taps) % (BK / 16) == 0 && ((uintptr_t)p.AT & 15) == 0 && m0 + BM <= p.M && n0 + BN <= p.N &&
                     lo >= p.x_lo && hi <= p.Tin;
-    if (in) codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, true>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
-    else codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, false>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
+    if (in) codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, true, OFF>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
+    else codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, false, OFF>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
 }
 
 // The encoders' strided convolutions: few tiles and a long K (768 x 296 outputs over K = 9216).  32 x 16 outputs per block, the four waves share the K range
@@ -333,14 +334,15 @@ static void launch_f32(const GemmParams& p, int batch, hipStream_t s) {
         F32Tiles q{cdiv(p.N, bn), cdiv(p.M, bm), cdiv(cdiv(p.N, bn), 8), MODE == GEMM_TAPS ? p.taps : 1};
         hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * q.npx * q.mt), batch), dim3(256), 0, s, p, q);
     };
-    if (p.M <= 64 && blocks(64, 128) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2>, 64, 128);
-    else if (p.M > 64 && blocks(128, 64) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 2, 2, 2, 1, 16, 2>, 128, 64);
-    else go(k_codec_gemm<MODE, SNAKE, 16, 2, 2, 1, 1, 64, 4>, 32, 32);
+    // A wave's 64 rows lie within 2^32 bytes up to 2^24 samples a row (699 s at 24 kHz); longer ones take 64-bit offsets.
+    if (std::max(p.ldx, p.ldy) > 1 << 24) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint64_t>, 64, 128);
+    else if (p.M <= 64 && blocks(64, 128) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint32_t>, 64, 128);
+    else if (p.M > 64 && blocks(128, 64) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 2, 2, 2, 1, 16, 2, uint32_t>, 128, 64);
+    else go(k_codec_gemm<MODE, SNAKE, 16, 2, 2, 1, 1, 64, 4, uint32_t>, 32, 32);
 }
 
 void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s) {
     MIS_REQUIRE(mode != GEMM_CONVT && p.M >= 1 && p.N >= 1 && (mode != GEMM_TAPS || (!snake && p.taps >= 1)), MIS_ERR_GENERATION_FAILED, "codec GEMM: bad mode");
-    MIS_REQUIRE((int64_t)128 * std::max(p.ldx, p.ldy) < (1ll << 29), MIS_ERR_GENERATION_FAILED, "codec GEMM: rows longer than 4 M samples");
     auto run = [&](auto m, auto sn) { launch_f32<decltype(m)::value, decltype(sn)::value>(p, batch, s); };
     const auto off = std::false_type{};
     if (mode == GEMM_PLAIN) run(std::integral_constant<int, GEMM_PLAIN>{}, off);
