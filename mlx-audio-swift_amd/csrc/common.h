@@ -109,6 +109,7 @@ struct HostRing {
     HostRing& operator=(const HostRing&) = delete;
     ~HostRing();
     void reserve();
+    static bool pageable(const void* p);
     void out(void* host, const void* dev, size_t n, hipStream_t s);
     void in(void* dev, const void* host, size_t n, hipStream_t s);
 private:

@@ -217,20 +217,20 @@ void HostRing::reserve() {
     for (auto& e : ev) if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     buf.alloc(SLOTS * SLOT);
 }
-static bool is_pageable(const void* p) {
+bool HostRing::pageable(const void* p) {
     hipPointerAttribute_t a{};
     if (hipPointerGetAttributes(&a, p) != hipSuccess) { (void)hipGetLastError(); return true; }
     return a.type == hipMemoryTypeUnregistered;
 }
 void HostRing::out(void* host, const void* dev, size_t n, hipStream_t s) {
     if (n == 0) { HIP_CHECK(hipStreamSynchronize(s)); return; }
-    if (buf.p && n >= MIN && is_pageable(host)) { run((uint8_t*)host, (uint8_t*)const_cast<void*>(dev), n, true, s); return; }
+    if (buf.p && n >= MIN && pageable(host)) { run((uint8_t*)host, (uint8_t*)const_cast<void*>(dev), n, true, s); return; }
     HIP_CHECK(hipMemcpyAsync(host, dev, n, hipMemcpyDefault, s));
     HIP_CHECK(hipStreamSynchronize(s));
 }
 void HostRing::in(void* dev, const void* host, size_t n, hipStream_t s) {
     if (n == 0) return;
-    if (buf.p && n >= MIN && is_pageable(host)) { run((uint8_t*)const_cast<void*>(host), (uint8_t*)dev, n, false, s); return; }
+    if (buf.p && n >= MIN && pageable(host)) { run((uint8_t*)const_cast<void*>(host), (uint8_t*)dev, n, false, s); return; }
     HIP_CHECK(hipMemcpyAsync(dev, host, n, hipMemcpyDefault, s));
     HIP_CHECK(hipStreamSynchronize(s));
 }

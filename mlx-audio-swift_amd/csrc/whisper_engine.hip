@@ -472,6 +472,19 @@ static void whisper_encode_device(mis_whisper* c, const float* features_dev, int
     whisper_decoder_reset(c);
 }
 
+// The caller's memory to the handle's and back.  Device and pinned memory may belong to work that the caller has queued on the default stream: the per-thread
+// stream is ordered with it, the handle's non-blocking stream is not.
+static void whisper_in(mis_whisper* c, void* dev, const void* src, size_t n) {
+    if (HostRing::pageable(src)) { c->ring.in(dev, src, n, c->stream); return; }
+    HIP_CHECK(hipStreamSynchronize(c->stream));
+    HIP_CHECK(copy_now(dev, src, n, hipMemcpyDefault));
+}
+static void whisper_out(mis_whisper* c, void* dst, const void* dev, size_t n) {
+    if (HostRing::pageable(dst)) { c->ring.out(dst, dev, n, c->stream); return; }
+    HIP_CHECK(hipStreamSynchronize(c->stream));
+    HIP_CHECK(copy_now(dst, dev, n, hipMemcpyDefault));
+}
+
 __global__ void k_bf16_to_f32_flat(const bf16_t* __restrict__ src, float* __restrict__ dst, size_t n) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) dst[i] = bf16_to_f32(src[i]);
@@ -484,14 +497,14 @@ extern "C" mis_status mis_whisper_encode(mis_whisper* c, const float* features, 
     HIP_CHECK(hipSetDevice(c->device));
     size_t n = (size_t)batch * 3000 * c->nmel;
     c->feats.alloc(n);
-    c->ring.in(c->feats.p, features, n * 4, c->stream);
+    whisper_in(c, c->feats.p, features, n * 4);
     whisper_encode_device(c, c->feats.p, batch);
     if (enc_out) {
         size_t ne = (size_t)batch * 1500 * c->d;
         c->enc_f32.alloc(ne);
         hipLaunchKernelGGL(k_bf16_to_f32_flat, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, c->stream, c->enc_out.p, c->enc_f32.p, ne);
         HIP_CHECK(hipGetLastError());
-        c->ring.out(enc_out, c->enc_f32.p, ne * 4, c->stream);
+        whisper_out(c, enc_out, c->enc_f32.p, ne * 4);
     }
     MIS_API_END
 }
@@ -639,7 +652,7 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     c->feats.alloc((size_t)batch * 3000 * c->nmel);
     c->pcm.alloc((size_t)batch * stride);
     const int64_t last = std::max<int64_t>(0, std::min(hl[batch - 1], stride));         // (the last row need not be as long as the others)
-    c->ring.in(c->pcm.p, pcm, ((size_t)(batch - 1) * stride + last) * 4, s);
+    whisper_in(c, c->pcm.p, pcm, ((size_t)(batch - 1) * stride + last) * 4);
     HIP_CHECK(hipMemsetAsync(c->padded.p, 0, (size_t)batch * W * 4, s));
     for (int b = 0; b < batch; ++b) {
         const int64_t n = std::min<int64_t>(std::min<int64_t>(hl[b], stride), W);
