@@ -650,13 +650,20 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     if (lens) HIP_CHECK(copy_now(hl.data(), lens, batch * sizeof(int64_t), hipMemcpyDefault));
     c->padded.alloc((size_t)batch * W);
     c->feats.alloc((size_t)batch * 3000 * c->nmel);
-    c->pcm.alloc((size_t)batch * stride);
-    const int64_t last = std::max<int64_t>(0, std::min(hl[batch - 1], stride));         // (the last row need not be as long as the others)
-    whisper_in(c, c->pcm.p, pcm, ((size_t)(batch - 1) * stride + last) * 4);
     HIP_CHECK(hipMemsetAsync(c->padded.p, 0, (size_t)batch * W * 4, s));
-    for (int b = 0; b < batch; ++b) {
-        const int64_t n = std::min<int64_t>(std::min<int64_t>(hl[b], stride), W);
-        if (n > 0) HIP_CHECK(hipMemcpyAsync(c->padded.p + (size_t)b * W, c->pcm.p + (size_t)b * stride, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
+    auto valid = [&](int b) { return (size_t)std::max<int64_t>(0, std::min(std::min(hl[b], stride), W)); };
+    // rows that are mostly samples come over in one copy, large enough for the ring; of long or mostly empty ones only what is read
+    const size_t block = (size_t)(batch - 1) * stride + valid(batch - 1);                // (the last row need not be as long as the others)
+    size_t total = 0;
+    for (int b = 0; b < batch; ++b) total += valid(b);
+    if (block <= 2 * total && HostRing::pageable(pcm)) {
+        c->pcm.alloc(block);
+        whisper_in(c, c->pcm.p, pcm, block * 4);
+        for (int b = 0; b < batch; ++b)
+            if (valid(b)) HIP_CHECK(hipMemcpyAsync(c->padded.p + (size_t)b * W, c->pcm.p + (size_t)b * stride, valid(b) * 4, hipMemcpyDeviceToDevice, s));
+    } else {
+        for (int b = 0; b < batch; ++b)
+            if (valid(b)) whisper_in(c, c->padded.p + (size_t)b * W, pcm + (size_t)b * stride, valid(b) * 4);
     }
     whisper_features_device(c->device, c->padded.p, batch, c->nmel, c->feats.p, s);
     whisper_encode_device(c, c->feats.p, batch);

@@ -1,4 +1,4 @@
-"""What Whisper's entry points take: device memory that work on the default stream still writes or reads."""
+"""What Whisper's entry points take: rows much longer than a window, device memory that work on the default stream still writes or reads."""
 import ctypes as C
 
 import numpy as np
@@ -30,6 +30,22 @@ def generate(dev, pcm_ptr, lens, stride, n=6):
     out = [arr[b, :nt[b]].tolist() for b in range(B)]
     _lib.lib().mis_free(toks)
     return out
+
+
+def test_samples_past_the_window_are_not_copied():
+    """Rows of 160 MB of which 3 s, and more than a window, are valid: no device memory for the rest, and the ids of rows cut to the window."""
+    ocfg, dev = model()
+    rng = np.random.default_rng(2)
+    lens, stride = [48000, 600000], 40_000_000
+    pcm = np.zeros((2, stride), np.float32)
+    for b, n in enumerate(lens):
+        pcm[b, :n] = 0.1 * rng.standard_normal(n)
+    short = np.ascontiguousarray(pcm[:, :480000])
+    ref = generate(dev, short.ctypes.data, [48000, 480000], 480000)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    assert generate(dev, pcm.ctypes.data, lens, stride) == ref
+    assert free - torch.cuda.mem_get_info()[0] < 32 << 20
 
 
 def busy():
