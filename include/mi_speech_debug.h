@@ -31,6 +31,9 @@ int32_t mis_debug_device_cus(int device);            /* compute units of a devic
 /* diagnostics / tests: launches of the one-launch sampler that reported a timed-out row barrier in this process so far */
 int32_t mis_debug_sampler_failures(void);
 
+/* tests: for how many floats d in [1, 2^14) the reciprocal of the Whisper encoder's GELU is not 1 / d rounded to nearest (none) */
+mis_status mis_debug_gelu_rcp_misses(int device, int64_t* misses);
+
 /* csrc/token_engine.hip (round 5): a whole batch-1 request in ONE persistent launch on the compute units of `xcds` (1, 2, 4 or 8) XCDs,
  * streaming the handle's own packed weights; compiled for Soprano-80M's LM widths (other shapes: MIS_ERR_INVALID_INPUT).  The product
  * reaches it through mis_soprano_generate at batch 1; this entry point is for tests and measurements.

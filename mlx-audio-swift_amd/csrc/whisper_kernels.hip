@@ -22,9 +22,15 @@
 // Here: erfc(|z|) = poly5(t) exp(-z^2), t = 1 / (1 + 0.3275911 |z|) (Abramowitz & Stegun 7.1.26, |error| <= 1.5e-7), branch-free, and
 // 1 + erf(z) taken as erfc(-z) for z < 0 - no cancellation on the negative side.  Against the float64 value, after the bf16 rounding
 // that follows: max |diff| 1.0e-6 of full scale, fewer mismatching roundings than the float32 0.5 x (1 + erf) form itself has.
+// 1 / d to the nearest float for 1 <= d < 2^14: the hardware reciprocal (1 ulp) and one Newton step, three instructions where the division takes ten.  Equal to the
+// division for each of the 117 M values (mis_debug_gelu_rcp_misses counts them; the reciprocal alone misses 12.6 M).
+__device__ __forceinline__ float rcp_nearest(float d) {
+    const float t = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, t, 1.0f), t, t);
+}
 __device__ __forceinline__ float gelu_erf_w(float x) {
-    const float z = fabsf(x) * 0.70710678118654752f;
-    const float t = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * z);      // (1 ulp: 6e-8 of a value good to 1.5e-7; the rounded division is ten instructions)
+    const float z = fminf(fabsf(x) * 0.70710678118654752f, 16.0f);      // (exp(-z^2) is 0 from 10.2 on)
+    const float t = rcp_nearest(1.0f + 0.3275911f * z);
     float p = 1.061405429f;
     p = p * t - 1.453152027f;
     p = p * t + 1.421413741f;
@@ -32,6 +38,25 @@ __device__ __forceinline__ float gelu_erf_w(float x) {
     p = p * t + 0.254829592f;
     const float ec = p * t * __expf(-(z * z));            // erfc(|x| / sqrt 2)
     return 0.5f * x * (x >= 0.0f ? 2.0f - ec : ec);
+}
+
+__global__ void k_rcp_misses(uint32_t lo, uint32_t n, unsigned long long* misses) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    const float d = __uint_as_float(lo + min(i, n - 1));
+    if (i < n && rcp_nearest(d) != 1.0f / d) atomicAdd(misses, 1ull);
+}
+extern "C" mis_status mis_debug_gelu_rcp_misses(int device, int64_t* misses) {
+    MIS_API_BEGIN
+    MIS_REQUIRE(misses, MIS_ERR_INVALID_INPUT, "null argument");
+    HIP_CHECK(hipSetDevice(device));
+    const uint32_t lo = 0x3f800000u, n = 0x46800000u - lo;                // 1.0f, 2^14
+    DevBuf<unsigned long long> c;
+    c.alloc(1);
+    HIP_CHECK(hipMemset(c.p, 0, 8));
+    hipLaunchKernelGGL(k_rcp_misses, dim3((n + 255) / 256), dim3(256), 0, 0, lo, n, c.p);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemcpy(misses, c.p, 8, hipMemcpyDeviceToHost));
+    MIS_API_END
 }
 
 // ============================================================================ big GEMM

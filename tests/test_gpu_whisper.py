@@ -475,3 +475,10 @@ def test_key_value_tiles_from_the_256x256_gemm_equal_the_scatter_kernel(monkeypa
             got[big] = enc, np.stack([dev.decoder_forward(toks[:, t]) for t in range(toks.shape[1])])
         for a, b in zip(got["0"], got["2"]):
             assert np.isfinite(b).all() and np.abs(b).max() > 0 and np.array_equal(a, b), B
+
+
+def test_reciprocal_of_the_encoder_gelu_is_rounded_to_nearest():
+    """gelu_erf_w divides: no bit of the quotient is given up for the hardware reciprocal (over the whole range of its argument)."""
+    import ctypes as C
+    n = C.c_int64(-1)
+    assert mas._lib.lib().mis_debug_gelu_rcp_misses(0, C.byref(n)) == 0 and n.value == 0
