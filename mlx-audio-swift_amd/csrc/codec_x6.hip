@@ -5,7 +5,8 @@
 // <= 2^-25 of the product).  One 16-deep step is 6 x 32 cycles instead of 8 x 64 of v_mfma_f32_32x32x2_f32.  Error against 64 bits (2-norm over 2-norm,
 // this kernel / the exact-f32 one; K = 96, 128, 192; operands normal): 1.38e-7 / 1.77e-7, 1.65e-7 / 2.06e-7, 2.04e-7 / 2.49e-7; all of one sign: 1.14 / 1.44,
 // 1.29 / 1.60, 1.64 / 2.05; normal times exp(2 normal): 1.25 / 1.93, 1.42 / 2.00, 1.84 / 2.45: lower each time (6 roundings of the sum per 16 products, not 16).
-// An infinite operand gives NaN where the f32 kernels may give an infinity; Snake in front of it turns infinities into NaN on both.
+// Infinite operands: k_x6_gemm takes the outputs they reach again in f32; behind the Snake of the other two kernels an infinity is NaN in any arithmetic (an
+// infinite WEIGHT there gives NaN where the f32 kernels give an infinity or NaN).
 //
 //   k_x6_pack_w   A^T f32 -> the three planes as MFMA-A fragments (once per weight matrix, kept in the model's CodecPack)
 //   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels, for the encoders and for MIS_CODEC_EXACT_F32=1)
@@ -19,6 +20,7 @@
 
 __device__ __forceinline__ float x6_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
 
+#define X6_MAX 3.38953138925153547590470800371487866880e+38f      // the largest bfloat16
 // x = h + m + l exactly (three bfloat16, each the nearest to what is left): eight values of consecutive channels -> one 16-byte piece per plane
 __device__ __forceinline__ void x6_split(const float (&v)[8], uint4& h, uint4& m, uint4& l) {
     uint32_t o[3][4];
@@ -27,7 +29,9 @@ __device__ __forceinline__ void x6_split(const float (&v)[8], uint4& h, uint4& m
         float a = v[2 * i], b = v[2 * i + 1];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            const uint32_t ab = (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
+            // (the first plane of a value past the largest bfloat16 is that one, not infinity; the rest still fits the other two)
+            const float ca = q ? a : __builtin_amdgcn_fmed3f(a, -X6_MAX, X6_MAX), cb = q ? b : __builtin_amdgcn_fmed3f(b, -X6_MAX, X6_MAX);
+            const uint32_t ab = (uint32_t)f32_to_bf16(ca) | ((uint32_t)f32_to_bf16(cb) << 16);
             o[q][i] = ab;
             a -= __uint_as_float(ab << 16);
             b -= __uint_as_float(ab & 0xffff0000u);
@@ -51,7 +55,7 @@ __global__ void k_x6_pack_w(const float* __restrict__ AT, uint16_t* __restrict__
         float v = (m < M && c < Cin) ? AT[((size_t)tap * Cin + c) * M + m] : 0.0f;
         const size_t o = (e >> 9) * 1536 + (size_t)lane * 8 + j;
         for (int q = 0; q < 3; ++q) {
-            const uint16_t h = f32_to_bf16(v);
+            const uint16_t h = f32_to_bf16(q ? v : __builtin_amdgcn_fmed3f(v, -X6_MAX, X6_MAX));
             wp[o + q * 512] = h;
             v -= bf16_to_f32(h);
         }
@@ -263,7 +267,8 @@ struct X6Gemm {
 template <int MTW, bool SNAKE, bool TAPS, bool WIDE>
 __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                              const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise,
-                                             const float* __restrict__ pa, const float* __restrict__ pra, const uint16_t* __restrict__ pwp) {
+                                             const float* __restrict__ pa, const float* __restrict__ pra, const float* __restrict__ pAT,
+                                             const uint16_t* __restrict__ pwp) {
     constexpr int PF = MTW == 8 ? 2 : 4, SPB = MTW == 8 ? 1 : 2;            // steps of X (narrow: of weights too) in flight; steps per staged chunk of weights
     constexpr int NA = (SPB * MTW * 192 + 255) / 256, APC = SPB * MTW * 192;
     __shared__ x6_u4 As[WIDE ? 2 : 1][WIDE ? APC : 1];
@@ -443,22 +448,50 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
         if ((mt0 + mi) * 32 >= p.M) break;
         const int m0 = (mt0 + mi) * 32 + 4 * lane_hi;
         if constexpr (WIDE) want(mi, lane_hi);
-        if (n < p.N) {
+        if (n >= p.N) continue;
+        auto finish = [&](float y, float b0, float s0, float e0) {
+            y += pbias ? b0 : 0.0f;
+            if (gelu) y = 0.5f * y * (1.0f + erff(y * 0.70710678118654752f));
+            else if (noise) y = e0 + nz * y;
+            else if (eb) { if (pscale) y *= s0; y = e0 + y; }
+            return y;
+        };
+        float* y = pY + (size_t)b * p.M * p.ldy + n;
+        // Three planes do not hold an infinity or a value past the largest bfloat16 (the planes of a product of two such cancel to NaN): a lane that sees a sum
+        // which is not finite takes its rows again as the f32 kernels do, channel by channel
+        float zero = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero = fmaf(acc[mi][r], 0.0f, zero);
+        if (zero == 0.0f) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + (r & 3) + 8 * (r >> 2);
-                float y = acc[mi][r] + (pbias ? bm[r] : 0.0f);
-                if (gelu) y = 0.5f * y * (1.0f + erff(y * 0.70710678118654752f));
-                else if (noise) y = e[r] + nz * y;
-                else if (eb) { if (pscale) y *= sc[r]; y = e[r] + y; }
-                if (m < p.M) pY[((size_t)b * p.M + m) * p.ldy + n] = y;
+                if (m < p.M) y[(size_t)m * p.ldy] = finish(acc[mi][r], bm[r], pscale ? sc[r] : 0.0f, eb ? e[r] : 0.0f);
+            }
+        } else {
+            const int T = TAPS ? P.ntaps : 1;
+#pragma unroll 1
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + (r & 3) + 8 * (r >> 2);
+                if (m >= p.M) break;
+                float v = 0.0f;
+#pragma unroll 1
+                for (int i = 0; i < Kx * T; ++i) {                          // 16 channels, within them the taps, within a tap the channels
+                    const int c = i / (16 * T) * 16 + (i & 15), j = i / 16 % T, t = TAPS ? n - p.pad + j * p.dil : n;
+                    if (TAPS && (t < p.x_lo || t >= p.Tin)) continue;
+                    float x = pX[((size_t)b * Kx + c) * p.ldx + t];
+                    if constexpr (SNAKE) x = x6_snake(x, x6_ab[c], x6_ab[Kx + c]);
+                    v = fmaf(pAT[((size_t)j * Kx + c) * p.M + m], x, v);
+                    if (v != v) break;                                      // (NaN it stays)
+                }
+                y[(size_t)m * p.ldy] = finish(v, pbias ? pbias[m] : 0.0f, pscale ? pscale[m] : 0.0f, eb ? eb[(size_t)m * lde + n] : 0.0f);
             }
         }
     }
 }
 template <int MTW, bool SNAKE, bool TAPS, bool WIDE>
 __global__ void __launch_bounds__(256, 2) k_x6_gemm(X6Gemm P, const uint16_t* wp) {
-    x6_gemm_body<MTW, SNAKE, TAPS, WIDE>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.g.alpha, P.g.ralpha, wp);
+    x6_gemm_body<MTW, SNAKE, TAPS, WIDE>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.g.alpha, P.g.ralpha, P.g.AT, wp);
 }
 
 template <bool SNAKE, bool TAPS>
