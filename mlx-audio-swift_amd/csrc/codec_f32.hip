@@ -3,13 +3,15 @@
 // 1x1 convolutions (plain, GELU, residual with optional Snake in front, NoiseBlock) and dense k-tap convolutions without an activation (the encoders'
 // strided convolutions over a phase-split tensor).  The k order is: 16 input channels, within them the taps, within a tap the channels.
 // v_mfma_f32 adds its products one after the other in k order (32x32x2, 16x16x4 and a chain of fmaf give the same bits: measured over random
-// operands), so EVERY tile shape below returns the same bits and the launcher is free to pick one by the number of blocks it gives:
+// operands), so EVERY tile shape below returns the same bits and the launcher is free to pick one by the number of blocks it gives.  Convolutions of K >= 1024 add four
+// partial sums, in every form that they may take:
 //
 //   wide   128 x 64 (M <= 64: 64 x 128), 4 waves of 64 x 32 on 32x32x2, 16 k per staged chunk, three blocks per compute unit: a block's loads and its
 //          epilogue hide behind the others' products.  Bound: 2.4 GB for 256 x 24576 outputs over K = 256 with residual, 32 rows: 1.18 ms of 1.34 ms
 //          before (64 x 128 tiles, two barriers per chunk, residual rows one by one); 128 x 128 tiles at two blocks per unit: 1.36 ms.
 //   small  32 x 32, 4 waves of one 16x16x4 tile, four chunks of 64 k in flight at once (a short K is ONE memory round trip).  Bound: latency.
-//          512 x 384 outputs over K = 512 with residual: 45 -> 7.5 us; the encoders' 384 x 2368 over K = 4608: 330 -> 154 us.
+//          512 x 384 outputs over K = 512 with residual: 45 -> 7.5 us.
+//   split  32 x 16, the four waves a quarter of a long K each (k_codec_gemm_split).
 //
 // One barrier per chunk (two LDS buffers): chunk c + 1 goes from registers to LDS and chunk c + 1 + PF is requested before chunk c is multiplied.
 // Blocks are dealt to the XCDs by id mod 8: an XCD takes a CONTIGUOUS range of column tiles, all row tiles of a column tile in a row.  Its L2 holds the
@@ -28,8 +30,8 @@ typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));       //
 // One tile.  WM x WN waves; a wave holds TM x TN MFMA tiles of MS x MS (MS = 32 or 16); BK k per chunk; PF chunks requested ahead.
 // IN: the tile lies inside the output, its columns at every tap inside the input, M is a multiple of 4, the channels of 16 and the k units of the chunk -
 // nothing to clamp or mask.  Otherwise every element is clamped when it is loaded and masked when it is put into LDS.
-// OFF: the type of an offset inside the tile's rows (see launch_f32).
-template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF, bool IN, typename OFF>
+// OFF: the type of an offset inside the tile's rows (see launch_f32).  QUARTERS: four partial sums (codec_quarters), the accumulators added to the total between them.
+template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF, bool IN, typename OFF, bool QUARTERS>
 __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int n0, int m0, int b, float* As, float* Xs, const float* __restrict__ pX, const float* __restrict__ pR,
                                                 float* __restrict__ pY, const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pAT) {
     constexpr int BM = WM * TM * MS, BN = WN * TN * MS, KS = MS == 32 ? 2 : 4;
@@ -181,6 +183,22 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
         }
     };
     if constexpr (PRE) want();
+    [[maybe_unused]] acc_t tot[QUARTERS ? TM : 1][QUARTERS ? TN : 1];
+    [[maybe_unused]] int quarter = 1;
+    [[maybe_unused]] auto close_quarter = [&]() {                        // (0 + p0 is p0: a sum that starts at 0 is never -0)
+#pragma unroll
+        for (int i = 0; i < (QUARTERS ? TM : 0); ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < NR; ++r) { tot[i][j][r] += acc[i][j][r]; acc[i][j][r] = 0.0f; }
+    };
+    if constexpr (QUARTERS) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) tot[i][j] = acc[i][j];
+    }
     // chunk c sits in LDS buffer c & 1; registers hold chunks c + 1 .. c + PF (slot = chunk % PF)
 #pragma unroll
     for (int i = 0; i < PF; ++i) load(i, i);
@@ -195,9 +213,19 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
             const int slot = (u + 1) % PF;
             put(c0 + u + 1, slot, (u + 1) & 1);
             load(c0 + u + 1 + PF, slot);
+            if constexpr (QUARTERS) {
+                if (quarter < 4 && (c0 + u) * (BK / 16) == codec_quarter(units, quarter)) { close_quarter(); ++quarter; }
+            }
             if (c0 + u < nchunks) math(u & 1);
             __syncthreads();
         }
+    }
+    if constexpr (QUARTERS) {
+        close_quarter();
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = tot[i][j];
     }
     if constexpr (!PRE) want();
 #pragma unroll
@@ -229,7 +257,7 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
         }
     }
 }
-template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF, typename OFF>
+template <int MODE, bool SNAKE, int MS, int WM, int WN, int TM, int TN, int BK, int PF, typename OFF, bool QUARTERS>
 __global__ void __launch_bounds__(256, MS == 32 && sizeof(OFF) == 4 ? 3 : 1) k_codec_gemm(GemmParams p, F32Tiles q) {
     constexpr int BM = WM * TM * MS, BN = WN * TN * MS, LA = MS == 32 ? BM : BM + 16, LX = MS == 32 ? BN : BN + 16;
     __shared__ __attribute__((aligned(16))) float As[2 * BK * LA];
@@ -240,22 +268,23 @@ __global__ void __launch_bounds__(256, MS == 32 && sizeof(OFF) == 4 ? 3 : 1) k_c
     const int lo = MODE == GEMM_TAPS ? n0 - p.pad : n0, hi = MODE == GEMM_TAPS ? n0 + BN + (q.taps - 1) * p.dil - p.pad : n0 + BN;
     const bool in = (p.M & 3) == 0 && (Cin & 15) == 0 && (Cin / 16 * q.taps) % (BK / 16) == 0 && ((uintptr_t)p.AT & 15) == 0 && m0 + BM <= p.M && n0 + BN <= p.N &&
                     lo >= p.x_lo && hi <= p.Tin;
-    if (in) codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, true, OFF>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
-    else codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, false, OFF>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
+    if (in) codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, true, OFF, QUARTERS>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
+    else codec_gemm_tile<MODE, SNAKE, MS, WM, WN, TM, TN, BK, PF, false, OFF, QUARTERS>(p, q.taps, n0, m0, b, As, Xs, p.X, p.R, p.Y, p.bias, p.scale, p.AT);
 }
 
-// The encoders' strided convolutions: few tiles and a long K (768 x 296 outputs over K = 9216).  32 x 16 outputs per block, the four waves share the K range
-// in units of 16 k and meet once in LDS; no staging, both operands come straight from global memory in fragment order (16 lanes = 64 contiguous
-// bytes), four units in flight.  652 us as 36 blocks of 64 x 128 -> 104 us.  The sums are four partial sums, so the choice goes by the shape of ONE row
-// alone: a row's bits do not depend on the batch it shares.
+// Convolutions with a long K (codec_quarters), the encoders' strided ones among them.  32 x 16 outputs per block, the four waves take a quarter of the K range each
+// and meet once in LDS; no staging, both operands come straight from global memory in fragment order (16 lanes = 64 contiguous bytes), four units in
+// flight.  768 rows, K = 9216, 296 columns: 94 us (64 x 128 tiles: 652).
+#define CODEC_SPLIT_NY 32768       // column tiles in the y dimension of the grid; more of them in z
 __device__ __forceinline__ void codec_gemm_split_body(const GemmParams& p, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
-                                                      const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pAT) {
+                                                      const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pAT, int batch) {
     constexpr int KW = 4;
     __shared__ float red[KW][32][17];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int m0 = blockIdx.x * 32, n0 = blockIdx.y * 16, b = blockIdx.z;
+    const int m0 = blockIdx.x * 32, b = blockIdx.z % batch, n0 = (blockIdx.z / batch * CODEC_SPLIT_NY + blockIdx.y) * 16;
+    if (n0 >= p.N) return;
     const int Cin = p.Cin, T = p.taps;
-    const int units = (Cin + 15) / 16 * T, u0 = units * wave / KW, u1 = units * (wave + 1) / KW;
+    const int units = (Cin + 15) / 16 * T, u0 = codec_quarter(units, wave), u1 = codec_quarter(units, wave + 1);
     const float* Xb = pX + (size_t)b * Cin * p.ldx;
     const int kl = lane >> 4, nl = lane & 15;
     const int ma = min(m0 + nl, p.M - 1), mb = min(m0 + 16 + nl, p.M - 1);       // (rows past M are computed and not stored)
@@ -317,16 +346,12 @@ __device__ __forceinline__ void codec_gemm_split_body(const GemmParams& p, const
         pY[o] = v;
     }
 }
-__global__ void __launch_bounds__(256) k_codec_gemm_split(GemmParams p) { codec_gemm_split_body(p, p.X, p.R, p.Y, p.bias, p.scale, p.AT); }
+__global__ void __launch_bounds__(256) k_codec_gemm_split(GemmParams p, int batch) { codec_gemm_split_body(p, p.X, p.R, p.Y, p.bias, p.scale, p.AT, batch); }
 
-bool codec_taps_split(const GemmParams& p) { return (long)cdiv(p.M, 64) * cdiv(p.N, 64) <= 64 && p.K >= 1024 && cdiv(p.N, 16) <= 65535; }
+bool codec_quarters(const GemmParams& p) { return p.K >= 1024; }
 
 template <int MODE, bool SNAKE>
 static void launch_f32(const GemmParams& p, int batch, hipStream_t s) {
-    if (MODE == GEMM_TAPS && codec_taps_split(p)) {
-        hipLaunchKernelGGL(k_codec_gemm_split, dim3(cdiv(p.M, 32), cdiv(p.N, 16), batch), dim3(256), 0, s, p);
-        return;
-    }
     // The widest tile that still gives two blocks per compute unit; below that the shape is bound by latency, and the smallest tile has the
     // shortest chain and the most loads in flight.  (Bits do not depend on the choice.)
     auto blocks = [&](int bm, int bn) { return (long)cdiv(p.M, bm) * cdiv(p.N, bn) * batch; };
@@ -335,10 +360,25 @@ static void launch_f32(const GemmParams& p, int batch, hipStream_t s) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * q.npx * q.mt), batch), dim3(256), 0, s, p, q);
     };
     // A wave's 64 rows lie within 2^32 bytes up to 2^24 samples a row (699 s at 24 kHz); longer ones take 64-bit offsets.
-    if (std::max(p.ldx, p.ldy) > 1 << 24) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint64_t>, 64, 128);
-    else if (p.M <= 64 && blocks(64, 128) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint32_t>, 64, 128);
-    else if (p.M > 64 && blocks(128, 64) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 2, 2, 2, 1, 16, 2, uint32_t>, 128, 64);
-    else go(k_codec_gemm<MODE, SNAKE, 16, 2, 2, 1, 1, 64, 4, uint32_t>, 32, 32);
+    const bool near = std::max(p.ldx, p.ldy) <= 1 << 24;
+    if constexpr (MODE == GEMM_TAPS) {
+        if (codec_quarters(p)) {
+            // The same bits in all of them.  us, tiles / split form: 128 rows, K = 1792, 64000 columns (1000 blocks of the wide tile) 318 / 471, 4000 columns 53 / 36; 64
+            // rows, K = 1536, 100000 columns (782) 256 / 336, 20000 columns 73 / 72; 384 rows, K = 4608, eight rows of 2368 columns (888) 1012 / 1031, one 148 / 143; 192
+            // rows, K = 1152, 18944 columns (592) 195 / 154; 32 rows, K = 1536, 200000 columns (half of the tile empty) 569 / 351
+            if (near && p.M > 32 && p.M <= 64 && blocks(64, 128) >= 768) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint32_t, true>, 64, 128);
+            else if (near && p.M > 64 && blocks(128, 64) >= 768) go(k_codec_gemm<MODE, SNAKE, 32, 2, 2, 2, 1, 16, 2, uint32_t, true>, 128, 64);
+            else {
+                const int nt = cdiv(p.N, 16);
+                hipLaunchKernelGGL(k_codec_gemm_split, dim3(cdiv(p.M, 32), std::min(nt, CODEC_SPLIT_NY), batch * cdiv(nt, CODEC_SPLIT_NY)), dim3(256), 0, s, p, batch);
+            }
+            return;
+        }
+    }
+    if (!near) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint64_t, false>, 64, 128);
+    else if (p.M <= 64 && blocks(64, 128) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint32_t, false>, 64, 128);
+    else if (p.M > 64 && blocks(128, 64) >= 512) go(k_codec_gemm<MODE, SNAKE, 32, 2, 2, 2, 1, 16, 2, uint32_t, false>, 128, 64);
+    else go(k_codec_gemm<MODE, SNAKE, 16, 2, 2, 1, 1, 64, 4, uint32_t, false>, 32, 32);
 }
 
 void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s) {

@@ -135,7 +135,10 @@ struct GemmParams {
 void launch_gemm(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // exact-f32 kernels (codec_f32.hip): every mode but CONVT, TAPS without Snake; p must have ldx / ldy resolved
 void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
-bool codec_taps_split(const GemmParams& p);      // k-tap contraction of few tiles and a long K: the k-split form of codec_f32.hip
+// k-tap contractions of K >= 1024 add four partial sums, over the ranges [codec_quarter(w), codec_quarter(w + 1)) of their steps of 16 channels of a tap, in order:
+// in waves that run beside each other or one after the other - the same bits, whatever the length and the batch
+bool codec_quarters(const GemmParams& p);
+__host__ __device__ inline int codec_quarter(int steps, int w) { return w >= 4 ? steps : steps * w / 16 * 4; }
 // three-plane split (codec_x6.hip): 1x1 and k-tap contractions of at least 48 rows and a multiple of 16 channels; false: not eligible, nothing launched
 bool launch_gemm_x6(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // three-plane split: transposed convolution of stride 2, two taps per phase, 32 .. 64 rows, behind Snake; false: another shape

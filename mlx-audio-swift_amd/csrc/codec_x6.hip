@@ -264,27 +264,32 @@ struct X6Gemm {
     int mode, ntaps, nsteps, MT32;        // steps of 16 channels of one tap
     int nbx, my, per, tiles;              // column tiles, row tiles, tiles per XCD, all tiles
 };
-template <int MTW, bool SNAKE, bool TAPS, bool WIDE>
+// QUARTERS (codec_quarters: K >= 1024): four partial sums.  The narrow form's four waves then share 32 columns and take a quarter of the steps each; the wide one
+// adds its accumulators to the total at the same steps, so a row's bits do not depend on which of them its length selects.
+template <int MTW, bool SNAKE, bool TAPS, bool WIDE, bool QUARTERS>
 __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                              const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise,
                                              const float* __restrict__ pa, const float* __restrict__ pra, const float* __restrict__ pAT,
                                              const uint16_t* __restrict__ pwp) {
-    constexpr int PF = MTW == 8 ? 2 : 4, SPB = MTW == 8 ? 1 : 2;            // steps of X (narrow: of weights too) in flight; steps per staged chunk of weights
+    constexpr bool TIGHT = MTW == 8 || (MTW == 4 && QUARTERS), KSPLIT = QUARTERS && !WIDE;
+    constexpr int PF = TIGHT ? 2 : 4, SPB = TIGHT ? 1 : 2;                  // steps of X (narrow: of weights too) in flight; steps per staged chunk of weights
     constexpr int NA = (SPB * MTW * 192 + 255) / 256, APC = SPB * MTW * 192;
     __shared__ x6_u4 As[WIDE ? 2 : 1][WIDE ? APC : 1];
+    __shared__ float red[KSPLIT ? 4 : 1][KSPLIT ? 16 : 1][KSPLIT ? 64 : 1];
     extern __shared__ float x6_ab[];                                        // SNAKE: alpha [K], 1 / alpha [K]
     const GemmParams& p = P.g;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kh = lane >> 5;
     const int tileid = (blockIdx.x & 7) * P.per + (blockIdx.x >> 3);
     if (tileid >= P.tiles) return;
     const int by = tileid % P.my, bxb = tileid / P.my, bx = bxb % P.nbx, b = bxb / P.nbx;
-    const int n = bx * 128 + wave * 32 + (lane & 31), nc = min(n, p.N - 1);
+    const int n = (KSPLIT ? bx * 32 : bx * 128 + wave * 32) + (lane & 31), nc = min(n, p.N - 1);
+    const int lo = KSPLIT ? codec_quarter(P.nsteps, wave) : 0, hi = KSPLIT ? codec_quarter(P.nsteps, wave + 1) : P.nsteps;      // this wave's steps
     const int mt0 = by * MTW, Kx = TAPS ? p.Cin : p.K;
     if constexpr (SNAKE) {
         for (int i = tid; i < Kx; i += 256) { x6_ab[i] = pa[i]; x6_ab[Kx + i] = pra[i]; }
         __syncthreads();
     }
-    if (!WIDE && bx * 128 + wave * 32 >= p.N) return;                       // (no barrier below)
+    if (!WIDE && !KSPLIT && bx * 128 + wave * 32 >= p.N) return;            // (no barrier below)
     const float* xb = pX + ((size_t)b * Kx + kh * 8) * p.ldx;
     const x6_u4* wsrc = reinterpret_cast<const x6_u4*>(pwp) + (size_t)mt0 * 192;
     const size_t wstep = (size_t)P.MT32 * 192;
@@ -292,8 +297,8 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
     float v[PF][8];
     bool ok[PF];
     x6_u4 aw[WIDE ? 1 : PF][MTW][3];
-    int fs = 0, ftap = 0;                                                   // next step to request
-    const float* fx = xb;
+    int fs = lo, ftap = KSPLIT ? lo % P.ntaps : 0;                          // next step to request
+    const float* fx = xb + (KSPLIT ? (size_t)(lo / P.ntaps) * 16 * p.ldx : 0);
     auto fetch = [&](int slot) {
         const int t = TAPS ? nc - p.pad + ftap * p.dil : nc;
         ok[slot] = !TAPS || (t >= p.x_lo && t < p.Tin);
@@ -306,7 +311,7 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
 #pragma unroll
                 for (int q = 0; q < 3; ++q) aw[slot][mi][q] = wsrc[(size_t)fs * wstep + min((mi * 3 + q) * 64 + lane, mtop)];
         }
-        if (fs + 1 < P.nsteps) {                                            // (past the end: the last step again)
+        if (fs + 1 < hi) {                                                  // (past the end: the last step again)
             ++fs;
             if (!TAPS || ++ftap == P.ntaps) { ftap = 0; fx += (size_t)16 * p.ldx; }
         }
@@ -336,18 +341,19 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
         if (pnoise) nz = pnoise[(size_t)b * p.N + n];
         else if (p.noise_rng) nz = codec_noise_value(p.noise_key, (uint64_t)(p.row_offset + (p.row_ids ? p.row_ids[b] : b)), n);
     }
-    float bm[16], sc[16], e[16];
+    constexpr int NR = KSPLIT ? 4 : 16;                                     // rows of a tile that a lane finishes
+    float bm[NR], sc[NR], e[NR];
     auto want = [&](int mi, int lane_hi) {
-        const int m0 = (mt0 + mi) * 32 + 4 * lane_hi;
+        const int m0 = (mt0 + mi) * 32 + 4 * lane_hi + (KSPLIT ? 8 * wave : 0);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) bm[r] = bp[min(m0 + (r & 3) + 8 * (r >> 2), btop)];
+        for (int r = 0; r < NR; ++r) bm[r] = bp[min(m0 + (r & 3) + 8 * (r >> 2), btop)];
         if (pscale) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sc[r] = pscale[min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1)];
+            for (int r = 0; r < NR; ++r) sc[r] = pscale[min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1)];
         }
         if (eb) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) e[r] = eb[(size_t)min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1) * lde + nc];
+            for (int r = 0; r < NR; ++r) e[r] = eb[(size_t)min(m0 + (r & 3) + 8 * (r >> 2), p.M - 1) * lde + nc];
         }
     };
     if constexpr (!WIDE) want(0, kh);
@@ -401,7 +407,24 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
         putA(0);
         loadA(1);
         __syncthreads();
+        f32x16_t tot[QUARTERS ? MTW : 1];
+        int quarter = 1;
+        [[maybe_unused]] auto close_quarter = [&]() {                       // (0 + p0 is p0: a sum that starts at 0 is never -0)
+#pragma unroll
+            for (int i = 0; i < MTW; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) { tot[QUARTERS ? i : 0][r] += acc[i][r]; acc[i][r] = 0.0f; }
+        };
+        if constexpr (QUARTERS) {
+#pragma unroll
+            for (int i = 0; i < MTW; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) tot[i][r] = 0.0f;
+        }
         auto group = [&](int c0, auto whole) {
+            if constexpr (QUARTERS) {
+                if (quarter < 4 && c0 * SPB == codec_quarter(P.nsteps, quarter)) { close_quarter(); ++quarter; }
+            }
 #pragma unroll
             for (int u = 0; u < CG; ++u) {
                 putA((u + 1) & 1);
@@ -421,6 +444,11 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
         int c0 = 0;
         for (; (c0 + CG) * SPB <= P.nsteps; c0 += CG) group(c0, std::true_type{});
         if (c0 < nchunks) group(c0, std::false_type{});
+        if constexpr (QUARTERS) {
+            close_quarter();
+#pragma unroll
+            for (int i = 0; i < MTW; ++i) acc[i] = tot[i];
+        }
     } else {
         auto group = [&](int s0, auto whole) {
 #pragma unroll
@@ -432,21 +460,28 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
                     for (int q = 0; q < 3; ++q) a[mi][q] = aw[u][mi][q];
                 __builtin_amdgcn_sched_barrier(0);
                 fetch(u);
-                if (decltype(whole)::value || s0 + u < P.nsteps) products(u & 1, [&](int mi, int q) { return a[mi][q]; });
+                if (decltype(whole)::value || s0 + u < hi) products(u & 1, [&](int mi, int q) { return a[mi][q]; });
                 convert((u + 1) % PF, (u + 1) & 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        int s0 = 0;
-        for (; s0 + PF <= P.nsteps; s0 += PF) group(s0, std::true_type{});
-        if (s0 < P.nsteps) group(s0, std::false_type{});
+        int s0 = lo;
+        for (; s0 + PF <= hi; s0 += PF) group(s0, std::true_type{});
+        if (s0 < hi) group(s0, std::false_type{});
+    }
+    if constexpr (KSPLIT) {                                                 // each wave finishes the rows of four registers
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[wave][r][lane] = acc[0][r];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[0][r] = ((red[0][4 * wave + r][lane] + red[1][4 * wave + r][lane]) + red[2][4 * wave + r][lane]) + red[3][4 * wave + r][lane];
     }
     int lane_hi = kh;                                                       // (opaque: the rows' addresses are not to be computed ahead of the contraction)
     asm volatile("" : "+v"(lane_hi));
 #pragma unroll
     for (int mi = 0; mi < MTW; ++mi) {
         if ((mt0 + mi) * 32 >= p.M) break;
-        const int m0 = (mt0 + mi) * 32 + 4 * lane_hi;
+        const int m0 = (mt0 + mi) * 32 + 4 * lane_hi + (KSPLIT ? 8 * wave : 0);
         if constexpr (WIDE) want(mi, lane_hi);
         if (n >= p.N) continue;
         auto finish = [&](float y, float b0, float s0, float e0) {
@@ -461,17 +496,17 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
         // which is not finite takes its rows again as the f32 kernels do, channel by channel
         float zero = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) zero = fmaf(acc[mi][r], 0.0f, zero);
+        for (int r = 0; r < NR; ++r) zero = fmaf(acc[mi][r], 0.0f, zero);
         if (zero == 0.0f) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < NR; ++r) {
                 const int m = m0 + (r & 3) + 8 * (r >> 2);
                 if (m < p.M) y[(size_t)m * p.ldy] = finish(acc[mi][r], bm[r], pscale ? sc[r] : 0.0f, eb ? e[r] : 0.0f);
             }
         } else {
             const int T = TAPS ? P.ntaps : 1;
 #pragma unroll 1
-            for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < NR; ++r) {
                 const int m = m0 + (r & 3) + 8 * (r >> 2);
                 if (m >= p.M) break;
                 float v = 0.0f;
@@ -489,9 +524,9 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
         }
     }
 }
-template <int MTW, bool SNAKE, bool TAPS, bool WIDE>
+template <int MTW, bool SNAKE, bool TAPS, bool WIDE, bool QUARTERS>
 __global__ void __launch_bounds__(256, 2) k_x6_gemm(X6Gemm P, const uint16_t* wp) {
-    x6_gemm_body<MTW, SNAKE, TAPS, WIDE>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.g.alpha, P.g.ralpha, P.g.AT, wp);
+    x6_gemm_body<MTW, SNAKE, TAPS, WIDE, QUARTERS>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.g.alpha, P.g.ralpha, P.g.AT, wp);
 }
 
 template <bool SNAKE, bool TAPS>
@@ -508,12 +543,26 @@ static void launch_x6_gemm(X6Gemm P, const uint16_t* wp, int batch, hipStream_t 
     // The form with the most rows per block (each converts its columns once) that still gives blocks enough; the same bits in all of them.  us:
     //   8 tiles / f32     256 x 256, 32 x 24576 columns 845 / 1133
     //   4 / 2 / 1         192 x 192, 18888 columns (296, 592 blocks of 4 and 2): 29 / 20 / 24; the same rows, two taps of 192 (K = 768): 105 / 72 / 102
-    //   2 / 1 / f32       384 x 384 with Snake, 10160 columns: 41 / 56 / 71; 384 rows, K = 1536, 2361 columns (114 blocks of 2): 156 / 124 / 154
+    //   2 / 1 / f32       384 x 384 with Snake, 10160 columns: 41 / 56 / 71
     auto blocks = [&](int mtw) { return (int64_t)P.nbx * ((P.MT32 + mtw - 1) / mtw) * batch; };
-    if (P.MT32 > 4 && blocks(8) >= 512) go(k_x6_gemm<8, SNAKE, TAPS, true>, 8);
-    else if (P.MT32 > 2 && blocks(4) >= 512) go(k_x6_gemm<4, SNAKE, TAPS, true>, 4);
-    else if (blocks(2) >= 256) go(k_x6_gemm<2, SNAKE, TAPS, true>, 2);
-    else go(k_x6_gemm<1, SNAKE, TAPS, false>, 1);
+    if constexpr (TAPS) {
+        if (codec_quarters(p)) {
+            // us, 4 tiles / 2 / the narrow form: 384 rows, K = 4608, 394 columns 204 / 155 / 31, 2368 columns (57, 114 blocks of 4 and 2) 204 / 154 / 91, eight such
+            // rows (456, 912) 336 / 469 / 583; 128 rows, K = 3072, 16000 columns (250 of 2) 146 / 110 / 123; 192 rows, K = 1152, 18944 columns (296, 444) 94 / 71 / 97,
+            // eight such rows 444 / 437 / 733; 768 rows, K = 9216, 296 columns 394 / 299 / 59 (f32: 94)
+            if (P.MT32 > 2 && blocks(4) >= 384) go(k_x6_gemm<4, SNAKE, TAPS, true, true>, 4);
+            else if (blocks(2) >= 192) go(k_x6_gemm<2, SNAKE, TAPS, true, true>, 2);
+            else {
+                P.nbx = (p.N + 31) / 32;
+                go(k_x6_gemm<1, SNAKE, TAPS, false, true>, 1);
+            }
+            return;
+        }
+    }
+    if (P.MT32 > 4 && blocks(8) >= 512) go(k_x6_gemm<8, SNAKE, TAPS, true, false>, 8);
+    else if (P.MT32 > 2 && blocks(4) >= 512) go(k_x6_gemm<4, SNAKE, TAPS, true, false>, 4);
+    else if (blocks(2) >= 256) go(k_x6_gemm<2, SNAKE, TAPS, true, false>, 2);
+    else go(k_x6_gemm<1, SNAKE, TAPS, false, false>, 1);
 }
 
 bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s) {
@@ -522,11 +571,10 @@ bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hip
     const bool taps = mode == GEMM_TAPS;
     if (!pack || codec_exact_f32() || mode == GEMM_CONVT || (snake && (mode != GEMM_RESID || !p.alpha))) return false;
     const int Cin = taps ? p.Cin : p.K, ntaps = taps ? p.taps : 1;
-    // By the shape of the matrix alone: a row's result must not depend on its length or its batch.  512 channels at one short row are bound by latency,
+    // By the matrix alone: a row's result must not depend on its length or its batch.  512 channels at one short row are bound by latency,
     // which the f32 kernel's four chunks of 64 channels in flight hide better (512 x 512, 96 columns: 15 us here, 8 there; 256 x 256, 768 columns: 11.3, 10.1);
     // a NoiseBlock of 64 channels is bound by memory (32 x 196608 columns: 918 us here, 842 there; 48 channels with residual, 37776 columns: 23, 34).
     if (p.M < (mode == GEMM_NOISE ? 96 : 48) || Cin < 32 || Cin % 16 || (!taps && Cin > 384)) return false;
-    if (taps && codec_taps_split(p)) return false;
     if (mode != GEMM_RESID && mode != GEMM_TAPS) p.R = p.scale = nullptr;
     const CodecPack::X6& e = pack->get_x6(p.AT, ntaps, Cin, p.M, s);
     X6Gemm P{};

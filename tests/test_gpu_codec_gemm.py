@@ -47,3 +47,24 @@ def test_encode(cfg, samples):
     assert np.sqrt(np.mean((z[:2] - ref) ** 2)) <= 1e-5 * np.sqrt(np.mean(ref ** 2))          # float32 sums over K <= 3072 through nine layers
     one, z1 = dev.encode(audio[3:4], return_latent=True)
     assert np.array_equal(z1[0], z[3]) and all(np.array_equal(a[0], c[3]) for a, c in zip(one, codes))
+
+
+# the same with a first convolution of 64 rows over K >= 1024
+LONG_K = dict(WIDE, encoder_rates=[16, 2, 2, 2])
+
+
+@pytest.mark.parametrize("exact", [False, True], ids=["three-planes", "f32"])
+@pytest.mark.parametrize("cfg", [WIDE, LONG_K], ids=["wide", "long-k"])
+def test_a_recording_and_its_beginning_have_the_same_bits(cfg, exact, monkeypatch):
+    """The strided convolutions' sums are taken in an order that only the matrix decides: the frames of a long recording that do not see where the short one
+    ends have its bits, on either side of the lengths - and batches - where the kernels' forms take turns."""
+    if exact:
+        monkeypatch.setenv("MIS_CODEC_EXACT_F32", "1")
+    ocfg, oracle, dev = pair(cfg)
+    audio = (0.3 * np.random.default_rng(9).standard_normal((1, 1400 * 128))).astype(np.float32)
+    _, z = dev.encode(audio, return_latent=True)
+    for frames in (80, 300, 700):
+        _, short = dev.encode(audio[:, :frames * 128], return_latent=True)
+        assert np.array_equal(short[:, :, :frames - 48], z[:, :, :frames - 48]), frames
+    _, many = dev.encode(np.repeat(audio, 10, axis=0), return_latent=True)
+    assert np.array_equal(many[0], z[0]) and np.array_equal(many[9], z[0])
