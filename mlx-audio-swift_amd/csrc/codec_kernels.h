@@ -109,8 +109,8 @@ struct GemmParams {
     const float* bias;    // [M] or null
     const float* X;       // [B][Kx][Tin]  (Kx = K; CONVT: Cin)
     float* Y;             // [B][M][Tout]
-    const float* R;       // RESID: [B][M][N]
-    const float* scale;   // RESID: optional per-row scale of (acc + bias)  (ConvNeXt gamma)
+    const float* R;       // RESID, TAPS (or null): [B][M][N]
+    const float* scale;   // with R: optional per-row scale of (acc + bias)  (ConvNeXt gamma)
     const float* noise;   // NOISE: explicit [B][N], or null
     int noise_rng;        // NOISE with noise == null: 1 = draw N(0,1) from the documented generator, 0 = zeros
     uint64_t noise_key;   // (seed, block) key of the generator

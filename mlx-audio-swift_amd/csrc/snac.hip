@@ -1182,6 +1182,7 @@ void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
     GemmParams p = p_in;
     if (!p.ldx) p.ldx = p.Tin;                                          // dense [B][C][T] tensors unless the caller says otherwise
     if (!p.ldy) p.ldy = p.Tout;
+    if (!p.R) p.scale = nullptr;                                        // the scale is the residual's, whichever kernel the shape selects
     MIS_REQUIRE(p.x_lo <= 0 && p.ldx >= p.Tin, MIS_ERR_GENERATION_FAILED, "bad codec GEMM strides");
     if (mode == GEMM_RESID && snake && p.alpha && p.R && !p.scale && p.bias && p.M == p.K && ru_fused_enabled() &&
         (p.M == 64 || p.M == 96 || p.M == 128 || p.M == 192)) {           // narrow unit tails: whole channel range per block (k_pw_fused)
