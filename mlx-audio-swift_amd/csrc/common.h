@@ -116,6 +116,14 @@ private:
     void run(uint8_t* host, uint8_t* dev, size_t n, bool to_host, hipStream_t s);
 };
 
+// Between a wave's LDS writes and its other lanes' reads of them (and the other way round).  The hardware keeps one wave's LDS accesses in order; the fences
+// keep the compiler from moving them, which the barrier alone, no memory operation, does not promise.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 static inline size_t round_up(size_t a, size_t b) { return (a + b - 1) / b * b; }
 static inline int cdiv(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 

@@ -320,7 +320,7 @@ __device__ __forceinline__ void grouped_decode_block(const GroupedDims& D, const
         float* dst = a < na ? L.q[a] : L.k;
 #pragma unroll
         for (int j = 0; j < 4; ++j) if (lane + 64 * j < D.Dp) dst[lane + 64 * j] = x[j] * inv * xw[j];
-        __builtin_amdgcn_wave_barrier();                                       // (one wave's LDS accesses stay in order)
+        wave_lds_fence();
 #pragma unroll
         for (int j = 0; j < 2; ++j) {                                          // rotation in place
             const int i = lane + 64 * j;

@@ -644,7 +644,7 @@ __global__ void __launch_bounds__(256) k_codec_final(const float* __restrict__ X
             for (int h = 0; h < 2; ++h) s[wave][i][h * 64 + lane] = ok[h] ? snake_f(v[i][h], a, ra) : 0.0f;
         }
         if (c0 + 4 * FIN_CH < C) load(c0 + 4 * FIN_CH);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
 #pragma unroll
         for (int i = 0; i < FIN_CH; ++i) {
             if (c0 + 4 * i >= C) break;
@@ -655,7 +655,7 @@ __global__ void __launch_bounds__(256) k_codec_final(const float* __restrict__ X
                 acc[1] += wk * s[wave][i][min(64 + lane + k, 127)];                  // (lanes 58 .. 63 of the second strip are halo)
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
     }
     __syncthreads();
     s[wave][0][lane] = acc[0];

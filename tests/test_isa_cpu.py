@@ -127,6 +127,20 @@ def test_whisper_cross_attention_keeps_two_pairs_of_key_tiles_in_flight():
             assert pro and min(pro) >= 8, (name, pro)
 
 
+def test_wave_barriers_stand_between_fences():
+    """__builtin_amdgcn_wave_barrier alone is no memory operation: a compiler may move the LDS accesses of other lanes' values across it (wave_lds_fence)."""
+    seen = 0
+    for src in sorted(os.listdir(CSRC)):
+        if not src.endswith((".hip", ".h")):
+            continue
+        lines = [l.split("//")[0].strip() for l in open(os.path.join(CSRC, src))]
+        for i, l in enumerate(lines):
+            if "__builtin_amdgcn_wave_barrier()" in l:
+                seen += 1
+                assert "fence(__ATOMIC_RELEASE" in lines[i - 1] and "fence(__ATOMIC_ACQUIRE" in lines[i + 1], (src, i + 1)
+    assert seen
+
+
 def test_token_engine_keeps_its_tile_buffers_in_registers():
     """csrc/token_engine.hip holds a phase's weight tiles in registers while the previous phase is still running (gate|up: 176 registers
     per matrix wave).  Two compiler behaviours once put them into scratch - tile addresses hoisted out of the layer loop (~200 registers
