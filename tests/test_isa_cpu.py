@@ -10,6 +10,8 @@ away silently - hipcc cross-compiles here.
 * The Whisper cross-attention schedule (`k_attn_decode<64, 2, XS>`) is plain C++ with compiler loads; what makes it fast is WHERE hipcc puts
   its waits - a pair of key tiles is requested before the wait for the pair in front of it (`s_waitcnt vmcnt(16)` behind sixteen requests,
   twice per tile count).  A loop form of the same code lost exactly that (vmcnt(0) at the loop header), so the property is pinned here.
+* k_gemm_big3 / k_gemm_kv_tiles read their second half's fragments (asm) under the first half's MFMAs, behind a counted wait that hipcc does not track: no
+  instruction on any path may touch a register whose read is still in flight.
 One compile per source file (lm_kernels.hip ~40 s, the others ~15 s each)."""
 import functools
 import os
@@ -91,6 +93,47 @@ def test_whisper_256_tile_gemm_and_quantised_r4_gemm_do_not_spill():
     assert len(q4) >= 24
     for k, v in q4.items():
         assert v["scratch"] == 0 and v["vgprs"] <= 256, (k, v)
+
+
+def _registers(operand):
+    m = re.fullmatch(r"([va])(?:(\d+)|\[(\d+):(\d+)\])", operand)
+    return frozenset((m[1], i) for i in range(int(m[2] or m[3]), int(m[2] or m[4]) + 1)) if m else frozenset()
+
+
+def test_whisper_256_tile_gemm_touches_no_fragment_in_flight():
+    text, _ = _compiled("whisper_kernels.hip")
+    names = re.findall(r"\n(_Z\w*(?:k_gemm_big3|k_gemm_kv_tiles)\w*):", text)
+    assert len(names) == 10
+    for name in names:
+        i = text.index("\n" + name + ":")
+        lines = [l.split(";")[0].strip() for l in text[i: text.index(".Lfunc_end", i)].split("\n")]
+        label = {l[:-1]: k for k, l in enumerate(lines) if re.fullmatch(r"\.LBB\w+:", l)}
+        todo, seen, most = [(0, ())], set(), 0
+        while todo:
+            k, flight = todo.pop()
+            while k < len(lines) and (k, flight) not in seen:
+                seen.add((k, flight))
+                l, k = lines[k], k + 1
+                if not re.match(r"[a-z]", l):
+                    continue
+                op, _, rest = l.partition(" ")
+                if op == "s_endpgm":
+                    break
+                if op == "s_waitcnt":
+                    m = re.search(r"lgkmcnt\((\d+)\)", l)
+                    flight = flight[max(0, len(flight) - int(m[1])):] if m else flight
+                    continue
+                if op == "s_branch" or op.startswith("s_cbranch"):
+                    todo.append((label[rest.strip()], flight))
+                    if op == "s_branch":
+                        break
+                    continue
+                operands = [_registers(t.strip().split(" ")[0]) for t in rest.split(",")]
+                assert not any(r & f for r in operands for f in flight), (name, l)
+                if op.startswith("ds_read"):
+                    flight += (operands[0],)
+                    most = max(most, len(flight))
+        assert most == 24, (name, most)                                 # both halves requested before the first is waited for
 
 
 def test_whisper_cross_attention_keeps_two_pairs_of_key_tiles_in_flight():
