@@ -126,11 +126,11 @@ struct AttnParams {
     const bf16_t *qp_lnw, *qp_lnb;
     float qp_eps;
     int qp_S, qp_KT;
-    // batched prefill: the rows of a launch are (position, sequence) pairs - row r uses the caches of sequence r % cache_rows (0 = r).
-    // append_only = 1: RoPE / norm the new key and value, write them to the caches, stop (all positions of a chunk first: the second
-    // launch then finds every earlier key of its own chunk in memory)
+    // short prompts (prefill_small): the rows of a launch are (position, sequence) pairs - row r uses the caches of sequence r % cache_rows (0 = r).
+    // append_only = 1: RoPE / norm the new key and value, write them to the caches, stop (all positions first: the second launch then finds
+    // every earlier key of its own prompt in memory)
     int cache_rows, append_only;
-    int first_schedule;      // 1: never k_attn_decode2 - the prefill's two arrangements must give the same bits whatever the batch size
+    int first_schedule;      // 1: never k_attn_decode2 - a prompt's pairs give the same bits whatever their number
 };
 void launch_attn_decode(const AttnParams& p, int batch, hipStream_t s);
 

@@ -4,9 +4,8 @@
 // the whole prompt through every layer at once.  The decode engine used to feed the prompt one position per step (L weight-streaming
 // passes: 56 ms of the 1.6 s bench job for 32-token prompts, and linear in L - voice-cloning prompts carry hundreds of audio tokens).
 // Here all L x B prompt tokens form the M dimension of four GEMMs per layer (M = 1024 at the bench shape), each weight byte is read
-// once per CHUNK of positions instead of once per position, and only the attention walks the positions one by one (the decode
-// attention kernel itself: it appends the position's key / value and attends causally, so caches, RoPE and q/k-norm are exactly the
-// sequential path's).  Rows are laid out position-major: row r = t * Mpad + b.
+// once per CHUNK of positions instead of once per position, and the attention takes the chunk's queries together over the decode step's
+// caches.  Rows are laid out position-major: row r = t * rs + b, rs rows per position (the batch).
 //
 //   k_pf_embed_rmsnorm  h[r] = E[token(b, t)], x[r] = RMSNorm(h[r]) (row-major), active / position tables of every (t, b)
 //   k_gemm_pf<EPI>      C[M][N] = X[M][K] . W^T with W in the decode path's packed MFMA-A tile layout [N/16][K/32][64][8]:
@@ -68,7 +67,7 @@ __global__ void __launch_bounds__(256) k_pf_embed_rmsnorm(const bf16_t* __restri
     }
 }
 // the same for engines that feed input embeddings instead of token ids (Qwen3-TTS talker): rows [Lmax][src_rows][d] computed by the
-// caller; `Mpad` here and in k_pf_embed_rmsnorm is the chunk's rows per position (the engine's Mpad, or the batch itself)
+// caller; `Mpad` here and in k_pf_embed_rmsnorm is the chunk's rows per position (the batch)
 __global__ void __launch_bounds__(256) k_pf_rows_rmsnorm(const bf16_t* __restrict__ rows, int src_rows, const int32_t* __restrict__ lens, int Lmax, int t0, int batch,
                                                          int Mpad, const bf16_t* __restrict__ wnorm, bf16_t* __restrict__ h, bf16_t* __restrict__ x,
                                                          int32_t* __restrict__ pos_tab, uint8_t* __restrict__ act_tab, int d, float eps) {

@@ -8,9 +8,12 @@ from oracle import llama as ollama
 pytestmark = pytest.mark.gpu
 
 WIDE = ollama.LlamaConfig(hidden_size=1024, num_hidden_layers=2, intermediate_size=1024, num_attention_heads=8, num_key_value_heads=1, head_dim=128, vocab_size=640)
+# eight kv heads: both shapes below reach 256 blocks of 256 queries, a row alone does not
+KV8 = {D: ollama.LlamaConfig(hidden_size=1024, num_hidden_layers=2, intermediate_size=1024, num_attention_heads=16, num_key_value_heads=8, head_dim=D, vocab_size=640)
+       for D in (64, 128)}
 
 
-@pytest.mark.parametrize("ocfg", [ollama.TINY, ollama.TINY_QWEN3, ollama.TINY64, WIDE], ids=["gqa3", "qknorm", "d64", "gqa8"])
+@pytest.mark.parametrize("ocfg", [ollama.TINY, ollama.TINY_QWEN3, ollama.TINY64, WIDE, KV8[64], KV8[128]], ids=["gqa3", "qknorm", "d64", "gqa8", "wide-d64", "wide-d128"])
 @pytest.mark.parametrize("shape", ["edges", "chunks"])
 def test_rows_have_the_same_bits_alone_and_in_a_batch_and_match_the_oracle(ocfg, shape):
     """A query's sums run over the key tiles in order whatever block, chunk or batch it belongs to, so a row's logits are the same bits in every
