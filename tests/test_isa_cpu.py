@@ -184,6 +184,13 @@ def test_wave_barriers_stand_between_fences():
     assert seen
 
 
+def test_streams_have_the_default_priority():
+    """Work on streams of different priorities has hung on this part for good."""
+    for src in sorted(os.listdir(CSRC)):
+        if src.endswith((".hip", ".h", ".cpp")):
+            assert "StreamCreateWithPriority" not in open(os.path.join(CSRC, src)).read(), src
+
+
 def test_token_engine_keeps_its_tile_buffers_in_registers():
     """csrc/token_engine.hip holds a phase's weight tiles in registers while the previous phase is still running (gate|up: 176 registers
     per matrix wave).  Two compiler behaviours once put them into scratch - tile addresses hoisted out of the layer loop (~200 registers
