@@ -5,8 +5,9 @@
 // <= 2^-25 of the product).  One 16-deep step is 6 x 32 cycles instead of 8 x 64 of v_mfma_f32_32x32x2_f32.  Error against 64 bits (2-norm over 2-norm,
 // this kernel / the exact-f32 one; K = 96, 128, 192; operands normal): 1.38e-7 / 1.77e-7, 1.65e-7 / 2.06e-7, 2.04e-7 / 2.49e-7; all of one sign: 1.14 / 1.44,
 // 1.29 / 1.60, 1.64 / 2.05; normal times exp(2 normal): 1.25 / 1.93, 1.42 / 2.00, 1.84 / 2.45: lower each time (6 roundings of the sum per 16 products, not 16).
-// Infinite operands: k_x6_gemm takes the outputs they reach again in f32; behind the Snake of the other two kernels an infinity is NaN in any arithmetic (an
-// infinite WEIGHT there gives NaN where the f32 kernels give an infinity or NaN).
+// Infinities and values past the largest bfloat16: k_x6_gemm takes the outputs they reach again in f32, k_x6_convt (whose Snake may be the identity) clamps the first
+// plane.  Behind a Snake that is none, an argument past 1e20 is infinite or NaN in any arithmetic.  (An infinite WEIGHT of the units or the transposed
+// convolution gives NaN where the f32 kernels give an infinity or NaN.)
 //
 //   k_x6_pack_w   A^T f32 -> the three planes as MFMA-A fragments (once per weight matrix, kept in the model's CodecPack)
 //   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels, for the encoders and for MIS_CODEC_EXACT_F32=1)
@@ -21,7 +22,9 @@
 __device__ __forceinline__ float x6_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
 
 #define X6_MAX 3.38953138925153547590470800371487866880e+38f      // the largest bfloat16
-// x = h + m + l exactly (three bfloat16, each the nearest to what is left): eight values of consecutive channels -> one 16-byte piece per plane
+// x = h + m + l exactly (three bfloat16, each the nearest to what is left): eight values of consecutive channels -> one 16-byte piece per plane.
+// CLAMP: the first plane of a value past the largest bfloat16 is that one, not infinity; the rest still fits the other two
+template <bool CLAMP>
 __device__ __forceinline__ void x6_split(const float (&v)[8], uint4& h, uint4& m, uint4& l) {
     uint32_t o[3][4];
 #pragma unroll
@@ -29,8 +32,7 @@ __device__ __forceinline__ void x6_split(const float (&v)[8], uint4& h, uint4& m
         float a = v[2 * i], b = v[2 * i + 1];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            // (the first plane of a value past the largest bfloat16 is that one, not infinity; the rest still fits the other two)
-            const float ca = q ? a : __builtin_amdgcn_fmed3f(a, -X6_MAX, X6_MAX), cb = q ? b : __builtin_amdgcn_fmed3f(b, -X6_MAX, X6_MAX);
+            const float ca = q || !CLAMP ? a : __builtin_amdgcn_fmed3f(a, -X6_MAX, X6_MAX), cb = q || !CLAMP ? b : __builtin_amdgcn_fmed3f(b, -X6_MAX, X6_MAX);
             const uint32_t ab = (uint32_t)f32_to_bf16(ca) | ((uint32_t)f32_to_bf16(cb) << 16);
             o[q][i] = ab;
             a -= __uint_as_float(ab << 16);
@@ -148,7 +150,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
                 for (int j = 0; j < 8; ++j) v[j] = x6_snake(v[j], pa2[c0 + kg * 8 + j], pra2[c0 + kg * 8 + j]);
                 uint4 h, m, l;
-                x6_split(v, h, m, l);
+                x6_split<false>(v, h, m, l);
                 ts[0][kg][n] = h; ts[1][kg][n] = m; ts[2][kg][n] = l;
             }
         }
@@ -171,7 +173,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                     v[j] = x6_snake(a + pb1[c], pa2[c], pra2[c]);
                 }
                 uint4 h, m, l;
-                x6_split(v, h, m, l);
+                x6_split<false>(v, h, m, l);
                 ts[0][kg][n] = h; ts[1][kg][n] = m; ts[2][kg][n] = l;
             }
         }
@@ -374,7 +376,7 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
             if constexpr (TAPS) x[j] = ok[slot] ? x[j] : 0.0f;
         }
         uint4 h, m, l;
-        x6_split(x, h, m, l);
+        x6_split<false>(x, h, m, l);
         bv[h2][0] = __builtin_bit_cast(bf16x8_t, h); bv[h2][1] = __builtin_bit_cast(bf16x8_t, m); bv[h2][2] = __builtin_bit_cast(bf16x8_t, l);
         if (!TAPS || ++tap == P.ntaps) { tap = 0; ++ks; }
     };
@@ -628,7 +630,7 @@ __device__ __forceinline__ void x6_convt_body(const GemmParams& p, const float* 
             x[j] = ok ? x6_snake(v[j], pa[c], pra[c]) : 0.0f;               // (the padding is zero behind Snake as well)
         }
         uint4 h, m, l;
-        x6_split(x, h, m, l);
+        x6_split<true>(x, h, m, l);
         __syncthreads();                                                    // the previous chunk's products are done
         ts[0][kg][col] = h; ts[1][kg][col] = m; ts[2][kg][col] = l;
 #pragma unroll
