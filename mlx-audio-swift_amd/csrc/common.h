@@ -25,6 +25,7 @@ mis_status mis_fail(mis_status code, const char* fmt, ...);
     do {                                                                                     \
         hipError_t _e = (expr);                                                              \
         if (_e != hipSuccess) {                                                              \
+            (void)hipGetLastError();      /* reported here, not by the next call's check */  \
             char _b[512];                                                                    \
             snprintf(_b, sizeof(_b), "%s failed: %s (%s:%d)", #expr, hipGetErrorString(_e),  \
                      __FILE__, __LINE__);                                                    \

@@ -771,7 +771,7 @@ static bool prefill_batched_ok(const mis_tts* c, int Lmax) {
 // profiles/r05_final_soprano_engine_kernel_stats.csv: 1.4 ms to prefill 23 positions of Soprano-80M - 7 % of a batch-1 generate; k_gemm_pf_ring,
 // which such grids take now, was not there to compare).  The
 // weight-streaming GEMMs of the decode step take up to 64 rows, their glue does residual + RMSNorm and writes the packed operand, and the
-// attention kernel already has the pair arrangement (append-only launch, then every pair as a row; first schedule, like the chunked pass).
+// attention kernel already has the pair arrangement (append-only launch, then every pair as a row of the first schedule).
 // Same rounding points as both other prefill forms; float32 summation orders are the decode step's.  MIS_PREFILL_SMALL=0 keeps k_gemm_pf / k_gemm_pf_ring.
 __global__ void k_pf_repack_rows(const bf16_t* __restrict__ src, int MT_src, int row0, bf16_t* __restrict__ dst, int MT_dst, int d) {
     const int m = blockIdx.x;

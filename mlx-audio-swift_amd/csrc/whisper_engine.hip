@@ -365,7 +365,8 @@ static void whisper_alloc_state(mis_whisper* c, int batch) {
     const int d = c->d, Ld = c->cfg.decoder_layers;
     int Mpad = (int)round_up(batch, 16);
     int Smax = (int)round_up(c->cfg.max_target_positions, 64);
-    c->batch = batch; c->Mpad = Mpad; c->Smax = Smax;
+    c->batch = 0;                                          // (until everything is there: an allocation that fails leaves no state for this batch behind)
+    c->Mpad = Mpad; c->Smax = Smax;
     c->S_qkv = split_for(3 * d / 16 / 2, d / 32, 8);      // attention prologue: <= 8 slabs
     c->S_o = split_for(d / 16 / 2, d / 32);
     c->S_cq = c->S_o;
@@ -387,6 +388,7 @@ static void whisper_alloc_state(mis_whisper* c, int batch) {
     c->part.alloc((size_t)std::max(std::max(c->S_o, c->S_cq), c->S_fc2) * Mpad * d);
     c->scratch.alloc(batch);
     sampler_scratch_init(c->scratch.p, batch, c->stream);
+    c->batch = batch;
 }
 
 static void whisper_decoder_reset(mis_whisper* c) {

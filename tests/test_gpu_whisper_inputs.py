@@ -1,4 +1,4 @@
-"""What Whisper's entry points take: rows much longer than a window, device memory that work on the default stream still writes or reads."""
+"""What Whisper's entry points take: rows much longer than a window, device memory that work on the default stream still writes or reads, more rows than memory."""
 import ctypes as C
 
 import numpy as np
@@ -7,7 +7,7 @@ import torch
 
 import mlx_audio_swift_amd as mas
 from mlx_audio_swift_amd import _lib
-from mlx_audio_swift_amd.generation import check
+from mlx_audio_swift_amd.generation import AudioGenerationError, check
 from oracle import whisper as owhisper
 
 pytestmark = pytest.mark.gpu
@@ -74,3 +74,17 @@ def test_device_memory_is_read_and_written_in_the_order_of_the_default_stream():
     busy()
     p.copy_(src_p)
     assert generate(dev, p.data_ptr(), [480000] * 9, 480000) == ids
+
+
+def test_an_allocation_that_fails_leaves_no_half_made_state():
+    """64 rows of 2 million decoder positions in 16 layers would be 1 TB of caches: refused each time, and one row still runs."""
+    ocfg = owhisper.TINY
+    cfg = mas.WhisperConfig(**{**{k: getattr(ocfg, k) for k in ocfg.__dataclass_fields__}, "decoder_layers": 16, "max_target_positions": 2_000_000})
+    dev = mas.WhisperModel.synthetic(cfg)
+    feats = np.random.default_rng(4).standard_normal((64, 3000, ocfg.num_mel_bins)).astype(np.float32)
+    for _ in range(2):
+        with pytest.raises(AudioGenerationError):
+            dev.encode(feats, want_output=False)
+    with pytest.raises(AudioGenerationError):
+        dev.decoder_forward(np.zeros(64, np.int32))
+    assert np.isfinite(dev.encode(feats[:1])).all()
