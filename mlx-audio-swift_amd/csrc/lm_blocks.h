@@ -60,6 +60,7 @@ public:
 
     // caches and step buffers for `batch` rows of up to Smax positions
     void reset(int batch, int Smax, hipStream_t s);
+    void forget() { batch_ = Smax_ = 0; }                         // the next reset sizes every buffer anew
     // one token of every active row (captured in the engine's decode graph); leaves the final norm of every row as the head's operand
     void enqueue_step(const BlockRows& r, hipStream_t s);
     void enqueue_head(hipStream_t s);   // logits of the batch rows: float32 [Mpad][Vpad]

@@ -576,11 +576,20 @@ static void build_rope_tables(mis_tts* c) {
     HIP_CHECK(hipStreamSynchronize(c->stream));
 }
 
+static void lm_reset_buffers(mis_tts* c, int batch, int max_context);
 static void lm_reset(mis_tts* c, int batch, int max_context) {
     MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "model not finalized");
     MIS_REQUIRE(batch >= 1 && batch <= 64, MIS_ERR_INVALID_INPUT, "batch per GPU must be 1..64 (got %d)", batch);
     MIS_REQUIRE(max_context >= 1, MIS_ERR_INVALID_INPUT, "max_context must be positive");
     HIP_CHECK(hipSetDevice(c->device));
+    try { lm_reset_buffers(c, batch, max_context); }
+    catch (...) {               // an allocation that fails half way leaves no shape behind: the next reset sizes caches and tables anew, and nothing runs before it
+        c->batch = c->Smax = 0;
+        if (c->blocks) c->blocks->forget();
+        throw;
+    }
+}
+static void lm_reset_buffers(mis_tts* c, int batch, int max_context) {
     hipStream_t s = c->stream;
     int Mpad = (int)round_up(batch, 16);
     int Smax = (int)round_up(max_context, 64);

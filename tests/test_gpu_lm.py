@@ -187,6 +187,27 @@ def test_batched_prefill_matches_oracle_and_the_position_by_position_path(ocfg, 
            rms_vs_sequential_worst=worst[2], rms_vs_sequential_mean=float(np.mean(d_all)), tol_max=TOL_MAX, tol_rms_mean=0.008, tol_rms_worst=0.016)
 
 
+def test_a_reset_that_fails_leaves_no_half_made_state():
+    """64 rows of 300 000 positions would be 2.5 GB x 64 of keys a layer: refused, and what runs after it has its own tables and caches."""
+    ocfg = ollama.LlamaConfig(hidden_size=256, num_hidden_layers=8, intermediate_size=256, num_attention_heads=8, num_key_value_heads=8, head_dim=128, vocab_size=640)
+    W, _, dev = lm_pair(ocfg, seed=5)
+    fresh = mas.LlamaTTSModel.from_weights(lm_host_config(ocfg), W)
+    ids = np.random.default_rng(1).integers(0, ocfg.vocab_size, 80).astype(np.int32)
+    dev.lm_reset(1, 64)
+    for _ in range(2):
+        with pytest.raises(mas.AudioGenerationError):
+            dev.lm_reset(64, 300_000)
+        with pytest.raises(mas.AudioGenerationError):
+            dev.lm_forward(np.zeros(64, np.int32))
+    for m in (dev, fresh):
+        m.lm_reset(1, 300_000)
+    with pytest.raises(mas.AudioGenerationError):
+        dev.lm_reset(65, 64)                                       # a refused argument changes nothing
+    for t in ids:                                                  # past the 64 positions of the first tables
+        a, b = dev.lm_forward(t[None]), fresh.lm_forward(t[None])
+    assert np.array_equal(a, b) and np.isfinite(a).all()
+
+
 @pytest.mark.parametrize("lens", [[23], [9, 4, 13], [2, 2], [16, 1, 7, 16]], ids=["1x23", "3_ragged", "2x2", "4x16_full"])
 def test_short_prompt_prefill_on_the_decode_step_kernels(lens, monkeypatch):
     """Round 6: prompts of at most 64 (position, row) pairs run on the DECODE STEP's kernels with the pairs as rows (`prefill_small`,

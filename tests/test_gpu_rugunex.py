@@ -372,3 +372,18 @@ def test_directory_and_commands(tmp_path):
     check(got[0], ref[[3, 19]], "float32")
     check(got[1], ref[[4, 20]], "float32")
     check(got[3], ref[[8]], "float32")
+
+
+def test_a_reset_that_fails_leaves_no_half_made_state():
+    """64 rows of 2.2 million positions of 576 values would be 324 GB a layer: refused each time, and one row still runs."""
+    W, m = build(wide(), "float32")
+    toks = tokens(40, 1000)
+    m.reset(1, 64)
+    want = run_all(m, toks)
+    for _ in range(2):
+        with pytest.raises(mas.AudioGenerationError):
+            m.reset(64, 2_200_000)
+        with pytest.raises(mas.AudioGenerationError):
+            m.extend([(0, toks)])
+    m.reset(1, 64)
+    assert np.array_equal(run_all(m, toks), want)
