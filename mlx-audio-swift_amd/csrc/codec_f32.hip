@@ -363,12 +363,15 @@ static void launch_f32(const GemmParams& p, int batch, hipStream_t s) {
     const bool near = std::max(p.ldx, p.ldy) <= 1 << 24;
     if constexpr (MODE == GEMM_TAPS) {
         if (codec_quarters(p)) {
-            // The same bits in all of them.  us, tiles / split form: 128 rows, K = 1792, 64000 columns (1000 blocks of the wide tile) 318 / 471, 4000 columns 53 / 36; 64
-            // rows, K = 1536, 100000 columns (782) 256 / 336, 20000 columns 73 / 72; 384 rows, K = 4608, eight rows of 2368 columns (888) 1012 / 1031, one 148 / 143; 192
-            // rows, K = 1152, 18944 columns (592) 195 / 154; 32 rows, K = 1536, 200000 columns (half of the tile empty) 569 / 351
-            if (near && p.M > 32 && p.M <= 64 && blocks(64, 128) >= 768) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint32_t, true>, 64, 128);
-            else if (near && p.M > 64 && blocks(128, 64) >= 768) go(k_codec_gemm<MODE, SNAKE, 32, 2, 2, 2, 1, 16, 2, uint32_t, true>, 128, 64);
-            else {
+            // The same bits in all of them.  The tiles where their rows are (nearly) full and their blocks come near to filling the chip once.  us, tiles / split form:
+            // 512 rows, K = 3840, 8000 / 9600 / 12000 columns (500 / 600 / 752 blocks) 439 / 500, 541 / 591, 545 / 744; 1024 rows, K = 12288, 5000 columns (632) 1715 /
+            // 1937, 1500 columns (192) 1033 / 601; 384 rows, K = 4608, 8000 columns (375) 528 / 450; 64 rows, K = 1536, 60000 columns (469) 187 / 201, 20000 columns
+            // 73 / 72; rows three quarters full: 192 rows, K = 1152, 60000 columns (1876) 490 / 442; 48 rows, K = 1536, 100000 columns (782) 370 / 326
+            const bool narrow = p.M <= 64;
+            if (near && 8 * p.M >= 7 * (narrow ? 64 : cdiv(p.M, 128) * 128) && blocks(narrow ? 64 : 128, narrow ? 128 : 64) >= 448) {
+                if (narrow) go(k_codec_gemm<MODE, SNAKE, 32, 1, 4, 2, 1, 16, 2, uint32_t, true>, 64, 128);
+                else go(k_codec_gemm<MODE, SNAKE, 32, 2, 2, 2, 1, 16, 2, uint32_t, true>, 128, 64);
+            } else {
                 const int nt = cdiv(p.N, 16);
                 hipLaunchKernelGGL(k_codec_gemm_split, dim3(cdiv(p.M, 32), std::min(nt, CODEC_SPLIT_NY), batch * cdiv(nt, CODEC_SPLIT_NY)), dim3(256), 0, s, p, batch);
             }
