@@ -96,6 +96,7 @@ int gemm_choose_split(int items, int KT, int ksb, int s_max);
 
 struct AttnParams;
 bool attn_qp_ok(const AttnParams& p);
+size_t attn_cross_part_floats(int rows, int H);
 struct AttnParams {
     const float* qkv_part;   // [S][Mpad][Nqkv]
     int S, Mpad, Nqkv;
@@ -116,7 +117,7 @@ struct AttnParams {
     int H, Hkv, D, Smax;
     float scale;
     unsigned long long* dbg; // phase timestamps (MIS_ATTN_TIMING builds only), else null
-    // cross-attention with the glue and the query projection in its prologue (qp_w != null; see attn_qp_row_gemv): q = T(W_q LN(h_new) + b),
+    // cross-attention with the glue and the query projection in its prologue (qp_w != null): q = T(W_q LN(h_new) + b),
     // h_new = T(h_in + T(sum of the qp_S slabs [qp_S][Mpad][H D])) written to qp_h_out (!= qp_h_in) by the head-0 blocks; qkv_part / S unused
     const bf16_t* qp_w;      // W_q packed [H D / 16][qp_KT][64][8]
     const bf16_t* qp_bias;   // [H D] or null
@@ -130,6 +131,8 @@ struct AttnParams {
     // append_only = 1: RoPE / norm the new key and value, write them to the caches, stop (all positions first: the second launch then finds
     // every earlier key of its own prompt in memory)
     int cache_rows, append_only;
+    float* xa_part;          // [B][H][16][66] partial sums and [B][H] counters (zero between launches) of a cross-attention over several blocks a head, or null
+    unsigned* xa_count;
     int first_schedule;      // 1: never k_attn_decode2 - a prompt's pairs give the same bits whatever their number
 };
 void launch_attn_decode(const AttnParams& p, int batch, hipStream_t s);

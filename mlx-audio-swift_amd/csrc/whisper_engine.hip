@@ -43,6 +43,8 @@ struct mis_whisper {
     DevBuf<bf16_t> cross_k, cross_v, self_k, self_v, enc_out;
     DevBuf<int32_t> ids, pos_cur, pos_next, n_gen, tokens_out, next_ids, done_count, sup, bsup;
     DevBuf<uint8_t> active;
+    DevBuf<float> xa_part;                               // partial sums of the cross-attention over several blocks a head; its counters
+    DevBuf<unsigned> xa_count;
     DevBuf<bf16_t> h, h2, x, attn_out, act, logits;      // h2: the other residual buffer of the folded glue (enqueue_decoder_step)
     DevBuf<float> qkv_part, part, e_buf, logits_f32;
     DevBuf<SamplerScratch> scratch;
@@ -386,6 +388,8 @@ static void whisper_alloc_state(mis_whisper* c, int batch) {
     c->logits.alloc((size_t)Mpad * c->Vpad); c->e_buf.alloc((size_t)Mpad * c->Vpad);
     c->qkv_part.alloc((size_t)c->S_qkv * Mpad * 3 * d);
     c->part.alloc((size_t)std::max(std::max(c->S_o, c->S_cq), c->S_fc2) * Mpad * d);
+    c->xa_part.alloc(attn_cross_part_floats(batch, c->Hd)); c->xa_count.alloc((size_t)batch * c->Hd);
+    c->xa_count.zero(c->stream);
     c->scratch.alloc(batch);
     sampler_scratch_init(c->scratch.p, batch, c->stream);
     c->batch = batch;
@@ -515,7 +519,7 @@ extern "C" mis_status mis_whisper_encode(mis_whisper* c, const float* features, 
 // Up to 16 rows (the BASELINE share: 8 windows per GPU) two of the three residual + LayerNorm glue launches of a layer - and one GEMM launch -
 // run inside the prologue of their consumer: 8 launches per layer instead of 11 (transcribe 228 -> 214 ms per 8 x 30 s, profiles/r06/c4, c5).
 //   bit 4 (16): h += self-attention output, LayerNorm 2 AND the cross-attention's query projection inside the cross-attention kernel
-//               (k_attn_decode<64, 2, true, QP>, lm_kernels.hip: a block is one (row, head) and rebuilds only its row);
+//               (k_attn_cross, lm_kernels.hip: a block is one (row, head) and rebuilds only its row);
 //   bit 2 (4):  h += cross-attention output and LayerNorm 3 inside fc1's prologue (k_gemm_skinny_norm: every block rebuilds all rows);
 //   bit 3 (8):  fail where a requested fold does not apply (tests).  MIS_WHISPER_FOLD=0 keeps the separate launches.
 // The residual stream alternates between two buffers: every block of a consumer still reads the old one while one of them writes the new.
@@ -532,7 +536,7 @@ static void enqueue_decoder_step(mis_whisper* c) {
     const char* fe = getenv("MIS_WHISPER_FOLD");
     const int want = fe ? atoi(fe) : WHISPER_FOLD_DEFAULT;
     AttnParams probe{};
-    probe.cross = 1; probe.cross_len = 1500; probe.D = D; probe.H = H; probe.Hkv = H; probe.qp_KT = d / 32; probe.qp_S = c->S_o;
+    probe.cross = 1; probe.cross_len = 1500; probe.D = D; probe.H = H; probe.Hkv = H; probe.qp_KT = d / 32; probe.qp_S = c->S_o; probe.xa_part = c->xa_part.p;
     const bool f_cqa = (want & 16) && Mpad == 16 && attn_qp_ok(probe);
     const bool f_fc1 = (want & 4) && gemm_skinny_norm_ok(EPI_GELU_PACKED, 2, d / 32, 1, c->S_o, Mpad, c->batch);
     MIS_REQUIRE(!(want & 8) || (f_cqa == !!(want & 16) && f_fc1 == !!(want & 4)), MIS_ERR_GENERATION_FAILED,
@@ -569,7 +573,7 @@ static void enqueue_decoder_step(mis_whisper* c) {
         cp.kcache = c->cross_k.p + li * cs; cp.vtcache = c->cross_v.p + li * cs;
         cp.pos = c->pos_cur.p; cp.active = c->active.p; cp.rope_cos = nullptr; cp.rope_sin = nullptr;
         cp.out = c->attn_out.p; cp.H = H; cp.Hkv = H; cp.D = D; cp.Smax = c->Spad; cp.scale = 1.0f / sqrtf((float)D);
-        cp.cross = 1; cp.cross_len = 1500;
+        cp.cross = 1; cp.cross_len = 1500; cp.xa_part = c->xa_part.p; cp.xa_count = c->xa_count.p;
         launch_attn_decode(cp, c->batch, s);
         launch_gemm_skinny(EPI_PARTIAL, 2, 4, L.co, c->attn_out.p, c->part.p, d / 16, d / 32, c->S_o, d, Mpad, s, L.cbo);
         // MLP (:245-249)
