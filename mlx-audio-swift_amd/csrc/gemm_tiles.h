@@ -1,0 +1,117 @@
+#pragma once
+#include "common.h"
+
+__device__ __forceinline__ uint32_t gt_lds_offset(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
+
+// acc[i][j] += W tile (128 wn + 16 i) x X tile (16 TM wm + 16 j) of a block of four waves (wn = wave >> 1, wm = wave & 1)
+template <int TM, bool PACKED>
+struct GemmTiles {
+    static constexpr int TN = 8, BN = 256, BM = 32 * TM, BK = 64, QW = 8, QX = TM, NQ = QW + QX;
+    static constexpr int WB = BN * BK * 2, XB = BM * BK * 2, STEP = WB + XB;       // bytes of a k-step
+    static constexpr int NBUF = STEP * 3 <= 160 * 1024 ? 3 : 2;
+    static constexpr int LDS = NBUF * STEP;
+
+    // tile t of `tiles` for t = first, first + stride, ...: woff(t, q, lane) / xoff(t, row): element offsets of a lane's piece of W and of the start of an X row;
+    // epi(t, acc) stores a finished tile
+    template <class FW, class FX, class FE>
+    static __device__ __forceinline__ void run(unsigned char* lds, const bf16_t* Wb, const bf16_t* Xb, int K, int first, int stride, int tiles, FW woff, FX xoff, FE epi) {
+        const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wave >> 1, wm = wave & 1;
+        const int KS = K / BK;
+        uint32_t off[NQ];                                            // bytes
+        auto point = [&](int t) {
+#pragma unroll
+            for (int q = 0; q < QW; ++q) off[q] = 2 * (uint32_t)woff(t, wave * QW + q, lane);
+#pragma unroll
+            for (int q = 0; q < QX; ++q) {
+                const int r = (wave * QX + q) * 8 + (lane >> 3);
+                off[QW + q] = 2 * ((uint32_t)xoff(t, r) + ((lane & 7) ^ ((r >> 1) & 7)) * 8);
+            }
+        };
+        auto stage1 = [&](int buf, int ks, int n) {                  // the n-th LDS load of a k-step
+            unsigned char* l = lds + buf * STEP;
+            const unsigned char* src = n < QW ? reinterpret_cast<const unsigned char*>(Wb) + (size_t)ks * (PACKED ? 2048 : 128) : reinterpret_cast<const unsigned char*>(Xb) + (size_t)ks * 128;
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + off[n]),
+                                             (__attribute__((address_space(3))) void*)(l + (n < QW ? (wave * QW + n) * 1024 : WB + (wave * QX + n - QW) * 1024)), 16, 0, 0);
+        };
+        const int sw = (lane >> 1) & 7;
+        const uint32_t base = gt_lds_offset(lds);
+        const uint32_t p0 = ((lane >> 4) ^ sw) * 16, p1 = ((4 + (lane >> 4)) ^ sw) * 16;
+        // fragment i of half h: PACKED image [16 n-tiles][2][1 KB] lane-linear, else rows of 128 bytes, swizzled
+        const uint32_t w0 = base + (PACKED ? wn * TN * 2048 + lane * 16 : (wn * TN * 16 + (lane & 15)) * 128 + p0);
+        const uint32_t w1 = base + (PACKED ? wn * TN * 2048 + 1024 + lane * 16 : (wn * TN * 16 + (lane & 15)) * 128 + p1);
+        const uint32_t x0 = base + WB + (wm * TM * 16 + (lane & 15)) * 128 + p0;
+        const uint32_t x1 = base + WB + (wm * TM * 16 + (lane & 15)) * 128 + p1;
+        bf16x8_t a[2][TN], b[2][TM];
+        auto read = [&](int n, uint32_t w, uint32_t x, bf16x8_t (&fa)[TN], bf16x8_t (&fb)[TM]) {        // the n-th fragment of a half: X first
+            if (n < TM) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[n < TM ? n : 0]) : "v"(x), "n"((n < TM ? n : 0) * 2048) : "memory");
+            else asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fa[n < TM ? 0 : n - TM]) : "v"(w), "n"((n < TM ? 0 : n - TM) * 2048) : "memory");
+        };
+        auto bind = [&](bf16x8_t (&fa)[TN], bf16x8_t (&fb)[TM]) {
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[0]) :: "memory");
+#pragma unroll
+            for (int i = 1; i < TN; ++i) asm volatile("" : "+v"(fa[i]));
+#pragma unroll
+            for (int j = 0; j < TM; ++j) asm volatile("" : "+v"(fb[j]));
+        };
+        constexpr int NF = TN + TM, S = TM > 6 ? 3 : 2;             // fragments of a half; one is requested behind every S-th MFMA
+        static_assert(NF == NQ && NF * S <= TN * TM, "every request of a half stands between its MFMAs");
+        f32x4_t acc[TN][TM];
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        int t = first, buf = 0;
+        point(t);
+#pragma unroll
+        for (int i = 0; i < NBUF; ++i)
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) stage1(i, i, n);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 1) * NQ) : "memory");
+        __builtin_amdgcn_s_barrier();
+#pragma unroll
+        for (int n = 0; n < NF; ++n) read(n, w0, x0, a[0], b[0]);
+        auto step = [&](int kn) {                                    // multiplies the k-step in `buf`, requests step kn behind it
+            const int nb = buf + 1 == NBUF ? 0 : buf + 1;
+            const uint32_t wo = w1 + buf * STEP, xo = x1 + buf * STEP, wx = w0 + nb * STEP, xx = x0 + nb * STEP;
+            bind(a[0], b[0]);
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j) {
+                    const int n = i * TM + j;
+                    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[0][i]), "v"(b[0][j]));
+                    if (n % S == S - 1 && n / S < NF) read(n / S, wo, xo, a[1], b[1]);
+                }
+            bind(a[1], b[1]);                                       // this wave's reads of the buffer are done
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * NQ) : "memory");        // its part of the next k-step has landed
+            __builtin_amdgcn_s_barrier();                           // everybody's
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j) {
+                    const int n = i * TM + j;
+                    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(a[1][i]), "v"(b[1][j]));
+                    if (n % S == S - 1 && n / S < NF) { read(n / S, wx, xx, a[0], b[0]); stage1(buf, kn, n / S); }
+                }
+            buf = nb;
+        };
+        for (;;) {
+#pragma unroll 1
+            for (int ks = NBUF; ks < KS; ++ks) step(ks);
+            const bool more = t + stride < tiles;                   // the last NBUF steps request the next tile's first ones (or their own last one again, never read)
+            if (more) point(t + stride);
+#pragma unroll 1
+            for (int i = 0; i < NBUF; ++i) step(more ? i : KS - 1);
+            bind(a[0], b[0]);
+            asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");         // (the last products are in their registers before anything reads them)
+            epi(t, acc);
+            if (!more) break;
+            t += stride;
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // (no DMA into the LDS of a block that has ended)
+    }
+};

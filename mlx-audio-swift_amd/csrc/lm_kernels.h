@@ -131,7 +131,7 @@ struct AttnParams {
     // append_only = 1: RoPE / norm the new key and value, write them to the caches, stop (all positions first: the second launch then finds
     // every earlier key of its own prompt in memory)
     int cache_rows, append_only;
-    float* xa_part;          // [B][H][16][66] partial sums and [B][H] counters (zero between launches) of a cross-attention over several blocks a head, or null
+    float* xa_part;          // [B][H][8][66] partial sums and [B][H] counters (zero between launches) of a cross-attention over several blocks a head, or null
     unsigned* xa_count;
     int first_schedule;      // 1: never k_attn_decode2 - a prompt's pairs give the same bits whatever their number
 };

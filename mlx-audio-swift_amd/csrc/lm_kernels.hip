@@ -1222,8 +1222,31 @@ void gemm_choose_dual_split(int items, int kt1, int kt2, int ksb, int s_max, int
 #define ATT_STAMP(i) do { } while (0)
 #endif
 
-template <int D, int NIT>
+// XS ("cross stream", round 4): the schedule for cross-attention over a LONG static cache (Whisper: 1500 keys = 47 tiles, five or six per
+// wave).  The loop below requests a pair of tiles, waits for it and multiplies - per wave two or three dependent round trips, of which
+// only the first hides behind the prologue.  With XS a wave holds TWO pairs in registers (D = 64: 4 x 32 registers): while one group is
+// multiplied the next pair streams, and the pair behind that is requested before the wait for it.  An odd tile count is taken out up
+// front (the first group is ONE tile, every later group a full pair); the code is straight-line per tile count (see the main loop for
+// why not a loop).  Tiles are multiplied in the same order as without XS - results are bit-identical.  The K/V loads are
+// non-temporal: a decode step reads each of them once (61 MB per layer at eight windows, 2 GB per step - nothing a cache can keep).
+// QP ("query projection", round 6; Whisper cross-attention at <= 16 rows): the residual add + LayerNorm glue in front of the
+// cross-attention AND its query projection run inside this kernel's prologue instead of as two launches of their own (k_glue4 4.6 us +
+// k_gemm_skinny 5.1 us per layer under the profiler).  A block is one (row, head): it needs ONE row of the glue - S_in slabs x 5 KB at
+// d = 1280, rebuilt by each of its eight waves with wave-local DPP sums (no barrier) - and 64 rows of W_q (164 KB out of L2: the eight
+// rows' blocks of a head share them).  Wave w owns k-tiles [KT w / 8, KT (w + 1) / 8): it rebuilds THAT slice of the row (<= 160 columns, one
+// group of four per lane), the row statistics meet in LDS (two raw barriers: mean, then variance - the glue's two-pass form), and it
+// multiplies its slice with the head's four n-tiles on the matrix core (B = the row as column 0); the eight partial vectors meet in LDS
+// behind the barrier the prologue has anyway.  The W_q tiles, the slice and the wave's first K/V tile are requested together, the second
+// tile behind the projection.  The head-0 blocks write h_new to the OTHER residual buffer.  Contrast with k_gemm_skinny_norm (same fold
+// on the GEMM side, measured neutral: every one of its 160-480 blocks re-reads ALL rows' slabs): a row-parallel consumer re-reads its row.
+// (First form, profiles/r06/c4: every wave rebuilt the WHOLE row and the K/V request waited behind the projection: 13.5 -> 17.8 us.)
+#define ATT_QP_KW 5
+#define ATT_QP_LDS ((size_t)ATT_WAVES * ATT_QP_KW * 32 * 2 + (size_t)ATT_WAVES * 64 * 4 + 2 * ATT_WAVES * 4)
+#define ATT_XS_MIN_J 5
+#define ATT_XS_MAX_J 6
+template <int D, int NIT, bool XS = false, int QP = 0>          // QP = slabs fetched per trip by the query-projection prologue (0: off)
 __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
+    static_assert(QP == 0 || (XS && D == 64), "QP: the cross-attention schedule at head_dim 64");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int kvh = blockIdx.x, b = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1254,8 +1277,38 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
     const int n_pro = p.cross ? G : G + 2;          // cross attention: queries only (K/V cached once per utterance)
     const int n_el = n_pro * D;
     float pv[NIT][8];                                // NIT * 512 >= (G + 2) * D
+    float* qp_part = sO + (size_t)ATT_WAVES * G * D + (size_t)ATT_WAVES * ATT_QP_KW * 16;      // [W][64] behind the waves' x strips (QP only)
+    float* qp_red = qp_part + ATT_WAVES * 64;                                                  // [2][W] row statistics
+    // QP, round trip 1: this wave's W_q tiles (k-tiles [k0, k1) of the head's four n-tiles) and its slice of the row
+    [[maybe_unused]] bf16x8_t qp_wt[QP > 0 ? ATT_QP_KW : 1][4];
+    [[maybe_unused]] uint2 qp_hq, qp_wq, qp_bq;
+    [[maybe_unused]] f32x4_t qp_v[QP > 0 ? QP : 1];
+    [[maybe_unused]] int qp_k0 = 0, qp_k1 = 0, qp_col = 0;
+    if constexpr (QP > 0) {
+        const int wq_ = __builtin_amdgcn_readfirstlane(wave);
+        const int KT = p.qp_KT, N = KT * 32;
+        qp_k0 = (KT * wq_) / ATT_WAVES; qp_k1 = (KT * (wq_ + 1)) / ATT_WAVES;
 #pragma unroll
-    for (int it = 0; it < NIT; ++it) {
+        for (int u = 0; u < ATT_QP_KW; ++u) {
+            int kk = qp_k0 + u;
+            kk = kk < KT ? kk : KT - 1;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)      // (cached loads: the other rows' blocks of this head read the same tiles)
+                qp_wt[u][r] = *(reinterpret_cast<const bf16x8_t*>(p.qp_w) + ((size_t)(kvh * 4 + r) * KT + kk) * 64 + lane);
+        }
+        qp_col = 32 * qp_k0 + 4 * lane;                                  // one group of four columns per lane (<= 160 per wave)
+        const int colc = qp_col < 32 * qp_k1 ? qp_col : N - 4;
+        qp_hq = *reinterpret_cast<const uint2*>(p.qp_h_in + (size_t)b * N + colc);
+        qp_wq = *reinterpret_cast<const uint2*>(p.qp_lnw + colc);
+        qp_bq = *reinterpret_cast<const uint2*>(p.qp_lnb + colc);
+#pragma unroll
+        for (int j = 0; j < QP; ++j) {
+            const int sj = j < p.qp_S ? j : p.qp_S - 1;
+            qp_v[j] = *reinterpret_cast<const f32x4_t*>(p.qp_slabs + ((size_t)sj * p.Mpad + b) * N + colc);
+        }
+    }
+#pragma unroll
+    for (int it = 0; it < (QP > 0 ? 0 : NIT); ++it) {
         const int idx = tid + it * 512;
         int hh = idx / D, d = idx - hh * D;
         if (idx >= n_el) { hh = 0; d = 0; }          // clamped: loaded, never used
@@ -1293,8 +1346,10 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
     // whole first tile pair, i.e. at contexts <= 512 for the entire KV stream of the launch)
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
+        if constexpr (QP == 0) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(pv[it][j]));
+            for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(pv[it][j]));
+        }
         asm volatile("" : "+v"(rc[it]));
         asm volatile("" : "+v"(rs[it]));
     }
@@ -1313,20 +1368,130 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
     const int n_tiles = p.append_only ? 0 : (kv_len + 31) >> 5;    // append-only launches request no tiles
     const int new_tile = p.cross ? -1 : (pos >> 5);
     bf16x8_t kA[2][D / 32], kB[2][D / 32], vA[D / 16], vB[D / 16];
+    if constexpr (XS && QP == 0) {                  // (an odd first group leaves B unrequested; the binding statement below names it)
+        const bf16x8_t z = (bf16x8_t){0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c) { kB[0][c] = z; kB[1][c] = z; }
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) vB[dt] = z;
+    }
     auto load_tile = [&](int tile, bf16x8_t (&ka)[2][D / 32], bf16x8_t (&vb)[D / 16]) {
+        if constexpr (XS) {
 #pragma unroll
-        for (int c = 0; c < D / 32; ++c) {
-            ka[0][c] = kbase[((size_t)tile * 2) * (D / 32) * 64 + c * 64];
-            ka[1][c] = kbase[((size_t)tile * 2 + 1) * (D / 32) * 64 + c * 64];
+            for (int c = 0; c < D / 32; ++c) {
+                ka[0][c] = __builtin_nontemporal_load(kbase + ((size_t)tile * 2) * (D / 32) * 64 + c * 64);
+                ka[1][c] = __builtin_nontemporal_load(kbase + ((size_t)tile * 2 + 1) * (D / 32) * 64 + c * 64);
+            }
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) vb[dt] = __builtin_nontemporal_load(vbase + ((size_t)tile * (D / 16) + dt) * 64);
+        } else {
+#pragma unroll
+            for (int c = 0; c < D / 32; ++c) {
+                ka[0][c] = kbase[((size_t)tile * 2) * (D / 32) * 64 + c * 64];
+                ka[1][c] = kbase[((size_t)tile * 2 + 1) * (D / 32) * 64 + c * 64];
+            }
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) vb[dt] = vbase[((size_t)tile * (D / 16) + dt) * 64];
         }
-#pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) vb[dt] = vbase[((size_t)tile * (D / 16) + dt) * 64];
     };
+    // XS: tiles of this wave (wave, wave + 8, ...); an odd count is taken out up front so that every later group is a full pair
+    // (the wave index as an SGPR: with `tid >> 6` the compiler treats every branch on it as divergent, lowers the loop below through
+    // exec masks and re-joins its arms - with a vmcnt(0) at the join)
+    const int wu = XS ? __builtin_amdgcn_readfirstlane(wave) : wave;
+    const int xs_nj = XS && wu < n_tiles ? (n_tiles - wu + ATT_WAVES - 1) / ATT_WAVES : 0;
+    const bool xs_odd = (xs_nj & 1) != 0;
     __builtin_amdgcn_sched_barrier(0);
     // wave-uniform guards: a wave without a tile requests nothing (at short contexts seven of eight waves would otherwise each
     // pull a redundant 32 KB pair through the CU's 64 B/clk return path - 2-3 us per launch on the small models)
-    if (wave < n_tiles) load_tile(wave, kA, vA);
-    if (wave + ATT_WAVES < n_tiles) load_tile(wave + ATT_WAVES, kB, vB);
+    if constexpr (QP > 0) {
+        // the first tile UNCONDITIONALLY (the launcher admits >= ATT_XS_MIN_J tiles per wave): no join between the requests above and the
+        // projection below, so its waits count loads instead of draining them; the second tile of an even count follows the projection
+        load_tile(wu, kA, vA);
+        __builtin_amdgcn_sched_barrier(0);
+        const int N = p.qp_KT * 32;
+        const bool live = qp_col < 32 * qp_k1;
+        float acc4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < QP; ++j) {                    // slab order 0, 1, 2, ... (fixed => deterministic)
+            const bool on = j < p.qp_S;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc4[e] += on ? qp_v[j][e] : 0.0f;
+        }
+        const float hv[4] = {bf16_to_f32((bf16_t)(qp_hq.x & 0xffffu)), bf16_to_f32((bf16_t)(qp_hq.x >> 16)), bf16_to_f32((bf16_t)(qp_hq.y & 0xffffu)),
+                             bf16_to_f32((bf16_t)(qp_hq.y >> 16))};
+        float hn[4], sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            hn[e] = bf16_round_f32(hv[e] + bf16_round_f32(acc4[e]));                // o = T(sum slabs); h = T(h + o)
+            sum += live ? hn[e] : 0.0f;
+        }
+        sum = wave_sum_dpp(sum);
+        if (lane == 0) qp_red[wu] = sum;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");          // (raw: __syncthreads() would wait for the K/V tile as well)
+        float tot = 0.f;
+#pragma unroll
+        for (int w = 0; w < ATT_WAVES; ++w) tot += qp_red[w];
+        const float mean = tot / (float)N;
+        float sq = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const float dl = hn[e] - mean; sq += live ? dl * dl : 0.0f; }
+        sq = wave_sum_dpp(sq);
+        if (lane == 0) qp_red[ATT_WAVES + wu] = sq;
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        float tq = 0.f;
+#pragma unroll
+        for (int w = 0; w < ATT_WAVES; ++w) tq += qp_red[ATT_WAVES + w];
+        const float rstd = 1.0f / sqrtf(tq / (float)N + p.qp_eps);
+        bf16_t* xrow = reinterpret_cast<bf16_t*>(sO + (size_t)ATT_WAVES * G * D) + (size_t)wu * ATT_QP_KW * 32;
+        if (live) {
+            const float wv[4] = {bf16_to_f32((bf16_t)(qp_wq.x & 0xffffu)), bf16_to_f32((bf16_t)(qp_wq.x >> 16)), bf16_to_f32((bf16_t)(qp_wq.y & 0xffffu)),
+                                 bf16_to_f32((bf16_t)(qp_wq.y >> 16))};
+            const float bv[4] = {bf16_to_f32((bf16_t)(qp_bq.x & 0xffffu)), bf16_to_f32((bf16_t)(qp_bq.x >> 16)), bf16_to_f32((bf16_t)(qp_bq.y & 0xffffu)),
+                                 bf16_to_f32((bf16_t)(qp_bq.y >> 16))};
+            bf16_t xb[4], hb[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                xb[e] = f32_to_bf16((hn[e] - mean) * rstd * wv[e] + bv[e]);
+                hb[e] = f32_to_bf16(hn[e]);
+            }
+            *reinterpret_cast<uint2*>(xrow + 4 * lane) = make_uint2((uint32_t)xb[0] | ((uint32_t)xb[1] << 16), (uint32_t)xb[2] | ((uint32_t)xb[3] << 16));
+            if (kvh == 0)                                 // the head-0 block of the row keeps the residual stream (its waves cover the row)
+                *reinterpret_cast<uint2*>(p.qp_h_out + (size_t)b * N + qp_col) =
+                    make_uint2((uint32_t)hb[0] | ((uint32_t)hb[1] << 16), (uint32_t)hb[2] | ((uint32_t)hb[3] << 16));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the strip is this wave's own: LDS operations of one wave execute in order)
+        f32x4_t qacc[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) qacc[r] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        const bf16x8_t z = (bf16x8_t){0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int u = 0; u < ATT_QP_KW; ++u) {
+            bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(xrow + u * 32 + (lane >> 4) * 8);
+            if ((lane & 15) != 0 || qp_k0 + u >= qp_k1) xf = z;         // B = the row as column m = 0; dead k-tiles multiply zero
+#pragma unroll
+            for (int r = 0; r < 4; ++r) qacc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qp_wt[u][r], xf, qacc[r], 0, 0, 0);
+        }
+        if ((lane & 15) == 0) {                               // C/D lane l, reg e: n = (l >> 4) * 4 + e, m = l & 15
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                *reinterpret_cast<float4*>(qp_part + wu * 64 + r * 16 + (lane >> 4) * 4) = make_float4(qacc[r][0], qacc[r][1], qacc[r][2], qacc[r][3]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        {                                               // (B's registers are free of the W_q tiles only now)
+            const bf16x8_t zb = (bf16x8_t){0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+            for (int c = 0; c < D / 32; ++c) { kB[0][c] = zb; kB[1][c] = zb; }
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) vB[dt] = zb;
+        }
+        if (xs_nj >= 2 && !xs_odd) load_tile(wu + ATT_WAVES, kB, vB);
+    } else if constexpr (XS) {
+        if (xs_nj >= 1) load_tile(wu, kA, vA);
+        if (xs_nj >= 2 && !xs_odd) load_tile(wu + ATT_WAVES, kB, vB);
+    } else {
+        if (wave < n_tiles) load_tile(wave, kA, vA);
+        if (wave + ATT_WAVES < n_tiles) load_tile(wave + ATT_WAVES, kB, vB);
+    }
     __builtin_amdgcn_sched_barrier(0);
     ATT_STAMP(2);
 #pragma unroll
@@ -1334,8 +1499,10 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
         const int idx = tid + it * 512;
         // unconditional (sraw is padded to NIT*512 entries; entries >= n_el hold clamped-address garbage nobody reads)
         float acc = 0.0f;
+        if constexpr (QP == 0) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc += (j < p.S) ? pv[it][j] : 0.0f;   // slab order 0..7 (S <= 8, checked by the launcher)
+            for (int j = 0; j < 8; ++j) acc += (j < p.S) ? pv[it][j] : 0.0f;   // slab order 0..7 (S <= 8, checked by the launcher)
+        }
         sraw[idx] = bf16_round_f32(acc);
     }
     for (int idx = tid; idx < 16 * D; idx += 512) qs[idx] = 0;
@@ -1366,7 +1533,14 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
         const int idx = tid + it * 512;
         if (idx >= n_rot_el) continue;
         int hh = idx / (D / 2), i = idx - hh * (D / 2);
-        const float x1 = sraw[hh * D + i], x2 = sraw[hh * D + i + D / 2];
+        float x1 = sraw[hh * D + i], x2 = sraw[hh * D + i + D / 2];
+        if constexpr (QP > 0) {                      // (cross-attention, G = 1: hh = 0) q = T(W_q x + b): the waves' partials in wave order
+            float a1 = 0.f, a2 = 0.f;
+#pragma unroll
+            for (int w = 0; w < ATT_WAVES; ++w) { a1 += qp_part[w * 64 + i]; a2 += qp_part[w * 64 + i + D / 2]; }
+            x1 = bf16_round_f32(a1 + (p.qp_bias ? bf16_to_f32(p.qp_bias[kvh * D + i]) : 0.0f));
+            x2 = bf16_round_f32(a2 + (p.qp_bias ? bf16_to_f32(p.qp_bias[kvh * D + i + D / 2]) : 0.0f));
+        }
         bf16_t r1, r2;
         if (p.rope_cos) {
             float c = rc[it], s = rs[it];
@@ -1472,18 +1646,64 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
             O[dt] = o;
         }
     };
-    for (int tile = wave; tile < n_tiles; tile += 2 * ATT_WAVES) {
-        const int tile2 = tile + ATT_WAVES;
-        const bool has2 = tile2 < n_tiles;
-        if (tile != wave) {                                             // later pairs (the first one was requested up front)
-            load_tile(tile, kA, vA);
-            if (has2) load_tile(tile2, kB, vB);
-        }
-        if (tile == new_tile) patch_new_key(kA, vA);
-        process(tile, kA, vA);
-        if (has2) {
-            if (tile2 == new_tile) patch_new_key(kB, vB);
-            process(tile2, kB, vB);
+    if constexpr (XS) {
+        // (cross-attention: no new key to patch.)  Straight-line code per tile count (ATT_XS_MIN_J .. ATT_XS_MAX_J; the launcher checks
+        // the cache length): group 0 sits in A (/ B), the pair behind it goes to C/D, the one behind that to A/B again.  A loop over
+        // pairs was tried first: across its back-edge hipcc rotates the buffers with v_mov copies of registers whose loads are
+        // still in flight (each behind its own wait) and waits for vmcnt(0) at the header - no two pairs in flight together.
+        // A pair is REQUESTED first and the group before it multiplied behind a binding statement that names its registers: the
+        // compiler's wait for them lands there, behind the requests (vmcnt(16): "everything but the youngest pair").
+        static_assert(!XS || D == 64, "XS: two pairs of tiles in registers (D = 64)");
+#define XS_BIND(KA, VA, KB, VB)                                                                                                   \
+        asm volatile("" : "+v"(KA[0][0]), "+v"(KA[0][1]), "+v"(KA[1][0]), "+v"(KA[1][1]), "+v"(VA[0]), "+v"(VA[1]), "+v"(VA[2]), "+v"(VA[3]), \
+                          "+v"(KB[0][0]), "+v"(KB[0][1]), "+v"(KB[1][0]), "+v"(KB[1][1]), "+v"(VB[0]), "+v"(VB[1]), "+v"(VB[2]), "+v"(VB[3]) :: "memory")
+        auto xs_run = [&](auto tag) {
+            constexpr int NJ = decltype(tag)::value, W = ATT_WAVES;
+            constexpr int G0 = (NJ & 1) ? 1 : 2, P = (NJ - G0) / 2;     // tiles in group 0, full pairs behind it (0 .. 2)
+            bf16x8_t kC[2][D / 32], kD[2][D / 32], vC[D / 16], vD[D / 16];
+            const int t1 = wu + G0 * W, t2 = t1 + 2 * W;
+            if constexpr (P >= 1) {
+                load_tile(t1, kC, vC);
+                load_tile(t1 + W, kD, vD);
+                XS_BIND(kA, vA, kB, vB);
+            }
+            process(wu, kA, vA);
+            if constexpr (G0 == 2) process(wu + W, kB, vB);
+            if constexpr (P >= 1) {
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (P >= 2) {
+                    load_tile(t2, kA, vA);
+                    load_tile(t2 + W, kB, vB);
+                }
+                XS_BIND(kC, vC, kD, vD);
+                process(t1, kC, vC);
+                process(t1 + W, kD, vD);
+            }
+            if constexpr (P >= 2) {
+                __builtin_amdgcn_sched_barrier(0);
+                XS_BIND(kA, vA, kB, vB);
+                process(t2, kA, vA);
+                process(t2 + W, kB, vB);
+            }
+        };
+        // (the launcher admits 40 .. 48 tiles: every wave has five or six - the only counts compiled, both run by every Whisper test)
+        if (xs_nj == 6) xs_run(std::integral_constant<int, 6>{});
+        else xs_run(std::integral_constant<int, 5>{});
+#undef XS_BIND
+    } else {
+        for (int tile = wave; tile < n_tiles; tile += 2 * ATT_WAVES) {
+            const int tile2 = tile + ATT_WAVES;
+            const bool has2 = tile2 < n_tiles;
+            if (tile != wave) {                                             // later pairs (the first one was requested up front)
+                load_tile(tile, kA, vA);
+                if (has2) load_tile(tile2, kB, vB);
+            }
+            if (tile == new_tile) patch_new_key(kA, vA);
+            process(tile, kA, vA);
+            if (has2) {
+                if (tile2 == new_tile) patch_new_key(kB, vB);
+                process(tile2, kB, vB);
+            }
         }
     }
     ATT_STAMP(5);
@@ -1521,299 +1741,279 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
     ATT_STAMP(7);
 }
 
-// Cross-attention over a LONG static cache (Whisper: 1500 keys = 47 tiles a head), head_dim 64, one query a (row, head).
-// What bounds it: with many (row, head) pairs the K/V stream (8 windows x 20 heads: 61 MB, 13.9 us alone); with few the chain of dependent steps
-// (glue, LayerNorm, query projection, scores, combine) and the 30 bytes a ns that one compute unit takes from HBM: 384 KB a pair.  The keys of
-// a pair are 16 groups (tile mod 16: three tiles each, two in the last) with a softmax of their own each: scores of all three tiles, ONE
-// maximum, no rescaling.  A wave owns GPW groups, a block has 16 / (NS GPW) waves, a pair NS blocks (launcher: NS 4 or 2 while every block has
-// a compute unit of its own).  Measured against blocks of eight waves with five or six tiles each and a running maximum: 6 pairs (one window, d = 384)
-// 14.0 -> 7.9 us with NS = 4 (NS = 2: 10.5, NS = 1: 12.8); 160 pairs (8 windows, d = 1280) 16.8 both, with NS = 2 26 (two rounds of blocks).
-// Results do not depend on NS: the query's partial sums are per 1/8 of W_q, and the groups' (m, l, O) are combined in one order - g with g + 8,
-// then the eight pairs - wherever they were computed.  With NS > 1 they meet in p.xa_part; the block that arrives last combines (nobody waits) and clears the counter.
-// K/V loads are non-temporal: a decode step reads each tile once (61 MB a layer at eight windows, 2 GB a step - nothing a cache can keep).
-//
-// KW > 0 ("query projection", at <= 16 rows): the residual add + LayerNorm glue in front of the cross-attention AND its query projection run in the
-// prologue instead of as two launches of their own (4.6 + 5.1 us a layer).  A block needs ONE row of the glue and 64 rows of W_q (49 - 164 KB
-// out of L2: the blocks of a head share them).  Wave w owns k-tiles [KT w / W, KT (w + 1) / W): it rebuilds THOSE columns of the row (four a lane),
-// the statistics meet in LDS per k-tile (two raw barriers: mean, then variance - the glue's two-pass form), and it multiplies them with the
-// head's four n-tiles on the matrix core (B = the row in every column).  Its first group's tiles are requested with W_q, a second group's when
-// W_q's registers are free.  Nothing is loaded under a condition: at the join every wait becomes one for all loads in flight.  The first block
-// of a row writes h_new to the OTHER residual buffer.
-#define XA_GROUPS 16
-#define XA_SLICES 8                              // partial sums of a query: slice i = k-tiles [KT i / 8, KT (i + 1) / 8)
+// The same for FEW (row, head) pairs: a pair on NS = 2 or 4 blocks.  With one block a pair, one window of the smallest model was a launch of six blocks: 384 KB
+// of keys and values each through one compute unit (30 bytes a ns from HBM at most) behind the chain glue - LayerNorm - query projection.
+// Bound now: that chain and the hand-over.  The work is cut where k_attn_decode cuts it - eight groups of tiles (tile mod 8), eight slices of K - and
+// summed in its order, so results are the bits of the one-block kernel whatever the split.  A block is two programs that meet at its barriers: 8 / NS
+// waves with ONE group each, whose keys and values (48 KB a wave) are all requested before the first wait, and four waves that rebuild the
+// row (glue, LayerNorm) and project it, two slices each.  The glue is requested before any keys, no load is conditional, and the scores of a
+// group's tiles are computed together - the running maximum is a chain of six fmaxf, not six rounds of products, exponentials and shuffles.
+// The groups' (m, l, O) meet in p.xa_part; the block that arrives last combines (nobody waits) and clears the counter.
+// Measured: one window, 6 heads (24 blocks) 14.0 -> 9.5 us; large-v3's 20 heads at one window: the call 68.0 -> 64.1 ms.
+#define XA_GROUPS 8
 #define XA_QP 4                                  // slabs of the glue at most
-template <int NS, int GPW, int KW>               // KW = k-tiles of W_q a wave holds (0: the query comes as slabs)
-__global__ void __launch_bounds__(XA_GROUPS / (NS * GPW) * 64) k_attn_cross(AttnParams p) {
-    constexpr int D = 64, W = XA_GROUPS / (NS * GPW), NSL = XA_SLICES / W;
-    __shared__ __attribute__((aligned(16))) bf16_t xs[KW > 0 ? W : 1][KW > 0 ? KW * 32 : 1];         // the row's columns of each wave after LayerNorm
-    __shared__ __attribute__((aligned(16))) float qpart[KW > 0 ? XA_SLICES : 1][D];
-    __shared__ float red[2][64];
+#define XA_PW 4                                  // waves of the query projection, two slices each
+#define XA_LD 66                                 // floats of a group's partial: O, m, l
+template <int NS, int KWS>                       // KWS = k-tiles of W_q in the longest slice (0: the query comes as slabs)
+__global__ void __launch_bounds__((XA_GROUPS / NS + (KWS > 0 ? XA_PW : 0)) * 64) k_attn_cross(AttnParams p) {
+    constexpr int D = 64, W = XA_GROUPS / NS, NJ = ATT_XS_MAX_J, NSL = XA_GROUPS / XA_PW;
+    __shared__ __attribute__((aligned(16))) bf16_t xs[KWS > 0 ? XA_GROUPS : 1][KWS > 0 ? KWS * 32 : 1];    // the row's slices after LayerNorm
+    __shared__ __attribute__((aligned(16))) float qpart[KWS > 0 ? XA_GROUPS : 1][D];
+    __shared__ float red[2][XA_GROUPS];
     __shared__ __attribute__((aligned(16))) bf16_t qs[W][D];
-    __shared__ float sm[XA_GROUPS / 2], sl[XA_GROUPS / 2], sO[XA_GROUPS / 2][D];
-    __shared__ unsigned s_last;
     const int kvh = blockIdx.x / NS, split = blockIdx.x % NS, b = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), group = split * W + min(wave, W - 1);
     const uint32_t active_word = reinterpret_cast<const uint32_t*>(p.active)[b >> 2];
     if (!((active_word >> (8 * (b & 3))) & 0xffu)) return;
-    const int kv_len = p.cross_len, n_tiles = (kv_len + 31) >> 5;                           // 33 .. 48 tiles (launcher): two or three a group
+    const int kv_len = p.cross_len, n_tiles = (kv_len + 31) >> 5;                           // 40 .. 48 tiles (launcher): five or six a group
     const bf16x8_t* kbase = reinterpret_cast<const bf16x8_t*>(p.kcache + ((size_t)(b * p.H + kvh) * p.Smax) * D) + lane;
     const bf16x8_t* vbase = reinterpret_cast<const bf16x8_t*>(p.vtcache + ((size_t)(b * p.H + kvh) * D) * p.Smax) + lane;
-    bf16x8_t ka[GPW][3][2][D / 32], va[GPW][3][D / 16];
-    auto group_of = [&](int i) { return split * (W * GPW) + i * W + wave; };
-    auto load_tile = [&](int i, int t) {
-        const int tile = min(group_of(i) + t * XA_GROUPS, n_tiles - 1);       // (a group of two tiles loads a masked third one: no branch around loads)
+    bf16x8_t ka[NJ][2][D / 32], va[NJ][D / 16];
+    auto load_tiles = [&]() {
 #pragma unroll
-        for (int c = 0; c < D / 32; ++c) {
-            ka[i][t][0][c] = __builtin_nontemporal_load(kbase + ((size_t)tile * 2) * (D / 32) * 64 + c * 64);
-            ka[i][t][1][c] = __builtin_nontemporal_load(kbase + ((size_t)tile * 2 + 1) * (D / 32) * 64 + c * 64);
+        for (int j = 0; j < NJ; ++j) {
+            const int tile = min(group + j * XA_GROUPS, n_tiles - 1);         // (a group of five tiles requests a sixth one that it does not use)
+#pragma unroll
+            for (int c = 0; c < D / 32; ++c) {
+                ka[j][0][c] = __builtin_nontemporal_load(kbase + ((size_t)tile * 2) * (D / 32) * 64 + c * 64);
+                ka[j][1][c] = __builtin_nontemporal_load(kbase + ((size_t)tile * 2 + 1) * (D / 32) * 64 + c * 64);
+            }
         }
 #pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) va[i][t][dt] = __builtin_nontemporal_load(vbase + ((size_t)tile * (D / 16) + dt) * 64);
+        for (int j = 0; j < NJ; ++j) {
+            const int tile = min(group + j * XA_GROUPS, n_tiles - 1);
+#pragma unroll
+            for (int dt = 0; dt < D / 16; ++dt) va[j][dt] = __builtin_nontemporal_load(vbase + ((size_t)tile * (D / 16) + dt) * 64);
+        }
     };
+    if constexpr (KWS > 0) {
+        if (wave >= W) {                                      // ---- the projection's program; its four barriers stand in the other one, too
+            const int pw = wave - W;
+            const int KT = p.qp_KT, N = KT * 32;
+            int k0[NSL], k1[NSL], col[NSL];
+            f32x4_t v[NSL][XA_QP];
+            uint2 hq[NSL], wq[NSL], bq[NSL];
+#pragma unroll
+            for (int i = 0; i < NSL; ++i) {                        // slice pw NSL + i: k-tiles [k0, k1), four columns a lane
+                const int sl = pw * NSL + i;
+                k0[i] = (KT * sl) / XA_GROUPS; k1[i] = (KT * (sl + 1)) / XA_GROUPS;
+                col[i] = 32 * k0[i] + 4 * lane;
+                const int colc = col[i] < 32 * k1[i] ? col[i] : N - 4;
+#pragma unroll
+                for (int j = 0; j < XA_QP; ++j)
+                    v[i][j] = *reinterpret_cast<const f32x4_t*>(p.qp_slabs + ((size_t)min(j, p.qp_S - 1) * p.Mpad + b) * N + colc);
+                hq[i] = *reinterpret_cast<const uint2*>(p.qp_h_in + (size_t)b * N + colc);
+                wq[i] = *reinterpret_cast<const uint2*>(p.qp_lnw + colc);
+                bq[i] = *reinterpret_cast<const uint2*>(p.qp_lnb + colc);
+            }
+            asm volatile("s_barrier" ::: "memory");              // (1) the glue is requested in front of any wave's W_q and keys
+            bf16x8_t wt[NSL][KWS][4];
+#pragma unroll
+            for (int i = 0; i < NSL; ++i)
+#pragma unroll
+                for (int u = 0; u < KWS; ++u) {
+                    const int kk = min(k0[i] + u, k1[i] > k0[i] ? k1[i] - 1 : KT - 1);         // (a shorter slice reads its last k-tile again: no branch around loads)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)      // (cached loads: the head's other blocks read the same tiles)
+                        wt[i][u][r] = *(reinterpret_cast<const bf16x8_t*>(p.qp_w) + ((size_t)(kvh * 4 + r) * KT + kk) * 64 + lane);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            float hn[NSL][4];
+#pragma unroll
+            for (int i = 0; i < NSL; ++i) {
+                float acc4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < XA_QP; ++j) {                 // slab order 0, 1, 2, ... (fixed => deterministic)
+                    const bool on = j < p.qp_S;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc4[e] += on ? v[i][j][e] : 0.0f;
+                }
+                const float hv[4] = {bf16_to_f32((bf16_t)(hq[i].x & 0xffffu)), bf16_to_f32((bf16_t)(hq[i].x >> 16)), bf16_to_f32((bf16_t)(hq[i].y & 0xffffu)),
+                                     bf16_to_f32((bf16_t)(hq[i].y >> 16))};
+                float sum = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hn[i][e] = bf16_round_f32(hv[e] + bf16_round_f32(acc4[e]));                // o = T(sum slabs); h = T(h + o)
+                    sum += col[i] < 32 * k1[i] ? hn[i][e] : 0.0f;
+                }
+                sum = wave_sum_dpp(sum);
+                if (lane == 0) red[0][pw * NSL + i] = sum;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");          // (raw: __syncthreads() would wait for the keys as well)
+            float tot = 0.f;
+#pragma unroll
+            for (int w = 0; w < XA_GROUPS; ++w) tot += red[0][w];
+            const float mean = tot / (float)N;
+#pragma unroll
+            for (int i = 0; i < NSL; ++i) {
+                float sq = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { const float dl = hn[i][e] - mean; sq += col[i] < 32 * k1[i] ? dl * dl : 0.0f; }
+                sq = wave_sum_dpp(sq);
+                if (lane == 0) red[1][pw * NSL + i] = sq;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            float tq = 0.f;
+#pragma unroll
+            for (int w = 0; w < XA_GROUPS; ++w) tq += red[1][w];
+            const float rstd = 1.0f / sqrtf(tq / (float)N + p.qp_eps);
+#pragma unroll
+            for (int i = 0; i < NSL; ++i) {
+                if (col[i] < 32 * k1[i]) {
+                    const float wv[4] = {bf16_to_f32((bf16_t)(wq[i].x & 0xffffu)), bf16_to_f32((bf16_t)(wq[i].x >> 16)), bf16_to_f32((bf16_t)(wq[i].y & 0xffffu)),
+                                         bf16_to_f32((bf16_t)(wq[i].y >> 16))};
+                    const float bv[4] = {bf16_to_f32((bf16_t)(bq[i].x & 0xffffu)), bf16_to_f32((bf16_t)(bq[i].x >> 16)), bf16_to_f32((bf16_t)(bq[i].y & 0xffffu)),
+                                         bf16_to_f32((bf16_t)(bq[i].y >> 16))};
+                    bf16_t xb[4], hb[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        xb[e] = f32_to_bf16((hn[i][e] - mean) * rstd * wv[e] + bv[e]);
+                        hb[e] = f32_to_bf16(hn[i][e]);
+                    }
+                    *reinterpret_cast<uint2*>(&xs[pw * NSL + i][4 * lane]) = make_uint2((uint32_t)xb[0] | ((uint32_t)xb[1] << 16), (uint32_t)xb[2] | ((uint32_t)xb[3] << 16));
+                    if (blockIdx.x == 0)                          // the first block of the row keeps the residual stream (the projection waves cover the row)
+                        *reinterpret_cast<uint2*>(p.qp_h_out + (size_t)b * N + col[i]) =
+                            make_uint2((uint32_t)hb[0] | ((uint32_t)hb[1] << 16), (uint32_t)hb[2] | ((uint32_t)hb[3] << 16));
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the slices are this wave's own: LDS operations of one wave execute in order)
+#pragma unroll
+            for (int i = 0; i < NSL; ++i) {
+                f32x4_t a[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[r] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < KWS; ++u) {
+                    bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(&xs[pw * NSL + i][u * 32 + (lane >> 4) * 8]);
+                    if (k0[i] + u >= k1[i]) xf = (bf16x8_t){0, 0, 0, 0, 0, 0, 0, 0};            // a dead k-tile multiplies zero
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) a[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[i][u][r], xf, a[r], 0, 0, 0);
+                }
+                // C/D lane l, reg e: n = (l >> 4) * 4 + e, the row in every column: the lanes of column r store n-tile r
+                const int m = lane & 15;
+                f32x4_t o = a[0];
+#pragma unroll
+                for (int r = 1; r < 4; ++r)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = m == r ? a[r][e] : o[e];
+                asm volatile("" : "+v"(o));
+                if (m < 4) *reinterpret_cast<f32x4_t*>(&qpart[pw * NSL + i][m * 16 + (lane >> 4) * 4]) = o;
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (4)
+            __syncthreads();                                  // (5)
+            return;
+        }
+    }
     float q;                                                                    // element `lane` of the query
-    if constexpr (KW > 0) {
-        const int KT = p.qp_KT, N = KT * 32;
-        const int k0 = (KT * wave) / W, k1 = (KT * (wave + 1)) / W;
-        const int col = 32 * k0 + 4 * lane;
-        const bool live = col < 32 * k1;
-        const int colc = live ? col : N - 4;
-        f32x4_t v[XA_QP];
-#pragma unroll
-        for (int j = 0; j < XA_QP; ++j) {
-            const int sj = j < p.qp_S ? j : p.qp_S - 1;
-            v[j] = *reinterpret_cast<const f32x4_t*>(p.qp_slabs + ((size_t)sj * p.Mpad + b) * N + colc);
-        }
-        const uint2 hq = *reinterpret_cast<const uint2*>(p.qp_h_in + (size_t)b * N + colc);
-        const uint2 wq = *reinterpret_cast<const uint2*>(p.qp_lnw + colc);
-        const uint2 bq = *reinterpret_cast<const uint2*>(p.qp_lnb + colc);
+    if constexpr (KWS > 0) {
         const bf16_t bias = (p.qp_bias ? p.qp_bias + kvh * D : p.qp_lnw)[lane];             // (no branch around the load)
-        if constexpr (NS > 1) asm volatile("s_barrier" ::: "memory");      // every wave's glue is requested in front of any wave's W_q and keys
-        bf16x8_t wt[KW][4];
-#pragma unroll
-        for (int u = 0; u < KW; ++u) {
-            const int kk = min(k0 + u, k1 > k0 ? k1 - 1 : KT - 1);     // (a wave with fewer k-tiles reads its last one again: no branch around loads)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {        // (cached loads: the other rows' blocks of this head read the same tiles)
-                const bf16_t* w = p.qp_w + (((size_t)(kvh * 4 + r) * KT + kk) * 64 + lane) * 8;
-                wt[u][r] = *reinterpret_cast<const bf16x8_t*>(w);
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < 3; ++t) load_tile(0, t);
+        asm volatile("s_barrier" ::: "memory");              // (1)
+        load_tiles();
         __builtin_amdgcn_sched_barrier(0);
-        auto sum8 = [](float x) {                            // over the eight lanes of a k-tile (every lane gets the sum)
-            x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xF, 0xF, true));     // quad_perm [1, 0, 3, 2]
-            x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xF, 0xF, true));     // quad_perm [2, 3, 0, 1]
-            x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xF, 0xF, true));    // row_half_mirror
-            return x;
-        };
-        float acc4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < XA_QP; ++j) {                    // slab order 0, 1, 2, ... (fixed => deterministic)
-            const bool on = j < p.qp_S;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc4[e] += on ? v[j][e] : 0.0f;
-        }
-        const float hv[4] = {bf16_to_f32((bf16_t)(hq.x & 0xffffu)), bf16_to_f32((bf16_t)(hq.x >> 16)), bf16_to_f32((bf16_t)(hq.y & 0xffffu)),
-                             bf16_to_f32((bf16_t)(hq.y >> 16))};
-        float hn[4], sum = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            hn[e] = bf16_round_f32(hv[e] + bf16_round_f32(acc4[e]));                // o = T(sum slabs); h = T(h + o)
-            sum += hn[e];
-        }
-        sum = sum8(sum);
-        if (live && (lane & 7) == 0) red[0][k0 + (lane >> 3)] = sum;
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");          // (raw: __syncthreads() would wait for the keys as well)
-        const float mean = wave_sum_dpp(lane < KT ? red[0][lane] : 0.0f) / (float)N;
-        float sq = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) { const float dl = hn[e] - mean; sq += dl * dl; }
-        sq = sum8(sq);
-        if (live && (lane & 7) == 0) red[1][k0 + (lane >> 3)] = sq;
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        const float rstd = 1.0f / sqrtf(wave_sum_dpp(lane < KT ? red[1][lane] : 0.0f) / (float)N + p.qp_eps);
-        if (live) {
-            const float wv[4] = {bf16_to_f32((bf16_t)(wq.x & 0xffffu)), bf16_to_f32((bf16_t)(wq.x >> 16)), bf16_to_f32((bf16_t)(wq.y & 0xffffu)),
-                                 bf16_to_f32((bf16_t)(wq.y >> 16))};
-            const float bv[4] = {bf16_to_f32((bf16_t)(bq.x & 0xffffu)), bf16_to_f32((bf16_t)(bq.x >> 16)), bf16_to_f32((bf16_t)(bq.y & 0xffffu)),
-                                 bf16_to_f32((bf16_t)(bq.y >> 16))};
-            bf16_t xb[4], hb[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                xb[e] = f32_to_bf16((hn[e] - mean) * rstd * wv[e] + bv[e]);
-                hb[e] = f32_to_bf16(hn[e]);
-            }
-            *reinterpret_cast<uint2*>(&xs[wave][4 * lane]) = make_uint2((uint32_t)xb[0] | ((uint32_t)xb[1] << 16), (uint32_t)xb[2] | ((uint32_t)xb[3] << 16));
-            if (blockIdx.x == 0)                              // the first block of the row keeps the residual stream (its waves cover the row)
-                *reinterpret_cast<uint2*>(p.qp_h_out + (size_t)b * N + col) =
-                    make_uint2((uint32_t)hb[0] | ((uint32_t)hb[1] << 16), (uint32_t)hb[2] | ((uint32_t)hb[3] << 16));
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (the columns are this wave's own: LDS operations of one wave execute in order)
-#pragma unroll
-        for (int i = 0; i < NSL; ++i) {                      // this wave's slices; a k-tile of another slice multiplies zero
-            const int s0 = KT * (wave * NSL + i) / XA_SLICES - k0, s1 = KT * (wave * NSL + i + 1) / XA_SLICES - k0;
-            f32x4_t a[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) a[r] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int u = 0; u < KW; ++u) {
-                bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(&xs[wave][u * 32 + (lane >> 4) * 8]);
-                if (u < s0 || u >= s1) xf = (bf16x8_t){0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-                for (int r = 0; r < 4; ++r) a[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[u][r], xf, a[r], 0, 0, 0);
-            }
-            // C/D lane l, reg e: n = (l >> 4) * 4 + e, in every column: the lanes of column r store n-tile r
-            const int m = lane & 15;
-            f32x4_t o = a[0];
-#pragma unroll
-            for (int r = 1; r < 4; ++r)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = m == r ? a[r][e] : o[e];
-            asm volatile("" : "+v"(o));
-            if (m < 4) *reinterpret_cast<f32x4_t*>(&qpart[wave * NSL + i][m * 16 + (lane >> 4) * 4]) = o;
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 1; i < GPW; ++i)
-#pragma unroll
-            for (int t = 0; t < 3; ++t) load_tile(i, t);
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        asm volatile("s_barrier\n\ts_barrier\n\ts_barrier" ::: "memory");      // (2) (3) the statistics, (4) the query's partial sums are in LDS
         q = 0.f;
 #pragma unroll
-        for (int i = 0; i < XA_SLICES; ++i) q += qpart[i][lane];
+        for (int w = 0; w < XA_GROUPS; ++w) q += qpart[w][lane];
         q += p.qp_bias ? bf16_to_f32(bias) : 0.0f;
     } else {
         float pv[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) pv[j] = p.qkv_part[((size_t)(j < p.S ? j : p.S - 1) * p.Mpad + b) * p.Nqkv + kvh * D + lane];
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int i = 0; i < GPW; ++i)
-#pragma unroll
-            for (int t = 0; t < 3; ++t) load_tile(i, t);
+        load_tiles();
         __builtin_amdgcn_sched_barrier(0);
         q = 0.f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) q += j < p.S ? pv[j] : 0.0f;           // slab order 0..7 (S <= 8, checked by the launcher)
     }
-    qs[wave][lane] = f32_to_bf16(q);                         // q = T(W_q x + b); every wave has its own copy (no barrier)
+    qs[wave][lane] = f32_to_bf16(q);                          // q = T(W_q x + b); every wave has its own copy (no barrier)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     const int g4 = lane >> 4, d0 = lane & 15;
-    bf16x8_t qf[D / 32];                                      // the query in all sixteen columns
+    bf16x8_t qf[D / 32];                                      // the query in all sixteen columns: every lane holds scores, maximum and sum of its keys
 #pragma unroll
     for (int c = 0; c < D / 32; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(&qs[wave][c * 32 + g4 * 8]);
-    f32x4_t O[GPW][D / 16];
-    float mg[GPW], lg[GPW];
+    float sc[NJ][8], mj[NJ];
 #pragma unroll
-    for (int i = 0; i < GPW; ++i) {
-        if (i > 0) __builtin_amdgcn_sched_barrier(0);        // (the first group does not wait for the second one's keys)
-        const int g = group_of(i);
-        float sc[3][8], mx = -INFINITY;
+    for (int j = 0; j < NJ; ++j) {
+        f32x4_t S0 = (f32x4_t){0.f, 0.f, 0.f, 0.f}, S1 = S0;
 #pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            f32x4_t S0 = (f32x4_t){0.f, 0.f, 0.f, 0.f}, S1 = S0;
-#pragma unroll
-            for (int c = 0; c < D / 32; ++c) {
-                S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[i][t][0][c], qf[c], S0, 0, 0, 0);
-                S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[i][t][1][c], qf[c], S1, 0, 0, 0);
-            }
-            const int base = (g + t * XA_GROUPS) * 32 + g4 * 8;                   // this lane's keys: base + e (the cache tiling)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float x = (e < 4 ? S0[e] : S1[e - 4]) * p.scale;
-                sc[t][e] = base + e < kv_len ? x : -INFINITY;
-                mx = fmaxf(mx, sc[t][e]);
-            }
+        for (int c = 0; c < D / 32; ++c) {
+            S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][0][c], qf[c], S0, 0, 0, 0);
+            S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][1][c], qf[c], S1, 0, 0, 0);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));              // (finite: the group's first two tiles are whole)
-        float ps = 0.0f;
+        const int base = (group + j * XA_GROUPS) * 32 + g4 * 8;                   // this lane's keys: base + e (the cache tiling)
+        float mx = -INFINITY;
 #pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) O[i][dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            bf16x8_t ph, pl;                                 // P in bf16 hi + lo parts (f32-accurate probabilities)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float pe = __expf(sc[t][e] - mx);
-                ps += pe;
-                const bf16_t hi = f32_to_bf16(pe);
-                ph[e] = (short)hi;
-                pl[e] = (short)f32_to_bf16(pe - bf16_to_f32(hi));
-            }
-#pragma unroll
-            for (int dt = 0; dt < D / 16; ++dt) {
-                O[i][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, va[i][t][dt], O[i][dt], 0, 0, 0);
-                O[i][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, va[i][t][dt], O[i][dt], 0, 0, 0);
-            }
+        for (int e = 0; e < 8; ++e) {
+            const float x = (e < 4 ? S0[e] : S1[e - 4]) * p.scale;
+            sc[j][e] = base + e < kv_len ? x : -INFINITY;
+            mx = fmaxf(mx, sc[j][e]);
         }
-        ps += __shfl_xor(ps, 16, 64);
-        ps += __shfl_xor(ps, 32, 64);
-        mg[i] = mx; lg[i] = ps;
+        mj[j] = mx;
     }
-    auto merge = [](float m0, float m1, float& f0, float& f1) {
-        const float m = fmaxf(m0, m1);
-        f0 = __expf(m0 - m); f1 = __expf(m1 - m);
-        return m;
-    };
-    // ---- the groups' partials: lanes 0 .. 15 hold O (its rows are equal), lane 0 m and l
-    constexpr int NP = XA_GROUPS / 2;
-    float o[NP], mm[NP], ll[NP];
-    if constexpr (NS > 1) {
-        constexpr int LD = D + 2;
-        float* part = p.xa_part + ((size_t)b * p.H + kvh) * XA_GROUPS * LD;
-        if (g4 == 0) {
 #pragma unroll
-            for (int i = 0; i < GPW; ++i) {
-                float* pg = part + group_of(i) * LD;
-#pragma unroll
-                for (int dt = 0; dt < D / 16; ++dt) __hip_atomic_store(pg + dt * 16 + d0, O[i][dt][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (d0 < 2) __hip_atomic_store(pg + D + d0, d0 ? lg[i] : mg[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's partials are where every XCD sees them ...
-        __syncthreads();                                     // ... and every wave's of the block, before the block arrives
-        unsigned* cnt = p.xa_count + (size_t)b * p.H + kvh;
-        if (tid == 0) s_last = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        if (s_last != NS - 1) return;
-        if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);      // (the next launch starts at zero)
-        if (wave != 0) return;
-        float og[XA_GROUPS], mgr[XA_GROUPS], lgr[XA_GROUPS];
-#pragma unroll
-        for (int w = 0; w < XA_GROUPS; ++w) {
-            og[w] = __hip_atomic_load(part + w * LD + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            mgr[w] = __hip_atomic_load(part + w * LD + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            lgr[w] = __hip_atomic_load(part + w * LD + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-#pragma unroll
-        for (int w = 0; w < NP; ++w) {
-            float f0, f1;
-            mm[w] = merge(mgr[w], mgr[w + NP], f0, f1);
-            o[w] = __builtin_fmaf(f0, og[w], f1 * og[w + NP]);
-            ll[w] = __builtin_fmaf(f0, lgr[w], f1 * lgr[w + NP]);
-        }
-    } else {
-        static_assert(NS > 1 || (GPW == 2 && W == NP), "a wave holds groups g and g + 8");
-        float f0, f1;
-        const float m2 = merge(mg[0], mg[GPW - 1], f0, f1);
-        if (g4 == 0) {
-#pragma unroll
-            for (int dt = 0; dt < D / 16; ++dt) sO[wave][dt * 16 + d0] = __builtin_fmaf(f0, O[0][dt][0], f1 * O[GPW - 1][dt][0]);
-            if (d0 == 0) { sm[wave] = m2; sl[wave] = __builtin_fmaf(f0, lg[0], f1 * lg[GPW - 1]); }
-        }
-        __syncthreads();
-        if (wave != 0) return;
-#pragma unroll
-        for (int w = 0; w < NP; ++w) { o[w] = sO[w][lane]; mm[w] = sm[w]; ll[w] = sl[w]; }
+    for (int j = 0; j < NJ; ++j) {
+        mj[j] = fmaxf(mj[j], __shfl_xor(mj[j], 16, 64));
+        mj[j] = fmaxf(mj[j], __shfl_xor(mj[j], 32, 64));
     }
-    float M = -INFINITY;
+    f32x4_t O[D / 16];
 #pragma unroll
-    for (int w = 0; w < NP; ++w) M = fmaxf(M, mm[w]);
-    float num = 0.0f, den = 0.0f;
+    for (int dt = 0; dt < D / 16; ++dt) O[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.0f;
 #pragma unroll
-    for (int w = 0; w < NP; ++w) {
+    for (int j = 0; j < NJ; ++j) {
+        if (j == NJ - 1 && group + j * XA_GROUPS >= n_tiles) break;               // (a group of five)
+        const float m_new = fmaxf(m_run, mj[j]), alpha = __expf(m_run - m_new);   // m_run = -inf -> 0
+        float psum = 0.0f;
+        bf16x8_t ph, pl;                                      // P in bf16 hi + lo parts (f32-accurate probabilities)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float pe = __expf(sc[j][e] - m_new);
+            psum += pe;
+            const bf16_t hi = f32_to_bf16(pe);
+            ph[e] = (short)hi;
+            pl[e] = (short)f32_to_bf16(pe - bf16_to_f32(hi));
+        }
+        l_run = l_run * alpha + psum;
+        m_run = m_new;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) {
+            f32x4_t o = O[dt];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] *= alpha;
+            o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, va[j][dt], o, 0, 0, 0);
+            O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, va[j][dt], o, 0, 0, 0);
+        }
+    }
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    // ---- the group's partial: lanes 0 .. 15 hold O (its rows are equal), lanes 0 and 1 store m and l
+    float* part = p.xa_part + ((size_t)b * p.H + kvh) * XA_GROUPS * XA_LD;
+    if (g4 == 0) {
+        float* pg = part + group * XA_LD;
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) __hip_atomic_store(pg + dt * 16 + d0, O[dt][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (d0 < 2) __hip_atomic_store(pg + D + d0, d0 ? l_run : m_run, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");          // this wave's partial is where every XCD sees it ...
+    __syncthreads();                                          // (5) ... and every wave's of the block, before the block arrives
+    unsigned* cnt = p.xa_count + (size_t)b * p.H + kvh;
+    if (wave != 0) return;
+    unsigned old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(old) != NS - 1) return;
+    if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);         // (the next launch starts at zero)
+    float o[XA_GROUPS], mm[XA_GROUPS], ll[XA_GROUPS], M = -INFINITY, num = 0.0f, den = 0.0f;
+#pragma unroll
+    for (int w = 0; w < XA_GROUPS; ++w) {
+        o[w] = __hip_atomic_load(part + w * XA_LD + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        mm[w] = __hip_atomic_load(part + w * XA_LD + D, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        ll[w] = __hip_atomic_load(part + w * XA_LD + D + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int w = 0; w < XA_GROUPS; ++w) M = fmaxf(M, mm[w]);
+#pragma unroll
+    for (int w = 0; w < XA_GROUPS; ++w) {
         const float f = __expf(mm[w] - M);
         num += f * o[w];
         den += f * ll[w];
@@ -2187,25 +2387,32 @@ size_t attn_smem_bytes(int G, int D) {
     return (size_t)attn_nit(G, D) * 512 * 4 + 16 * D * 2 + D * 2 + 2 * ATT_WAVES * 16 * 4 + (size_t)ATT_WAVES * G * D * 4;
 }
 
-// cross-attention launches that k_attn_cross takes: head_dim 64, a head of its own for every query, 33 .. 48 key tiles (two or three a group)
-static bool attn_cross_ok(const AttnParams& p) {
-    const int tiles = (p.cross_len + 31) / 32;
-    return p.cross && p.D == 64 && p.H == p.Hkv && !p.append_only && !p.cache_rows && !p.rope_cos && !p.qnorm_w && !p.out_ld && tiles > 2 * XA_GROUPS && tiles <= 3 * XA_GROUPS;
-}
-// ... and those whose prologue can take the LayerNorm glue and the query projection (a block of eight waves at least holds W_q).  MIS_ATTN_XS=0
-// (parity tests): the separate launches and one block a (row, head)
-static bool attn_xs_on() { const char* xe = getenv("MIS_ATTN_XS"); return !(xe && atoi(xe) == 0); }
+// the cross-attention launches whose prologue can take the LayerNorm glue and the query projection (k_attn_decode<64, 2, true, QP>)
 bool attn_qp_ok(const AttnParams& p) {
-    return attn_xs_on() && attn_cross_ok(p) && p.qp_KT >= 1 && p.qp_KT <= 40 && p.qp_KT * 32 == p.H * p.D && p.qp_S >= 1 && p.qp_S <= XA_QP;
+    const char* xe = getenv("MIS_ATTN_XS");
+    return !(xe && atoi(xe) == 0) && p.cross && p.D == 64 && p.H == p.Hkv && !p.append_only && !p.cache_rows && !p.rope_cos && !p.qnorm_w &&
+           (p.cross_len + 31) / 32 >= ATT_WAVES * ATT_XS_MIN_J && (p.cross_len + 31) / 32 <= ATT_WAVES * ATT_XS_MAX_J && p.qp_KT >= 1 &&
+           (p.qp_KT + ATT_WAVES - 1) / ATT_WAVES <= ATT_QP_KW && p.qp_KT * 32 == p.H * p.D && p.qp_S >= 1 && p.qp_S <= 8;
 }
-size_t attn_cross_part_floats(int rows, int H) { return (size_t)rows * H * XA_GROUPS * (64 + 2); }
-template <int NS, int GPW>
-static void launch_attn_cross(const AttnParams& p, int batch, hipStream_t s) {
-    const dim3 grid(p.H * NS, batch), block(XA_GROUPS / (NS * GPW) * 64);
-    const int kw = (p.qp_KT + XA_GROUPS / (NS * GPW) - 1) / (XA_GROUPS / (NS * GPW));
-    if (!p.qp_w) hipLaunchKernelGGL((k_attn_cross<NS, GPW, 0>), grid, block, 0, s, p);
-    else if (kw <= 3) hipLaunchKernelGGL((k_attn_cross<NS, GPW, 3>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((k_attn_cross<NS, GPW, 5>), grid, block, 0, s, p);
+size_t attn_cross_part_floats(int rows, int H) { return (size_t)rows * H * XA_GROUPS * XA_LD; }
+// k_attn_cross where every block of the launch has a compute unit of its own (a second round of blocks costs more than the split gains: 160 pairs 17 us with
+// one block each, 26 with two); false: one block a pair
+static bool launch_attn_cross(const AttnParams& p, int batch, hipStream_t s) {
+    const int pairs = p.H * batch, cus = 256;
+    if (!p.xa_part || p.H != p.Hkv || p.rope_cos || p.qnorm_w || p.out_ld || 2 * pairs > cus || (p.qp_w && p.qp_S > XA_QP)) return false;
+#define XA_GO(NS, KWS) { hipLaunchKernelGGL((k_attn_cross<NS, KWS>), dim3(p.H * NS, batch), dim3((XA_GROUPS / NS + (KWS > 0 ? XA_PW : 0)) * 64), 0, s, p); return true; }
+    const int kws = !p.qp_w ? 0 : p.qp_KT <= 16 ? 2 : p.qp_KT <= 24 ? 3 : 5;                // (attn_qp_ok: at most 40 k-tiles)
+    if (4 * pairs <= cus) {
+        if (kws == 0) XA_GO(4, 0)
+        if (kws == 2) XA_GO(4, 2)
+        if (kws == 3) XA_GO(4, 3)
+        XA_GO(4, 5)
+    }
+    if (kws == 0) XA_GO(2, 0)
+    if (kws == 2) XA_GO(2, 2)
+    if (kws == 3) XA_GO(2, 3)
+    XA_GO(2, 5)
+#undef XA_GO
 }
 void launch_attn_decode(const AttnParams& p, int batch, hipStream_t s) {
     int G = p.H / p.Hkv;
@@ -2240,18 +2447,24 @@ void launch_attn_decode(const AttnParams& p, int batch, hipStream_t s) {
 #else
     const AttnParams& p2 = p;
 #endif
+    const char* xe = getenv("MIS_ATTN_XS");                                                // 0: the pair-at-a-time loop for cross-attention too (A/B,
+    const bool xs_on = !(xe && atoi(xe) == 0);                                             // parity tests: read per launch)
     if (p.D == 128 && n_el <= 1024) hipLaunchKernelGGL((k_attn_decode<128, 2>), grid, block, smem, s, p2);
     else if (p.D == 128) hipLaunchKernelGGL((k_attn_decode<128, 5>), grid, block, smem, s, p2);
-    else if (attn_cross_ok(p)) {
+    else if (p.D == 64 && n_el <= 1024 && p.cross && !p.append_only && !p.cache_rows && xs_on && (p.cross_len + 31) / 32 >= ATT_WAVES * ATT_XS_MIN_J &&
+             (p.cross_len + 31) / 32 <= ATT_WAVES * ATT_XS_MAX_J)
+    {
         MIS_REQUIRE(!p.qp_w || attn_qp_ok(p), MIS_ERR_GENERATION_FAILED, "attention: the query-projection prologue does not apply to this launch");
-        // NS: the most blocks of one (row, head) that leave every block a compute unit of its own (a second round costs more than the split gains:
-        // 160 pairs 16.8 us with NS = 1, 26 with NS = 2) and its waves room for W_q
-        const int pairs = p.H * batch, cus = 256;
-        const bool four = !p.qp_w || p.qp_KT <= 20;
-        const int ns = !p.xa_part || !attn_xs_on() ? 1 : four && 4 * pairs <= cus ? 4 : 2 * pairs <= cus ? 2 : 1;
-        if (ns == 4 && four) launch_attn_cross<4, 1>(p2, batch, s);
-        else if (ns == 2) launch_attn_cross<2, 1>(p2, batch, s);
-        else launch_attn_cross<1, 2>(p2, batch, s);
+        if (launch_attn_cross(p2, batch, s)) return;
+        if (p.qp_w) {                                                                       // LayerNorm + query projection in the prologue
+            AttnParams pq = p2;                            // (the kernel's unconditional dummy loads - norm weights, RoPE rows - read qkv_part[0])
+            if (!pq.qkv_part) pq.qkv_part = pq.qp_slabs;
+            const AttnParams& p2 = pq;
+            const size_t smq = smem + ATT_QP_LDS;
+            if (p.qp_S <= 4) hipLaunchKernelGGL((k_attn_decode<64, 2, true, 4>), grid, block, smq, s, p2);
+            else hipLaunchKernelGGL((k_attn_decode<64, 2, true, 8>), grid, block, smq, s, p2);
+        } else
+        hipLaunchKernelGGL((k_attn_decode<64, 2, true>), grid, block, smem, s, p2);       // cross-attention: two pairs of tiles in flight
     }
     else if (p.D == 64 && n_el <= 1024) hipLaunchKernelGGL((k_attn_decode<64, 2>), grid, block, smem, s, p2);
     else if (p.D == 64) hipLaunchKernelGGL((k_attn_decode<64, 3>), grid, block, smem, s, p2);

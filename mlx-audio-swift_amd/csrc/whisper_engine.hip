@@ -519,7 +519,7 @@ extern "C" mis_status mis_whisper_encode(mis_whisper* c, const float* features, 
 // Up to 16 rows (the BASELINE share: 8 windows per GPU) two of the three residual + LayerNorm glue launches of a layer - and one GEMM launch -
 // run inside the prologue of their consumer: 8 launches per layer instead of 11 (transcribe 228 -> 214 ms per 8 x 30 s, profiles/r06/c4, c5).
 //   bit 4 (16): h += self-attention output, LayerNorm 2 AND the cross-attention's query projection inside the cross-attention kernel
-//               (k_attn_cross, lm_kernels.hip: a block is one (row, head) and rebuilds only its row);
+//               (k_attn_decode<64, 2, true, QP> or k_attn_cross, lm_kernels.hip: a block is one (row, head) and rebuilds only its row);
 //   bit 2 (4):  h += cross-attention output and LayerNorm 3 inside fc1's prologue (k_gemm_skinny_norm: every block rebuilds all rows);
 //   bit 3 (8):  fail where a requested fold does not apply (tests).  MIS_WHISPER_FOLD=0 keeps the separate launches.
 // The residual stream alternates between two buffers: every block of a consumer still reads the old one while one of them writes the new.
@@ -536,7 +536,7 @@ static void enqueue_decoder_step(mis_whisper* c) {
     const char* fe = getenv("MIS_WHISPER_FOLD");
     const int want = fe ? atoi(fe) : WHISPER_FOLD_DEFAULT;
     AttnParams probe{};
-    probe.cross = 1; probe.cross_len = 1500; probe.D = D; probe.H = H; probe.Hkv = H; probe.qp_KT = d / 32; probe.qp_S = c->S_o; probe.xa_part = c->xa_part.p;
+    probe.cross = 1; probe.cross_len = 1500; probe.D = D; probe.H = H; probe.Hkv = H; probe.qp_KT = d / 32; probe.qp_S = c->S_o;
     const bool f_cqa = (want & 16) && Mpad == 16 && attn_qp_ok(probe);
     const bool f_fc1 = (want & 4) && gemm_skinny_norm_ok(EPI_GELU_PACKED, 2, d / 32, 1, c->S_o, Mpad, c->batch);
     MIS_REQUIRE(!(want & 8) || (f_cqa == !!(want & 16) && f_fc1 == !!(want & 4)), MIS_ERR_GENERATION_FAILED,

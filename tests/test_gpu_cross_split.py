@@ -1,5 +1,5 @@
-"""-m gpu: Whisper's cross-attention on one, two or four blocks a (row, head) (`k_attn_cross`): a row's logits do not depend on the split, and
-every split is within the tolerance that the whole decoder is held to (bf16 at every primitive boundary: 0.022 of the largest logit)."""
+"""-m gpu: Whisper's cross-attention on one (`k_attn_decode<64, 2, true, QP>`), two or four blocks a (row, head) (`k_attn_cross`): a row's logits do
+not depend on the split, and every split is within the tolerance that the whole decoder is held to (bf16 at every primitive boundary: 0.022 of the largest logit)."""
 import numpy as np
 import pytest
 
@@ -16,8 +16,8 @@ def _model(d, heads):
     return cfg, ow.WhisperOracle(cfg, W, round="bf16"), mas.WhisperModel.from_weights(mas.WhisperConfig(**{k: getattr(cfg, k) for k in mas.WhisperConfig.__dataclass_fields__}), W)
 
 
-# (width, heads, rows): four blocks up to 64 (row, head) pairs and a width of 640, two up to 128, one beyond; the projection folded in up to 16 rows (3 or 5
-# k-tiles a wave, ragged slices at widths 320 and 832), as slabs beyond
+# (width, heads, rows): four blocks up to 64 (row, head) pairs, two up to 128, one beyond; the projection folded in up to 16 rows (two, three or five
+# k-tiles a slice, ragged slices at widths 320 and 832), as slabs beyond
 @pytest.mark.parametrize("d,heads,rows,fold", [(256, 4, (1, 16), None), (320, 5, (1, 12, 13, 16), None), (832, 13, (1, 4, 9, 10), None), (640, 10, (1, 6, 7, 13), None),
                                                (256, 4, (1, 16, 17, 32, 33), "0")])
 def test_rows_do_not_depend_on_the_split(monkeypatch, d, heads, rows, fold):
