@@ -1,9 +1,24 @@
+// gemm_tiles.h - bf16 matrix products on tiles of 32 TM x 256 outputs, four waves, one persistent block a compute unit.
+//
+// What bounds a bf16 product on this part once its operands come from L2 is the LDS: a compute unit reads 128 bytes a cycle, and the eight waves of a
+// 256 x 256 tile with 64 x 128 outputs each ask for 192 KB of fragments a k-step of 64 (1536 cycles, and 512 for the LDS-DMA that fills the
+// buffers) beside 2048 cycles of MFMA.  Four waves with 128 x 16 TM outputs each read 128 KB; a wave then has a SIMD's 512 registers for itself
+// (accumulators in the AGPRs, two halves of a k-step's fragments in VGPRs), and nothing but its own instruction order overlaps its work:
+//   * the fragments of the next half are requested between the MFMAs of this one, every S-th instruction, and have arrived when it ends;
+//   * a k-step has ONE barrier, in its middle: behind it the buffer just read is refilled (NBUF - 1 k-steps ahead) and the next one is read;
+//   * MFMAs, LDS reads and waits are asm statements, so that their order is the one written here and the accumulators stay where they are
+//     (with the builtins hipcc moved 200 of them between the register files every k-step: 855 against 1103 TFLOP/s);
+//   * the block goes on to its next tile without a gap: the last k-steps of a tile request the first ones of the next, the epilogue runs meanwhile.
+// Measured (8192^3, us): TM 8 862, TM 6 903, TM 5 903, TM 4 924 - 1275 .. 1190 TFLOP/s; torch.matmul 935.  Smaller TM are there because tiles come in whole
+// rounds of 256 blocks (the callers choose).  Products are added in the order of k: the bits of k_gemm_pf and k_gemm_big2 / 3.
 #pragma once
 #include "common.h"
 
 __device__ __forceinline__ uint32_t gt_lds_offset(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
 
-// acc[i][j] += W tile (128 wn + 16 i) x X tile (16 TM wm + 16 j) of a block of four waves (wn = wave >> 1, wm = wave & 1)
+// Wave (wn, wm) = (wave >> 1, wave & 1) holds W rows 128 wn + 16 i and X rows 16 TM wm + 16 j of the tile in acc[i][j] (the MFMA's C/D layout).
+// PACKED: W as the decode step's tiles [N/16][K/32][64][8], a fragment 1 KB lane-linear in memory and in LDS; else rows of K elements, their 16-byte
+// pieces swizzled on the way to LDS.  X: rows.  K: a multiple of 64, NBUF k-steps at least.  Offsets are 32-bit: operands of less than 2^31 elements.
 template <int TM, bool PACKED>
 struct GemmTiles {
     static constexpr int TN = 8, BN = 256, BM = 32 * TM, BK = 64, QW = 8, QX = TM, NQ = QW + QX;
@@ -11,8 +26,8 @@ struct GemmTiles {
     static constexpr int NBUF = STEP * 3 <= 160 * 1024 ? 3 : 2;
     static constexpr int LDS = NBUF * STEP;
 
-    // tile t of `tiles` for t = first, first + stride, ...: woff(t, q, lane) / xoff(t, row): element offsets of a lane's piece of W and of the start of an X row;
-    // epi(t, acc) stores a finished tile
+    // tiles first, first + stride, ... < tiles.  woff(t, q, lane): element offset of the lane's 16 bytes of the tile's q-th KB of W at k = 0; xoff(t, r): of row r
+    // of its X; epi(t, acc) stores a finished tile
     template <class FW, class FX, class FE>
     static __device__ __forceinline__ void run(unsigned char* lds, const bf16_t* Wb, const bf16_t* Xb, int K, int first, int stride, int tiles, FW woff, FX xoff, FE epi) {
         const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wave >> 1, wm = wave & 1;
@@ -96,6 +111,7 @@ struct GemmTiles {
             buf = nb;
         };
         for (;;) {
+            asm volatile("s_nop 7" ::: "memory");                   // (cleared accumulators: written by the VALU, next read by an MFMA that the compiler does not see)
 #pragma unroll 1
             for (int ks = NBUF; ks < KS; ++ks) step(ks);
             const bool more = t + stride < tiles;                   // the last NBUF steps request the next tile's first ones (or their own last one again, never read)

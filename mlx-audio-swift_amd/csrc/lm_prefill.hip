@@ -21,6 +21,7 @@
 //   k_pf_pack_rows      rows of the last position -> the packed x operand of the decode step (lm_head of the first new token)
 // Rounding points are those of the decode step (bf16 at every MLX primitive boundary); only float32 summation orders differ.
 #include "common.h"
+#include "gemm_tiles.h"
 #include "lm_kernels.h"
 
 #include <type_traits>
@@ -282,6 +283,49 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf(PfGemmParams p) {
     pf_epilogue<EPI, 4, 4>(p, acc, (n0 >> 4) + wn * 4, m0 + wm * 64, lane);
 }
 
+// Many rows: tiles of 32 TM rows x 256 columns on four waves (gemm_tiles.h), persistent blocks.  Orpheus-3B, 3600 rows, us per launch, k_gemm_pf / here: gate | up
+// 348 / 318, q|k|v 134 / 115, o and down together 160 / 125 on average (696 tiles of 128 x 128 are 1.4 rounds of 512 blocks; 228 tiles of 192 rows one
+// of 256).  From 300 rows on no size was slower.  TM: the rounds decide - o and down at 3075 rows: 240 tiles with TM 5 132 us, 204 with TM 6 148, 300 with
+// TM 4 188.  The same MFMA instruction and k order: the bits of k_gemm_pf, which keeps the epilogues of the layer-list models.
+template <int EPI, int TM>
+__global__ void __launch_bounds__(256, 1) k_gemm_pf_wide(PfGemmParams p, int mt, int tiles) {
+    using G = GemmTiles<TM, true>;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[G::LDS];
+    // the tiles of an XCD (blocks are dealt to the XCDs by id mod 8) are one range, row tiles fastest: its L2 holds the X tiles and passes over W once
+    const int xcd = blockIdx.x & 7, lo = (int)((int64_t)tiles * xcd / 8), hi = (int)((int64_t)tiles * (xcd + 1) / 8), first = lo + (blockIdx.x >> 3);
+    if (first >= hi) return;
+    const int NT = p.N >> 4, KT = p.K >> 5, ldx = EPI == PF_ROWS_BF16 ? p.ex.ldx : p.K;
+    G::run(lds, p.Wp, p.X, p.K, first, gridDim.x >> 3, hi,
+           [&](int t, int q, int lane) { return ((uint32_t)min(t / mt * (G::BN / 16) + (q >> 1), NT - 1) * KT + (q & 1)) * 512u + lane * 8; },
+           [&](int t, int r) { return (uint32_t)min(t % mt * G::BM + r, p.M - 1) * ldx; },
+           [&](int t, const f32x4_t (&acc)[G::TN][TM]) {
+               const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+               pf_epilogue<EPI, G::TN, TM>(p, acc, t / mt * (G::BN / 16) + (wave >> 1) * G::TN, t % mt * G::BM + (wave & 1) * TM * 16, lane);
+           });
+}
+template <int EPI>
+static bool launch_gemm_pf_wide(const PfGemmParams& p, hipStream_t s) {
+    const int64_t ldx = EPI == PF_ROWS_BF16 ? p.ex.ldx : p.K;
+    // (32-bit byte offsets; three k-steps at least fill the ring)
+    if (p.K < 3 * PF_BK || (EPI == PF_ROWS_BF16 && p.ex.xrow) || (int64_t)p.N * p.K >= (1ll << 31) || (int64_t)p.M * ldx >= (1ll << 31)) return false;
+    const int nt = cdiv(p.N, 256);
+    int best = 0;
+    double least = 0;
+    for (int tm = 4; tm <= 6; ++tm) {                      // rounds of 256 blocks, each as long as its tiles are high and a little
+        const double cost = cdiv(nt * cdiv(p.M, 32 * tm), 256) * (tm + 0.4);
+        if (!best || cost < least) { best = tm; least = cost; }
+    }
+    auto go = [&](auto tag) {
+        constexpr int TM = decltype(tag)::value;
+        const int mt = cdiv(p.M, 32 * TM), tiles = mt * nt;
+        hipLaunchKernelGGL((k_gemm_pf_wide<EPI, TM>), dim3(std::min((int)round_up(tiles, 8), 256)), dim3(256), 0, s, p, mt, tiles);
+    };
+    if (best == 4) go(std::integral_constant<int, 4>{});
+    else if (best == 5) go(std::integral_constant<int, 5>{});
+    else go(std::integral_constant<int, 6>{});
+    return true;
+}
+
 // Few rows: k_gemm_pf waits 0.6 us for each of its 48 - 128 k-steps, and a short prompt's 24 - 128 tiles of 128 x 128 leave most of the chip idle meanwhile.
 // Tiles of 32 rows x 32 columns (gate | up: 64, the pairs of a wave) on two waves, with a ring of NBUF k-steps in LDS requested ahead under counted waits: bound
 // by the weights' way from memory.  The same MFMA instruction and k order: the bits of k_gemm_pf.  Orpheus-3B, us per launch, k_gemm_pf / here: 24 rows:
@@ -377,6 +421,9 @@ void launch_gemm_pf(int epi, const bf16_t* X, const bf16_t* Wp, void* C, int M, 
     if (epi == PF_RESID && few(std::integral_constant<int, PF_RESID>{})) return;
     if (epi == PF_SILU && few(std::integral_constant<int, PF_SILU>{})) return;
     if (epi == PF_ROWS_BF16 && few(std::integral_constant<int, PF_ROWS_BF16>{})) return;
+    if (epi == PF_RESID && launch_gemm_pf_wide<PF_RESID>(p, s)) return;
+    if (epi == PF_SILU && launch_gemm_pf_wide<PF_SILU>(p, s)) return;
+    if (epi == PF_ROWS_BF16 && launch_gemm_pf_wide<PF_ROWS_BF16>(p, s)) return;
     // column tiles rounded up to the 8 XCDs: blocks are dealt to the XCDs by linear id, so that every row of tiles finds its weight tiles in the
     // L2 that held them for the row before
     const int nx = cdiv(N, PF_BN);
