@@ -814,9 +814,9 @@ static void prefill_small(mis_tts* c, const int32_t* prompt_mat_dev, const int32
     HIP_CHECK(hipMemsetAsync(c->pf_xpk.p, 0, Mc * d * 2, s));
     HIP_CHECK(hipMemsetAsync(c->pf_pos.p, 0, Mc * 4, s));
     HIP_CHECK(hipMemsetAsync(c->pf_on.p, 0, Mc, s));
-    if (embed_rows) launch_pf_rows_rmsnorm(embed_rows, Mpad, lens_dev, Lmax, 0, Lmax, batch, batch, c->norms.p, c->pf_h.p, c->pf_x.p, c->pf_pos.p, c->pf_on.p, d, eps, s);
+    if (embed_rows) launch_pf_rows_rmsnorm(embed_rows, Mpad, lens_dev, Lmax, 0, Lmax, batch, batch, c->norms.p, c->pf_h.p, c->pf_x.p, c->pf_pos.p, c->pf_on.p, Mr, d, eps, s);
     else launch_pf_embed_rmsnorm(c->emb.p, prompt_mat_dev, lens_dev, Lmax, 0, Lmax, batch, batch, c->V, c->norms.p, c->pf_h.p, c->pf_x.p, c->pf_pos.p,
-                                 c->pf_on.p, d, eps, s);
+                                 c->pf_on.p, Mr, d, eps, s);
     launch_pf_pack_rows(c->pf_x.p, c->pf_xpk.p, Mp, d, s);
     const size_t lkv = (size_t)batch * c->Hkv * c->Smax * c->D;
     for (int li = 0; li < c->L; ++li) {
@@ -865,15 +865,18 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     hipStream_t s = c->stream;
     const int d = c->d, HD = c->H * c->D, Mpad = c->Mpad, batch = c->batch;
     const float eps = c->cfg.rms_norm_eps;
-    // rows of the chunk: position-major, one row per sequence (no padding between positions)
-    const int rs = batch;
-    const int Tc = std::min(Lmax, std::max(1, 4096 / rs));                   // positions per chunk: <= 4096 rows of activations
-    const size_t Mc = round_up((size_t)Tc * rs, 16) + Mpad;                  // GEMM rows round up to 16; the last position is read Mpad rows wide
+    // rows of the chunk: the positions of each sequence one after the other (no rows for padding)
+    const int Tc = std::min(Lmax, std::max(1, 4096 / batch));                // positions per chunk: <= 4096 rows of activations
+    auto rows_of = [&](int t0, int tc) {
+        int n = 0;
+        for (int b = 0; b < batch; ++b) n += std::max(0, std::min(tc, t0 + tc - (Lmax - lens[b])));
+        return n;
+    };
+    int most = 1;
+    for (int t0 = 0; t0 < Lmax; t0 += Tc) most = std::max(most, rows_of(t0, std::min(Tc, Lmax - t0)));
+    const size_t Mc = round_up((size_t)most, 16);                            // GEMM rows round up to 16
     c->pf_h.alloc(Mc * d); c->pf_x.alloc(Mc * d); c->pf_attn.alloc(Mc * HD);
     c->pf_q.alloc(Mc * HD); c->pf_pos.alloc(Mc); c->pf_on.alloc(Mc);
-    HIP_CHECK(hipMemsetAsync(c->pf_attn.p, 0, Mc * HD * 2, s));             // rows of padded positions are never written by the attention
-    HIP_CHECK(hipMemsetAsync(c->pf_x.p, 0, Mc * d * 2, s));                 // rows past the chunk (rounding, slack) hold zeros, not stale bits
-    HIP_CHECK(hipMemsetAsync(c->pf_h.p, 0, Mc * d * 2, s));
     // quantised checkpoints (every role streamed as codes): each GEMM of the chunk runs the decode step's k_gemm_skinny_q on 64-row
     // slices - rows packed into MFMA fragments first, float32 sums out, the residual add as its own small kernel; gate|up writes the
     // packed activation its down projection reads.  The weights are streamed once per 64 rows instead of once per position.
@@ -891,16 +894,17 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     int t0 = 0;
     for (; t0 < Lmax; t0 += Tc) {
         const int tc = std::min(Tc, Lmax - t0);
-        const int Mr = tc * rs;                                              // rows that exist
+        const int Mr = rows_of(t0, tc);                                      // rows that exist
         const int M = (int)round_up((size_t)Mr, 16);                         // rows the GEMMs run over
-        if (t0 > 0 && (size_t)Mr < Mc) {                                     // a shorter last chunk: the rows behind it held the previous chunk's
-            HIP_CHECK(hipMemsetAsync(c->pf_x.p + (size_t)Mr * d, 0, (Mc - Mr) * d * 2, s));       // values - zeros again, as the comments below say
-            HIP_CHECK(hipMemsetAsync(c->pf_h.p + (size_t)Mr * d, 0, (Mc - Mr) * d * 2, s));
-            HIP_CHECK(hipMemsetAsync(c->pf_attn.p + (size_t)Mr * HD, 0, (Mc - Mr) * HD * 2, s));
+        if (Mr == 0) continue;                                               // (the longest prompt reaches every chunk; a guard)
+        if (Mr < M) {                                                        // the rounding rows: zeros, not stale bits
+            HIP_CHECK(hipMemsetAsync(c->pf_x.p + (size_t)Mr * d, 0, (size_t)(M - Mr) * d * 2, s));
+            HIP_CHECK(hipMemsetAsync(c->pf_h.p + (size_t)Mr * d, 0, (size_t)(M - Mr) * d * 2, s));
+            HIP_CHECK(hipMemsetAsync(c->pf_attn.p + (size_t)Mr * HD, 0, (size_t)(M - Mr) * HD * 2, s));
         }
-        if (embed_rows) launch_pf_rows_rmsnorm(embed_rows, Mpad, lens_dev, Lmax, t0, tc, batch, rs, c->norms.p, c->pf_h.p, c->pf_x.p, c->pf_pos.p, c->pf_on.p, d, eps, s);
-        else launch_pf_embed_rmsnorm(c->emb.p, prompt_mat_dev, lens_dev, Lmax, t0, tc, batch, rs, c->V, c->norms.p, c->pf_h.p, c->pf_x.p,
-                                     c->pf_pos.p, c->pf_on.p, d, eps, s);
+        if (embed_rows) launch_pf_rows_rmsnorm(embed_rows, Mpad, lens_dev, Lmax, t0, tc, batch, 0, c->norms.p, c->pf_h.p, c->pf_x.p, c->pf_pos.p, c->pf_on.p, Mr, d, eps, s);
+        else launch_pf_embed_rmsnorm(c->emb.p, prompt_mat_dev, lens_dev, Lmax, t0, tc, batch, 0, c->V, c->norms.p, c->pf_h.p, c->pf_x.p,
+                                     c->pf_pos.p, c->pf_on.p, Mr, d, eps, s);
         for (int li = 0; li < c->L; ++li) {
             if (coded) q_rows(M, [&](int r0, int mp) {
                 launch_pf_pack_rows(c->pf_x.p + (size_t)r0 * d, c->pf_xpk.p, mp, d, s);
@@ -915,7 +919,7 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
             pa.qkv = coded ? (const void*)c->pf_qkv.p : (const void*)c->pf_qkv16.p; pa.qkv_f32 = coded;
             pa.q = c->pf_q.p; pa.out = c->pf_attn.p;
             pa.kcache = c->kcache.p + lkv * li; pa.vcache = c->vtcache.p + lkv * li;
-            pa.lens = lens_dev; pa.Lmax = Lmax; pa.t0 = t0; pa.tc = tc; pa.rs = rs; pa.batch = batch;
+            pa.lens = lens_dev; pa.Lmax = Lmax; pa.t0 = t0; pa.tc = tc; pa.batch = batch;
             pa.Nqkv = c->Nqkv; pa.H = c->H; pa.Hkv = c->Hkv; pa.D = c->D; pa.Smax = c->Smax;
             pa.rope_cos = c->rope_cos.p; pa.rope_sin = c->rope_sin.p; pa.scale = 1.0f / sqrtf((float)c->D);
             if (c->cfg.qk_norm) {
@@ -946,10 +950,8 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
             const bf16_t* next_norm = c->norms.p + (size_t)(li + 1 < c->L ? 2 * (li + 1) : 2 * c->L) * d;
             launch_pf_rmsnorm(c->pf_h.p, next_norm, c->pf_x.p, M, d, eps, s);
         }
-        if (t0 + tc >= Lmax) {                                               // left-padded prompts: every row's last token is position Lmax - 1
-            // rows batch .. Mpad-1 of the packed x belong to no sequence: what follows the last position in pf_x (zeros, or the rounding rows)
-            launch_pf_pack_rows(c->pf_x.p + (size_t)(tc - 1) * rs * d, c->x.p, Mpad, d, s);
-        }
+        if (t0 + tc >= Lmax)                                                 // left-padded prompts: the last chunk holds every row's last token
+            launch_pf_pack_last(c->pf_x.p, lens_dev, Lmax, t0, tc, batch, c->x.p, Mpad, d, s);
     }
     std::vector<int32_t> pn(Mpad, 0), pc(Mpad, 0);
     for (int b = 0; b < batch; ++b) { pn[b] = lens[b]; pc[b] = lens[b] - 1; }

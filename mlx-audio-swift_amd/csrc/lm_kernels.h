@@ -69,21 +69,22 @@ enum { PF_F32 = 0, PF_RESID = 1, PF_SILU = 2,
 struct PfExtra { int ldx = 0; const int32_t* xrow = nullptr; int ldc = 0; void* out2 = nullptr; int split = 0, ld2 = 0; const bf16_t* ls = nullptr; float scale = 1.0f, cap = 0.0f; };
 void launch_gemm_pf(int epi, const bf16_t* X, const bf16_t* Wp, void* C, int M, int N, int K, hipStream_t s, const PfExtra& ex = PfExtra());
 void launch_pf_embed_rmsnorm(const bf16_t* emb, const int32_t* prompt, const int32_t* lens, int Lmax, int t0, int Tc, int batch, int Mpad, int vocab,
-                             const bf16_t* wnorm, bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int d, float eps, hipStream_t s);
+                             const bf16_t* wnorm, bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int rows, int d, float eps, hipStream_t s);
+void launch_pf_pack_last(const bf16_t* rows, const int32_t* lens, int Lmax, int t0, int Tc, int batch, bf16_t* xpk, int Mpad, int d, hipStream_t s);
 void launch_pf_add_resid(bf16_t* h, const float* part, size_t n, hipStream_t s);
 void launch_pf_rows_rmsnorm(const bf16_t* rows, int src_rows, const int32_t* lens, int Lmax, int t0, int Tc, int batch, int Mpad, const bf16_t* wnorm,
-                            bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int d, float eps, hipStream_t s);
+                            bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int n_rows, int d, float eps, hipStream_t s);
 void launch_pf_rmsnorm(const bf16_t* h, const bf16_t* wnorm, bf16_t* x, int rows, int d, float eps, hipStream_t s);
 void launch_pf_pack_rows(const bf16_t* rows, bf16_t* xpk, int Mpad, int d, hipStream_t s);
 
-// causal attention of the chunk of positions [t0, t0 + tc) of `batch` left-padded prompts (row (t - t0) * rs + b; lens: device): q|k|v -> norm, rotation,
-// cache append, attention over the caches.  q: scratch for the roped queries, out: bf16 [rows][H D] (rows of padded positions are not written)
+// causal attention of the chunk of positions [t0, t0 + tc) of `batch` left-padded prompts (packed rows: the positions of sequence 0, of sequence 1, ...; lens: device): q|k|v -> norm, rotation,
+// cache append, attention over the caches.  q: scratch for the roped queries, out: bf16 [rows][H D] 
 struct PfAttn {
     const void* qkv; int qkv_f32;            // [rows][Nqkv] float32 or bf16
     bf16_t *q, *out;
     bf16_t *kcache, *vcache;                 // layer slices, tiled
     const int32_t* lens;
-    int Lmax, t0, tc, rs, batch, Nqkv, H, Hkv, D, Smax;
+    int Lmax, t0, tc, batch, Nqkv, H, Hkv, D, Smax;
     const float *rope_cos, *rope_sin;
     const bf16_t *qnorm_w, *knorm_w;         // null: no per-head norm
     float qk_eps, scale;

@@ -5,7 +5,8 @@
 // passes: 56 ms of the 1.6 s bench job for 32-token prompts, and linear in L - voice-cloning prompts carry hundreds of audio tokens).
 // Here all L x B prompt tokens form the M dimension of four GEMMs per layer (M = 1024 at the bench shape), each weight byte is read
 // once per CHUNK of positions instead of once per position, and the attention takes the chunk's queries together over the decode step's
-// caches.  Rows are laid out position-major: row r = t * rs + b, rs rows per position (the batch).
+// caches.  Rows are PACKED: the chunk's positions of sequence 0, then those of sequence 1, ... - no row stands for the padding of a shorter prompt
+// (prompts of 300 .. 450 tokens padded to 450: 15 % of every GEMM).
 //
 //   k_pf_embed_rmsnorm  h[r] = E[token(b, t)], x[r] = RMSNorm(h[r]) (row-major), active / position tables of every (t, b)
 //   k_gemm_pf<EPI>      C[M][N] = X[M][K] . W^T with W in the decode path's packed MFMA-A tile layout [N/16][K/32][64][8]:
@@ -40,17 +41,45 @@ __device__ __forceinline__ float pf_block_sum_256(float v, float* red) {
     return t;
 }
 
-// one 256-thread block per row r = t*Mpad + b of the chunk [t0, t0 + Tc)
+// The chunk [t0, t0 + tc) of left-padded prompts: sequence b has n = hi - lo positions [lo, hi) in it, position p is packed row row0 + p
+struct PfSpan { int lo, hi, row0; };
+__device__ __forceinline__ int pf_count(const int32_t* lens, int b, int Lmax, int t0, int tc, int& lo) {
+    const int shift = Lmax - lens[b] - t0;
+    lo = max(0, -shift);
+    return max(0, tc - shift - lo);
+}
+__device__ __forceinline__ PfSpan pf_span(const int32_t* lens, int b, int Lmax, int t0, int tc) {
+    int row = 0, lo;
+    for (int i = 0; i < b; ++i) row += pf_count(lens, i, Lmax, t0, tc, lo);
+    const int n = pf_count(lens, b, Lmax, t0, tc, lo);
+    return PfSpan{lo, lo + n, row - lo};
+}
+// (sequence, left-padded position) of row r; Mpad = 0: packed rows, else row t * Mpad + b
+__device__ __forceinline__ bool pf_row(const int32_t* lens, int r, int Lmax, int t0, int tc, int batch, int Mpad, int& b, int& t) {
+    if (Mpad) {
+        const int tl = r / Mpad;
+        b = r - tl * Mpad; t = t0 + tl;
+        return b < batch && t >= Lmax - lens[b];
+    }
+    for (b = 0; b < batch; ++b) {
+        int lo;
+        const int n = pf_count(lens, b, Lmax, t0, tc, lo);
+        if (r < n) { t = Lmax - lens[b] + lo + r; return true; }
+        r -= n;
+    }
+    b = 0; t = t0;
+    return false;
+}
+// one 256-thread block per row of the chunk [t0, t0 + tc)
 __global__ void __launch_bounds__(256) k_pf_embed_rmsnorm(const bf16_t* __restrict__ emb, const int32_t* __restrict__ prompt /*[batch][Lmax] left padded*/,
-                                                          const int32_t* __restrict__ lens, int Lmax, int t0, int batch, int Mpad, int vocab,
+                                                          const int32_t* __restrict__ lens, int Lmax, int t0, int tc, int batch, int Mpad, int vocab,
                                                           const bf16_t* __restrict__ wnorm, bf16_t* __restrict__ h, bf16_t* __restrict__ x,
                                                           int32_t* __restrict__ pos_tab, uint8_t* __restrict__ act_tab, int d, float eps) {
     __shared__ float red[4];
-    const int r = blockIdx.x, tl = r / Mpad, b = r - tl * Mpad, t = t0 + tl;
-    const bool row = b < batch;
-    const int len = row ? lens[b] : 0;
-    const bool on = row && t >= Lmax - len;
-    if (threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - len) : 0; act_tab[r] = on ? 1 : 0; }
+    const int r = blockIdx.x;
+    int b, t;
+    const bool on = pf_row(lens, r, Lmax, t0, tc, batch, Mpad, b, t);
+    if (threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - lens[b]) : 0; act_tab[r] = on ? 1 : 0; }
     int id = on ? prompt[(size_t)b * Lmax + t] : -1;
     if (id >= vocab) id = -1;
     const bf16_t* e = emb + (size_t)(id < 0 ? 0 : id) * d;
@@ -68,16 +97,15 @@ __global__ void __launch_bounds__(256) k_pf_embed_rmsnorm(const bf16_t* __restri
     }
 }
 // the same for engines that feed input embeddings instead of token ids (Qwen3-TTS talker): rows [Lmax][src_rows][d] computed by the
-// caller; `Mpad` here and in k_pf_embed_rmsnorm is the chunk's rows per position (the batch)
-__global__ void __launch_bounds__(256) k_pf_rows_rmsnorm(const bf16_t* __restrict__ rows, int src_rows, const int32_t* __restrict__ lens, int Lmax, int t0, int batch,
+// caller; `Mpad` here and in k_pf_embed_rmsnorm is the chunk's rows per position (the batch), 0 for packed rows
+__global__ void __launch_bounds__(256) k_pf_rows_rmsnorm(const bf16_t* __restrict__ rows, int src_rows, const int32_t* __restrict__ lens, int Lmax, int t0, int tc, int batch,
                                                          int Mpad, const bf16_t* __restrict__ wnorm, bf16_t* __restrict__ h, bf16_t* __restrict__ x,
                                                          int32_t* __restrict__ pos_tab, uint8_t* __restrict__ act_tab, int d, float eps) {
     __shared__ float red[4];
-    const int r = blockIdx.x, tl = r / Mpad, b = r - tl * Mpad, t = t0 + tl;
-    const bool row = b < batch;
-    const int len = row ? lens[b] : 0;
-    const bool on = row && t >= Lmax - len;
-    if (threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - len) : 0; act_tab[r] = on ? 1 : 0; }
+    const int r = blockIdx.x;
+    int b, t;
+    const bool on = pf_row(lens, r, Lmax, t0, tc, batch, Mpad, b, t);
+    if (threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - lens[b]) : 0; act_tab[r] = on ? 1 : 0; }
     const bf16_t* e = rows + ((size_t)t * src_rows + b) * d;                   // the caller's matrix keeps its own rows per position
     float ss = 0.0f;
     for (int i = threadIdx.x; i < d; i += 256) {
@@ -101,6 +129,14 @@ __global__ void __launch_bounds__(256) k_pf_rmsnorm(const bf16_t* __restrict__ h
     const float inv = 1.0f / sqrtf(pf_block_sum_256(ss, red) / (float)d + eps);
     for (int i = threadIdx.x; i < d; i += 256)
         x[r * d + i] = f32_to_bf16(bf16_to_f32(wnorm[i]) * bf16_round_f32(bf16_to_f32(h[r * d + i]) * inv));
+}
+// the row of every sequence's last position (packed rows; Mpad - batch rows of zeros behind them) -> packed MFMA-B fragments of the decode step's x operand
+__global__ void k_pf_pack_last(const bf16_t* __restrict__ rows, const int32_t* __restrict__ lens, int Lmax, int t0, int tc, int batch, bf16_t* __restrict__ xpk, int d, int MT) {
+    const int m = blockIdx.x;
+    const PfSpan sp = pf_span(lens, min(m, batch - 1), Lmax, t0, tc);
+    const bool on = m < batch && sp.hi > sp.lo;                    // (an empty prompt has no row)
+    const bf16_t* src = rows + (size_t)(on ? sp.row0 + sp.hi - 1 : 0) * d;
+    for (int k = threadIdx.x; k < d; k += blockDim.x) xpk[xpk_index(m, k, MT)] = on ? src[k] : (bf16_t)0;
 }
 // rows [Mpad][d] row-major -> packed MFMA-B fragments of the decode step's x operand
 __global__ void k_pf_pack_rows(const bf16_t* __restrict__ rows, bf16_t* __restrict__ xpk, int d, int MT) {
@@ -440,13 +476,13 @@ void launch_gemm_pf(int epi, const bf16_t* X, const bf16_t* Wp, void* C, int M, 
     else throw MisError(MIS_ERR_GENERATION_FAILED, "unknown prefill GEMM epilogue");
 }
 void launch_pf_embed_rmsnorm(const bf16_t* emb, const int32_t* prompt, const int32_t* lens, int Lmax, int t0, int Tc, int batch, int Mpad, int vocab,
-                             const bf16_t* wnorm, bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int d, float eps, hipStream_t s) {
-    hipLaunchKernelGGL(k_pf_embed_rmsnorm, dim3(Tc * Mpad), dim3(256), 0, s, emb, prompt, lens, Lmax, t0, batch, Mpad, vocab, wnorm, h, x, pos_tab,
+                             const bf16_t* wnorm, bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int rows, int d, float eps, hipStream_t s) {
+    hipLaunchKernelGGL(k_pf_embed_rmsnorm, dim3(rows), dim3(256), 0, s, emb, prompt, lens, Lmax, t0, Tc, batch, Mpad, vocab, wnorm, h, x, pos_tab,
                        act_tab, d, eps);
 }
 void launch_pf_rows_rmsnorm(const bf16_t* rows, int src_rows, const int32_t* lens, int Lmax, int t0, int Tc, int batch, int Mpad, const bf16_t* wnorm,
-                            bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int d, float eps, hipStream_t s) {
-    hipLaunchKernelGGL(k_pf_rows_rmsnorm, dim3(Tc * Mpad), dim3(256), 0, s, rows, src_rows, lens, Lmax, t0, batch, Mpad, wnorm, h, x, pos_tab, act_tab, d, eps);
+                            bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int n_rows, int d, float eps, hipStream_t s) {
+    hipLaunchKernelGGL(k_pf_rows_rmsnorm, dim3(n_rows), dim3(256), 0, s, rows, src_rows, lens, Lmax, t0, Tc, batch, Mpad, wnorm, h, x, pos_tab, act_tab, d, eps);
 }
 void launch_pf_rmsnorm(const bf16_t* h, const bf16_t* wnorm, bf16_t* x, int rows, int d, float eps, hipStream_t s) {
     hipLaunchKernelGGL(k_pf_rmsnorm, dim3(rows), dim3(256), 0, s, h, wnorm, x, d, eps);
@@ -459,6 +495,9 @@ __global__ void k_pf_add_resid(bf16_t* __restrict__ h, const float* __restrict__
 }
 void launch_pf_add_resid(bf16_t* h, const float* part, size_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_pf_add_resid, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, h, part, n);
+}
+void launch_pf_pack_last(const bf16_t* rows, const int32_t* lens, int Lmax, int t0, int Tc, int batch, bf16_t* xpk, int Mpad, int d, hipStream_t s) {
+    hipLaunchKernelGGL(k_pf_pack_last, dim3(Mpad), dim3(256), 0, s, rows, lens, Lmax, t0, Tc, batch, xpk, d, Mpad / 16);
 }
 void launch_pf_pack_rows(const bf16_t* rows, bf16_t* xpk, int Mpad, int d, hipStream_t s) {
     hipLaunchKernelGGL(k_pf_pack_rows, dim3(Mpad), dim3(256), 0, s, rows, xpk, d, Mpad / 16);
@@ -481,21 +520,12 @@ struct PfAttnDev {
     const void* qkv; int Nqkv;
     bf16_t *q, *kc, *vc, *out;
     const int32_t* lens;
-    int Lmax, t0, tc, rs, H, Hkv, Smax;
+    int Lmax, t0, tc, H, Hkv, Smax;
     const float *rope_cos, *rope_sin;
     const bf16_t *qnorm_w, *knorm_w;
     float qk_eps, scale;
     int rope_in_dtype;
 };
-// positions of sequence b that the chunk holds: [lo, hi); position p is row (p + shift) * rs + b
-struct PfSpan { int lo, hi, shift; };
-__device__ __forceinline__ PfSpan pf_span(const PfAttnDev& p, int b) {
-    PfSpan r;
-    r.shift = p.Lmax - p.lens[b] - p.t0;
-    r.lo = max(0, -r.shift);
-    r.hi = p.tc - r.shift;
-    return r;
-}
 __device__ __forceinline__ void pf_load8(const float* src, float (&v)[8]) {
     const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
     v[0] = bf16_round_f32(a.x); v[1] = bf16_round_f32(a.y); v[2] = bf16_round_f32(a.z); v[3] = bf16_round_f32(a.w);
@@ -511,7 +541,7 @@ __global__ void __launch_bounds__(256) k_pf_rope_append(PfAttnDev p) {
     constexpr int VT = D / 16;                                   // threads per head row: 8 dimensions and their 8 rotation partners each
     __shared__ __attribute__((aligned(16))) bf16_t vs[32][D + 8];
     const int b = blockIdx.z, kvh = blockIdx.y, tid = threadIdx.x;
-    const PfSpan sp = pf_span(p, b);
+    const PfSpan sp = pf_span(p.lens, b, p.Lmax, p.t0, p.tc);
     const int tile = (sp.lo >> 5) + blockIdx.x, p0 = max(tile * 32, sp.lo), p1 = min(tile * 32 + 32, sp.hi);
     if (p0 >= p1) return;
     const int G = p.H / p.Hkv;
@@ -520,7 +550,7 @@ __global__ void __launch_bounds__(256) k_pf_rope_append(PfAttnDev p) {
     bf16_t* vc = p.vc + ((size_t)(b * p.Hkv + kvh) * p.Smax) * D;
     for (int it = tid; it < (p1 - p0) * VT * 2; it += 256) {     // V rows -> LDS
         const int i = it / (VT * 2), c = it - i * (VT * 2), pos = p0 + i;
-        const size_t row = (size_t)(pos + sp.shift) * p.rs + b;
+        const size_t row = sp.row0 + pos;
         float v[8];
         pf_load8(qkv + row * p.Nqkv + (size_t)(p.H + p.Hkv + kvh) * D + c * 8, v);
         bf16x8_t o;
@@ -530,7 +560,7 @@ __global__ void __launch_bounds__(256) k_pf_rope_append(PfAttnDev p) {
     }
     for (int it = tid; it < (p1 - p0) * (G + 1) * VT; it += 256) {
         const int j = it % VT, hr = it / VT, i = hr / (G + 1), hh = hr - i * (G + 1), pos = p0 + i;
-        const size_t row = (size_t)(pos + sp.shift) * p.rs + b;
+        const size_t row = sp.row0 + pos;
         const int col = (hh < G ? kvh * G + hh : p.H + kvh) * D + j * 8;
         float x1[8], x2[8];
         pf_load8(qkv + row * p.Nqkv + col, x1);
@@ -600,7 +630,7 @@ __global__ void __launch_bounds__(NW * 64) k_pf_attn(PfAttnDev p) {
     __shared__ __attribute__((aligned(16))) bf16_t kv[2][2 * IMG];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int kvh = blockIdx.y, b = blockIdx.z, G = p.H / p.Hkv;
-    const PfSpan sp = pf_span(p, b);
+    const PfSpan sp = pf_span(p.lens, b, p.Lmax, p.t0, p.tc);
     const int nq = (sp.hi - sp.lo) * G;
     const int nb = (nq + 32 * NW - 1) / (32 * NW), blk = nb - 1 - (int)blockIdx.x;   // the longest blocks first
     if (blk < 0) return;
@@ -614,7 +644,7 @@ __global__ void __launch_bounds__(NW * 64) k_pf_attn(PfAttnDev p) {
         const int n = min(w0 + 16 * g + j, nq - 1);                  // (queries past the list repeat the last one; never written)
         const int pos = sp.lo + n / G;
         qpos[g] = pos;
-        const bf16_t* src = p.q + ((size_t)(pos + sp.shift) * p.rs + b) * HD + (size_t)(kvh * G + n % G) * D + g4 * 8;
+        const bf16_t* src = p.q + (size_t)(sp.row0 + pos) * HD + (size_t)(kvh * G + n % G) * D + g4 * 8;
 #pragma unroll
         for (int c = 0; c < D / 32; ++c) qf[g][c] = *reinterpret_cast<const bf16x8_t*>(src + c * 32);
     }
@@ -726,7 +756,7 @@ __global__ void __launch_bounds__(NW * 64) k_pf_attn(PfAttnDev p) {
             const float lr = __shfl(l, g4 * 4 + r, 64);
             const int n = w0 + 16 * g + g4 * 4 + r;
             if (n < nq) {
-                bf16_t* o = p.out + ((size_t)(sp.lo + n / G + sp.shift) * p.rs + b) * HD + (size_t)(kvh * G + n % G) * D + j;
+                bf16_t* o = p.out + (size_t)(sp.row0 + sp.lo + n / G) * HD + (size_t)(kvh * G + n % G) * D + j;
 #pragma unroll
                 for (int dt = 0; dt < D / 16; ++dt) o[dt * 16] = f32_to_bf16(O[g][dt][r] / lr);
             }
@@ -736,10 +766,10 @@ __global__ void __launch_bounds__(NW * 64) k_pf_attn(PfAttnDev p) {
 
 void launch_pf_attention(const PfAttn& a, hipStream_t s) {
     MIS_REQUIRE(a.D == 64 || a.D == 128, MIS_ERR_INVALID_INPUT, "head_dim must be 64 or 128");
-    MIS_REQUIRE(a.H % a.Hkv == 0 && a.Smax % 32 == 0 && a.t0 + a.tc <= a.Smax && a.Nqkv == (a.H + 2 * a.Hkv) * a.D && a.rs >= a.batch, MIS_ERR_GENERATION_FAILED,
+    MIS_REQUIRE(a.H % a.Hkv == 0 && a.Smax % 32 == 0 && a.t0 + a.tc <= a.Smax && a.Nqkv == (a.H + 2 * a.Hkv) * a.D, MIS_ERR_GENERATION_FAILED,
                 "prompt attention: bad dimensions");
     MIS_REQUIRE((((uintptr_t)a.qkv | (uintptr_t)a.q | (uintptr_t)a.kcache | (uintptr_t)a.vcache) & 15) == 0, MIS_ERR_GENERATION_FAILED, "prompt attention: misaligned buffers");
-    PfAttnDev p{a.qkv, a.Nqkv, a.q, a.kcache, a.vcache, a.out, a.lens, a.Lmax, a.t0, a.tc, a.rs, a.H, a.Hkv, a.Smax, a.rope_cos, a.rope_sin, a.qnorm_w, a.knorm_w,
+    PfAttnDev p{a.qkv, a.Nqkv, a.q, a.kcache, a.vcache, a.out, a.lens, a.Lmax, a.t0, a.tc, a.H, a.Hkv, a.Smax, a.rope_cos, a.rope_sin, a.qnorm_w, a.knorm_w,
                 a.qk_eps, a.scale, a.rope_in_dtype};
     const dim3 ga(a.tc / 32 + 2, a.Hkv, a.batch);                    // 32-key tiles that tc consecutive positions can touch
     const int nq = a.tc * (a.H / a.Hkv);
