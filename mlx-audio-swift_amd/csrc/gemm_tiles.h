@@ -34,12 +34,14 @@ struct GemmTiles {
         const int KS = K / BK;
         uint32_t off[NQ];                                            // bytes
         auto point = [&](int t) {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));                             // (computed here for each tile: hoisted, these take the registers that TM = 8 has not got)
 #pragma unroll
-            for (int q = 0; q < QW; ++q) off[q] = 2 * (uint32_t)woff(t, wave * QW + q, lane);
+            for (int q = 0; q < QW; ++q) off[q] = 2 * (uint32_t)woff(t, wave * QW + q, ln);
 #pragma unroll
             for (int q = 0; q < QX; ++q) {
-                const int r = (wave * QX + q) * 8 + (lane >> 3);
-                off[QW + q] = 2 * ((uint32_t)xoff(t, r) + ((lane & 7) ^ ((r >> 1) & 7)) * 8);
+                const int r = (wave * QX + q) * 8 + (ln >> 3);
+                off[QW + q] = 2 * ((uint32_t)xoff(t, r) + ((ln & 7) ^ ((r >> 1) & 7)) * 8);
             }
         };
         auto stage1 = [&](int buf, int ks, int n) {                  // the n-th LDS load of a k-step

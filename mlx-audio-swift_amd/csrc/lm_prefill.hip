@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf(PfGemmParams p) {
 }
 
 // Many rows: tiles of 32 TM rows x 256 columns on four waves (gemm_tiles.h), persistent blocks.  Orpheus-3B, 3600 rows, us per launch, k_gemm_pf / here: gate | up
-// 348 / 318, q|k|v 134 / 115, o and down together 160 / 125 on average (696 tiles of 128 x 128 are 1.4 rounds of 512 blocks; 228 tiles of 192 rows one
+// 348 / 318, q|k|v 134 / 115, o and down together 160 / 121 on average (696 tiles of 128 x 128 are 1.4 rounds of 512 blocks; 228 tiles of 192 rows one
 // of 256).  From 300 rows on no size was slower.  TM: the rounds decide - o and down at 3075 rows: 240 tiles with TM 5 132 us, 204 with TM 6 148, 300 with
 // TM 4 188.  The same MFMA instruction and k order: the bits of k_gemm_pf, which keeps the epilogues of the layer-list models.
 template <int EPI, int TM>
@@ -335,7 +335,40 @@ __global__ void __launch_bounds__(256, 1) k_gemm_pf_wide(PfGemmParams p, int mt,
            [&](int t, int q, int lane) { return ((uint32_t)min(t / mt * (G::BN / 16) + (q >> 1), NT - 1) * KT + (q & 1)) * 512u + lane * 8; },
            [&](int t, int r) { return (uint32_t)min(t % mt * G::BM + r, p.M - 1) * ldx; },
            [&](int t, const f32x4_t (&acc)[G::TN][TM]) {
-               const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+               int lane = threadIdx.x & 63;
+               asm volatile("" : "+v"(lane));
+               const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+               if constexpr (EPI == PF_RESID) {            // one row of tiles at a time, its residuals requested a row ahead (a wave has no other to wait with)
+                   const int nb = t / mt * G::BN + (wave >> 1) * 128 + (lane >> 4) * 4, mb = t % mt * G::BM + (wave & 1) * TM * 16 + (lane & 15);
+                   bf16_t* h = reinterpret_cast<bf16_t*>(p.C);
+                   uint2 r[2][G::TN];
+                   auto residual = [&](int j, uint2 (&o)[G::TN]) {
+                       const bf16_t* row = h + (size_t)min(mb + j * 16, p.M - 1) * p.N;
+#pragma unroll
+                       for (int i = 0; i < G::TN; ++i) o[i] = *reinterpret_cast<const uint2*>(row + min(nb + i * 16, p.N - 4));
+                   };
+                   residual(0, r[0]);
+#pragma unroll
+                   for (int j = 0; j < TM; ++j) {
+                       if (j + 1 < TM) residual(j + 1, r[(j + 1) & 1]);
+                       __builtin_amdgcn_sched_barrier(0);
+                       const int m = mb + j * 16;
+#pragma unroll
+                       for (int i = 0; i < G::TN; ++i) {
+                           uint2& o = r[j & 1][i];
+                           const float hv[4] = {__uint_as_float(o.x << 16), __uint_as_float(o.x & 0xffff0000u), __uint_as_float(o.y << 16), __uint_as_float(o.y & 0xffff0000u)};
+                           uint16_t v[4];
+#pragma unroll
+                           for (int e = 0; e < 4; ++e) v[e] = f32_to_bf16(hv[e] + bf16_round_f32(acc[i][j][e]));       // h = T(h + T(x W^T))
+                           o = make_uint2((uint32_t)v[0] | ((uint32_t)v[1] << 16), (uint32_t)v[2] | ((uint32_t)v[3] << 16));
+                           asm volatile("" : "+v"(o.x), "+v"(o.y));          // (not inside the branch below: a wait there waits for every store before it)
+                       }
+#pragma unroll
+                       for (int i = 0; i < G::TN; ++i)
+                           if (m < p.M && nb + i * 16 < p.N) *reinterpret_cast<uint2*>(h + (size_t)m * p.N + nb + i * 16) = r[j & 1][i];
+                   }
+                   return;
+               }
                pf_epilogue<EPI, G::TN, TM>(p, acc, t / mt * (G::BN / 16) + (wave >> 1) * G::TN, t % mt * G::BM + (wave & 1) * TM * 16, lane);
            });
 }
