@@ -67,7 +67,7 @@ struct mis_tts {
     DevBuf<float> rope_cos, rope_sin;
     DevBuf<int32_t> ids, pos_cur, pos_next;
     DevBuf<uint8_t> active;
-    DevBuf<bf16_t> h, x, attn_out, act, logits;
+    DevBuf<bf16_t> h, h2, x, attn_out, act, logits;      // h2: the other residual buffer of the folded glue (enqueue_layers)
     DevBuf<float> qkv_part, part, e_buf, logits_f32, samp_l32;
     // generation state
     DevBuf<int32_t> prompt_mat, prompt_lens, step_counter, window, window_len, n_gen, tokens_out, all_ids, all_len,
@@ -683,13 +683,13 @@ static void lm_reset_buffers(mis_tts* c, int batch, int max_context) {
     if (new_tables || !c->rope_cos.p) build_rope_tables(c);
     c->ids.alloc(Mpad); c->pos_cur.alloc(Mpad); c->pos_next.alloc(Mpad); c->active.alloc(Mpad);
     c->ids.zero(s); c->pos_cur.zero(s); c->pos_next.zero(s); c->active.zero(s);
-    c->h.alloc((size_t)Mpad * d); c->x.alloc((size_t)Mpad * d);
+    c->h.alloc((size_t)Mpad * d); c->h2.alloc((size_t)Mpad * d); c->x.alloc((size_t)Mpad * d);
     c->attn_out.alloc((size_t)Mpad * HD); c->act.alloc((size_t)Mpad * c->ff);
     c->logits.alloc((size_t)Mpad * c->Vpad);
     c->e_buf.alloc((size_t)Mpad * c->Vpad);
     c->qkv_part.alloc((size_t)c->S_qkv * Mpad * c->Nqkv);
     c->part.alloc((size_t)std::max(c->S_o, c->S_down) * Mpad * d);
-    c->h.zero(s); c->x.zero(s); c->attn_out.zero(s); c->act.zero(s); c->logits.zero(s);
+    c->h.zero(s); c->h2.zero(s); c->x.zero(s); c->attn_out.zero(s); c->act.zero(s); c->logits.zero(s);
     HIP_CHECK(hipStreamSynchronize(s));
 }
 
@@ -719,6 +719,14 @@ static void gemm_down(mis_tts* c, size_t li, hipStream_t s) {
                             c->d, c->Mpad, s, nullptr, c->a_down.U);
 }
 
+// at one or two rows the glue runs inside the GEMM behind it (k_gemm_glue; MIS_GLUE_FOLD=0: separate launches - parity tests, read per enqueue)
+static bool fold_on() { const char* e = getenv("MIS_GLUE_FOLD"); return !(e && atoi(e) == 0); }
+static bool fold_gate_up(const mis_tts* c) {
+    return fold_on() && !c->blocks && !c->q_gu.on && gemm_glue_ok(EPI_SILU_MUL, c->batch, c->r_gu, c->ksb_gu, 0, c->S_o, c->d, c->Mpad);
+}
+static bool fold_qkv(const mis_tts* c) {
+    return fold_on() && !c->blocks && !c->q_qkv.on && gemm_glue_ok(EPI_PARTIAL, c->batch, c->a_qkv.R, c->a_qkv.ksb, c->a_qkv.U, c->S_down, c->d, c->Mpad);
+}
 // embed -> L x block.  Leaves x = final-norm(h) ready for lm_head.   (LlamaTTS.swift:335-345,303-310)
 // table/rows/ids: embedding source override (composite engines feed input embeddings as a [rows][d] table)
 static void enqueue_layers(mis_tts* c, const bf16_t* table = nullptr, int table_rows = 0, const int32_t* ids = nullptr) {
@@ -726,11 +734,19 @@ static void enqueue_layers(mis_tts* c, const bf16_t* table = nullptr, int table_
     if (c->blocks) { c->blocks->enqueue_step(BlockRows{c->ids.p, c->active.p, c->pos_cur.p, c->pos_next.p}, s); return; }
     const int d = c->d, Mpad = c->Mpad;
     const float eps = c->cfg.rms_norm_eps;
+    // a folded glue leaves the new residual stream in the other buffer: begun so that the last one is c->h
+    const bool f_gu = fold_gate_up(c), f_qkv = fold_qkv(c);
+    bf16_t *hcur = c->h.p, *hoth = c->h2.p;
+    if (((f_gu ? c->L : 0) + (f_qkv ? c->L - 1 : 0)) & 1) std::swap(hcur, hoth);
     launch_embed_rmsnorm(table ? table : c->emb.p, ids ? ids : c->ids.p, c->active.p, c->pos_cur.p, c->pos_next.p, c->norms.p,
-                         c->h.p, c->x.p, d, table ? table_rows : c->V, eps, c->batch, Mpad, s);
+                         hcur, c->x.p, d, table ? table_rows : c->V, eps, c->batch, Mpad, s);
     for (int li = 0; li < c->L; ++li) {
         const size_t lkv = (size_t)c->batch * c->Hkv * c->Smax * c->D;
-        gemm_qkv(c, li, s);
+        if (f_qkv && li > 0) {
+            launch_gemm_glue(EPI_PARTIAL, c->batch, c->wqkv.p + layer_qkv_elems(c) * li, c->part.p, c->S_down, hcur, hoth, c->norms.p + (size_t)(2 * li) * d, eps, c->qkv_part.p,
+                             c->Nqkv / 16, d / 32, c->S_qkv, c->Nqkv, Mpad, s);
+            std::swap(hcur, hoth);
+        } else gemm_qkv(c, li, s);
         AttnParams ap{};
         ap.qkv_part = c->qkv_part.p; ap.S = c->S_qkv; ap.Mpad = Mpad; ap.Nqkv = c->Nqkv;
         ap.kcache = c->kcache.p + lkv * li; ap.vtcache = c->vtcache.p + lkv * li;
@@ -746,11 +762,18 @@ static void enqueue_layers(mis_tts* c, const bf16_t* table = nullptr, int table_
         ap.rope_in_dtype = c->cfg.rope_ops_in_dtype;
         launch_attn_decode(ap, c->batch, s);
         gemm_o(c, li, s);
-        launch_reduce_residual_rmsnorm(c->part.p, c->S_o, Mpad, d, c->h.p, c->norms.p + (size_t)(2 * li + 1) * d, c->x.p, eps, s);
-        gemm_gate_up(c, li, s);
+        if (f_gu) {
+            launch_gemm_glue(EPI_SILU_MUL, c->batch, c->wgu.p + layer_gu_elems(c) * li, c->part.p, c->S_o, hcur, hoth, c->norms.p + (size_t)(2 * li + 1) * d, eps, c->act.p,
+                             2 * c->ff / 16, d / 32, 1, c->ff, Mpad, s);
+            std::swap(hcur, hoth);
+        } else {
+            launch_reduce_residual_rmsnorm(c->part.p, c->S_o, Mpad, d, hcur, c->norms.p + (size_t)(2 * li + 1) * d, c->x.p, eps, s);
+            gemm_gate_up(c, li, s);
+        }
         gemm_down(c, li, s);
+        if (f_qkv && li + 1 < c->L) continue;
         const bf16_t* next_norm = c->norms.p + (size_t)(li + 1 < c->L ? 2 * (li + 1) : 2 * c->L) * d;
-        launch_reduce_residual_rmsnorm(c->part.p, c->S_down, Mpad, d, c->h.p, next_norm, c->x.p, eps, s);
+        launch_reduce_residual_rmsnorm(c->part.p, c->S_down, Mpad, d, hcur, next_norm, c->x.p, eps, s);
     }
 }
 static void enqueue_lm_head(mis_tts* c, const bf16_t* head = nullptr) {
@@ -1430,13 +1453,13 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         uint64_t key = 1469598103934665603ull;
         auto mix = [&](const void* p, size_t n) { const unsigned char* q = (const unsigned char*)p; for (size_t i = 0; i < n; ++i) { key ^= q[i]; key *= 1099511628211ull; } };
         mix(&sp, sizeof(sp));
-        const void* ptrs[] = {c->prompt_mat.p, c->prompt_lens.p, c->step_counter.p, c->ids.p, c->active.p, c->h.p, c->x.p,
+        const void* ptrs[] = {c->prompt_mat.p, c->prompt_lens.p, c->step_counter.p, c->ids.p, c->active.p, c->h.p, c->h2.p, c->x.p,
                               c->attn_out.p, c->act.p, c->logits.p, c->qkv_part.p, c->part.p, c->kcache.p, c->vtcache.p,
                               c->rope_cos.p, c->rope_sin.p, c->pos_cur.p, c->pos_next.p};
         mix(ptrs, sizeof(ptrs));
         int ints[] = {batch, Lmax, max_tokens, c->Mpad, c->Smax, c->S_qkv, c->S_o, c->S_down, hidden_mode ? 1 : 0,
                       c->a_qkv.R, c->a_qkv.ksb, c->a_qkv.U, c->a_o.R, c->a_o.ksb, c->a_o.U, c->a_down.R, c->a_down.ksb, c->a_down.U,
-                      c->a_head.R, c->a_head.ksb, c->a_head.U, c->r_gu, c->ksb_gu, c->qa_gu.R, c->qa_gu.ksb, c->qa_head.R, c->qa_head.ksb};
+                      c->a_head.R, c->a_head.ksb, c->a_head.U, c->r_gu, c->ksb_gu, c->qa_gu.R, c->qa_gu.ksb, c->qa_head.R, c->qa_head.ksb, fold_gate_up(c), fold_qkv(c)};
         mix(ints, sizeof(ints));
         const void* hp[] = {collect_hidden ? (const void*)hm->hidden->p : nullptr, collect_hidden ? (const void*)hid_count.p : nullptr};
         mix(hp, sizeof(hp));

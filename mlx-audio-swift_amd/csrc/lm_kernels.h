@@ -97,6 +97,9 @@ int gemm_choose_split(int items, int KT, int ksb, int s_max);
 
 struct AttnParams;
 bool attn_qp_ok(const AttnParams& p);
+bool gemm_glue_ok(int epi, int rows, int R, int ksb, int U, int S_in, int d, int Mpad);
+void launch_gemm_glue(int epi, int rows, const bf16_t* Wp, const float* slabs, int S_in, const bf16_t* h_in, bf16_t* h_out, const bf16_t* wnorm, float eps, void* out, int NT,
+                      int KT, int S, int N_out, int Mpad, hipStream_t s);
 size_t attn_cross_part_floats(int rows, int H);
 struct AttnParams {
     const float* qkv_part;   // [S][Mpad][Nqkv]

@@ -1154,6 +1154,182 @@ void launch_gemm_skinny_norm(int epi, int R, const bf16_t* Wp, const float* slab
     throw MisError(MIS_ERR_GENERATION_FAILED, "unsupported norm-in-prologue GEMM variant");
 }
 
+// ---------------------------------------------------------------------------- the glue inside the weight-streaming GEMM behind it (one or two rows)
+//
+// k_glue_cpt is one dependent round trip on Mpad blocks of a 256-CU chip: 4.0 us (two slabs) and 4.6 us (eight) of a 57 us layer at one row.  For
+// one or two rows every block of the consumer can afford to rebuild the rows itself (36 - 110 KB a row out of L2): it requests the slabs, the
+// residual and the norm weights FIRST and its first 2 U k-tiles of weights behind them, so that the weight stream runs while the row is summed
+// and normalised; x goes to LDS, from where every wave takes its fragments.  What bounds it is what bounded k_gemm_skinny, the weights.
+// The arithmetic is k_glue_cpt's to the last bit - thread t of its 256 is lane t & 63 of a "virtual" wave t >> 6, of which a wave plays 4 / KSB - and
+// the products are k_gemm_skinny<1, R, EPI, KSB, U>'s: a row has the bits that it has in a large batch.  Block 0 writes the new residual
+// stream to the OTHER buffer (the other blocks still read the old one).
+// Measured (Orpheus-3B, one row): gate | up 17.9 and its glue 4.0 -> 18.1 us, q|k|v 7.6 and 4.6 -> 9.7; a generate of 70 steps 127.3 -> 117.8 ms; two rows (gate | up
+// only) 105.4 -> 102.1 for 56 steps.
+template <int NR, int R, int EPI, int KSB, int U, int SG, int CPT>
+__global__ void __launch_bounds__(KSB * 64, 1) k_gemm_glue(const bf16_t* Wp, const float* slabs, int S_in, const bf16_t* h_in, bf16_t* h_out, const bf16_t* wnorm, float eps,
+                                                           void* out, int NT, int KT, int S, int N_out, int Mpad) {
+    constexpr int N = 4 * CPT * 256, VW = 4 / KSB;               // columns of a row; virtual waves a wave plays
+    __shared__ __attribute__((aligned(16))) bf16_t xs[NR][N];
+    __shared__ float rsum[NR][4];
+    __shared__ float4 red[KSB][R][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ntg = blockIdx.x / S, ks = blockIdx.x - ntg * S;
+    int kt0 = (int)(((long long)KT * ks) / S), kt1 = (int)(((long long)KT * (ks + 1)) / S);
+    {                                                            // this wave's part of the item's K range (as k_gemm_skinny)
+        const int len = kt1 - kt0;
+        const int a = kt0 + (int)(((long long)len * wave) / KSB), b = kt0 + (int)(((long long)len * (wave + 1)) / KSB);
+        kt0 = a; kt1 = b;
+    }
+    // ---- the glue's loads, all of them, then the first two groups of weights
+    uint2 hq[NR][VW][CPT], wq[VW][CPT];
+    f32x4_t v[NR][VW][CPT][SG];
+#pragma unroll
+    for (int i = 0; i < VW; ++i)
+#pragma unroll
+        for (int g = 0; g < CPT; ++g) {
+            const int c = 4 * ((wave * VW + i) * 64 + lane + g * 256);
+            wq[i][g] = *reinterpret_cast<const uint2*>(wnorm + c);
+#pragma unroll
+            for (int m = 0; m < NR; ++m) {
+                hq[m][i][g] = *reinterpret_cast<const uint2*>(h_in + (size_t)m * N + c);
+#pragma unroll
+                for (int j = 0; j < SG; ++j) v[m][i][g][j] = *reinterpret_cast<const f32x4_t*>(slabs + ((size_t)(j < S_in ? j : S_in - 1) * Mpad + m) * N + c);
+            }
+        }
+    const bf16x8_t* wp[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) wp[r] = reinterpret_cast<const bf16x8_t*>(Wp) + (size_t)min(ntg * R + r, NT - 1) * KT * 64 + lane;
+    bf16x8_t wA[U][R], wB[U][R];
+    const int klast = kt1 - 1;
+#define GG_LOAD(BUF, KBASE)                                                                                                          \
+    _Pragma("unroll") for (int u = 0; u < U; ++u) {                                                                                  \
+        const int kk = min((KBASE) + u, klast);                                                                                     \
+        _Pragma("unroll") for (int r = 0; r < R; ++r) BUF[u][r] = __builtin_nontemporal_load(wp[r] + (size_t)kk * 64);               \
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    GG_LOAD(wA, kt0)
+    GG_LOAD(wB, kt0 + U)
+    __builtin_amdgcn_sched_barrier(0);
+    // ---- residual, RMSNorm
+    float hn[NR][VW][CPT][4];
+#pragma unroll
+    for (int m = 0; m < NR; ++m)
+#pragma unroll
+        for (int i = 0; i < VW; ++i) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int g = 0; g < CPT; ++g) {
+                float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < SG; ++j) {                   // slab order 0, 1, 2, ... (fixed => deterministic)
+                    const bool on = j < S_in;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[e] += on ? v[m][i][g][j][e] : 0.0f;
+                }
+                const uint2 q = hq[m][i][g];
+                const float hv[4] = {__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xffff0000u), __uint_as_float(q.y << 16), __uint_as_float(q.y & 0xffff0000u)};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hn[m][i][g][e] = bf16_round_f32(hv[e] + bf16_round_f32(acc[e]));             // o = T(sum slabs); h = T(h + o)
+                    ss += hn[m][i][g][e] * hn[m][i][g][e];
+                }
+            }
+            ss = wave_sum_dpp(ss);
+            if (lane == 0) rsum[m][wave * VW + i] = ss;
+        }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (raw: __syncthreads() would wait for the weights as well)
+#pragma unroll
+    for (int m = 0; m < NR; ++m) {
+        float tot = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) tot += rsum[m][w];
+        const float inv = 1.0f / sqrtf(tot / (float)N + eps);
+#pragma unroll
+        for (int i = 0; i < VW; ++i)
+#pragma unroll
+            for (int g = 0; g < CPT; ++g) {
+                const int c = 4 * ((wave * VW + i) * 64 + lane + g * 256);
+                const uint2 q = wq[i][g];
+                const float wv[4] = {__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xffff0000u), __uint_as_float(q.y << 16), __uint_as_float(q.y & 0xffff0000u)};
+                bf16_t xb[4], hb[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hb[e] = f32_to_bf16(hn[m][i][g][e]);
+                    xb[e] = f32_to_bf16(wv[e] * bf16_round_f32(hn[m][i][g][e] * inv));
+                }
+                *reinterpret_cast<uint2*>(&xs[m][c]) = make_uint2((uint32_t)xb[0] | ((uint32_t)xb[1] << 16), (uint32_t)xb[2] | ((uint32_t)xb[3] << 16));
+                if (blockIdx.x == 0)
+                    *reinterpret_cast<uint2*>(h_out + (size_t)m * N + c) = make_uint2((uint32_t)hb[0] | ((uint32_t)hb[1] << 16), (uint32_t)hb[2] | ((uint32_t)hb[3] << 16));
+            }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // ---- the products: rows past NR multiply zero
+    const int m = lane & 15;
+    const bf16_t* xrow = &xs[m < NR ? m : 0][(lane >> 4) * 8];
+    f32x4_t acc[R][1];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r][0] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#define GG_MATH(BUF, KBASE, GUARD)                                                                                                   \
+    _Pragma("unroll") for (int u = 0; u < U; ++u) {                                                                                  \
+        if (!(GUARD) || (KBASE) + u < kt1) {                                                                                         \
+            bf16x8_t xf = *reinterpret_cast<const bf16x8_t*>(xrow + ((KBASE) + u) * 32);                                             \
+            if (m >= NR) xf = (bf16x8_t){0, 0, 0, 0, 0, 0, 0, 0};                                                                    \
+            _Pragma("unroll") for (int r = 0; r < R; ++r) acc[r][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(BUF[u][r], xf, acc[r][0], 0, 0, 0);  \
+        }                                                                                                                            \
+    }
+    int kt = kt0;
+    while (kt + 4 * U <= kt1) {                                  // groups kt and kt + U are here or on their way, the two behind them exist
+        GG_MATH(wA, kt, false)
+        __builtin_amdgcn_sched_barrier(0);
+        GG_LOAD(wA, kt + 2 * U)
+        __builtin_amdgcn_sched_barrier(0);
+        GG_MATH(wB, kt + U, false)
+        __builtin_amdgcn_sched_barrier(0);
+        GG_LOAD(wB, kt + 3 * U)
+        __builtin_amdgcn_sched_barrier(0);
+        kt += 2 * U;
+    }
+    GG_MATH(wA, kt, true)                                        // up to four (partial) groups left, the first two of them requested
+    if (kt + 2 * U < kt1) { GG_LOAD(wA, kt + 2 * U) }
+    GG_MATH(wB, kt + U, true)
+    if (kt + 2 * U < kt1) {
+        if (kt + 3 * U < kt1) { GG_LOAD(wB, kt + 3 * U) }
+        GG_MATH(wA, kt + 2 * U, true)
+        GG_MATH(wB, kt + 3 * U, true)
+    }
+#undef GG_LOAD
+#undef GG_MATH
+#pragma unroll
+    for (int r = 0; r < R; ++r) red[wave][r][lane] = make_float4(acc[r][0][0], acc[r][0][1], acc[r][0][2], acc[r][0][3]);
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        float4 s0 = red[0][r][lane];
+#pragma unroll
+        for (int w = 1; w < KSB; ++w) {
+            const float4 t = red[w][r][lane];
+            s0.x += t.x; s0.y += t.y; s0.z += t.z; s0.w += t.w;
+        }
+        acc[r][0] = (f32x4_t){s0.x, s0.y, s0.z, s0.w};
+    }
+    gemm_epilogue<1, R, EPI>(acc, out, ntg, ks, NT, N_out, Mpad, lane, -1, nullptr);
+}
+// the two instances: gate | up behind the output projection's slabs (one or two rows), q|k|v behind the down projection's (one row: with two, their 200 KB a
+// block cost more than the launch).  Arrangements other than these keep the separate launches.
+bool gemm_glue_ok(int epi, int rows, int R, int ksb, int U, int S_in, int d, int Mpad) {
+    if (d != 3072 || Mpad != 16 || R != 4) return false;         // (d = 3072: the width of k_glue_cpt)
+    if (epi == EPI_SILU_MUL) return rows <= 2 && ksb == 4 && (U == 0 || U == 3) && S_in <= 2;
+    return epi == EPI_PARTIAL && rows == 1 && ksb == 2 && U == 2 && S_in <= 8;
+}
+void launch_gemm_glue(int epi, int rows, const bf16_t* Wp, const float* slabs, int S_in, const bf16_t* h_in, bf16_t* h_out, const bf16_t* wnorm, float eps, void* out, int NT,
+                      int KT, int S, int N_out, int Mpad, hipStream_t s) {
+    const dim3 grid((NT + 3) / 4 * S);
+    if (epi == EPI_PARTIAL) hipLaunchKernelGGL((k_gemm_glue<1, 4, EPI_PARTIAL, 2, 2, 8, 3>), grid, dim3(128), 0, s, Wp, slabs, S_in, h_in, h_out, wnorm, eps, out, NT, KT, S, N_out, Mpad);
+    else if (rows == 1) hipLaunchKernelGGL((k_gemm_glue<1, 4, EPI_SILU_MUL, 4, 3, 2, 3>), grid, dim3(256), 0, s, Wp, slabs, S_in, h_in, h_out, wnorm, eps, out, NT, KT, S, N_out, Mpad);
+    else hipLaunchKernelGGL((k_gemm_glue<2, 4, EPI_SILU_MUL, 4, 3, 2, 3>), grid, dim3(256), 0, s, Wp, slabs, S_in, h_in, h_out, wnorm, eps, out, NT, KT, S, N_out, Mpad);
+}
+
 // Inter-block split-K factor of a weight-streaming GEMM with `items` n-tile groups and KT k-tiles.  All blocks of a launch are
 // co-resident and share their CU's load bandwidth, so the launch takes as long as the most loaded CU needs:
 //   time ~ ceil(blocks / CUs) / blocks            (the share of the weight bytes behind the busiest CU)
