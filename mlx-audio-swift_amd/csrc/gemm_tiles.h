@@ -30,10 +30,17 @@ struct GemmTiles {
     // of its X; epi(t, acc) stores a finished tile
     template <class FW, class FX, class FE>
     static __device__ __forceinline__ void run(unsigned char* lds, const bf16_t* Wb, const bf16_t* Xb, int K, int first, int stride, int tiles, FW woff, FX xoff, FE epi) {
+        run(lds, K, first, stride, tiles, [&](int, const bf16_t*& w, const bf16_t*& x) { w = Wb; x = Xb; }, woff, xoff, epi);
+    }
+    // operands(t, W, X): the two operands of tile t
+    template <class FO, class FW, class FX, class FE>
+    static __device__ __forceinline__ void run(unsigned char* lds, int K, int first, int stride, int tiles, FO operands, FW woff, FX xoff, FE epi) {
         const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wave >> 1, wm = wave & 1;
         const int KS = K / BK;
         uint32_t off[NQ];                                            // bytes
+        const bf16_t *Wb, *Xb;
         auto point = [&](int t) {
+            operands(t, Wb, Xb);
             int ln = lane;
             asm volatile("" : "+v"(ln));                             // (computed here for each tile: hoisted, these take the registers that TM = 8 has not got)
 #pragma unroll
@@ -122,6 +129,10 @@ struct GemmTiles {
             for (int i = 0; i < NBUF; ++i) step(more ? i : KS - 1);
             bind(a[0], b[0]);
             asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");         // (the last products are in their registers before anything reads them)
+#pragma unroll
+            for (int i = 0; i < TN; ++i)
+#pragma unroll
+                for (int j = 0; j < TM; ++j) asm volatile("" : "+a"(acc[i][j]));      // (nor may a copy of an accumulator stand in front of that wait)
             epi(t, acc);
             if (!more) break;
             t += stride;

@@ -13,6 +13,7 @@
 //   k_scatter_kv    [M][*] K and V columns -> the tiled MFMA-fragment cache layouts of lm_kernels.hip
 //   k_attn_prefill  non-causal flash attention over the tiled K/V, 16 query rows per wave
 #include "common.h"
+#include "gemm_tiles.h"
 #include "whisper_kernels.h"
 #include <type_traits>
 
@@ -470,34 +471,204 @@ static bool launch_big3(const BigGemmParams& p, hipStream_t s) {
     return (p.N >= 4096 || p.K >= 4096) ? launch_big3_one<EPI, 2, 4>(p, s) : launch_big3_one<EPI, 4, 2>(p, s);
 }
 
+// ---------------------------------------------------------------------------- tiles of 32 TM x 256 outputs, four waves (gemm_tiles.h)
+// What it gives over k_gemm_big3 (large-v3, us per launch): 8 x 1500 rows q|k|v 122 / 140, o 55 / 60, fc1 204 / 211, fc2 146 / 172, cross k|v 88 / 101; 6 x 1500
+// (k_gemm_big2 where 180 tiles of 256 x 256 were too few) 100 / 128, 44 / 58, 155 / 159, 122 / 173, 66 / 90; 4 x 1500 71 / 89, 33 / 34, 107 / 107, 85 / 95, 45 / 50.
+// k_gemm_big3 keeps what these offsets or rings cannot hold and GELUs of 200 - 255 tiles.
+// TM by the rounds of 256 persistent blocks it makes (launch_gemm_rows).  Products in the order of k: the bits of k_gemm_big2.
+// The tiles are numbered in bands of G row tiles, row tiles fastest, and an XCD (blocks are dealt to the XCDs by id mod 8) takes one range of them: the 32
+// blocks it runs together share G row tiles of X and 32 / G column tiles of W in its L2.
+struct TileOrder {
+    int mt, nt;
+    template <int G> __device__ __forceinline__ void at(int t, int& mi, int& ni) const {
+        const int band = t / (G * nt), left = t - band * G * nt, rows = min(G, mt - band * G);
+        ni = left / rows;
+        mi = band * G + left - ni * rows;
+    }
+};
+template <int EPI, int TM>
+__device__ __forceinline__ void gemm_rows_body(const BigGemmParams& p) {
+    using T = GemmTiles<TM, false>;
+    constexpr int G = TM >= 6 ? 6 : 8;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
+    // Value tiles of BG_KV swap the operands: a lane then holds four consecutive KEYS of one dim, which are one 8-byte piece of the value image (two bytes each
+    // the other way round).  They are numbered behind the others, 256 keys x 32 TM dims each; the products and their order are the same.
+    const int N0 = EPI == BG_KV ? p.vcol0 : p.N;
+    const TileOrder o0{(p.M + T::BM - 1) / T::BM, (N0 + T::BN - 1) / T::BN}, o1{(p.M + T::BN - 1) / T::BN, EPI == BG_KV ? (p.N - N0 + T::BM - 1) / T::BM : 0};
+    const int tiles0 = o0.mt * o0.nt, tiles = tiles0 + o1.mt * o1.nt;
+    const int xcd = blockIdx.x & 7, lo = (int)((int64_t)tiles * xcd / 8), hi = (int)((int64_t)tiles * (xcd + 1) / 8), first = lo + (blockIdx.x >> 3);
+    if (first >= hi) return;
+    auto where = [&](int t, bool& swp, int& m0, int& n0) {
+        int mi, ni;
+        swp = EPI == BG_KV && t >= tiles0;
+        if (swp) { o1.template at<G>(t - tiles0, mi, ni); m0 = mi * T::BN; n0 = N0 + ni * T::BM; }
+        else { o0.template at<G>(t, mi, ni); m0 = mi * T::BM; n0 = ni * T::BN; }
+    };
+    bool sw; int mt0, nt0;                                   // of the tile being requested
+    T::run(lds, p.K, first, gridDim.x >> 3, hi,
+           [&](int t, const bf16_t*& Wb, const bf16_t*& Xb) {
+               where(t, sw, mt0, nt0);
+               Wb = sw ? p.X : p.W;
+               Xb = sw ? p.W : p.X;
+           },
+           [&](int, int q, int lane) {
+               const int r = q * 8 + (lane >> 3);
+               return (sw ? (uint32_t)min(mt0 + r, p.M - 1) * p.ldx : (uint32_t)min(nt0 + r, N0 - 1) * p.K) + ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+           },
+           [&](int, int r) { return sw ? (uint32_t)min(nt0 + r, p.N - 1) * p.K : (uint32_t)min(mt0 + r, p.M - 1) * p.ldx; },
+           [&](int t, const f32x4_t (&acc)[T::TN][TM]) {
+               bool swp; int m0, n0;
+               where(t, swp, m0, n0);
+               int lane = threadIdx.x & 63;
+               asm volatile("" : "+v"(lane));
+               const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = (wave >> 1) * 128 + (lane >> 4) * 4, xr = (wave & 1) * TM * 16 + (lane & 15);
+               auto pack4 = [](float a, float b, float c, float d) {
+                   return make_uint2((uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16), (uint32_t)f32_to_bf16(c) | ((uint32_t)f32_to_bf16(d) << 16));
+               };
+               auto part = [](const uint2& b, int e) { return __uint_as_float(e & 1 ? (e < 2 ? b.x : b.y) & 0xffff0000u : (e < 2 ? b.x : b.y) << 16); };
+               uint2 bv[T::TN];
+#pragma unroll
+               for (int i = 0; i < T::TN; ++i) bv[i] = p.bias ? *reinterpret_cast<const uint2*>(p.bias + min(n0 + wr + i * 16, N0 - 4)) : make_uint2(0, 0);
+               if constexpr (EPI == BG_KV) {
+                   // an output's byte offset is the sum of one of its W row and one of its X row, in C, in the key image [2][D/32][64 lanes][8] (the key permutation
+                   // of k_scatter_kv) and in the value image [D/16][64 lanes][8] (lane (key / 8) 16 + d & 15, key & 7); one loop for the three
+                   const bool key = !swp && n0 >= p.kcol0;
+                   unsigned char* const base = reinterpret_cast<unsigned char*>(swp ? p.vc : key ? p.kc : p.C);
+                   auto of_key = [&](int m) {                // (M and T are multiples of 4: four keys share a batch row and a piece)
+                       const uint32_t br = (uint32_t)m / (uint32_t)p.T, tk = m - br * p.T, pr = tk & 31;
+                       return br * p.H * p.Spad * 128u + (tk & ~31u) * 128u + (swp ? (pr >> 3) * 256 + (pr & 7) * 2 : ((pr >> 2) & 1) * 2048 + (((pr >> 3) << 2) | (pr & 3)) * 16);
+                   };
+                   auto of_dim = [&](int dd) {
+                       const uint32_t d = dd & 63;
+                       return (uint32_t)(dd >> 6) * p.Spad * 128u + (swp ? (d >> 4) * 1024 + (d & 15) * 16 : ((d >> 5) * 512 + ((d & 31) >> 3) * 128 + (d & 7)) * 2);
+                   };
+                   uint32_t at[T::TN];
+                   bool ok[T::TN];
+#pragma unroll
+                   for (int i = 0; i < T::TN; ++i) {
+                       ok[i] = !swp || m0 + wr + i * 16 < p.M;
+                       at[i] = swp ? of_key(m0 + wr + i * 16) : key ? of_dim(n0 - p.kcol0 + wr + i * 16) : (uint32_t)(n0 + wr + i * 16) * 2;
+                       if (swp) bv[i] = make_uint2(0, 0);
+                   }
+#pragma unroll
+                   for (int j = 0; j < TM; ++j) {
+                       __builtin_amdgcn_sched_barrier(0);
+                       const int x = (swp ? n0 : m0) + xr + j * 16, xn = swp ? min(x, p.N - 1) : 0;
+                       const float b = swp && p.bias ? bf16_to_f32(p.bias[xn]) : 0.0f;
+                       const bool okx = x < (swp ? p.N : p.M);
+                       const uint32_t to = swp ? of_dim(xn - N0) : key ? of_key(x) : (uint32_t)x * p.N * 2u;
+#pragma unroll
+                       for (int i = 0; i < T::TN; ++i) {
+                           float v[4];
+#pragma unroll
+                           for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + part(bv[i], e) + b;
+                           const uint2 o = pack4(v[0], v[1], v[2], v[3]);
+                           if (okx & ok[i]) *reinterpret_cast<uint2*>(base + at[i] + to) = o;
+                       }
+                   }
+                   return;
+               }
+               // residual or positional values are requested eight outputs ahead; an output is packed before the branch of its store (a load consumed inside it
+               // waits for every store before it)
+               constexpr bool RES = EPI == BG_RESID || EPI == BG_GELU_POS;
+               uint2 r[T::TN];
+               auto residual = [&](int j, int i) {
+                   const int m = min(m0 + xr + j * 16, p.M - 1);
+                   r[i] = *reinterpret_cast<const uint2*>(reinterpret_cast<const unsigned char*>(p.R) + (uint32_t)(EPI == BG_RESID ? m : m % p.pos_rows) * p.N * 2u + min(n0 + wr + i * 16, p.N - 4) * 2);
+               };
+               if constexpr (RES) {
+#pragma unroll
+                   for (int i = 0; i < T::TN; ++i) residual(0, i);
+               }
+#pragma unroll
+               for (int j = 0; j < TM; ++j) {
+                   __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                   for (int i = 0; i < T::TN; ++i) {
+                       float v[4];
+#pragma unroll
+                       for (int e = 0; e < 4; ++e) {
+                           v[e] = bf16_round_f32(acc[i][j][e] + part(bv[i], e));        // T(xW^T + b)
+                           if (EPI == BG_GELU || EPI == BG_GELU_POS) v[e] = bf16_round_f32(gelu_erf_w(v[e]));
+                           if (RES) v[e] += part(r[i], e);
+                       }
+                       uint2 o = pack4(v[0], v[1], v[2], v[3]);
+                       asm volatile("" : "+v"(o.x), "+v"(o.y));
+                       if constexpr (RES) {
+                           if (j + 1 < TM) residual(j + 1, i);
+                       }
+                       const int m = m0 + xr + j * 16;
+                       if (m < p.M && n0 + wr + i * 16 < N0) *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(p.C) + (uint32_t)m * p.N * 2u + (n0 + wr + i * 16) * 2) = o;
+                   }
+               }
+           });
+}
+template <int EPI, int TM>
+__global__ void __launch_bounds__(256, 1) k_gemm_rows(BigGemmParams p) { gemm_rows_body<EPI, TM>(p); }
+template <int TM>
+__global__ void __launch_bounds__(256, 1) k_gemm_rows_kv(BigGemmParams p) { gemm_rows_body<BG_KV, TM>(p); }
+template <int EPI>
+static bool launch_gemm_rows(const BigGemmParams& p, hipStream_t s) {
+    // (32-bit byte offsets; three k-steps at least fill the ring)
+    if (p.K % BG2_BK || p.K < 3 * BG2_BK || (int64_t)p.N * p.K >= (1ll << 31) || (int64_t)p.M * p.ldx >= (1ll << 31)) return false;
+    if ((int64_t)p.M * p.N >= (1ll << 31) || (EPI == BG_KV && (int64_t)(p.M / p.T) * p.H * p.Spad * 128 >= (1ll << 32))) return false;
+    const int N0 = EPI == BG_KV ? p.vcol0 : p.N;
+    auto count = [&](int tm) { return cdiv(p.M, 32 * tm) * cdiv(N0, 256) + (EPI == BG_KV ? cdiv(p.M, 256) * cdiv(p.N - N0, 32 * tm) : 0); };
+    int best = 0;
+    double least = 0;
+    for (int tm : {8, 6, 5, 4}) {                                  // rounds of 256 blocks, each as long as its tiles are high and a little
+        const double cost = cdiv(count(tm), 256) * (tm + 0.4);
+        if (!best || cost < least) { best = tm; least = cost; }
+    }
+    // fewer tiles leave compute units idle that more blocks of the smaller kernels fill (one window: o 23.9 us there); a GELU has no other block's products
+    // beside it here (240 tiles: 31 and 57 us against 30 and 56)
+    if (count(best) < (EPI == BG_GELU ? 256 : 200)) return false;
+    auto go = [&](auto tag) {
+        constexpr int TM = decltype(tag)::value;
+        void (*kernel)(BigGemmParams);
+        if constexpr (EPI == BG_KV) kernel = k_gemm_rows_kv<TM>;
+        else kernel = k_gemm_rows<EPI, TM>;
+        hipLaunchKernelGGL(kernel, dim3(std::min((int)round_up(count(TM), 8), 256)), dim3(256), 0, s, p);
+    };
+    if (best == 8) go(std::integral_constant<int, 8>{});
+    else if (best == 6) go(std::integral_constant<int, 6>{});
+    else if (best == 5) go(std::integral_constant<int, 5>{});
+    else go(std::integral_constant<int, 4>{});
+    return true;
+}
+
 bool launch_gemm_big_kv(const BigGemmParams& p, hipStream_t s) {
     const char* e3 = getenv("MIS_GEMM_BIG3");
     const int mode = e3 ? atoi(e3) : 1;
     // key and value columns start at tile boundaries; pieces of four keys stay inside a batch row
-    if (mode == 0 || p.K % BG2_BK != 0 || p.K < 2 * BG2_BK || (mode != 2 && (long)cdiv(p.N, BG3_BN) * cdiv(p.M, BG3_BM) < 200)) return false;
-    if (p.ldx % 8 || p.kcol0 % BG3_BN || p.vcol0 % BG3_BN || p.N % BG3_BN || p.T % 4 || p.M % 4 || p.Spad % 32) return false;
+    if (mode == 0 || p.ldx % 8 || p.kcol0 % BG3_BN || p.vcol0 % BG3_BN || p.N % BG3_BN || p.T % 4 || p.M % 4 || p.Spad % 32) return false;
+    if (mode == 1 && launch_gemm_rows<BG_KV>(p, s)) return true;
+    if (p.K % BG2_BK != 0 || p.K < 2 * BG2_BK || (mode != 2 && (long)cdiv(p.N, BG3_BN) * cdiv(p.M, BG3_BM) < 200)) return false;
     return launch_big3<BG_KV>(p, s);
 }
 
 void launch_gemm_big(int epi, const BigGemmParams& p, hipStream_t s) {
     MIS_REQUIRE(p.K % BG_BK == 0 && p.ldx % 8 == 0 && p.N % 4 == 0, MIS_ERR_INVALID_INPUT, "big GEMM needs K %% 32 == 0");
     dim3 grid(cdiv(p.N, BG_BN), cdiv(p.M, BG_BM)), block(256);
-    {   // the 256 x 256 tile where its grid still fills most of the chip (out_proj of 8 windows: 235 blocks, 52.0 -> 44.6 us); below that the
-        // 128 x 128 kernel has four times the blocks.  MIS_GEMM_BIG3=0: never (A/B); =2: whenever the shape allows (parity tests)
+    {   // large tiles where their grid still fills most of the chip; below that the 128 x 128 kernel has four times the blocks.
+        // MIS_GEMM_BIG3=0: never (A/B); =2: the eight-wave kernel whenever the shape allows (parity tests)
         const char* e3 = getenv("MIS_GEMM_BIG3");
         const int mode = e3 ? atoi(e3) : 1;
         const long blocks3 = (long)cdiv(p.N, BG3_BN) * cdiv(p.M, BG3_BM);
-        if (mode != 0 && p.K % BG2_BK == 0 && p.K >= 2 * BG2_BK && (mode == 2 || blocks3 >= 200)) {
-            bool done = false;
-            switch (epi) {
-                case BG_NONE: done = launch_big3<BG_NONE>(p, s); break;
-                case BG_GELU: done = launch_big3<BG_GELU>(p, s); break;
-                case BG_RESID: done = launch_big3<BG_RESID>(p, s); break;
-                case BG_GELU_POS: done = launch_big3<BG_GELU_POS>(p, s); break;
-                default: throw MisError(MIS_ERR_GENERATION_FAILED, "unknown big GEMM epilogue");
-            }
-            if (done) return;
+        const bool big3 = p.K % BG2_BK == 0 && p.K >= 2 * BG2_BK && (mode == 2 || blocks3 >= 200);
+        auto large = [&](auto tag) {
+            constexpr int E = decltype(tag)::value;
+            return (mode == 1 && launch_gemm_rows<E>(p, s)) || (mode != 0 && big3 && launch_big3<E>(p, s));
+        };
+        bool done = false;
+        switch (epi) {
+            case BG_NONE: done = large(std::integral_constant<int, BG_NONE>{}); break;
+            case BG_GELU: done = large(std::integral_constant<int, BG_GELU>{}); break;
+            case BG_RESID: done = large(std::integral_constant<int, BG_RESID>{}); break;
+            case BG_GELU_POS: done = large(std::integral_constant<int, BG_GELU_POS>{}); break;
+            default: throw MisError(MIS_ERR_GENERATION_FAILED, "unknown big GEMM epilogue");
         }
+        if (done) return;
     }
     if (p.K % BG2_BK == 0 && p.K >= 2 * BG2_BK) {
         switch (epi) {

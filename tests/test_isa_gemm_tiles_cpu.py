@@ -7,7 +7,7 @@ import pytest
 from test_isa_cpu import _compiled, _registers, pytestmark  # noqa: F401
 
 
-@pytest.mark.parametrize("src, pattern", [("lm_prefill.hip", "k_gemm_pf_wide")])
+@pytest.mark.parametrize("src, pattern", [("lm_prefill.hip", "k_gemm_pf_wide"), ("whisper_kernels.hip", "k_gemm_rows")])
 def test_no_fragment_in_flight_is_touched(src, pattern):
     text, use = _compiled(src)
     names = re.findall(r"\n(_Z\w*%s\w*):" % pattern, text)
