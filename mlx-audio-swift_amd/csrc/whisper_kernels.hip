@@ -29,7 +29,7 @@ __device__ __forceinline__ float rcp_nearest(float d) {
     const float t = __builtin_amdgcn_rcpf(d);
     return fmaf(fmaf(-d, t, 1.0f), t, t);
 }
-__device__ __forceinline__ float gelu_erf_w(float x) {
+__device__ __forceinline__ float gelu_erfc_w(float x) {                   // erfc(|x| / sqrt 2)
     const float z = fminf(fabsf(x) * 0.70710678118654752f, 16.0f);      // (exp(-z^2) is 0 from 10.2 on)
     const float t = rcp_nearest(1.0f + 0.3275911f * z);
     float p = 1.061405429f;
@@ -37,7 +37,10 @@ __device__ __forceinline__ float gelu_erf_w(float x) {
     p = p * t + 1.421413741f;
     p = p * t - 0.284496736f;
     p = p * t + 0.254829592f;
-    const float ec = p * t * __expf(-(z * z));            // erfc(|x| / sqrt 2)
+    return p * t * __expf(-(z * z));
+}
+__device__ __forceinline__ float gelu_erf_w(float x) {
+    const float ec = gelu_erfc_w(x);
     return 0.5f * x * (x >= 0.0f ? 2.0f - ec : ec);
 }
 
@@ -472,12 +475,49 @@ static bool launch_big3(const BigGemmParams& p, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------------------- tiles of 32 TM x 256 outputs, four waves (gemm_tiles.h)
-// What it gives over k_gemm_big3 (large-v3, us per launch): 8 x 1500 rows q|k|v 122 / 140, o 55 / 60, fc1 204 / 211, fc2 146 / 172, cross k|v 88 / 101; 6 x 1500
-// (k_gemm_big2 where 180 tiles of 256 x 256 were too few) 100 / 128, 44 / 58, 155 / 159, 122 / 173, 66 / 90; 4 x 1500 71 / 89, 33 / 34, 107 / 107, 85 / 95, 45 / 50.
-// k_gemm_big3 keeps what these offsets or rings cannot hold and GELUs of 200 - 255 tiles.
+// What it gives over k_gemm_big3 (large-v3, us per launch): 8 x 1500 rows q|k|v 122 / 140, o 55 / 60, fc1 171 / 211, fc2 146 / 172, cross k|v 88 / 101; 6 x 1500
+// (k_gemm_big2 where 180 tiles of 256 x 256 were too few) 100 / 128, 44 / 58, 128 / 159, 122 / 173, 66 / 90; 4 x 1500 71 / 89, 33 / 34, 93 / 107, 85 / 95, 45 / 50.
+// k_gemm_big3 keeps what these offsets or rings cannot hold.
 // TM by the rounds of 256 persistent blocks it makes (launch_gemm_rows).  Products in the order of k: the bits of k_gemm_big2.
 // The tiles are numbered in bands of G row tiles, row tiles fastest, and an XCD (blocks are dealt to the XCDs by id mod 8) takes one range of them: the 32
 // blocks it runs together share G row tiles of X and 32 / G column tiles of W in its L2.
+// A GELU after T(xW^T + b) is a function of sixteen bits: gelu_erf_w(v) = v f(v), f in an LDS table over |v| = 2^-10 .. 16 and the sign (14 KB; below 2^-10 the
+// result is v / 2, above 16 it is v or -0: the values that the clamped factors round to).  The same bits as the formula, in 12 instructions an
+// output and an LDS read for 31, two of them of quarter rate - a block's only waves wait for them.  fc1, eight windows 204 -> 171 us, one 31 -> 28.
+struct GeluTable {
+    static constexpr uint32_t LO = 0x3a80, HI = 0x4180, N = HI - LO + 1;           // bf16 of 2^-10 and 16
+    static __device__ __forceinline__ void fill(float* tab) {                      // (ends with a barrier)
+        for (uint32_t i = threadIdx.x; i < N; i += 256) {
+            const float z = __uint_as_float((LO + i) << 16), ec = gelu_erfc_w(z);
+            tab[i] = 0.5f * (2.0f - ec);
+            tab[N + i] = 0.5f * ec;
+        }
+        __syncthreads();
+    }
+    // x[e] = gelu(x[e]) before its rounding; x of 16 bits.  base: LDS offset of the table
+    static __device__ __forceinline__ void apply(uint32_t base, float (&x)[16]) {
+        uint32_t a[16];
+        float f[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const float y = __builtin_amdgcn_fmed3f(fabsf(x[e]), __uint_as_float(LO << 16), __uint_as_float(HI << 16));
+            a[e] = (__float_as_uint(y) >> 14) + ((uint32_t)((int)__float_as_uint(x[e]) >> 31) & (4 * N)) + (base - 4 * LO);
+        }
+        // (reads and their wait in one block: behind an LDS-DMA the compiler would wait for every load and store in flight)
+        asm volatile("ds_read_b32 %0, %16\n\tds_read_b32 %1, %17\n\tds_read_b32 %2, %18\n\tds_read_b32 %3, %19\n\t"
+                     "ds_read_b32 %4, %20\n\tds_read_b32 %5, %21\n\tds_read_b32 %6, %22\n\tds_read_b32 %7, %23\n\t"
+                     "ds_read_b32 %8, %24\n\tds_read_b32 %9, %25\n\tds_read_b32 %10, %26\n\tds_read_b32 %11, %27\n\t"
+                     "ds_read_b32 %12, %28\n\tds_read_b32 %13, %29\n\tds_read_b32 %14, %30\n\tds_read_b32 %15, %31\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(f[0]), "=&v"(f[1]), "=&v"(f[2]), "=&v"(f[3]), "=&v"(f[4]), "=&v"(f[5]), "=&v"(f[6]), "=&v"(f[7]),
+                       "=&v"(f[8]), "=&v"(f[9]), "=&v"(f[10]), "=&v"(f[11]), "=&v"(f[12]), "=&v"(f[13]), "=&v"(f[14]), "=&v"(f[15])
+                     : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), "v"(a[4]), "v"(a[5]), "v"(a[6]), "v"(a[7]),
+                       "v"(a[8]), "v"(a[9]), "v"(a[10]), "v"(a[11]), "v"(a[12]), "v"(a[13]), "v"(a[14]), "v"(a[15])
+                     : "memory");
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[e] *= f[e];
+    }
+};
 struct TileOrder {
     int mt, nt;
     template <int G> __device__ __forceinline__ void at(int t, int& mi, int& ni) const {
@@ -490,7 +530,9 @@ template <int EPI, int TM>
 __device__ __forceinline__ void gemm_rows_body(const BigGemmParams& p) {
     using T = GemmTiles<TM, false>;
     constexpr int G = TM >= 6 ? 6 : 8;
+    constexpr bool GELU = EPI == BG_GELU || EPI == BG_GELU_POS;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
+    __shared__ float gelu_tab[GELU ? 2 * GeluTable::N : 1];
     // Value tiles of BG_KV swap the operands: a lane then holds four consecutive KEYS of one dim, which are one 8-byte piece of the value image (two bytes each
     // the other way round).  They are numbered behind the others, 256 keys x 32 TM dims each; the products and their order are the same.
     const int N0 = EPI == BG_KV ? p.vcol0 : p.N;
@@ -498,6 +540,7 @@ __device__ __forceinline__ void gemm_rows_body(const BigGemmParams& p) {
     const int tiles0 = o0.mt * o0.nt, tiles = tiles0 + o1.mt * o1.nt;
     const int xcd = blockIdx.x & 7, lo = (int)((int64_t)tiles * xcd / 8), hi = (int)((int64_t)tiles * (xcd + 1) / 8), first = lo + (blockIdx.x >> 3);
     if (first >= hi) return;
+    if constexpr (GELU) GeluTable::fill(gelu_tab);
     auto where = [&](int t, bool& swp, int& m0, int& n0) {
         int mi, ni;
         swp = EPI == BG_KV && t >= tiles0;
@@ -523,7 +566,9 @@ __device__ __forceinline__ void gemm_rows_body(const BigGemmParams& p) {
                asm volatile("" : "+v"(lane));
                const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wr = (wave >> 1) * 128 + (lane >> 4) * 4, xr = (wave & 1) * TM * 16 + (lane & 15);
                auto pack4 = [](float a, float b, float c, float d) {
-                   return make_uint2((uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16), (uint32_t)f32_to_bf16(c) | ((uint32_t)f32_to_bf16(d) << 16));
+                   typedef float f2_t __attribute__((ext_vector_type(2)));
+                   typedef __bf16 h2_t __attribute__((ext_vector_type(2)));
+                   return make_uint2(__builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){a, b}, h2_t)), __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){c, d}, h2_t)));
                };
                auto part = [](const uint2& b, int e) { return __uint_as_float(e & 1 ? (e < 2 ? b.x : b.y) & 0xffff0000u : (e < 2 ? b.x : b.y) << 16); };
                uint2 bv[T::TN];
@@ -584,21 +629,26 @@ __device__ __forceinline__ void gemm_rows_body(const BigGemmParams& p) {
                for (int j = 0; j < TM; ++j) {
                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                   for (int i = 0; i < T::TN; ++i) {
-                       float v[4];
+                   for (int ih = 0; ih < T::TN; ih += 4) {
+                       float v[16];
 #pragma unroll
-                       for (int e = 0; e < 4; ++e) {
-                           v[e] = bf16_round_f32(acc[i][j][e] + part(bv[i], e));        // T(xW^T + b)
-                           if (EPI == BG_GELU || EPI == BG_GELU_POS) v[e] = bf16_round_f32(gelu_erf_w(v[e]));
-                           if (RES) v[e] += part(r[i], e);
+                       for (int e = 0; e < 16; ++e) v[e] = bf16_round_f32(acc[ih + (e >> 2)][j][e & 3] + part(bv[ih + (e >> 2)], e & 3));        // T(xW^T + b)
+                       if constexpr (GELU) GeluTable::apply(gt_lds_offset(gelu_tab), v);
+#pragma unroll
+                       for (int i = ih; i < ih + 4; ++i) {
+                           float* w = v + (i - ih) * 4;
+                           if constexpr (RES) {
+#pragma unroll
+                               for (int e = 0; e < 4; ++e) w[e] = (GELU ? bf16_round_f32(w[e]) : w[e]) + part(r[i], e);
+                           }
+                           uint2 o = pack4(w[0], w[1], w[2], w[3]);
+                           asm volatile("" : "+v"(o.x), "+v"(o.y));
+                           if constexpr (RES) {
+                               if (j + 1 < TM) residual(j + 1, i);
+                           }
+                           const int m = m0 + xr + j * 16;
+                           if (m < p.M && n0 + wr + i * 16 < N0) *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(p.C) + (uint32_t)m * p.N * 2u + (n0 + wr + i * 16) * 2) = o;
                        }
-                       uint2 o = pack4(v[0], v[1], v[2], v[3]);
-                       asm volatile("" : "+v"(o.x), "+v"(o.y));
-                       if constexpr (RES) {
-                           if (j + 1 < TM) residual(j + 1, i);
-                       }
-                       const int m = m0 + xr + j * 16;
-                       if (m < p.M && n0 + wr + i * 16 < N0) *reinterpret_cast<uint2*>(reinterpret_cast<unsigned char*>(p.C) + (uint32_t)m * p.N * 2u + (n0 + wr + i * 16) * 2) = o;
                    }
                }
            });
@@ -618,11 +668,11 @@ static bool launch_gemm_rows(const BigGemmParams& p, hipStream_t s) {
     double least = 0;
     for (int tm : {8, 6, 5, 4}) {                                  // rounds of 256 blocks, each as long as its tiles are high and a little
         const double cost = cdiv(count(tm), 256) * (tm + 0.4);
+        if (tm == 5 && (EPI == BG_GELU || EPI == BG_GELU_POS)) continue;      // (its ring leaves no LDS for the table)
         if (!best || cost < least) { best = tm; least = cost; }
     }
-    // fewer tiles leave compute units idle that more blocks of the smaller kernels fill (one window: o 23.9 us there); a GELU has no other block's products
-    // beside it here (240 tiles: 31 and 57 us against 30 and 56)
-    if (count(best) < (EPI == BG_GELU ? 256 : 200)) return false;
+    // fewer tiles leave compute units idle that more blocks of the smaller kernels fill (one window: o 23.9 us there; fc1, 240 tiles: 28 here, 30 there)
+    if (count(best) < 200) return false;
     auto go = [&](auto tag) {
         constexpr int TM = decltype(tag)::value;
         void (*kernel)(BigGemmParams);
@@ -632,7 +682,7 @@ static bool launch_gemm_rows(const BigGemmParams& p, hipStream_t s) {
     };
     if (best == 8) go(std::integral_constant<int, 8>{});
     else if (best == 6) go(std::integral_constant<int, 6>{});
-    else if (best == 5) go(std::integral_constant<int, 5>{});
+    else if (best == 5) go(std::integral_constant<int, EPI == BG_GELU || EPI == BG_GELU_POS ? 4 : 5>{});
     else go(std::integral_constant<int, 4>{});
     return true;
 }
