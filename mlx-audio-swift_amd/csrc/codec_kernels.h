@@ -150,8 +150,8 @@ void launch_dw7(const float* X, float* Y, const float* w7 /*[C][7]*/, const floa
 // Snake -> 7-tap conv (C -> 1, weights at w[c cs + k ks]) -> tanh
 void launch_codec_final(const float* X, float* out, int64_t out_stride, const float* w, int cs, int ks, float bias, const float* alpha, const float* ralpha, int batch, int C, int T,
                         hipStream_t s);
-// encoder pieces (SNAC / DAC): first conv k7 "same" 1 -> C (w [C][7]); Snake + phase split for a stride-s conv
-// (y[(c*s + r)][m] = snake(x[c][s*m + r])); nearest code of the L2-normalised latent (first index on ties; cn = normalised codebook
+// encoder pieces (SNAC / DAC): first conv k7 "same" 1 -> C (w [C][7]); Snake + phase split for a stride-s conv of kernel 2 s
+// and padding p = ceil(s / 2) (y[(c*s + r)][m] = snake(x[c][s*m + r - p]), m <= T / s); nearest code of the L2-normalised latent (first index on ties; cn = normalised codebook
 // [CB][CD], cn2 = its squared norms); residual -= table[code] (table [CB][C], code index t / stride)
 void launch_enc_first(const float* audio, float* y, const float* w, const float* bias, int batch, int C, int T, hipStream_t s);
 void launch_enc_phase_split(const float* x, float* y, const float* a, const float* ra, int batch, int C, int T, int stride, hipStream_t s);

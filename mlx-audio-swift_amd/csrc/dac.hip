@@ -241,20 +241,17 @@ extern "C" mis_status mis_dac_finalize(mis_dac* c) {
                     E.ru[ri].dil = dils[ri];
                 }
                 snake(p + ".3.alpha", ch, E.a, E.ra);
-                {   // WNConv1d(k = 2s, stride s, pad ceil(s/2)) over the phase-split input [ch*s][T/s]:
-                    // y[n] = sum_{q in -1..1} sum_{c,r} W[co][s*q + r + pad][c] * xph[c*s + r][n + q]
-                    const int sdn = E.stride, K = 2 * sdn, pad = (sdn + 1) / 2;
+                {   // WNConv1d(k = 2s, stride s, pad ceil(s/2)) over the shifted phase-split input [ch*s][T/s + 1]:
+                    // y[n] = sum_{q in 0..1} sum_{c,r} W[co][s*q + r][c] * xph[c*s + r][n + q]
+                    const int sdn = E.stride, K = 2 * sdn;
                     std::vector<float> w = wn(p + ".4", E.cout, K, ch, 0);
-                    std::vector<float> at((size_t)3 * sdn * ch * E.cout, 0.0f);
-                    for (int qi = 0; qi < 3; ++qi)
+                    std::vector<float> at((size_t)K * ch * E.cout);
+                    for (int qi = 0; qi < 2; ++qi)
                         for (int64_t ci = 0; ci < ch; ++ci)
-                            for (int r = 0; r < sdn; ++r) {
-                                const int j = sdn * (qi - 1) + r + pad;
-                                if (j < 0 || j >= K) continue;
+                            for (int r = 0; r < sdn; ++r)
                                 for (int co = 0; co < E.cout; ++co)
-                                    at[(((size_t)qi * ch * sdn) + (size_t)ci * sdn + r) * E.cout + co] = w[((size_t)co * K + j) * ch + ci];
-                            }
-                    E.down.M = E.cout; E.down.K = 3 * sdn * (int)ch; E.down.w = push(at); E.down.b = push(dneed(c, p + ".4.bias", {E.cout}));
+                                    at[(((size_t)qi * ch * sdn) + (size_t)ci * sdn + r) * E.cout + co] = w[((size_t)co * K + sdn * qi + r) * ch + ci];
+                    E.down.M = E.cout; E.down.K = K * (int)ch; E.down.w = push(at); E.down.b = push(dneed(c, p + ".4.bias", {E.cout}));
                 }
                 c->hop *= E.stride;
                 ch = E.cout;
@@ -315,7 +312,7 @@ extern "C" mis_status mis_dac_encode(mis_dac* c, const float* audio, int batch, 
     size_t cap = (size_t)c->enc_dim * Tp;
     {
         int64_t T = Tp;
-        for (auto& b : c->enc_blocks) { cap = std::max(cap, (size_t)b.cin * T); T /= b.stride; cap = std::max(cap, (size_t)b.cout * T); }
+        for (auto& b : c->enc_blocks) { cap = std::max(cap, (size_t)b.cin * (T + b.stride)); T /= b.stride; cap = std::max(cap, (size_t)b.cout * T); }
         cap = std::max(cap, (size_t)D * T);
     }
     cap *= (size_t)batch;
@@ -347,7 +344,8 @@ extern "C" mis_status mis_dac_encode(mis_dac* c, const float* audio, int batch, 
         launch_enc_phase_split(x, f1, W + E.a, W + E.ra, batch, E.cin, (int)T, E.stride, s);
         T /= E.stride;
         GemmParams g = gp(E.down, f1, f2, (int)T);
-        g.Cin = E.stride * E.cin; g.taps = 3; g.dil = 1; g.pad = 1;
+        g.Tin = (int)T + 1;
+        g.Cin = E.stride * E.cin; g.taps = 2; g.dil = 1; g.pad = 0;
         launch_gemm(GEMM_TAPS, false, g, batch, s);
         std::swap(x, f2);
     }

@@ -428,14 +428,21 @@ __global__ void __launch_bounds__(256) k_enc_first(const float* __restrict__ aud
         y[((size_t)b * C + c) * T + t] = acc;
     }
 }
-// Snake, then phase split for a stride-s conv: y[(c*s + r)][m] = snake(x[c][s*m + r])   (T = s*Tm)
+// Snake, then phase split for a conv of stride s, kernel 2 s and padding `pad`: y[(c*s + r)][m] = snake(x[c][s*m + r - pad]), m <= T / s, zero outside the row
+// (T = s*Tm).  Shifted by the padding, the kernel covers two columns of each phase and no product meets a weight that is not there (unshifted: three
+// columns, a third of the weights zero).  A thread makes the s phases of one m: coalesced stores, loads of s values that lie together.
 __global__ void k_enc_phase_split(const float* __restrict__ x, float* __restrict__ y, const float* __restrict__ a, const float* __restrict__ ra,
-                                  int C, int T, int s) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y, b = blockIdx.z;
-    if (t >= T) return;
-    const int Tm = T / s, m = t / s, r = t - m * s;
-    float v = snake_f(x[((size_t)b * C + c) * T + t], a[c], ra[c]);
-    y[((size_t)b * C * s + (size_t)c * s + r) * Tm + m] = v;
+                                  int C, int T, int s, int pad) {
+    const int m = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y, b = blockIdx.z, Tm = T / s + 1;
+    if (m >= Tm) return;
+    const float* row = x + ((size_t)b * C + c) * T;
+    float* o = y + ((size_t)b * C + c) * s * Tm + m;
+    const float al = a[c], ral = ra[c];
+    for (int r = 0; r < s; ++r) {
+        const int t = m * s + r - pad;
+        const float v = row[min(max(t, 0), T - 1)];
+        o[(size_t)r * Tm] = t >= 0 && t < T ? snake_f(v, al, ral) : 0.0f;
+    }
 }
 // average pool over `stride` consecutive samples (VQ.swift:47-57)
 __global__ void k_vq_pool(const float* __restrict__ x, float* __restrict__ y, int C, int T, int stride) {
@@ -703,7 +710,7 @@ struct mis_snac {
         int cin, cout, stride;
         struct RU { SnakeW s1, s2; ConvW dw, pw; } ru[3];
         SnakeW snake;
-        ConvW down;                       // strided conv as a 3-tap conv over the phase-split tensor: A^T [3*s*cin][cout]
+        ConvW down;                       // strided conv as a 2-tap conv over the shifted phase-split tensor: A^T [2*s*cin][cout]
     };
     // LocalMHA of the 32 / 44 kHz models (Attention.swift): decoder layer 2, encoder layer n + 1
     struct MhaW { bool on = false; int dim = 0; size_t ln_w = 0, ln_b = 0, qkv = 0, out = 0, inv_freq = 0; };
@@ -985,19 +992,16 @@ extern "C" mis_status mis_snac_finalize(mis_snac* c) {
                 eb.ru[j].pw = push_pw(r + ".3", ch, ch, true);
             }
             eb.snake = push_snake(b + ".3.alpha", ch);
-            {   // WNConv1d(k = 2s, stride s, pad ceil(s/2)) (Layers.swift:248-254) over the phase-split input [ch*s][T/s]:
-                // y[n] = sum_{q in -1..1} sum_{c,r} W[co][s*q + r + pad][c] * xph[c*s + r][n + q]
-                const int sdn = eb.stride, K = 2 * sdn, pad = (sdn + 1) / 2;
+            {   // WNConv1d(k = 2s, stride s, pad ceil(s/2)) (Layers.swift:248-254) over the shifted phase-split input [ch*s][T/s + 1]:
+                // y[n] = sum_{q in 0..1} sum_{c,r} W[co][s*q + r][c] * xph[c*s + r][n + q]
+                const int sdn = eb.stride, K = 2 * sdn;
                 std::vector<float> w = fold_weight_norm(need(c, b + ".4.weight_g", {eb.cout, 1, 1}), need(c, b + ".4.weight_v", {eb.cout, K, ch}), 1e-12f);
-                std::vector<float> at((size_t)3 * sdn * ch * eb.cout, 0.0f);
-                for (int qi = 0; qi < 3; ++qi)
+                std::vector<float> at((size_t)K * ch * eb.cout);
+                for (int qi = 0; qi < 2; ++qi)
                     for (int64_t ci = 0; ci < ch; ++ci)
-                        for (int r = 0; r < sdn; ++r) {
-                            const int j = sdn * (qi - 1) + r + pad;
-                            if (j < 0 || j >= K) continue;
+                        for (int r = 0; r < sdn; ++r)
                             for (int co = 0; co < eb.cout; ++co)
-                                at[(((size_t)qi * ch * sdn) + (size_t)ci * sdn + r) * eb.cout + co] = w[((size_t)co * K + j) * ch + ci];
-                        }
+                                at[(((size_t)qi * ch * sdn) + (size_t)ci * sdn + r) * eb.cout + co] = w[((size_t)co * K + sdn * qi + r) * ch + ci];
                 eb.down.w = push(at); eb.down.has_bias = true; eb.down.b = push(need(c, b + ".4.bias", {eb.cout}).v);
             }
             ch = eb.cout;
@@ -1066,7 +1070,7 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
     size_t cap = (size_t)c->enc_dim * Tp;
     {
         int64_t T = Tp;
-        for (auto& b : c->enc_blocks) { cap = std::max(cap, (size_t)b.cin * T); T /= b.stride; cap = std::max(cap, (size_t)b.cout * T); }
+        for (auto& b : c->enc_blocks) { cap = std::max(cap, (size_t)b.cin * (T + b.stride)); T /= b.stride; cap = std::max(cap, (size_t)b.cout * T); }
     }
     if (c->enc_attn.on) cap = std::max(cap, (size_t)3 * D * (Tp / std::max<int64_t>(1, mis_snac_hop_for_encoder(c))));
     cap *= (size_t)batch;
@@ -1092,12 +1096,12 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
             std::swap(x, f2);
         }
         MIS_REQUIRE(T % eb.stride == 0, MIS_ERR_AUDIO_ENCODE, "internal: length not divisible by the stride");
-        hipLaunchKernelGGL(k_enc_phase_split, dim3(cdiv(T, 256), eb.cin, batch), dim3(256), 0, s, x, f1, W + eb.snake.a, W + eb.snake.ra, eb.cin, (int)T, eb.stride);
+        launch_enc_phase_split(x, f1, W + eb.snake.a, W + eb.snake.ra, batch, eb.cin, (int)T, eb.stride, s);
         T /= eb.stride;
         GemmParams g{};
         g.AT = W + eb.down.w; g.bias = W + eb.down.b; g.X = f1; g.Y = f2;
-        g.M = eb.cout; g.K = 3 * eb.stride * eb.cin; g.N = (int)T; g.Tin = (int)T; g.Tout = (int)T;
-        g.Cin = eb.stride * eb.cin; g.taps = 3; g.dil = 1; g.pad = 1;
+        g.M = eb.cout; g.K = 2 * eb.stride * eb.cin; g.N = (int)T; g.Tin = (int)T + 1; g.Tout = (int)T;
+        g.Cin = eb.stride * eb.cin; g.taps = 2; g.dil = 1; g.pad = 0;
         launch_gemm(GEMM_TAPS, false, g, batch, s);
         std::swap(x, f2);
     }
@@ -1168,7 +1172,7 @@ void launch_enc_first(const float* audio, float* y, const float* w, const float*
     hipLaunchKernelGGL(k_enc_first, dim3(cdiv(T, 256), cdiv(C, ENC_FIRST_CH), batch), dim3(256), 0, s, audio, y, w, bias, C, T);
 }
 void launch_enc_phase_split(const float* x, float* y, const float* a, const float* ra, int batch, int C, int T, int stride, hipStream_t s) {
-    hipLaunchKernelGGL(k_enc_phase_split, dim3(cdiv(T, 256), C, batch), dim3(256), 0, s, x, y, a, ra, C, T, stride);
+    hipLaunchKernelGGL(k_enc_phase_split, dim3(cdiv(T / stride + 1, 256), C, batch), dim3(256), 0, s, x, y, a, ra, C, T, stride, (stride + 1) / 2);
 }
 void launch_vq_nearest(const float* ze, const float* cn, const float* cn2, int32_t* codes, int batch, int CD, int CB, int Tm, hipStream_t s) {
     MIS_REQUIRE(CD <= 64, MIS_ERR_INVALID_INPUT, "codebook_dim > 64 unsupported by the nearest-code kernel");
