@@ -10,7 +10,7 @@
 // convolution gives NaN where the f32 kernels give an infinity or NaN.)
 //
 //   k_x6_pack_w   A^T f32 -> the three planes as MFMA-A fragments (once per weight matrix, kept in the model's CodecPack)
-//   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels, for the encoders and for MIS_CODEC_EXACT_F32=1)
+//   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels and for MIS_CODEC_EXACT_F32=1) and its encoder's units of 48 and 96
 //   k_x6_gemm     1x1 and k-tap contractions (codec_f32.hip keeps the rest)
 //   k_x6_convt    transposed convolutions of stride 2 and at most 64 rows
 #include "common.h"
@@ -89,7 +89,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                                            const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
                                            const float* __restrict__ pra1, const float* __restrict__ pa2, const float* __restrict__ pra2,
                                            const uint16_t* __restrict__ pwp, const float* __restrict__ pb2, const PwScalars p) {
-    constexpr int KG = KC / 8, MT = C / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
+    constexpr int KG = KC / 8, MT = (C + 31) / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
     constexpr int XR = KC / 4, GS = KG * (NT / 64) / 4, XS = NT + 2 * CODEC_DW_HALO + 2, NS = (XS + 61) / 64;      // (XS - 2 columns in strips of 64)
                                // rows of x and (group, strip) pairs per wave
     __shared__ float xs[DW ? KC : 1][DW ? XS : 1];
@@ -217,12 +217,12 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = (wr + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
-                yb[(size_t)m * p.ldy + n] = rb[(size_t)m * p.ldr + n] + (acc[mi][ni][r] + pb2[m]);
+                if (C % 32 == 0 || m < C) yb[(size_t)m * p.ldy + n] = rb[(size_t)m * p.ldr + n] + (acc[mi][ni][r] + pb2[m]);
             }
     }
 }
 template <int C, bool DW, int KC, int NT>
-__global__ void __launch_bounds__(256, KC == 32 ? 2 : C == 128 && DW ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp) {
+__global__ void __launch_bounds__(256, KC == 32 ? 2 : DW && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp) {
     pw_x6_body<C, DW, KC, NT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
 }
 
@@ -230,25 +230,28 @@ __global__ void __launch_bounds__(256, KC == 32 ? 2 : C == 128 && DW ? 3 : 4) k_
 // 192 and 248: 23 and 25 (384 of 128 columns: 34).  (The next chunk's loads ahead of this one's products instead: 31 us, no registers left.)
 // Chunk depth (the same bits): 32 channels need half the barriers, 16 let three or four blocks (not two, C = 96: three) share a compute unit.  32 while its
 // blocks are all resident at once, else 16 (us, chunks of 32 / 16): 128 channels 96 blocks 28 / 33, 384: 34 / 38, 576: 61 / 45, 24576: 1584 / 1430;
-// 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150.  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32.
+// 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150 (with taps 16: 592 blocks, two rounds of 32).  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32.
 template <int C, bool DW>
 static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hipStream_t s) {
     const dim3 grid((p.T + 127) / 128, batch);
     if constexpr (C == 128) {
         if ((int64_t)grid.x * batch <= 256) { hipLaunchKernelGGL((k_pw_x6<C, DW, 32, 64>), dim3((p.T + 63) / 64, batch), dim3(256), 0, s, p, wp); return; }
     }
-    if constexpr (C <= 128) {
-        if ((int64_t)grid.x * batch > (C == 96 ? 768 : 512)) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16, 128>), grid, dim3(256), 0, s, p, wp); return; }
+    if constexpr (C == 48) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16, 128>), grid, dim3(256), 0, s, p, wp); return; }
+    else if constexpr (C <= 128) {
+        if ((int64_t)grid.x * batch > (C == 96 && !DW ? 768 : 512)) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16, 128>), grid, dim3(256), 0, s, p, wp); return; }
     }
-    hipLaunchKernelGGL((k_pw_x6<C, DW, 32, 128>), grid, dim3(256), 0, s, p, wp);
+    if constexpr (C != 48) hipLaunchKernelGGL((k_pw_x6<C, DW, 32, 128>), grid, dim3(256), 0, s, p, wp);
 }
 
 // 64 channels stay on k_pw_fused: twice the columns per product, bound by memory and by the units' VALU work (1.16 ms here, 1.10 there)
 bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s) {
     if (!pack) pack = codec_x6_scope();
-    if (!pack || codec_exact_f32() || !(dw ? C == 128 : (C == 96 || C == 128 || C == 192))) return false;
+    if (!pack || codec_exact_f32() || !(dw ? C == 48 || C == 96 || C == 128 : (C == 96 || C == 128 || C == 192))) return false;
     const uint16_t* wp = pack->get_x6(p.AT, 1, C, C, s).wp;
-    if (dw) launch_x6<128, true>(p, wp, batch, s);
+    if (dw && C == 48) launch_x6<48, true>(p, wp, batch, s);
+    else if (dw && C == 96) launch_x6<96, true>(p, wp, batch, s);
+    else if (dw) launch_x6<128, true>(p, wp, batch, s);
     else if (C == 96) launch_x6<96, false>(p, wp, batch, s);
     else if (C == 128) launch_x6<128, false>(p, wp, batch, s);
     else launch_x6<192, false>(p, wp, batch, s);

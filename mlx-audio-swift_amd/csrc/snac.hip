@@ -41,6 +41,11 @@ __global__ void __launch_bounds__(256) k_snac_embed(EmbedParams p, float* __rest
     });
 }
 
+static bool ru_fused_enabled() {                       // MIS_CODEC_FUSED_UNITS=0: the unfused kernels (A/B)
+    const char* v = getenv("MIS_CODEC_FUSED_UNITS");
+    return !v || atoi(v) != 0;
+}
+
 // ---- depthwise conv k=7 ---------------------------------------------------------------------------
 #define DW_TILE 1024
 #define DW_HALO CODEC_DW_HALO
@@ -1087,12 +1092,21 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
     for (auto& eb : c->enc_blocks) {
         for (int j = 0; j < 3; ++j) {
             const auto& ru = eb.ru[j];
-            hipLaunchKernelGGL((k_snac_dw<true, true>), dim3(cdiv(T, DW_TILE), eb.cin, batch), dim3(256), 0, s, x, f1, W + ru.dw.w, W + ru.dw.b,
-                               W + ru.s1.a, W + ru.s1.ra, W + ru.s2.a, W + ru.s2.ra, eb.cin, (int)T, dils[j]);
-            GemmParams g{};
-            g.AT = W + ru.pw.w; g.bias = W + ru.pw.b; g.X = f1; g.Y = f2; g.R = x;
-            g.M = eb.cin; g.K = eb.cin; g.N = (int)T; g.Tin = (int)T; g.Tout = (int)T;
-            launch_gemm(GEMM_RESID, false, g, batch, s);
+            PwFusedParams fp{};
+            fp.X = x; fp.R = x; fp.Y = f2; fp.w7 = W + ru.dw.w; fp.b1 = W + ru.dw.b; fp.a1 = W + ru.s1.a; fp.ra1 = W + ru.s1.ra;
+            fp.a2 = W + ru.s2.a; fp.ra2 = W + ru.s2.ra; fp.AT = W + ru.pw.w; fp.b2 = W + ru.pw.b;
+            fp.T = (int)T; fp.dil = dils[j]; fp.ldx = fp.ldr = fp.ldy = (int)T;
+            // Fused where its blocks of 128 columns (serial chains of chunks) fill the chip; the same bits.  us, fused / two kernels: 96 channels 592 blocks 41 / 49,
+            // 48 channels 1184 32 / 38; a row of 30011 samples (118 and 235 blocks) as a whole 603 / 569, four of 240000 (3752 and 7504) 3625 / 4081
+            const bool fused = ru_fused_enabled() && (eb.cin == 48 || eb.cin == 96) && cdiv(T, RU_NT) * (int64_t)batch >= 512;
+            if (!fused || !launch_pw_x6(eb.cin, true, fp, nullptr, batch, s)) {
+                hipLaunchKernelGGL((k_snac_dw<true, true>), dim3(cdiv(T, DW_TILE), eb.cin, batch), dim3(256), 0, s, x, f1, W + ru.dw.w, W + ru.dw.b,
+                                   W + ru.s1.a, W + ru.s1.ra, W + ru.s2.a, W + ru.s2.ra, eb.cin, (int)T, dils[j]);
+                GemmParams g{};
+                g.AT = W + ru.pw.w; g.bias = W + ru.pw.b; g.X = f1; g.Y = f2; g.R = x;
+                g.M = eb.cin; g.K = eb.cin; g.N = (int)T; g.Tin = (int)T; g.Tout = (int)T;
+                launch_gemm(GEMM_RESID, false, g, batch, s);
+            }
             std::swap(x, f2);
         }
         MIS_REQUIRE(T % eb.stride == 0, MIS_ERR_AUDIO_ENCODE, "internal: length not divisible by the stride");
@@ -1160,11 +1174,6 @@ extern "C" int64_t mis_snac_noise_len(const mis_snac* c, int block, int t_coarse
 void launch_dw7(const float* X, float* Y, const float* w7, const float* bias, int batch, int C, int T, int dil, hipStream_t s) {
     hipLaunchKernelGGL((k_snac_dw<false, false>), dim3(cdiv(T, DW_TILE), C, batch), dim3(256), 0, s, X, Y, w7, bias, nullptr,
                        nullptr, nullptr, nullptr, C, T, dil);
-}
-
-static bool ru_fused_enabled() {                       // MIS_CODEC_FUSED_UNITS=0: the unfused kernels (A/B)
-    const char* v = getenv("MIS_CODEC_FUSED_UNITS");
-    return !v || atoi(v) != 0;
 }
 
 // encoder pieces shared with the Descript DAC encoder (dac.hip)
