@@ -900,13 +900,17 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     const size_t Mc = round_up((size_t)most, 16);                            // GEMM rows round up to 16
     c->pf_h.alloc(Mc * d); c->pf_x.alloc(Mc * d); c->pf_attn.alloc(Mc * HD);
     c->pf_q.alloc(Mc * HD); c->pf_pos.alloc(Mc); c->pf_on.alloc(Mc);
-    // quantised checkpoints (every role streamed as codes): each GEMM of the chunk runs the decode step's k_gemm_skinny_q on 64-row
-    // slices - rows packed into MFMA fragments first, float32 sums out, the residual add as its own small kernel; gate|up writes the
+    // quantised checkpoints (every role streamed as codes): k_gemm_pf_codes on the chunk's rows; a chunk of few rows runs the decode step's k_gemm_skinny_q on
+    // 64-row slices - rows packed into MFMA fragments first, float32 sums out, the residual add as its own small kernel; gate|up writes the
     // packed activation its down projection reads.  The weights are streamed once per 64 rows instead of once per position.
     const bool coded = c->q_qkv.on;
     if (coded) c->pf_qkv.alloc(Mc * c->Nqkv); else c->pf_qkv16.alloc(Mc * c->Nqkv);
-    if (coded) { c->pf_xpk.alloc((size_t)64 * std::max(d, HD)); c->pf_actpk.alloc((size_t)64 * c->ff); c->pf_tmp.alloc((size_t)64 * d); }
+    const bool tiled = coded && Mc > 96;                                      // (70 rows: 5.7 ms in slices, 7.7 tiled; 107: 8.3, 7.7)
+    if (coded && !tiled) { c->pf_xpk.alloc((size_t)64 * std::max(d, HD)); c->pf_actpk.alloc((size_t)64 * c->ff); c->pf_tmp.alloc((size_t)64 * d); }
     else c->pf_act.alloc(Mc * c->ff);
+    auto q_tiled = [&](int epi, const mis_tts::QRole& q, int li, const bf16_t* x, void* out, int M, int N, int K) {
+        launch_gemm_pf_codes(epi, q.bits, x, q.q.p + q.q_layer * li, q.sb.p + q.sb_layer * li, out, M, N, K, s);
+    };
     auto q_rows = [&](int M, const std::function<void(int r0, int mp)>& body) {
         for (int r0 = 0; r0 < M; r0 += 64) body(r0, std::min(64, M - r0));
     };
@@ -929,7 +933,8 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
         else launch_pf_embed_rmsnorm(c->emb.p, prompt_mat_dev, lens_dev, Lmax, t0, tc, batch, 0, c->V, c->norms.p, c->pf_h.p, c->pf_x.p,
                                      c->pf_pos.p, c->pf_on.p, Mr, d, eps, s);
         for (int li = 0; li < c->L; ++li) {
-            if (coded) q_rows(M, [&](int r0, int mp) {
+            if (tiled) q_tiled(PF_F32, c->q_qkv, li, c->pf_x.p, c->pf_qkv.p, M, c->Nqkv, d);
+            else if (coded) q_rows(M, [&](int r0, int mp) {
                 launch_pf_pack_rows(c->pf_x.p + (size_t)r0 * d, c->pf_xpk.p, mp, d, s);
                 q_partial(c->q_qkv, li, c->pf_xpk.p, c->pf_qkv.p + (size_t)r0 * c->Nqkv, c->Nqkv, d, mp);
             });
@@ -952,14 +957,18 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
             }
             pa.rope_in_dtype = c->cfg.rope_ops_in_dtype;
             launch_pf_attention(pa, s);
-            if (coded) q_rows(M, [&](int r0, int mp) {
+            if (tiled) q_tiled(PF_RESID, c->q_o, li, c->pf_attn.p, c->pf_h.p, M, d, HD);
+            else if (coded) q_rows(M, [&](int r0, int mp) {
                 launch_pf_pack_rows(c->pf_attn.p + (size_t)r0 * HD, c->pf_xpk.p, mp, HD, s);
                 q_partial(c->q_o, li, c->pf_xpk.p, c->pf_tmp.p, d, HD, mp);
                 launch_pf_add_resid(c->pf_h.p + (size_t)r0 * d, c->pf_tmp.p, (size_t)mp * d, s);
             });
             else launch_gemm_pf(PF_RESID, c->pf_attn.p, c->wo.p + layer_o_elems(c) * li, c->pf_h.p, M, d, HD, s);
             launch_pf_rmsnorm(c->pf_h.p, c->norms.p + (size_t)(2 * li + 1) * d, c->pf_x.p, M, d, eps, s);
-            if (coded) q_rows(M, [&](int r0, int mp) {
+            if (tiled) {
+                q_tiled(PF_SILU, c->q_gu, li, c->pf_x.p, c->pf_act.p, M, 2 * c->ff, d);
+                q_tiled(PF_RESID, c->q_down, li, c->pf_act.p, c->pf_h.p, M, d, c->ff);
+            } else if (coded) q_rows(M, [&](int r0, int mp) {
                 launch_pf_pack_rows(c->pf_x.p + (size_t)r0 * d, c->pf_xpk.p, mp, d, s);
                 launch_gemm_skinny_q(c->q_gu.bits, EPI_SILU_MUL, 2, c->ksb_gu, c->q_gu.q.p + c->q_gu.q_layer * li, c->q_gu.sb.p + c->q_gu.sb_layer * li,
                                      c->pf_xpk.p, c->pf_actpk.p, 2 * c->ff / 16, d / 64, 1, c->ff, mp, s);
