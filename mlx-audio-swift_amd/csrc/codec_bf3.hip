@@ -478,7 +478,11 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
         p.pack->part.alloc((size_t)ksplit * batch * p.M * p.ldy);
         P.ksplit = ksplit; P.part = p.pack->part.p; P.batch = batch;
     }
-    const int bm = few ? 64 : B3_BM;
+    // Rows that are no multiple of 128 leave a wave row of the large tile without any, and its blocks (7 taps: one a compute unit) come in whole rounds: 64 x 128 there,
+    // two blocks a compute unit.  us, 128 x 128 / 64 x 128: 192 rows, 7 taps, 40000 columns 91 / 63, 2 taps (5 phases) 62 / 54; 96 rows, 80000 columns 67 / 45, 47 / 39;
+    // whole tiles: 384 rows, 7 taps, 10000 columns 60 / 64, 2 taps of 512 .. 128 rows (SNAC, 32 rows) 588 / 767, 1395 / 1748, 1734 / 1966
+    const bool half = !few && ntaps != 1 && p.M % B3_BM != 0;
+    const int bm = few || half ? 64 : B3_BM;
     P.nbx = nbx; P.my = (p.M + bm - 1) / bm; P.inner = phases * ksplit;
     P.tiles = nbx * P.my * batch; P.per = (P.tiles + 7) / 8;
     dim3 grid(8 * P.per * P.inner), block(B3_THREADS);
@@ -494,6 +498,9 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
         else if (span <= 16) B3_GO(1, 2, 9, 4, 7, 7, 2);
         else B3_GO(1, 2, 12, 4, 7, 7, 2);
     }
+    else if (half && ntaps == 2) B3_GO(1, 2, 9, 4, 2, 4, 3);
+    else if (half && span <= 16) B3_GO(1, 2, 9, 4, 7, 4, 3);
+    else if (half) B3_GO(1, 2, 12, 3, 7, 4, 3);
     // MINW 3 = two blocks (ten waves) per CU, 168 registers: fits 1 and 2 taps; the 7-tap body would spill (measured 2.3x slower), so it
     // runs one block per CU (a persistent loop over column tiles was measured too: no gain, profiles/r02_codec/ab_record.json)
     else if (ntaps == 1) B3_GO(2, 2, 9, 4, 1, 3, 3);
