@@ -555,6 +555,7 @@ static void launch_x6_gemm(X6Gemm P, const uint16_t* wp, int batch, hipStream_t 
             // us, 4 tiles / 2 / the narrow form: 384 rows, K = 4608, 394 columns 204 / 155 / 31, 2368 columns (57, 114 blocks of 4 and 2) 204 / 154 / 91, eight such
             // rows (456, 912) 336 / 469 / 583; 128 rows, K = 3072, 16000 columns (250 of 2) 146 / 110 / 123; 192 rows, K = 1152, 18944 columns (296, 444) 94 / 71 / 97,
             // eight such rows 444 / 437 / 733; 768 rows, K = 9216, 296 columns 394 / 299 / 59 (f32: 94)
+            // (strided convolutions of three taps then; on two, narrow: 384 rows, K = 3072, 2368 columns 72, 768 rows, K = 6144, 296 columns 45)
             if (P.MT32 > 2 && blocks(4) >= 384) go(k_x6_gemm<4, SNAKE, TAPS, true, true>, 4);
             else if (blocks(2) >= 192) go(k_x6_gemm<2, SNAKE, TAPS, true, true>, 2);
             else {
