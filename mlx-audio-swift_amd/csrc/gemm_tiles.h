@@ -14,6 +14,17 @@
 #pragma once
 #include "common.h"
 
+// The tiles are numbered in bands of G row tiles, row tiles fastest, and an XCD (blocks are dealt to the XCDs by id mod 8) takes one range of them: the 32
+// blocks it runs together share G row tiles of X and 32 / G column tiles of W in its L2.
+struct TileOrder {
+    int mt, nt;
+    __device__ __forceinline__ void at(int G, int t, int& mi, int& ni) const {
+        const int band = t / (G * nt), left = t - band * G * nt, rows = min(G, mt - band * G);
+        ni = left / rows;
+        mi = band * G + left - ni * rows;
+    }
+};
+
 __device__ __forceinline__ uint32_t gt_lds_offset(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
 
 // Wave (wn, wm) = (wave >> 1, wave & 1) holds W rows 128 wn + 16 i and X rows 16 TM wm + 16 j of the tile in acc[i][j] (the MFMA's C/D layout).
@@ -28,10 +39,6 @@ struct GemmTiles {
 
     // tiles first, first + stride, ... < tiles.  woff(t, q, lane): element offset of the lane's 16 bytes of the tile's q-th KB of W at k = 0; xoff(t, r): of row r
     // of its X; epi(t, acc) stores a finished tile
-    template <class FW, class FX, class FE>
-    static __device__ __forceinline__ void run(unsigned char* lds, const bf16_t* Wb, const bf16_t* Xb, int K, int first, int stride, int tiles, FW woff, FX xoff, FE epi) {
-        run(lds, K, first, stride, tiles, [&](int, const bf16_t*& w, const bf16_t*& x) { w = Wb; x = Xb; }, woff, xoff, epi);
-    }
     // operands(t, W, X): the two operands of tile t
     template <class FO, class FW, class FX, class FE>
     static __device__ __forceinline__ void run(unsigned char* lds, int K, int first, int stride, int tiles, FO operands, FW woff, FX xoff, FE epi) {

@@ -479,8 +479,6 @@ static bool launch_big3(const BigGemmParams& p, hipStream_t s) {
 // (k_gemm_big2 where 180 tiles of 256 x 256 were too few) 100 / 128, 44 / 58, 128 / 159, 122 / 173, 66 / 90; 4 x 1500 71 / 89, 33 / 34, 93 / 107, 85 / 95, 45 / 50.
 // k_gemm_big3 keeps what these offsets or rings cannot hold.
 // TM by the rounds of 256 persistent blocks it makes (launch_gemm_rows).  Products in the order of k: the bits of k_gemm_big2.
-// The tiles are numbered in bands of G row tiles, row tiles fastest, and an XCD (blocks are dealt to the XCDs by id mod 8) takes one range of them: the 32
-// blocks it runs together share G row tiles of X and 32 / G column tiles of W in its L2.
 // A GELU after T(xW^T + b) is a function of sixteen bits: gelu_erf_w(v) = v f(v), f in an LDS table over |v| = 2^-10 .. 16 and the sign (14 KB; below 2^-10 the
 // result is v / 2, above 16 it is v or -0: the values that the clamped factors round to).  The same bits as the formula, in 12 instructions an
 // output and an LDS read for 31, two of them of quarter rate - a block's only waves wait for them.  fc1, eight windows 204 -> 171 us, one 31 -> 28.
@@ -518,14 +516,6 @@ struct GeluTable {
         for (int e = 0; e < 16; ++e) x[e] *= f[e];
     }
 };
-struct TileOrder {
-    int mt, nt;
-    template <int G> __device__ __forceinline__ void at(int t, int& mi, int& ni) const {
-        const int band = t / (G * nt), left = t - band * G * nt, rows = min(G, mt - band * G);
-        ni = left / rows;
-        mi = band * G + left - ni * rows;
-    }
-};
 template <int EPI, int TM>
 __device__ __forceinline__ void gemm_rows_body(const BigGemmParams& p) {
     using T = GemmTiles<TM, false>;
@@ -544,8 +534,8 @@ __device__ __forceinline__ void gemm_rows_body(const BigGemmParams& p) {
     auto where = [&](int t, bool& swp, int& m0, int& n0) {
         int mi, ni;
         swp = EPI == BG_KV && t >= tiles0;
-        if (swp) { o1.template at<G>(t - tiles0, mi, ni); m0 = mi * T::BN; n0 = N0 + ni * T::BM; }
-        else { o0.template at<G>(t, mi, ni); m0 = mi * T::BM; n0 = ni * T::BN; }
+        if (swp) { o1.at(G, t - tiles0, mi, ni); m0 = mi * T::BN; n0 = N0 + ni * T::BM; }
+        else { o0.at(G, t, mi, ni); m0 = mi * T::BM; n0 = ni * T::BN; }
     };
     bool sw; int mt0, nt0;                                   // of the tile being requested
     T::run(lds, p.K, first, gridDim.x >> 3, hi,
