@@ -905,7 +905,7 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     // packed activation its down projection reads.  The weights are streamed once per 64 rows instead of once per position.
     const bool coded = c->q_qkv.on;
     if (coded) c->pf_qkv.alloc(Mc * c->Nqkv); else c->pf_qkv16.alloc(Mc * c->Nqkv);
-    const bool tiled = coded && Mc > 96;                                      // (70 rows: 5.7 ms in slices, 7.7 tiled; 107: 8.3, 7.7)
+    const bool tiled = coded && Mc > 96;                                      // (90 rows: 5.9 ms in slices, 7.3 tiled; 107: 8.3, 7.3; the same bits)
     if (coded && !tiled) { c->pf_xpk.alloc((size_t)64 * std::max(d, HD)); c->pf_actpk.alloc((size_t)64 * c->ff); c->pf_tmp.alloc((size_t)64 * d); }
     else c->pf_act.alloc(Mc * c->ff);
     auto q_tiled = [&](int epi, const mis_tts::QRole& q, int li, const bf16_t* x, void* out, int M, int N, int K) {

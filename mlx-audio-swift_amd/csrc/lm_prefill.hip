@@ -482,8 +482,11 @@ __global__ void __launch_bounds__(128) k_gemm_pf_ring(PfGemmParams p) {
 // ---- prompt GEMMs on 8- / 4-bit codes (layouts and arithmetic of lm_qgemm.hip: y = sum over groups of 64 of scale * sum(q x) + bias * sum(x), codes exact in
 // bf16, float32 sums).  The decode step's kernels take 64 rows a launch and read the weights again for each; here a block of 64 TM/2 x 64 TN/2 outputs unpacks a
 // code once for all its rows, into the fragment image that k_gemm_pf reads.  A k-step is a scale group: X by LDS-DMA and codes and scales through registers one step
-// ahead, one barrier.  Bound: a group costs an output eight FMAs beside its 64 products - VALU and matrix pipe are level, two blocks a compute unit share both.
-// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 107 rows 8.3 / 7.7, 175 10.8 / 8.5, 274 15.8 / 9.5, 413 21.0 / 10.9, 804 38.4 / 15.8, 3202 151 / 46.
+// ahead, one barrier.  Bound: a group costs an output a product, an FMA and an addition beside its 64 products - VALU above matrix pipe, two blocks a compute unit
+// share both.  (Two FMAs into one chain of sums are 10 % faster at 128 x 128 - gate | up of 3216 rows 583 us, 641 here - but then a prompt's bits depend on the
+// other prompts of its call, which decide between slices and tiles.)
+// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 70 rows 5.7 / 7.3, 90 5.9 / 7.3, 107 8.3 / 7.3, 175 10.8 / 8.6, 274 15.8 / 9.4, 413 21.0 / 10.6,
+// 804 38.4 / 16.2, 3202 151 / 46.6.
 __device__ __forceinline__ uint4 pf_codes(uint2 w) {
     uint32_t o[4];
 #pragma unroll
@@ -507,7 +510,8 @@ template <> struct PfCode<4> { typedef uint32_t type; };
 template <int EPI, int TN, int TM, int GS, int BITS>
 __global__ void __launch_bounds__(256, 2) k_gemm_pf_codes(PfGemmParams p, const void* __restrict__ Qp, const bf16_t* __restrict__ SB) {
     typedef typename PfCode<BITS>::type WT;
-    constexpr int BN = 32 * TN, BM = 32 * TM;
+    constexpr int BN = 32 * TN, BM = 32 * TM, HELD = TN == 4 ? 2 : 0;
+    __shared__ f32x4_t held[HELD ? HELD : 1][256];
     __shared__ __attribute__((aligned(1024))) bf16_t Ws[2][GS][BN * PF_BK];
     __shared__ __attribute__((aligned(1024))) bf16_t Xs[2][GS][BM * PF_BK];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -520,33 +524,33 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf_codes(PfGemmParams p, const 
 #pragma unroll
         for (int j = 0; j < TM; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     // a wave stages TN of the block's 4 TN weight fragments (2 TN n-tiles x 2 k-tiles) and TM KB of X (k_gemm_pf's image); it reads the scales of its own n-tiles
+    // (bases per wave in scalar registers, 32-bit offsets per lane: the totals need the others)
     const WT* wsrc[TN];
     const uint2* sbp[TN];
-    const bf16_t* xsrc[TM];
+    uint32_t xoff[TM];
 #pragma unroll
     for (int q = 0; q < TN; ++q) {
         const int f = wave * TN + q;
-        wsrc[q] = reinterpret_cast<const WT*>(Qp) + ((size_t)min((n0 >> 4) + (f >> 1), NT - 1) * KT + (f & 1)) * 64 + lane;
-        sbp[q] = reinterpret_cast<const uint2*>(SB) + (size_t)min((n0 >> 4) + wn * TN + q, NT - 1) * G * 8 + (lane >> 4);
+        wsrc[q] = reinterpret_cast<const WT*>(Qp) + ((size_t)min((n0 >> 4) + (f >> 1), NT - 1) * KT + (f & 1)) * 64;
+        sbp[q] = reinterpret_cast<const uint2*>(SB) + (size_t)min((n0 >> 4) + wn * TN + q, NT - 1) * G * 8;
     }
 #pragma unroll
     for (int q = 0; q < TM; ++q) {
         const int r = (wave * TM + q) * 8 + (lane >> 3);
-        xsrc[q] = p.X + (size_t)min(m0 + r, p.M - 1) * p.K + ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+        xoff[q] = ((uint32_t)min(m0 + r, p.M - 1) * p.K + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2;
     }
+    const uint32_t sl = lane >> 4;
     WT w[GS][TN];
-    uint2 sb[GS][TN][2], sbn[GS][TN][2];
+    uint2 sb[GS][TN][2];
     auto loadW = [&](int g0) {                          // (groups past the end: the last one again, never multiplied)
 #pragma unroll
         for (int u = 0; u < GS; ++u)
 #pragma unroll
-            for (int q = 0; q < TN; ++q) w[u][q] = wsrc[q][(size_t)min(g0 + u, G - 1) * 128];
+            for (int q = 0; q < TN; ++q) w[u][q] = (wsrc[q] + (size_t)min(g0 + u, G - 1) * 128)[(uint32_t)lane];
     };
-    auto loadS = [&](int g0) {
-#pragma unroll
-        for (int u = 0; u < GS; ++u)
-#pragma unroll
-            for (int q = 0; q < TN; ++q) { const size_t o = (size_t)min(g0 + u, G - 1) * 8; sbn[u][q][0] = sbp[q][o]; sbn[u][q][1] = sbp[q][o + 4]; }
+    auto loadS = [&](int g, int u, int q) {
+        const uint2* o = sbp[q] + (size_t)min(g, G - 1) * 8;
+        sb[u][q][0] = o[sl]; sb[u][q][1] = o[sl + 4];
     };
     auto putW = [&](int buf) {
 #pragma unroll
@@ -559,18 +563,43 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf_codes(PfGemmParams p, const 
         for (int u = 0; u < GS; ++u)
 #pragma unroll
             for (int q = 0; q < TM; ++q)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xsrc[q] + (size_t)min(g0 + u, G - 1) * PF_BK),
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(reinterpret_cast<const unsigned char*>(p.X + (size_t)min(g0 + u, G - 1) * PF_BK) + xoff[q]),
                                                  (__attribute__((address_space(3))) void*)&Xs[buf][u][(wave * TM + q) * 8 * PF_BK], 16, 0, 0);
     };
     bf16x8_t ones;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ones[e] = (short)0x3F80;
     const f32x4_t zero = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    // A row is to have the bits that k_gemm_skinny_q gives it: its four waves sum a quarter of the groups each, the quarters are added in order.  The total of the
+    // large tile's last HELD products waits in LDS: the registers hold 248 values beside it
+    f32x4_t tot[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) tot[i][j] = zero;
+    auto close = [&](bool first) {                      // (0 + p0 is p0: a sum that starts at 0 is never -0)
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+            for (int j = 0; j < TM; ++j) {
+                const int h = i * TM + j - (TN * TM - HELD);
+                f32x4_t t = h < 0 ? tot[i][j] : first ? zero : held[h < 0 ? 0 : h][tid];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) t[e] += acc[i][j][e];
+                acc[i][j] = zero;
+                if (h < 0) tot[i][j] = t;
+                else held[h < 0 ? 0 : h][tid] = t;
+            }
+    };
+    int part = 1;                                       // the quarter of the groups that begins next
     const int sw = (lane >> 1) & 7;
     loadW(0);
     putW(0);
     loadW(GS);
-    loadS(0);
+#pragma unroll
+    for (int u = 0; u < GS; ++u)
+#pragma unroll
+        for (int q = 0; q < TN; ++q) loadS(u, u, q);
     stageX(0, 0);
     for (int g0 = 0, buf = 0; g0 < G; g0 += GS, buf ^= 1) {
         __syncthreads();                                // X and codes of this step are in LDS, the codes of the next and the scales of this one in registers
@@ -587,46 +616,53 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf_codes(PfGemmParams p, const 
             }
         const bool more = g0 + GS < G;
         if (more) putW(buf ^ 1);                        // (the other buffer: read by everybody before this step's barrier)
-#pragma unroll
-        for (int u = 0; u < GS; ++u)
-#pragma unroll
-            for (int q = 0; q < TN; ++q) { sb[u][q][0] = sbn[u][q][0]; sb[u][q][1] = sbn[u][q][1]; }
         __builtin_amdgcn_sched_barrier(0);
         loadW(g0 + 2 * GS);
-        loadS(g0 + GS);
         if (more) stageX(buf ^ 1, g0 + GS);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < GS; ++u) {
             if (u && g0 + u >= G) break;
-            f32x4_t sx[TM];
+            if (part < 4 && g0 + u == G * part / 4) {
+                close(part == 1);
+                do ++part; while (part < 4 && G * part / 4 == g0 + u);
+            }
+            float sx[TM];                               // (the rows of a tile of ones are one row)
 #pragma unroll
             for (int j = 0; j < TM; ++j) {
-                sx[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[u][0][j], zero, 0, 0, 0);
-                sx[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[u][1][j], sx[j], 0, 0, 0);
+                f32x4_t t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[u][0][j], zero, 0, 0, 0);
+                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[u][1][j], t, 0, 0, 0);
+                sx[j] = t[0];
             }
 #pragma unroll
             for (int i = 0; i < TN; ++i) {
                 const uint2 s0 = sb[u][i][0], b0 = sb[u][i][1];
                 const float sc[4] = {__uint_as_float(s0.x << 16), __uint_as_float(s0.x & 0xffff0000u), __uint_as_float(s0.y << 16), __uint_as_float(s0.y & 0xffff0000u)};
                 const float bi[4] = {__uint_as_float(b0.x << 16), __uint_as_float(b0.x & 0xffff0000u), __uint_as_float(b0.y << 16), __uint_as_float(b0.y & 0xffff0000u)};
-                f32x4_t ag[TM];
 #pragma unroll
-                for (int j = 0; j < TM; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][0][i], b[u][0][j], zero, 0, 0, 0);
+                for (int j0 = 0; j0 < TM; j0 += 2) {
+                    f32x4_t ag[2];
 #pragma unroll
-                for (int j = 0; j < TM; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][1][i], b[u][1][j], ag[j], 0, 0, 0);
+                    for (int j = 0; j < 2; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][0][i], b[u][0][j0 + j], zero, 0, 0, 0);
 #pragma unroll
-                for (int j = 0; j < TM; ++j)
+                    for (int j = 0; j < 2; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][1][i], b[u][1][j0 + j], ag[j], 0, 0, 0);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][j][e] = fmaf(bi[e], sx[j][e], fmaf(sc[e], ag[j][e], acc[i][j][e]));
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][j0 + j][e] += fmaf(sc[e], ag[j][e], bi[e] * sx[j0 + j]);
+                }
+                loadS(g0 + GS + u, u, i);               // (the next step's, into the registers just read)
             }
         }
     }
-    pf_epilogue<EPI, TN, TM>(p, acc, (n0 >> 4) + wn * TN, m0 + wm * TM * 16, lane);
+    close(false);
+#pragma unroll
+    for (int h = 0; h < HELD; ++h) tot[(TN * TM - HELD + h) / TM][(TN * TM - HELD + h) % TM] = held[h][tid];
+    pf_epilogue<EPI, TN, TM>(p, tot, (n0 >> 4) + wn * TN, m0 + wm * TM * 16, lane);
 }
 void launch_gemm_pf_codes(int epi, int bits, const bf16_t* X, const void* Qp, const bf16_t* SB, void* C, int M, int N, int K, hipStream_t s) {
-    MIS_REQUIRE(K % PF_BK == 0 && K >= PF_BK && N % 16 == 0 && M >= 1 && (bits == 8 || bits == 4) && (epi != PF_SILU || N % 32 == 0), MIS_ERR_GENERATION_FAILED,
-                "prefill GEMM on codes: bad shape");
+    MIS_REQUIRE(K % PF_BK == 0 && K >= PF_BK && N % 16 == 0 && M >= 1 && (bits == 8 || bits == 4) && (epi != PF_SILU || N % 32 == 0) && (int64_t)M * K < (1ll << 31),
+                MIS_ERR_GENERATION_FAILED, "prefill GEMM on codes: bad shape");
     PfGemmParams p{X, nullptr, C, M, N, K, PfExtra()};
     auto go = [&](auto e, auto t, auto gs, auto b) {
         constexpr int E = decltype(e)::value, T = decltype(t)::value, GS = decltype(gs)::value, B = decltype(b)::value;
@@ -634,9 +670,10 @@ void launch_gemm_pf_codes(int epi, int bits, const bf16_t* X, const void* Qp, co
         hipLaunchKernelGGL((k_gemm_pf_codes<E, T, T, GS, B>), dim3(nx >= 16 ? (int)round_up(nx, 8) : nx, cdiv(M, 32 * T)), dim3(256), 0, s, p, Qp, SB);
     };
     auto tile = [&](auto e, auto b) {
-        // Few blocks of 64 x 64 wait for a step's loads alone on their compute unit: more groups a step.  Orpheus-3B, 8 bits, us, 1 / 2 / 4 groups: o 160 rows (144
-        // blocks) 54 / - / 39, down 139 / - / 96; q|k|v 160 (240) 54 / - / 38, 272 (400) 54 / 44 / -, 416 (560) 57 / 78 / -; o 416 (336) 54 / 43 / -, 816 (624) 57 / 80 / -;
-        // gate | up 112 (512) 57 / 46 / -.  128 x 128: o 1632 rows (312 blocks) 96, gate | up 3216 (3328) 583: 550 TFLOP/s
+        // Few blocks of 64 x 64 wait for a step's loads alone on their compute unit: more groups a step.  Orpheus-3B, 8 bits, us, 1 / 2 / 4 groups (one chain of sums): o
+        // 160 rows (144 blocks) 54 / - / 39, down 139 / - / 96; q|k|v 160 (240) 54 / - / 38, 272 (400) 54 / 44 / -, 416 (560) 57 / 78 / -; o 416 (336) 54 / 43 / -, 816
+        // (624) 57 / 80 / -; gate | up 112 (512) 57 / 46 / -.  In quarters, by this rule: 36, 89; 36, 46, 57; 45, 56; 49.  128 x 128: o 1632 rows (312 blocks) 107,
+        // gate | up 3216 (3328) 641: 500 TFLOP/s
         const int64_t nb = (int64_t)cdiv(N, 64) * cdiv(M, 64);
         if ((int64_t)cdiv(N, 128) * cdiv(M, 128) >= 256) go(e, std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{}, b);
         else if (nb > 512) go(e, std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{}, b);

@@ -16,6 +16,9 @@
 //           codes instead of values: 8 bytes (uint2) per lane at 8 bit, 4 bytes at 4 bit (code e in bits [bits*e, bits*(e+1)))
 //   scales  [NT][G][2][16] bf16: scale then bias of rows 16nt .. 16nt+15 for scale group g (a lane reads its 4 C/D rows as 8 bytes)
 // Work decomposition, epilogues and the in-block split-K combine are those of k_gemm_skinny; K ranges are cut at scale groups.
+// A group's share of a sum is fma(scale, sum q x, bias * sum x), written out: contracted as the compiler likes, it was the other way round in some
+// unrolled copies of the loop and not in others, and a prompt's bits depended on how many rows shared its slice.  k_gemm_pf_codes (lm_prefill.hip) has the same.
+// (Four n-tiles per wave run decode steps only, where 16 and 32 rows agree.)
 #include "common.h"
 #include "lm_kernels.h"
 
@@ -247,7 +250,8 @@ __global__ void __launch_bounds__(KSB == 8 ? 512 : 256, 2) k_gemm_skinny_q(const
             unpack_bf16x4(SBUF[U][r][1], bi);                                                       \
             _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                       \
                 _Pragma("unroll") for (int e = 0; e < 4; ++e)                                       \
-                    acc[r][mt][e] += sc[e] * ag[r][mt][e] + bi[e] * sx[mt][e];                      \
+                    acc[r][mt][e] += R == 4 ? sc[e] * ag[r][mt][e] + bi[e] * sx[mt][e]              \
+                                            : fmaf(sc[e], ag[r][mt][e], bi[e] * sx[mt][e]);         \
         }                                                                                           \
     }
 #endif
@@ -439,7 +443,7 @@ __global__ void __launch_bounds__(256, 2) k_gemm_skinny_q1(const void* Qp, const
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[r][mt][e] += sc * ag[r][mt][e] + bi * sx[mt][e];
+                    for (int e = 0; e < 4; ++e) acc[r][mt][e] += fmaf(sc, ag[r][mt][e], bi * sx[mt][e]);
             }
             __builtin_amdgcn_sched_barrier(0);             // groups are consumed in the order their loads were issued (vmcnt is in order)
         }
