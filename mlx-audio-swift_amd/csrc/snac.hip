@@ -492,7 +492,7 @@ __global__ void __launch_bounds__(256) k_vq_nearest(const float* __restrict__ ze
     __syncthreads();
     if (tid == 0) {
         for (int w = 1; w < 4; ++w) if (redv[w] < best || (redv[w] == best && redi[w] < bi)) { best = redv[w]; bi = redi[w]; }
-        codes[(size_t)b * Tm + t] = bi;
+        codes[(size_t)b * Tm + t] = bi < CB ? bi : 0;              // no entry is nearest to a NaN: the first, as argmax has it
     }
 }
 // residual -= repeat_interleave(out_proj(codebook[code]), stride)   (VQ.swift:60-80,151-158); table [CB][C]
@@ -562,9 +562,10 @@ __global__ void __launch_bounds__(256) k_vq_level(VqLevel p) {
     best = redv[0]; bi = redi[0];
 #pragma unroll
     for (int w = 1; w < 4; ++w) if (redv[w] < best || (redv[w] == best && redi[w] < bi)) { best = redv[w]; bi = redi[w]; }
+    if (bi >= p.CB) bi = 0;                                   // (as k_vq_nearest)
     if (tid == 0) p.codes[(size_t)b * Tm + m] = bi;
     if (!p.dst) return;
-    const float* row = p.table + (size_t)min(bi, p.CB - 1) * p.C;          // (no entry is nearest to a NaN)
+    const float* row = p.table + (size_t)bi * p.C;
     float* y = p.dst + (size_t)b * p.C * p.T + (size_t)m * p.st;
     for (int c = tid; c < p.C; c += 256) {
         const float q = row[c];
