@@ -5,8 +5,8 @@
 // <= 2^-25 of the product).  One 16-deep step is 6 x 32 cycles instead of 8 x 64 of v_mfma_f32_32x32x2_f32.  Error against 64 bits (2-norm over 2-norm,
 // this kernel / the exact-f32 one; K = 96, 128, 192; operands normal): 1.38e-7 / 1.77e-7, 1.65e-7 / 2.06e-7, 2.04e-7 / 2.49e-7; all of one sign: 1.14 / 1.44,
 // 1.29 / 1.60, 1.64 / 2.05; normal times exp(2 normal): 1.25 / 1.93, 1.42 / 2.00, 1.84 / 2.45: lower each time (6 roundings of the sum per 16 products, not 16).
-// Infinities and values past the largest bfloat16: k_x6_gemm takes the outputs they reach again in f32, k_x6_convt (whose Snake may be the identity) clamps the first
-// plane.  Behind a Snake that is none, an argument past 1e20 is infinite or NaN in any arithmetic.  (An infinite WEIGHT of the units or the transposed
+// Infinities and values past the largest bfloat16: k_x6_gemm and the encoder's units take the outputs they reach again in f32, k_x6_convt (whose Snake may be the identity) clamps the first
+// plane.  Behind a Snake that is none, an argument past 1e20 is infinite or NaN in any arithmetic.  (An infinite WEIGHT of the decoder's units or the transposed
 // convolution gives NaN where the f32 kernels give an infinity or NaN.)
 //
 //   k_x6_pack_w   A^T f32 -> the three planes as MFMA-A fragments (once per weight matrix, kept in the model's CodecPack)
@@ -88,13 +88,15 @@ template <int C, bool DW, int KC, int NT>
 __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                            const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
                                            const float* __restrict__ pra1, const float* __restrict__ pa2, const float* __restrict__ pra2,
-                                           const uint16_t* __restrict__ pwp, const float* __restrict__ pb2, const PwScalars p) {
+                                           const uint16_t* __restrict__ pwp, const float* __restrict__ pAT, const float* __restrict__ pb2, const PwScalars p) {
     constexpr int KG = KC / 8, MT = (C + 31) / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
     constexpr int XR = KC / 4, GS = KG * (NT / 64) / 4, XS = NT + 2 * CODEC_DW_HALO + 2, NS = (XS + 61) / 64;      // (XS - 2 columns in strips of 64)
                                // rows of x and (group, strip) pairs per wave
     __shared__ float xs[DW ? KC : 1][DW ? XS : 1];
     __shared__ uint4 ts[3][KG][NT];
     __shared__ uint4 As[APC];
+    // The encoder's units take the place of k_x6_gemm in long rows only: a lane that sees a sum which is not finite takes its rows again as that kernel does
+    constexpr bool RETAKE = DW && C <= 96;
     constexpr bool SQ = C == 128;                         // 2 x 2 waves of 64 x 64; else every wave: all C rows x 32 columns
     constexpr int MTW = SQ ? 2 : MT, NTW = SQ ? NT / 64 : 1;
     static_assert(SQ || NT == 128, "four waves of 32 columns");
@@ -213,17 +215,43 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
         const int n = n0 + wc + ni * 32 + (lane & 31);
         if (n >= T) continue;
 #pragma unroll
-        for (int mi = 0; mi < MTW; ++mi)
+        for (int mi = 0; mi < MTW; ++mi) {
+            if constexpr (RETAKE) {
+                float zero = 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) zero = fmaf(acc[mi][ni][r], 0.0f, zero);
+                if (zero != 0.0f) {
+#pragma unroll 1
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = (wr + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
+                        if (m >= C) break;
+                        float v = 0.0f;
+#pragma unroll 1
+                        for (int c = 0; c < C && v == v; ++c) {            // (NaN it stays)
+                            float a = 0.0f;
+#pragma unroll 1
+                            for (int k = 0; k < 7; ++k) {
+                                const int t = n + (k - 3) * p.dil;
+                                a = fmaf(pw7[c * 7 + k], x6_snake(t >= 0 && t < T ? xb[(size_t)c * p.ldx + t] : 0.0f, pa1[c], pra1[c]), a);
+                            }
+                            v = fmaf(pAT[(size_t)c * C + m], x6_snake(a + pb1[c], pa2[c], pra2[c]), v);
+                        }
+                        yb[(size_t)m * p.ldy + n] = rb[(size_t)m * p.ldr + n] + (v + pb2[m]);
+                    }
+                    continue;
+                }
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = (wr + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5);
                 if (C % 32 == 0 || m < C) yb[(size_t)m * p.ldy + n] = rb[(size_t)m * p.ldr + n] + (acc[mi][ni][r] + pb2[m]);
             }
+        }
     }
 }
 template <int C, bool DW, int KC, int NT>
 __global__ void __launch_bounds__(256, KC == 32 ? 2 : DW && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp) {
-    pw_x6_body<C, DW, KC, NT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
+    pw_x6_body<C, DW, KC, NT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
 }
 
 // 128 channels, at most 256 blocks of 128 columns (a compute unit each, one serial chain of chunks): 64 columns per block.  96 blocks: 28 -> 22 us;
