@@ -503,74 +503,135 @@ __global__ void k_vq_residual(float* __restrict__ r, const int32_t* __restrict__
     r[((size_t)b * C + c) * T + t] -= table[(size_t)code * C + c];
 }
 
-// One level of the residual quantiser (codebook_dim 8) in one launch: a block owns a code's `st` columns - their mean, the projection (a T, [C][8]), the nearest
-// entry as in k_vq_nearest, and the residual without it (dst; not written behind the last level).  Each of the four kernels this takes the place of was one
-// dependent round trip on few blocks: 74, 148 and 296 codes of 768 channels 14.4, 12.7 and 8.0 us, the four kernels 41, 39 and 31 without the waits between them.
+// One level of the residual quantiser (codebook_dim 8) in one launch: a block owns the `st` columns of NB neighbouring codes - their means, the projection (a T,
+// [C][8]), the nearest entry as in k_vq_nearest, and the residual without it (dst; not written behind the last level).  A code's sums are the same for either NB.
+// Few codes, one a block: each of the four kernels this takes the place of was one dependent round trip on few blocks: 74, 148 and 296 codes of 768 channels 14.4,
+// 12.7 and 8.0 us, the four kernels 41, 39 and 31 without the waits between them.  Many codes, VQ_MANY a block: bound by the 64 bytes that a code's column costs in every
+// channel's row and by the codebook's way from L2, so neighbours share both, and an XCD takes one range of codes.  A row of ten minutes (7032, 14064 and 28128 codes of
+// strides 4, 2 and 1), us: one a block over all XCDs 760, 612, 262, here 236, 207, 122, the four kernels 143, 188, 211.
 struct VqLevel {
     const float *src; float* dst;
     const float *at, *bias, *cn, *cn2, *table;
     int32_t* codes;
-    int C, T, st, CB;
+    int C, T, st, CB, nblk, batch;        // nblk: blocks a row
 };
+#define VQ_MANY 4
+template <int NB>
 __global__ void __launch_bounds__(256) k_vq_level(VqLevel p) {
-    __shared__ float part[4][8];
-    __shared__ float redv[4];
-    __shared__ int redi[4];
-    const int m = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, Tm = p.T / p.st;
-    const float* x = p.src + (size_t)b * p.C * p.T + (size_t)m * p.st;
-    float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    __shared__ float part[4][NB][8];
+    __shared__ float redv[4][NB];
+    __shared__ int redi[4][NB];
+    const int tid = threadIdx.x, wave = tid >> 6, Tm = p.T / p.st, per = (p.nblk * p.batch + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (id >= p.nblk * p.batch) return;
+    const int b = id / p.nblk, m0 = (id - b * p.nblk) * NB;
+    const float* x = p.src + (size_t)b * p.C * p.T;
+    int col[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) col[i] = min(m0 + i, Tm - 1) * p.st;          // (codes past the row: the last one again, not stored)
+    float e[NB][8];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int d = 0; d < 8; ++d) e[i][d] = 0.0f;
     for (int c = tid; c < p.C; c += 256) {
-        float v = 0.0f;
-        for (int j = 0; j < p.st; ++j) v += x[(size_t)c * p.T + j];
-        if (p.st > 1) v /= (float)p.st;
+        const float* r = x + (size_t)c * p.T;
+        float v[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) v[i] = 0.0f;
+        for (int j = 0; j < p.st; ++j)
+#pragma unroll
+            for (int i = 0; i < NB; ++i) v[i] += r[col[i] + j];
+        if (p.st > 1)
+#pragma unroll
+            for (int i = 0; i < NB; ++i) v[i] /= (float)p.st;
         const float4 lo = *reinterpret_cast<const float4*>(p.at + (size_t)c * 8), hi = *reinterpret_cast<const float4*>(p.at + (size_t)c * 8 + 4);
-        e[0] = fmaf(lo.x, v, e[0]); e[1] = fmaf(lo.y, v, e[1]); e[2] = fmaf(lo.z, v, e[2]); e[3] = fmaf(lo.w, v, e[3]);
-        e[4] = fmaf(hi.x, v, e[4]); e[5] = fmaf(hi.y, v, e[5]); e[6] = fmaf(hi.z, v, e[6]); e[7] = fmaf(hi.w, v, e[7]);
+        const float a[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int d = 0; d < 8; ++d) e[i][d] = fmaf(a[d], v[i], e[i][d]);
     }
 #pragma unroll
-    for (int d = 0; d < 8; ++d) {
-        const float t = wave_sum_dpp(e[d]);
-        if ((tid & 63) == 0) part[wave][d] = t;
-    }
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int d = 0; d < 8; ++d) {
+            const float t = wave_sum_dpp(e[i][d]);
+            if ((tid & 63) == 0) part[wave][i][d] = t;
+        }
     __syncthreads();
-    float n2 = 0.0f, en2 = 0.0f;
+    float en2[NB], best[NB];
+    int bi[NB];
 #pragma unroll
-    for (int d = 0; d < 8; ++d) { e[d] = ((part[0][d] + part[1][d]) + (part[2][d] + part[3][d])) + p.bias[d]; n2 += e[d] * e[d]; }
-    const float inv = 1.0f / fmaxf(sqrtf(n2), 1e-12f);
+    for (int i = 0; i < NB; ++i) {
+        float n2 = 0.0f;
+        en2[i] = 0.0f;
 #pragma unroll
-    for (int d = 0; d < 8; ++d) { e[d] *= inv; en2 += e[d] * e[d]; }
-    float best = INFINITY;
-    int bi = 0x7fffffff;
+        for (int d = 0; d < 8; ++d) { e[i][d] = ((part[0][i][d] + part[1][i][d]) + (part[2][i][d] + part[3][i][d])) + p.bias[d]; n2 = fmaf(e[i][d], e[i][d], n2); }
+        const float inv = 1.0f / fmaxf(sqrtf(n2), 1e-12f);
+#pragma unroll
+        for (int d = 0; d < 8; ++d) { e[i][d] *= inv; en2[i] = fmaf(e[i][d], e[i][d], en2[i]); }
+        best[i] = INFINITY;
+        bi[i] = 0x7fffffff;
+    }
 #pragma unroll 4
     for (int k = tid; k < p.CB; k += 256) {
         const float4 lo = *reinterpret_cast<const float4*>(p.cn + (size_t)k * 8), hi = *reinterpret_cast<const float4*>(p.cn + (size_t)k * 8 + 4);
-        const float q[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        float dot = 0.0f;
+        const float q[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w}, c2 = p.cn2[k];
 #pragma unroll
-        for (int d = 0; d < 8; ++d) dot += e[d] * q[d];
-        const float dist = en2 - 2.0f * dot + p.cn2[k];
-        if (dist < best) { best = dist; bi = k; }
+        for (int i = 0; i < NB; ++i) {
+            float dot = 0.0f;
+#pragma unroll
+            for (int d = 0; d < 8; ++d) dot = fmaf(e[i][d], q[d], dot);
+            const float dist = fmaf(-2.0f, dot, en2[i]) + c2;
+            if (dist < best[i]) { best[i] = dist; bi[i] = k; }
+        }
     }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ob = __shfl_xor(best, o, 64);
-        const int oi = __shfl_xor(bi, o, 64);
-        if (ob < best || (ob == best && oi < bi)) { best = ob; bi = oi; }
+    for (int i = 0; i < NB; ++i) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const float ob = __shfl_xor(best[i], o, 64);
+            const int oi = __shfl_xor(bi[i], o, 64);
+            if (ob < best[i] || (ob == best[i] && oi < bi[i])) { best[i] = ob; bi[i] = oi; }
+        }
+        if ((tid & 63) == 0) { redv[wave][i] = best[i]; redi[wave][i] = bi[i]; }
     }
-    if ((tid & 63) == 0) { redv[wave] = best; redi[wave] = bi; }
     __syncthreads();
-    best = redv[0]; bi = redi[0];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) if (redv[w] < best || (redv[w] == best && redi[w] < bi)) { best = redv[w]; bi = redi[w]; }
-    if (bi >= p.CB) bi = 0;                                   // (as k_vq_nearest)
-    if (tid == 0) p.codes[(size_t)b * Tm + m] = bi;
-    if (!p.dst) return;
-    const float* row = p.table + (size_t)bi * p.C;
-    float* y = p.dst + (size_t)b * p.C * p.T + (size_t)m * p.st;
-    for (int c = tid; c < p.C; c += 256) {
-        const float q = row[c];
-        for (int j = 0; j < p.st; ++j) y[(size_t)c * p.T + j] = x[(size_t)c * p.T + j] - q;
+    for (int i = 0; i < NB; ++i) {
+        best[i] = redv[0][i]; bi[i] = redi[0][i];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) if (redv[w][i] < best[i] || (redv[w][i] == best[i] && redi[w][i] < bi[i])) { best[i] = redv[w][i]; bi[i] = redi[w][i]; }
+        if (bi[i] >= p.CB) bi[i] = 0;                         // (as k_vq_nearest)
+        if (tid == 0 && m0 + i < Tm) p.codes[(size_t)b * Tm + m0 + i] = bi[i];
     }
+    if (!p.dst) return;
+    float* y = p.dst + (size_t)b * p.C * p.T;
+    const int n = min(NB, Tm - m0);
+    for (int c = tid; c < p.C; c += 256) {
+        float q[NB];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) q[i] = p.table[(size_t)bi[i] * p.C + c];
+        const size_t o = (size_t)c * p.T;
+        for (int j = 0; j < p.st; ++j) {
+            float v[NB];
+#pragma unroll
+            for (int i = 0; i < NB; ++i) v[i] = x[o + col[i] + j];
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+                if (i < n) y[o + col[i] + j] = v[i] - q[i];
+        }
+    }
+}
+static void launch_vq_level(VqLevel p, int batch, hipStream_t s) {
+    const int Tm = p.T / p.st;
+    // us, one / four codes a block: 1172 codes of stride 4, 2, 1 53 / 57, 35 / 40, 16 / 21; about 1600 - / -, 48 / 41, 21 / 22; 2344 104 / 92, 64 / 53, 27 / 24
+    const bool many = (int64_t)Tm * batch > 1536;
+    p.nblk = many ? cdiv(Tm, VQ_MANY) : Tm;
+    p.batch = batch;
+    const dim3 grid((unsigned)round_up((size_t)p.nblk * batch, 8));
+    if (many) hipLaunchKernelGGL(k_vq_level<VQ_MANY>, grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL(k_vq_level<1>, grid, dim3(256), 0, s, p);
 }
 
 // ---- dense k-tap conv on f32 MFMA (Qwen3-TTS / DAC-style decoders: dilated k7 convs with Cin = Cout up to 1536) ---------
@@ -1216,8 +1277,8 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
         const auto& q = c->vq_enc[i];
         const float* table = W + c->tables_off + (size_t)i * cf.codebook_size * D;
         if (one) {
-            VqLevel v{i ? f2 : f1, last ? nullptr : f2, W + q.in_proj.w, W + q.in_proj.b, W + q.cn, W + q.cn2, table, codes, D, (int)T, st, cf.codebook_size};
-            hipLaunchKernelGGL(k_vq_level, dim3(Tm, batch), dim3(256), 0, s, v);
+            VqLevel v{i ? f2 : f1, last ? nullptr : f2, W + q.in_proj.w, W + q.in_proj.b, W + q.cn, W + q.cn2, table, codes, D, (int)T, st, cf.codebook_size, 0, 0};
+            launch_vq_level(v, batch, s);
         } else {
             if (i == 0) HIP_CHECK(hipMemcpyAsync(f2, f1, (size_t)batch * D * T * 4, hipMemcpyDeviceToDevice, s));
             const float* pooled = f2;

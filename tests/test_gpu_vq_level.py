@@ -27,3 +27,16 @@ def test_codes_are_the_nearest_entries(dim, enc, entries, strides, rows, samples
         assert np.array_equal(got[open_row][sure[open_row]], want[open_row][sure[open_row]])
         open_row &= (got == want).all(-1)
     assert open_row.mean() > 0.5
+
+
+# From 1537 codes of a level on a block owns four neighbours (the last block of a row fewer): the codes that a row has alone, one code a block
+@pytest.mark.parametrize("strides, rows, samples", [([4, 2, 1], 17, 1617), ([1], 3, 9511), ([6, 3, 2, 1], 29, 1137)])
+def test_codes_do_not_depend_on_the_codes_of_a_block(strides, rows, samples):
+    cfg = dict(encoder_dim=24, encoder_rates=[2, 2, 2, 2], decoder_dim=32, decoder_rates=[2, 2, 2, 2], codebook_size=700, codebook_dim=8, vq_strides=strides)
+    dev = mas.SNAC.from_weights(mas.SNACConfig(**cfg), osnac.make_synthetic_weights(osnac.SnacConfig(**cfg), seed=5, with_encoder=True))
+    audio = (0.3 * np.random.default_rng(rows).standard_normal((rows, samples))).astype(np.float32)
+    many, z = dev.encode(audio, return_latent=True)
+    assert many[-1].size > 1536
+    for b in range(rows):
+        alone, za = dev.encode(audio[b:b + 1], return_latent=True)
+        assert np.array_equal(za[0], z[b]) and all(np.array_equal(a[0], m[b]) for a, m in zip(alone, many)), b
