@@ -899,7 +899,7 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     for (int t0 = 0; t0 < Lmax; t0 += Tc) most = std::max(most, rows_of(t0, std::min(Tc, Lmax - t0)));
     const size_t Mc = round_up((size_t)most, 16);                            // GEMM rows round up to 16
     c->pf_h.alloc(Mc * d); c->pf_x.alloc(Mc * d); c->pf_attn.alloc(Mc * HD);
-    c->pf_q.alloc(Mc * HD); c->pf_pos.alloc(Mc); c->pf_on.alloc(Mc);
+    c->pf_q.alloc(Mc * HD);
     // quantised checkpoints (every role streamed as codes): k_gemm_pf_codes on the chunk's rows; a chunk of few rows runs the decode step's k_gemm_skinny_q on
     // 64-row slices - rows packed into MFMA fragments first, float32 sums out, the residual add as its own small kernel; gate|up writes the
     // packed activation its down projection reads.  The weights are streamed once per 64 rows instead of once per position.
@@ -929,9 +929,8 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
             HIP_CHECK(hipMemsetAsync(c->pf_h.p + (size_t)Mr * d, 0, (size_t)(M - Mr) * d * 2, s));
             HIP_CHECK(hipMemsetAsync(c->pf_attn.p + (size_t)Mr * HD, 0, (size_t)(M - Mr) * HD * 2, s));
         }
-        if (embed_rows) launch_pf_rows_rmsnorm(embed_rows, Mpad, lens_dev, Lmax, t0, tc, batch, 0, c->norms.p, c->pf_h.p, c->pf_x.p, c->pf_pos.p, c->pf_on.p, Mr, d, eps, s);
-        else launch_pf_embed_rmsnorm(c->emb.p, prompt_mat_dev, lens_dev, Lmax, t0, tc, batch, 0, c->V, c->norms.p, c->pf_h.p, c->pf_x.p,
-                                     c->pf_pos.p, c->pf_on.p, Mr, d, eps, s);
+        if (embed_rows) launch_pf_rows_rmsnorm(embed_rows, Mpad, lens_dev, Lmax, t0, tc, batch, 0, c->norms.p, c->pf_h.p, c->pf_x.p, nullptr, nullptr, Mr, d, eps, s);
+        else launch_pf_embed_rmsnorm(c->emb.p, prompt_mat_dev, lens_dev, Lmax, t0, tc, batch, 0, c->V, c->norms.p, c->pf_h.p, c->pf_x.p, nullptr, nullptr, Mr, d, eps, s);
         for (int li = 0; li < c->L; ++li) {
             if (tiled) q_tiled(PF_F32, c->q_qkv, li, c->pf_x.p, c->pf_qkv.p, M, c->Nqkv, d);
             else if (coded) q_rows(M, [&](int r0, int mp) {

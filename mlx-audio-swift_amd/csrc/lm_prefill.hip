@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(256) k_pf_embed_rmsnorm(const bf16_t* __restri
     const int r = blockIdx.x;
     int b, t;
     const bool on = pf_row(lens, r, Lmax, t0, tc, batch, Mpad, b, t);
-    if (threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - lens[b]) : 0; act_tab[r] = on ? 1 : 0; }
+    if (pos_tab && threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - lens[b]) : 0; act_tab[r] = on ? 1 : 0; }
     int id = on ? prompt[(size_t)b * Lmax + t] : -1;
     if (id >= vocab) id = -1;
     const bf16_t* e = emb + (size_t)(id < 0 ? 0 : id) * d;
@@ -105,7 +105,7 @@ __global__ void __launch_bounds__(256) k_pf_rows_rmsnorm(const bf16_t* __restric
     const int r = blockIdx.x;
     int b, t;
     const bool on = pf_row(lens, r, Lmax, t0, tc, batch, Mpad, b, t);
-    if (threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - lens[b]) : 0; act_tab[r] = on ? 1 : 0; }
+    if (pos_tab && threadIdx.x == 0) { pos_tab[r] = on ? t - (Lmax - lens[b]) : 0; act_tab[r] = on ? 1 : 0; }
     const bf16_t* e = rows + ((size_t)t * src_rows + b) * d;                   // the caller's matrix keeps its own rows per position
     float ss = 0.0f;
     for (int i = threadIdx.x; i < d; i += 256) {
