@@ -793,7 +793,7 @@ static void enqueue_lm_head(mis_tts* c, const bf16_t* head = nullptr) {
 static bool prefill_batched_ok(const mis_tts* c, int Lmax) {
     const bool off = getenv("MIS_PREFILL_SEQ") && atoi(getenv("MIS_PREFILL_SEQ")) != 0;             // A/B and parity tests (read per call)
     const int HD = c->H * c->D;
-    // dense weights: k_gemm_pf; all four roles streamed as codes: the decode step's k_gemm_skinny_q on 64-row chunks; a mix: position by position
+    // dense weights: k_gemm_pf and its forms; all four roles streamed as codes: k_gemm_pf_codes or slices of k_gemm_skinny_q; a mix: position by position
     const bool dense = !c->q_qkv.on && !c->q_o.on && !c->q_gu.on && !c->q_down.on;
     const bool coded = c->q_qkv.on && c->q_o.on && c->q_gu.on && c->q_down.on;
     return !off && Lmax >= 2 && (dense || coded) && c->d % 64 == 0 && HD % 64 == 0 && c->ff % 64 == 0 && c->d >= 128 && HD >= 128 && c->ff >= 128;

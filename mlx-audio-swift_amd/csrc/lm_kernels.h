@@ -68,8 +68,9 @@ enum { PF_F32 = 0, PF_RESID = 1, PF_SILU = 2,
        PF_ACT_ROWS = 8 };        // bf16 row-major [M][ldc]: T(silu(y)) in the tiles below PfExtra::split, T(sigmoid(y)) in the others
 struct PfExtra { int ldx = 0; const int32_t* xrow = nullptr; int ldc = 0; void* out2 = nullptr; int split = 0, ld2 = 0; const bf16_t* ls = nullptr; float scale = 1.0f, cap = 0.0f; };
 void launch_gemm_pf(int epi, const bf16_t* X, const bf16_t* Wp, void* C, int M, int N, int K, hipStream_t s, const PfExtra& ex = PfExtra());
-// the same on codes and scales (lm_qgemm.hip): PF_F32, PF_RESID, PF_SILU
+// the same on codes and scales in the layouts of lm_qgemm.hip: PF_F32, PF_RESID, PF_SILU
 void launch_gemm_pf_codes(int epi, int bits, const bf16_t* X, const void* Qp, const bf16_t* SB, void* C, int M, int N, int K, hipStream_t s);
+// pos_tab, act_tab: null, or position and activity of every row (the short-prompt form)
 void launch_pf_embed_rmsnorm(const bf16_t* emb, const int32_t* prompt, const int32_t* lens, int Lmax, int t0, int Tc, int batch, int Mpad, int vocab,
                              const bf16_t* wnorm, bf16_t* h, bf16_t* x, int32_t* pos_tab, uint8_t* act_tab, int rows, int d, float eps, hipStream_t s);
 void launch_pf_pack_last(const bf16_t* rows, const int32_t* lens, int Lmax, int t0, int Tc, int batch, bf16_t* xpk, int Mpad, int d, hipStream_t s);
@@ -80,7 +81,7 @@ void launch_pf_rmsnorm(const bf16_t* h, const bf16_t* wnorm, bf16_t* x, int rows
 void launch_pf_pack_rows(const bf16_t* rows, bf16_t* xpk, int Mpad, int d, hipStream_t s);
 
 // causal attention of the chunk of positions [t0, t0 + tc) of `batch` left-padded prompts (packed rows: the positions of sequence 0, of sequence 1, ...; lens: device): q|k|v -> norm, rotation,
-// cache append, attention over the caches.  q: scratch for the roped queries, out: bf16 [rows][H D] 
+// cache append, attention over the caches.  q: scratch for the roped queries, out: bf16 [rows][H D]
 struct PfAttn {
     const void* qkv; int qkv_f32;            // [rows][Nqkv] float32 or bf16
     bf16_t *q, *out;

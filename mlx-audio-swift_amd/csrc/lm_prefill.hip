@@ -8,7 +8,7 @@
 // caches.  Rows are PACKED: the chunk's positions of sequence 0, then those of sequence 1, ... - no row stands for the padding of a shorter prompt
 // (prompts of 300 .. 450 tokens padded to 450: 15 % of every GEMM).
 //
-//   k_pf_embed_rmsnorm  h[r] = E[token(b, t)], x[r] = RMSNorm(h[r]) (row-major), active / position tables of every (t, b)
+//   k_pf_embed_rmsnorm  h[r] = E[token(b, t)], x[r] = RMSNorm(h[r]) (row-major); active / position tables for the short-prompt form
 //   k_gemm_pf<EPI>      C[M][N] = X[M][K] . W^T with W in the decode path's packed MFMA-A tile layout [N/16][K/32][64][8]:
 //                       a weight fragment is one 1 KiB global_load_lds piece and its LDS image IS the A fragment (lane-linear:
 //                       ds_read_b128 at lane*16, conflict free); X tiles as in k_gemm_big2 (whisper_kernels.hip: source-side
@@ -16,10 +16,14 @@
 //                         PF_ROWS_BF16  T(acc) [M][N]                    (q|k|v)
 //                         PF_RESID  h = T(h + T(acc)) in place, bf16      (o_proj, down_proj: LlamaTTS.swift:306-309)
 //                         PF_SILU   act = T(T(g T(sigmoid g)) u), gate / up tiles interleaved as packed (:283)
+//   k_gemm_pf_wide      the same on tiles of 128 .. 192 x 256, four waves (gemm_tiles.h): many rows
+//   k_gemm_pf_ring      the same on tiles of 32 x 32: few rows
+//   k_gemm_pf_codes     the same on 8- and 4-bit codes, more than 96 rows (fewer: k_gemm_skinny_q, lm_qgemm.hip, the same bits)
 //   k_pf_rope_append    q|k|v of the chunk -> roped queries (bf16 rows) and the tiled K / V caches of the decode step
 //   k_pf_attn           causal attention of the chunk's queries over the caches (MFMA, K / V tiles shared by 128 or 256 queries)
 //   k_pf_rmsnorm        x[r] = RMSNorm(h[r]) row-major
-//   k_pf_pack_rows      rows of the last position -> the packed x operand of the decode step (lm_head of the first new token)
+//   k_pf_pack_last      every sequence's last row -> the packed x operand of the decode step (lm_head of the first new token)
+//   k_pf_pack_rows      rows -> packed x operand of a slice of k_gemm_skinny_q
 // Rounding points are those of the decode step (bf16 at every MLX primitive boundary); only float32 summation orders differ.
 #include "common.h"
 #include "gemm_tiles.h"

@@ -477,10 +477,10 @@ static bool launch_big3(const BigGemmParams& p, hipStream_t s) {
 // ---------------------------------------------------------------------------- tiles of 32 TM x 256 outputs, four waves (gemm_tiles.h)
 // What it gives over k_gemm_big3 (large-v3, us per launch): 8 x 1500 rows q|k|v 122 / 140, o 55 / 60, fc1 171 / 211, fc2 146 / 172, cross k|v 88 / 101; 6 x 1500
 // (k_gemm_big2 where 180 tiles of 256 x 256 were too few) 100 / 128, 44 / 58, 128 / 159, 122 / 173, 66 / 90; 4 x 1500 71 / 89, 33 / 34, 93 / 107, 85 / 95, 45 / 50.
-// k_gemm_big3 keeps what these offsets or rings cannot hold.
+// k_gemm_big3 keeps K = 128 (the ring takes three k-steps) and operands past 32-bit offsets; no size of the family has either.
 // TM by the rounds of 256 persistent blocks it makes (launch_gemm_rows).  Products in the order of k: the bits of k_gemm_big2.
 // A GELU after T(xW^T + b) is a function of sixteen bits: gelu_erf_w(v) = v f(v), f in an LDS table over |v| = 2^-10 .. 16 and the sign (14 KB; below 2^-10 the
-// result is v / 2, above 16 it is v or -0: the values that the clamped factors round to).  The same bits as the formula, in 12 instructions an
+// result is v / 2, exact from 2^-125 on, above 16 it is v or -0: the values that the clamped factors round to).  The same bits as the formula, in 12 instructions an
 // output and an LDS read for 31, two of them of quarter rate - a block's only waves wait for them.  fc1, eight windows 204 -> 171 us, one 31 -> 28.
 struct GeluTable {
     static constexpr uint32_t LO = 0x3a80, HI = 0x4180, N = HI - LO + 1;           // bf16 of 2^-10 and 16
