@@ -8,8 +8,10 @@ from oracle import llama as ollama
 pytestmark = pytest.mark.gpu
 
 
-# rows in all: 2500 .. 4090 of the largest chunk; N = 640 / 1088 / 2432 (not whole 256-column tiles), K = 192 (three k-steps), 384, 1088, 1216
-@pytest.mark.parametrize("hidden, heads, ff, total", [(1088, 3, 1216, 2500), (1088, 3, 1216, 3333), (1088, 3, 1216, 4090), (192, 8, 1216, 4075)])
+# rows in all: 2500 .. 4090 of the largest chunk; N = 640 / 1088 / 2432 (not whole 256-column tiles), K = 192 (three k-steps), 384, 1088, 1216: the 128 x 128 tiles where K is
+# short and their blocks few, the others here.  2112 wide: every product here, on 128 rows a tile (1333), 160 (3333) and 192 (4090)
+@pytest.mark.parametrize("hidden, heads, ff, total", [(1088, 3, 1216, 2500), (1088, 3, 1216, 3333), (1088, 3, 1216, 4090), (192, 8, 1216, 4075), (2112, 16, 1216, 1333),
+                                                      (2112, 16, 1216, 3333), (2112, 16, 1216, 4090)])
 def test_rows_of_ragged_prompts_have_the_bits_they_have_alone(hidden, heads, ff, total):
     from gpu_util import logits_errors
     from test_gpu_lm import lm_pair
