@@ -67,7 +67,7 @@ struct mis_tts {
     DevBuf<float> rope_cos, rope_sin;
     DevBuf<int32_t> ids, pos_cur, pos_next;
     DevBuf<uint8_t> active;
-    DevBuf<bf16_t> h, h2, x, attn_out, act, logits;      // h2: the other residual buffer of the folded glue (enqueue_layers)
+    DevBuf<bf16_t> h, x, attn_out, act, logits;          // h: two buffers [Mpad][d], the second one for the folded glue (enqueue_layers)
     DevBuf<float> qkv_part, part, e_buf, logits_f32, samp_l32;
     // generation state
     DevBuf<int32_t> prompt_mat, prompt_lens, step_counter, window, window_len, n_gen, tokens_out, all_ids, all_len,
@@ -683,13 +683,13 @@ static void lm_reset_buffers(mis_tts* c, int batch, int max_context) {
     if (new_tables || !c->rope_cos.p) build_rope_tables(c);
     c->ids.alloc(Mpad); c->pos_cur.alloc(Mpad); c->pos_next.alloc(Mpad); c->active.alloc(Mpad);
     c->ids.zero(s); c->pos_cur.zero(s); c->pos_next.zero(s); c->active.zero(s);
-    c->h.alloc((size_t)Mpad * d); c->h2.alloc((size_t)Mpad * d); c->x.alloc((size_t)Mpad * d);
+    c->h.alloc((size_t)2 * Mpad * d); c->x.alloc((size_t)Mpad * d);
     c->attn_out.alloc((size_t)Mpad * HD); c->act.alloc((size_t)Mpad * c->ff);
     c->logits.alloc((size_t)Mpad * c->Vpad);
     c->e_buf.alloc((size_t)Mpad * c->Vpad);
     c->qkv_part.alloc((size_t)c->S_qkv * Mpad * c->Nqkv);
     c->part.alloc((size_t)std::max(c->S_o, c->S_down) * Mpad * d);
-    c->h.zero(s); c->h2.zero(s); c->x.zero(s); c->attn_out.zero(s); c->act.zero(s); c->logits.zero(s);
+    c->h.zero(s); c->x.zero(s); c->attn_out.zero(s); c->act.zero(s); c->logits.zero(s);
     HIP_CHECK(hipStreamSynchronize(s));
 }
 
@@ -736,7 +736,7 @@ static void enqueue_layers(mis_tts* c, const bf16_t* table = nullptr, int table_
     const float eps = c->cfg.rms_norm_eps;
     // a folded glue leaves the new residual stream in the other buffer: begun so that the last one is c->h
     const bool f_gu = fold_gate_up(c), f_qkv = fold_qkv(c);
-    bf16_t *hcur = c->h.p, *hoth = c->h2.p;
+    bf16_t *hcur = c->h.p, *hoth = c->h.p + (size_t)Mpad * d;
     if (((f_gu ? c->L : 0) + (f_qkv ? c->L - 1 : 0)) & 1) std::swap(hcur, hoth);
     launch_embed_rmsnorm(table ? table : c->emb.p, ids ? ids : c->ids.p, c->active.p, c->pos_cur.p, c->pos_next.p, c->norms.p,
                          hcur, c->x.p, d, table ? table_rows : c->V, eps, c->batch, Mpad, s);
@@ -1461,7 +1461,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         uint64_t key = 1469598103934665603ull;
         auto mix = [&](const void* p, size_t n) { const unsigned char* q = (const unsigned char*)p; for (size_t i = 0; i < n; ++i) { key ^= q[i]; key *= 1099511628211ull; } };
         mix(&sp, sizeof(sp));
-        const void* ptrs[] = {c->prompt_mat.p, c->prompt_lens.p, c->step_counter.p, c->ids.p, c->active.p, c->h.p, c->h2.p, c->x.p,
+        const void* ptrs[] = {c->prompt_mat.p, c->prompt_lens.p, c->step_counter.p, c->ids.p, c->active.p, c->h.p, c->x.p,
                               c->attn_out.p, c->act.p, c->logits.p, c->qkv_part.p, c->part.p, c->kcache.p, c->vtcache.p,
                               c->rope_cos.p, c->rope_sin.p, c->pos_cur.p, c->pos_next.p};
         mix(ptrs, sizeof(ptrs));
