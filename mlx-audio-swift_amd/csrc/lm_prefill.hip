@@ -398,11 +398,10 @@ static bool launch_gemm_pf_wide(const PfGemmParams& p, hipStream_t s) {
     // A block fills its ring and drains its last tile alone on its compute unit; k_gemm_pf has two, and is faster where K is short and its blocks are all there at
     // once, or in one and a half rounds against two.  us, k_gemm_pf / here: gate | up (N = 6144) K = 1024, 300 rows (144 blocks) 15 / 17, 1200 (480) 20 / 21, 1536
     // (576; 240 tiles) 31 / 25, 2048 (768; 384) 34 / 37; q|k|v (N = 4096) K = 1024, 600 rows 14 / 17, 2048 22 / 23, 2400 33 / 26; K = 512 (N = 4096), 900 rows 11 / 14, 3200
-    // (800; 400) 23 / 25; K = 1536: N = 2048, 1200 rows (160) 24 / 26, 2816 (352) 29 / 27, N = 17920, 384 (420) 30 / 29, 608 (700; 350) 49 / 52; K = 2048, N = 1024, 2048 rows
-    // (128) 29 / 33, N = 2048, 2048 (256) 36 / 34
+    // (800; 400) 23 / 25; K = 1536: N = 2048, 1200 rows (160) 24 / 26, 2816 (352) 29 / 27, N = 17920, 384 (420) 30 / 29, 608 (700; 350) 49 / 52; K = 2048, N = 1024, 1500 rows
+    // (96) 32 / 31, N = 2048, 1800 (240) 35 / 35, 2816 40 / 36
     const int nx = cdiv(p.N, PF_BN), blocks = (nx >= 16 ? (int)round_up(nx, 8) : nx) * cdiv(p.M, PF_BM), rounds = cdiv(nt * cdiv(p.M, 32 * best), 256);
     if (p.K <= 1536 && (blocks <= (p.K <= 1024 ? 512 : 256) || (rounds > 1 && blocks <= (p.K <= 512 ? 1024 : 768)))) return false;
-    if (p.K <= 2048 && blocks <= 128) return false;
     auto go = [&](auto tag) {
         constexpr int TM = decltype(tag)::value;
         const int mt = cdiv(p.M, 32 * TM), tiles = mt * nt;
