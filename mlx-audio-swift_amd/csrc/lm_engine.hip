@@ -905,7 +905,9 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     // packed activation its down projection reads.  The weights are streamed once per 64 rows instead of once per position.
     const bool coded = c->q_qkv.on;
     if (coded) c->pf_qkv.alloc(Mc * c->Nqkv); else c->pf_qkv16.alloc(Mc * c->Nqkv);
-    const bool tiled = coded && Mc > 96;                                      // (90 rows: 5.9 ms in slices, 7.3 tiled; 107: 8.3, 7.3; the same bits)
+    // (the same bits.  A second slice costs less than the tiles while gate | up has more of them than compute units for two slices' rows; us for 3 - 4 layers at 8 bits,
+    // slices / tiles: width 3072, 90 rows 770 / 910, 113 820 / 920, 129 (three slices) 1014 / 1049, 161 1076 / 1059; 2048, 113 850 / 890, 129 1053 / 913; 1024, 113 667 / 639)
+    const bool tiled = coded && Mc > (2 * cdiv(2 * c->ff, 64) > 256 ? 128u : 96u);
     if (coded && !tiled) { c->pf_xpk.alloc((size_t)64 * std::max(d, HD)); c->pf_actpk.alloc((size_t)64 * c->ff); c->pf_tmp.alloc((size_t)64 * d); }
     else c->pf_act.alloc(Mc * c->ff);
     auto q_tiled = [&](int epi, const mis_tts::QRole& q, int li, const bf16_t* x, void* out, int M, int N, int K) {

@@ -18,7 +18,7 @@
 //                         PF_SILU   act = T(T(g T(sigmoid g)) u), gate / up tiles interleaved as packed (:283)
 //   k_gemm_pf_wide      the same on tiles of 128 .. 192 x 256, four waves (gemm_tiles.h): many rows
 //   k_gemm_pf_ring      the same on tiles of 32 x 32: few rows
-//   k_gemm_pf_codes     the same on 8- and 4-bit codes, more than 96 rows (fewer: k_gemm_skinny_q, lm_qgemm.hip, the same bits)
+//   k_gemm_pf_codes     the same on 8- and 4-bit codes, more than 96 or 128 rows (fewer: k_gemm_skinny_q, lm_qgemm.hip, the same bits)
 //   k_pf_rope_append    q|k|v of the chunk -> roped queries (bf16 rows) and the tiled K / V caches of the decode step
 //   k_pf_attn           causal attention of the chunk's queries over the caches (MFMA, K / V tiles shared by 128 or 256 queries)
 //   k_pf_rmsnorm        x[r] = RMSNorm(h[r]) row-major
@@ -496,8 +496,8 @@ __global__ void __launch_bounds__(128) k_gemm_pf_ring(PfGemmParams p) {
 // ahead, one barrier.  Bound: a group costs an output a product, an FMA and an addition beside its 64 products - VALU above matrix pipe, two blocks a compute unit
 // share both.  (Two FMAs into one chain of sums are 10 % faster at 128 x 128 - gate | up of 3216 rows 583 us, 641 here - but then a prompt's bits depend on the
 // other prompts of its call, which decide between slices and tiles.)
-// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 70 rows 5.7 / 7.3, 90 5.9 / 7.3, 107 8.3 / 7.3, 175 10.8 / 8.6, 274 15.8 / 9.4, 413 21.0 / 10.6,
-// 804 38.4 / 16.2, 3202 151 / 46.6.
+// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 70 rows 5.7 / 7.3, 107 6.1 / 7.3, 175 8.7 / 8.6, 274 13.8 / 9.4, 413 18.5 / 10.6, 804 33.6 / 16.2,
+// 3202 129 / 46.6.
 __device__ __forceinline__ uint4 pf_codes(uint2 w) {
     uint32_t o[4];
 #pragma unroll

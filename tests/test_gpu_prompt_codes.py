@@ -1,4 +1,4 @@
-"""Prompt GEMMs on 8- and 4-bit codes: slices of 64 rows up to 96 (csrc/lm_qgemm.hip, a second slice among them), tiles behind (csrc/lm_prefill.hip, k_gemm_pf_codes:
+"""Prompt GEMMs on 8- and 4-bit codes: slices of 64 rows up to 96 (up to 128 where ff > 4096; csrc/lm_qgemm.hip, a second slice among them), tiles behind (csrc/lm_prefill.hip, k_gemm_pf_codes:
 64 x 64 with one, two and four scale groups a step, 128 x 128), remainders in rows, columns and groups; ragged prompts.  Against the oracle on the float32 weights
 s q + b; and a prompt has the bits that it has alone, whatever slices or tiles its call takes."""
 import numpy as np
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 # hidden 1088 = 17 groups, ff 1216 = 19, heads 3 x 128 = 6: steps of two and four groups end inside; 1024 / 3072: 128 x 128 tiles for gate | up from 641 rows on
 @pytest.mark.parametrize("hidden, heads, ff, bits, total", [(1088, 3, 1216, 8, 75), (1088, 3, 1216, 4, 96), (1088, 3, 1216, 8, 97), (1088, 3, 1216, 4, 431), (1088, 3, 1216, 8, 1000), (1024, 16, 3072, 8, 130),
-                                                            (1024, 16, 3072, 4, 333), (1024, 16, 3072, 8, 700)])
+                                                            (1024, 16, 3072, 4, 333), (1024, 16, 3072, 8, 700), (1024, 16, 4160, 8, 128), (1024, 16, 4160, 4, 129)])
 def test_prompts_on_codes(hidden, heads, ff, bits, total):
     from gpu_util import logits_errors
     from gpu_util import lm_host_config
