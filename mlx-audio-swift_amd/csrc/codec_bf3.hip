@@ -20,6 +20,12 @@
 //                  to seven steps ahead) and the activation fragments from LDS (XOR-swizzled at the DMA source, conflict-free ds_read_b128).
 //                  One s_barrier per chunk.  Taps (dense k-tap convs), transposed-conv phases and 1x1 convs share the tile code:
 //                  tap j reads the staged tile at a column offset.
+//
+// Between two contractions the planes come from the epilogue in front (launch_gemm_chain): Snake and the split run there, on registers, and the pre-pass - a launch, a read and a
+// write of the tensor - is gone, with the f32 tensor where nothing else reads it.  DAC, one row of 30 / 250 frames, four of 400: 951 / 1688 / 8060 -> 748 / 1472 / 7490 us.
+// An operand may have three planes instead (NP = 3, the arithmetic and the bits of codec_x6.hip): the 1x1 contractions of 193 .. 384 channels behind Snake, which k_x6_gemm converts
+// once per 64 rows (384 x 384, 10005 columns: 45 us, 52 with planes out; 34 here).  Of up to 192 channels k_pw_x6 converts once in all and reads four bytes, not six: 192 channels,
+// 40021 columns: 42 us there, 43 here and 4 more in front; 96, 80043 columns: 36 and 41.
 #include "common.h"
 #include "codec_kernels.h"
 
@@ -33,9 +39,11 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 struct Bf3Params {
     GemmParams g;
     const uint16_t* wp;
-    const uint16_t* xh;
-    const uint16_t* xl;
-    int mode, ntaps, MT32, KS, Cp, Tp, t_org;
+    const uint16_t* xp;   // planes [plane][B][Tp][Cp]
+    size_t xplane;        // elements of one plane
+    size_t wtap, wmt, wks;                // weight fragments: elements from a tap, a row tile, a 16-channel step to the next
+    CodecPlanes out;      // .p: the output (also) as the planes of the contraction behind it
+    int mode, ntaps, MT32, Cp, Tp, t_org;
     int ksplit;           // > 1: a tile has that many blocks; a block contracts chunks [nchunks slice / ksplit, nchunks (slice + 1) / ksplit)
     float* part;          //      and writes its raw float32 sums to part[slice][b][M][ldy] (k_bf3_splitk_epilogue finishes)
     int batch;
@@ -119,29 +127,46 @@ __global__ void __launch_bounds__(256) k_bf3_split(const float* __restrict__ X, 
 }
 
 // ---- the contraction -----------------------------------------------------------------------------------------------------------------
-template <int MI> struct Bf3A { bf16x8_t v[MI][2]; };     // [m tile][hi, lo]
-template <int NI> struct Bf3B { bf16x8_t v[NI][2]; };     // [n tile][hi, lo]
+template <int NP, int MI> struct Bf3A { bf16x8_t v[MI][NP]; };     // [m tile][plane]
+template <int NP, int NI> struct Bf3B { bf16x8_t v[NI][NP]; };     // [n tile][plane]
 
-// sched_group_barrier masks: 0x008 MFMA, 0x002 VALU, 0x020 VMEM read, 0x100 DS read
-#define B3_IL_V __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x002, 3, 0); __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-#define B3_IL_D __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x002, 3, 0); __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-#define B3_IL_M __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-#define B3_INTERLEAVE_22 B3_IL_V B3_IL_V B3_IL_V B3_IL_V B3_IL_D B3_IL_D B3_IL_D B3_IL_D B3_IL_M B3_IL_M B3_IL_M B3_IL_M
-#define B3_INTERLEAVE_12 B3_IL_V B3_IL_V B3_IL_D B3_IL_D B3_IL_D B3_IL_D
-#define B3_INTERLEAVE_11 B3_IL_V B3_IL_V B3_IL_D
+// One step's order: an MFMA with a weight load behind it, then one with a tile read, then the rest (sched_group_barrier masks: 0x008 MFMA, 0x002 VALU,
+// 0x020 VMEM read, 0x100 DS read)
+template <int NV, int ND, int NM> __device__ __forceinline__ void bf3_interleave() {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+    }
+}
 
 // The body takes the arrays the epilogue touches as restrict-qualified PARAMETERS: GemmParams is a struct, clang ignores restrict on
 // struct members, and without it every bias / residual load of the epilogue waits behind the previous row's store (the same effect
 // cost the fused unit kernel of snac.hip 25 %).
-template <int MI, int NI, int NQ, int NBUF, int NTAPS, int AR>
+template <int NP, int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, bool OUT>
 __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
-                                         const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise) {
+                                         const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise,
+                                         const float* __restrict__ poa, const float* __restrict__ pora, uint16_t* __restrict__ pout) {
     constexpr int PLANE = NQ * 512;                       // bf16 per plane: NQ DMA instructions of 1 KiB (16 columns x 32 channels)
-    constexpr int BUF = 2 * PLANE;
+    constexpr int BUF = NP * PLANE;
     constexpr int NST = 2 * NTAPS;                        // MFMA steps (16 channels of one tap) per chunk
     constexpr int CG = NST % AR == 0 ? 1 : (2 * NST) % AR == 0 ? 2 : (3 * NST) % AR == 0 ? 3 : 4;      // chunks per straight-line group: whole turns of the weight ring
     static_assert(CG * NST % AR == 0 && CG * NST % 2 == 0, "registers rotate in whole turns");
-    constexpr int BN = 64 * NI;
+    constexpr int BN = 64 * NI, NPROD = NP == 2 ? 3 : 6, ND = NPROD * MI * NI - NP * MI < NP * NI ? NPROD * MI * NI - NP * MI : NP * NI;
+    static_assert(!OUT || NBUF * BUF >= 4 * NI * CP_LDS(3), "the ring holds the waves' output tiles");
+    static_assert((NBUF - 2) * NP * NQ < 64, "the loader's wait counts the younger chunks");
     __shared__ __attribute__((aligned(1024))) uint16_t lds[NBUF * BUF];
     const GemmParams& p = P.g;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -166,23 +191,21 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
         // lane slot gs holds channel group gs ^ ((i >> 2) & 3) (the swizzle is on the SOURCE address, the LDS side of a DMA is lane-linear)
         const int il = lane >> 2, grp = (lane & 3) ^ ((il >> 2) & 3);
         const size_t col0 = ((size_t)b * P.Tp + (size_t)(n0 + shmin - P.t_org + il)) * P.Cp + grp * 8;
-        const uint16_t* sh = P.xh + col0 + (size_t)c_lo * B3_KC;
-        const uint16_t* sl = P.xl + col0 + (size_t)c_lo * B3_KC;
+        const uint16_t* sx = P.xp + col0 + (size_t)c_lo * B3_KC;
         const size_t qstride = (size_t)16 * P.Cp;
         auto issue = [&](int cc) {
-            const uint16_t* h = sh + cc * B3_KC;
-            const uint16_t* l = sl + cc * B3_KC;
+            const uint16_t* h = sx + cc * B3_KC;
             const int buf = cc % NBUF;
 #pragma unroll
-            for (int q = 0; q < NQ; ++q) {
-                __builtin_amdgcn_global_load_lds((gptr_t)(h + q * qstride), (lptr_t)&lds[buf * BUF + q * 512], 16, 0, 0);
-                __builtin_amdgcn_global_load_lds((gptr_t)(l + q * qstride), (lptr_t)&lds[buf * BUF + PLANE + q * 512], 16, 0, 0);
-            }
+            for (int q = 0; q < NQ; ++q)
+#pragma unroll
+                for (int i = 0; i < NP; ++i)
+                    __builtin_amdgcn_global_load_lds((gptr_t)(h + q * qstride + i * P.xplane), (lptr_t)&lds[buf * BUF + i * PLANE + q * 512], 16, 0, 0);
         };
         for (int c = 0; c < NBUF - 1 && c < nchunks; ++c) issue(c);
         for (int cc = 0; cc < nchunks; ++cc) {
             // chunk cc must have landed; up to NBUF-2 younger chunks stay in flight
-            if (nchunks - 1 - cc >= NBUF - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * 2 * NQ) : "memory");
+            if (nchunks - 1 - cc >= NBUF - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * NP * NQ) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             if (cc + NBUF - 1 < nchunks) issue(cc + NBUF - 1);
@@ -204,36 +227,35 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
     // never stored).  The body below is CG chunks (CG * NST steps) of straight-line code: the weight registers rotate with period AR,
     // the tile-fragment registers with period 2, every index is a compile-time constant and there is no branch between the MFMAs,
     // so the waitcnt pass keeps exactly the AR - 2 younger weight loads in flight (with branches in the body it fell back to vmcnt(0)).
-    const size_t tap_stride = (size_t)P.MT32 * P.KS * 1024, mt_stride = (size_t)P.KS * 1024;
-    const uint16_t* wbase = P.wp + (size_t)lane * 8 + (size_t)tapbase * tap_stride + (size_t)mt0 * mt_stride + (size_t)c_lo * 2 * 1024;
-    const size_t mt1 = (mt0 + 1 < P.MT32) ? mt_stride : 0;
+    const uint16_t* wbase = P.wp + (size_t)lane * 8 + (size_t)tapbase * P.wtap + (size_t)mt0 * P.wmt + (size_t)c_lo * 2 * P.wks;
+    const size_t mt1 = (mt0 + 1 < P.MT32) ? P.wmt : 0;
     const int ncol = wn * 32 * NI + (lane & 31), kgrp = lane >> 5;
-    Bf3A<MI> aq[AR];
-    Bf3B<NI> bq[2];
-    auto loadA = [&](Bf3A<MI>& f, int chunk, int tap, int ks) {
+    Bf3A<NP, MI> aq[AR];
+    Bf3B<NP, NI> bq[2];
+    auto loadA = [&](Bf3A<NP, MI>& f, int chunk, int tap, int ks) {
         chunk = min(chunk, nchunks - 1);                     // the last steps prefetch past the end: re-read the last chunk
-        const uint16_t* q = wbase + (size_t)tap * tap_stride + (size_t)(chunk * 2 + ks) * 1024;
+        const uint16_t* q = wbase + (size_t)tap * P.wtap + (size_t)(chunk * 2 + ks) * P.wks;
 #pragma unroll
-        for (int mi = 0; mi < MI; ++mi) {
-            f.v[mi][0] = *reinterpret_cast<const bf16x8_t*>(q + (mi ? mt1 : 0));
-            f.v[mi][1] = *reinterpret_cast<const bf16x8_t*>(q + (mi ? mt1 : 0) + 512);
-        }
+        for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+            for (int i = 0; i < NP; ++i) f.v[mi][i] = *reinterpret_cast<const bf16x8_t*>(q + (mi ? mt1 : 0) + i * 512);
     };
-    auto readB = [&](Bf3B<NI>& f, const uint16_t* tile, int tap, int ks) {
+    auto readB = [&](Bf3B<NP, NI>& f, const uint16_t* tile, int tap, int ks) {
         const int toff = sh0 + tap * dsh - shmin;
 #pragma unroll
         for (int ni = 0; ni < NI; ++ni) {
             const int i = ncol + ni * 32 + toff;
             const uint16_t* q = tile + i * 32 + (((ks * 2 + kgrp) ^ ((i >> 2) & 3)) * 8);
-            f.v[ni][0] = *reinterpret_cast<const bf16x8_t*>(q);
-            f.v[ni][1] = *reinterpret_cast<const bf16x8_t*>(q + PLANE);
+#pragma unroll
+            for (int j = 0; j < NP; ++j) f.v[ni][j] = *reinterpret_cast<const bf16x8_t*>(q + j * PLANE);
         }
     };
-    // three products per tile pair: hi.hi, hi.lo, lo.hi; MI * NI independent accumulators between dependent MFMAs
-    auto products = [&](const Bf3A<MI>& A, const Bf3B<NI>& B) {
+    // products per tile pair, two planes: hi.hi, hi.lo, lo.hi; three: the six of codec_x6.hip, smallest first; MI * NI independent accumulators between dependent MFMAs
+    auto products = [&](const Bf3A<NP, MI>& A, const Bf3B<NP, NI>& B) {
+        constexpr int QA[2][6] = {{0, 0, 1}, {2, 0, 1, 1, 0, 0}}, QB[2][6] = {{0, 1, 0}, {0, 2, 1, 0, 1, 0}};
 #pragma unroll
-        for (int term = 0; term < 3; ++term) {
-            const int ta = term == 2 ? 1 : 0, tb = term == 1 ? 1 : 0;
+        for (int term = 0; term < (NP == 2 ? 3 : 6); ++term) {
+            const int ta = QA[NP - 2][term], tb = QB[NP - 2][term];
 #pragma unroll
             for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
@@ -246,8 +268,19 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
     const uint16_t* tile = lds;
     int gbuf = 0;                                           // ring slot of the next chunk
     const float* Xb = pX + (size_t)b * p.Cin * p.ldx;
-    const bool convt = P.mode == GEMM_CONVT, gelu = P.mode == GEMM_GELU, noise = P.mode == GEMM_NOISE;
+    const bool convt = P.mode == GEMM_CONVT, gelu = !OUT && P.mode == GEMM_GELU, noise = !OUT && P.mode == GEMM_NOISE;
     const float* Rr = (convt || gelu || noise) ? nullptr : pR;
+    constexpr bool EARLY = OUT && MI == 1 && NTAPS == 1;
+    float early[EARLY ? NI : 1][EARLY ? 16 : 1];
+    if constexpr (EARLY) {
+        if (Rr) {
+#pragma unroll
+            for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    early[ni][r] = Rr[((size_t)b * p.M + min(mt0 * 32 + (r & 3) + 8 * (r >> 2) + 4 * kgrp, p.M - 1)) * p.ldy + min(n0 + (wn * NI + ni) * 32 + (lane & 31), p.N - 1)];
+        }
+    }
 
     {
 #pragma unroll
@@ -275,7 +308,7 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                 const int J = I + AR - 1;
                 loadA(aq[J % AR], cc + J / NST, (J % NST) >> 1, J & 1);
                 products(aq[I % AR], bq[I & 1]);
-                if constexpr (MI == 2) { B3_INTERLEAVE_22 } else if constexpr (NI == 2) { B3_INTERLEAVE_12 } else { B3_INTERLEAVE_11 }
+                bf3_interleave<NP * MI, ND, NPROD * MI * NI - NP * MI - ND>();
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -297,7 +330,7 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                     const int J = I + AR - 1;
                     loadA(aq[J % AR], cc + J / NST, (J % NST) >> 1, J & 1);
                     products(aq[I % AR], bq[I & 1]);
-                    if constexpr (MI == 2) { B3_INTERLEAVE_22 } else if constexpr (NI == 2) { B3_INTERLEAVE_12 } else { B3_INTERLEAVE_11 }
+                    bf3_interleave<NP * MI, ND, NPROD * MI * NI - NP * MI - ND>();
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -322,6 +355,92 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                     }
                 }
             }
+            return;
+        }
+        if constexpr (NP == 3) {
+            // Three planes hold an infinity as one beside a NaN: a lane that sees a sum which is not finite takes its rows again as the f32 kernels do
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni) {
+                    const int n = n0 + (wn * NI + ni) * 32 + (lane & 31);
+                    float zero = 0.0f;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) zero = fmaf(acc[mi][ni][r], 0.0f, zero);
+                    if (zero == 0.0f || n >= p.N) continue;
+#pragma unroll 1
+                    for (int r = 0; r < 16; ++r) {
+                        const int m = (mt0 + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * lane_hi;
+                        float v = 0.0f;
+#pragma unroll 1
+                        for (int i = 0; i < P.Cp * NTAPS && m < p.M && v == v; ++i) {       // 16 channels, within them the taps, within a tap the channels (NaN it stays)
+                            const int c = i / (16 * NTAPS) * 16 + (i & 15), j = i / 16 % NTAPS;
+                            const uint16_t* x = P.xp + ((size_t)b * P.Tp + (n + sh0 + j * dsh - P.t_org)) * P.Cp + c;
+                            const float hm = bf16_to_f32(x[0]) + bf16_to_f32(x[P.xplane]), xv = fabsf(hm) < INFINITY ? hm + bf16_to_f32(x[2 * P.xplane]) : hm;
+                            if (c < p.Cin) v = fmaf(p.AT[((size_t)j * p.Cin + c) * p.M + m], xv, v);
+                        }
+#pragma unroll
+                        for (int q = 0; q < 16; ++q) acc[mi][ni][q] = q == r ? v : acc[mi][ni][q];
+                    }
+                }
+        }
+        if constexpr (OUT) {
+            // the output as the operand of the contraction behind this one (its pre-pass's values), and in f32 where something else reads it; the ring is free by now.
+            // Eight rows at a time, their values (the residual's of both column tiles too) requested together; EARLY: the residual came with the first weights
+            __syncthreads();
+            uint16_t* st = lds + wave * NI * CP_LDS(3);
+#pragma unroll
+            for (int mi = 0; mi < MI; ++mi) {
+                const int mt = (mt0 + mi) * 32;
+                if (mt >= p.M) break;
+#pragma unroll
+                for (int r0 = 0; r0 < 16; r0 += 8) {
+                    const int m0 = mt + 2 * r0 + 4 * lane_hi;
+                    float bm[8], al[8], ra[8], e[NI][8];
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) {
+                        const int m = m0 + (r & 3) + 8 * (r >> 2);
+                        bm[r] = pbias ? pbias[m] : 0.0f;
+                        if (poa) { al[r] = poa[m]; ra[r] = pora[m]; }
+                        if (Rr && !EARLY) {
+#pragma unroll
+                            for (int ni = 0; ni < NI; ++ni) e[ni][r] = Rr[((size_t)b * p.M + m) * p.ldy + min(n0 + (wn * NI + ni) * 32 + (lane & 31), p.N - 1)];
+                        }
+                    }
+#pragma unroll
+                    for (int ni = 0; ni < NI; ++ni) {
+                        const int n = n0 + (wn * NI + ni) * 32 + (lane & 31), o = convt ? p.s * n + phase : n;
+                        float y[8];
+#pragma unroll
+                        for (int r = 0; r < 8; ++r) {
+                            y[r] = acc[mi][ni][r0 + r] + bm[r];
+                            if (convt && n == 0 && p.dup_bias_n0) y[r] += bm[r];
+                            if (Rr) y[r] += EARLY ? early[EARLY ? ni : 0][EARLY ? r0 + r : 0] : e[ni][r];
+                        }
+                        if (pY && n < p.N && o < p.Tout) {
+#pragma unroll
+                            for (int r = 0; r < 8; ++r) pY[((size_t)b * p.M + m0 + (r & 3) + 8 * (r >> 2)) * p.ldy + o] = y[r];
+                        }
+                        if (poa) {
+#pragma unroll
+                            for (int r = 0; r < 8; ++r) y[r] = bf3_snake(y[r], al[r], ra[r]);
+                        }
+                        if (P.out.n == 3) codec_tile_put<3>(y, st + ni * CP_LDS(3), r0, lane);
+                        else codec_tile_put<2>(y, st + ni * CP_LDS(3), r0, lane);
+                    }
+                }
+                uint16_t* d = pout + (size_t)b * P.out.Tp * P.out.Cp + mt;
+#pragma unroll
+                for (int ni = 0; ni < NI; ++ni) {
+                    auto row = [&](int c) {
+                        const int n = n0 + (wn * NI + ni) * 32 + c, o = convt ? p.s * n + phase : n, r = o - P.out.t_org;
+                        return n < p.N && o < p.Tout && r < P.out.Tp ? r : -1;
+                    };
+                    if (P.out.n == 3) codec_tile_flush<3>(st + ni * CP_LDS(3), d, P.out.stride, P.out.Cp, lane, row);
+                    else codec_tile_flush<2>(st + ni * CP_LDS(3), d, P.out.stride, P.out.Cp, lane, row);
+                }
+            }
+            if (phase == 0) codec_plane_ends(P.out, b, p.Tout, mt0 * 32, min(MI * 32, p.M - mt0 * 32), bx == 0 && wn == 0, bx == P.nbx - 1 && wn == 1, lane, 64);
             return;
         }
         // a tile's bias and residual (or NoiseBlock input) values are requested together, clamped; one by one under their guards each was a round trip
@@ -368,9 +487,9 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
     }
 }
 
-template <int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, int MINW>
+template <int NP, int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, int MINW, bool OUT>
 __global__ void __launch_bounds__(B3_THREADS, MINW) k_bf3_gemm(Bf3Params P) {
-    bf3_body<MI, NI, NQ, NBUF, NTAPS, AR>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise);
+    bf3_body<NP, MI, NI, NQ, NBUF, NTAPS, AR, OUT>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.out.alpha, P.out.ralpha, P.out.p);
 }
 
 // split-K: Y = epilogue(sum over slices in slice order + bias) - the 1x1 modes' epilogues of bf3_body (plain / GELU / residual with scale)
@@ -420,55 +539,106 @@ static int bf3_env(const char* name, int dflt) {
 CodecPack* codec_x6_scope() { return tl_x6; }
 bool codec_exact_f32() { return bf3_env("MIS_CODEC_EXACT_F32", 0) != 0; }
 
-bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s) {
-    GemmParams p = p_in;
-    if (!p.pack) p.pack = tl_pack;
-    if (!p.pack || bf3_env("MIS_CODEC_EXACT_F32", 0)) return false;
+// What the two-plane contractions take.  What pays: MFMA-bound shapes.  A 1x1 conv over few channels is HBM-bound and the pre-pass would only add traffic
+// (measured per dispatch, profiles/r02_codec/: 1x1 over <= 512 channels and the last SNAC transposed conv, M*K = 16 K,
+// are faster on the exact-f32 kernels; every 7-tap conv and the transposed convs from M*K = 36 K up gain 2.3 - 4x)
+struct Bf3Shape { int ntaps, Cin, span, t_org, wtaps, phases, extra; };
+static bool bf3_shape(int mode, const GemmParams& p, Bf3Shape& h) {
     const bool one = mode == GEMM_PLAIN || mode == GEMM_GELU || mode == GEMM_RESID || mode == GEMM_NOISE;
-    int ntaps = 1, Cin = p.K, span = 0, t_org = 0, wtaps = 1;
-    if (mode == GEMM_TAPS) { ntaps = p.taps; Cin = p.Cin; span = (p.taps - 1) * p.dil; t_org = -p.pad; wtaps = ntaps; }
+    h = Bf3Shape{1, p.K, 0, 0, 1, 1, 0};
+    if (mode == GEMM_TAPS) { h.ntaps = p.taps; h.Cin = p.Cin; h.span = (p.taps - 1) * p.dil; h.t_org = -p.pad; h.wtaps = p.taps; }
     else if (mode == GEMM_CONVT) {
         if (p.Cin <= 0 || p.K % p.Cin || p.K / p.Cin > 2) return false;
-        ntaps = p.K / p.Cin;                                         // 2: kernel 2s (overlap-add); 1: kernel = stride (A^T holds one tap)
-        Cin = p.Cin; span = ntaps - 1; wtaps = ntaps * p.s;
-        t_org = p.pad / p.s - (ntaps - 1);                           // phase 0 has the smallest q = (phase + pad) / s
-        if ((p.s - 1 + p.pad) / p.s - p.pad / p.s > 1) return false;
+        h.ntaps = p.K / p.Cin;                                       // 2: kernel 2s (overlap-add); 1: kernel = stride (A^T holds one tap)
+        h.Cin = p.Cin; h.span = h.ntaps - 1; h.wtaps = h.ntaps * p.s; h.phases = p.s;
+        h.t_org = p.pad / p.s - (h.ntaps - 1);                       // phase 0 has the smallest q = (phase + pad) / s
+        h.extra = (p.s - 1 + p.pad) / p.s - p.pad / p.s;             // the phases share one operand: columns from the smallest shift of any phase to the largest
+        if (h.extra > 1) return false;
     } else if (!one) return false;
-    // what pays: MFMA-bound shapes.  A 1x1 conv over few channels is HBM-bound and the pre-pass would only add traffic
-    // (measured per dispatch, profiles/r02_codec/: 1x1 over <= 512 channels and the last SNAC transposed conv, M*K = 16 K,
-    // are faster on the exact-f32 kernels; every 7-tap conv and the transposed convs from M*K = 36 K up gain 2.3 - 4x)
+    return p.M >= 32 && h.span <= 64 && (h.ntaps == 1 || h.ntaps == 2 || h.ntaps == 7);
+}
+static bool bf3_takes(int mode, const GemmParams& p, const Bf3Shape& h) {
     const int min_k1 = bf3_env("MIS_BF3_MIN_K1", 768), min_k = bf3_env("MIS_BF3_MIN_K", 32), min_mk = bf3_env("MIS_BF3_MIN_MK_CONVT", 32768);
-    if (one ? Cin < min_k1 : Cin < min_k) return false;
-    if (mode == GEMM_CONVT && (int64_t)p.M * p.K < min_mk) return false;
-    if (p.M < 32 || span > 64 || (ntaps != 1 && ntaps != 2 && ntaps != 7)) return false;
-    const CodecPack::Entry& e = p.pack->get(p.AT, wtaps, Cin, p.M, s);
-
-    // Tile: 128 x 128 (64 x 64 per wave); 64 x 128 while those are at most 128 blocks - half of the chip idle, each block one serial chain of chunks -
-    // and 64 x 64 while 64 x 128 still are (or no more than 64 columns exist).  The same bits: the order of the products of an output does not change.
-    // The small tiles run alone on a compute unit, with registers to spare: weights seven (not two) steps ahead, which covers a trip to HBM.
-    // us, 128 x 128 / 64 x 128 / 64 x 64: 768 rows, 7 taps of 768, 2080 columns: 102 / 60 / 79; 768 rows, K = 768: 51 / 24 / 26;
-    // 1536 rows, 7 taps of 1024, 250 columns: 140 / 70 / 55; SNAC, one row of 12 groups: 48 / - / 19, 41 / 22 / 15, 33 / - / 14, 29 / 17 / 16.
-    const int phases = mode == GEMM_CONVT ? p.s : 1;
+    if (mode == GEMM_CONVT) return h.Cin >= min_k && (int64_t)p.M * p.K >= min_mk;
+    return h.Cin >= (mode == GEMM_TAPS ? min_k : min_k1);
+}
+// Tile: 128 x 128 (64 x 64 per wave); 64 x 128 while those are at most 128 blocks - half of the chip idle, each block one serial chain of chunks -
+// and 64 x 64 while 64 x 128 still are (or no more than 64 columns exist).  The same bits: the order of the products of an output does not change.
+// The small tiles run alone on a compute unit, with registers to spare: weights seven (not two) steps ahead, which covers a trip to HBM.
+// us, 128 x 128 / 64 x 128 / 64 x 64: 768 rows, 7 taps of 768, 2080 columns: 102 / 60 / 79; 768 rows, K = 768: 51 / 24 / 26;
+// 1536 rows, 7 taps of 1024, 250 columns: 140 / 70 / 55; SNAC, one row of 12 groups: 48 / - / 19, 41 / 22 / 15, 33 / - / 14, 29 / 17 / 16.
+struct Bf3Tile { bool few; int NI, nbx, nq, Tp; };
+static Bf3Tile bf3_tile(const GemmParams& p, const Bf3Shape& h, int batch) {
     const int nb128 = (p.N + 127) / 128;
-    const bool few = (int64_t)nb128 * ((p.M + B3_BM - 1) / B3_BM) * batch * phases <= 128;
-    const int NI = few && (p.N <= 64 || (int64_t)nb128 * ((p.M + 63) / 64) * batch * phases <= 128) ? 1 : 2, bn = 64 * NI, nbx = (p.N + bn - 1) / bn;
-    const int nq = span <= 16 ? 4 * NI + 1 : 4 * NI + 4;
-    // the transposed conv's phases share one pre-pass: columns from the smallest shift of any phase to the largest
-    const int extra = mode == GEMM_CONVT ? ((p.s - 1 + p.pad) / p.s - p.pad / p.s) : 0;
-    const int Tp = (nbx - 1) * bn + nq * 16 + extra;
-    p.pack->xh.alloc((size_t)batch * Tp * e.Cp);
-    p.pack->xl.alloc((size_t)batch * Tp * e.Cp);
-    const bool sn = snake && p.alpha;
-    hipLaunchKernelGGL(k_bf3_split, dim3((Tp + 63) / 64, (e.Cp + SP_CB - 1) / SP_CB, batch), dim3(256), 0, s, p.X, p.pack->xh.p, p.pack->xl.p,
-                       sn ? p.alpha : nullptr, sn ? p.ralpha : nullptr, Cin, p.ldx, p.x_lo, p.Tin, e.Cp, Tp, t_org);
+    Bf3Tile t{};
+    t.few = (int64_t)nb128 * ((p.M + B3_BM - 1) / B3_BM) * batch * h.phases <= 128;
+    t.NI = t.few && (p.N <= 64 || (int64_t)nb128 * ((p.M + 63) / 64) * batch * h.phases <= 128) ? 1 : 2;
+    t.nbx = (p.N + 64 * t.NI - 1) / (64 * t.NI);
+    t.nq = 4 * t.NI + (h.span == 0 ? 0 : h.span <= 16 ? 1 : 4);
+    t.Tp = (t.nbx - 1) * 64 * t.NI + t.nq * 16 + h.extra;
+    return t;
+}
+// Three planes, where the epilogue in front writes them: 1x1 contractions with Snake and a residual that k_x6_gemm would convert for itself
+static bool bf3_three(int mode, const GemmParams& p) { return mode == GEMM_RESID && p.alpha && p.M >= 48 && p.K > 192 && p.K <= 384; }
+
+bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot, CodecPlanes& out) {
+    CodecPack* pack = p.pack ? p.pack : tl_pack;
+    Bf3Shape h;
+    if (!pack || codec_exact_f32() || !bf3_shape(mode, p, h) || h.Cin % 32) return false;
+    const bool two = bf3_takes(mode, p, h);
+    if (!two && !(snake && bf3_three(mode, p))) return false;
+    const Bf3Tile t = bf3_tile(p, h, batch);
+    out = CodecPlanes{};
+    out.n = two ? 2 : 3; out.Cp = h.Cin; out.Tp = t.Tp; out.t_org = h.t_org; out.ends = h.span > 0 || h.extra > 0;
+    out.stride = (size_t)batch * t.Tp * h.Cin;
+    if (snake) { out.alpha = p.alpha; out.ralpha = p.ralpha; }
+    pack->planes[slot].alloc(out.n * out.stride);
+    out.p = pack->planes[slot].p;
+    return true;
+}
+
+bool bf3_writes_planes(int mode, const GemmParams& p) { return p.M % 32 == 0 && !p.split_k_ok && !p.scale && (mode == GEMM_TAPS || mode == GEMM_CONVT || mode == GEMM_PLAIN || mode == GEMM_RESID); }
+
+bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s, const CodecPlanes* in, const CodecPlanes* out) {
+    GemmParams p = p_in;
+    if (!p.pack) p.pack = tl_pack;
+    if (!p.pack || codec_exact_f32()) return false;
+    Bf3Shape h;
+    if (!bf3_shape(mode, p, h) || (!in && !bf3_takes(mode, p, h))) return false;
+    if (out) {
+        MIS_REQUIRE(bf3_writes_planes(mode, p) && out->Cp == p.M, MIS_ERR_GENERATION_FAILED, "codec contraction: %d rows for an operand of %d channels", p.M, out->Cp);
+    }
+    const int ntaps = h.ntaps, Cin = h.Cin, span = h.span;
+    const Bf3Tile t = bf3_tile(p, h, batch);
+    const bool few = t.few;
+    const int NI = t.NI, nb128 = (p.N + 127) / 128;
     Bf3Params P{};
     P.g = p; P.g.Cin = Cin;
-    P.wp = e.wp; P.xh = p.pack->xh.p; P.xl = p.pack->xl.p;
-    P.mode = mode; P.ntaps = ntaps; P.MT32 = e.MT32; P.KS = e.KS; P.Cp = e.Cp; P.Tp = Tp; P.t_org = t_org;
+    P.mode = mode; P.ntaps = ntaps; P.Tp = t.Tp; P.t_org = h.t_org;
+    if (in && in->n == 3) {
+        const CodecPack::X6& e = p.pack->get_x6(p.AT, h.wtaps, Cin, p.M, s);
+        P.wp = e.wp; P.MT32 = e.MT32;
+        P.wmt = 1536; P.wtap = (size_t)e.MT32 * 1536; P.wks = h.wtaps * P.wtap;
+    } else {
+        const CodecPack::Entry& e = p.pack->get(p.AT, h.wtaps, Cin, p.M, s);
+        P.wp = e.wp; P.MT32 = e.MT32;
+        P.wks = 1024; P.wmt = (size_t)e.KS * 1024; P.wtap = e.MT32 * P.wmt;
+    }
+    P.Cp = (Cin + B3_KC - 1) / B3_KC * B3_KC;
+    if (in) { P.xp = in->p; P.xplane = in->stride; }
+    else {
+        P.xplane = (size_t)batch * t.Tp * P.Cp;
+        p.pack->xs.alloc(2 * P.xplane);
+        P.xp = p.pack->xs.p;
+        const bool sn = snake && p.alpha;
+        hipLaunchKernelGGL(k_bf3_split, dim3((t.Tp + 63) / 64, (P.Cp + SP_CB - 1) / SP_CB, batch), dim3(256), 0, s, p.X, p.pack->xs.p, p.pack->xs.p + P.xplane,
+                           sn ? p.alpha : nullptr, sn ? p.ralpha : nullptr, Cin, p.ldx, p.x_lo, p.Tin, P.Cp, t.Tp, h.t_org);
+    }
+    if (out) P.out = *out;
     // launch-shaped 1x1 contractions (Soprano's ConvNeXt GEMMs at 257 frames: 18 or 54 blocks per row of a 256-CU part, 60 us per launch):
     // the K range split over blocks.  The factor is a function of the SHAPE of one batch row only (a row's bits do not depend on the batch
     // it shares); float32 slabs, summed in slice order by k_bf3_splitk_epilogue
-    const int nchunks = e.Cp / B3_KC, per_row = nb128 * ((p.M + B3_BM - 1) / B3_BM);
+    const int nchunks = P.Cp / B3_KC, per_row = nb128 * ((p.M + B3_BM - 1) / B3_BM);
     int ksplit = 1;
     if (p.split_k_ok && ntaps == 1 && (mode == GEMM_PLAIN || mode == GEMM_GELU || mode == GEMM_RESID) && !bf3_env("MIS_BF3_NO_SPLITK", 0)) {
         if (per_row <= 32 && nchunks >= 32) ksplit = 4;
@@ -481,35 +651,62 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
     // Rows that are no multiple of 128 leave a wave row of the large tile without any, and its blocks (7 taps: one a compute unit) come in whole rounds: 64 x 128 there,
     // two blocks a compute unit.  us, 128 x 128 / 64 x 128: 192 rows, 7 taps, 40000 columns 91 / 63, 2 taps (5 phases) 62 / 54; 96 rows, 80000 columns 67 / 45, 47 / 39;
     // whole tiles: 384 rows, 7 taps, 10000 columns 60 / 64, 2 taps of 512 .. 128 rows (SNAC, 32 rows) 588 / 767, 1395 / 1748, 1734 / 1966
-    const bool half = !few && ntaps != 1 && p.M % B3_BM != 0;
+    const bool three = in && in->n == 3, half = !few && (three || (ntaps != 1 && p.M % B3_BM != 0));
     const int bm = few || half ? 64 : B3_BM;
-    P.nbx = nbx; P.my = (p.M + bm - 1) / bm; P.inner = phases * ksplit;
-    P.tiles = nbx * P.my * batch; P.per = (P.tiles + 7) / 8;
-    dim3 grid(8 * P.per * P.inner), block(B3_THREADS);
-#define B3_GO(...) hipLaunchKernelGGL((k_bf3_gemm<__VA_ARGS__>), grid, block, 0, s, P)
-    if (few && NI == 1) {
-        if (ntaps == 1) B3_GO(1, 1, 5, 8, 1, 8, 2);
-        else if (ntaps == 2) B3_GO(1, 1, 5, 8, 2, 8, 2);
-        else if (span <= 16) B3_GO(1, 1, 5, 4, 7, 7, 2);
-        else B3_GO(1, 1, 8, 4, 7, 7, 2);
-    } else if (few) {
-        if (ntaps == 1) B3_GO(1, 2, 9, 5, 1, 8, 2);
-        else if (ntaps == 2) B3_GO(1, 2, 9, 5, 2, 8, 2);
-        else if (span <= 16) B3_GO(1, 2, 9, 4, 7, 7, 2);
-        else B3_GO(1, 2, 12, 4, 7, 7, 2);
+    P.nbx = t.nbx; P.my = (p.M + bm - 1) / bm; P.inner = h.phases * ksplit;
+    P.tiles = P.nbx * P.my * batch; P.per = (P.tiles + 7) / 8;
+    const dim3 grid(8 * P.per * P.inner), block(B3_THREADS);
+#define B3_GO(...) do { \
+        if (out) hipLaunchKernelGGL((k_bf3_gemm<__VA_ARGS__, true>), grid, block, 0, s, P); \
+        else hipLaunchKernelGGL((k_bf3_gemm<__VA_ARGS__, false>), grid, block, 0, s, P); } while (0)
+    if (three) {
+        if (NI == 1) B3_GO(3, 1, 1, 4, 6, 1, 6, 2);
+        else B3_GO(3, 1, 2, 8, 3, 1, 4, 3);
     }
-    else if (half && ntaps == 2) B3_GO(1, 2, 9, 4, 2, 4, 3);
-    else if (half && span <= 16) B3_GO(1, 2, 9, 4, 7, 4, 3);
-    else if (half) B3_GO(1, 2, 12, 3, 7, 4, 3);
+    else if (few && NI == 1) {
+        if (ntaps == 1) B3_GO(2, 1, 1, 4, 8, 1, 8, 2);
+        else if (ntaps == 2) B3_GO(2, 1, 1, 5, 8, 2, 8, 2);
+        else if (span <= 16) B3_GO(2, 1, 1, 5, 4, 7, 7, 2);
+        else B3_GO(2, 1, 1, 8, 4, 7, 7, 2);
+    } else if (few) {
+        if (ntaps == 1) B3_GO(2, 1, 2, 8, 5, 1, 8, 2);
+        else if (ntaps == 2) B3_GO(2, 1, 2, 9, 5, 2, 8, 2);
+        else if (span <= 16) B3_GO(2, 1, 2, 9, 4, 7, 7, 2);
+        else B3_GO(2, 1, 2, 12, 4, 7, 7, 2);
+    }
+    else if (half && ntaps == 2) B3_GO(2, 1, 2, 9, 4, 2, 4, 3);
+    else if (half && span <= 16) B3_GO(2, 1, 2, 9, 4, 7, 4, 3);
+    else if (half) B3_GO(2, 1, 2, 12, 3, 7, 4, 3);
     // MINW 3 = two blocks (ten waves) per CU, 168 registers: fits 1 and 2 taps; the 7-tap body would spill (measured 2.3x slower), so it
     // runs one block per CU (a persistent loop over column tiles was measured too: no gain, profiles/r02_codec/ab_record.json)
-    else if (ntaps == 1) B3_GO(2, 2, 9, 4, 1, 3, 3);
-    else if (ntaps == 2) B3_GO(2, 2, 9, 4, 2, 3, 3);
-    else if (span <= 16) B3_GO(2, 2, 9, 4, 7, 4, 2);
-    else B3_GO(2, 2, 12, 4, 7, 4, 2);
+    else if (ntaps == 1) B3_GO(2, 2, 2, 8, 4, 1, 3, 3);
+    else if (ntaps == 2) B3_GO(2, 2, 2, 9, 4, 2, 3, 3);
+    else if (span <= 16) B3_GO(2, 2, 2, 9, 4, 7, 4, 2);
+    else B3_GO(2, 2, 2, 12, 4, 7, 4, 2);
 #undef B3_GO
     if (ksplit > 1)
         hipLaunchKernelGGL(k_bf3_splitk_epilogue, dim3((p.N + 255) / 256, p.M, batch), dim3(256), 0, s, P.part, ksplit, batch, mode, p.bias, p.scale, p.R, p.Y, p.M,
                            p.N, p.ldy);
     return true;
+}
+
+void launch_gemm_chain(const CodecOp* ops, int n, int batch, hipStream_t s) {
+    CodecPlanes cur{}, nxt{};
+    bool have = false;
+    for (int i = 0; i < n; ++i) {
+        const CodecOp& o = ops[i];
+        const bool want = i + 1 < n && codec_planes(ops[i + 1].mode, ops[i + 1].snake, ops[i + 1].g, batch, i & 1, nxt);
+        if (have) {
+            GemmParams g = o.g;
+            if (!g.ldx) g.ldx = g.Tin;
+            if (!g.ldy) g.ldy = g.Tout;
+            if (!g.R) g.scale = nullptr;
+            const bool outs = want && bf3_writes_planes(o.mode, g);
+            if (outs && !o.keep) g.Y = nullptr;
+            MIS_REQUIRE(launch_gemm_bf3(o.mode, o.snake, g, batch, s, &cur, outs ? &nxt : nullptr), MIS_ERR_GENERATION_FAILED, "codec contraction refused its own operand");
+            have = outs;
+        } else
+            have = launch_gemm(o.mode, o.snake, o.g, batch, s, want ? &nxt : nullptr, o.keep);
+        cur = nxt;
+    }
 }

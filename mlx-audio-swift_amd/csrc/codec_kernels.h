@@ -72,7 +72,7 @@ struct CodecPack {
     std::vector<Entry> entries;
     struct X6 { const float* at; int ntaps, Cin, M, KS, MT32; uint16_t* wp; };
     std::vector<X6> x6;   // three-plane fragments (codec_x6.hip)
-    DevBuf<uint16_t> xh, xl;
+    DevBuf<uint16_t> xs, planes[2];      // operands: split by the pre-pass; written by the epilogue in front (two, in turns)
     DevBuf<float> part;   // split-K slabs of launch-shaped contractions (GemmParams.split_k_ok)
     CodecPack() {}
     CodecPack(const CodecPack&) = delete;
@@ -92,6 +92,69 @@ struct CodecPackScope {
 CodecPack* codec_x6_scope();          // the innermost scope's, or null
 bool codec_exact_f32();               // MIS_CODEC_EXACT_F32=1
 
+// An operand as bf16 planes, time-major: [n planes, stride elements apart][batch][Tp][Cp]; row r holds column r + t_org, through Snake where alpha is given.
+// ends: rows without a column are zero (an operand of one tap does not need them)
+struct CodecPlanes {
+    uint16_t* p;
+    int n, Cp, Tp, t_org;
+    bool ends;
+    size_t stride;
+    const float *alpha, *ralpha;
+};
+// A wave's 32 x 32 C/D tile (column lane & 31, row (r & 3) + 8 (r >> 2) + 4 (lane >> 5)) to NP bf16 planes, each the nearest to what is left, through CP_LDS(NP) bytes of LDS of its
+// own: put takes registers 0 - 7 (r0 = 0) and 8 - 15 (r0 = 8) - lanes l and l + 32 trade halves, so that each writes eight consecutive channels - and flush stores 64 bytes of a
+// column's channels per four lanes (straight from the registers they were 32.  96 x 96 with residual, 80043 columns: 28 us without planes, 42 and 36 with; the pre-pass 15).
+// Three planes: a value past the largest bfloat16 has that one as its first.
+#define CP_LD 40
+#define CP_LDS(NP) ((NP) * 32 * CP_LD)       // in bf16
+template <int NP>
+__device__ __forceinline__ void codec_tile_put(float (&y)[8], uint16_t* st, int r0, int lane) {
+    constexpr float TOP = 3.38953138925153547590470800371487866880e+38f;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float &a = y[2 * i], &b = y[2 * i + 1];
+            const float ca = NP == 3 && q == 0 ? __builtin_amdgcn_fmed3f(a, -TOP, TOP) : a, cb = NP == 3 && q == 0 ? __builtin_amdgcn_fmed3f(b, -TOP, TOP) : b;
+            w[i] = (uint32_t)f32_to_bf16(ca) | ((uint32_t)f32_to_bf16(cb) << 16);
+            a -= __uint_as_float(w[i] << 16);
+            b -= __uint_as_float(w[i] & 0xffff0000u);
+        }
+        const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+        *reinterpret_cast<uint4*>(st + (q * 32 + (lane & 31)) * CP_LD + 2 * r0 + 8 * (lane >> 5)) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+    }
+}
+// d: channel 0 of the tile in row 0; row(c): the operand's row of the tile's column c, < 0: none
+template <int NP, class Row>
+__device__ __forceinline__ void codec_tile_flush(const uint16_t* st, uint16_t* d, size_t stride, int Cp, int lane, Row row) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int c = i * 16 + (lane >> 2), r = row(c);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const uint4 v = *reinterpret_cast<const uint4*>(st + (q * 32 + c) * CP_LD + (lane & 3) * 8);
+            if (r >= 0) *reinterpret_cast<uint4*>(d + q * stride + (size_t)r * Cp + (lane & 3) * 8) = v;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// rows without a column, [0, -t_org) and behind column T, of the channels [c0, c0 + nc): by the blocks that hold the first and the last columns
+__device__ __forceinline__ void codec_plane_ends(const CodecPlanes& o, int b, int T, int c0, int nc, bool first, bool last, int tid, int threads) {
+    if (!o.ends) return;
+    const int lo = max(0, -o.t_org), hi = min(o.Tp, T - o.t_org), i0 = first ? 0 : lo, rows = lo + (last ? o.Tp - hi : 0) - i0, per = nc / 8 * o.n;
+    for (int i = tid; i < rows * per; i += threads) {
+        const int r = i0 + i / per, j = i % per;
+        *reinterpret_cast<uint4*>(o.p + (size_t)(j / (nc / 8)) * o.stride + ((size_t)b * o.Tp + (r < lo ? r : hi + r - lo)) * o.Cp + c0 + j % (nc / 8) * 8) = make_uint4(0, 0, 0, 0);
+    }
+}
+
 #define CODEC_DW_HALO 27              // 3 * max dilation (9)
 struct PwFusedParams {
     const float* X; const float* R; float* Y;
@@ -99,6 +162,7 @@ struct PwFusedParams {
     const float *a2, *ra2;                 // Snake in front of the 1x1 conv
     const float *AT, *b2;                  // W2^T [C][C] ([k][m]), bias
     int T, dil, ldx, ldr, ldy;
+    const CodecPlanes* out;                // units without taps: the operand of the contraction behind, or null
 };
 // three-plane split of the unit tails (codec_x6.hip); false: no pack, exact-f32 asked for, or another width - nothing launched
 bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s);
@@ -132,7 +196,8 @@ struct GemmParams {
                           // pad = (taps-1)*dil: causal, (taps-1)*dil/2: "same"; optional R (+scale) residual epilogue
 };
 // snake: Snake prologue on the X rows (CONVT always runs it: pass alpha = ralpha = zeros for identity)
-void launch_gemm(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
+// out: the operand of the contraction behind; true: written (and p.Y with it if keep), false: p.Y as ever
+bool launch_gemm(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s, const CodecPlanes* out = nullptr, bool keep = true);
 // exact-f32 kernels (codec_f32.hip): every mode but CONVT, TAPS without Snake; p must have ldx / ldy resolved
 void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
 // k-tap contractions of K >= 1024 add four partial sums, over the ranges [codec_quarter(w), codec_quarter(w + 1)) of their steps of 16 channels of a tap, in order:
@@ -140,11 +205,17 @@ void launch_gemm_f32(int mode, bool snake, const GemmParams& p, int batch, hipSt
 bool codec_quarters(const GemmParams& p);
 __host__ __device__ inline int codec_quarter(int steps, int w) { return w >= 4 ? steps : steps * w / 16 * 4; }
 // three-plane split (codec_x6.hip): 1x1 and k-tap contractions of at least 48 rows and a multiple of 16 channels; false: not eligible, nothing launched
-bool launch_gemm_x6(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
+bool launch_gemm_x6(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s, const CodecPlanes* out = nullptr);
+// (out: whether that form writes it)
+bool codec_x6_writes_planes(int mode, const GemmParams& p);
 // three-plane split: transposed convolution of stride 2, two taps per phase, 32 .. 64 rows, behind Snake; false: another shape
 bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s);
 // split-bf16 path; false = shape not eligible (or MIS_CODEC_EXACT_F32=1), nothing launched.  p must have ldx / ldy resolved
-bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s);
+// in: the operand is there already (codec_planes of the same call); out: the epilogue also writes (p.Y null: only) the operand of the contraction behind
+bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s, const CodecPlanes* in = nullptr, const CodecPlanes* out = nullptr);
+bool bf3_writes_planes(int mode, const GemmParams& p);
+// the operand of this call as the epilogue in front of it can write it (scope's pack, buffer `slot`); false: the call wants f32
+bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot, CodecPlanes& out);
 // depthwise 7-tap conv (zero padded, dilation dil): shorter odd kernels ride in centred 7-tap weights
 void launch_dw7(const float* X, float* Y, const float* w7 /*[C][7]*/, const float* bias, int batch, int C, int T, int dil, hipStream_t s);
 // Snake -> 7-tap conv (C -> 1, weights at w[c cs + k ks]) -> tanh
@@ -157,3 +228,8 @@ void launch_enc_first(const float* audio, float* y, const float* w, const float*
 void launch_enc_phase_split(const float* x, float* y, const float* a, const float* ra, int batch, int C, int T, int stride, hipStream_t s);
 void launch_vq_nearest(const float* ze, const float* cn, const float* cn2, int32_t* codes, int batch, int CD, int CB, int Tm, hipStream_t s);
 void launch_vq_residual(float* r, const int32_t* codes, const float* table, int batch, int C, int T, int stride, hipStream_t s);
+
+// Contractions one behind the other, each reading the output of the one in front (g.X = its g.Y): where both sides can, that output goes over as the planes its reader
+// multiplies, and as f32 only if something else reads it (keep)
+struct CodecOp { int mode; bool snake, keep; GemmParams g; };
+void launch_gemm_chain(const CodecOp* ops, int n, int batch, hipStream_t s);

@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 __device__ __forceinline__ float x6_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
 
@@ -84,25 +85,27 @@ const CodecPack::X6& CodecPack::get_x6(const float* at, int ntaps, int Cin, int 
 // What bounds it: k_pw_fused<128, DW> took 1.05 ms without its MFMAs (4.8 GB of loads and stores, 32 rows of 98304 columns) and 1.75 ms with: the f32
 // matrix time adds to the memory time.  Six bf16 products take 0.25 instead of 0.68 ms of it: 1.95 -> 1.44 ms.
 struct PwScalars { int T, dil, ldx, ldr, ldy; };
-template <int C, bool DW, int KC, int NT>
+template <int C, bool DW, int KC, int NT, bool OUT>
 __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                            const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
                                            const float* __restrict__ pra1, const float* __restrict__ pa2, const float* __restrict__ pra2,
-                                           const uint16_t* __restrict__ pwp, const float* __restrict__ pAT, const float* __restrict__ pb2, const PwScalars p) {
+                                           const uint16_t* __restrict__ pwp, const float* __restrict__ pAT, const float* __restrict__ pb2, const PwScalars p, const CodecPlanes po,
+                                           const float* __restrict__ poa, const float* __restrict__ pora, uint16_t* __restrict__ pout) {
     constexpr int KG = KC / 8, MT = (C + 31) / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
     constexpr int XR = KC / 4, GS = KG * (NT / 64) / 4, XS = NT + 2 * CODEC_DW_HALO + 2, NS = (XS + 61) / 64;      // (XS - 2 columns in strips of 64)
                                // rows of x and (group, strip) pairs per wave
     __shared__ float xs[DW ? KC : 1][DW ? XS : 1];
-    __shared__ uint4 ts[3][KG][NT];
-    __shared__ uint4 As[APC];
+    __shared__ uint4 sm[3 * KG * NT + APC];
+    uint4 (&ts)[3][KG][NT] = *reinterpret_cast<uint4 (*)[3][KG][NT]>(sm);
+    uint4 (&As)[APC] = *reinterpret_cast<uint4 (*)[APC]>(sm + 3 * KG * NT);
     // The encoder's units take the place of k_x6_gemm in long rows only: a lane that sees a sum which is not finite takes its rows again as that kernel does
     constexpr bool RETAKE = DW && C <= 96;
-    constexpr bool SQ = C == 128;                         // 2 x 2 waves of 64 x 64; else every wave: all C rows x 32 columns
-    constexpr int MTW = SQ ? 2 : MT, NTW = SQ ? NT / 64 : 1;
-    static_assert(SQ || NT == 128, "four waves of 32 columns");
+    constexpr bool SQ = C == 128 || NT == 64;             // 2 x 2 waves of half the rows and half the columns; else every wave: all C rows x 32 columns
+    constexpr int MTW = SQ ? MT / 2 : MT, NTW = SQ ? NT / 64 : 1;
+    static_assert(SQ ? MT % 2 == 0 : NT == 128, "2 x 2 waves, or four of 32 columns");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = blockIdx.x * NT, b = blockIdx.y;
-    const int wr = SQ ? (wave >> 1) * 2 : 0;              // first row tile / first column of the wave's tile
+    const int wr = SQ ? (wave >> 1) * MTW : 0;              // first row tile / first column of the wave's tile
     const int wc = SQ ? (wave & 1) * (NT / 2) : wave * 32;
     const float* xb = pX + (size_t)b * C * p.ldx;
     const int T = p.T, halo = 3 * p.dil, ncols = NT + 2 * halo;
@@ -210,6 +213,44 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
     // epilogue: + bias + residual (C/D layout: col = lane & 31, row = (r & 3) + 8 (r >> 2) + 4 (lane >> 5))
     const float* rb = pR + (size_t)b * C * p.ldr;
     float* yb = pY + (size_t)b * C * p.ldy;
+    if constexpr (OUT) {                                       // as the operand of the contraction behind, and in f32 where something else reads it; the next tile's residual requested ahead
+        static_assert(sizeof(sm) >= 4 * CP_LDS(2) * sizeof(uint16_t), "the staging buffers hold the waves' output tiles");
+        uint16_t* st = reinterpret_cast<uint16_t*>(sm) + wave * CP_LDS(2);
+        __syncthreads();                                       // (the other waves' products)
+        float e[2][16];
+        auto want = [&](int t, float (&v)[16]) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) v[r] = rb[(size_t)((wr + t / NTW) * 32 + (r & 3) + 8 * (r >> 2) + 4 * (lane >> 5)) * p.ldr + min(n0 + wc + t % NTW * 32 + (lane & 31), T - 1)];
+        };
+        want(0, e[0]);
+#pragma unroll
+        for (int t = 0; t < MTW * NTW; ++t) {
+            const int mi = t / NTW, ni = t % NTW, nb = n0 + wc + ni * 32, n = nb + (lane & 31);
+            if (t + 1 < MTW * NTW) want(t + 1, e[(t + 1) & 1]);
+#pragma unroll
+            for (int r0 = 0; r0 < 16; r0 += 8) {
+                const int m0 = (wr + mi) * 32 + 2 * r0 + 4 * (lane >> 5);
+                float y[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) y[r] = e[t & 1][r0 + r] + (acc[mi][ni][r0 + r] + pb2[m0 + (r & 3) + 8 * (r >> 2)]);
+                if (pY && n < T) {
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) yb[(size_t)(m0 + (r & 3) + 8 * (r >> 2)) * p.ldy + n] = y[r];
+                }
+                if (poa) {
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) { const int m = m0 + (r & 3) + 8 * (r >> 2); y[r] = x6_snake(y[r], poa[m], pora[m]); }
+                }
+                codec_tile_put<2>(y, st, r0, lane);
+            }
+            codec_tile_flush<2>(st, pout + (size_t)b * po.Tp * C + (wr + mi) * 32, po.stride, C, lane, [&](int c) {
+                const int r = nb + c - po.t_org;
+                return nb + c < T && r < po.Tp ? r : -1;
+            });
+        }
+        codec_plane_ends(po, b, T, 0, C, n0 == 0, n0 + NT >= T, tid, 256);
+        return;
+    }
 #pragma unroll
     for (int ni = 0; ni < NTW; ++ni) {
         const int n = n0 + wc + ni * 32 + (lane & 31);
@@ -249,27 +290,37 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
         }
     }
 }
-template <int C, bool DW, int KC, int NT>
-__global__ void __launch_bounds__(256, KC == 32 ? 2 : DW && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp) {
-    pw_x6_body<C, DW, KC, NT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy});
+template <int C, bool DW, int KC, int NT, bool OUT>
+__global__ void __launch_bounds__(256, KC == 32 ? 2 : DW && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
+    pw_x6_body<C, DW, KC, NT, OUT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy}, o, o.alpha, o.ralpha, o.p);
 }
 
 // 128 channels, at most 256 blocks of 128 columns (a compute unit each, one serial chain of chunks): 64 columns per block.  96 blocks: 28 -> 22 us;
 // 192 and 248: 23 and 25 (384 of 128 columns: 34).  (The next chunk's loads ahead of this one's products instead: 31 us, no registers left.)
 // Chunk depth (the same bits): 32 channels need half the barriers, 16 let three or four blocks (not two, C = 96: three) share a compute unit.  32 while its
 // blocks are all resident at once, else 16 (us, chunks of 32 / 16): 128 channels 96 blocks 28 / 33, 384: 34 / 38, 576: 61 / 45, 24576: 1584 / 1430;
-// 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150 (with taps 16: 592 blocks, two rounds of 32).  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32.
+// 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150 (with taps 16: 592 blocks, two rounds of 32).  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32;
+// up to 512 blocks 64 columns (half the conversions and accumulators per thread, three blocks a compute unit): 313 blocks with planes out 50 -> 42.
 template <int C, bool DW>
 static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hipStream_t s) {
     const dim3 grid((p.T + 127) / 128, batch);
+#define X6_GO(KC, NT) do { \
+        const dim3 g((p.T + NT - 1) / NT, batch); \
+        if (!DW && p.out) hipLaunchKernelGGL((k_pw_x6<C, DW, KC, NT, !DW>), g, dim3(256), 0, s, p, wp, *p.out); \
+        else hipLaunchKernelGGL((k_pw_x6<C, DW, KC, NT, false>), g, dim3(256), 0, s, p, wp, CodecPlanes{}); \
+        return; } while (0)
     if constexpr (C == 128) {
-        if ((int64_t)grid.x * batch <= 256) { hipLaunchKernelGGL((k_pw_x6<C, DW, 32, 64>), dim3((p.T + 63) / 64, batch), dim3(256), 0, s, p, wp); return; }
+        if ((int64_t)grid.x * batch <= 256) X6_GO(32, 64);
     }
-    if constexpr (C == 48) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16, 128>), grid, dim3(256), 0, s, p, wp); return; }
+    if constexpr (C == 48) X6_GO(16, 128);
     else if constexpr (C <= 128) {
-        if ((int64_t)grid.x * batch > (C == 96 && !DW ? 768 : 512)) { hipLaunchKernelGGL((k_pw_x6<C, DW, 16, 128>), grid, dim3(256), 0, s, p, wp); return; }
+        if ((int64_t)grid.x * batch > (C == 96 && !DW ? 768 : 512)) X6_GO(16, 128);
     }
-    if constexpr (C != 48) hipLaunchKernelGGL((k_pw_x6<C, DW, 32, 128>), grid, dim3(256), 0, s, p, wp);
+    if constexpr (C == 192) {
+        if ((int64_t)grid.x * batch <= 512) X6_GO(32, 64);
+    }
+    if constexpr (C != 48) X6_GO(32, 128);
+#undef X6_GO
 }
 
 // 64 channels stay on k_pw_fused: twice the columns per product, bound by memory and by the units' VALU work (1.16 ms here, 1.10 there)
@@ -296,19 +347,23 @@ struct X6Gemm {
     GemmParams g;
     int mode, ntaps, nsteps, MT32;        // steps of 16 channels of one tap
     int nbx, my, per, tiles;              // column tiles, row tiles, tiles per XCD, all tiles
+    CodecPlanes out;
 };
 // QUARTERS (codec_quarters: K >= 1024): four partial sums.  The narrow form's four waves then share 32 columns and take a quarter of the steps each; the wide one
 // adds its accumulators to the total at the same steps, so a row's bits do not depend on which of them its length selects.
-template <int MTW, bool SNAKE, bool TAPS, bool WIDE, bool QUARTERS>
+template <class F, int... I>
+__device__ __forceinline__ void x6_each(F& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int MTW, bool SNAKE, bool TAPS, bool WIDE, bool QUARTERS, bool OUT>
 __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                              const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise,
                                              const float* __restrict__ pa, const float* __restrict__ pra, const float* __restrict__ pAT,
-                                             const uint16_t* __restrict__ pwp) {
+                                             const uint16_t* __restrict__ pwp, const float* __restrict__ poa, const float* __restrict__ pora, uint16_t* __restrict__ pout) {
     constexpr bool TIGHT = MTW == 8 || (MTW == 4 && QUARTERS), KSPLIT = QUARTERS && !WIDE;
     constexpr int PF = TIGHT ? 2 : 4, SPB = TIGHT ? 1 : 2;                  // steps of X (narrow: of weights too) in flight; steps per staged chunk of weights
     constexpr int NA = (SPB * MTW * 192 + 255) / 256, APC = SPB * MTW * 192;
     __shared__ x6_u4 As[WIDE ? 2 : 1][WIDE ? APC : 1];
     __shared__ float red[KSPLIT ? 4 : 1][KSPLIT ? 16 : 1][KSPLIT ? 64 : 1];
+    __shared__ __attribute__((aligned(16))) uint16_t tiles[OUT ? 4 : 1][OUT ? CP_LDS(2) : 1];
     extern __shared__ float x6_ab[];                                        // SNAKE: alpha [K], 1 / alpha [K]
     const GemmParams& p = P.g;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), kh = lane >> 5;
@@ -511,12 +566,13 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
     }
     int lane_hi = kh;                                                       // (opaque: the rows' addresses are not to be computed ahead of the contraction)
     asm volatile("" : "+v"(lane_hi));
-#pragma unroll
-    for (int mi = 0; mi < MTW; ++mi) {
-        if ((mt0 + mi) * 32 >= p.M) break;
+    [[maybe_unused]] uint16_t* st = tiles[OUT ? wave : 0];
+    auto tile = [&](auto index) {                                           // (a compile-time index: as a loop, eight tiles of this are not unrolled and the sums go to scratch)
+        constexpr int mi = decltype(index)::value;
+        if ((mt0 + mi) * 32 >= p.M) return;
         const int m0 = (mt0 + mi) * 32 + 4 * lane_hi + (KSPLIT ? 8 * wave : 0);
         if constexpr (WIDE) want(mi, lane_hi);
-        if (n >= p.N) continue;
+        if (!OUT && n >= p.N) return;
         auto finish = [&](float y, float b0, float s0, float e0) {
             y += pbias ? b0 : 0.0f;
             if (gelu) y = 0.5f * y * (1.0f + erff(y * 0.70710678118654752f));
@@ -530,13 +586,7 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
         float zero = 0.0f;
 #pragma unroll
         for (int r = 0; r < NR; ++r) zero = fmaf(acc[mi][r], 0.0f, zero);
-        if (zero == 0.0f) {
-#pragma unroll
-            for (int r = 0; r < NR; ++r) {
-                const int m = m0 + (r & 3) + 8 * (r >> 2);
-                if (m < p.M) y[(size_t)m * p.ldy] = finish(acc[mi][r], bm[r], pscale ? sc[r] : 0.0f, eb ? e[r] : 0.0f);
-            }
-        } else {
+        if (zero != 0.0f && n < p.N) {
             const int T = TAPS ? P.ntaps : 1;
 #pragma unroll 1
             for (int r = 0; r < NR; ++r) {
@@ -552,17 +602,45 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
                     v = fmaf(pAT[((size_t)j * Kx + c) * p.M + m], x, v);
                     if (v != v) break;                                      // (NaN it stays)
                 }
-                y[(size_t)m * p.ldy] = finish(v, pbias ? pbias[m] : 0.0f, pscale ? pscale[m] : 0.0f, eb ? eb[(size_t)m * lde + n] : 0.0f);
+#pragma unroll
+                for (int q = 0; q < NR; ++q) acc[mi][q] = q == r ? v : acc[mi][q];
             }
         }
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int m = m0 + (r & 3) + 8 * (r >> 2);
+            acc[mi][r] = finish(acc[mi][r], bm[r], pscale ? sc[r] : 0.0f, eb ? e[r] : 0.0f);
+            if ((!OUT || (pY && n < p.N)) && m < p.M) y[(size_t)m * p.ldy] = acc[mi][r];
+        }
+        if constexpr (OUT) {                                                // also (pY null: only) as the operand of the contraction behind
+#pragma unroll
+            for (int r0 = 0; r0 < 16; r0 += 8) {
+                float o[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    const int m = m0 + 2 * r0 + (r & 3) + 8 * (r >> 2);
+                    o[r] = acc[mi][r0 + r];
+                    if (poa) o[r] = x6_snake(o[r], poa[m], pora[m]);
+                }
+                codec_tile_put<2>(o, st, r0, lane);
+            }
+            codec_tile_flush<2>(st, pout + (size_t)b * P.out.Tp * P.out.Cp + (mt0 + mi) * 32, P.out.stride, P.out.Cp, lane, [&](int c) {
+                const int nn = n - (lane & 31) + c, r = nn - P.out.t_org;
+                return nn < p.N && r < P.out.Tp ? r : -1;
+            });
+        }
+    };
+    x6_each(tile, std::make_integer_sequence<int, MTW>{});
+    if constexpr (OUT) {                                                    // (the narrow form's other waves may be gone)
+        if (wave == 0) codec_plane_ends(P.out, b, p.Tout, mt0 * 32, min(MTW * 32, p.M - mt0 * 32), bx == 0, bx == P.nbx - 1, lane, 64);
     }
 }
-template <int MTW, bool SNAKE, bool TAPS, bool WIDE, bool QUARTERS>
+template <int MTW, bool SNAKE, bool TAPS, bool WIDE, bool QUARTERS, bool OUT>
 __global__ void __launch_bounds__(256, 2) k_x6_gemm(X6Gemm P, const uint16_t* wp) {
-    x6_gemm_body<MTW, SNAKE, TAPS, WIDE, QUARTERS>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.g.alpha, P.g.ralpha, P.g.AT, wp);
+    x6_gemm_body<MTW, SNAKE, TAPS, WIDE, QUARTERS, OUT>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.g.alpha, P.g.ralpha, P.g.AT, wp, P.out.alpha, P.out.ralpha, P.out.p);
 }
 
-template <bool SNAKE, bool TAPS>
+template <bool SNAKE, bool TAPS, bool OUT>
 static void launch_x6_gemm(X6Gemm P, const uint16_t* wp, int batch, hipStream_t s) {
     const GemmParams& p = P.g;
     P.nbx = (p.N + 127) / 128;
@@ -584,22 +662,24 @@ static void launch_x6_gemm(X6Gemm P, const uint16_t* wp, int batch, hipStream_t 
             // rows (456, 912) 336 / 469 / 583; 128 rows, K = 3072, 16000 columns (250 of 2) 146 / 110 / 123; 192 rows, K = 1152, 18944 columns (296, 444) 94 / 71 / 97,
             // eight such rows 444 / 437 / 733; 768 rows, K = 9216, 296 columns 394 / 299 / 59 (f32: 94)
             // (strided convolutions of three taps then; on two, narrow: 384 rows, K = 3072, 2368 columns 72, 768 rows, K = 6144, 296 columns 45)
-            if (P.MT32 > 2 && blocks(4) >= 384) go(k_x6_gemm<4, SNAKE, TAPS, true, true>, 4);
-            else if (blocks(2) >= 192) go(k_x6_gemm<2, SNAKE, TAPS, true, true>, 2);
+            if (P.MT32 > 2 && blocks(4) >= 384) go(k_x6_gemm<4, SNAKE, TAPS, true, true, false>, 4);
+            else if (blocks(2) >= 192) go(k_x6_gemm<2, SNAKE, TAPS, true, true, false>, 2);
             else {
                 P.nbx = (p.N + 31) / 32;
-                go(k_x6_gemm<1, SNAKE, TAPS, false, true>, 1);
+                go(k_x6_gemm<1, SNAKE, TAPS, false, true, false>, 1);
             }
             return;
         }
     }
-    if (P.MT32 > 4 && blocks(8) >= 512) go(k_x6_gemm<8, SNAKE, TAPS, true, false>, 8);
-    else if (P.MT32 > 2 && blocks(4) >= 512) go(k_x6_gemm<4, SNAKE, TAPS, true, false>, 4);
-    else if (blocks(2) >= 256) go(k_x6_gemm<2, SNAKE, TAPS, true, false>, 2);
-    else go(k_x6_gemm<1, SNAKE, TAPS, false, false>, 1);
+    if (P.MT32 > 4 && blocks(8) >= 512) go(k_x6_gemm<8, SNAKE, TAPS, true, false, OUT>, 8);
+    else if (P.MT32 > 2 && blocks(4) >= 512) go(k_x6_gemm<4, SNAKE, TAPS, true, false, OUT>, 4);
+    else if (blocks(2) >= 256) go(k_x6_gemm<2, SNAKE, TAPS, true, false, OUT>, 2);
+    else go(k_x6_gemm<1, SNAKE, TAPS, false, false, OUT>, 1);
 }
 
-bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s) {
+bool codec_x6_writes_planes(int mode, const GemmParams& p) { return mode == GEMM_RESID && p.M % 32 == 0; }
+
+bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s, const CodecPlanes* out) {
     GemmParams p = p_in;
     CodecPack* pack = p.pack ? p.pack : codec_x6_scope();
     const bool taps = mode == GEMM_TAPS;
@@ -613,9 +693,12 @@ bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hip
     const CodecPack::X6& e = pack->get_x6(p.AT, ntaps, Cin, p.M, s);
     X6Gemm P{};
     P.g = p; P.mode = mode; P.ntaps = ntaps; P.nsteps = e.KS * ntaps; P.MT32 = e.MT32;
-    if (taps) launch_x6_gemm<false, true>(P, e.wp, batch, s);
-    else if (snake) launch_x6_gemm<true, false>(P, e.wp, batch, s);
-    else launch_x6_gemm<false, false>(P, e.wp, batch, s);
+    if (out) P.out = *out;
+    if (taps) launch_x6_gemm<false, true, false>(P, e.wp, batch, s);
+    else if (out && snake) launch_x6_gemm<true, false, true>(P, e.wp, batch, s);
+    else if (out) launch_x6_gemm<false, false, true>(P, e.wp, batch, s);
+    else if (snake) launch_x6_gemm<true, false, false>(P, e.wp, batch, s);
+    else launch_x6_gemm<false, false, false>(P, e.wp, batch, s);
     return true;
 }
 

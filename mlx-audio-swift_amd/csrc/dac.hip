@@ -392,10 +392,11 @@ static const float* dac_run(mis_dac* c, const int32_t* codes_dev, int batch, int
         return g;
     };
     hipLaunchKernelGGL(k_dac_embed, dim3(cdiv(T, 32), cdiv(c->latent, 32), batch), dim3(256), 0, s, codes_dev, W + c->tables, x, cf.n_codebooks, cf.codebook_size, c->latent, T);
+    std::vector<CodecOp> ops;
     {
         GemmParams g = gp(c->first, x, y, T, T, T);
         g.Cin = c->latent; g.taps = 7; g.dil = 1; g.pad = 3;
-        launch_gemm(GEMM_TAPS, false, g, batch, s);
+        ops.push_back({GEMM_TAPS, false, false, g});
         std::swap(x, y);
     }
     int64_t Tc = T;
@@ -404,22 +405,27 @@ static const float* dac_run(mis_dac* c, const int32_t* codes_dev, int batch, int
         const int64_t To = (Tc - 1) * B.s - 2 * B.pad + 2 * B.s + 1;
         GemmParams g = gp(B.ct, x, y, (int)((To + B.s - 1) / B.s), (int)Tc, (int)To);
         g.s = B.s; g.pad = B.pad; g.Cin = B.cin; g.alpha = W + B.a; g.ralpha = W + B.ra;
-        launch_gemm(GEMM_CONVT, true, g, batch, s);
+        ops.push_back({GEMM_CONVT, true, true, g});                          // (kept: the first unit's residual)
         Tc = To;
         std::swap(x, y);
         for (int ri = 0; ri < 3; ++ri) {
             const auto& R = B.ru[ri];
             GemmParams g1 = gp(R.c1, x, t1, (int)Tc, (int)Tc, (int)Tc);
             g1.Cin = B.cout; g1.taps = 7; g1.dil = R.dil; g1.pad = 3 * R.dil; g1.alpha = W + R.a1; g1.ralpha = W + R.ra1;
-            launch_gemm(GEMM_TAPS, true, g1, batch, s);
+            ops.push_back({GEMM_TAPS, true, false, g1});
             GemmParams g2 = gp(R.c2, t1, y, (int)Tc, (int)Tc, (int)Tc);
             g2.R = x; g2.alpha = W + R.a2; g2.ralpha = W + R.ra2;
-            launch_gemm(GEMM_RESID, true, g2, batch, s);
+            ops.push_back({GEMM_RESID, true, ri < 2, g2});
             std::swap(x, y);
         }
-        if (stage == 1 + bi) { *outC = B.cout; *outT = Tc; return x; }
+        if (stage == 1 + bi) {
+            launch_gemm_chain(ops.data(), (int)ops.size(), batch, s);
+            *outC = B.cout; *outT = Tc;
+            return x;
+        }
         ++bi;
     }
+    launch_gemm_chain(ops.data(), (int)ops.size(), batch, s);
     // DescriptDAC.swift:146-148
     launch_codec_final(x, wav_dev, wav_stride, W + c->fin_w, 1, c->fin_c, c->fin_b, W + c->fin_a, W + c->fin_ra, batch, c->fin_c, (int)Tc, s);
     HIP_CHECK(hipGetLastError());

@@ -1348,7 +1348,7 @@ void launch_vq_residual(float* r, const int32_t* codes, const float* table, int 
     hipLaunchKernelGGL(k_vq_residual, dim3(cdiv(T, 256), C, batch), dim3(256), 0, s, r, codes, table, C, T, stride);
 }
 
-void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s) {
+bool launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s, const CodecPlanes* out, bool keep) {
     GemmParams p = p_in;
     if (!p.ldx) p.ldx = p.Tin;                                          // dense [B][C][T] tensors unless the caller says otherwise
     if (!p.ldy) p.ldy = p.Tout;
@@ -1359,19 +1359,33 @@ void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
         PwFusedParams fp{};
         fp.X = p.X; fp.R = p.R; fp.Y = p.Y; fp.a2 = p.alpha; fp.ra2 = p.ralpha; fp.AT = p.AT; fp.b2 = p.bias;
         fp.T = p.N; fp.dil = 0; fp.ldx = p.ldx; fp.ldr = p.ldy; fp.ldy = p.ldy;
-        if (launch_pw_x6(p.M, false, fp, p.pack, batch, s)) return;
+        fp.out = out;
+        if (out && !keep) fp.Y = nullptr;
+        if (launch_pw_x6(p.M, false, fp, p.pack, batch, s)) return out != nullptr;
+        fp.Y = p.Y;
         dim3 fg(cdiv(p.N, RU_NT), batch);
         if (p.M == 64) hipLaunchKernelGGL((k_pw_fused<64, false, 32>), fg, dim3(256), 0, s, fp);
         else if (p.M == 96) hipLaunchKernelGGL((k_pw_fused<96, false, 32>), fg, dim3(256), 0, s, fp);
         else if (p.M == 128) hipLaunchKernelGGL((k_pw_fused<128, false, 32>), fg, dim3(256), 0, s, fp);
         else hipLaunchKernelGGL((k_pw_fused<192, false, 32>), fg, dim3(256), 0, s, fp);
-        return;
+        return false;
     }
-    if (launch_gemm_bf3(mode, snake, p, batch, s)) return;
+    {
+        GemmParams g = p;
+        const CodecPlanes* o = out && bf3_writes_planes(mode, p) ? out : nullptr;
+        if (o && !keep) g.Y = nullptr;
+        if (launch_gemm_bf3(mode, snake, g, batch, s, nullptr, o)) return o != nullptr;
+    }
     MIS_REQUIRE(mode != GEMM_TAPS || (p.taps >= 1 && p.taps <= CT_MAXT && (p.taps - 1) * p.dil + 3 + G_BN <= CT_XS), MIS_ERR_INVALID_INPUT,
                 "dense conv: %d taps with dilation %d exceed the staged halo", p.taps, p.dil);
-    if (launch_gemm_x6(mode, snake, p, batch, s) || (mode == GEMM_CONVT && snake && launch_convt_x6(p, batch, s))) return;
-    if (mode != GEMM_CONVT && (mode != GEMM_TAPS || !snake)) { launch_gemm_f32(mode, snake, p, batch, s); return; }
+    {
+        GemmParams g = p;
+        const CodecPlanes* o = out && codec_x6_writes_planes(mode, p) ? out : nullptr;
+        if (o && !keep) g.Y = nullptr;
+        if (launch_gemm_x6(mode, snake, g, batch, s, o)) return o != nullptr;
+    }
+    if (mode == GEMM_CONVT && snake && launch_convt_x6(p, batch, s)) return false;
+    if (mode != GEMM_CONVT && (mode != GEMM_TAPS || !snake)) { launch_gemm_f32(mode, snake, p, batch, s); return false; }
     const int phases = mode == GEMM_CONVT ? p.s : 1;
     dim3 grid(cdiv(p.N, G_BN), cdiv(p.M, G_BM), batch * phases), block(256);
     if (mode == GEMM_TAPS) {             // dense conv with Snake in front: the activation runs once per staged element
@@ -1379,6 +1393,7 @@ void launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
         else hipLaunchKernelGGL((k_conv_taps<false>), grid, block, 0, s, p);
     }
     else { MIS_REQUIRE(snake, MIS_ERR_GENERATION_FAILED, "convT without snake"); hipLaunchKernelGGL(k_snac_convt, grid, block, 0, s, p); }
+    return false;
 }
 
 static int64_t mis_snac_hop_for_encoder(const mis_snac* c) {
@@ -1436,6 +1451,7 @@ static const float* snac_run(mis_snac* c, const int32_t* const* codes, int batch
     ep.n_q = cf.n_codebooks; ep.codebook_size = cf.codebook_size; ep.C = cf.latent_dim; ep.T0 = (int)T0;
     hipLaunchKernelGGL(k_snac_embed, dim3(cdiv(T0, 32), cdiv(cf.latent_dim, 32), batch), dim3(256), 0, s, ep, A);
     if (stop_after == 0) { *outC = cf.latent_dim; *outT = T0; return A; }
+    std::vector<CodecOp> chain;                              // what only the next transposed convolution reads
     // stem: depthwise k7 then 1x1 (Layers.swift:378-388)
     hipLaunchKernelGGL((k_snac_dw<false, false>), dim3(cdiv(T0, DW_TILE), cf.latent_dim, batch), dim3(256), 0, s,
                        A, B, W + c->stem_dw.w, W + c->stem_dw.b, nullptr, nullptr, nullptr, nullptr, cf.latent_dim, (int)T0, 1);
@@ -1444,7 +1460,8 @@ static const float* snac_run(mis_snac* c, const int32_t* const* codes, int batch
         GemmParams g{};
         g.AT = W + c->stem_pw.w; g.bias = W + c->stem_pw.b; g.X = B; g.Y = A;
         g.M = cf.decoder_dim; g.K = cf.latent_dim; g.N = (int)T0; g.Tin = (int)T0; g.Tout = (int)T0;
-        launch_gemm(GEMM_PLAIN, false, g, batch, s);
+        if (stop_after == 2 || c->dec_attn.on) launch_gemm(GEMM_PLAIN, false, g, batch, s);
+        else chain.push_back({GEMM_PLAIN, false, false, g});
     }
     if (stop_after == 2) { *outC = cf.decoder_dim; *outT = T0; return A; }
     float* x = A;        // current activation
@@ -1466,7 +1483,9 @@ static const float* snac_run(mis_snac* c, const int32_t* const* codes, int batch
             g.M = blk.cout; g.K = 2 * blk.cin; g.Tin = (int)T; g.Tout = (int)To;
             g.s = blk.stride; g.pad = blk.pad; g.Cin = blk.cin;
             g.N = (int)((To + blk.stride - 1) / blk.stride);     // columns per phase; stores are bounds-checked
-            launch_gemm(GEMM_CONVT, true, g, batch, s);
+            chain.push_back({GEMM_CONVT, true, true, g});
+            launch_gemm_chain(chain.data(), (int)chain.size(), batch, s);
+            chain.clear();
         }
         std::swap(x, f1);
         T = To;
@@ -1503,7 +1522,8 @@ static const float* snac_run(mis_snac* c, const int32_t* const* codes, int batch
             GemmParams g{};
             g.AT = W + ru.pw.w; g.bias = W + ru.pw.b; g.X = f1; g.Y = f2; g.R = x;
             g.M = blk.cout; g.K = blk.cout; g.N = (int)T; g.Tin = (int)T; g.Tout = (int)T;
-            launch_gemm(GEMM_RESID, false, g, batch, s);
+            if (j < 2 || bi + 1 == c->blocks.size() || stop_after == 3 + (int)bi) launch_gemm(GEMM_RESID, false, g, batch, s);
+            else chain.push_back({GEMM_RESID, false, false, g});
             std::swap(x, f2);
         }
         if (stop_after == 3 + (int)bi) { *outC = blk.cout; *outT = T; return x; }
