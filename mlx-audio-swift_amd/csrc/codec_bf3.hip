@@ -23,7 +23,9 @@
 //
 // Between two contractions the planes come from the epilogue in front (launch_gemm_chain): Snake and the split run there, on registers, and the pre-pass - a launch, a read and a
 // write of the tensor - is gone, with the f32 tensor where nothing else reads it.  DAC, one row of 30 / 250 frames, four of 400: 951 / 1688 / 8060 -> 748 / 1472 / 7490 us.
-// An operand may have three planes instead (NP = 3, the arithmetic and the bits of codec_x6.hip): the 1x1 contractions of 193 .. 384 channels behind Snake, which k_x6_gemm converts
+// An operand may have three planes instead (NP = 3, the arithmetic and the bits of codec_x6.hip): the strided convolutions of SNAC's encoder, whose phase split writes them
+// (k_enc_phase_planes; k_x6_gemm converts a column once per block of rows: 96 / 192 / 384 / 768 rows of one recording of 151111 samples 46 + 52 + 71 + 44 us, 33 + 39 + 46 + 31 here, and
+// 7 more in the phase splits), and the 1x1 contractions of 193 .. 384 channels behind Snake, which k_x6_gemm converts
 // once per 64 rows (384 x 384, 10005 columns: 45 us, 52 with planes out; 34 here).  Of up to 192 channels k_pw_x6 converts once in all and reads four bytes, not six: 192 channels,
 // 40021 columns: 42 us there, 43 here and 4 more in front; 96, 80043 columns: 36 and 41.
 #include "common.h"
@@ -152,10 +154,23 @@ template <int NV, int ND, int NM> __device__ __forceinline__ void bf3_interleave
     }
 }
 
+// One output of a three-plane contraction as the f32 kernels make it: 16 channels, within them the taps (a column each), within a tap the channels; NaN it stays
+__device__ __forceinline__ float bf3_retake(const uint16_t* __restrict__ x, size_t plane, int Cp, const float* __restrict__ at, int Cin, int M, int ntaps) {
+    float v = 0.0f;
+#pragma unroll 1
+    for (int i = 0; i < Cin * ntaps && v == v; ++i) {
+        const int c = i / (16 * ntaps) * 16 + (i & 15), j = i / 16 % ntaps;
+        const uint16_t* q = x + (size_t)j * Cp + c;
+        const float hm = bf16_to_f32(q[0]) + bf16_to_f32(q[plane]);
+        v = fmaf(at[((size_t)j * Cin + c) * M], fabsf(hm) < INFINITY ? hm + bf16_to_f32(q[2 * plane]) : hm, v);
+    }
+    return v;
+}
+
 // The body takes the arrays the epilogue touches as restrict-qualified PARAMETERS: GemmParams is a struct, clang ignores restrict on
 // struct members, and without it every bias / residual load of the epilogue waits behind the previous row's store (the same effect
 // cost the fused unit kernel of snac.hip 25 %).
-template <int NP, int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, bool OUT>
+template <int NP, int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, bool QUARTERS, bool OUT>
 __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                          const float* __restrict__ pbias, const float* __restrict__ pscale, const float* __restrict__ pnoise,
                                          const float* __restrict__ poa, const float* __restrict__ pora, uint16_t* __restrict__ pout) {
@@ -179,7 +194,7 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
     int phase = 0, sh0 = 0, dsh = 0, tapbase = 0, slice = 0;
     if (P.mode == GEMM_CONVT) { phase = in; sh0 = (phase + p.pad) / p.s; dsh = -1; tapbase = phase * NTAPS; }
     else if (P.mode == GEMM_TAPS) { sh0 = -p.pad; dsh = p.dil; }
-    else if (P.ksplit > 1) slice = in;
+    if (P.ksplit > 1) slice = in;
     const int shmin = min(sh0, sh0 + (NTAPS - 1) * dsh);
     const int nchunks_all = P.Cp / B3_KC;
     const int c_lo = P.ksplit > 1 ? nchunks_all * slice / P.ksplit : 0;                        // this block's chunks (split-K: a slice of them)
@@ -263,8 +278,11 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                     acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.v[mi][ta], B.v[ni][tb], acc[mi][ni], 0, 0, 0);
         }
     };
+    // a chunk's steps: tap by tap; three planes: 16 channels at a time, within them the taps (k_x6_gemm's order)
+    constexpr auto TAP = [](int t) { return NP == 2 ? t >> 1 : t % NTAPS; };
+    constexpr auto KSTEP = [](int t) { return NP == 2 ? t & 1 : t / NTAPS; };
 #pragma unroll
-    for (int J = 0; J < AR - 1; ++J) loadA(aq[J], J / NST, (J % NST) >> 1, J & 1);
+    for (int J = 0; J < AR - 1; ++J) loadA(aq[J], J / NST, TAP(J % NST), KSTEP(J % NST));
     const uint16_t* tile = lds;
     int gbuf = 0;                                           // ring slot of the next chunk
     const float* Xb = pX + (size_t)b * p.Cin * p.ldx;
@@ -290,7 +308,24 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
         int cc = 0;
+        f32x16_t tot[QUARTERS ? MI : 1][QUARTERS ? NI : 1];
+        [[maybe_unused]] auto close_quarter = [&](bool first) {              // (a sum that starts at 0 is never -0: the first may be taken over)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        tot[QUARTERS ? i : 0][QUARTERS ? j : 0][r] = first ? acc[i][j][r] : tot[QUARTERS ? i : 0][QUARTERS ? j : 0][r] + acc[i][j][r];
+                        acc[i][j][r] = 0.0f;
+                    }
+        };
+        [[maybe_unused]] int quarter = 1;
+        static_assert(!QUARTERS || CG == 1, "a quarter ends where a group does");
         for (; cc + CG <= nchunks; cc += CG) {
+            if constexpr (QUARTERS) {
+                if (quarter < 4 && cc == nchunks * quarter / 4) { close_quarter(quarter == 1); ++quarter; }
+            }
 #pragma unroll
             for (int I = 0; I < CG * NST; ++I) {
                 const int t = I % NST;
@@ -304,9 +339,9 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                 // them next to their use), and inside it they are spread over the shadows of the MFMAs instead of running ahead
                 // of them with the matrix pipe idle: MFMA, then a weight load or a tile read with its address arithmetic
                 __builtin_amdgcn_sched_barrier(0);
-                if (t + 1 < NST) readB(bq[(I + 1) & 1], tile, (t + 1) >> 1, (t + 1) & 1);
+                if (t + 1 < NST) readB(bq[(I + 1) & 1], tile, TAP(t + 1), KSTEP(t + 1));
                 const int J = I + AR - 1;
-                loadA(aq[J % AR], cc + J / NST, (J % NST) >> 1, J & 1);
+                loadA(aq[J % AR], cc + J / NST, TAP(J % NST), KSTEP(J % NST));
                 products(aq[I % AR], bq[I & 1]);
                 bf3_interleave<NP * MI, ND, NPROD * MI * NI - NP * MI - ND>();
                 __builtin_amdgcn_sched_barrier(0);
@@ -326,9 +361,9 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                         readB(bq[I & 1], tile, 0, 0);
                     }
                     __builtin_amdgcn_sched_barrier(0);
-                    if (t + 1 < NST) readB(bq[(I + 1) & 1], tile, (t + 1) >> 1, (t + 1) & 1);
+                    if (t + 1 < NST) readB(bq[(I + 1) & 1], tile, TAP(t + 1), KSTEP(t + 1));
                     const int J = I + AR - 1;
-                    loadA(aq[J % AR], cc + J / NST, (J % NST) >> 1, J & 1);
+                    loadA(aq[J % AR], cc + J / NST, TAP(J % NST), KSTEP(J % NST));
                     products(aq[I % AR], bq[I & 1]);
                     bf3_interleave<NP * MI, ND, NPROD * MI * NI - NP * MI - ND>();
                     __builtin_amdgcn_sched_barrier(0);
@@ -336,6 +371,13 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
             }
         }
 
+        if constexpr (QUARTERS) {
+            close_quarter(false);
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NI; ++j) acc[i][j] = tot[i][j];
+        }
         // ---- epilogue (the modes of k_codec_gemm / k_conv_taps / k_snac_convt).  C/D layout: col = lane & 31, row = (r & 3) + 8 (r >> 2) + 4 (lane >> 5)
         // opaque: left visible, the 32 rows' 64-bit offsets are computed ahead of the main loop and spilled (860 B of scratch per
         // lane in the multi-tile experiment: 1.9x slower)
@@ -371,14 +413,7 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
 #pragma unroll 1
                     for (int r = 0; r < 16; ++r) {
                         const int m = (mt0 + mi) * 32 + (r & 3) + 8 * (r >> 2) + 4 * lane_hi;
-                        float v = 0.0f;
-#pragma unroll 1
-                        for (int i = 0; i < P.Cp * NTAPS && m < p.M && v == v; ++i) {       // 16 channels, within them the taps, within a tap the channels (NaN it stays)
-                            const int c = i / (16 * NTAPS) * 16 + (i & 15), j = i / 16 % NTAPS;
-                            const uint16_t* x = P.xp + ((size_t)b * P.Tp + (n + sh0 + j * dsh - P.t_org)) * P.Cp + c;
-                            const float hm = bf16_to_f32(x[0]) + bf16_to_f32(x[P.xplane]), xv = fabsf(hm) < INFINITY ? hm + bf16_to_f32(x[2 * P.xplane]) : hm;
-                            if (c < p.Cin) v = fmaf(p.AT[((size_t)j * p.Cin + c) * p.M + m], xv, v);
-                        }
+                        const float v = m < p.M ? bf3_retake(P.xp + ((size_t)b * P.Tp + (n + sh0 - P.t_org)) * P.Cp, P.xplane, P.Cp, p.AT + m, p.Cin, p.M, NTAPS) : 0.0f;
 #pragma unroll
                         for (int q = 0; q < 16; ++q) acc[mi][ni][q] = q == r ? v : acc[mi][ni][q];
                     }
@@ -487,19 +522,22 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
     }
 }
 
-template <int NP, int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, int MINW, bool OUT>
+template <int NP, int MI, int NI, int NQ, int NBUF, int NTAPS, int AR, int MINW, bool QUARTERS, bool OUT>
 __global__ void __launch_bounds__(B3_THREADS, MINW) k_bf3_gemm(Bf3Params P) {
-    bf3_body<NP, MI, NI, NQ, NBUF, NTAPS, AR, OUT>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.out.alpha, P.out.ralpha, P.out.p);
+    bf3_body<NP, MI, NI, NQ, NBUF, NTAPS, AR, QUARTERS, OUT>(P, P.g.X, P.g.R, P.g.Y, P.g.bias, P.g.scale, P.g.noise, P.out.alpha, P.out.ralpha, P.out.p);
 }
 
-// split-K: Y = epilogue(sum over slices in slice order + bias) - the 1x1 modes' epilogues of bf3_body (plain / GELU / residual with scale)
+// split-K: Y = epilogue(sum over slices in slice order + bias) - the 1x1 modes' epilogues of bf3_body (plain / GELU / residual with scale).  xp: three planes, whose sums
+// that are not finite are taken again (taps at consecutive columns)
 __global__ void k_bf3_splitk_epilogue(const float* __restrict__ part, int S, int batch, int mode, const float* __restrict__ bias, const float* __restrict__ scale,
-                                      const float* __restrict__ R, float* __restrict__ Y, int M, int N, int ldy) {
+                                      const float* __restrict__ R, float* __restrict__ Y, int M, int N, int ldy, const uint16_t* __restrict__ xp, size_t xplane, int Tp, int Cp,
+                                      const float* __restrict__ at, int Cin, int ntaps) {
     const int n = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y, b = blockIdx.z;
     if (n >= N) return;
     const size_t rowo = ((size_t)b * M + m) * ldy;
     float v = 0.0f;
     for (int s = 0; s < S; ++s) v += part[(((size_t)s * batch + b) * M + m) * ldy + n];
+    if (xp && !(fabsf(v) < INFINITY)) v = bf3_retake(xp + ((size_t)b * Tp + n) * Cp, xplane, Cp, at + m, Cin, M, ntaps);
     v += bias ? bias[m] : 0.0f;
     if (mode == GEMM_GELU) v = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
     if (mode == GEMM_RESID && R) { if (scale) v *= scale[m]; v += R[rowo + n]; }
@@ -542,10 +580,11 @@ bool codec_exact_f32() { return bf3_env("MIS_CODEC_EXACT_F32", 0) != 0; }
 // What the two-plane contractions take.  What pays: MFMA-bound shapes.  A 1x1 conv over few channels is HBM-bound and the pre-pass would only add traffic
 // (measured per dispatch, profiles/r02_codec/: 1x1 over <= 512 channels and the last SNAC transposed conv, M*K = 16 K,
 // are faster on the exact-f32 kernels; every 7-tap conv and the transposed convs from M*K = 36 K up gain 2.3 - 4x)
-struct Bf3Shape { int ntaps, Cin, span, t_org, wtaps, phases, extra; };
+struct Bf3Shape { int ntaps, Cin, span, t_org, wtaps, phases, extra, parts; };
 static bool bf3_shape(int mode, const GemmParams& p, Bf3Shape& h) {
     const bool one = mode == GEMM_PLAIN || mode == GEMM_GELU || mode == GEMM_RESID || mode == GEMM_NOISE;
-    h = Bf3Shape{1, p.K, 0, 0, 1, 1, 0};
+    h = Bf3Shape{1, p.K, 0, 0, 1, 1, 0, 1};
+    if (mode == GEMM_TAPS && p.taps == 2 && codec_quarters(p)) h.parts = 4;
     if (mode == GEMM_TAPS) { h.ntaps = p.taps; h.Cin = p.Cin; h.span = (p.taps - 1) * p.dil; h.t_org = -p.pad; h.wtaps = p.taps; }
     else if (mode == GEMM_CONVT) {
         if (p.Cin <= 0 || p.K % p.Cin || p.K / p.Cin > 2) return false;
@@ -567,12 +606,14 @@ static bool bf3_takes(int mode, const GemmParams& p, const Bf3Shape& h) {
 // The small tiles run alone on a compute unit, with registers to spare: weights seven (not two) steps ahead, which covers a trip to HBM.
 // us, 128 x 128 / 64 x 128 / 64 x 64: 768 rows, 7 taps of 768, 2080 columns: 102 / 60 / 79; 768 rows, K = 768: 51 / 24 / 26;
 // 1536 rows, 7 taps of 1024, 250 columns: 140 / 70 / 55; SNAC, one row of 12 groups: 48 / - / 19, 41 / 22 / 15, 33 / - / 14, 29 / 17 / 16.
+// A quarter of K a block (three planes, two taps of at least 512 channels): counted as the blocks they are, 64 x 64 up to 256 of 64 x 128 (us, 64 x 128 / 64 x 64: 384 rows,
+// K = 3072, 2361 columns, 456 blocks: 40 / 45; 768 rows, K = 6144, 296 columns, 144: 36 / 26; k_x6_gemm: 71, 44).
 struct Bf3Tile { bool few; int NI, nbx, nq, Tp; };
 static Bf3Tile bf3_tile(const GemmParams& p, const Bf3Shape& h, int batch) {
     const int nb128 = (p.N + 127) / 128;
     Bf3Tile t{};
-    t.few = (int64_t)nb128 * ((p.M + B3_BM - 1) / B3_BM) * batch * h.phases <= 128;
-    t.NI = t.few && (p.N <= 64 || (int64_t)nb128 * ((p.M + 63) / 64) * batch * h.phases <= 128) ? 1 : 2;
+    t.few = (int64_t)nb128 * ((p.M + B3_BM - 1) / B3_BM) * batch * h.phases * h.parts <= 128;
+    t.NI = t.few && (p.N <= 64 || (int64_t)nb128 * ((p.M + 63) / 64) * batch * h.phases * h.parts <= (h.parts > 1 ? 256 : 128)) ? 1 : 2;
     t.nbx = (p.N + 64 * t.NI - 1) / (64 * t.NI);
     t.nq = 4 * t.NI + (h.span == 0 ? 0 : h.span <= 16 ? 1 : 4);
     t.Tp = (t.nbx - 1) * 64 * t.NI + t.nq * 16 + h.extra;
@@ -580,6 +621,20 @@ static Bf3Tile bf3_tile(const GemmParams& p, const Bf3Shape& h, int batch) {
 }
 // Three planes, where the epilogue in front writes them: 1x1 contractions with Snake and a residual that k_x6_gemm would convert for itself
 static bool bf3_three(int mode, const GemmParams& p) { return mode == GEMM_RESID && p.alpha && p.M >= 48 && p.K > 192 && p.K <= 384; }
+
+// Strided convolutions of the encoders, on two taps of the phase split: three planes, written by k_enc_phase_planes
+bool codec_planes_strided(const GemmParams& p, int batch, CodecPlanes& out) {
+    CodecPack* pack = codec_x6_scope();
+    Bf3Shape h;
+    if (!pack || codec_exact_f32() || p.taps != 2 || p.dil != 1 || p.pad != 0 || p.Cin % 32 || p.M < 48 || !bf3_shape(GEMM_TAPS, p, h)) return false;
+    const Bf3Tile t = bf3_tile(p, h, batch);
+    out = CodecPlanes{};
+    out.n = 3; out.Cp = h.Cin; out.Tp = t.Tp;
+    out.stride = (size_t)batch * t.Tp * h.Cin;
+    pack->planes[0].alloc(3 * out.stride);
+    out.p = pack->planes[0].p;
+    return true;
+}
 
 bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot, CodecPlanes& out) {
     CodecPack* pack = p.pack ? p.pack : tl_pack;
@@ -606,7 +661,7 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
     Bf3Shape h;
     if (!bf3_shape(mode, p, h) || (!in && !bf3_takes(mode, p, h))) return false;
     if (out) {
-        MIS_REQUIRE(bf3_writes_planes(mode, p) && out->Cp == p.M, MIS_ERR_GENERATION_FAILED, "codec contraction: %d rows for an operand of %d channels", p.M, out->Cp);
+        MIS_REQUIRE(bf3_writes_planes(mode, p) && out->Cp == p.M && !(in && in->n == 3 && h.ntaps == 2), MIS_ERR_GENERATION_FAILED, "codec contraction: %d rows for an operand of %d channels", p.M, out->Cp);
     }
     const int ntaps = h.ntaps, Cin = h.Cin, span = h.span;
     const Bf3Tile t = bf3_tile(p, h, batch);
@@ -644,6 +699,9 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
         if (per_row <= 32 && nchunks >= 32) ksplit = 4;
         else if (per_row <= 64 && nchunks >= 16) ksplit = 2;
     }
+    // Three planes, K >= 1024: four partial sums in every form (codec_quarters), in blocks of their own while that is what fills the chip
+    const bool three = in && in->n == 3, quarters = three && ntaps == 2 && codec_quarters(p);
+    if (quarters && (int64_t)t.nbx * ((p.M + 63) / 64) * batch < 512) ksplit = 4;
     if (ksplit > 1) {
         p.pack->part.alloc((size_t)ksplit * batch * p.M * p.ldy);
         P.ksplit = ksplit; P.part = p.pack->part.p; P.batch = batch;
@@ -651,15 +709,19 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
     // Rows that are no multiple of 128 leave a wave row of the large tile without any, and its blocks (7 taps: one a compute unit) come in whole rounds: 64 x 128 there,
     // two blocks a compute unit.  us, 128 x 128 / 64 x 128: 192 rows, 7 taps, 40000 columns 91 / 63, 2 taps (5 phases) 62 / 54; 96 rows, 80000 columns 67 / 45, 47 / 39;
     // whole tiles: 384 rows, 7 taps, 10000 columns 60 / 64, 2 taps of 512 .. 128 rows (SNAC, 32 rows) 588 / 767, 1395 / 1748, 1734 / 1966
-    const bool three = in && in->n == 3, half = !few && (three || (ntaps != 1 && p.M % B3_BM != 0));
+    const bool half = !few && (three || (ntaps != 1 && p.M % B3_BM != 0));
     const int bm = few || half ? 64 : B3_BM;
     P.nbx = t.nbx; P.my = (p.M + bm - 1) / bm; P.inner = h.phases * ksplit;
     P.tiles = P.nbx * P.my * batch; P.per = (P.tiles + 7) / 8;
     const dim3 grid(8 * P.per * P.inner), block(B3_THREADS);
-#define B3_GO(...) do { \
-        if (out) hipLaunchKernelGGL((k_bf3_gemm<__VA_ARGS__, true>), grid, block, 0, s, P); \
-        else hipLaunchKernelGGL((k_bf3_gemm<__VA_ARGS__, false>), grid, block, 0, s, P); } while (0)
-    if (three) {
+#define B3_RUN(...) hipLaunchKernelGGL((k_bf3_gemm<__VA_ARGS__>), grid, block, 0, s, P)
+#define B3_GO(...) do { if (out) B3_RUN(__VA_ARGS__, false, true); else B3_RUN(__VA_ARGS__, false, false); } while (0)
+    if (three && ntaps == 2) {
+        if (NI == 1) B3_RUN(3, 1, 1, 5, 5, 2, 6, 2, false, false);
+        else if (quarters && ksplit == 1) B3_RUN(3, 1, 2, 9, 4, 2, 4, 2, true, false);
+        else B3_RUN(3, 1, 2, 9, 2, 2, 4, 3, false, false);
+    }
+    else if (three) {
         if (NI == 1) B3_GO(3, 1, 1, 4, 6, 1, 6, 2);
         else B3_GO(3, 1, 2, 8, 3, 1, 4, 3);
     }
@@ -684,9 +746,10 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
     else if (span <= 16) B3_GO(2, 2, 2, 9, 4, 7, 4, 2);
     else B3_GO(2, 2, 2, 12, 4, 7, 4, 2);
 #undef B3_GO
+#undef B3_RUN
     if (ksplit > 1)
         hipLaunchKernelGGL(k_bf3_splitk_epilogue, dim3((p.N + 255) / 256, p.M, batch), dim3(256), 0, s, P.part, ksplit, batch, mode, p.bias, p.scale, p.R, p.Y, p.M,
-                           p.N, p.ldy);
+                           p.N, p.ldy, three ? P.xp : nullptr, P.xplane, P.Tp, P.Cp, p.AT, Cin, ntaps);
     return true;
 }
 

@@ -92,6 +92,9 @@ struct CodecPackScope {
 CodecPack* codec_x6_scope();          // the innermost scope's, or null
 bool codec_exact_f32();               // MIS_CODEC_EXACT_F32=1
 
+// (strided convolutions: their input's, two taps)
+struct CodecPlanes;
+bool codec_planes_strided(const struct GemmParams& p, int batch, CodecPlanes& out);
 // An operand as bf16 planes, time-major: [n planes, stride elements apart][batch][Tp][Cp]; row r holds column r + t_org, through Snake where alpha is given.
 // ends: rows without a column are zero (an operand of one tap does not need them)
 struct CodecPlanes {
@@ -105,22 +108,26 @@ struct CodecPlanes {
 // own: put takes registers 0 - 7 (r0 = 0) and 8 - 15 (r0 = 8) - lanes l and l + 32 trade halves, so that each writes eight consecutive channels - and flush stores 64 bytes of a
 // column's channels per four lanes (straight from the registers they were 32.  96 x 96 with residual, 80043 columns: 28 us without planes, 42 and 36 with; the pre-pass 15).
 // Three planes: a value past the largest bfloat16 has that one as its first.
+// (one plane of eight values, two to a word; v: what is left)
+__device__ __forceinline__ void codec_split_pairs(float (&v)[8], uint32_t (&w)[4], bool clamp) {
+    constexpr float TOP = 3.38953138925153547590470800371487866880e+38f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float &a = v[2 * i], &b = v[2 * i + 1];
+        const float ca = clamp ? __builtin_amdgcn_fmed3f(a, -TOP, TOP) : a, cb = clamp ? __builtin_amdgcn_fmed3f(b, -TOP, TOP) : b;
+        w[i] = (uint32_t)f32_to_bf16(ca) | ((uint32_t)f32_to_bf16(cb) << 16);
+        a -= __uint_as_float(w[i] << 16);
+        b -= __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
 #define CP_LD 40
 #define CP_LDS(NP) ((NP) * 32 * CP_LD)       // in bf16
 template <int NP>
 __device__ __forceinline__ void codec_tile_put(float (&y)[8], uint16_t* st, int r0, int lane) {
-    constexpr float TOP = 3.38953138925153547590470800371487866880e+38f;
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
         uint32_t w[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float &a = y[2 * i], &b = y[2 * i + 1];
-            const float ca = NP == 3 && q == 0 ? __builtin_amdgcn_fmed3f(a, -TOP, TOP) : a, cb = NP == 3 && q == 0 ? __builtin_amdgcn_fmed3f(b, -TOP, TOP) : b;
-            w[i] = (uint32_t)f32_to_bf16(ca) | ((uint32_t)f32_to_bf16(cb) << 16);
-            a -= __uint_as_float(w[i] << 16);
-            b -= __uint_as_float(w[i] & 0xffff0000u);
-        }
+        codec_split_pairs(y, w, NP == 3 && q == 0);
         const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
         *reinterpret_cast<uint4*>(st + (q * 32 + (lane & 31)) * CP_LD + 2 * r0 + 8 * (lane >> 5)) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
     }

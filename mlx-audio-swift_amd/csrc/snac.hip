@@ -449,6 +449,57 @@ __global__ void k_enc_phase_split(const float* __restrict__ x, float* __restrict
         o[(size_t)r * Tm] = t >= 0 && t < T ? snake_f(v, al, ral) : 0.0f;
     }
 }
+// The same as three planes, [m][c*s + r] (codec_kernels.h, CodecPlanes): a block makes 64 columns of 64 phases, a thread eight phases of a column at a time; through LDS, so that
+// a column's 64 phases are stored as one 128-byte piece
+#define EP_LD 72
+__global__ void __launch_bounds__(256) k_enc_phase_planes(const float* __restrict__ x, const float* __restrict__ a, const float* __restrict__ ra, int C, int T, int s, int pad,
+                                                          const CodecPlanes o) {
+    __shared__ __attribute__((aligned(16))) uint16_t st[3][64 * EP_LD];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);           // (scalar: the phases' divisions and parameters)
+    const int m = blockIdx.x * 64 + lane, c0 = blockIdx.y * 64, b = blockIdx.z, rows = T / s + 1;
+    float v[2][8], al[2][8], ral[2][8];                                    // (all requested before the first use, the samples clamped and masked there)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        int c = (c0 + (wave + 4 * h) * 8) / s, r = (c0 + (wave + 4 * h) * 8) % s;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int cc = min(c, C - 1);
+            v[h][j] = x[((size_t)b * C + cc) * T + min(max(m * s + r - pad, 0), T - 1)];
+            al[h][j] = a[cc]; ral[h][j] = ra[cc];
+            if (++r == s) { r = 0; ++c; }
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(v[h][j]));
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = (wave + 4 * h) * 8;
+        int r = (c0 + k) % s;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int t = m * s + r - pad;
+            v[h][j] = snake_f(t >= 0 && t < T ? v[h][j] : 0.0f, al[h][j], ral[h][j]);      // (Snake of 0 is 0)
+            if (++r == s) r = 0;
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            uint32_t w[4];
+            codec_split_pairs(v[h], w, q == 0);
+            *reinterpret_cast<uint4*>(&st[q][lane * EP_LD + k]) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+    }
+    __syncthreads();
+    const int pieces = min(64, o.Cp - c0) / 8;
+    for (int i = threadIdx.x; i < 64 * pieces; i += 256) {
+        const int row = i / pieces, k = i % pieces * 8;
+        if (blockIdx.x * 64 + row >= rows) break;
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            *reinterpret_cast<uint4*>(o.p + q * o.stride + ((size_t)b * o.Tp + blockIdx.x * 64 + row) * o.Cp + c0 + k) = *reinterpret_cast<const uint4*>(&st[q][row * EP_LD + k]);
+    }
+}
 // average pool over `stride` consecutive samples (VQ.swift:47-57)
 __global__ void k_vq_pool(const float* __restrict__ x, float* __restrict__ y, int C, int T, int stride) {
     int m = blockIdx.x * blockDim.x + threadIdx.x, c = blockIdx.y, b = blockIdx.z;
@@ -1240,13 +1291,23 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
             std::swap(x, f2);
         }
         MIS_REQUIRE(T % eb.stride == 0, MIS_ERR_AUDIO_ENCODE, "internal: length not divisible by the stride");
-        launch_enc_phase_split(x, f1, W + eb.snake.a, W + eb.snake.ra, batch, eb.cin, (int)T, eb.stride, s);
+        const int Tx = (int)T;
         T /= eb.stride;
         GemmParams g{};
         g.AT = W + eb.down.w; g.bias = W + eb.down.b; g.X = f1; g.Y = f2;
         g.M = eb.cout; g.K = 2 * eb.stride * eb.cin; g.N = (int)T; g.Tin = (int)T + 1; g.Tout = (int)T;
         g.Cin = eb.stride * eb.cin; g.taps = 2; g.dil = 1; g.pad = 0;
-        launch_gemm(GEMM_TAPS, false, g, batch, s);
+        CodecPlanes pl;
+        if (codec_planes_strided(g, batch, pl)) {
+            hipLaunchKernelGGL(k_enc_phase_planes, dim3(cdiv(Tx / eb.stride + 1, 64), cdiv(pl.Cp, 64), batch), dim3(256), 0, s, x, W + eb.snake.a, W + eb.snake.ra, eb.cin, Tx, eb.stride,
+                               (eb.stride + 1) / 2, pl);
+            g.pack = &c->pack;
+            g.ldx = g.Tin; g.ldy = g.Tout;
+            MIS_REQUIRE(launch_gemm_bf3(GEMM_TAPS, false, g, batch, s, &pl), MIS_ERR_AUDIO_ENCODE, "internal: strided convolution refused its operand");
+        } else {
+            launch_enc_phase_split(x, f1, W + eb.snake.a, W + eb.snake.ra, batch, eb.cin, Tx, eb.stride, s);
+            launch_gemm(GEMM_TAPS, false, g, batch, s);
+        }
         std::swap(x, f2);
     }
     if (c->enc_attn.on) {                                                 // Layers.swift:339-341
