@@ -601,6 +601,10 @@ static bool bf3_takes(int mode, const GemmParams& p, const Bf3Shape& h) {
     if (mode == GEMM_CONVT) return h.Cin >= min_k && (int64_t)p.M * p.K >= min_mk;
     return h.Cin >= (mode == GEMM_TAPS ? min_k : min_k1);
 }
+bool bf3_takes_convt(const GemmParams& p) {
+    Bf3Shape h;
+    return (p.pack || tl_pack) && !codec_exact_f32() && bf3_shape(GEMM_CONVT, p, h) && bf3_takes(GEMM_CONVT, p, h);
+}
 // Tile: 128 x 128 (64 x 64 per wave); 64 x 128 while those are at most 128 blocks - half of the chip idle, each block one serial chain of chunks -
 // and 64 x 64 while 64 x 128 still are (or no more than 64 columns exist).  The same bits: the order of the products of an output does not change.
 // The small tiles run alone on a compute unit, with registers to spare: weights seven (not two) steps ahead, which covers a trip to HBM.

@@ -120,16 +120,20 @@ __device__ __forceinline__ void codec_split_pairs(float (&v)[8], uint32_t (&w)[4
         b -= __uint_as_float(w[i] & 0xffff0000u);
     }
 }
+// (registers 0 - 7 or 8 - 15 of a 32 x 32 C/D tile: lanes l and l + 32 trade halves, then each holds eight consecutive channels of its column - an MFMA-B fragment of 16 channels)
+__device__ __forceinline__ uint4 codec_tile_piece(float (&y)[8], bool clamp) {
+    uint32_t w[4];
+    codec_split_pairs(y, w, clamp);
+    const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+    return make_uint4(s0[0], s1[0], s0[1], s1[1]);
+}
 #define CP_LD 40
 #define CP_LDS(NP) ((NP) * 32 * CP_LD)       // in bf16
 template <int NP>
 __device__ __forceinline__ void codec_tile_put(float (&y)[8], uint16_t* st, int r0, int lane) {
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
-        uint32_t w[4];
-        codec_split_pairs(y, w, NP == 3 && q == 0);
-        const auto s0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false), s1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
-        *reinterpret_cast<uint4*>(st + (q * 32 + (lane & 31)) * CP_LD + 2 * r0 + 8 * (lane >> 5)) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+        *reinterpret_cast<uint4*>(st + (q * 32 + (lane & 31)) * CP_LD + 2 * r0 + 8 * (lane >> 5)) = codec_tile_piece(y, NP == 3 && q == 0);
     }
 }
 // d: channel 0 of the tile in row 0; row(c): the operand's row of the tile's column c, < 0: none
@@ -216,11 +220,13 @@ bool launch_gemm_x6(int mode, bool snake, const GemmParams& p, int batch, hipStr
 // (out: whether that form writes it)
 bool codec_x6_writes_planes(int mode, const GemmParams& p);
 // three-plane split: transposed convolution of stride 2, two taps per phase, 32 .. 64 rows, behind Snake; false: another shape
-bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s);
+// noise: with the NoiseBlock behind it (its X is p.Y, its Y unused)
+bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s, const GemmParams* noise = nullptr);
 // split-bf16 path; false = shape not eligible (or MIS_CODEC_EXACT_F32=1), nothing launched.  p must have ldx / ldy resolved
 // in: the operand is there already (codec_planes of the same call); out: the epilogue also writes (p.Y null: only) the operand of the contraction behind
 bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s, const CodecPlanes* in = nullptr, const CodecPlanes* out = nullptr);
 bool bf3_writes_planes(int mode, const GemmParams& p);
+bool bf3_takes_convt(const GemmParams& p);
 // the operand of this call as the epilogue in front of it can write it (scope's pack, buffer `slot`); false: the call wants f32
 bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot, CodecPlanes& out);
 // depthwise 7-tap conv (zero padded, dilation dil): shorter odd kernels ride in centred 7-tap weights

@@ -707,10 +707,14 @@ bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hip
 // the split run once per element (k_snac_convt: per phase and tap), the taps read the planes at column offsets, and a lane stores its two phases as one
 // float2.  Chunks of 16 channels; weights of the four (phase, tap) pairs through LDS.  128 -> 64 channels, 32 x 98304 columns: 3.34 -> 1.44 ms (3.2 GB
 // are 0.65 ms, the products 1.05); one row of 12288: 43 -> 27 us.
+struct X6Noise { const float* noise; int rng; uint64_t key; const int32_t* row_ids; int64_t row_offset; };      // as in GemmParams
+// NOISE: the NoiseBlock behind it, y = x + noise (W x), on the registers: a wave holds all rows of its columns, lanes l and l + 32 trade halves of x's planes, which
+// makes them fragments, and W takes the place of the last chunk's weights (fragments [Cin / 16][MT][plane], the size of a chunk's).  As a launch of its own, in f32, it read and
+// wrote the tensor: 16 us for one row of 24576 columns, 0.90 ms for 32 of 196608; here NOISE_US.
 #define X6_CT 126
-template <int MT>
-__device__ __forceinline__ void x6_convt_body(const GemmParams& p, const float* __restrict__ pX, float* __restrict__ pY, const float* __restrict__ pbias,
-                                              const float* __restrict__ pa, const float* __restrict__ pra, const uint16_t* __restrict__ pwp) {
+template <int MT, bool NOISE>
+__device__ __forceinline__ void x6_convt_body(const GemmParams& p, const X6Noise& nb, const float* __restrict__ pX, float* __restrict__ pY, const float* __restrict__ pbias,
+                                              const float* __restrict__ pa, const float* __restrict__ pra, const uint16_t* __restrict__ pwp, const uint16_t* __restrict__ pnw) {
     constexpr int APC = 4 * MT * 192, NA = APC / 256;
     __shared__ x6_u4 As[APC];
     __shared__ uint4 ts[3][2][128];
@@ -773,10 +777,26 @@ __device__ __forceinline__ void x6_convt_body(const GemmParams& p, const float* 
             }
     }
     const int nl = wave * 32 + (lane & 31), n = n0 + nl, o = 2 * n;
-    if (nl >= X6_CT || n >= p.N || o >= p.Tout) return;
+    const bool in = nl < X6_CT && n < p.N && o < p.Tout;
+    if (!NOISE && !in) return;
     const bool two = o + 1 < p.Tout, wide = two && !(p.ldy & 1) && !((uintptr_t)pY & 7), dup = n == 0 && p.dup_bias_n0;
     const float* bp = pbias ? pbias : pX;                                   // (loaded either way: a guard per value would be a round trip per value)
     const int btop = pbias ? p.M - 1 : 0;
+    float nz[2] = {0.0f, 0.0f};
+    if constexpr (NOISE) {
+        x6_u4 nw[NA];
+#pragma unroll
+        for (int i = 0; i < NA; ++i) nw[i] = reinterpret_cast<const x6_u4*>(pnw)[min(tid + i * 256, MT * MT * 2 * 192 - 1)];
+        if (in && nb.noise) { nz[0] = nb.noise[(size_t)b * p.Tout + o]; nz[1] = two ? nb.noise[(size_t)b * p.Tout + o + 1] : 0.0f; }
+        else if (in && nb.rng) {
+            const uint64_t row = (uint64_t)(nb.row_offset + (nb.row_ids ? nb.row_ids[b] : b));
+            nz[0] = codec_noise_value(nb.key, row, o); nz[1] = codec_noise_value(nb.key, row, o + 1);
+        }
+        __syncthreads();                                                    // the last chunk's products are done
+#pragma unroll
+        for (int i = 0; i < NA; ++i) As[tid + i * 256] = nw[i];
+        __syncthreads();
+    }
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi) {
         const int m0 = mi * 32 + 4 * (lane >> 5);
@@ -785,26 +805,79 @@ __device__ __forceinline__ void x6_convt_body(const GemmParams& p, const float* 
         for (int r = 0; r < 16; ++r) bm[r] = bp[min(m0 + (r & 3) + 8 * (r >> 2), btop)];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int m = m0 + (r & 3) + 8 * (r >> 2);
             const float bv = pbias ? bm[r] : 0.0f;
-            float y0 = acc[0][mi][r] + bv, y1 = acc[1][mi][r] + bv;
-            if (dup) { y0 += bv; y1 += bv; }                                // streaming overlap-add counts the bias twice (GemmParams)
+#pragma unroll
+            for (int ph = 0; ph < 2; ++ph) {
+                acc[ph][mi][r] += bv;
+                if (dup) acc[ph][mi][r] += bv;                              // streaming overlap-add counts the bias twice (GemmParams)
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (NOISE) {
+#pragma unroll
+        for (int ph = 0; ph < 2; ++ph) {
+            f32x16_t w[MT];
+#pragma unroll
+            for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) w[mi][r] = 0.0f;
+            constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int ks = 0; ks < 2 * MT; ++ks) {
+                float x[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) x[r] = acc[ph][ks / 2][ks % 2 * 8 + r];
+                bf16x8_t bv[3], av[MT][3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) bv[q] = __builtin_bit_cast(bf16x8_t, codec_tile_piece(x, q == 0));
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, As[((ks * MT + mi) * 3 + q) * 64 + lane]);
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int mi = 0; mi < MT; ++mi) w[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[QB[q]], w[mi], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);                          // (a step's fragments at a time: all of them do not fit the registers)
+            }
+#pragma unroll
+            for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[ph][mi][r] += nz[ph] * w[mi][r];
+        }
+        if (!in) return;
+    }
+    int hi = lane >> 5;                                                     // (opaque: the rows' addresses are not to be computed ahead)
+    asm volatile("" : "+v"(hi));
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = mi * 32 + 4 * hi + (r & 3) + 8 * (r >> 2);
             float* y = pY + ((size_t)b * p.M + m) * p.ldy + o;
             if (m >= p.M) continue;
-            if (wide) *reinterpret_cast<float2*>(y) = make_float2(y0, y1);
-            else { y[0] = y0; if (two) y[1] = y1; }
+            if (wide) *reinterpret_cast<float2*>(y) = make_float2(acc[0][mi][r], acc[1][mi][r]);
+            else { y[0] = acc[0][mi][r]; if (two) y[1] = acc[1][mi][r]; }
         }
-    }
 }
-template <int MT>
-__global__ void __launch_bounds__(256, 3) k_x6_convt(GemmParams p, const uint16_t* wp) { x6_convt_body<MT>(p, p.X, p.Y, p.bias, p.alpha, p.ralpha, wp); }
+template <int MT, bool NOISE>
+__global__ void __launch_bounds__(256, 3) k_x6_convt(GemmParams p, X6Noise nb, const uint16_t* wp, const uint16_t* nw) {
+    x6_convt_body<MT, NOISE>(p, nb, p.X, p.Y, p.bias, p.alpha, p.ralpha, wp, nw);
+}
 
-bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s) {
+bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s, const GemmParams* noise) {
     CodecPack* pack = p.pack ? p.pack : codec_x6_scope();
     if (!pack || codec_exact_f32() || p.s != 2 || p.K != 2 * p.Cin || p.M > 64 || p.M < 32 || p.Cin % 16 || !p.alpha) return false;
+    // (a NoiseBlock of as many rows as the tiles have and of this row's whole output)
+    if (noise && (noise->M != p.M || noise->K != p.M || p.M % 32 || noise->N != p.Tout || noise->bias)) return false;
     const uint16_t* wp = pack->get_x6(p.AT, 4, p.Cin, p.M, s).wp;           // [phase][tap][Cin][M]
+    const uint16_t* nw = noise ? pack->get_x6(noise->AT, 1, p.M, p.M, s).wp : nullptr;
+    const X6Noise nb = noise ? X6Noise{noise->noise, noise->noise_rng, noise->noise_key, noise->row_ids, noise->row_offset} : X6Noise{};
     const dim3 grid((p.N + X6_CT - 1) / X6_CT, batch);
-    if (p.M > 32) hipLaunchKernelGGL(k_x6_convt<2>, grid, dim3(256), 0, s, p, wp);
-    else hipLaunchKernelGGL(k_x6_convt<1>, grid, dim3(256), 0, s, p, wp);
+    if (p.M > 32 && noise) hipLaunchKernelGGL((k_x6_convt<2, true>), grid, dim3(256), 0, s, p, nb, wp, nw);
+    else if (p.M > 32) hipLaunchKernelGGL((k_x6_convt<2, false>), grid, dim3(256), 0, s, p, nb, wp, nw);
+    else if (noise) hipLaunchKernelGGL((k_x6_convt<1, true>), grid, dim3(256), 0, s, p, nb, wp, nw);
+    else hipLaunchKernelGGL((k_x6_convt<1, false>), grid, dim3(256), 0, s, p, nb, wp, nw);
     return true;
 }

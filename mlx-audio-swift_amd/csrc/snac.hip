@@ -1409,6 +1409,12 @@ void launch_vq_residual(float* r, const int32_t* codes, const float* table, int 
     hipLaunchKernelGGL(k_vq_residual, dim3(cdiv(T, 256), C, batch), dim3(256), 0, s, r, codes, table, C, T, stride);
 }
 
+// a transposed convolution that the two-plane path leaves to k_x6_convt, and the NoiseBlock behind it, as one
+static bool launch_convt_noise(GemmParams p, const GemmParams& noise, int batch, hipStream_t s) {
+    p.ldx = p.Tin; p.ldy = p.Tout;
+    return !bf3_takes_convt(p) && launch_convt_x6(p, batch, s, &noise);
+}
+
 bool launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s, const CodecPlanes* out, bool keep) {
     GemmParams p = p_in;
     if (!p.ldx) p.ldx = p.Tin;                                          // dense [B][C][T] tensors unless the caller says otherwise
@@ -1545,22 +1551,24 @@ static const float* snac_run(mis_snac* c, const int32_t* const* codes, int batch
             g.s = blk.stride; g.pad = blk.pad; g.Cin = blk.cin;
             g.N = (int)((To + blk.stride - 1) / blk.stride);     // columns per phase; stores are bounds-checked
             chain.push_back({GEMM_CONVT, true, true, g});
-            launch_gemm_chain(chain.data(), (int)chain.size(), batch, s);
-            chain.clear();
         }
+        const GemmParams ct = chain.back().g;
         std::swap(x, f1);
         T = To;
+        GemmParams g{};
         if (cf.noise) {   // NoiseBlock (Layers.swift:270-278)
-            GemmParams g{};
             g.AT = W + blk.noise.w; g.bias = nullptr; g.X = x; g.Y = f1;
             g.noise = noise ? noise[bi] : nullptr;
             g.noise_rng = (!noise && rng.enabled) ? 1 : 0;
             g.noise_key = mis_splitmix64(rng.seed + 0x51AC0000ull + (uint64_t)bi);
             g.row_ids = rng.row_ids; g.row_offset = rng.row_offset;
             g.M = blk.cout; g.K = blk.cout; g.N = (int)T; g.Tin = (int)T; g.Tout = (int)T;
-            launch_gemm(GEMM_NOISE, false, g, batch, s);
-            std::swap(x, f1);
         }
+        if (chain.size() > 1 || !cf.noise || !launch_convt_noise(ct, g, batch, s)) {
+            launch_gemm_chain(chain.data(), (int)chain.size(), batch, s);
+            if (cf.noise) { launch_gemm(GEMM_NOISE, false, g, batch, s); std::swap(x, f1); }
+        }
+        chain.clear();
         const int dils[3] = {1, 3, 9};
         for (int j = 0; j < 3; ++j) {   // ResidualUnit (Layers.swift:202-231)
             const auto& ru = blk.ru[j];
