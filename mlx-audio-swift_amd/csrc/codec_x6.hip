@@ -291,7 +291,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
     }
 }
 template <int C, bool DW, int KC, int NT, bool OUT>
-__global__ void __launch_bounds__(256, KC == 32 ? 2 : DW && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
+__global__ void __launch_bounds__(256, KC == 32 ? 2 : (DW || OUT) && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
     pw_x6_body<C, DW, KC, NT, OUT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy}, o, o.alpha, o.ralpha, o.p);
 }
 
