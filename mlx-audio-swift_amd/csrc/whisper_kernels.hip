@@ -886,38 +886,52 @@ void launch_scatter_kv(const bf16_t* src, int ld, int kcol0, int vcol0, bf16_t* 
 // ============================================================================ encoder self attention (non causal)
 //
 // One 32-key tile of 16 queries: raw scores (lane = query j, key group g4: keys g4*8 + e) -> P as bf16 hi + lo in the P.V operand layout.  The softmax is
-// bound by VALU issue (360 M scores per layer of 8 windows), so: scores stay raw, p = 2^(S c - m) with c = scale log2 e in one fma; the maximum that p is
-// taken against moves only when some score passes it by more than 2^8 (`lim`: one compare per lane, no cross-lane traffic on the usual tile) - the ratio
-// numerator / denominator does not depend on it, and sums of at most 256 T stay far inside float32; hi / lo are converted two at a time.
-// Returns true where the maximum moved (wave-uniform): the output so far must be scaled by alpha.
-struct AttnRow { float m = -INFINITY, lim = -INFINITY, l = 0.0f; };
+// bound by VALU issue (360 M scores per layer of 8 windows), so: p = 2^t, t = S c - m with c = scale log2 e in one fma; the maximum that p is
+// taken against moves only when some t passes 8 (no cross-lane traffic on the usual tile; taken over t and not over S, a maximum needs no quieting of the matrix core's output) - the
+// ratio numerator / denominator does not depend on it, and sums of at most 256 T stay far inside float32; hi / lo are converted two at a time.
+struct AttnRow { float m = -INFINITY, l = 0.0f; };
 template <bool MASKED>
-__device__ __forceinline__ bool attn_softmax_tile(const f32x4_t& S0, const f32x4_t& S1, int key0, int T, float c, AttnRow& r, bf16x8_t& ph, bf16x8_t& pl, float& alpha) {
+__device__ __forceinline__ void attn_mask(f32x4_t& S0, f32x4_t& S1, int key0, int T) {
+    if constexpr (MASKED) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float& s = e < 4 ? reinterpret_cast<float*>(&S0)[e] : reinterpret_cast<float*>(&S1)[e - 4];
+            s = key0 + e < T ? s : -INFINITY;
+        }
+    }
+}
+__device__ __forceinline__ float attn_shift(const f32x4_t& S0, const f32x4_t& S1, float c, const AttnRow& r, float (&t)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t[e] = fmaf(e < 4 ? S0[e] : S1[e - 4], c, -r.m);
+    return fmaxf(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])), fmaxf(fmaxf(t[4], t[5]), fmaxf(t[6], t[7])));
+}
+// the maximum moves (all of the wave's rows): the output so far and the sum are scaled
+template <int ND>
+__device__ __forceinline__ void attn_move(const f32x4_t& S0, const f32x4_t& S1, float c, AttnRow& r, float (&t)[8], f32x4_t (&O)[ND], int g4) {
+    float mx = fmaxf(fmaxf(fmaxf(S0[0], S0[1]), fmaxf(S0[2], S0[3])), fmaxf(fmaxf(S1[0], S1[1]), fmaxf(S1[2], S1[3])));
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(r.m, mx * c), alpha = __builtin_amdgcn_exp2f(r.m - m_new);       // (first tile: 2^-inf = 0)
+    r.m = m_new;
+    r.l *= alpha;
+    float ar[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ar[q] = __shfl(alpha, g4 * 4 + q, 64);
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) O[dt][q] *= ar[q];
+    (void)attn_shift(S0, S1, c, r, t);
+}
+__device__ __forceinline__ void attn_probs(const float (&t)[8], AttnRow& r, bf16x8_t& ph, bf16x8_t& pl) {
     typedef float f2_t __attribute__((ext_vector_type(2)));
     typedef __bf16 h2_t __attribute__((ext_vector_type(2)));
-    float s[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        s[e] = e < 4 ? S0[e] : S1[e - 4];
-        if constexpr (MASKED) s[e] = key0 + e < T ? s[e] : -INFINITY;
-    }
-    float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-    const bool moved = __any(mx > r.lim);
-    if (moved) {
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(r.m, mx * c);
-        alpha = __builtin_amdgcn_exp2f(r.m - m_new);                // (first tile: 2^-inf = 0)
-        r.m = m_new;
-        r.lim = (m_new + 8.0f) / c;
-        r.l *= alpha;
-    }
     float psum = 0.0f;
     uint32_t hw[4], lw[4];
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(s[e], c, -r.m)), p1 = __builtin_amdgcn_exp2f(fmaf(s[e + 1], c, -r.m));
-        psum += p0;
+        const float p0 = __builtin_amdgcn_exp2f(t[e]), p1 = __builtin_amdgcn_exp2f(t[e + 1]);
+        psum = e ? psum + p0 : p0;
         psum += p1;
         const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t){p0, p1}, h2_t));
         hw[e >> 1] = h;
@@ -926,7 +940,6 @@ __device__ __forceinline__ bool attn_softmax_tile(const f32x4_t& S0, const f32x4
     r.l += psum;
     ph = __builtin_bit_cast(bf16x8_t, make_uint4(hw[0], hw[1], hw[2], hw[3]));
     pl = __builtin_bit_cast(bf16x8_t, make_uint4(lw[0], lw[1], lw[2], lw[3]));
-    return moved;
 }
 // grid (ceil(T/64), H, B), 4 waves x 16 query rows.  S^T = K Q^T (A = K fragment, B = Q^T): lane (q row j, group g4)
 // holds the scores of keys base + g4*8 + e; online softmax per query row; O += P V with P split into bf16 hi + lo.
@@ -965,16 +978,10 @@ __global__ void __launch_bounds__(256) k_attn_prefill(const bf16_t* __restrict__
             S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, qf[c], S1, 0, 0, 0);
         }
         bf16x8_t ph, pl;
-        float alpha = 1.0f;
-        if (attn_softmax_tile<true>(S0, S1, kb + g4 * 8, T, sc2, row, ph, pl, alpha)) {
-            float ar[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, g4 * 4 + r, 64);
-#pragma unroll
-            for (int dt = 0; dt < D / 16; ++dt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) O[dt][r] *= ar[r];
-        }
+        float t[8];
+        attn_mask<true>(S0, S1, kb + g4 * 8, T);
+        if (__any(attn_shift(S0, S1, sc2, row, t) > 8.0f)) attn_move(S0, S1, sc2, row, t, O, g4);
+        attn_probs(t, row, ph, pl);
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) {
             bf16x8_t vb = vbase[((size_t)tile * (D / 16) + dt) * 64];
@@ -1008,7 +1015,7 @@ __global__ void __launch_bounds__(256) k_attn_prefill(const bf16_t* __restrict__
 // (tests/test_gpu_whisper.py).  Bound: the softmax's VALU work, not the matrix core: 228 us per layer of 8 windows x 20 heads (260 us with the score's scale,
 // its logarithm base and a cross-lane maximum per tile in the loop; two tiles per barrier: 251).
 template <int D>
-__global__ void __launch_bounds__(512, 1) k_attn_prefill2(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kc,
+__global__ void __launch_bounds__(512, 4) k_attn_prefill2(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kc,
                                                           const bf16_t* __restrict__ vc, bf16_t* __restrict__ out, int ldo,
                                                           int T, int H, int Spad, float scale) {
     static_assert(D == 64, "one 16-byte piece of the tile's 8 KB per thread");
@@ -1052,25 +1059,31 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill2(const bf16_t* __restri
         for (int c = 0; c < D / 32; ++c) { a0[c] = kf[c * 64]; a1[c] = kf[((D / 32) + c) * 64]; }
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) vb[dt] = vf[dt * 64];
+        f32x4_t S0[2], S1[2];
+        float t[2][8], mx[2];
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            f32x4_t S0 = (f32x4_t){0.f, 0.f, 0.f, 0.f}, S1 = S0;
+            S0[g] = S1[g] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int c = 0; c < D / 32; ++c) {
-                S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[c], qf[g][c], S0, 0, 0, 0);
-                S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[c], qf[g][c], S1, 0, 0, 0);
+                S0[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[c], qf[g][c], S0[g], 0, 0, 0);
+                S1[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[c], qf[g][c], S1[g], 0, 0, 0);
             }
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            attn_mask<MASKED>(S0[g], S1[g], kb + g4 * 8, T);
+            mx[g] = attn_shift(S0[g], S1[g], sc2, row[g], t[g]);
+        }
+        if (__any(fmaxf(mx[0], mx[1]) > 8.0f)) {
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+                if (__any(mx[g] > 8.0f)) attn_move(S0[g], S1[g], sc2, row[g], t[g], O[g], g4);
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
             bf16x8_t ph, pl;
-            float alpha = 1.0f;
-            if (attn_softmax_tile<MASKED>(S0, S1, kb + g4 * 8, T, sc2, row[g], ph, pl, alpha)) {
-                float ar[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, g4 * 4 + r, 64);
-#pragma unroll
-                for (int dt = 0; dt < D / 16; ++dt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) O[g][dt][r] *= ar[r];
-            }
+            attn_probs(t[g], row[g], ph, pl);
 #pragma unroll
             for (int dt = 0; dt < D / 16; ++dt) {
                 f32x4_t o = O[g][dt];
@@ -1080,14 +1093,14 @@ __global__ void __launch_bounds__(512, 1) k_attn_prefill2(const bf16_t* __restri
             }
         }
     };
-    for (int tile = 0; tile < n_tiles; ++tile) {
-        const bool more = tile + 1 < n_tiles;
-        if (more) st = src[(size_t)(tile + 1) * (IMG / 8)];
-        if (more || (T & 31) == 0) tile_math(tile, kv[tile & 1], std::false_type{});
-        else tile_math(tile, kv[tile & 1], std::true_type{});
-        if (more) *(reinterpret_cast<uint4*>(kv[(tile + 1) & 1]) + dst_piece) = st;
+    // (the last tile on its own: with its mask inside the loop the outputs are copied between the two forms' registers, 38 moves a tile)
+    for (int tile = 0; tile + 1 < n_tiles; ++tile) {
+        st = src[(size_t)(tile + 1) * (IMG / 8)];
+        tile_math(tile, kv[tile & 1], std::false_type{});
+        *(reinterpret_cast<uint4*>(kv[(tile + 1) & 1]) + dst_piece) = st;
         __syncthreads();
     }
+    tile_math(n_tiles - 1, kv[(n_tiles - 1) & 1], std::true_type{});
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
         float lr_all = row[g].l;
