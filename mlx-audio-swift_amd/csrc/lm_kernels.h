@@ -206,6 +206,18 @@ struct SamplerParams {
     int force_multi;         // 1: the multi-launch kernels whatever the range (shared device, recovery after a time-out, MIS_SAMPLER_WIDE)
     int spin;                // polls per row barrier of the one-launch sampler before it gives up
 };
+// Whisper's greedy step behind the logits: suppress masks, first index of the maximum, the loop's bookkeeping, and the token's embedding row with the first LayerNorm
+// (k_whisper_suppress, k_samp_cluster and k_whisper_embed_ln, which it has the results of)
+struct GreedyStep {
+    const int32_t *sup, *bsup;
+    int n_sup, n_bsup;
+    const bf16_t *emb, *pos_emb, *lw, *lb;
+    int *pos_cur, *pos_next;
+    bf16_t *h, *x;
+    int d, max_pos, batch;
+};
+bool greedy_step_ok(const SamplerParams& p, int d);
+void launch_greedy_step(const SamplerParams& p, const GreedyStep& g, int Mpad, hipStream_t s);
 // resolves the launcher's choices once (environment + the caller's multi_launch_only) into p
 void sampler_resolve(SamplerParams& p, bool multi_launch_only);
 // failure flags of the one-launch sampler (one per row): queued copy into pinned host memory, to be read after the caller's next

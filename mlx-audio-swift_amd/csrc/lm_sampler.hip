@@ -984,6 +984,191 @@ bool sampler_check_failed(SamplerScratch* scratch, int batch, hipStream_t s) {
     if (any) sampler_note_failure(scratch, batch, s);
     return any;
 }
+// ---- greedy step of the Whisper decoder ---------------------------------------------------------------------------------------------------
+// One block a row.  Everything that does not wait for the token is requested first: the row's logits (seven 16-byte loads a thread for 51 866 ids), the row's state, the suppressed ids,
+// the norm's weights.  The ids become a bit each in LDS; a logit becomes an ordered 16-bit integer, two to a word (four instructions a word; 64-bit keys of value and index, as the kernels
+// above have them, were 5 us of the 12.7 this took at first); the threads that hold the maximum look for its first index.  Latency bound: the three launches it replaces took
+// 3.9 + 9.0 + 4.0 us for one row (5.1 + 9.0 + 5.7 for eight), 8.4 and 9.4 here.  (Eight blocks a row, as for sampling, would meet at a barrier first.)
+#define GS_NT 1024
+#define GS_L 7
+typedef unsigned int gs_u32x4 __attribute__((ext_vector_type(4)));
+typedef short gs_s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void gs_load(const bf16_t* row, int n16, int c0, uint32_t (&q)[GS_L * 4]) {
+    gs_u32x4 v[GS_L];
+#pragma unroll
+    for (int j = 0; j < GS_L; ++j) v[j] = reinterpret_cast<const gs_u32x4*>(row)[min(c0 + (int)threadIdx.x + j * GS_NT, n16 - 1)];
+#pragma unroll
+    for (int j = 0; j < GS_L; ++j) { q[4 * j] = v[j].x; q[4 * j + 1] = v[j].y; q[4 * j + 2] = v[j].z; q[4 * j + 3] = v[j].w; }
+}
+// logits -> ordered integers, masked and out of range ones lowered
+__device__ __forceinline__ void gs_keys(uint32_t (&q)[GS_L * 4], const uint32_t* bits, int n16, int c0, int lo, int hi) {
+#pragma unroll
+    for (int j = 0; j < GS_L; ++j) {
+        const int i0 = min(c0 + (int)threadIdx.x + j * GS_NT, n16 - 1) * 8;
+        const unsigned masked = bits[i0 >> 5] >> (i0 & 31) & 0xffu;
+        const bool edge = i0 < lo || i0 + 8 > hi;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            uint32_t v = q[4 * j + w];
+            if (masked) {
+                const unsigned a = f32_to_bf16(bf16_to_f32((bf16_t)(v & 0xffffu)) + -1e9f), h = f32_to_bf16(bf16_to_f32((bf16_t)(v >> 16)) + -1e9f);
+                v = (masked >> (2 * w) & 1 ? a : v & 0xffffu) | (masked >> (2 * w + 1) & 1 ? h << 16 : v & 0xffff0000u);
+            }
+            const gs_s16x2 x = __builtin_bit_cast(gs_s16x2, v);
+            v = __builtin_bit_cast(uint32_t, (gs_s16x2)(x ^ ((x >> 15) & (short)0x7fff)));
+            if (edge) {
+                const int i = i0 + 2 * w;
+                v = (i < lo || i >= hi ? 0x8000u : v & 0xffffu) | (i + 1 < lo || i + 1 >= hi ? 0x80000000u : v & 0xffff0000u);
+            }
+            q[4 * j + w] = v;
+        }
+    }
+}
+__global__ void __launch_bounds__(GS_NT) k_greedy_step(SamplerParams p, GreedyStep g) {
+    __shared__ uint32_t bits[SC_NB * SC_NT * SC_PER / 32];
+    __shared__ int redk[GS_NT / 64];
+    __shared__ float red[4];
+    __shared__ int s_first, s_id, s_pos;
+    const int b = blockIdx.x, tid = threadIdx.x, Mt = gridDim.x >> 4, bc = min(b, g.batch - 1);
+    const bool row = b < g.batch;
+    const bf16_t* lp = p.logits + (size_t)bc * p.Vpad;
+    const int n16 = p.Vpad >> 3;
+    uint32_t q[GS_L * 4];
+    gs_load(lp, n16, 0, q);
+    const int step = p.n_gen[bc], was = p.active[bc], ps = g.pos_next[bc], last_id = p.next_ids[bc];
+    int sup = g.sup[min(tid, max(g.n_sup - 1, 0))], bsup = g.bsup[min(tid, max(g.n_bsup - 1, 0))];
+    constexpr int NE = 8;
+    bf16_t lw[NE], lb[NE];
+#pragma unroll
+    for (int k = 0; k < NE; ++k) {
+        const int i = min((tid & 255) + k * 256, g.d - 1);
+        lw[k] = g.lw[i]; lb[k] = g.lb[i];
+    }
+    const bool live = row && was && step < p.max_tokens;
+    if (live) {
+        int lo, hi;
+        allowed_range(p, step, lo, hi);
+        for (int i = tid; i < (p.Vpad + 31) >> 5; i += GS_NT) bits[i] = 0;
+        if (tid == 0) s_first = 0x7fffffff;
+        __syncthreads();
+        for (int i = tid; i < g.n_sup; i += GS_NT) {
+            const int id = i == tid ? sup : g.sup[i];
+            if (id >= 0 && id < p.vocab) atomicOr(&bits[id >> 5], 1u << (id & 31));
+        }
+        if (step == 0)
+            for (int i = tid; i < g.n_bsup; i += GS_NT) {
+                const int id = i == tid ? bsup : g.bsup[i];
+                if (id >= 0 && id < p.vocab) atomicOr(&bits[id >> 5], 1u << (id & 31));
+            }
+        __syncthreads();
+        int best = -32768;
+        for (int c0 = 0; c0 < n16; c0 += GS_L * GS_NT) {
+            if (c0) gs_load(lp, n16, c0, q);
+            gs_keys(q, bits, n16, c0, lo, hi);
+            gs_s16x2 m = {-32768, -32768};
+#pragma unroll
+            for (int j = 0; j < GS_L * 4; ++j) m = __builtin_elementwise_max(m, __builtin_bit_cast(gs_s16x2, q[j]));
+            best = max(best, max((int)m.x, (int)m.y));
+        }
+        int all = best;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) all = max(all, __shfl_xor(all, o, 64));
+        if ((tid & 63) == 0) redk[tid >> 6] = all;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < GS_NT / 64; ++w) all = max(all, redk[w]);
+        if (best == all && all > -32768) {
+            int first = 0x7fffffff;
+            for (int c0 = 0; c0 < n16; c0 += GS_L * GS_NT) {
+                if (n16 > GS_L * GS_NT) { gs_load(lp, n16, c0, q); gs_keys(q, bits, n16, c0, lo, hi); }
+#pragma unroll
+                for (int j = 0; j < GS_L; ++j) {
+                    const int i0 = min(c0 + tid + j * GS_NT, n16 - 1) * 8;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        const int a = (int)(short)(q[4 * j + w] & 0xffffu), h = (int)q[4 * j + w] >> 16;
+                        first = a == all ? min(first, i0 + 2 * w) : first;
+                        first = h == all ? min(first, i0 + 2 * w + 1) : first;
+                    }
+                }
+            }
+            atomicMin(&s_first, first);
+        }
+        __syncthreads();
+        if (tid == 0) {      // bookkeeping of the generate loop, as k_samp_cluster (no window, no list of all ids here)
+            const int token = s_first < 0x7fffffff ? s_first : lo < p.vocab ? lo : 0;
+            if (p.tokens_out && step < p.tokens_stride) p.tokens_out[(size_t)b * p.tokens_stride + step] = token;
+            p.n_gen[b] = step + 1;
+            p.next_ids[b] = token;
+            const bool end = token == p.eos_id;
+            if (end) p.active[b] = 0;
+            if (end || step + 1 >= p.max_tokens) atomicAdd(p.done_count, 1);
+            g.pos_cur[b] = ps;
+            if (!end) g.pos_next[b] = ps + 1;
+            s_id = token;
+            s_pos = ps;
+        }
+    } else if (tid == 0) {   // a row that is done, or padding
+        if (row) {
+            g.pos_cur[b] = ps;
+            if (was) g.pos_next[b] = ps + 1;
+        }
+        s_id = row ? last_id : 0;
+        s_pos = row ? ps : 0;
+    }
+    __syncthreads();
+    // k_whisper_embed_ln on the first four waves: the same sums in the same order
+    const int id = s_id < 0 || s_id >= p.vocab ? 0 : s_id, pos = min(s_pos, g.max_pos - 1);
+    float f[NE], s = 0.0f;
+    const bool on = tid < 256;
+    if (on) {
+        bf16_t ev[NE], pv[NE];
+#pragma unroll
+        for (int k = 0; k < NE; ++k) {
+            const int i = min(tid + k * 256, g.d - 1);
+            ev[k] = g.emb[(size_t)id * g.d + i];
+            pv[k] = g.pos_emb[(size_t)pos * g.d + i];
+        }
+#pragma unroll
+        for (int k = 0; k < NE; ++k) {
+            f[k] = bf16_round_f32(bf16_to_f32(ev[k]) + bf16_to_f32(pv[k]));
+            if (tid + k * 256 < g.d) { g.h[(size_t)b * g.d + tid + k * 256] = f32_to_bf16(f[k]); s += f[k]; }
+        }
+        s = wave_sum(s);
+        if ((tid & 63) == 0) red[tid >> 6] = s;
+    }
+    __syncthreads();
+    const float mean = (red[0] + red[1] + red[2] + red[3]) / (float)g.d;
+    __syncthreads();
+    if (on) {
+        float q = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NE; ++k)
+            if (tid + k * 256 < g.d) { const float t = f[k] - mean; q += t * t; }
+        q = wave_sum(q);
+        if ((tid & 63) == 0) red[tid >> 6] = q;
+    }
+    __syncthreads();
+    if (!on) return;
+    const float rstd = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)g.d + 1e-5f);
+#pragma unroll
+    for (int k = 0; k < NE; ++k) {
+        const int i = tid + k * 256;
+        if (i >= g.d) break;
+        const size_t off = ((((size_t)(i >> 5) * Mt + (b >> 4)) * 64) + (((i & 31) >> 3) << 4) + (b & 15)) * 8 + (i & 7);
+        g.x[off] = f32_to_bf16((f[k] - mean) * rstd * bf16_to_f32(lw[k]) + bf16_to_f32(lb[k]));
+    }
+}
+// (a spin limit of 0, which makes every row barrier time out, asks for the kernel that has barriers)
+bool greedy_step_ok(const SamplerParams& p, int d) {
+    return p.path_resolved && !p.force_multi && p.spin > 0 && p.temperature == 0.0f && p.penalty == 0.0f && !p.frame_constrained && !p.logits32 && !p.step_override && !p.all_ids &&
+           !p.window && p.active && p.active == p.active_in && p.next_ids && p.n_gen && p.done_count && p.Vpad % 16 == 0 && p.vocab <= SC_NB * SC_NT * SC_PER && d <= 2048;
+}
+void launch_greedy_step(const SamplerParams& p, const GreedyStep& g, int Mpad, hipStream_t s) {
+    MIS_REQUIRE(greedy_step_ok(p, g.d) && Mpad % 16 == 0 && g.batch <= Mpad, MIS_ERR_GENERATION_FAILED, "greedy step: unsupported parameters");
+    hipLaunchKernelGGL(k_greedy_step, dim3(Mpad), dim3(GS_NT), 0, s, p, g);
+}
+
 // the one-launch sampler's 8 x batch blocks spin on each other: all of them have to be resident at once.  The capacity (occupancy query
 // x compute units) is cached per DEVICE: the replicas of a group may sit on devices of different sizes or partition modes.
 static bool sampler_cluster_fits(int batch) {

@@ -41,7 +41,7 @@ struct mis_whisper {
     int batch = 0, Mpad = 0, Smax = 0, Spad = 1536;
     int S_qkv = 1, S_o = 1, S_cq = 1, S_fc2 = 1;
     DevBuf<bf16_t> cross_k, cross_v, self_k, self_v, enc_out;
-    DevBuf<int32_t> ids, pos_cur, pos_next, n_gen, tokens_out, next_ids, done_count, sup, bsup;
+    DevBuf<int32_t> ids, pos_cur, pos_next, n_gen, tokens_out, next_ids, done_count, sup, bsup, prompt_rows;
     DevBuf<uint8_t> active;
     DevBuf<float> xa_part;                               // partial sums of the cross-attention over several blocks a head; its counters
     DevBuf<unsigned> xa_count;
@@ -529,7 +529,8 @@ extern "C" mis_status mis_whisper_encode(mis_whisper* c, const float* features, 
 // arrangement (profiles/r06/c9: every producer GEMM as eight-wave items over the whole K range writing one float32 slab, so that LayerNorm 1
 // could move into q|k|v's prologue as well - 7 launches per layer, parity green, transcribe 214 -> 224 ms: fc2 at 80 blocks 5.2 -> 8.5 us).
 #define WHISPER_FOLD_DEFAULT 20
-static void enqueue_decoder_step(mis_whisper* c) {
+// ids: the tokens that the step reads, one a row; null: their embeddings and first LayerNorm are there already (launch_greedy_step)
+static void enqueue_decoder_step(mis_whisper* c, const int32_t* ids) {
     hipStream_t s = c->stream;
     const int d = c->d, fd = c->cfg.decoder_ffn_dim, Mpad = c->Mpad, H = c->Hd, D = c->D;
     const DecLayer& L0 = c->dec[0];
@@ -543,7 +544,8 @@ static void enqueue_decoder_step(mis_whisper* c) {
                 "MIS_WHISPER_FOLD: the folded decoder step does not apply to this shape");
     bf16_t* hcur = c->h.p;
     bf16_t* hoth = c->h2.p;
-    launch_whisper_embed_ln(c->emb, c->dec_pos, c->ids.p, c->active.p, c->pos_cur.p, c->pos_next.p, L0.ln1w, L0.ln1b, hcur,
+    if (ids)
+        launch_whisper_embed_ln(c->emb, c->dec_pos, ids, c->active.p, c->pos_cur.p, c->pos_next.p, L0.ln1w, L0.ln1b, hcur,
                             c->x.p, d, c->V, c->cfg.max_target_positions, c->batch, Mpad, s);
     for (size_t li = 0; li < c->dec.size(); ++li) {
         const DecLayer& L = c->dec[li];
@@ -624,7 +626,7 @@ extern "C" mis_status mis_whisper_decoder_forward(mis_whisper* c, const int32_t*
         MIS_REQUIRE(!act[b] || pn[b] < c->cfg.max_target_positions, MIS_ERR_INVALID_INPUT, "row %d exceeds max_target_positions", b);
     HIP_CHECK(hipMemcpyAsync(c->ids.p, tokens, c->batch * 4, hipMemcpyDefault, s));
     HIP_CHECK(hipMemcpyAsync(c->active.p, act.data(), c->batch, hipMemcpyHostToDevice, s));
-    enqueue_decoder_step(c);
+    enqueue_decoder_step(c, c->ids.p);
     if (logits_out) {
         enqueue_vocab(c);
         size_t n = (size_t)c->batch * c->V;
@@ -680,6 +682,9 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     int max_tokens = std::max(1, std::min(sp->max_tokens > 0 ? sp->max_tokens : c->cfg.max_target_positions,
                                           c->cfg.max_target_positions - n_prompt - 1));
     std::vector<uint8_t> ones(batch, 1);
+    std::vector<int32_t> prompt_rows((size_t)n_prompt * batch);
+    for (size_t i = 0; i < prompt_rows.size(); ++i) prompt_rows[i] = prompt[i / batch];
+    c->prompt_rows.alloc(prompt_rows.size());
     for (int j = 0; j < n_prompt; ++j) MIS_REQUIRE(prompt[j] >= 0 && prompt[j] < c->V, MIS_ERR_INVALID_INPUT, "prompt token outside the vocabulary");
     std::vector<int32_t> emitted(batch, 0);              // ids already announced to the callback (kept across a second attempt)
     // One attempt of prompt prefill + decode loop on the encoder output already in place.  Returns false when a row barrier of the
@@ -687,13 +692,10 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     // id of that poll interval is announced; the caller resets the decoder state and runs the attempt again on the multi-launch
     // sampler (deterministic: same ids, the callback continues behind `emitted`).
     auto attempt = [&](bool multi_launch_only) -> bool {
-        for (int j = 0; j < n_prompt; ++j) {
-            std::vector<int32_t> row(batch, prompt[j]);
-            HIP_CHECK(hipMemcpyAsync(c->ids.p, row.data(), batch * 4, hipMemcpyHostToDevice, s));
-            HIP_CHECK(hipMemcpyAsync(c->active.p, ones.data(), batch, hipMemcpyHostToDevice, s));
-            enqueue_decoder_step(c);
-            HIP_CHECK(hipStreamSynchronize(s));
-        }
+        // (one upload and no wait between the steps: a step's launches are queued while the one in front runs)
+        HIP_CHECK(hipMemcpyAsync(c->prompt_rows.p, prompt_rows.data(), prompt_rows.size() * 4, hipMemcpyHostToDevice, s));
+        HIP_CHECK(hipMemcpyAsync(c->active.p, ones.data(), batch, hipMemcpyHostToDevice, s));
+        for (int j = 0; j < n_prompt; ++j) enqueue_decoder_step(c, c->prompt_rows.p + (size_t)j * batch);
         // ---- decode loop
         c->tokens_out.alloc((size_t)batch * max_tokens);
         c->tokens_out.zero(s);
@@ -719,10 +721,16 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
         // is a device pointer that stays put, so the step is captured once and replayed (≈430 kernel nodes per step)
         auto step_body = [&]() {
             enqueue_vocab(c);
+            if (greedy_step_ok(q, c->d)) {
+                launch_greedy_step(q, GreedyStep{c->sup.p, c->bsup.p, sp->n_suppress, sp->n_begin_suppress, c->emb, c->dec_pos, c->dec[0].ln1w, c->dec[0].ln1b, c->pos_cur.p, c->pos_next.p,
+                                                 c->h.p, c->x.p, c->d, c->cfg.max_target_positions, batch}, c->Mpad, s);
+                enqueue_decoder_step(c, nullptr);
+                return;
+            }
             launch_whisper_suppress(c->logits.p, c->Vpad, c->V, c->sup.p, sp->n_suppress, c->bsup.p, sp->n_begin_suppress, c->n_gen.p,
                                     c->active.p, batch, s);
             launch_sampler(q, batch, s);
-            enqueue_decoder_step(c);
+            enqueue_decoder_step(c, c->ids.p);
     };
     hipGraphExec_t gexec = nullptr;
     const bool use_graph = getenv("MIS_NO_GRAPH") == nullptr;
