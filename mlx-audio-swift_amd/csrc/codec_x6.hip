@@ -84,7 +84,10 @@ const CodecPack::X6& CodecPack::get_x6(const float* at, int ntaps, int Cin, int 
 // channels of a column per thread are split and written as one 16-byte piece per plane, [plane][channel / 8][column], which is the MFMA-B fragment.
 // What bounds it: k_pw_fused<128, DW> took 1.05 ms without its MFMAs (4.8 GB of loads and stores, 32 rows of 98304 columns) and 1.75 ms with: the f32
 // matrix time adds to the memory time.  Six bf16 products take 0.25 instead of 0.68 ms of it: 1.95 -> 1.44 ms.
+typedef uint32_t x6_u4 __attribute__((ext_vector_type(4)));
 struct PwScalars { int T, dil, ldx, ldr, ldy; };
+// LDS alone: __syncthreads() would wait for the next chunk's samples and weights as well
+__device__ __forceinline__ void pw_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 template <int C, bool DW, int KC, int NT, bool OUT>
 __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                            const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
@@ -97,9 +100,13 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
     __shared__ float xs[DW ? KC : 1][DW ? XS : 1];
     __shared__ uint4 sm[3 * KG * NT + APC];
     uint4 (&ts)[3][KG][NT] = *reinterpret_cast<uint4 (*)[3][KG][NT]>(sm);
-    uint4 (&As)[APC] = *reinterpret_cast<uint4 (*)[APC]>(sm + 3 * KG * NT);
+    x6_u4 (&As)[APC] = *reinterpret_cast<x6_u4 (*)[APC]>(sm + 3 * KG * NT);
     // The encoder's units take the place of k_x6_gemm in long rows only: a lane that sees a sum which is not finite takes its rows again as that kernel does
     constexpr bool RETAKE = DW && C <= 96;
+    // The next chunk's samples and weights are requested behind this one's staging (behind barriers that wait for LDS alone), where the registers allow: 128 channels with taps in
+    // blocks of 128 columns keep three blocks a compute unit instead (32 x 98304 columns: 1.40 ms; two blocks and the requests 1.65).  us, without / with: 128 channels with taps,
+    // 192 blocks 22.0 / 20.0; 96, 592 blocks 41.8 / 38.6; 48, 1184 blocks (three a compute unit instead of four) 33.0 / 31.3PW_PLAIN.
+    constexpr bool PF = !(DW && C == 128 && NT == 128);
     constexpr bool SQ = C == 128 || NT == 64;             // 2 x 2 waves of half the rows and half the columns; else every wave: all C rows x 32 columns
     constexpr int MTW = SQ ? MT / 2 : MT, NTW = SQ ? NT / 64 : 1;
     static_assert(SQ ? MT % 2 == 0 : NT == 128, "2 x 2 waves, or four of 32 columns");
@@ -116,44 +123,51 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
         for (int j = 0; j < NTW; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-    for (int c0 = 0; c0 < C; c0 += KC) {
-        __syncthreads();                                   // the previous chunk's MFMAs are done with ts / As
-        uint4 wv[(APC + 255) / 256];
-        const uint4* wsrc = reinterpret_cast<const uint4*>(pwp) + (size_t)(c0 / 16) * MT * 192;
+    x6_u4 wv[(APC + 255) / 256];
+    float vx[DW ? XR : GS][DW ? NS : 8];
+    auto fetch = [&](int c0) {
+        const x6_u4* wsrc = reinterpret_cast<const x6_u4*>(pwp) + (size_t)(c0 / 16) * MT * 192;
 #pragma unroll
         for (int i = 0; i < (APC + 255) / 256; ++i) wv[i] = wsrc[min(tid + i * 256, APC - 1)];
-        if (DW) {
-            float v[XR][NS];
+        if constexpr (DW) {
 #pragma unroll
-            for (int r = 0; r < XR; ++r) {
-                const int c = c0 + wave + 4 * r;
+            for (int r = 0; r < XR; ++r)
 #pragma unroll
-                for (int sx = 0; sx < NS; ++sx) {
-                    const int j = sx * 64 + lane, t = n0 - halo + j;
-                    const bool ok = j < ncols && t >= 0 && t < T;
-                    v[r][sx] = xb[(size_t)c * p.ldx + (ok ? t : 0)];
-                    v[r][sx] = ok ? v[r][sx] : 0.0f;
-                }
+                for (int sx = 0; sx < NS; ++sx) vx[r][sx] = xb[(size_t)(c0 + wave + 4 * r) * p.ldx + min(max(n0 - halo + sx * 64 + lane, 0), T - 1)];
+        } else {
+#pragma unroll
+            for (int g = 0; g < GS; ++g) {
+                const int kg = KC == 32 ? wave : wave >> 1, n = (KC == 32 ? g : wave & 1) * 64 + lane;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) vx[g][j] = xb[(size_t)(c0 + kg * 8 + j) * p.ldx + min(n0 + n, T - 1)];
             }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (PF) fetch(0);
+    for (int c0 = 0; c0 < C; c0 += KC) {
+        if constexpr (PF) pw_lds_barrier(); else __syncthreads();          // the previous chunk's MFMAs are done with ts / As
+        if (!PF) fetch(c0);
+        if (DW) {
 #pragma unroll
             for (int r = 0; r < XR; ++r) {
                 const int cc = wave + 4 * r, c = c0 + cc;
                 const float al = pa1[c], ral = pra1[c];
 #pragma unroll
                 for (int sx = 0; sx < NS; ++sx) {
-                    const int j = sx * 64 + lane;
-                    if (j < XS) xs[cc][j] = x6_snake(v[r][sx], al, ral);
+                    const int j = sx * 64 + lane, t = n0 - halo + j;
+                    const float u = j < ncols && t >= 0 && t < T ? vx[r][sx] : 0.0f;
+                    if (j < XS) xs[cc][j] = x6_snake(u, al, ral);
                 }
+                __builtin_amdgcn_sched_barrier(0);                          // (a row at a time: the values in flight take the registers)
             }
         } else {
 #pragma unroll
             for (int g = 0; g < GS; ++g) {
-                const int kg = KC == 32 ? wave : wave >> 1, n = (KC == 32 ? g : wave & 1) * 64 + lane, t = n0 + n;
+                const int kg = KC == 32 ? wave : wave >> 1, n = (KC == 32 ? g : wave & 1) * 64 + lane;
                 float v[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = xb[(size_t)(c0 + kg * 8 + j) * p.ldx + (t < T ? t : 0)];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = x6_snake(v[j], pa2[c0 + kg * 8 + j], pra2[c0 + kg * 8 + j]);
+                for (int j = 0; j < 8; ++j) v[j] = x6_snake(vx[g][j], pa2[c0 + kg * 8 + j], pra2[c0 + kg * 8 + j]);
                 uint4 h, m, l;
                 x6_split<false>(v, h, m, l);
                 ts[0][kg][n] = h; ts[1][kg][n] = m; ts[2][kg][n] = l;
@@ -162,8 +176,12 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
         for (int i = 0; i < (APC + 255) / 256; ++i)
             if (APC % 256 == 0 || tid + i * 256 < APC) As[tid + i * 256] = wv[i];
+        if constexpr (PF) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (c0 + KC < C) fetch(c0 + KC);                                // (in flight behind this chunk's taps and products)
+        }
         if (DW) {
-            __syncthreads();
+            if constexpr (PF) pw_lds_barrier(); else __syncthreads();
             // depthwise taps + bias + Snake -> eight channels of one column per thread (consecutive lanes read consecutive LDS words)
 #pragma unroll
             for (int g = 0; g < GS; ++g) {
@@ -176,13 +194,14 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
                     for (int k = 0; k < 7; ++k) a += pw7[c * 7 + k] * xs[cc][n + k * p.dil];
                     v[j] = x6_snake(a + pb1[c], pa2[c], pra2[c]);
+                    if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
                 }
                 uint4 h, m, l;
                 x6_split<false>(v, h, m, l);
                 ts[0][kg][n] = h; ts[1][kg][n] = m; ts[2][kg][n] = l;
             }
         }
-        __syncthreads();
+        if constexpr (PF) pw_lds_barrier(); else __syncthreads();
 #pragma unroll
         for (int ks = 0; ks < KC / 16; ++ks) {
             bf16x8_t bv[NTW][3];
@@ -291,7 +310,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
     }
 }
 template <int C, bool DW, int KC, int NT, bool OUT>
-__global__ void __launch_bounds__(256, KC == 32 ? 2 : (DW || OUT) && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
+__global__ void __launch_bounds__(256, KC == 32 ? 2 : DW || (OUT && C >= 96) ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
     pw_x6_body<C, DW, KC, NT, OUT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy}, o, o.alpha, o.ralpha, o.p);
 }
 
@@ -342,7 +361,6 @@ bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int b
 // with all its rows, so the activations need neither LDS nor a barrier.  WIDE: the four waves of a block share the weights, staged in LDS two chunks deep;
 // else (few blocks) one row tile per block, weights straight into registers.  k order: 16 channels, within them the taps, six products each.
 // Bound (256 x 256 with residual, 32 x 24576 columns): 2.4 GB = 0.49 ms of the 0.85; the products' 0.53 ms run half behind it.
-typedef uint32_t x6_u4 __attribute__((ext_vector_type(4)));
 struct X6Gemm {
     GemmParams g;
     int mode, ntaps, nsteps, MT32;        // steps of 16 channels of one tap
