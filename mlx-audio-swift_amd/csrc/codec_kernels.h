@@ -173,6 +173,7 @@ struct PwFusedParams {
     const float *a2, *ra2;                 // Snake in front of the 1x1 conv
     const float *AT, *b2;                  // W2^T [C][C] ([k][m]), bias
     int T, dil, ldx, ldr, ldy;
+    int nbx, per, tiles;                   // blocks of columns a row, blocks an XCD, blocks (the launcher's)
     const CodecPlanes* out;                // units without taps: the operand of the contraction behind, or null
 };
 // three-plane split of the unit tails (codec_x6.hip); false: no pack, exact-f32 asked for, or another width - nothing launched

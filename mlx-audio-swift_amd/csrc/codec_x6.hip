@@ -10,7 +10,7 @@
 // convolution gives NaN where the f32 kernels give an infinity or NaN.)
 //
 //   k_x6_pack_w   A^T f32 -> the three planes as MFMA-A fragments (once per weight matrix, kept in the model's CodecPack)
-//   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels and for MIS_CODEC_EXACT_F32=1) and its encoder's units of 48 and 96
+//   k_pw_x6       the fused unit tails of snac.hip (k_pw_fused, which stays for 64 channels without taps and for MIS_CODEC_EXACT_F32=1) and its encoder's units of 48 and 96
 //   k_x6_gemm     1x1 and k-tap contractions (codec_f32.hip keeps the rest)
 //   k_x6_convt    transposed convolutions of stride 2 and at most 64 rows
 #include "common.h"
@@ -85,37 +85,38 @@ const CodecPack::X6& CodecPack::get_x6(const float* at, int ntaps, int Cin, int 
 // What bounds it: k_pw_fused<128, DW> took 1.05 ms without its MFMAs (4.8 GB of loads and stores, 32 rows of 98304 columns) and 1.75 ms with: the f32
 // matrix time adds to the memory time.  Six bf16 products take 0.25 instead of 0.68 ms of it: 1.95 -> 1.44 ms.
 typedef uint32_t x6_u4 __attribute__((ext_vector_type(4)));
-struct PwScalars { int T, dil, ldx, ldr, ldy; };
+struct PwScalars { int T, ldx, ldr, ldy, nbx, per, tiles; };
 // LDS alone: __syncthreads() would wait for the next chunk's samples and weights as well
 __device__ __forceinline__ void pw_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-template <int C, bool DW, int KC, int NT, bool OUT>
+template <int C, int DIL, int KC, int NT, bool PF, bool OUT>
 __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const float* __restrict__ pR, float* __restrict__ pY,
                                            const float* __restrict__ pw7, const float* __restrict__ pb1, const float* __restrict__ pa1,
                                            const float* __restrict__ pra1, const float* __restrict__ pa2, const float* __restrict__ pra2,
                                            const uint16_t* __restrict__ pwp, const float* __restrict__ pAT, const float* __restrict__ pb2, const PwScalars p, const CodecPlanes po,
                                            const float* __restrict__ poa, const float* __restrict__ pora, uint16_t* __restrict__ pout) {
     constexpr int KG = KC / 8, MT = (C + 31) / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
-    constexpr int XR = KC / 4, GS = KG * (NT / 64) / 4, XS = NT + 2 * CODEC_DW_HALO + 2, NS = (XS + 61) / 64;      // (XS - 2 columns in strips of 64)
-                               // rows of x and (group, strip) pairs per wave
+    constexpr bool DW = DIL > 0;
+    constexpr int XR = KC / 4, NS = NT / 64, GS = KG * NS / 4;                      // rows of x, strips of columns, (group, strip) pairs per wave
+    // (the dilation is a constant: as many columns are staged as it needs - the halo of a wave's rows one behind the other, 64 values at a time)
+    constexpr int HALO = 3 * DIL, XS = NT + 2 * HALO + 2, HP = (XR * 2 * HALO + 63) / 64;
     __shared__ float xs[DW ? KC : 1][DW ? XS : 1];
     __shared__ uint4 sm[3 * KG * NT + APC];
     uint4 (&ts)[3][KG][NT] = *reinterpret_cast<uint4 (*)[3][KG][NT]>(sm);
     x6_u4 (&As)[APC] = *reinterpret_cast<x6_u4 (*)[APC]>(sm + 3 * KG * NT);
     // The encoder's units take the place of k_x6_gemm in long rows only: a lane that sees a sum which is not finite takes its rows again as that kernel does
     constexpr bool RETAKE = DW && C <= 96;
-    // The next chunk's samples and weights are requested behind this one's staging (behind barriers that wait for LDS alone), where the registers allow: 128 channels with taps in
-    // blocks of 128 columns keep three blocks a compute unit instead (32 x 98304 columns: 1.40 ms; two blocks and the requests 1.65).  us, without / with: 128 channels with taps,
-    // 192 blocks 22.0 / 20.0; 96, 592 blocks 41.8 / 38.6; 48, 1184 blocks (three a compute unit instead of four) 33.0 / 31.3PW_PLAIN.
-    constexpr bool PF = !(DW && C == 128 && NT == 128);
     constexpr bool SQ = C == 128 || NT == 64;             // 2 x 2 waves of half the rows and half the columns; else every wave: all C rows x 32 columns
     constexpr int MTW = SQ ? MT / 2 : MT, NTW = SQ ? NT / 64 : 1;
     static_assert(SQ ? MT % 2 == 0 : NT == 128, "2 x 2 waves, or four of 32 columns");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n0 = blockIdx.x * NT, b = blockIdx.y;
+    // (an XCD takes a contiguous range of blocks: a neighbour's halo and the other half of a line are in its L2)
+    const int tileid = (blockIdx.x & 7) * p.per + (blockIdx.x >> 3);
+    if (tileid >= p.tiles) return;
+    const int b = tileid / p.nbx, n0 = (tileid - b * p.nbx) * NT;
     const int wr = SQ ? (wave >> 1) * MTW : 0;              // first row tile / first column of the wave's tile
     const int wc = SQ ? (wave & 1) * (NT / 2) : wave * 32;
     const float* xb = pX + (size_t)b * C * p.ldx;
-    const int T = p.T, halo = 3 * p.dil, ncols = NT + 2 * halo;
+    const int T = p.T;
     f32x16_t acc[MTW][NTW];
 #pragma unroll
     for (int i = 0; i < MTW; ++i)
@@ -124,7 +125,14 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     x6_u4 wv[(APC + 255) / 256];
-    float vx[DW ? XR : GS][DW ? NS : 8];
+    float vx[DW ? XR : GS][DW ? NS : 8], vh[DW ? HP : 1], ah[DW ? HP : 1], rah[DW ? HP : 1];
+    const auto halo = [&](int h, int& r, int& j) {                         // value h 64 + lane of the halo: its row, its column of xs
+        const int e = h * 64 + lane;
+        r = e / max(2 * HALO, 1);
+        j = e - r * 2 * HALO;
+        j += j < HALO ? 0 : NT;
+        r = min(r, XR - 1);
+    };
     auto fetch = [&](int c0) {
         const x6_u4* wsrc = reinterpret_cast<const x6_u4*>(pwp) + (size_t)(c0 / 16) * MT * 192;
 #pragma unroll
@@ -133,7 +141,15 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
             for (int r = 0; r < XR; ++r)
 #pragma unroll
-                for (int sx = 0; sx < NS; ++sx) vx[r][sx] = xb[(size_t)(c0 + wave + 4 * r) * p.ldx + min(max(n0 - halo + sx * 64 + lane, 0), T - 1)];
+                for (int sx = 0; sx < NS; ++sx) vx[r][sx] = xb[(size_t)(c0 + wave + 4 * r) * p.ldx + min(n0 + sx * 64 + lane, T - 1)];
+#pragma unroll
+            for (int h = 0; h < HP; ++h) {
+                int r, j;
+                halo(h, r, j);
+                const int c = c0 + wave + 4 * r;
+                vh[h] = xb[(size_t)c * p.ldx + min(max(n0 - HALO + j, 0), T - 1)];
+                ah[h] = pa1[c]; rah[h] = pra1[c];
+            }
         } else {
 #pragma unroll
             for (int g = 0; g < GS; ++g) {
@@ -155,11 +171,18 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                 const float al = pa1[c], ral = pra1[c];
 #pragma unroll
                 for (int sx = 0; sx < NS; ++sx) {
-                    const int j = sx * 64 + lane, t = n0 - halo + j;
-                    const float u = j < ncols && t >= 0 && t < T ? vx[r][sx] : 0.0f;
-                    if (j < XS) xs[cc][j] = x6_snake(u, al, ral);
+                    const int j = sx * 64 + lane;
+                    xs[cc][HALO + j] = x6_snake(n0 + j < T ? vx[r][sx] : 0.0f, al, ral);
                 }
                 __builtin_amdgcn_sched_barrier(0);                          // (a row at a time: the values in flight take the registers)
+            }
+#pragma unroll
+            for (int h = 0; h < HP; ++h) {
+                int r, j;
+                halo(h, r, j);
+                const int t = n0 - HALO + j;
+                const float u = x6_snake(t >= 0 && t < T ? vh[h] : 0.0f, ah[h], rah[h]);
+                if (h * 64 + lane < XR * 2 * HALO) xs[wave + 4 * r][j] = u;
             }
         } else {
 #pragma unroll
@@ -192,7 +215,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                     const int cc = kg * 8 + j, c = c0 + cc;
                     float a = 0.0f;
 #pragma unroll
-                    for (int k = 0; k < 7; ++k) a += pw7[c * 7 + k] * xs[cc][n + k * p.dil];
+                    for (int k = 0; k < 7; ++k) a += pw7[c * 7 + k] * xs[cc][n + k * DIL];
                     v[j] = x6_snake(a + pb1[c], pa2[c], pra2[c]);
                     if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
                 }
@@ -291,7 +314,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                             float a = 0.0f;
 #pragma unroll 1
                             for (int k = 0; k < 7; ++k) {
-                                const int t = n + (k - 3) * p.dil;
+                                const int t = n + (k - 3) * DIL;
                                 a = fmaf(pw7[c * 7 + k], x6_snake(t >= 0 && t < T ? xb[(size_t)c * p.ldx + t] : 0.0f, pa1[c], pra1[c]), a);
                             }
                             v = fmaf(pAT[(size_t)c * C + m], x6_snake(a + pb1[c], pa2[c], pra2[c]), v);
@@ -309,9 +332,11 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
         }
     }
 }
-template <int C, bool DW, int KC, int NT, bool OUT>
-__global__ void __launch_bounds__(256, KC == 32 ? 2 : DW || (OUT && C >= 96) ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
-    pw_x6_body<C, DW, KC, NT, OUT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.dil, p.ldx, p.ldr, p.ldy}, o, o.alpha, o.ralpha, o.p);
+// Blocks a compute unit: chunks of 32 channels two; chunks of 16 as many as the registers of a dilation allow without spills that cost more than they give (us at three, at the bound
+// taken: 48 channels, 1181 blocks, dilation 1 28.6 / 23.3 at five, 9 28.6 / 36.1; 64, 49152 blocks, 1 1169 / 1067, 3 1182 / 1175, 9 1169 / 1891)
+template <int C, int DIL, int KC, int NT, bool PF, bool OUT>
+__global__ void __launch_bounds__(256, KC == 32 ? 2 : DIL == 9 ? 3 : DIL ? (C <= 64 ? 5 : C == 96 ? 4 : 3) : OUT && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
+    pw_x6_body<C, DIL, KC, NT, PF, OUT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.ldx, p.ldr, p.ldy, p.nbx, p.per, p.tiles}, o, o.alpha, o.ralpha, o.p);
 }
 
 // 128 channels, at most 256 blocks of 128 columns (a compute unit each, one serial chain of chunks): 64 columns per block.  96 blocks: 28 -> 22 us;
@@ -320,39 +345,52 @@ __global__ void __launch_bounds__(256, KC == 32 ? 2 : DW || (OUT && C >= 96) ? 3
 // blocks are all resident at once, else 16 (us, chunks of 32 / 16): 128 channels 96 blocks 28 / 33, 384: 34 / 38, 576: 61 / 45, 24576: 1584 / 1430;
 // 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150 (with taps 16: 592 blocks, two rounds of 32).  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32;
 // up to 512 blocks 64 columns (half the conversions and accumulators per thread, three blocks a compute unit): 313 blocks with planes out 50 -> 42.
-template <int C, bool DW>
+// PF, the next chunk's samples and weights requested behind this one's staging (us, without / with): 192 channels 42.4 / 40.1 and 259 / 246, 96 without taps 24.0 / 22.8 and 145.7 / 138,
+// 128 in 64 columns 22 / 16-20; chunks of 16 with taps are slower for it (64 channels, 49152 blocks: 1169 / 1364-1522; 48, 7500: 149 / 179-202), 128 in blocks of 128 columns keep a
+// third block a compute unit instead (24576 blocks 1400 / 1650).
+template <int C, int DIL>
 static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hipStream_t s) {
-    const dim3 grid((p.T + 127) / 128, batch);
-#define X6_GO(KC, NT) do { \
-        const dim3 g((p.T + NT - 1) / NT, batch); \
-        if (!DW && p.out) hipLaunchKernelGGL((k_pw_x6<C, DW, KC, NT, !DW>), g, dim3(256), 0, s, p, wp, *p.out); \
-        else hipLaunchKernelGGL((k_pw_x6<C, DW, KC, NT, false>), g, dim3(256), 0, s, p, wp, CodecPlanes{}); \
+#define X6_GO(KC, NT, PF) do { \
+        PwFusedParams f = p; \
+        f.nbx = (p.T + NT - 1) / NT; f.tiles = f.nbx * batch; f.per = (f.tiles + 7) / 8; \
+        const dim3 g(8 * f.per); \
+        if (!DIL && p.out) hipLaunchKernelGGL((k_pw_x6<C, DIL, KC, NT, PF, !DIL>), g, dim3(256), 0, s, f, wp, *p.out); \
+        else hipLaunchKernelGGL((k_pw_x6<C, DIL, KC, NT, PF, false>), g, dim3(256), 0, s, f, wp, CodecPlanes{}); \
         return; } while (0)
-    if constexpr (C == 128) {
-        if ((int64_t)grid.x * batch <= 256) X6_GO(32, 64);
+    const int64_t blocks = (int64_t)((p.T + 127) / 128) * batch;
+    if constexpr (C == 48) X6_GO(16, 128, false);
+    else if constexpr (C == 192) {
+        if (blocks <= 512) X6_GO(32, 64, true);
+        X6_GO(32, 128, true);
+    } else {
+        if constexpr (C == 128) {
+            if (blocks <= 256) X6_GO(32, 64, true);
+        }
+        if (blocks > (C == 96 && !DIL ? 768 : 512)) X6_GO(16, 128, DIL == 0 && C != 128);
+        X6_GO(32, 128, C != 128);
     }
-    if constexpr (C == 48) X6_GO(16, 128);
-    else if constexpr (C <= 128) {
-        if ((int64_t)grid.x * batch > (C == 96 && !DW ? 768 : 512)) X6_GO(16, 128);
-    }
-    if constexpr (C == 192) {
-        if ((int64_t)grid.x * batch <= 512) X6_GO(32, 64);
-    }
-    if constexpr (C != 48) X6_GO(32, 128);
 #undef X6_GO
 }
 
-// 64 channels stay on k_pw_fused: twice the columns per product, bound by memory and by the units' VALU work (1.16 ms here, 1.10 there)
+// 64 channels with taps: one form for every length, as a row's bits must not change with it.  us, k_pw_fused / here, dilations of 1, 3 and 9: 96 blocks 17.2 / 13.5 12.8 13.4,
+// 288: 23.6 / 21.3 22.1 21.4, 768: 41 / 39.5 43.1 42.1, 49152: 1120 / 1067 1175 1212.  Without taps (HBM-bound there: twice the columns per product) they stay on k_pw_fused.
 bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s) {
     if (!pack) pack = codec_x6_scope();
-    if (!pack || codec_exact_f32() || !(dw ? C == 48 || C == 96 || C == 128 : (C == 96 || C == 128 || C == 192))) return false;
+    if (!pack || codec_exact_f32() || (dw && p.dil != 1 && p.dil != 3 && p.dil != 9) || !(dw ? C == 48 || C == 64 || C == 96 || C == 128 : (C == 96 || C == 128 || C == 192))) return false;
     const uint16_t* wp = pack->get_x6(p.AT, 1, C, C, s).wp;
-    if (dw && C == 48) launch_x6<48, true>(p, wp, batch, s);
-    else if (dw && C == 96) launch_x6<96, true>(p, wp, batch, s);
-    else if (dw) launch_x6<128, true>(p, wp, batch, s);
-    else if (C == 96) launch_x6<96, false>(p, wp, batch, s);
-    else if (C == 128) launch_x6<128, false>(p, wp, batch, s);
-    else launch_x6<192, false>(p, wp, batch, s);
+    auto taps = [&](auto c) {
+        constexpr int W = decltype(c)::value;
+        if (p.dil == 1) launch_x6<W, 1>(p, wp, batch, s);
+        else if (p.dil == 3) launch_x6<W, 3>(p, wp, batch, s);
+        else launch_x6<W, 9>(p, wp, batch, s);
+    };
+    if (dw && C == 48) taps(std::integral_constant<int, 48>{});
+    else if (dw && C == 64) taps(std::integral_constant<int, 64>{});
+    else if (dw && C == 96) taps(std::integral_constant<int, 96>{});
+    else if (dw) taps(std::integral_constant<int, 128>{});
+    else if (C == 96) launch_x6<96, 0>(p, wp, batch, s);
+    else if (C == 128) launch_x6<128, 0>(p, wp, batch, s);
+    else launch_x6<192, 0>(p, wp, batch, s);
     return true;
 }
 
