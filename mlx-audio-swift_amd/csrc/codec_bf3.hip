@@ -640,10 +640,10 @@ bool codec_planes_strided(const GemmParams& p, int batch, CodecPlanes& out) {
     return true;
 }
 
-bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot, CodecPlanes& out) {
-    CodecPack* pack = p.pack ? p.pack : tl_pack;
+// (the planes a contraction takes; the memory is codec_planes')
+static bool codec_planes_shape(int mode, bool snake, const GemmParams& p, int batch, CodecPlanes& out) {
     Bf3Shape h;
-    if (!pack || codec_exact_f32() || !bf3_shape(mode, p, h) || h.Cin % 32) return false;
+    if (!(p.pack ? p.pack : tl_pack) || codec_exact_f32() || !bf3_shape(mode, p, h) || h.Cin % 32) return false;
     const bool two = bf3_takes(mode, p, h);
     if (!two && !(snake && bf3_three(mode, p))) return false;
     const Bf3Tile t = bf3_tile(p, h, batch);
@@ -651,6 +651,11 @@ bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot
     out.n = two ? 2 : 3; out.Cp = h.Cin; out.Tp = t.Tp; out.t_org = h.t_org; out.ends = h.span > 0 || h.extra > 0;
     out.stride = (size_t)batch * t.Tp * h.Cin;
     if (snake) { out.alpha = p.alpha; out.ralpha = p.ralpha; }
+    return true;
+}
+bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot, CodecPlanes& out) {
+    if (!codec_planes_shape(mode, snake, p, batch, out)) return false;
+    CodecPack* pack = p.pack ? p.pack : tl_pack;
     pack->planes[slot].alloc(out.n * out.stride);
     out.p = pack->planes[slot].p;
     return true;
@@ -760,6 +765,13 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
 void launch_gemm_chain(const CodecOp* ops, int n, int batch, hipStream_t s) {
     CodecPlanes cur{}, nxt{};
     bool have = false;
+    // (the largest of each turn first: a buffer that grows along the chain waits for the device at every step of its first pass)
+    int top[2] = {-1, -1};
+    size_t most[2] = {0, 0};
+    for (int i = 0; i + 1 < n; ++i)
+        if (codec_planes_shape(ops[i + 1].mode, ops[i + 1].snake, ops[i + 1].g, batch, nxt) && nxt.n * nxt.stride > most[i & 1]) { most[i & 1] = nxt.n * nxt.stride; top[i & 1] = i + 1; }
+    for (int slot = 0; slot < 2; ++slot)
+        if (top[slot] >= 0) codec_planes(ops[top[slot]].mode, ops[top[slot]].snake, ops[top[slot]].g, batch, slot, nxt);
     for (int i = 0; i < n; ++i) {
         const CodecOp& o = ops[i];
         const bool want = i + 1 < n && codec_planes(ops[i + 1].mode, ops[i + 1].snake, ops[i + 1].g, batch, i & 1, nxt);
