@@ -18,7 +18,6 @@
 // Work decomposition, epilogues and the in-block split-K combine are those of k_gemm_skinny; K ranges are cut at scale groups.
 // A group's share of a sum is fma(scale, sum q x, bias * sum x), written out: contracted as the compiler likes, it was the other way round in some
 // unrolled copies of the loop and not in others, and a prompt's bits depended on how many rows shared its slice.  k_gemm_pf_codes (lm_prefill.hip) has the same.
-// (Four n-tiles per wave run decode steps only, where 16 and 32 rows agree.)
 #include "common.h"
 #include "lm_kernels.h"
 
@@ -250,8 +249,7 @@ __global__ void __launch_bounds__(KSB == 8 ? 512 : 256, 2) k_gemm_skinny_q(const
             unpack_bf16x4(SBUF[U][r][1], bi);                                                       \
             _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                       \
                 _Pragma("unroll") for (int e = 0; e < 4; ++e)                                       \
-                    acc[r][mt][e] += R == 4 ? sc[e] * ag[r][mt][e] + bi[e] * sx[mt][e]              \
-                                            : fmaf(sc[e], ag[r][mt][e], bi[e] * sx[mt][e]);         \
+                    acc[r][mt][e] += fmaf(sc[e], ag[r][mt][e], bi[e] * sx[mt][e]);                  \
         }                                                                                           \
     }
 #endif
@@ -332,16 +330,17 @@ __global__ void __launch_bounds__(KSB == 8 ? 512 : 256, 2) k_gemm_skinny_q(const
 // index is made scalar, so tile and K-range arithmetic and the base addresses live in SGPRs.  Groups past the wave's range are loaded
 // from its last group (clamped) and enter with scale = bias = 0: straight-line code, no load can sink behind a branch.  The
 // accumulators pass through LDS once at the end (a 16 x 16 float tile per (r, mt), written [m][n], read back as the streaming
-// kernel's lanes hold them), so the epilogues and the in-block split-K combine are shared; eight waves per item are possible here.
+// kernel's lanes hold them), so the epilogues and the in-block split-K combine are shared.  The wide form (four n-tiles, eight waves: gate and up at up to 16 rows) requests six
+// groups a wave, as many as the 63 loads a wave may have in flight allow, and a wave closes each pair of gate and up tiles: 3072 -> 2 x 8192 at 8 bits (53 MB) 14.8 us streaming,
+// 13.2 so, 12.6 with the pairs on two waves (4.2 TB/s).  Scales and biases through LDS instead of 2-byte loads: 14.2; x fragments of the live rows alone: nothing.
 // Per-element arithmetic is that of k_gemm_skinny_q; the in-block combine adds KSB partials in wave order.
 template <int MT, int R, int EPI, int KSB, int BITS, int U>
-__global__ void __launch_bounds__(256, 2) k_gemm_skinny_q1(const void* Qp, const bf16_t* SB, const bf16_t* X,     // not __restrict__: see the
+__global__ void __launch_bounds__(KSB * 64, 2) k_gemm_skinny_q1(const void* Qp, const bf16_t* SB, const bf16_t* X,     // not __restrict__: see the
                                                                             void* __restrict__ out, int NT, int G, int S, int n_items, int N_out, int Mpad,   // fence below
                                                                             const bf16_t* __restrict__ bias) {
-    static_assert(EPI != EPI_SILU_MUL || R == 2, "silu-mul epilogue pairs a gate tile with an up tile");
+    static_assert(EPI != EPI_SILU_MUL || (R & 1) == 0, "silu-mul epilogue pairs a gate tile with an up tile");
     typedef typename QTile<BITS>::type WT;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    static_assert(KSB == 4, "one block of four waves per item, its waves split the item's K range (eight waves measured worse and were removed)");
     const int item = blockIdx.x;
     if (item >= n_items) return;
     const int ntg = item / S, ks = item - ntg * S;
@@ -461,6 +460,24 @@ __global__ void __launch_bounds__(256, 2) k_gemm_skinny_q1(const void* Qp, const
         }
     const int rd = (lane & 15) * 4 + (lane >> 4);
     __syncthreads();
+    if constexpr (EPI == EPI_SILU_MUL && R == 4) {         // a wave for each pair of gate and up tiles
+        const int mt = wave / (R / 2), pr = wave % (R / 2);
+        if (mt >= MT || ntg * R + 2 * pr + 1 >= NT) return;
+        f32x4_t two[2][MT];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            float4 s0 = red[0][(2 * pr + r) * MT + mt][rd];
+#pragma unroll
+            for (int wv = 1; wv < KSB; ++wv) {
+                float4 t = red[wv][(2 * pr + r) * MT + mt][rd];
+                s0.x += t.x; s0.y += t.y; s0.z += t.z; s0.w += t.w;
+            }
+#pragma unroll
+            for (int m2 = 0; m2 < MT; ++m2) two[r][m2] = (f32x4_t){s0.x, s0.y, s0.z, s0.w};
+        }
+        qgemm_epilogue<MT, 2, EPI>(two, out, ntg * (R / 2) + pr, ks, NT, N_out, Mpad, lane, mt, bias);
+        return;
+    }
     for (int mt = wave; mt < MT; mt += KSB) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -482,7 +499,7 @@ template <int MT, int BITS, int U>
 static void launch_qgemm1_mt(int epi, int R, int ksb, const void* Qp, const bf16_t* SB, const bf16_t* X, void* out, int NT, int G, int S,
                              int N_out, int Mpad, const bf16_t* bias, hipStream_t s) {
     int n_items = ((NT + R - 1) / R) * S;
-    dim3 grid(n_items), block(256);
+    dim3 grid(n_items), block(64 * ksb);
 #define QGEMM1_CASE(E, RR, KS)                                                                                      \
     if (epi == E && R == RR && ksb == KS) {                                                                         \
         hipLaunchKernelGGL((k_gemm_skinny_q1<MT, RR, E, KS, BITS, U>), grid, block, 0, s, Qp, SB, X, out, NT, G, S, n_items, \
@@ -493,6 +510,7 @@ static void launch_qgemm1_mt(int epi, int R, int ksb, const void* Qp, const bf16
     QGEMM1_CASE(EPI_PARTIAL, 2, 4)
     QGEMM1_CASE(EPI_BF16, 2, 4)
     QGEMM1_CASE(EPI_SILU_MUL, 2, 4)
+    if constexpr (MT == 1 && U == 6) QGEMM1_CASE(EPI_SILU_MUL, 4, 8)
 #undef QGEMM1_CASE
     throw MisError(MIS_ERR_GENERATION_FAILED, "unsupported quantised GEMM variant");
 }
@@ -548,6 +566,12 @@ void launch_gemm_skinny_q(int bits, int epi, int R, int ksb, const void* Qp, con
         { if (bits == 8) launch_qgemm_mt<M, 8, UU>(epi, R, ksb, Qp, SB, X, out, NT, G, S, N_out, Mpad, bias, s);         \
           else launch_qgemm_mt<M, 4, UU>(epi, R, ksb, Qp, SB, X, out, NT, G, S, N_out, Mpad, bias, s);                   \
           return; }
+        // 33 to 48 groups: up to six a wave.  Fewer leave part of its buffer to clamped reloads, and more than 16 rows need 48 registers more than a wave has
+        if (v2 && R == 4 && ksb == 8 && epi == EPI_SILU_MUL && Mpad == 16 && G > 32 && G <= 48) {
+            if (bits == 8) launch_qgemm1_mt<1, 8, 6>(epi, R, ksb, Qp, SB, X, out, NT, G, S, N_out, Mpad, bias, s);
+            else launch_qgemm1_mt<1, 4, 6>(epi, R, ksb, Qp, SB, X, out, NT, G, S, N_out, Mpad, bias, s);
+            return;
+        }
         if (R == 4) { if (Mpad / 16 == 1) QGEMM_R4(1, 1) else QGEMM_R4(2, 1) }
         else { if (Mpad / 16 == 1) QGEMM_R4(1, 2) else QGEMM_R4(2, 2) }
 #undef QGEMM_R4
