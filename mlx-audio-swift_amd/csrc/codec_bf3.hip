@@ -635,7 +635,7 @@ bool codec_planes_strided(const GemmParams& p, int batch, CodecPlanes& out) {
     out = CodecPlanes{};
     out.n = 3; out.Cp = h.Cin; out.Tp = t.Tp;
     out.stride = (size_t)batch * t.Tp * h.Cin;
-    pack->planes[0].alloc(3 * out.stride);
+    if (3 * out.stride > pack->planes[0].n) pack->planes[0].alloc(3 * out.stride * 9 / 8);       // (the convolutions behind take as much, but for their tiles' ends)
     out.p = pack->planes[0].p;
     return true;
 }
