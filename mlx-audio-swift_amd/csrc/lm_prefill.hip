@@ -18,12 +18,12 @@
 //                         PF_SILU   act = T(T(g T(sigmoid g)) u), gate / up tiles interleaved as packed (:283)
 //   k_gemm_pf_wide      the same on tiles of 128 .. 192 x 256, four waves (gemm_tiles.h): many rows
 //   k_gemm_pf_ring      the same on tiles of 32 x 32: few rows
-//   k_gemm_pf_codes     the same on 8- and 4-bit codes, more than 96 or 128 rows (fewer: k_gemm_skinny_q, lm_qgemm.hip, the same bits)
+//   k_gemm_pf_codes     the same on 8- and 4-bit codes, more than 64 rows (fewer: k_gemm_skinny_q, lm_qgemm.hip, the same bits)
 //   k_pf_rope_append    q|k|v of the chunk -> roped queries (bf16 rows) and the tiled K / V caches of the decode step
 //   k_pf_attn           causal attention of the chunk's queries over the caches (MFMA, K / V tiles shared by 128 or 256 queries)
 //   k_pf_rmsnorm        x[r] = RMSNorm(h[r]) row-major
 //   k_pf_pack_last      every sequence's last row -> the packed x operand of the decode step (lm_head of the first new token)
-//   k_pf_pack_rows      rows -> packed x operand of a slice of k_gemm_skinny_q
+//   k_pf_pack_rows      rows -> packed x operand of k_gemm_skinny_q
 // Rounding points are those of the decode step (bf16 at every MLX primitive boundary); only float32 summation orders differ.
 #include "common.h"
 #include "gemm_tiles.h"
@@ -496,8 +496,7 @@ __global__ void __launch_bounds__(128) k_gemm_pf_ring(PfGemmParams p) {
 // ahead, one barrier.  Bound: a group costs an output a product, an FMA and an addition beside its 64 products - VALU above matrix pipe, two blocks a compute unit
 // share both.  (Two FMAs into one chain of sums are 10 % faster at 128 x 128 - gate | up of 3216 rows 583 us, 641 here - but then a prompt's bits depend on the
 // other prompts of its call, which decide between slices and tiles.)
-// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 70 rows 5.7 / 7.3, 107 6.1 / 7.3, 175 8.7 / 8.6, 274 13.8 / 9.4, 413 18.5 / 10.6, 804 33.6 / 16.2,
-// 3202 129 / 46.6.
+// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 64 rows 5.2 / 6.5, 96 7.9 / 7.0, 128 8.0 / 7.1, 274 13.8 / 8.8, 804 33.6 / 16.2, 3202 129 / 46.6.
 __device__ __forceinline__ uint4 pf_codes(uint2 w) {
     uint32_t o[4];
 #pragma unroll
@@ -517,18 +516,23 @@ __device__ __forceinline__ uint4 pf_codes(uint32_t w) {
 template <int BITS> struct PfCode { typedef uint2 type; };
 template <> struct PfCode<4> { typedef uint32_t type; };
 
-// GS: scale groups a k-step
-template <int EPI, int TN, int TM, int GS, int BITS>
-__global__ void __launch_bounds__(256, 2) k_gemm_pf_codes(PfGemmParams p, const void* __restrict__ Qp, const bf16_t* __restrict__ SB) {
+// Q: teams of four waves, each with a quarter of the groups (4) or all of them (1)
+template <int EPI, int TN, int TM, int BITS, int Q>
+__global__ void __launch_bounds__(256 * Q, Q == 1 ? 2 : 4) k_gemm_pf_codes(PfGemmParams p, const void* __restrict__ Qp, const bf16_t* __restrict__ SB) {
     typedef typename PfCode<BITS>::type WT;
     constexpr int BN = 32 * TN, BM = 32 * TM, HELD = TN == 4 ? 2 : 0;
     __shared__ f32x4_t held[HELD ? HELD : 1][256];
-    __shared__ __attribute__((aligned(1024))) bf16_t Ws[2][GS][BN * PF_BK];
-    __shared__ __attribute__((aligned(1024))) bf16_t Xs[2][GS][BM * PF_BK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    static_assert(Q == 1 || (Q == 4 && !HELD), "one team, or one a quarter");
+    __shared__ __attribute__((aligned(1024))) bf16_t Wt[Q][2][BN * PF_BK];
+    __shared__ __attribute__((aligned(1024))) bf16_t Xt[Q][2][BM * PF_BK];
+    const int tid = Q == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int team = Q == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    bf16_t (&Ws)[2][BN * PF_BK] = Wt[team];
+    bf16_t (&Xs)[2][BM * PF_BK] = Xt[team];
     const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
     if (n0 >= p.N) return;                              // (padding of the grid, see launch_gemm_pf)
     const int wn = wave >> 1, wm = wave & 1, NT = p.N >> 4, KT = p.K >> 5, G = p.K / PF_BK;
+    const int ga = G * team / Q, gb = G * (team + 1) / Q, steps = (G + Q - 1) / Q;         // (ceil(G / 4): the longest quarter)
     f32x4_t acc[TN][TM];
 #pragma unroll
     for (int i = 0; i < TN; ++i)
@@ -551,31 +555,25 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf_codes(PfGemmParams p, const 
         xoff[q] = ((uint32_t)min(m0 + r, p.M - 1) * p.K + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2;
     }
     const uint32_t sl = lane >> 4;
-    WT w[GS][TN];
-    uint2 sb[GS][TN][2];
-    auto loadW = [&](int g0) {                          // (groups past the end: the last one again, never multiplied)
+    WT w[TN];
+    uint2 sb[TN][2];
+    auto loadW = [&](int g) {                           // (groups past the end: the last one again, never multiplied)
 #pragma unroll
-        for (int u = 0; u < GS; ++u)
-#pragma unroll
-            for (int q = 0; q < TN; ++q) w[u][q] = (wsrc[q] + (size_t)min(g0 + u, G - 1) * 128)[(uint32_t)lane];
+        for (int q = 0; q < TN; ++q) w[q] = (wsrc[q] + (size_t)min(g, G - 1) * 128)[(uint32_t)lane];
     };
-    auto loadS = [&](int g, int u, int q) {
+    auto loadS = [&](int g, int q) {
         const uint2* o = sbp[q] + (size_t)min(g, G - 1) * 8;
-        sb[u][q][0] = o[sl]; sb[u][q][1] = o[sl + 4];
+        sb[q][0] = o[sl]; sb[q][1] = o[sl + 4];
     };
     auto putW = [&](int buf) {
 #pragma unroll
-        for (int u = 0; u < GS; ++u)
-#pragma unroll
-            for (int q = 0; q < TN; ++q) *reinterpret_cast<uint4*>(&Ws[buf][u][(wave * TN + q) * 512 + lane * 8]) = pf_codes(w[u][q]);
+        for (int q = 0; q < TN; ++q) *reinterpret_cast<uint4*>(&Ws[buf][(wave * TN + q) * 512 + lane * 8]) = pf_codes(w[q]);
     };
-    auto stageX = [&](int buf, int g0) {
+    auto stageX = [&](int buf, int g) {
 #pragma unroll
-        for (int u = 0; u < GS; ++u)
-#pragma unroll
-            for (int q = 0; q < TM; ++q)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(reinterpret_cast<const unsigned char*>(p.X + (size_t)min(g0 + u, G - 1) * PF_BK) + xoff[q]),
-                                                 (__attribute__((address_space(3))) void*)&Xs[buf][u][(wave * TM + q) * 8 * PF_BK], 16, 0, 0);
+        for (int q = 0; q < TM; ++q)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(reinterpret_cast<const unsigned char*>(p.X + (size_t)min(g, G - 1) * PF_BK) + xoff[q]),
+                                             (__attribute__((address_space(3))) void*)&Xs[buf][(wave * TM + q) * 8 * PF_BK], 16, 0, 0);
     };
     bf16x8_t ones;
 #pragma unroll
@@ -604,69 +602,81 @@ __global__ void __launch_bounds__(256, 2) k_gemm_pf_codes(PfGemmParams p, const 
     };
     int part = 1;                                       // the quarter of the groups that begins next
     const int sw = (lane >> 1) & 7;
-    loadW(0);
+    loadW(ga);
     putW(0);
-    loadW(GS);
+    loadW(ga + 1);
 #pragma unroll
-    for (int u = 0; u < GS; ++u)
-#pragma unroll
-        for (int q = 0; q < TN; ++q) loadS(u, u, q);
-    stageX(0, 0);
-    for (int g0 = 0, buf = 0; g0 < G; g0 += GS, buf ^= 1) {
+    for (int q = 0; q < TN; ++q) loadS(ga, q);
+    stageX(0, ga);
+    for (int g = ga, st = 0, buf = 0; st < steps; ++st, ++g, buf ^= 1) {
         __syncthreads();                                // X and codes of this step are in LDS, the codes of the next and the scales of this one in registers
-        bf16x8_t a[GS][2][TN], b[GS][2][TM];            // all fragment reads first, then the next DMA (see k_gemm_pf)
+        bf16x8_t a[2][TN], b[2][TM];                    // all fragment reads first, then the next DMA (see k_gemm_pf)
 #pragma unroll
-        for (int u = 0; u < GS; ++u)
+        for (int kk = 0; kk < 2; ++kk) {
+            const int pos = ((kk * 4 + (lane >> 4)) ^ sw) * 8;
 #pragma unroll
-            for (int kk = 0; kk < 2; ++kk) {
-                const int pos = ((kk * 4 + (lane >> 4)) ^ sw) * 8;
+            for (int i = 0; i < TN; ++i) a[kk][i] = *reinterpret_cast<const bf16x8_t*>(&Ws[buf][((wn * TN + i) * 2 + kk) * 512 + lane * 8]);
 #pragma unroll
-                for (int i = 0; i < TN; ++i) a[u][kk][i] = *reinterpret_cast<const bf16x8_t*>(&Ws[buf][u][((wn * TN + i) * 2 + kk) * 512 + lane * 8]);
-#pragma unroll
-                for (int j = 0; j < TM; ++j) b[u][kk][j] = *reinterpret_cast<const bf16x8_t*>(&Xs[buf][u][(wm * TM * 16 + j * 16 + (lane & 15)) * PF_BK + pos]);
-            }
-        const bool more = g0 + GS < G;
+            for (int j = 0; j < TM; ++j) b[kk][j] = *reinterpret_cast<const bf16x8_t*>(&Xs[buf][(wm * TM * 16 + j * 16 + (lane & 15)) * PF_BK + pos]);
+        }
+        const bool more = st + 1 < steps;
         if (more) putW(buf ^ 1);                        // (the other buffer: read by everybody before this step's barrier)
         __builtin_amdgcn_sched_barrier(0);
-        loadW(g0 + 2 * GS);
-        if (more) stageX(buf ^ 1, g0 + GS);
+        loadW(g + 2);
+        if (more) stageX(buf ^ 1, g + 1);
         __builtin_amdgcn_sched_barrier(0);
+        if (Q > 1 && g >= gb) continue;                 // (a shorter quarter: the barriers of the others)
+        if (Q == 1 && part < 4 && g == G * part / 4) {
+            close(part == 1);
+            do ++part; while (part < 4 && G * part / 4 == g);
+        }
+        float sx[TM];                               // (the rows of a tile of ones are one row)
 #pragma unroll
-        for (int u = 0; u < GS; ++u) {
-            if (u && g0 + u >= G) break;
-            if (part < 4 && g0 + u == G * part / 4) {
-                close(part == 1);
-                do ++part; while (part < 4 && G * part / 4 == g0 + u);
+        for (int j = 0; j < TM; ++j) {
+            f32x4_t t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[0][j], zero, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[1][j], t, 0, 0, 0);
+            sx[j] = t[0];
+        }
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+            const uint2 s0 = sb[i][0], b0 = sb[i][1];
+            const float sc[4] = {__uint_as_float(s0.x << 16), __uint_as_float(s0.x & 0xffff0000u), __uint_as_float(s0.y << 16), __uint_as_float(s0.y & 0xffff0000u)};
+            const float bi[4] = {__uint_as_float(b0.x << 16), __uint_as_float(b0.x & 0xffff0000u), __uint_as_float(b0.y << 16), __uint_as_float(b0.y & 0xffff0000u)};
+#pragma unroll
+            for (int j0 = 0; j0 < TM; j0 += 2) {
+                f32x4_t ag[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0][i], b[0][j0 + j], zero, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1][i], b[1][j0 + j], ag[j], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j0 + j][e] += fmaf(sc[e], ag[j][e], bi[e] * sx[j0 + j]);
             }
-            float sx[TM];                               // (the rows of a tile of ones are one row)
-#pragma unroll
-            for (int j = 0; j < TM; ++j) {
-                f32x4_t t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[u][0][j], zero, 0, 0, 0);
-                t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[u][1][j], t, 0, 0, 0);
-                sx[j] = t[0];
-            }
-#pragma unroll
-            for (int i = 0; i < TN; ++i) {
-                const uint2 s0 = sb[u][i][0], b0 = sb[u][i][1];
-                const float sc[4] = {__uint_as_float(s0.x << 16), __uint_as_float(s0.x & 0xffff0000u), __uint_as_float(s0.y << 16), __uint_as_float(s0.y & 0xffff0000u)};
-                const float bi[4] = {__uint_as_float(b0.x << 16), __uint_as_float(b0.x & 0xffff0000u), __uint_as_float(b0.y << 16), __uint_as_float(b0.y & 0xffff0000u)};
-#pragma unroll
-                for (int j0 = 0; j0 < TM; j0 += 2) {
-                    f32x4_t ag[2];
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][0][i], b[u][0][j0 + j], zero, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) ag[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][1][i], b[u][1][j0 + j], ag[j], 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i][j0 + j][e] += fmaf(sc[e], ag[j][e], bi[e] * sx[j0 + j]);
-                }
-                loadS(g0 + GS + u, u, i);               // (the next step's, into the registers just read)
-            }
+            loadS(g + 1, i);               // (the next step's, into the registers just read)
         }
     }
-    close(false);
+    if constexpr (Q > 1) {                              // the quarters in order: those of the others through LDS
+        f32x4_t (*sums)[TN * TM][256] = reinterpret_cast<f32x4_t (*)[TN * TM][256]>(&Wt[0][0][0]);
+        static_assert((Q - 1) * TN * TM * 256 * sizeof(f32x4_t) <= sizeof(Wt), "the sums fit where the codes were");
+        __syncthreads();
+        if (team)
+#pragma unroll
+            for (int i = 0; i < TN * TM; ++i) sums[team - 1][i][tid] = acc[i / TM][i % TM];
+        __syncthreads();
+        if (team) return;
+#pragma unroll
+        for (int i = 0; i < TN * TM; ++i) {
+            f32x4_t t = acc[i / TM][i % TM];
+#pragma unroll
+            for (int w2 = 0; w2 < Q - 1; ++w2)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) t[e] += sums[w2][i][tid][e];
+            tot[i / TM][i % TM] = t;
+        }
+    } else
+        close(false);
 #pragma unroll
     for (int h = 0; h < HELD; ++h) tot[(TN * TM - HELD + h) / TM][(TN * TM - HELD + h) % TM] = held[h][tid];
     pf_epilogue<EPI, TN, TM>(p, tot, (n0 >> 4) + wn * TN, m0 + wm * TM * 16, lane);
@@ -675,20 +685,19 @@ void launch_gemm_pf_codes(int epi, int bits, const bf16_t* X, const void* Qp, co
     MIS_REQUIRE(K % PF_BK == 0 && K >= PF_BK && N % 16 == 0 && M >= 1 && (bits == 8 || bits == 4) && (epi != PF_SILU || N % 32 == 0) && (int64_t)M * K < (1ll << 31),
                 MIS_ERR_GENERATION_FAILED, "prefill GEMM on codes: bad shape");
     PfGemmParams p{X, nullptr, C, M, N, K, PfExtra()};
-    auto go = [&](auto e, auto t, auto gs, auto b) {
-        constexpr int E = decltype(e)::value, T = decltype(t)::value, GS = decltype(gs)::value, B = decltype(b)::value;
+    auto go = [&](auto e, auto t, auto q, auto b) {
+        constexpr int E = decltype(e)::value, T = decltype(t)::value, Q = decltype(q)::value, B = decltype(b)::value;
         const int nx = cdiv(N, 32 * T);
-        hipLaunchKernelGGL((k_gemm_pf_codes<E, T, T, GS, B>), dim3(nx >= 16 ? (int)round_up(nx, 8) : nx, cdiv(M, 32 * T)), dim3(256), 0, s, p, Qp, SB);
+        hipLaunchKernelGGL((k_gemm_pf_codes<E, T, T, B, Q>), dim3(nx >= 16 ? (int)round_up(nx, 8) : nx, cdiv(M, 32 * T)), dim3(256 * Q), 0, s, p, Qp, SB);
     };
     auto tile = [&](auto e, auto b) {
-        // Few blocks of 64 x 64 wait for a step's loads alone on their compute unit: more groups a step.  Orpheus-3B, 8 bits, us, 1 / 2 / 4 groups (one chain of sums): o
-        // 160 rows (144 blocks) 54 / - / 39, down 139 / - / 96; q|k|v 160 (240) 54 / - / 38, 272 (400) 54 / 44 / -, 416 (560) 57 / 78 / -; o 416 (336) 54 / 43 / -, 816
-        // (624) 57 / 80 / -; gate | up 112 (512) 57 / 46 / -.  In quarters, by this rule: 36, 89; 36, 46, 57; 45, 56; 49.  128 x 128: o 1632 rows (312 blocks) 107,
-        // gate | up 3216 (3328) 641: 500 TFLOP/s
+        // Up to 512 tiles of 64 x 64: a team of waves for each quarter of K, one block a compute unit (131 KB).  With one team and four groups a step (two from 257 tiles on) a
+        // wave a SIMD waited for each step's loads, fragments and conversions in turn.  Orpheus-3B, 8 bits, us, one team / four: 176 rows o (144 tiles) 36 / 23, down 89 / 54,
+        // q|k|v (240) 38 / 24; 256 rows q|k|v (320) 46 / 41; 400 rows o (336) 45 / 42.  More tiles: 800 rows o (624) 57 / 60, q|k|v (1040) 73 / 79.  128 x 128: o 1632 rows
+        // (312 blocks) 107, gate | up 3216 (3328) 641: 500 TFLOP/s
         const int64_t nb = (int64_t)cdiv(N, 64) * cdiv(M, 64);
         if ((int64_t)cdiv(N, 128) * cdiv(M, 128) >= 256) go(e, std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{}, b);
         else if (nb > 512) go(e, std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{}, b);
-        else if (nb > 256) go(e, std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{}, b);
         else go(e, std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{}, b);
     };
     auto width = [&](auto e) {
