@@ -495,8 +495,8 @@ __global__ void __launch_bounds__(128) k_gemm_pf_ring(PfGemmParams p) {
 // code once for all its rows, into the fragment image that k_gemm_pf reads.  A k-step is a scale group: X by LDS-DMA and codes and scales through registers one step
 // ahead, one barrier.  Bound: a group costs an output a product, an FMA and an addition beside its 64 products - VALU above matrix pipe, two blocks a compute unit
 // share both.  (Two FMAs into one chain of sums are 10 % faster at 128 x 128 - gate | up of 3216 rows 583 us, 641 here - but then a prompt's bits depend on the
-// other prompts of its call, which decide between slices and tiles.)
-// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 64 rows 5.2 / 6.5, 96 7.9 / 7.0, 128 8.0 / 7.1, 274 13.8 / 8.8, 804 33.6 / 16.2, 3202 129 / 46.6.
+// other prompts of its call, which decide between the kernels.)
+// Prompt pass of Orpheus-3B at 8 bits, ms, slices of 64 rows / here: 804 rows 33.6 / 16.2, 3202 129 / 46.6; here, the kernels of 176 rows: 6.4 (8.2 with one team a block).
 __device__ __forceinline__ uint4 pf_codes(uint2 w) {
     uint32_t o[4];
 #pragma unroll

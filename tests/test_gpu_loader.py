@@ -154,8 +154,8 @@ def test_quantised_role_with_a_per_layer_override_falls_back_to_the_dense_copy()
 def test_batched_prefill_on_code_streamed_weights(bits, monkeypatch):
     """`model(inputIds, cache:)` on a quantised checkpoint: the [positions x rows] pass runs on the packed rows of the prompts instead of
     falling back to one position at a time.  Against the float32-dequant oracle (quantizedMatmul's arithmetic) and against the
-    position-by-position path; a decode step continues behind it.  Ragged rows, 110 of 7 prompts: k_gemm_pf_codes (slices of
-    k_gemm_skinny_q take up to 96: test_gpu_prompt_codes.py)."""
+    position-by-position path; a decode step continues behind it.  Ragged rows, 110 of 7 prompts: k_gemm_pf_codes
+    (k_gemm_skinny_q takes up to 64: test_gpu_prompt_codes.py)."""
     from gpu_util import logits_errors, record
     W = ollama.make_synthetic_weights(QCFG, seed=99)
     m = mas.LlamaTTSModel(lm_host_config(QCFG))

@@ -1,6 +1,6 @@
-"""Prompt GEMMs on 8- and 4-bit codes: slices of 64 rows up to 96 (up to 128 where ff > 4096; csrc/lm_qgemm.hip, a second slice among them), tiles behind (csrc/lm_prefill.hip, k_gemm_pf_codes:
-64 x 64 with one, two and four scale groups a step, 128 x 128), remainders in rows, columns and groups; ragged prompts.  Against the oracle on the float32 weights
-s q + b; and a prompt has the bits that it has alone, whatever slices or tiles its call takes."""
+"""Prompt GEMMs on 8- and 4-bit codes: tiles (csrc/lm_prefill.hip, k_gemm_pf_codes: 64 x 64 with four teams of waves or one, 128 x 128) for more than 64 rows, the decode step's
+kernel (csrc/lm_qgemm.hip) for fewer - each prompt alone -, remainders in rows, columns and groups; ragged prompts.  Against the oracle on the float32 weights
+s q + b; and a prompt has the bits that it has alone, whatever kernels its call takes."""
 import numpy as np
 import pytest
 import torch
@@ -41,7 +41,7 @@ def test_prompts_on_codes(hidden, heads, ff, bits, total):
     many = dev.lm_prefill(rows, max_context=128)
     oracle = ollama.LlamaOracle(cfg, W32, round="bf16")
     for b in range(len(rows)):
-        alone = dev.lm_prefill([rows[b]], max_context=128)                                             # one to four tiles of 16 rows a slice
+        alone = dev.lm_prefill([rows[b]], max_context=128)                                             # one to four tiles of 16 rows
         assert np.array_equal(alone[0], many[b]), (b, lens[b])
     for b in (0, 1, len(rows) - 1):
         oracle.reset(1)
