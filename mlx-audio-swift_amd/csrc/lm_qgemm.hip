@@ -556,11 +556,11 @@ void launch_gemm_skinny_q(int bits, int epi, int R, int ksb, const void* Qp, con
     MIS_REQUIRE(bits == 8 || bits == 4, MIS_ERR_GENERATION_FAILED, "quantised GEMM: 8 or 4 bits");
     MIS_REQUIRE(S >= 1 && S <= G, MIS_ERR_GENERATION_FAILED, "quantised GEMM: %d K slices for %d scale groups", S, G);   // a wave may get none
     // one-shot arrangement (k_gemm_skinny_q1) wherever a wave's K share fits its buffer.  MIS_QGEMM_V2=0 (read once per process) sends
-    // those launches through the streaming kernel instead: that kernel is the product path of the wide roles at Orpheus width, and the
-    // switch is how tests/test_gpu_loader.py holds it to the oracle at small widths too.  (Eight waves per item and capped buffer sizes
+    // those launches through the streaming kernel instead: that kernel is the product path of the wide roles at Orpheus width (but for gate and up at up to 16 rows), and the
+    // switch is how tests/test_gpu_loader.py holds it to the oracle at small widths too.  (For the split-K roles eight waves per item and capped buffer sizes
     // were measured and removed: profiles/r03/qgemm_one_shot.jsonl.)
     static const int v2 = getenv("MIS_QGEMM_V2") ? atoi(getenv("MIS_QGEMM_V2")) : 1;
-    if (R == 4 || ksb == 8) {                      // the wide roles' arrangement (streaming kernel only): R = 4 -> one group per buffer
+    if (R == 4 || ksb == 8) {                      // the wide roles' arrangement: R = 4 -> one group per buffer of the streaming kernel
         MIS_REQUIRE(Mpad / 16 <= 2, MIS_ERR_GENERATION_FAILED, "quantised GEMM: four n-tiles per wave / eight waves per item are built for <= 32 rows");
 #define QGEMM_R4(M, UU)                                                                                              \
         { if (bits == 8) launch_qgemm_mt<M, 8, UU>(epi, R, ksb, Qp, SB, X, out, NT, G, S, N_out, Mpad, bias, s);         \
