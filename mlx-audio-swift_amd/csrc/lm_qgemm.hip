@@ -18,6 +18,7 @@
 // Work decomposition, epilogues and the in-block split-K combine are those of k_gemm_skinny; K ranges are cut at scale groups.
 // A group's share of a sum is fma(scale, sum q x, bias * sum x), written out: contracted as the compiler likes, it was the other way round in some
 // unrolled copies of the loop and not in others, and a prompt's bits depended on how many rows shared its slice.  k_gemm_pf_codes (lm_prefill.hip) has the same.
+// Four n-tiles a wave, which decode steps alone run, keep what they were built with: a wave's groups but its last one or two (qg_first) are fma(bias, sum x, scale * sum q x).
 #include "common.h"
 #include "lm_kernels.h"
 
@@ -49,6 +50,9 @@ __device__ __forceinline__ void unpack_bf16x4(uint2 v, float (&o)[4]) {
     o[0] = __uint_as_float(v.x << 16); o[1] = __uint_as_float(v.x & 0xffff0000u);
     o[2] = __uint_as_float(v.y << 16); o[3] = __uint_as_float(v.y & 0xffff0000u);
 }
+// a group's share of a sum; first: one of the groups that k_gemm_skinny_q takes in its steady state of two, four n-tiles a wave
+__device__ __forceinline__ float qg_share(bool first, float sc, float ag, float bi, float sx) { return first ? fmaf(bi, sx, sc * ag) : fmaf(sc, ag, bi * sx); }
+__device__ __forceinline__ int qg_first(int groups) { return (groups - 1) / 2 * 2; }
 
 // epilogues: identical arithmetic to gemm_epilogue of lm_kernels.hip (kept in step with it)
 template <int MT, int R, int EPI>
@@ -208,7 +212,7 @@ __global__ void __launch_bounds__(KSB == 8 ? 512 : 256, 2) k_gemm_skinny_q(const
     }
 #endif
 #if defined(MIS_QGEMM_ABLATE) && MIS_QGEMM_ABLATE == 1   /* diagnostics build: loads only - every loaded register is consumed by one xor */
-#define QG_GROUP(WBUF, XBUF, SBUF, U)                                                               \
+#define QG_GROUP(WBUF, XBUF, SBUF, U, FIRST)                                                        \
     {                                                                                               \
         uint32_t h = 0;                                                                             \
         _Pragma("unroll") for (int j = 0; j < 2; ++j) {                                             \
@@ -227,7 +231,7 @@ __global__ void __launch_bounds__(KSB == 8 ? 512 : 256, 2) k_gemm_skinny_q(const
         acc[0][0][0] += __uint_as_float(h & 0x007fffffu);                                           \
     }
 #else
-#define QG_GROUP(WBUF, XBUF, SBUF, U)                                                               \
+#define QG_GROUP(WBUF, XBUF, SBUF, U, FIRST)                                                        \
     {                                                                                               \
         f32x4_t ag[R][MT], sx[MT];                                                                  \
         _Pragma("unroll") for (int mt = 0; mt < MT; ++mt) {                                         \
@@ -249,15 +253,15 @@ __global__ void __launch_bounds__(KSB == 8 ? 512 : 256, 2) k_gemm_skinny_q(const
             unpack_bf16x4(SBUF[U][r][1], bi);                                                       \
             _Pragma("unroll") for (int mt = 0; mt < MT; ++mt)                                       \
                 _Pragma("unroll") for (int e = 0; e < 4; ++e)                                       \
-                    acc[r][mt][e] += fmaf(sc[e], ag[r][mt][e], bi[e] * sx[mt][e]);                  \
+                    acc[r][mt][e] += qg_share(R == 4 && FIRST, sc[e], ag[r][mt][e], bi[e], sx[mt][e]); \
         }                                                                                           \
     }
 #endif
 #define QG_MATH_FULL(WBUF, XBUF, SBUF)                                                              \
-    _Pragma("unroll") for (int u = 0; u < QGEMM_U; ++u) QG_GROUP(WBUF, XBUF, SBUF, u)
+    _Pragma("unroll") for (int u = 0; u < QGEMM_U; ++u) QG_GROUP(WBUF, XBUF, SBUF, u, true)
 #define QG_MATH_TAIL(WBUF, XBUF, SBUF, GBASE)                                                       \
     _Pragma("unroll") for (int u = 0; u < QGEMM_U; ++u) {                                           \
-        if ((GBASE) + u < g1) QG_GROUP(WBUF, XBUF, SBUF, u)                                         \
+        if ((GBASE) + u < g1) QG_GROUP(WBUF, XBUF, SBUF, u, false)                                  \
     }
     if (g0 < g1) {
         int g = g0;
@@ -403,7 +407,7 @@ __global__ void __launch_bounds__(KSB * 64, 2) k_gemm_skinny_q1(const void* Qp, 
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const bool live = g0 + u < g1;
+            const bool live = g0 + u < g1, first = R == 4 && u < qg_first(U) && u < qg_first(g1 - g0);
             // nothing that consumes a loaded value may rise above the fence (conversions and the x-only MFMA are pure and would,
             // taking their vmcnt wait with them): every buffer register passes through an empty volatile asm here, which is also
             // where the wait for this group's loads belongs
@@ -442,7 +446,7 @@ __global__ void __launch_bounds__(KSB * 64, 2) k_gemm_skinny_q1(const void* Qp, 
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[r][mt][e] += fmaf(sc, ag[r][mt][e], bi * sx[mt][e]);
+                    for (int e = 0; e < 4; ++e) acc[r][mt][e] += qg_share(first, sc, ag[r][mt][e], bi, sx[mt][e]);
             }
             __builtin_amdgcn_sched_barrier(0);             // groups are consumed in the order their loads were issued (vmcnt is in order)
         }
