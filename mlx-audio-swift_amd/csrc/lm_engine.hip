@@ -17,7 +17,6 @@
 #include <string.h>
 #include <algorithm>
 #include <chrono>
-#include <functional>
 #include <set>
 
 #define ORPHEUS_END_OF_SPEECH 128258
@@ -793,7 +792,7 @@ static void enqueue_lm_head(mis_tts* c, const bf16_t* head = nullptr) {
 static bool prefill_batched_ok(const mis_tts* c, int Lmax) {
     const bool off = getenv("MIS_PREFILL_SEQ") && atoi(getenv("MIS_PREFILL_SEQ")) != 0;             // A/B and parity tests (read per call)
     const int HD = c->H * c->D;
-    // dense weights: k_gemm_pf and its forms; all four roles streamed as codes: k_gemm_pf_codes or, up to 64 rows, k_gemm_skinny_q; a mix: position by position
+    // dense weights: k_gemm_pf and its forms; all four roles streamed as codes: k_gemm_pf_codes or slices of k_gemm_skinny_q; a mix: position by position
     const bool dense = !c->q_qkv.on && !c->q_o.on && !c->q_gu.on && !c->q_down.on;
     const bool coded = c->q_qkv.on && c->q_o.on && c->q_gu.on && c->q_down.on;
     return !off && Lmax >= 2 && (dense || coded) && c->d % 64 == 0 && HD % 64 == 0 && c->ff % 64 == 0 && c->d >= 128 && HD >= 128 && c->ff >= 128;
@@ -900,17 +899,23 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
     const size_t Mc = round_up((size_t)most, 16);                            // GEMM rows round up to 16
     c->pf_h.alloc(Mc * d); c->pf_x.alloc(Mc * d); c->pf_attn.alloc(Mc * HD);
     c->pf_q.alloc(Mc * HD);
-    // quantised checkpoints (every role streamed as codes): k_gemm_pf_codes on the chunk's rows; a chunk of up to 64 rows runs the decode step's
-    // k_gemm_skinny_q - rows packed into MFMA fragments first, float32 sums out, the residual add as its own small kernel; gate|up writes the packed activation its
+    // quantised checkpoints (every role streamed as codes): k_gemm_pf_codes on the chunk's rows; a chunk of few rows runs the decode step's k_gemm_skinny_q on
+    // 64-row slices - rows packed into MFMA fragments first, float32 sums out, the residual add as its own small kernel; gate|up writes the packed activation its
     // down projection reads.
     const bool coded = c->q_qkv.on;
     if (coded) c->pf_qkv.alloc(Mc * c->Nqkv); else c->pf_qkv16.alloc(Mc * c->Nqkv);
-    // (the same bits.  us more or less of a prompt pass of Orpheus-3B with the tiles than with slices of 64 rows: 32 rows +1300, 64 +1290, 96 -930, 112 -600, 128 -890)
-    const bool tiled = coded && Mc > 64;
+    // (the same bits.  us more or less of a prompt pass of Orpheus-3B with the tiles than with slices of 64 rows: 32 rows +1300, 64 +1290, 96 -930, 112 -600, 128 -890.
+    // 4-bit codes of a large matrix are read twice for less than a tile converts them: pass in us, slices / tiles, gate | up of 2048 x 16384 80 rows 1023 / 1002, of 2560 x 19456
+    // 80 1297 / 1341, 88 1383 / 1351, 3072 x 16384 80 1574 / 1596, 88 1676 / 1618, 4096 x 22016 80 1543 / 1678, 96 1637 / 1685, 112 1691 / 1697; 8 bits, that one 80 1651 / 1643)
+    const int64_t wide = (int64_t)2 * c->ff * d;
+    const bool tiled = coded && Mc > (c->q_gu.bits != 4 || wide < 40'000'000 ? 64u : wide < 70'000'000 ? 80u : 96u);
     if (coded && !tiled) { c->pf_xpk.alloc((size_t)64 * std::max(d, HD)); c->pf_actpk.alloc((size_t)64 * c->ff); c->pf_tmp.alloc((size_t)64 * d); }
     else c->pf_act.alloc(Mc * c->ff);
     auto q_tiled = [&](int epi, const mis_tts::QRole& q, int li, const bf16_t* x, void* out, int M, int N, int K) {
         launch_gemm_pf_codes(epi, q.bits, x, q.q.p + q.q_layer * li, q.sb.p + q.sb_layer * li, out, M, N, K, s);
+    };
+    auto q_rows = [&](int M, auto body) {
+        for (int r0 = 0; r0 < M; r0 += 64) body(r0, std::min(64, M - r0));
     };
     auto q_partial = [&](const mis_tts::QRole& q, int li, const bf16_t* xpk, float* out, int N, int K, int mp) {
         launch_gemm_skinny_q(q.bits, EPI_PARTIAL, c->r_part, c->ksb_part, q.q.p + q.q_layer * li, q.sb.p + q.sb_layer * li, xpk, out, N / 16, K / 64, 1, N, mp, s);
@@ -931,10 +936,11 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
         else launch_pf_embed_rmsnorm(c->emb.p, prompt_mat_dev, lens_dev, Lmax, t0, tc, batch, 0, c->V, c->norms.p, c->pf_h.p, c->pf_x.p, nullptr, nullptr, Mr, d, eps, s);
         for (int li = 0; li < c->L; ++li) {
             if (tiled) q_tiled(PF_F32, c->q_qkv, li, c->pf_x.p, c->pf_qkv.p, M, c->Nqkv, d);
-            else if (coded) {
-                launch_pf_pack_rows(c->pf_x.p, c->pf_xpk.p, M, d, s);
-                q_partial(c->q_qkv, li, c->pf_xpk.p, c->pf_qkv.p, c->Nqkv, d, M);
-            } else {
+            else if (coded) q_rows(M, [&](int r0, int mp) {
+                launch_pf_pack_rows(c->pf_x.p + (size_t)r0 * d, c->pf_xpk.p, mp, d, s);
+                q_partial(c->q_qkv, li, c->pf_xpk.p, c->pf_qkv.p + (size_t)r0 * c->Nqkv, c->Nqkv, d, mp);
+            });
+            else {
                 PfExtra ex;
                 ex.ldx = d; ex.ldc = c->Nqkv;
                 launch_gemm_pf(PF_ROWS_BF16, c->pf_x.p, c->wqkv.p + layer_qkv_elems(c) * li, c->pf_qkv16.p, M, c->Nqkv, d, s, ex);
@@ -954,22 +960,24 @@ static void prefill_batched(mis_tts* c, const int32_t* prompt_mat_dev, const int
             pa.rope_in_dtype = c->cfg.rope_ops_in_dtype;
             launch_pf_attention(pa, s);
             if (tiled) q_tiled(PF_RESID, c->q_o, li, c->pf_attn.p, c->pf_h.p, M, d, HD);
-            else if (coded) {
-                launch_pf_pack_rows(c->pf_attn.p, c->pf_xpk.p, M, HD, s);
-                q_partial(c->q_o, li, c->pf_xpk.p, c->pf_tmp.p, d, HD, M);
-                launch_pf_add_resid(c->pf_h.p, c->pf_tmp.p, (size_t)M * d, s);
-            } else launch_gemm_pf(PF_RESID, c->pf_attn.p, c->wo.p + layer_o_elems(c) * li, c->pf_h.p, M, d, HD, s);
+            else if (coded) q_rows(M, [&](int r0, int mp) {
+                launch_pf_pack_rows(c->pf_attn.p + (size_t)r0 * HD, c->pf_xpk.p, mp, HD, s);
+                q_partial(c->q_o, li, c->pf_xpk.p, c->pf_tmp.p, d, HD, mp);
+                launch_pf_add_resid(c->pf_h.p + (size_t)r0 * d, c->pf_tmp.p, (size_t)mp * d, s);
+            });
+            else launch_gemm_pf(PF_RESID, c->pf_attn.p, c->wo.p + layer_o_elems(c) * li, c->pf_h.p, M, d, HD, s);
             launch_pf_rmsnorm(c->pf_h.p, c->norms.p + (size_t)(2 * li + 1) * d, c->pf_x.p, M, d, eps, s);
             if (tiled) {
                 q_tiled(PF_SILU, c->q_gu, li, c->pf_x.p, c->pf_act.p, M, 2 * c->ff, d);
                 q_tiled(PF_RESID, c->q_down, li, c->pf_act.p, c->pf_h.p, M, d, c->ff);
-            } else if (coded) {
-                launch_pf_pack_rows(c->pf_x.p, c->pf_xpk.p, M, d, s);
+            } else if (coded) q_rows(M, [&](int r0, int mp) {
+                launch_pf_pack_rows(c->pf_x.p + (size_t)r0 * d, c->pf_xpk.p, mp, d, s);
                 launch_gemm_skinny_q(c->q_gu.bits, EPI_SILU_MUL, 2, c->ksb_gu, c->q_gu.q.p + c->q_gu.q_layer * li, c->q_gu.sb.p + c->q_gu.sb_layer * li,
-                                     c->pf_xpk.p, c->pf_actpk.p, 2 * c->ff / 16, d / 64, 1, c->ff, M, s);
-                q_partial(c->q_down, li, c->pf_actpk.p, c->pf_tmp.p, d, c->ff, M);
-                launch_pf_add_resid(c->pf_h.p, c->pf_tmp.p, (size_t)M * d, s);
-            } else {
+                                     c->pf_xpk.p, c->pf_actpk.p, 2 * c->ff / 16, d / 64, 1, c->ff, mp, s);
+                q_partial(c->q_down, li, c->pf_actpk.p, c->pf_tmp.p, d, c->ff, mp);
+                launch_pf_add_resid(c->pf_h.p + (size_t)r0 * d, c->pf_tmp.p, (size_t)mp * d, s);
+            });
+            else {
                 launch_gemm_pf(PF_SILU, c->pf_x.p, c->wgu.p + layer_gu_elems(c) * li, c->pf_act.p, M, 2 * c->ff, d, s);
                 launch_gemm_pf(PF_RESID, c->pf_act.p, c->wdown.p + layer_down_elems(c) * li, c->pf_h.p, M, d, c->ff, s);
             }

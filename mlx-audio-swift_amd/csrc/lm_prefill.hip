@@ -18,12 +18,12 @@
 //                         PF_SILU   act = T(T(g T(sigmoid g)) u), gate / up tiles interleaved as packed (:283)
 //   k_gemm_pf_wide      the same on tiles of 128 .. 192 x 256, four waves (gemm_tiles.h): many rows
 //   k_gemm_pf_ring      the same on tiles of 32 x 32: few rows
-//   k_gemm_pf_codes     the same on 8- and 4-bit codes, more than 64 rows (fewer: k_gemm_skinny_q, lm_qgemm.hip, the same bits)
+//   k_gemm_pf_codes     the same on 8- and 4-bit codes, more than 64 rows (fewer, and up to 96 of large 4-bit matrices: k_gemm_skinny_q, lm_qgemm.hip, the same bits)
 //   k_pf_rope_append    q|k|v of the chunk -> roped queries (bf16 rows) and the tiled K / V caches of the decode step
 //   k_pf_attn           causal attention of the chunk's queries over the caches (MFMA, K / V tiles shared by 128 or 256 queries)
 //   k_pf_rmsnorm        x[r] = RMSNorm(h[r]) row-major
 //   k_pf_pack_last      every sequence's last row -> the packed x operand of the decode step (lm_head of the first new token)
-//   k_pf_pack_rows      rows -> packed x operand of k_gemm_skinny_q
+//   k_pf_pack_rows      rows -> packed x operand of a slice of k_gemm_skinny_q
 // Rounding points are those of the decode step (bf16 at every MLX primitive boundary); only float32 summation orders differ.
 #include "common.h"
 #include "gemm_tiles.h"
@@ -694,7 +694,8 @@ void launch_gemm_pf_codes(int epi, int bits, const bf16_t* X, const void* Qp, co
         // Up to 512 tiles of 64 x 64: a team of waves for each quarter of K, one block a compute unit (131 KB).  With one team and four groups a step (two from 257 tiles on) a
         // wave a SIMD waited for each step's loads, fragments and conversions in turn.  Orpheus-3B, 8 bits, us, one team / four: 176 rows o (144 tiles) 36 / 23, down 89 / 54,
         // q|k|v (240) 38 / 24; 256 rows q|k|v (320) 46 / 41; 400 rows o (336) 45 / 42.  More tiles: 800 rows o (624) 57 / 60, q|k|v (1040) 73 / 79.  128 x 128: o 1632 rows
-        // (312 blocks) 107, gate | up 3216 (3328) 641: 500 TFLOP/s
+        // (312 blocks) 107, gate | up 3216 (3328) 641: 500 TFLOP/s.  Narrower, a prompt pass of four layers in us, teams up to 256 tiles / up to 512: width 1024 (q|k|v 320 - 512
+        // tiles) 257 rows 626 / 618, 512 707 / 702; 2048 128 rows (gate | up 384) 690 / 663, 257 (q|k|v 320) 966 / 927; at 4 bits 257 986 / 974, 512 1069 / 1053
         const int64_t nb = (int64_t)cdiv(N, 64) * cdiv(M, 64);
         if ((int64_t)cdiv(N, 128) * cdiv(M, 128) >= 256) go(e, std::integral_constant<int, 4>{}, std::integral_constant<int, 1>{}, b);
         else if (nb > 512) go(e, std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{}, b);

@@ -1,5 +1,5 @@
-"""Prompt GEMMs on 8- and 4-bit codes: tiles (csrc/lm_prefill.hip, k_gemm_pf_codes: 64 x 64 with four teams of waves or one, 128 x 128) for more than 64 rows, the decode step's
-kernel (csrc/lm_qgemm.hip) for fewer - each prompt alone -, remainders in rows, columns and groups; ragged prompts.  Against the oracle on the float32 weights
+"""Prompt GEMMs on 8- and 4-bit codes: tiles (csrc/lm_prefill.hip, k_gemm_pf_codes: 64 x 64 with four teams of waves or one, 128 x 128) for more than 64 rows, slices of the
+decode step's kernel (csrc/lm_qgemm.hip) for fewer, and for up to 96 of large 4-bit matrices; remainders in rows, columns and groups; ragged prompts.  Against the oracle on the float32 weights
 s q + b; and a prompt has the bits that it has alone, whatever kernels its call takes."""
 import numpy as np
 import pytest
@@ -12,8 +12,10 @@ from oracle import mlxquant as mq
 pytestmark = pytest.mark.gpu
 
 
-# hidden 1088 = 17 groups, ff 1216 = 19, heads 3 x 128 = 6: steps of two and four groups end inside; 1024 / 3072: 128 x 128 tiles for gate | up from 641 rows on
-@pytest.mark.parametrize("hidden, heads, ff, bits, total", [(1088, 3, 1216, 8, 75), (1088, 3, 1216, 4, 96), (1088, 3, 1216, 8, 97), (1088, 3, 1216, 4, 431), (1088, 3, 1216, 8, 1000), (1024, 16, 3072, 8, 130),
+# hidden 1088 = 17 groups, ff 1216 = 19, heads 3 x 128 = 6: quarters of unequal length; 60 and 64 rows: three or more prompts in one slice, 65: the first in tiles; 3072 / 8192 at
+# 4 bits: slices of 64 and 16 rows, then tiles; 1024 / 3072: 128 x 128 tiles for gate | up from 641 rows on
+@pytest.mark.parametrize("hidden, heads, ff, bits, total", [(1088, 3, 1216, 8, 60), (1088, 3, 1216, 4, 64), (1088, 3, 1216, 8, 64), (1088, 3, 1216, 8, 65), (1088, 3, 1216, 4, 65),
+                                                            (3072, 16, 8192, 4, 72), (3072, 16, 8192, 4, 81), (1088, 3, 1216, 8, 75), (1088, 3, 1216, 4, 96), (1088, 3, 1216, 8, 97), (1088, 3, 1216, 4, 431), (1088, 3, 1216, 8, 1000), (1024, 16, 3072, 8, 130),
                                                             (1024, 16, 3072, 4, 333), (1024, 16, 3072, 8, 700), (1024, 16, 4160, 8, 128), (1024, 16, 4160, 4, 129)])
 def test_prompts_on_codes(hidden, heads, ff, bits, total):
     from gpu_util import logits_errors
