@@ -97,13 +97,18 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
     constexpr int KG = KC / 8, MT = (C + 31) / 32, APC = KC / 16 * MT * 192;       // channel groups, row tiles, 16-byte pieces of weights per chunk
     constexpr bool DW = DIL > 0;
     constexpr int XR = KC / 4, NS = NT / 64, GS = KG * NS / 4;                      // rows of x, strips of columns, (group, strip) pairs per wave
-    // (the dilation is a constant: as many columns are staged as it needs - the halo of a wave's rows one behind the other, 64 values at a time)
-    constexpr int HALO = 3 * DIL, XS = NT + 2 * HALO + 2, HP = (XR * 2 * HALO + 63) / 64;
+    // The dilation is a constant: as many columns are staged as it needs.  The halo of a wave's rows comes one row behind the other, 64 values at a time, each with its Snake's
+    // parameters; in chunks of 16 at most HR rows a load, whose parameters are scalar then - 16 registers less, a block more a compute unit (us, without / with: 64 channels,
+    // 49152 blocks, dilation 3 1180 / 1100, 9 1212 / 1097; 48, 1181 blocks, 9 28.4 / 22.8; 96, 592 blocks, 9 36.8 / 34.8, 3776 blocks 182 / 158; 128, 24576 blocks, 9 1440 / 1395;
+    // but 3 1400 / 1500, 96 channels 3 32.4 / 33.6; chunks of 32, 128 channels in 64 columns: 3 19.7 / 21.2, 9 17.1 / 21.8; 64 channels 3 12.7 / 13.4)
+    constexpr int HALO = 3 * DIL, XS = NT + 2 * HALO + 2, HR = KC != 16 ? 0 : DIL == 9 ? 1 : DIL == 3 && C <= 64 ? 2 : 0, HP = HR ? XR / (HR ? HR : 1) : (XR * 2 * HALO + 63) / 64;
+    static_assert(HR * 2 * HALO <= 64 && (!HR || XR % HR == 0), "a wave holds the halo of HR rows");
     __shared__ float xs[DW ? KC : 1][DW ? XS : 1];
     __shared__ uint4 sm[3 * KG * NT + APC];
     uint4 (&ts)[3][KG][NT] = *reinterpret_cast<uint4 (*)[3][KG][NT]>(sm);
     x6_u4 (&As)[APC] = *reinterpret_cast<x6_u4 (*)[APC]>(sm + 3 * KG * NT);
-    // The encoder's units take the place of k_x6_gemm in long rows only: a lane that sees a sum which is not finite takes its rows again as that kernel does
+    // Units of 48 and 96 channels (the encoder's) take the place of k_x6_gemm in long rows only, those of 64 (the decoder's) of an f32 kernel: a lane that sees a sum which is not
+    // finite takes its rows again as those do
     constexpr bool RETAKE = DW && C <= 96;
     constexpr bool SQ = C == 128 || NT == 64;             // 2 x 2 waves of half the rows and half the columns; else every wave: all C rows x 32 columns
     constexpr int MTW = SQ ? MT / 2 : MT, NTW = SQ ? NT / 64 : 1;
@@ -125,13 +130,13 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
     x6_u4 wv[(APC + 255) / 256];
-    float vx[DW ? XR : GS][DW ? NS : 8], vh[DW ? HP : 1], ah[DW ? HP : 1], rah[DW ? HP : 1];
-    const auto halo = [&](int h, int& r, int& j) {                         // value h 64 + lane of the halo: its row, its column of xs
-        const int e = h * 64 + lane;
-        r = e / max(2 * HALO, 1);
-        j = e - r * 2 * HALO;
+    float vx[DW ? XR : GS][DW ? NS : 8], vh[DW ? HP : 1], ah[DW && !HR ? HP : 1], rah[DW && !HR ? HP : 1];
+    const auto halo = [&](int h, int& r, int& j) {                         // the lane's value of load h of the halo: its row, its column of xs; false: none
+        const int i = HR ? (HR == 2 && lane >= 2 * HALO) : (h * 64 + lane) / max(2 * HALO, 1);
+        j = min((HR ? 0 : h * 64) + lane - i * 2 * HALO, max(2 * HALO - 1, 0));
         j += j < HALO ? 0 : NT;
-        r = min(r, XR - 1);
+        r = min(h * HR + i, XR - 1);
+        return HR ? lane < HR * 2 * HALO : h * 64 + lane < XR * 2 * HALO;
     };
     auto fetch = [&](int c0) {
         const x6_u4* wsrc = reinterpret_cast<const x6_u4*>(pwp) + (size_t)(c0 / 16) * MT * 192;
@@ -148,7 +153,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                 halo(h, r, j);
                 const int c = c0 + wave + 4 * r;
                 vh[h] = xb[(size_t)c * p.ldx + min(max(n0 - HALO + j, 0), T - 1)];
-                ah[h] = pa1[c]; rah[h] = pra1[c];
+                if constexpr (!HR) { ah[h] = pa1[c]; rah[h] = pra1[c]; }
             }
         } else {
 #pragma unroll
@@ -179,10 +184,16 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
             for (int h = 0; h < HP; ++h) {
                 int r, j;
-                halo(h, r, j);
+                const bool on = halo(h, r, j);
                 const int t = n0 - HALO + j;
-                const float u = x6_snake(t >= 0 && t < T ? vh[h] : 0.0f, ah[h], rah[h]);
-                if (h * 64 + lane < XR * 2 * HALO) xs[wave + 4 * r][j] = u;
+                float al = ah[HR ? 0 : h], ral = rah[HR ? 0 : h];
+                if constexpr (HR > 0) {
+                    const int c = c0 + wave + 4 * HR * h;
+                    al = pa1[c]; ral = pra1[c];
+                    if constexpr (HR == 2) { const float a1 = pa1[c + 4], ra1 = pra1[c + 4]; if (r & 1) { al = a1; ral = ra1; } }
+                }
+                const float u = x6_snake(t >= 0 && t < T ? vh[h] : 0.0f, al, ral);
+                if (on) xs[wave + 4 * r][j] = u;
             }
         } else {
 #pragma unroll
@@ -332,15 +343,15 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
         }
     }
 }
-// Blocks a compute unit: chunks of 32 channels two; chunks of 16 as many as the registers of a dilation allow without spills that cost more than they give (us at three, at the bound
-// taken: 48 channels, 1181 blocks, dilation 1 28.6 / 23.3 at five, 9 28.6 / 36.1; 64, 49152 blocks, 1 1169 / 1067, 3 1182 / 1175, 9 1169 / 1891)
+// Blocks a compute unit: chunks of 32 channels two; chunks of 16 as many as the registers allow without spills (us, three / five: 48 channels, 1181 blocks, dilation 1 28.6 / 23.3;
+// 64, 49152 blocks, dilation 1 1169 / 1067; dilation 9 with its halo's parameters in registers spilled at five: 1891)
 template <int C, int DIL, int KC, int NT, bool PF, bool OUT>
-__global__ void __launch_bounds__(256, KC == 32 ? 2 : DIL == 9 ? 3 : DIL ? (C <= 64 ? 5 : C == 96 ? 4 : 3) : OUT && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
+__global__ void __launch_bounds__(256, KC == 32 ? 2 : DIL ? (C <= 64 ? 5 : C == 96 ? 4 : 3) : OUT && C >= 96 ? 3 : 4) k_pw_x6(PwFusedParams p, const uint16_t* wp, CodecPlanes o) {
     pw_x6_body<C, DIL, KC, NT, PF, OUT>(p.X, p.R, p.Y, p.w7, p.b1, p.a1, p.ra1, p.a2, p.ra2, wp, p.AT, p.b2, PwScalars{p.T, p.ldx, p.ldr, p.ldy, p.nbx, p.per, p.tiles}, o, o.alpha, o.ralpha, o.p);
 }
 
 // 128 channels, at most 256 blocks of 128 columns (a compute unit each, one serial chain of chunks): 64 columns per block.  96 blocks: 28 -> 22 us;
-// 192 and 248: 23 and 25 (384 of 128 columns: 34).  (The next chunk's loads ahead of this one's products instead: 31 us, no registers left.)
+// 192 and 248: 23 and 25 (384 of 128 columns: 34).
 // Chunk depth (the same bits): 32 channels need half the barriers, 16 let three or four blocks (not two, C = 96: three) share a compute unit.  32 while its
 // blocks are all resident at once, else 16 (us, chunks of 32 / 16): 128 channels 96 blocks 28 / 33, 384: 34 / 38, 576: 61 / 45, 24576: 1584 / 1430;
 // 96 channels 626 blocks: 26.5 / 28.3, 4004: 162 / 150 (with taps 16: 592 blocks, two rounds of 32).  192 channels hold 96 accumulators either way: 313 blocks 36.6 / 52.4, 2004: 193 / 215, always 32;
@@ -372,8 +383,8 @@ static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hip
 #undef X6_GO
 }
 
-// 64 channels with taps: one form for every length, as a row's bits must not change with it.  us, k_pw_fused / here, dilations of 1, 3 and 9: 96 blocks 17.2 / 13.5 12.8 13.4,
-// 288: 23.6 / 21.3 22.1 21.4, 768: 41 / 39.5 43.1 42.1, 49152: 1120 / 1067 1175 1212.  Without taps (HBM-bound there: twice the columns per product) they stay on k_pw_fused.
+// 64 channels with taps: one form for every length, as a row's bits must not change with it.  us, k_pw_fused / here, dilations of 1, 3 and 9: 192 blocks 17.2 / 13.5 12.8 13.4,
+// 288: 19.0 / 15.1 14.9 15.6, 768: 26.1 / 23.8 23.8 23.8, 49152: 1122 / 1067 1090 1083.  Without taps (HBM-bound there: twice the columns per product) they stay on k_pw_fused.
 bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s) {
     if (!pack) pack = codec_x6_scope();
     if (!pack || codec_exact_f32() || (dw && p.dil != 1 && p.dil != 3 && p.dil != 9) || !(dw ? C == 48 || C == 64 || C == 96 || C == 128 : (C == 96 || C == 128 || C == 192))) return false;

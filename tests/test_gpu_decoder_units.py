@@ -22,7 +22,7 @@ def test_units_against_the_oracle(groups):
     assert got.shape == ref.shape and rms(got, ref) < 1e-4
 
 
-@pytest.mark.parametrize("rows, groups", [(3, 7), (2, 515), (9, 131)])      # 12, 516 and 594 blocks of 64 channels; a row alone: 4, 258, 66
+@pytest.mark.parametrize("rows, groups", [(3, 7), (2, 515), (9, 131), (4, 515)])      # 12, 516, 594 and 1032 blocks of 64 channels; a row alone: 4, 258, 66, 258
 def test_a_row_alone_has_its_bits(rows, groups):
     ocfg, _, dev = snac_pair(CFG)
     codes, noise = osnac.synthetic_codes(ocfg, rows, groups), osnac.synthetic_noise(ocfg, rows, groups)
