@@ -626,6 +626,18 @@ static Bf3Tile bf3_tile(const GemmParams& p, const Bf3Shape& h, int batch) {
 // Three planes, where the epilogue in front writes them: 1x1 contractions with Snake and a residual that k_x6_gemm would convert for itself
 static bool bf3_three(int mode, const GemmParams& p) { return mode == GEMM_RESID && p.alpha && p.M >= 48 && p.K > 192 && p.K <= 384; }
 
+// memory for planes; where there is none left the caller goes on without them
+static bool planes_fit(CodecPack& pack, int slot, size_t n, size_t spare) {
+    if (pack.plain) return false;
+    DevBuf<uint16_t>& b = pack.planes[slot];
+    if (b.p && n <= b.n) return true;
+    for (const size_t more : {spare, (size_t)0}) {
+        try { b.alloc(n + more); return true; }
+        catch (const MisNoMemory&) { if (!more) return false; }
+    }
+    return false;
+}
+
 // Strided convolutions of the encoders, on two taps of the phase split: three planes, written by k_enc_phase_planes
 bool codec_planes_strided(const GemmParams& p, int batch, CodecPlanes& out) {
     CodecPack* pack = codec_x6_scope();
@@ -635,7 +647,7 @@ bool codec_planes_strided(const GemmParams& p, int batch, CodecPlanes& out) {
     out = CodecPlanes{};
     out.n = 3; out.Cp = h.Cin; out.Tp = t.Tp;
     out.stride = (size_t)batch * t.Tp * h.Cin;
-    if (3 * out.stride > pack->planes[0].n) pack->planes[0].alloc(3 * out.stride * 9 / 8);       // (the convolutions behind take as much, but for their tiles' ends)
+    if (!planes_fit(*pack, 0, 3 * out.stride, 3 * out.stride / 8)) return false;                  // (the convolutions behind take as much, but for their tiles' ends)
     out.p = pack->planes[0].p;
     return true;
 }
@@ -656,7 +668,7 @@ static bool codec_planes_shape(int mode, bool snake, const GemmParams& p, int ba
 bool codec_planes(int mode, bool snake, const GemmParams& p, int batch, int slot, CodecPlanes& out) {
     if (!codec_planes_shape(mode, snake, p, batch, out)) return false;
     CodecPack* pack = p.pack ? p.pack : tl_pack;
-    pack->planes[slot].alloc(out.n * out.stride);
+    if (!planes_fit(*pack, slot, out.n * out.stride, 0)) return false;
     out.p = pack->planes[slot].p;
     return true;
 }
@@ -692,10 +704,11 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
     if (in) { P.xp = in->p; P.xplane = in->stride; }
     else {
         P.xplane = (size_t)batch * t.Tp * P.Cp;
-        p.pack->xs.alloc(2 * P.xplane);
-        P.xp = p.pack->xs.p;
+        DevBuf<uint16_t>& xs = p.pack->planes[out && out->p == p.pack->planes[0].p ? 1 : 0];
+        xs.alloc(2 * P.xplane);
+        P.xp = xs.p;
         const bool sn = snake && p.alpha;
-        hipLaunchKernelGGL(k_bf3_split, dim3((t.Tp + 63) / 64, (P.Cp + SP_CB - 1) / SP_CB, batch), dim3(256), 0, s, p.X, p.pack->xs.p, p.pack->xs.p + P.xplane,
+        hipLaunchKernelGGL(k_bf3_split, dim3((t.Tp + 63) / 64, (P.Cp + SP_CB - 1) / SP_CB, batch), dim3(256), 0, s, p.X, xs.p, xs.p + P.xplane,
                            sn ? p.alpha : nullptr, sn ? p.ralpha : nullptr, Cin, p.ldx, p.x_lo, p.Tin, P.Cp, t.Tp, h.t_org);
     }
     if (out) P.out = *out;

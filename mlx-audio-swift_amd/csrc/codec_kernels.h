@@ -72,7 +72,8 @@ struct CodecPack {
     std::vector<Entry> entries;
     struct X6 { const float* at; int ntaps, Cin, M, KS, MT32; uint16_t* wp; };
     std::vector<X6> x6;   // three-plane fragments (codec_x6.hip)
-    DevBuf<uint16_t> xs, planes[2];      // operands: split by the pre-pass; written by the epilogue in front (two, in turns)
+    DevBuf<uint16_t> planes[2];          // operands: written by the epilogue in front (in turns), or split by a pre-pass into the one that this call's epilogue does not write
+    bool plain = false;                  // no epilogue writes planes (codec_run)
     DevBuf<float> part;   // split-K slabs of launch-shaped contractions (GemmParams.split_k_ok)
     CodecPack() {}
     CodecPack(const CodecPack&) = delete;
@@ -81,6 +82,15 @@ struct CodecPack {
     const Entry& get(const float* at, int ntaps, int Cin, int M, hipStream_t s);
     const X6& get_x6(const float* at, int ntaps, int Cin, int M, hipStream_t s);
 };
+
+// One call of a codec.  Where it runs out of memory, the planes are given back and it runs once more without them - the pre-pass alone, half of the memory; the same bits
+template <class F> void codec_run(CodecPack& pack, F body) {
+    try { body(); return; }
+    catch (const MisNoMemory&) { if (!pack.planes[0].p && !pack.planes[1].p) throw; }
+    for (auto& b : pack.planes) b.release();                          // (waits for the device)
+    struct Plain { bool& on; explicit Plain(bool& b) : on(b) { on = true; } ~Plain() { on = false; } } plain(pack.plain);
+    body();
+}
 
 // Decoders open a scope around their launches: launch_gemm picks the scope's CodecPack up when GemmParams.pack is null.  Encoders (codebook decisions) open
 // one with bf3 = false: the three-plane contractions, which are as accurate as the f32 kernels, and none of two planes.  null: exact-f32 kernels only.

@@ -18,6 +18,7 @@ struct MisError : std::runtime_error {
     mis_status code;
     MisError(mis_status c, const std::string& m) : std::runtime_error(m), code(c) {}
 };
+struct MisNoMemory : MisError { using MisError::MisError; };         // the device's
 void mis_set_error(const char* fmt, ...);
 mis_status mis_fail(mis_status code, const char* fmt, ...);
 
@@ -29,6 +30,7 @@ mis_status mis_fail(mis_status code, const char* fmt, ...);
             char _b[512];                                                                    \
             snprintf(_b, sizeof(_b), "%s failed: %s (%s:%d)", #expr, hipGetErrorString(_e),  \
                      __FILE__, __LINE__);                                                    \
+            if (_e == hipErrorOutOfMemory) throw MisNoMemory(MIS_ERR_DEVICE, _b);            \
             throw MisError(MIS_ERR_DEVICE, _b);                                              \
         }                                                                                    \
     } while (0)
@@ -51,6 +53,9 @@ mis_status mis_fail(mis_status code, const char* fmt, ...);
     return MIS_OK;
 
 // ---------------------------------------------------------------------------- device memory
+// bytes that the library's buffers hold; an allocation past mis_debug_device_limit's limit fails as one past the card's memory does
+hipError_t mis_device_malloc(void** p, size_t bytes);
+void mis_device_free(void* p, size_t bytes);
 template <typename T>
 struct DevBuf {
     T* p = nullptr;
@@ -60,14 +65,14 @@ struct DevBuf {
     DevBuf& operator=(const DevBuf&) = delete;
     ~DevBuf() { release(); }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) mis_device_free(p, std::max<size_t>(n, 1) * sizeof(T));
         p = nullptr;
         n = 0;
     }
     void alloc(size_t count) {
         if (count <= n && p) return;
         release();
-        HIP_CHECK(hipMalloc((void**)&p, (count ? count : 1) * sizeof(T)));
+        HIP_CHECK(mis_device_malloc((void**)&p, (count ? count : 1) * sizeof(T)));
         n = count;
     }
     void zero(hipStream_t s) { if (p && n) HIP_CHECK(hipMemsetAsync(p, 0, n * sizeof(T), s)); }

@@ -296,14 +296,7 @@ extern "C" int64_t mis_dac_padded_length(const mis_dac* c, int64_t n_samples) {
 // audio f32 [batch, n_samples] (host or device) -> codes int32 [batch, nq, T], T = padded_length / hop (host or device), nq = n_quantizers
 // (0 = all codebooks; the reference's nQuantizers, DescriptQuantization.swift:120-147);
 // z_out (nullable) f32 [batch, latent, T]: the encoder output before quantisation
-extern "C" mis_status mis_dac_encode(mis_dac* c, const float* audio, int batch, int64_t n_samples, int n_quantizers, int32_t* codes_out, float* z_out) {
-    MIS_API_BEGIN
-    MIS_REQUIRE(c && audio && codes_out && batch >= 1 && n_samples >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
-    MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "DAC model not finalized");
-    MIS_REQUIRE(c->has_encoder, MIS_ERR_AUDIO_ENCODE, "this DAC handle was loaded without encoder weights");
-    MIS_REQUIRE(n_quantizers >= 0 && n_quantizers <= c->cfg.n_codebooks, MIS_ERR_INVALID_INPUT, "n_quantizers out of range");
-    const int nq = n_quantizers ? n_quantizers : c->cfg.n_codebooks;
-    HIP_CHECK(hipSetDevice(c->device));
+static void dac_encode(mis_dac* c, const float* audio, int batch, int64_t n_samples, int nq, int32_t* codes_out, float* z_out) {
     hipStream_t s = c->stream;
     const mis_dac_config& cf = c->cfg;
     const float* W = c->arena.p;
@@ -368,6 +361,16 @@ extern "C" mis_status mis_dac_encode(mis_dac* c, const float* audio, int batch, 
         HIP_CHECK(hipStreamSynchronize(s));                                // enc_codes is reused by the next quantizer
     }
     HIP_CHECK(hipGetLastError());
+}
+extern "C" mis_status mis_dac_encode(mis_dac* c, const float* audio, int batch, int64_t n_samples, int n_quantizers, int32_t* codes_out, float* z_out) {
+    MIS_API_BEGIN
+    MIS_REQUIRE(c && audio && codes_out && batch >= 1 && n_samples >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
+    MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "DAC model not finalized");
+    MIS_REQUIRE(c->has_encoder, MIS_ERR_AUDIO_ENCODE, "this DAC handle was loaded without encoder weights");
+    MIS_REQUIRE(n_quantizers >= 0 && n_quantizers <= c->cfg.n_codebooks, MIS_ERR_INVALID_INPUT, "n_quantizers out of range");
+    const int nq = n_quantizers ? n_quantizers : c->cfg.n_codebooks;
+    HIP_CHECK(hipSetDevice(c->device));
+    codec_run(c->pack, [&] { dac_encode(c, audio, batch, n_samples, nq, codes_out, z_out); });
     MIS_API_END
 }
 
@@ -439,12 +442,14 @@ extern "C" mis_status mis_dac_decode_codes(mis_dac* c, const int32_t* codes, int
     MIS_REQUIRE(c && codes && wav_out && batch >= 1 && T >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
     const int64_t n = mis_dac_num_samples(c, T);
-    c->codes_dev.alloc((size_t)batch * c->cfg.n_codebooks * T);
-    HIP_CHECK(hipMemcpyAsync(c->codes_dev.p, codes, (size_t)batch * c->cfg.n_codebooks * T * 4, hipMemcpyDefault, c->stream));
     DevBuf<float> wav;
-    wav.alloc((size_t)batch * n);
-    int C; int64_t Tt;
-    dac_run(c, c->codes_dev.p, batch, T, wav.p, n, 0, &C, &Tt);
+    codec_run(c->pack, [&] {
+        int C; int64_t Tt;
+        c->codes_dev.alloc((size_t)batch * c->cfg.n_codebooks * T);
+        HIP_CHECK(hipMemcpyAsync(c->codes_dev.p, codes, (size_t)batch * c->cfg.n_codebooks * T * 4, hipMemcpyDefault, c->stream));
+        wav.alloc((size_t)batch * n);
+        dac_run(c, c->codes_dev.p, batch, T, wav.p, n, 0, &C, &Tt);
+    });
     HIP_CHECK(hipMemcpyAsync(wav_out, wav.p, (size_t)batch * n * 4, hipMemcpyDefault, c->stream));
     HIP_CHECK(hipStreamSynchronize(c->stream));
     MIS_API_END
@@ -454,12 +459,15 @@ extern "C" mis_status mis_dac_debug_tap(mis_dac* c, const int32_t* codes, int ba
     MIS_API_BEGIN
     MIS_REQUIRE(c && codes && out && channels && length && block >= 0 && block < c->cfg.n_decoder_rates, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
-    c->codes_dev.alloc((size_t)batch * c->cfg.n_codebooks * T);
-    HIP_CHECK(hipMemcpyAsync(c->codes_dev.p, codes, (size_t)batch * c->cfg.n_codebooks * T * 4, hipMemcpyDefault, c->stream));
     DevBuf<float> wav;
-    wav.alloc((size_t)batch * mis_dac_num_samples(c, T));
     int C = 0; int64_t Tt = 0;
-    const float* res = dac_run(c, c->codes_dev.p, batch, T, wav.p, mis_dac_num_samples(c, T), 1 + block, &C, &Tt);
+    const float* res = nullptr;
+    codec_run(c->pack, [&] {
+        c->codes_dev.alloc((size_t)batch * c->cfg.n_codebooks * T);
+        HIP_CHECK(hipMemcpyAsync(c->codes_dev.p, codes, (size_t)batch * c->cfg.n_codebooks * T * 4, hipMemcpyDefault, c->stream));
+        wav.alloc((size_t)batch * mis_dac_num_samples(c, T));
+        res = dac_run(c, c->codes_dev.p, batch, T, wav.p, mis_dac_num_samples(c, T), 1 + block, &C, &Tt);
+    });
     MIS_REQUIRE((int64_t)batch * C * Tt <= capacity, MIS_ERR_INVALID_INPUT, "tap buffer too small");
     HIP_CHECK(hipMemcpyAsync(out, res, (size_t)batch * C * Tt * 4, hipMemcpyDefault, c->stream));
     HIP_CHECK(hipStreamSynchronize(c->stream));

@@ -16,6 +16,24 @@
 #include <sstream>
 #include <thread>
 
+static std::atomic<int64_t> g_device_held{0}, g_device_limit{INT64_MAX};
+hipError_t mis_device_malloc(void** p, size_t bytes) {
+    *p = nullptr;
+    if (g_device_held.fetch_add((int64_t)bytes) + (int64_t)bytes > g_device_limit.load()) { g_device_held -= (int64_t)bytes; return hipErrorOutOfMemory; }
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) { g_device_held -= (int64_t)bytes; *p = nullptr; }
+    return e;
+}
+void mis_device_free(void* p, size_t bytes) {
+    (void)hipFree(p);
+    g_device_held -= (int64_t)bytes;
+}
+extern "C" int64_t mis_debug_device_limit(int64_t more) {
+    const int64_t held = g_device_held.load();
+    g_device_limit = more < 0 ? INT64_MAX : held + more;
+    return held;
+}
+
 static thread_local std::string g_last_error;
 
 void mis_set_error(const char* fmt, ...) {

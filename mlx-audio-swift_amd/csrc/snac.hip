@@ -1242,12 +1242,7 @@ extern "C" int64_t mis_snac_padded_length(const mis_snac* c, int64_t n_samples) 
 
 // audio f32 [batch, n_samples] (host or device) -> codes_out[i] int32 [batch, T_i], T_i = padded / hop / vq_strides[i];
 // z_out (optional) f32 [batch, latent, padded / hop] = encoder output before quantisation (parity taps)
-extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_samples, int32_t* const* codes_out, float* z_out) {
-    MIS_API_BEGIN
-    MIS_REQUIRE(c && audio && codes_out && batch >= 1 && n_samples >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
-    MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "SNAC model not finalized");
-    MIS_REQUIRE(c->has_encoder, MIS_ERR_AUDIO_ENCODE, "this SNAC handle was loaded without encoder weights");
-    HIP_CHECK(hipSetDevice(c->device));
+static void snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_samples, int32_t* const* codes_out, float* z_out) {
     hipStream_t s = c->stream;
     CodecPackScope pack_scope(&c->pack, false);                           // three-plane contractions (f32 accuracy), none of two planes
     const mis_snac_config& cf = c->cfg;
@@ -1372,6 +1367,14 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
         for (auto& r : results) c->ring.out(r.to, r.from, r.bytes, s);
     }
     HIP_CHECK(hipGetLastError());
+}
+extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_samples, int32_t* const* codes_out, float* z_out) {
+    MIS_API_BEGIN
+    MIS_REQUIRE(c && audio && codes_out && batch >= 1 && n_samples >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
+    MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "SNAC model not finalized");
+    MIS_REQUIRE(c->has_encoder, MIS_ERR_AUDIO_ENCODE, "this SNAC handle was loaded without encoder weights");
+    HIP_CHECK(hipSetDevice(c->device));
+    codec_run(c->pack, [&] { snac_encode(c, audio, batch, n_samples, codes_out, z_out); });
     MIS_API_END
 }
 
@@ -1611,7 +1614,7 @@ void snac_decode_device(mis_snac* c, const int32_t* const* codes_dev, int batch,
     int C; int64_t T;
     NoiseRng rng;
     rng.enabled = rng_enabled; rng.seed = rng_seed; rng.row_ids = row_ids; rng.row_offset = row_offset;
-    snac_run(c, codes_dev, batch, t_coarse, noise_dev, rng, pcm_dev, pcm_stride, -1, &C, &T, s);
+    codec_run(c->pack, [&] { snac_run(c, codes_dev, batch, t_coarse, noise_dev, rng, pcm_dev, pcm_stride, -1, &C, &T, s); });
     HIP_CHECK(hipGetLastError());
 }
 
@@ -1660,13 +1663,15 @@ extern "C" mis_status mis_snac_decode(mis_snac* c, const int32_t* const* codes, 
     HIP_CHECK(hipSetDevice(c->device));
     std::vector<const int32_t*> dcodes;
     std::vector<const float*> dnoise;
-    snac_stage_inputs(c, codes, batch, t_coarse, noise, dcodes, dnoise);
-    int64_t N = mis_snac_num_samples(c, t_coarse);
-    c->pcm_ws.alloc((size_t)batch * N);
-    int C; int64_t T;
+    const int64_t N = mis_snac_num_samples(c, t_coarse);
     NoiseRng rng;
     rng.enabled = c->null_noise_zero ? 0 : 1; rng.seed = c->noise_seed;
-    snac_run(c, dcodes.data(), batch, t_coarse, dnoise.empty() ? nullptr : dnoise.data(), rng, c->pcm_ws.p, N, -1, &C, &T, c->stream);
+    codec_run(c->pack, [&] {
+        int C; int64_t T;
+        snac_stage_inputs(c, codes, batch, t_coarse, noise, dcodes, dnoise);
+        c->pcm_ws.alloc((size_t)batch * N);
+        snac_run(c, dcodes.data(), batch, t_coarse, dnoise.empty() ? nullptr : dnoise.data(), rng, c->pcm_ws.p, N, -1, &C, &T, c->stream);
+    });
     HIP_CHECK(hipGetLastError());
     c->ring.out(pcm_out, c->pcm_ws.p, (size_t)batch * N * sizeof(float), c->stream);
     c->last_batch = batch; c->last_t = t_coarse;
@@ -1698,8 +1703,10 @@ extern "C" mis_status mis_snac_debug_tap(mis_snac* c, const char* name, float* o
     int C; int64_t T;
     NoiseRng rng;
     rng.enabled = c->null_noise_zero ? 0 : 1; rng.seed = c->noise_seed;
-    const float* src = snac_run(c, c->last_codes.data(), c->last_batch, c->last_t,
-                                c->last_noise ? c->last_noise_ptrs.data() : nullptr, rng, nullptr, 0, stop, &C, &T, c->stream);
+    const float* src = nullptr;
+    codec_run(c->pack, [&] {
+        src = snac_run(c, c->last_codes.data(), c->last_batch, c->last_t, c->last_noise ? c->last_noise_ptrs.data() : nullptr, rng, nullptr, 0, stop, &C, &T, c->stream);
+    });
     HIP_CHECK(hipGetLastError());
     size_t n_el = (size_t)c->last_batch * C * T;
     MIS_REQUIRE((int64_t)n_el <= capacity, MIS_ERR_INVALID_INPUT, "tap buffer too small (%zu needed)", n_el);
