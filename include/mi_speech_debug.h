@@ -52,6 +52,11 @@ mis_status mis_debug_gelu_rcp_misses(int device, int64_t* misses);
 mis_status mis_debug_token_engine(mis_tts* lm, const int32_t* prompt, int n_prompt, int n_new, int xcds, const mis_gen_params* sampling,
                                   int stop_id, int32_t* next_tokens, float* logits_out, float* hidden_out, int32_t* counts, double* ms_out);
 
+/* tests: n residual 1x1 contractions one behind the other, y <- y + W_i snake(y) + b_i (alpha, ralpha: Snake's, [channels] each for all), as the codecs launch them.
+ * x, y_out f32 [batch][channels][columns], wt f32 [n][channels in][channels out], bias f32 [n][channels]; host memory */
+mis_status mis_debug_codec_chain(int device, int n, int channels, int batch, int columns, const float* x, const float* wt, const float* bias, const float* alpha, const float* ralpha,
+                                 float* y_out);
+
 /* rotary tables of the layer-list models: cos / sin f32 [positions][dims / 2] (host memory; no device involved).  yarn = 0: factor / original /
  * fast / slow unused */
 mis_status mis_debug_rotary_tables(int dims, double base, int yarn, double factor, double original, double fast, double slow, int positions,

@@ -802,3 +802,35 @@ void launch_gemm_chain(const CodecOp* ops, int n, int batch, hipStream_t s) {
         cur = nxt;
     }
 }
+
+extern "C" mis_status mis_debug_codec_chain(int device, int n, int channels, int batch, int columns, const float* x, const float* wt, const float* bias, const float* alpha, const float* ralpha,
+                                            float* y_out) {
+    MIS_API_BEGIN
+    MIS_REQUIRE(n >= 1 && channels >= 32 && channels % 32 == 0 && batch >= 1 && columns >= 1 && x && wt && bias && alpha && ralpha && y_out, MIS_ERR_INVALID_INPUT, "bad argument");
+    HIP_CHECK(hipSetDevice(device));
+    const size_t C = channels, elems = C * batch * columns;
+    CodecPack pack;
+    DevBuf<float> w, v[3], buf[2];                                   // matrices; biases, Snake's parameters; tensors in turns
+    w.alloc(n * C * C); v[0].alloc(n * C); v[1].alloc(C); v[2].alloc(C);
+    for (auto& b : buf) b.alloc(elems);
+    HIP_CHECK(copy_now(w.p, wt, n * C * C * 4, hipMemcpyHostToDevice));
+    HIP_CHECK(copy_now(v[0].p, bias, n * C * 4, hipMemcpyHostToDevice));
+    HIP_CHECK(copy_now(v[1].p, alpha, C * 4, hipMemcpyHostToDevice));
+    HIP_CHECK(copy_now(v[2].p, ralpha, C * 4, hipMemcpyHostToDevice));
+    HIP_CHECK(copy_now(buf[0].p, x, elems * 4, hipMemcpyHostToDevice));
+    std::vector<CodecOp> ops;
+    for (int i = 0; i < n; ++i) {
+        GemmParams g{};
+        g.AT = w.p + i * C * C; g.bias = v[0].p + i * C; g.alpha = v[1].p; g.ralpha = v[2].p;
+        g.X = g.R = buf[i & 1].p; g.Y = buf[(i + 1) & 1].p;
+        g.M = g.K = channels; g.N = g.Tin = g.Tout = columns;
+        ops.push_back({GEMM_RESID, true, true, g});
+    }
+    {
+        CodecPackScope scope(&pack);
+        launch_gemm_chain(ops.data(), n, batch, hipStreamPerThread);
+    }
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(copy_now(y_out, buf[n & 1].p, elems * 4, hipMemcpyDeviceToHost));
+    MIS_API_END
+}

@@ -228,8 +228,8 @@ bool codec_quarters(const GemmParams& p);
 __host__ __device__ inline int codec_quarter(int steps, int w) { return w >= 4 ? steps : steps * w / 16 * 4; }
 // three-plane split (codec_x6.hip): 1x1 and k-tap contractions of at least 48 rows and a multiple of 16 channels; false: not eligible, nothing launched
 bool launch_gemm_x6(int mode, bool snake, const GemmParams& p, int batch, hipStream_t s, const CodecPlanes* out = nullptr);
-// (out: whether that form writes it)
-bool codec_x6_writes_planes(int mode, const GemmParams& p);
+// (out: whether the forms of codec_x6.hip write it: two planes, of as many channels as they have rows)
+inline bool codec_x6_writes_planes(int mode, const GemmParams& p, const CodecPlanes& out) { return mode == GEMM_RESID && p.M % 32 == 0 && out.n == 2 && out.Cp == p.M; }
 // three-plane split: transposed convolution of stride 2, two taps per phase, 32 .. 64 rows, behind Snake; false: another shape
 // noise: with the NoiseBlock behind it (its X is p.Y, its Y unused)
 bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s, const GemmParams* noise = nullptr);

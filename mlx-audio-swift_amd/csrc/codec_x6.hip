@@ -388,6 +388,7 @@ static void launch_x6(const PwFusedParams& p, const uint16_t* wp, int batch, hip
 bool launch_pw_x6(int C, bool dw, const PwFusedParams& p, CodecPack* pack, int batch, hipStream_t s) {
     if (!pack) pack = codec_x6_scope();
     if (!pack || codec_exact_f32() || (dw && p.dil != 1 && p.dil != 3 && p.dil != 9) || !(dw ? C == 48 || C == 64 || C == 96 || C == 128 : (C == 96 || C == 128 || C == 192))) return false;
+    MIS_REQUIRE(!p.out || (!dw && p.out->n == 2 && p.out->Cp == C), MIS_ERR_GENERATION_FAILED, "codec unit: %d rows for %d planes of %d channels", C, p.out->n, p.out->Cp);
     const uint16_t* wp = pack->get_x6(p.AT, 1, C, C, s).wp;
     auto taps = [&](auto c) {
         constexpr int W = decltype(c)::value;
@@ -744,8 +745,6 @@ static void launch_x6_gemm(X6Gemm P, const uint16_t* wp, int batch, hipStream_t 
     else go(k_x6_gemm<1, SNAKE, TAPS, false, false, OUT>, 1);
 }
 
-bool codec_x6_writes_planes(int mode, const GemmParams& p) { return mode == GEMM_RESID && p.M % 32 == 0; }
-
 bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hipStream_t s, const CodecPlanes* out) {
     GemmParams p = p_in;
     CodecPack* pack = p.pack ? p.pack : codec_x6_scope();
@@ -757,6 +756,7 @@ bool launch_gemm_x6(int mode, bool snake, const GemmParams& p_in, int batch, hip
     // a NoiseBlock of 64 channels is bound by memory (32 x 196608 columns: 918 us here, 842 there; 48 channels with residual, 37776 columns: 23, 34).
     if (p.M < (mode == GEMM_NOISE ? 96 : 48) || Cin < 32 || Cin % 16 || (!taps && Cin > 384)) return false;
     if (mode != GEMM_RESID && mode != GEMM_TAPS) p.R = p.scale = nullptr;
+    MIS_REQUIRE(!out || codec_x6_writes_planes(mode, p, *out), MIS_ERR_GENERATION_FAILED, "codec contraction: %d rows for %d planes of %d channels", p.M, out->n, out->Cp);
     const CodecPack::X6& e = pack->get_x6(p.AT, ntaps, Cin, p.M, s);
     X6Gemm P{};
     P.g = p; P.mode = mode; P.ntaps = ntaps; P.nsteps = e.KS * ntaps; P.MT32 = e.MT32;

@@ -1429,9 +1429,9 @@ bool launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
         PwFusedParams fp{};
         fp.X = p.X; fp.R = p.R; fp.Y = p.Y; fp.a2 = p.alpha; fp.ra2 = p.ralpha; fp.AT = p.AT; fp.b2 = p.bias;
         fp.T = p.N; fp.dil = 0; fp.ldx = p.ldx; fp.ldr = p.ldy; fp.ldy = p.ldy;
-        fp.out = out;
-        if (out && !keep) fp.Y = nullptr;
-        if (launch_pw_x6(p.M, false, fp, p.pack, batch, s)) return out != nullptr;
+        fp.out = out && codec_x6_writes_planes(mode, p, *out) ? out : nullptr;
+        if (fp.out && !keep) fp.Y = nullptr;
+        if (launch_pw_x6(p.M, false, fp, p.pack, batch, s)) return fp.out != nullptr;
         fp.Y = p.Y;
         dim3 fg(cdiv(p.N, RU_NT), batch);
         if (p.M == 64) hipLaunchKernelGGL((k_pw_fused<64, false, 32>), fg, dim3(256), 0, s, fp);
@@ -1450,7 +1450,7 @@ bool launch_gemm(int mode, bool snake, const GemmParams& p_in, int batch, hipStr
                 "dense conv: %d taps with dilation %d exceed the staged halo", p.taps, p.dil);
     {
         GemmParams g = p;
-        const CodecPlanes* o = out && codec_x6_writes_planes(mode, p) ? out : nullptr;
+        const CodecPlanes* o = out && codec_x6_writes_planes(mode, p, *out) ? out : nullptr;
         if (o && !keep) g.Y = nullptr;
         if (launch_gemm_x6(mode, snake, g, batch, s, o)) return o != nullptr;
     }
