@@ -580,10 +580,10 @@ bool codec_exact_f32() { return bf3_env("MIS_CODEC_EXACT_F32", 0) != 0; }
 // What the two-plane contractions take.  What pays: MFMA-bound shapes.  A 1x1 conv over few channels is HBM-bound and the pre-pass would only add traffic
 // (measured per dispatch, profiles/r02_codec/: 1x1 over <= 512 channels and the last SNAC transposed conv, M*K = 16 K,
 // are faster on the exact-f32 kernels; every 7-tap conv and the transposed convs from M*K = 36 K up gain 2.3 - 4x)
-struct Bf3Shape { int ntaps, Cin, span, t_org, wtaps, phases, extra, parts; };
+struct Bf3Shape { int ntaps, Cin, span, t_org, wtaps, phases, extra, parts; bool three; };      // three: planes (the caller's)
 static bool bf3_shape(int mode, const GemmParams& p, Bf3Shape& h) {
     const bool one = mode == GEMM_PLAIN || mode == GEMM_GELU || mode == GEMM_RESID || mode == GEMM_NOISE;
-    h = Bf3Shape{1, p.K, 0, 0, 1, 1, 0, 1};
+    h = Bf3Shape{1, p.K, 0, 0, 1, 1, 0, 1, false};
     if (mode == GEMM_TAPS && p.taps == 2 && codec_quarters(p)) h.parts = 4;
     if (mode == GEMM_TAPS) { h.ntaps = p.taps; h.Cin = p.Cin; h.span = (p.taps - 1) * p.dil; h.t_org = -p.pad; h.wtaps = p.taps; }
     else if (mode == GEMM_CONVT) {
@@ -611,13 +611,14 @@ bool bf3_takes_convt(const GemmParams& p) {
 // us, 128 x 128 / 64 x 128 / 64 x 64: 768 rows, 7 taps of 768, 2080 columns: 102 / 60 / 79; 768 rows, K = 768: 51 / 24 / 26;
 // 1536 rows, 7 taps of 1024, 250 columns: 140 / 70 / 55; SNAC, one row of 12 groups: 48 / - / 19, 41 / 22 / 15, 33 / - / 14, 29 / 17 / 16.
 // A quarter of K a block (three planes, two taps of at least 512 channels): counted as the blocks they are, 64 x 64 up to 256 of 64 x 128 (us, 64 x 128 / 64 x 64: 384 rows,
-// K = 3072, 2361 columns, 456 blocks: 40 / 45; 768 rows, K = 6144, 296 columns, 144: 36 / 26; k_x6_gemm: 71, 44).
+// K = 3072, 2361 columns, 456 blocks: 40 / 45; 768 rows, K = 6144, 296 columns, 144: 36 / 26; k_x6_gemm: 71, 44), and always for rows of at most 64 columns (that one,
+// rows of 4 columns, 8: 67 / 41, 64: 371 / 268; of 24, 8: 68 / 42; k_x6_gemm: 43, 439, 43).
 struct Bf3Tile { bool few; int NI, nbx, nq, Tp; };
 static Bf3Tile bf3_tile(const GemmParams& p, const Bf3Shape& h, int batch) {
     const int nb128 = (p.N + 127) / 128;
     Bf3Tile t{};
     t.few = (int64_t)nb128 * ((p.M + B3_BM - 1) / B3_BM) * batch * h.phases * h.parts <= 128;
-    t.NI = t.few && (p.N <= 64 || (int64_t)nb128 * ((p.M + 63) / 64) * batch * h.phases * h.parts <= (h.parts > 1 ? 256 : 128)) ? 1 : 2;
+    t.NI = (h.three && h.parts > 1 && p.N <= 64) || (t.few && (p.N <= 64 || (int64_t)nb128 * ((p.M + 63) / 64) * batch * h.phases * h.parts <= (h.parts > 1 ? 256 : 128))) ? 1 : 2;
     t.nbx = (p.N + 64 * t.NI - 1) / (64 * t.NI);
     t.nq = 4 * t.NI + (h.span == 0 ? 0 : h.span <= 16 ? 1 : 4);
     t.Tp = (t.nbx - 1) * 64 * t.NI + t.nq * 16 + h.extra;
@@ -643,6 +644,7 @@ bool codec_planes_strided(const GemmParams& p, int batch, CodecPlanes& out) {
     CodecPack* pack = codec_x6_scope();
     Bf3Shape h;
     if (!pack || codec_exact_f32() || p.taps != 2 || p.dil != 1 || p.pad != 0 || p.Cin % 32 || p.M < 48 || !bf3_shape(GEMM_TAPS, p, h)) return false;
+    h.three = true;
     const Bf3Tile t = bf3_tile(p, h, batch);
     out = CodecPlanes{};
     out.n = 3; out.Cp = h.Cin; out.Tp = t.Tp;
@@ -685,13 +687,14 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
         MIS_REQUIRE(bf3_writes_planes(mode, p) && out->Cp == p.M && !(in && in->n == 3 && h.ntaps == 2), MIS_ERR_GENERATION_FAILED, "codec contraction: %d rows for an operand of %d channels", p.M, out->Cp);
     }
     const int ntaps = h.ntaps, Cin = h.Cin, span = h.span;
+    const bool three = h.three = in && in->n == 3;
     const Bf3Tile t = bf3_tile(p, h, batch);
     const bool few = t.few;
     const int NI = t.NI, nb128 = (p.N + 127) / 128;
     Bf3Params P{};
     P.g = p; P.g.Cin = Cin;
     P.mode = mode; P.ntaps = ntaps; P.Tp = t.Tp; P.t_org = h.t_org;
-    if (in && in->n == 3) {
+    if (three) {
         const CodecPack::X6& e = p.pack->get_x6(p.AT, h.wtaps, Cin, p.M, s);
         P.wp = e.wp; P.MT32 = e.MT32;
         P.wmt = 1536; P.wtap = (size_t)e.MT32 * 1536; P.wks = h.wtaps * P.wtap;
@@ -721,9 +724,9 @@ bool launch_gemm_bf3(int mode, bool snake, const GemmParams& p_in, int batch, hi
         if (per_row <= 32 && nchunks >= 32) ksplit = 4;
         else if (per_row <= 64 && nchunks >= 16) ksplit = 2;
     }
-    // Three planes, K >= 1024: four partial sums in every form (codec_quarters), in blocks of their own while that is what fills the chip
-    const bool three = in && in->n == 3, quarters = three && ntaps == 2 && codec_quarters(p);
-    if (quarters && (int64_t)t.nbx * ((p.M + 63) / 64) * batch < 512) ksplit = 4;
+    // Three planes, K >= 1024: four partial sums in every form (codec_quarters), in blocks of their own while that is what fills the chip (tiles of 64 columns: always)
+    const bool quarters = three && ntaps == 2 && codec_quarters(p);
+    if (quarters && (NI == 1 || (int64_t)t.nbx * ((p.M + 63) / 64) * batch < 512)) ksplit = 4;
     if (ksplit > 1) {
         p.pack->part.alloc((size_t)ksplit * batch * p.M * p.ldy);
         P.ksplit = ksplit; P.part = p.pack->part.p; P.batch = batch;

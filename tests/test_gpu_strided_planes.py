@@ -12,8 +12,8 @@ pytestmark = pytest.mark.gpu
 CFG = dict(encoder_dim=48, encoder_rates=[2, 4, 8, 8], decoder_dim=64, decoder_rates=[8, 8, 4, 2], codebook_size=64, codebook_dim=8, vq_strides=[4, 2, 1])
 
 
-# one frame of codes (a column behind the last stride); a row whose K = 3072 has 456 blocks of 64 x 128; a call in which a tile takes its quarters itself
-@pytest.mark.parametrize("rows, samples", [(1, 2048), (1, 60001), (1, 151111), (48, 24000)])
+# one frame of codes (a column behind the last stride) alone, in eight rows and, twelve columns, in 48; a row whose K = 3072 has 456 blocks of 64 x 128; a call in which a tile takes its quarters itself
+@pytest.mark.parametrize("rows, samples", [(1, 2048), (8, 2048), (48, 6000), (1, 60001), (1, 151111), (48, 24000)])
 def test_strided_convolutions(rows, samples):
     W = osnac.make_synthetic_weights(osnac.SnacConfig(**CFG), seed=21, with_encoder=True)
     dev = mas.SNAC.from_weights(mas.SNACConfig(**CFG), W)
