@@ -1012,8 +1012,9 @@ __global__ void __launch_bounds__(256) k_attn_prefill(const bf16_t* __restrict__
 // tiling) are staged ONCE per block through LDS, one 16-byte piece per thread, tile t + 1 requested before tile t is multiplied (two LDS buffers, one
 // barrier per tile); a wave reads each fragment once (lane-linear ds_read_b128, conflict-free) and uses it for both of its row groups: 24 MFMAs per 8 LDS
 // reads.  The key mask is applied on the last tile only.  Same operations per query row in the same order as k_attn_prefill: results are bit-identical
-// (tests/test_gpu_whisper.py).  Bound: the softmax's VALU work, not the matrix core: 228 us per layer of 8 windows x 20 heads (260 us with the score's scale,
-// its logarithm base and a cross-lane maximum per tile in the loop; two tiles per barrier: 251).
+// (tests/test_gpu_whisper.py).  Bound: the softmax's VALU work (issued in 71 % of the cycles; MFMA 41 %): 149 - 158 us per layer of 8 windows x 20 heads.  228 with the
+// maximum taken over the raw scores, the row groups one after the other and the mask inside the loop; 260 with the score's scale, its logarithm base and a cross-lane maximum per
+// tile there as well; that form with two tiles per barrier 251.
 template <int D>
 __global__ void __launch_bounds__(512, 4) k_attn_prefill2(const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kc,
                                                           const bf16_t* __restrict__ vc, bf16_t* __restrict__ out, int ldo,
