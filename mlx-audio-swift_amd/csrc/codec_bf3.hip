@@ -52,7 +52,6 @@ struct Bf3Params {
     int nbx, my, inner, per, tiles;       // column tiles, row tiles, phases or K slices of a tile, tiles per XCD, all tiles
 };
 
-__device__ __forceinline__ float bf3_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
 
 // ---- weights: A^T [ntaps][Cin][M] f32 -> fragments --------------------------------------------------------------------------------
 __global__ void k_bf3_pack_w(const float* __restrict__ AT, uint16_t* __restrict__ wp, int ntaps, int Cin, int M, int MT32, int KS) {
@@ -108,7 +107,7 @@ __global__ void __launch_bounds__(256) k_bf3_split(const float* __restrict__ X, 
             for (int i = 0; i < 2; ++i) {
                 const int c = c0 + cc + j + i;
                 x[i] = v[o][j + i];
-                if (alpha) x[i] = bf3_snake(x[i], alpha[min(c, C - 1)], ralpha[min(c, C - 1)]);
+                if (alpha) x[i] = mis_snake(x[i], alpha[min(c, C - 1)], ralpha[min(c, C - 1)]);
                 x[i] = tin && c < C ? x[i] : 0.0f;
             }
             h[j / 2] = (uint32_t)f32_to_bf16(x[0]) | ((uint32_t)f32_to_bf16(x[1]) << 16);
@@ -458,7 +457,7 @@ __device__ __forceinline__ void bf3_body(const Bf3Params& P, const float* __rest
                         }
                         if (poa) {
 #pragma unroll
-                            for (int r = 0; r < 8; ++r) y[r] = bf3_snake(y[r], al[r], ra[r]);
+                            for (int r = 0; r < 8; ++r) y[r] = mis_snake(y[r], al[r], ra[r]);
                         }
                         if (P.out.n == 3) codec_tile_put<3>(y, st + ni * CP_LDS(3), r0, lane);
                         else codec_tile_put<2>(y, st + ni * CP_LDS(3), r0, lane);
@@ -818,7 +817,9 @@ extern "C" mis_status mis_debug_codec_chain(int device, int n, int channels, int
     for (auto& b : buf) b.alloc(elems);
     HIP_CHECK(copy_now(w.p, wt, n * C * C * 4, hipMemcpyHostToDevice));
     HIP_CHECK(copy_now(v[0].p, bias, n * C * 4, hipMemcpyHostToDevice));
-    HIP_CHECK(copy_now(v[1].p, alpha, C * 4, hipMemcpyHostToDevice));
+    std::vector<float> ap(channels);
+    for (int i = 0; i < channels; ++i) ap[i] = snake_alpha(alpha[i]);
+    HIP_CHECK(copy_now(v[1].p, ap.data(), C * 4, hipMemcpyHostToDevice));
     HIP_CHECK(copy_now(v[2].p, ralpha, C * 4, hipMemcpyHostToDevice));
     HIP_CHECK(copy_now(buf[0].p, x, elems * 4, hipMemcpyHostToDevice));
     std::vector<CodecOp> ops;

@@ -22,7 +22,6 @@
 #include <algorithm>
 #include <type_traits>
 
-__device__ __forceinline__ float f32_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
 
 struct F32Tiles { int nt, mt, npx, taps; };      // column tiles, row tiles, column tiles per XCD
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));       // four columns of a row at any column: global loads need 4-byte alignment only
@@ -119,7 +118,7 @@ __device__ __forceinline__ void codec_gemm_tile(const GemmParams& p, int T, int 
             if constexpr (SNAKE) {
                 const int ch = min(c16 + (rr & 15), Cin - 1);
                 const float a = p.alpha[ch], al = p.ralpha[ch];
-                v = make_float4(f32_snake(v.x, a, al), f32_snake(v.y, a, al), f32_snake(v.z, a, al), f32_snake(v.w, a, al));      // snake(0) = 0 keeps the zero pad
+                v = make_float4(mis_snake(v.x, a, al), mis_snake(v.y, a, al), mis_snake(v.z, a, al), mis_snake(v.w, a, al));      // snake(0) = 0 keeps the zero pad
             }
             *reinterpret_cast<float4*>(Xs + buf * (BK * LX) + rr * LX + nl) = v;
         }

@@ -5,23 +5,23 @@
 
 enum { GEMM_PLAIN = 0, GEMM_RESID = 1, GEMM_NOISE = 2, GEMM_CONVT = 3, GEMM_GELU = 4, GEMM_TAPS = 5 };
 
-// Y[b][m][n] = sum_k A[m][k] X[b][k][n] on v_mfma_f32_32x32x2_f32 (activations NCT, time contiguous)
-// sin^2(y) for the Snake activations of the streaming-rate kernels: y is reduced by multiples of pi (two-term Cody-Waite, exact for
-// |y| < 1e5) to |r| <= pi/2, sin r by the degree-11 odd polynomial (truncation 5.7e-8 at the interval end), and the sign drops out
-// in the square.  12 VALU instructions instead of the ~30 of the full-range sinf: the split pre-pass and the final conv were bound by
-// that (33 instructions per element measured from their element rate); absolute error <= 3.3e-7 for |y| <= 274 (CPU sweep).
-__device__ __forceinline__ float mis_sin_sq(float y) {
-    const float n = rintf(y * 0.318309886183790672f);
-    float r = fmaf(n, -3.140625f, y);
-    r = fmaf(n, -9.67653589793e-4f, r);
-    const float s = r * r;
-    float p = fmaf(s, -2.50521084e-8f, 2.75573192e-6f);
-    p = fmaf(s, p, -1.98412698e-4f);
-    p = fmaf(s, p, 8.33333333e-3f);
-    p = fmaf(s, p, -1.66666667e-1f);
-    p = fmaf(r * s, p, r);
-    return p * p;
+// Snake, x + sin^2(alpha x) ra, with the factor as `a` = alpha / pi (snake_alpha below, rounded once when the weights are laid out): t = a x is reduced to the
+// nearest whole number, exactly, and sin^2(pi f), |f| <= 1/2, is f^2 times a polynomial of degree five in f^2 (least maximum, found by reweighted least squares;
+// 5.9e-9 before rounding).  Eleven VALU instructions: the product alpha x reduced by multiples of pi and the square of a polynomial for the sine were fourteen, in
+// kernels that issue VALU in 60 - 90 % of their cycles.  Off 64 bits by 4.6e-8 (rms) where |alpha x| is about one, 1.1e-7 at three, 3.6e-7 at ten, rounding of
+// t; the form before: 5.1e-8, 1.1e-7, 3.2e-7.
+__device__ __forceinline__ float mis_snake(float x, float a, float ra) {
+    const float t = a * x;
+    const float f = t - rintf(t);
+    const float s = f * f;
+    float p = fmaf(s, -3.27294594e+0f, 1.29907303e+1f);
+    p = fmaf(s, p, -3.00859532e+1f);
+    p = fmaf(s, p, 4.27253848e+1f);
+    p = fmaf(s, p, -3.24695811e+1f);
+    p = fmaf(s, p, 9.86960292e+0f);
+    return fmaf(ra, p * s, x);
 }
+inline float snake_alpha(float alpha) { return (float)((double)alpha * 0.31830988618379067154); }
 
 // z[c][t] = sum over q in order of tables[q][code(q, t)][c]: a block takes 32 channels x 32 frames (table rows are read along c, z written along t); four
 // quantisers' codes, then their table rows are requested together (one by one they were two dependent round trips per quantiser and frame: SNAC
@@ -202,7 +202,7 @@ struct GemmParams {
     uint64_t noise_key;   // (seed, block) key of the generator
     const int32_t* row_ids;   // optional global row id per batch row (rng keyed by GLOBAL row)
     int64_t row_offset;
-    const float* alpha;   // Snake prologue on X rows (null = none)
+    const float* alpha;   // Snake prologue on X rows (null = none): alpha / pi (snake_alpha), here and wherever a kernel takes a Snake
     const float* ralpha;
     int M, K, N;          // N = output columns per phase
     int Tin, Tout;

@@ -20,7 +20,6 @@
 #include <type_traits>
 #include <utility>
 
-__device__ __forceinline__ float x6_snake(float x, float a, float ra) { return fmaf(ra, mis_sin_sq(a * x), x); }
 
 #define X6_MAX 3.38953138925153547590470800371487866880e+38f      // the largest bfloat16
 // x = h + m + l exactly (three bfloat16, each the nearest to what is left): eight values of consecutive channels -> one 16-byte piece per plane.
@@ -177,7 +176,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll
                 for (int sx = 0; sx < NS; ++sx) {
                     const int j = sx * 64 + lane;
-                    xs[cc][HALO + j] = x6_snake(n0 + j < T ? vx[r][sx] : 0.0f, al, ral);
+                    xs[cc][HALO + j] = mis_snake(n0 + j < T ? vx[r][sx] : 0.0f, al, ral);
                 }
                 __builtin_amdgcn_sched_barrier(0);                          // (a row at a time: the values in flight take the registers)
             }
@@ -192,7 +191,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                     al = pa1[c]; ral = pra1[c];
                     if constexpr (HR == 2) { const float a1 = pa1[c + 4], ra1 = pra1[c + 4]; if (r & 1) { al = a1; ral = ra1; } }
                 }
-                const float u = x6_snake(t >= 0 && t < T ? vh[h] : 0.0f, al, ral);
+                const float u = mis_snake(t >= 0 && t < T ? vh[h] : 0.0f, al, ral);
                 if (on) xs[wave + 4 * r][j] = u;
             }
         } else {
@@ -201,7 +200,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                 const int kg = KC == 32 ? wave : wave >> 1, n = (KC == 32 ? g : wave & 1) * 64 + lane;
                 float v[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = x6_snake(vx[g][j], pa2[c0 + kg * 8 + j], pra2[c0 + kg * 8 + j]);
+                for (int j = 0; j < 8; ++j) v[j] = mis_snake(vx[g][j], pa2[c0 + kg * 8 + j], pra2[c0 + kg * 8 + j]);
                 uint4 h, m, l;
                 x6_split<false>(v, h, m, l);
                 ts[0][kg][n] = h; ts[1][kg][n] = m; ts[2][kg][n] = l;
@@ -227,7 +226,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                     float a = 0.0f;
 #pragma unroll
                     for (int k = 0; k < 7; ++k) a += pw7[c * 7 + k] * xs[cc][n + k * DIL];
-                    v[j] = x6_snake(a + pb1[c], pa2[c], pra2[c]);
+                    v[j] = mis_snake(a + pb1[c], pa2[c], pra2[c]);
                     if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
                 }
                 uint4 h, m, l;
@@ -292,7 +291,7 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
                 }
                 if (poa) {
 #pragma unroll
-                    for (int r = 0; r < 8; ++r) { const int m = m0 + (r & 3) + 8 * (r >> 2); y[r] = x6_snake(y[r], poa[m], pora[m]); }
+                    for (int r = 0; r < 8; ++r) { const int m = m0 + (r & 3) + 8 * (r >> 2); y[r] = mis_snake(y[r], poa[m], pora[m]); }
                 }
                 codec_tile_put<2>(y, st, r0, lane);
             }
@@ -326,9 +325,9 @@ __device__ __forceinline__ void pw_x6_body(const float* __restrict__ pX, const f
 #pragma unroll 1
                             for (int k = 0; k < 7; ++k) {
                                 const int t = n + (k - 3) * DIL;
-                                a = fmaf(pw7[c * 7 + k], x6_snake(t >= 0 && t < T ? xb[(size_t)c * p.ldx + t] : 0.0f, pa1[c], pra1[c]), a);
+                                a = fmaf(pw7[c * 7 + k], mis_snake(t >= 0 && t < T ? xb[(size_t)c * p.ldx + t] : 0.0f, pa1[c], pra1[c]), a);
                             }
-                            v = fmaf(pAT[(size_t)c * C + m], x6_snake(a + pb1[c], pa2[c], pra2[c]), v);
+                            v = fmaf(pAT[(size_t)c * C + m], mis_snake(a + pb1[c], pa2[c], pra2[c]), v);
                         }
                         yb[(size_t)m * p.ldy + n] = rb[(size_t)m * p.ldr + n] + (v + pb2[m]);
                     }
@@ -526,7 +525,7 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             x[j] = v[slot][j];
-            if constexpr (SNAKE) x[j] = x6_snake(x[j], x6_ab[kc + j], x6_ab[Kx + kc + j]);
+            if constexpr (SNAKE) x[j] = mis_snake(x[j], x6_ab[kc + j], x6_ab[Kx + kc + j]);
             if constexpr (TAPS) x[j] = ok[slot] ? x[j] : 0.0f;
         }
         uint4 h, m, l;
@@ -666,7 +665,7 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
                     const int c = i / (16 * T) * 16 + (i & 15), j = i / 16 % T, t = TAPS ? n - p.pad + j * p.dil : n;
                     if (TAPS && (t < p.x_lo || t >= p.Tin)) continue;
                     float x = pX[((size_t)b * Kx + c) * p.ldx + t];
-                    if constexpr (SNAKE) x = x6_snake(x, x6_ab[c], x6_ab[Kx + c]);
+                    if constexpr (SNAKE) x = mis_snake(x, x6_ab[c], x6_ab[Kx + c]);
                     v = fmaf(pAT[((size_t)j * Kx + c) * p.M + m], x, v);
                     if (v != v) break;                                      // (NaN it stays)
                 }
@@ -688,7 +687,7 @@ __device__ __forceinline__ void x6_gemm_body(const X6Gemm& P, const float* __res
                 for (int r = 0; r < 8; ++r) {
                     const int m = m0 + 2 * r0 + (r & 3) + 8 * (r >> 2);
                     o[r] = acc[mi][r0 + r];
-                    if (poa) o[r] = x6_snake(o[r], poa[m], pora[m]);
+                    if (poa) o[r] = mis_snake(o[r], poa[m], pora[m]);
                 }
                 codec_tile_put<2>(o, st, r0, lane);
             }
@@ -813,7 +812,7 @@ __device__ __forceinline__ void x6_convt_body(const GemmParams& p, const X6Noise
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int c = c0 + kg * 8 + j;
-            x[j] = ok ? x6_snake(v[j], pa[c], pra[c]) : 0.0f;               // (the padding is zero behind Snake as well)
+            x[j] = ok ? mis_snake(v[j], pa[c], pra[c]) : 0.0f;               // (the padding is zero behind Snake as well)
         }
         uint4 h, m, l;
         x6_split<true>(x, h, m, l);

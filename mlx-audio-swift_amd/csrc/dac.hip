@@ -156,9 +156,9 @@ extern "C" mis_status mis_dac_finalize(mis_dac* c) {
     };
     auto snake = [&](const std::string& p, int64_t C, size_t& a, size_t& ra) {
         const auto& al = dneed(c, p, {1, 1, C});
-        std::vector<float> rv(C);
-        for (int64_t i = 0; i < C; ++i) rv[i] = 1.0f / (al[i] + 1e-9f);
-        a = push(al); ra = push(rv);
+        std::vector<float> av(C), rv(C);
+        for (int64_t i = 0; i < C; ++i) { av[i] = snake_alpha(al[i]); rv[i] = 1.0f / (al[i] + 1e-9f); }
+        a = push(av); ra = push(rv);
     };
     {   // fromCodes: sum_i outProj_i(codebook_i[code]) -> tables [n_cb][bins][D] (bias included once per codebook)
         std::vector<float> tables((size_t)cf.n_codebooks * bins * D);

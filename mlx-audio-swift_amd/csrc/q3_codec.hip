@@ -257,7 +257,7 @@ __global__ void __launch_bounds__(256) k_q3_final(const float* __restrict__ x, f
             float v = 0.0f;
             if (c < C && t >= x_lo && t < T) {
                 v = x[((int64_t)b * C + c) * ld + t];
-                v = fmaf(ra[c], mis_sin_sq(a[c] * v), v);
+                v = mis_snake(v, a[c], ra[c]);
             }
             sx[cc][j] = v;
         }
@@ -363,7 +363,7 @@ mis_status mis_q3dec_finalize(mis_q3dec* d) {
     auto snake_pair = [&](const std::string& pa, const std::string& pb, int64_t C, size_t& a, size_t& ra) {
         const auto& al = need(d, pa, {C}); const auto& be = need(d, pb, {C});
         std::vector<float> av(C), rv(C);
-        for (int64_t i = 0; i < C; ++i) { av[i] = expf(al[i]); rv[i] = 1.0f / (expf(be[i]) + 1e-9f); }   // SnakeBeta :236-254
+        for (int64_t i = 0; i < C; ++i) { av[i] = snake_alpha(expf(al[i])); rv[i] = 1.0f / (expf(be[i]) + 1e-9f); }   // SnakeBeta :236-254
         a = push(av); ra = push(rv);
     };
     d->zeros = push(std::vector<float>((size_t)std::max<int64_t>({ld, dd, Cd, 4}), 0.0f));

@@ -21,10 +21,6 @@
 
 // ============================================================================ device kernels
 
-__device__ __forceinline__ float snake_f(float x, float a, float ra) {
-    return fmaf(ra, mis_sin_sq(a * x), x);      // Layers.swift:44-50: x + 1/(alpha+1e-9) * sin(alpha x)^2 (mis_sin_sq: codec_kernels.h)
-}
-
 // ---- fromCodes ---------------------------------------------------------------------------------
 struct EmbedParams {
     const float* tables;        // [n_q][codebook_size][C]
@@ -73,7 +69,7 @@ __global__ void __launch_bounds__(256) k_snac_dw(const float* __restrict__ X, fl
     for (int h = 0; h < NL; ++h) {
         const int i = tid + h * 256, t = t0 - halo + i;
         float u = t >= 0 && t < T ? v[h] : 0.0f;               // zero padding AFTER snake == snake(0) = 0
-        if (SNAKE_IN) u = snake_f(u, ai, rai);
+        if (SNAKE_IN) u = mis_snake(u, ai, rai);
         if (i < DW_TILE + 2 * DW_HALO) s[i] = u;
     }
     __syncthreads();
@@ -90,7 +86,7 @@ __global__ void __launch_bounds__(256) k_snac_dw(const float* __restrict__ X, fl
 #pragma unroll
         for (int k = 0; k < 7; ++k) acc += wk[k] * s[i + k * dil];
         acc += bv;
-        if (SNAKE_OUT) acc = snake_f(acc, ao, rao);
+        if (SNAKE_OUT) acc = mis_snake(acc, ao, rao);
         if (t < T) y[t] = acc;
     }
 }
@@ -229,7 +225,7 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
 #pragma unroll
                 for (int sx = 0; sx < 3; ++sx) {
                     const int j = sx * 64 + lane;
-                    if (j < RU_XS) xs[cc][j] = snake_f(v[r][sx], al, ral);
+                    if (j < RU_XS) xs[cc][j] = mis_snake(v[r][sx], al, ral);
                 }
             }
         } else {
@@ -249,7 +245,7 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
                 const int cc = wave + 4 * r, c = c0 + cc;
                 const float al = p.a2[c], ral = p.ra2[c];
 #pragma unroll
-                for (int hx = 0; hx < 2; ++hx) ts[cc][hx * 64 + lane] = snake_f(v[r][hx], al, ral);
+                for (int hx = 0; hx < 2; ++hx) ts[cc][hx * 64 + lane] = mis_snake(v[r][hx], al, ral);
             }
         }
         for (int i = tid; i < KC * (C / 4); i += 256) { // rows c0 .. c0+31 of W2^T
@@ -274,7 +270,7 @@ __device__ __forceinline__ void pw_fused_body(const float* __restrict__ pX, cons
 #pragma unroll
                     for (int k = 0; k < 7; ++k) a += wk[k] * xs[cc][n + k * p.dil];
                     a += bv;
-                    ts[cc][n] = snake_f(a, ao, rao);
+                    ts[cc][n] = mis_snake(a, ao, rao);
                 }
             }
         }
@@ -367,7 +363,7 @@ __device__ __forceinline__ void snac_convt_body(const GemmParams& p, const float
             if (kin) {
                 float a = p.alpha[row], r = p.ralpha[row];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) rx[h][e] = snake_f(rx[h][e], a, r);   // snake(0)=0 keeps the zero pad
+                for (int e = 0; e < 4; ++e) rx[h][e] = mis_snake(rx[h][e], a, r);   // snake(0)=0 keeps the zero pad
             }
         }
     };
@@ -446,7 +442,7 @@ __global__ void k_enc_phase_split(const float* __restrict__ x, float* __restrict
     for (int r = 0; r < s; ++r) {
         const int t = m * s + r - pad;
         const float v = row[min(max(t, 0), T - 1)];
-        o[(size_t)r * Tm] = t >= 0 && t < T ? snake_f(v, al, ral) : 0.0f;
+        o[(size_t)r * Tm] = t >= 0 && t < T ? mis_snake(v, al, ral) : 0.0f;
     }
 }
 // The same as three planes, [m][c*s + r] (codec_kernels.h, CodecPlanes): a block makes 64 columns of 64 phases, a thread eight phases of a column at a time; through LDS, so that
@@ -480,7 +476,7 @@ __global__ void __launch_bounds__(256) k_enc_phase_planes(const float* __restric
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int t = m * s + r - pad;
-            v[h][j] = snake_f(t >= 0 && t < T ? v[h][j] : 0.0f, al[h][j], ral[h][j]);      // (Snake of 0 is 0)
+            v[h][j] = mis_snake(t >= 0 && t < T ? v[h][j] : 0.0f, al[h][j], ral[h][j]);      // (Snake of 0 is 0)
             if (++r == s) r = 0;
         }
 #pragma unroll
@@ -746,7 +742,7 @@ __device__ __forceinline__ void conv_taps_body(const GemmParams& p, const float*
                 if (p.alpha) {
                     const float al = p.alpha[c0 + row], ra_ = p.ralpha[c0 + row];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = snake_f(v[e], al, ra_);      // snake(0) = 0 keeps the zero padding
+                    for (int e = 0; e < 4; ++e) v[e] = mis_snake(v[e], al, ra_);      // snake(0) = 0 keeps the zero padding
                 }
             }
             rx[i] = make_float4(v[0], v[1], v[2], v[3]);
@@ -835,7 +831,7 @@ __global__ void __launch_bounds__(256) k_codec_final(const float* __restrict__ X
             const int c = min(c0 + 4 * i, C - 1);
             const float a = alpha[c], ra = ralpha[c];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) s[wave][i][h * 64 + lane] = ok[h] ? snake_f(v[i][h], a, ra) : 0.0f;
+            for (int h = 0; h < 2; ++h) s[wave][i][h * 64 + lane] = ok[h] ? mis_snake(v[i][h], a, ra) : 0.0f;
         }
         if (c0 + 4 * FIN_CH < C) load(c0 + 4 * FIN_CH);
         wave_lds_fence();
@@ -1029,10 +1025,10 @@ extern "C" mis_status mis_snac_finalize(mis_snac* c) {
     auto push = [&](const std::vector<float>& v) { size_t o = arena.size(); arena.insert(arena.end(), v.begin(), v.end()); while (arena.size() & 3) arena.push_back(0.f); return o; };
     auto push_snake = [&](const std::string& name, int64_t C) {
         const HostTensor& a = need(c, name, {1, C, 1});
-        std::vector<float> ra(C);
-        for (int64_t i = 0; i < C; ++i) ra[i] = 1.0f / (a.v[i] + 1e-9f);
+        std::vector<float> av(C), ra(C);                                   // Layers.swift:44-50: x + 1 / (alpha + 1e-9) sin(alpha x)^2
+        for (int64_t i = 0; i < C; ++i) { av[i] = snake_alpha(a.v[i]); ra[i] = 1.0f / (a.v[i] + 1e-9f); }
         SnakeW s;
-        s.a = push(a.v);
+        s.a = push(av);
         s.ra = push(ra);
         return s;
     };
