@@ -12,6 +12,7 @@
 #include "kernels.h"
 #include "lm_kernels.h"
 #include "lm_blocks.h"
+#include "lm_step.h"
 
 #include <math.h>
 #include <string.h>
@@ -79,6 +80,10 @@ struct mis_tts {
     DevBuf<int32_t> pf_pos;
     DevBuf<uint8_t> pf_on;
     DevBuf<SamplerScratch> samp_scratch;
+    DevBuf<unsigned char> step_exch;             // decode steps in one launch (lm_step.hip): values handed between blocks, flags
+    DevBuf<unsigned> step_sync;
+    unsigned* step_lock = nullptr;               // the device's, not this handle's
+    bool step_off = false;                       // a launch has timed out: this handle stays on the launch chain
     HostRing ring;
     hipGraphExec_t g_prefill = nullptr, g_decode = nullptr;
     bool shared_device = false;      // another replica's streams run on this device (group.hip): never a kernel that waits for co-resident blocks
@@ -726,6 +731,23 @@ static bool fold_gate_up(const mis_tts* c) {
 static bool fold_qkv(const mis_tts* c) {
     return fold_on() && !c->blocks && !c->q_qkv.on && gemm_glue_ok(EPI_PARTIAL, c->batch, c->a_qkv.R, c->a_qkv.ksb, c->a_qkv.U, c->S_down, c->d, c->Mpad);
 }
+static AttnParams decode_attention(const mis_tts* c, int li) {
+    const size_t lkv = (size_t)c->batch * c->Hkv * c->Smax * c->D;
+    AttnParams ap{};
+    ap.qkv_part = c->qkv_part.p; ap.S = c->S_qkv; ap.Mpad = c->Mpad; ap.Nqkv = c->Nqkv;
+    ap.kcache = c->kcache.p + lkv * li; ap.vtcache = c->vtcache.p + lkv * li;
+    ap.pos = c->pos_cur.p; ap.active = c->active.p;
+    ap.rope_cos = c->rope_cos.p; ap.rope_sin = c->rope_sin.p;
+    ap.out = c->attn_out.p; ap.H = c->H; ap.Hkv = c->Hkv; ap.D = c->D; ap.Smax = c->Smax;
+    ap.scale = 1.0f / sqrtf((float)c->D);
+    if (c->cfg.qk_norm) {
+        ap.qnorm_w = c->qknorm.p + (size_t)(2 * li) * c->D;
+        ap.knorm_w = c->qknorm.p + (size_t)(2 * li + 1) * c->D;
+        ap.qk_eps = c->cfg.rms_norm_eps;
+    }
+    ap.rope_in_dtype = c->cfg.rope_ops_in_dtype;
+    return ap;
+}
 // embed -> L x block.  Leaves x = final-norm(h) ready for lm_head.   (LlamaTTS.swift:335-345,303-310)
 // table/rows/ids: embedding source override (composite engines feed input embeddings as a [rows][d] table)
 static void enqueue_layers(mis_tts* c, const bf16_t* table = nullptr, int table_rows = 0, const int32_t* ids = nullptr) {
@@ -740,26 +762,12 @@ static void enqueue_layers(mis_tts* c, const bf16_t* table = nullptr, int table_
     launch_embed_rmsnorm(table ? table : c->emb.p, ids ? ids : c->ids.p, c->active.p, c->pos_cur.p, c->pos_next.p, c->norms.p,
                          hcur, c->x.p, d, table ? table_rows : c->V, eps, c->batch, Mpad, s);
     for (int li = 0; li < c->L; ++li) {
-        const size_t lkv = (size_t)c->batch * c->Hkv * c->Smax * c->D;
         if (f_qkv && li > 0) {
             launch_gemm_glue(EPI_PARTIAL, c->batch, c->wqkv.p + layer_qkv_elems(c) * li, c->part.p, c->S_down, hcur, hoth, c->norms.p + (size_t)(2 * li) * d, eps, c->qkv_part.p,
                              c->Nqkv / 16, d / 32, c->S_qkv, c->Nqkv, Mpad, s);
             std::swap(hcur, hoth);
         } else gemm_qkv(c, li, s);
-        AttnParams ap{};
-        ap.qkv_part = c->qkv_part.p; ap.S = c->S_qkv; ap.Mpad = Mpad; ap.Nqkv = c->Nqkv;
-        ap.kcache = c->kcache.p + lkv * li; ap.vtcache = c->vtcache.p + lkv * li;
-        ap.pos = c->pos_cur.p; ap.active = c->active.p;
-        ap.rope_cos = c->rope_cos.p; ap.rope_sin = c->rope_sin.p;
-        ap.out = c->attn_out.p; ap.H = c->H; ap.Hkv = c->Hkv; ap.D = c->D; ap.Smax = c->Smax;
-        ap.scale = 1.0f / sqrtf((float)c->D);
-        if (c->cfg.qk_norm) {
-            ap.qnorm_w = c->qknorm.p + (size_t)(2 * li) * c->D;
-            ap.knorm_w = c->qknorm.p + (size_t)(2 * li + 1) * c->D;
-            ap.qk_eps = c->cfg.rms_norm_eps;
-        }
-        ap.rope_in_dtype = c->cfg.rope_ops_in_dtype;
-        launch_attn_decode(ap, c->batch, s);
+        launch_attn_decode(decode_attention(c, li), c->batch, s);
         gemm_o(c, li, s);
         if (f_gu) {
             launch_gemm_glue(EPI_SILU_MUL, c->batch, c->wgu.p + layer_gu_elems(c) * li, c->part.p, c->S_o, hcur, hoth, c->norms.p + (size_t)(2 * li + 1) * d, eps, c->act.p,
@@ -774,6 +782,50 @@ static void enqueue_layers(mis_tts* c, const bf16_t* table = nullptr, int table_
         const bf16_t* next_norm = c->norms.p + (size_t)(li + 1 < c->L ? 2 * (li + 1) : 2 * c->L) * d;
         launch_reduce_residual_rmsnorm(c->part.p, c->S_down, Mpad, d, hcur, next_norm, c->x.p, eps, s);
     }
+}
+// The layers of a decode step as one launch (lm_step.hip) where the shape is one that it takes: bf16 weights, one or two rows (k_step_layers says what bounds it; three rows and more carry
+// as many values between blocks as their granules cost time).  The same bits, whichever runs.
+static bool step_params(const mis_tts* c, StepParams& p) {
+    if (c->blocks || c->cfg.qk_norm || c->cfg.rope_ops_in_dtype || c->q_qkv.on || c->q_o.on || c->q_gu.on || c->q_down.on || c->Mpad != 16) return false;
+    if (c->a_qkv.ksb < 2 || c->a_o.ksb < 2 || c->a_down.ksb < 2 || c->ksb_gu < 2) return false;
+    auto role = [](const bf16_t* w, size_t layer, int items, int kt, int S, int ksb) {
+        return StepRole{reinterpret_cast<const unsigned char*>(w), layer * 2, items, kt, S * ksb, ksb, kt % (S * ksb) == 0 ? kt / (S * ksb) : 0};
+    };
+    p.qkv = role(c->wqkv.p, layer_qkv_elems(c), c->Nqkv / 16, c->d / 32, c->S_qkv, c->a_qkv.ksb);
+    p.o = role(c->wo.p, layer_o_elems(c), c->d / 16, c->H * c->D / 32, c->S_o, c->a_o.ksb);
+    p.gu = role(c->wgu.p, layer_gu_elems(c), c->ff / 16, c->d / 32, 1, c->ksb_gu);
+    p.down = role(c->wdown.p, layer_down_elems(c), c->d / 16, c->ff / 32, c->S_down, c->a_down.ksb);
+    p.x0 = c->x.p; p.h0 = c->h.p; p.x_out = c->x.p; p.h_out = c->h.p;
+    p.norms = c->norms.p; p.kcache = c->kcache.p; p.vcache = c->vtcache.p;
+    p.kv_layer = (size_t)c->batch * c->Hkv * c->Smax * c->D;
+    p.pos = c->pos_cur.p; p.active = c->active.p; p.rope_cos = c->rope_cos.p; p.rope_sin = c->rope_sin.p;
+    p.exch = c->step_exch.p; p.sync = c->step_sync.p; p.lock = c->step_lock;
+    const char* us = getenv("MIS_LM_STEP_US");                             // (tests force the time-out)
+    p.limit = us ? 100ull * (unsigned long long)std::max(0, atoi(us)) : 5000000ull;       // 50 ms: a step takes one to two
+    p.L = c->L; p.d = c->d; p.H = c->H; p.Hkv = c->Hkv; p.Smax = c->Smax; p.rows = c->batch; p.Mpad = c->Mpad;
+    p.schedule2 = attn_second_schedule(decode_attention(c, 0));
+    p.eps = c->cfg.rms_norm_eps; p.scale = 1.0f / sqrtf((float)c->D);
+    return true;
+}
+// Whether a request takes it, and its buffers.  `alone`: no kernel of the request may wait for another block's (the second attempt behind a time-out, a device shared by replicas).
+static bool step_begin(mis_tts* c, bool alone) {
+    const StepShape shape{c->L, c->d, c->ff, c->H, c->Hkv, c->D, c->batch};
+    const char* e = getenv("MIS_LM_STEP");                                 // 0: the launch chain (parity tests, read per call)
+    StepParams p{};
+    if (alone || c->step_off || (e && atoi(e) == 0) || !step_params(c, p) || !step_ok(shape, p, c->device)) return false;
+    c->step_lock = step_lock(c->device);
+    c->step_exch.alloc(step_exch_bytes(shape));
+    c->step_sync.alloc(SYNC_WORDS);
+    c->step_exch.zero(c->stream);                                          // (tags begin again)
+    c->step_sync.zero(c->stream);
+    return true;
+}
+static void enqueue_step(mis_tts* c) {
+    StepParams p{};
+    step_params(c, p);
+    p.fail = &c->samp_scratch.p->c_fail;
+    launch_embed_rmsnorm(c->emb.p, c->ids.p, c->active.p, c->pos_cur.p, c->pos_next.p, c->norms.p, c->h.p, c->x.p, c->d, c->V, p.eps, c->batch, c->Mpad, c->stream);
+    launch_step(p, c->stream);
 }
 static void enqueue_lm_head(mis_tts* c, const bf16_t* head = nullptr) {
     if (c->blocks) { c->blocks->enqueue_head(c->stream); return; }
@@ -1458,6 +1510,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         HIP_CHECK(hipMemcpyAsync(hid_count.p, ones_i.data(), batch * 4, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipStreamSynchronize(s));
     }
+    const bool one_launch = step_begin(c, multi_launch_only);
     sampler_resolve(sp, multi_launch_only);              // (environment switches read once per call; part of the graph key through sp)
     c->sp = sp;
     {   // the captured graphs bake in every pointer and scalar below: re-capture when any of them changes
@@ -1470,8 +1523,11 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         mix(ptrs, sizeof(ptrs));
         int ints[] = {batch, Lmax, max_tokens, c->Mpad, c->Smax, c->S_qkv, c->S_o, c->S_down, hidden_mode ? 1 : 0,
                       c->a_qkv.R, c->a_qkv.ksb, c->a_qkv.U, c->a_o.R, c->a_o.ksb, c->a_o.U, c->a_down.R, c->a_down.ksb, c->a_down.U,
-                      c->a_head.R, c->a_head.ksb, c->a_head.U, c->r_gu, c->ksb_gu, c->qa_gu.R, c->qa_gu.ksb, c->qa_head.R, c->qa_head.ksb, fold_gate_up(c), fold_qkv(c)};
+                      c->a_head.R, c->a_head.ksb, c->a_head.U, c->r_gu, c->ksb_gu, c->qa_gu.R, c->qa_gu.ksb, c->qa_head.R, c->qa_head.ksb, fold_gate_up(c), fold_qkv(c), one_launch};
         mix(ints, sizeof(ints));
+        const unsigned long long limit = getenv("MIS_LM_STEP_US") ? 1ull + (unsigned long long)std::max(0, atoi(getenv("MIS_LM_STEP_US"))) : 0ull;
+        const void* st[] = {c->step_exch.p, c->step_sync.p, reinterpret_cast<const void*>(limit)};
+        mix(st, sizeof(st));
         const void* hp[] = {collect_hidden ? (const void*)hm->hidden->p : nullptr, collect_hidden ? (const void*)hid_count.p : nullptr};
         mix(hp, sizeof(hp));
         if (key != c->graph_key) destroy_graphs(c);
@@ -1491,7 +1547,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
     auto decode_body = [&]() {
         enqueue_lm_head(c);
         launch_sampler(c->sp, batch, s);
-        enqueue_layers(c);
+        if (one_launch) enqueue_step(c); else enqueue_layers(c);
         collect(0);
     };
     auto capture = [&](hipGraphExec_t* exec, auto&& body) {
@@ -1557,6 +1613,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
             // k_samp_cluster).  The reference's loop cannot fail for lack of free compute units (LlamaTTS.swift:714-744): the caller
             // runs the request again on kernels that do not wait for each other.
             sampler_note_failure(c->samp_scratch.p, batch, s);
+            if (one_launch) c->step_off = true;
             for (auto& e : ev) (void)hipEventDestroy(e);
             throw SamplerTimeout{};
         }

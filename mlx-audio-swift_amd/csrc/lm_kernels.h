@@ -142,6 +142,7 @@ struct AttnParams {
     unsigned* xa_count;
     int first_schedule;      // 1: never k_attn_decode2 - a prompt's pairs give the same bits whatever their number
 };
+bool attn_second_schedule(const AttnParams& p);
 void launch_attn_decode(const AttnParams& p, int batch, hipStream_t s);
 
 #define SAMP_MAX_CHUNKS 64

@@ -1724,7 +1724,7 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
                 c = bf16_round_f32(c); s = bf16_round_f32(s);
                 r1 = f32_to_bf16(bf16_round_f32(x1 * c) + bf16_round_f32(-x2 * s));
                 r2 = f32_to_bf16(bf16_round_f32(x2 * c) + bf16_round_f32(x1 * s));
-            } else { r1 = f32_to_bf16(x1 * c - x2 * s); r2 = f32_to_bf16(x1 * s + x2 * c); }
+            } else { r1 = f32_to_bf16(fmaf(x1, c, -(x2 * s))); r2 = f32_to_bf16(fmaf(x1, s, x2 * c)); }
         } else { r1 = f32_to_bf16(x1); r2 = f32_to_bf16(x2); }      // Whisper: learned positions, no rotary
         if (hh < G) { qs[hh * D + i] = r1; qs[hh * D + i + D / 2] = r2; }
         else {
@@ -2364,8 +2364,8 @@ __global__ void __launch_bounds__(512) k_attn_decode2(AttnParams p) {
                 for (int e = 0; e < 8; ++e) {
                     const float x1 = x[c][e >> 2][e & 3], x2 = x[c + 2][e >> 2][e & 3];
                     const float cs = rc[c][e >> 2][e & 3], sn = rs[c][e >> 2][e & 3];
-                    out[c][e] = (short)f32_to_bf16(x1 * cs - x2 * sn);
-                    out[c + 2][e] = (short)f32_to_bf16(x1 * sn + x2 * cs);
+                    out[c][e] = (short)f32_to_bf16(fmaf(x1, cs, -(x2 * sn)));                 // (k_attn_decode rounds the other product of the second one)
+                    out[c + 2][e] = (short)f32_to_bf16(fmaf(x2, cs, x1 * sn));
                 }
         };
         bf16x8_t qf[4];
@@ -2590,6 +2590,12 @@ static bool launch_attn_cross(const AttnParams& p, int batch, hipStream_t s) {
     XA_GO(2, 5)
 #undef XA_GO
 }
+// second schedule (k_attn_decode2) where it applies: head_dim 128, RoPE tables, no q/k norm, <= 4 slabs, a decode step (the batched
+// prefill keeps the first schedule: its two arrangements must give the same bits whatever the batch size)
+bool attn_second_schedule(const AttnParams& p) {
+    return !p.first_schedule && !p.cache_rows && !p.append_only && p.D == 128 && !p.cross && p.rope_cos && !p.rope_in_dtype && !p.qnorm_w && p.S <= 4 && p.H / p.Hkv <= 4 &&
+           p.Smax <= 32 * ATT_WAVES * ATT2_MAX_J && p.Smax % 32 == 0 && ((uintptr_t)p.qkv_part & 15) == 0 && p.Nqkv % 4 == 0;
+}
 void launch_attn_decode(const AttnParams& p, int batch, hipStream_t s) {
     int G = p.H / p.Hkv;
     MIS_REQUIRE(G >= 1 && G <= 16 && p.H % p.Hkv == 0, MIS_ERR_INVALID_INPUT, "GQA group size must be 1..16");
@@ -2599,10 +2605,7 @@ void launch_attn_decode(const AttnParams& p, int batch, hipStream_t s) {
     MIS_REQUIRE(((uintptr_t)p.active & 3) == 0, MIS_ERR_GENERATION_FAILED, "attention: the active-flag array must be 4-byte aligned");
     dim3 grid(p.Hkv, batch), block(512);
     const int n_el = (G + 2) * p.D;
-    // second schedule (k_attn_decode2) where it applies: head_dim 128, RoPE tables, no q/k norm, <= 4 slabs, a decode step (the batched
-    // prefill keeps the first schedule: its two arrangements must give the same bits whatever the batch size)
-    if (!p.first_schedule && !p.cache_rows && !p.append_only && p.D == 128 && !p.cross && p.rope_cos && !p.rope_in_dtype && !p.qnorm_w && p.S <= 4 && G <= 4 && p.Smax <= 32 * ATT_WAVES * ATT2_MAX_J &&
-        p.Smax % 32 == 0 && ((uintptr_t)p.qkv_part & 15) == 0 && p.Nqkv % 4 == 0) {
+    if (attn_second_schedule(p)) {
         const size_t sm2 = attn2_smem_bytes(G);
         // k_attn_decode2 is compiled for 0 .. ATT2_MAX_J key tiles per wave (its switch has no case beyond): the cache must not hold more
         MIS_REQUIRE((p.Smax / 32 + ATT_WAVES - 1) / ATT_WAVES <= ATT2_MAX_J, MIS_ERR_GENERATION_FAILED,

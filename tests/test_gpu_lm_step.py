@@ -1,0 +1,108 @@
+"""-m gpu: the layers of a decode step as one launch (csrc/lm_step.hip): the bits of the launch chain - tokens, samples, and the logits behind the caches it leaves - over depth,
+rows, contexts at the edges of key tiles and of the chain's waves, a row that has ended, a launch that runs out of time, two handles at once."""
+import threading
+
+import numpy as np
+import pytest
+
+import mlx_audio_swift_amd as mas
+from mlx_audio_swift_amd.synthetic import snac_synthetic_weights
+
+pytestmark = pytest.mark.gpu
+
+SMALL = dict(encoder_dim=4, encoder_rates=[2, 4, 8, 8], decoder_dim=64, decoder_rates=[8, 8, 4, 2], codebook_size=4096, codebook_dim=8, vq_strides=[4, 2, 1])
+
+
+def model(layers, **kw):
+    cfg = mas.SNACConfig(**SMALL)
+    codec = mas.SNAC.from_weights(cfg, snac_synthetic_weights(cfg, seed=1))
+    lm = mas.LlamaTTSModel(mas.LlamaTTSConfiguration(hidden_size=3072, num_hidden_layers=layers, intermediate_size=8192, num_attention_heads=24, num_key_value_heads=8, head_dim=128,
+                                                     vocab_size=156940, rms_norm_eps=1e-5, rope_theta=500000.0, **kw), codec)
+    mas.generation.check(mas._lib.lib().mis_tts_init_synthetic(lm._h, 7))
+    lm.finalize()
+    return lm
+
+
+def prompts(rows, n):
+    r = np.random.default_rng(3)
+    return [np.concatenate([[128259], r.integers(0, 128000, n - 4 - 3 * b), [128009, 128260, 128257]]).astype(np.int32) for b in range(rows)]
+
+
+def run(lm, rows, n, tokens):
+    pcm, tok = lm.generate_batch(prompts(rows, n), mas.GenerateParameters(max_tokens=tokens, seed=5, temperature=0.8, frame_constrained=2), return_tokens=True)
+    return [np.concatenate(pcm), np.concatenate(tok), lm.lm_forward([128258] * rows)]
+
+
+def same(a, b):
+    return all(np.array_equal(x, y) for x, y in zip(a, b)) and np.isfinite(a[2]).all()
+
+
+@pytest.fixture(scope="module")
+def three():
+    return model(3)
+
+
+# positions 26 .. 46, 245 .. 265 and 1018 .. 1038: into the second key tile, past the eight waves' first tiles, past k_attn_decode2's caches
+@pytest.mark.parametrize("rows,n", [(1, 26), (2, 26), (1, 245), (2, 245), (1, 1018)])
+def test_bits_of_the_launch_chain(monkeypatch, three, rows, n):
+    monkeypatch.setenv("MIS_LM_STEP", "0")
+    chain = run(three, rows, n, 21)
+    monkeypatch.delenv("MIS_LM_STEP")
+    for _ in range(2):
+        assert same(run(three, rows, n, 21), chain)
+
+
+@pytest.mark.parametrize("layers", [1, 2])
+def test_depth(monkeypatch, layers):
+    lm = model(layers)
+    monkeypatch.setenv("MIS_LM_STEP", "0")
+    chain = run(lm, 2, 40, 70)                                             # more steps than one poll of the host's
+    monkeypatch.delenv("MIS_LM_STEP")
+    assert same(run(lm, 2, 40, 70), chain)
+
+
+def test_a_row_alone_and_among_others(three):
+    """One row (here), two (here) and three (the chain) of the same batch."""
+    a, b, c = run(three, 1, 40, 14), run(three, 2, 40, 14), run(three, 3, 40, 14)
+    assert np.array_equal(a[1], b[1][:14]) and np.array_equal(b[1], c[1][:28]) and np.array_equal(a[2][0], b[2][0]) and np.array_equal(b[2], c[2][:2])
+
+
+def test_a_row_that_has_ended(monkeypatch):
+    lm = model(2)
+    gp = mas.GenerateParameters(max_tokens=28, seed=5, temperature=0.8, frame_constrained=2)
+    tok = lm.generate_batch(prompts(2, 40), gp, return_tokens=True)[1]
+    ends = [int(t) for t in tok[1][9:12] if t not in tok[0]][0]             # row 1 ends early, row 0 goes on
+    lm = model(2, end_of_speech_id=ends)
+    monkeypatch.setenv("MIS_LM_STEP", "0")
+    chain = lm.generate_batch(prompts(2, 40), gp, return_tokens=True)
+    monkeypatch.delenv("MIS_LM_STEP")
+    here = lm.generate_batch(prompts(2, 40), gp, return_tokens=True)
+    assert len(chain[1][1]) < len(chain[1][0])
+    assert all(np.array_equal(x, y) for i in range(2) for x, y in zip(chain[i], here[i]))
+
+
+def test_out_of_time_runs_on_the_chain(monkeypatch):
+    """No time to wait at all: the first poll in vain ends every launch, the request runs again on the launch chain, and so do the handle's later ones."""
+    lm = model(2)
+    monkeypatch.setenv("MIS_LM_STEP", "0")
+    chain = run(lm, 1, 40, 14)
+    monkeypatch.delenv("MIS_LM_STEP")
+    monkeypatch.setenv("MIS_LM_STEP_US", "0")
+    assert same(run(lm, 1, 40, 14), chain)
+    monkeypatch.delenv("MIS_LM_STEP_US")
+    assert same(run(lm, 1, 40, 14), chain)
+
+
+def test_two_handles_at_once(three):
+    other = model(3)
+    want = run(three, 1, 40, 70)
+    got = {}
+
+    def work(name, lm):
+        got[name] = [run(lm, 1, 40, 70) for _ in range(3)]
+    threads = [threading.Thread(target=work, args=(k, m)) for k, m in (("a", three), ("b", other))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(same(r, want) for k in "ab" for r in got[k])
