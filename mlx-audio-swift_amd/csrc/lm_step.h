@@ -36,3 +36,5 @@ bool step_ok(const StepShape& s, const StepParams& p, int device);
 void launch_step(const StepParams& p, hipStream_t s);
 // A word per device, for all handles of the process: two launches that each hold part of the compute units and wait for the rest would both run out of time
 unsigned* step_lock(int device);
+// in front of a launch that needs the whole device; that launch gives it back (sync[SYNC_LOCKED])
+void launch_step_lock(unsigned* lock, unsigned* sync, unsigned* fail, hipStream_t s);

@@ -799,10 +799,12 @@ bool step_ok(const StepShape& s, const StepParams& p, int device) {
 
 void launch_step(const StepParams& p, hipStream_t s) {
     const int ring = ring_of(p), lds = lds_bytes(p, ring);
-    hipLaunchKernelGGL(k_step_lock, dim3(1), dim3(64), 0, s, p.lock, p.sync, p.fail, LOCK_LIMIT);
+    launch_step_lock(p.lock, p.sync, p.fail, s);
     if (ring == 16) hipLaunchKernelGGL((k_step_layers<16>), dim3(CU), dim3(THREADS), lds, s, p);
     else hipLaunchKernelGGL((k_step_layers<12>), dim3(CU), dim3(THREADS), lds, s, p);
 }
+
+void launch_step_lock(unsigned* lock, unsigned* sync, unsigned* fail, hipStream_t s) { hipLaunchKernelGGL(k_step_lock, dim3(1), dim3(64), 0, s, lock, sync, fail, LOCK_LIMIT); }
 
 unsigned* step_lock(int device) {
     static std::mutex m;

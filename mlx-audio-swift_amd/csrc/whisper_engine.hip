@@ -8,6 +8,7 @@
 #include "kernels.h"
 #include "lm_kernels.h"
 #include "whisper_kernels.h"
+#include "whisper_step.h"
 
 #include <math.h>
 #include <string.h>
@@ -48,6 +49,12 @@ struct mis_whisper {
     DevBuf<bf16_t> h, h2, x, attn_out, act, logits;      // h2: the other residual buffer of the folded glue (enqueue_decoder_step)
     DevBuf<float> qkv_part, part, e_buf, logits_f32;
     DevBuf<SamplerScratch> scratch;
+    // a step's layers as one launch (whisper_step.hip)
+    DevBuf<WsLayer> step_layers;
+    DevBuf<unsigned char> step_exch;
+    DevBuf<unsigned> step_sync, step_table;
+    unsigned* step_lock = nullptr;       // the device's, not this handle's
+    bool step_off = false;               // a launch ran out of time: the launch chain from then on
     // encoder workspace (a sub-batch of up to 8 windows), audio and features of a call: kept, they are the same size call after call
     DevBuf<bf16_t> e_col1, e_tight, e_h1, e_col2, e_h, e_x, e_qkv, e_att, e_ff, e_kc, e_vc, e_ckv;
     DevBuf<float> pcm, padded, feats, enc_f32;
@@ -593,6 +600,61 @@ static void enqueue_decoder_step(mis_whisper* c, const int32_t* ids) {
         launch_reduce_residual_rmsnorm(c->part.p, c->S_fc2, Mpad, d, hcur, nw, c->x.p, LN_EPS, s, nb);
     }
 }
+// The same layers as one launch (whisper_step.hip), same bits, where the rows' tasks fit the compute units: false where they do not, or where the chain would not take the folds
+// whose order of sums that launch has.
+static bool step_params(const mis_whisper* c, WsParams& p) {
+    const int d = c->d, KT = d / 32;
+    const char* fe = getenv("MIS_WHISPER_FOLD");
+    AttnParams probe{};
+    probe.cross = 1; probe.cross_len = 1500; probe.D = c->D; probe.H = probe.Hkv = c->Hd; probe.qp_KT = KT; probe.qp_S = c->S_o;
+    if ((fe && atoi(fe) != WHISPER_FOLD_DEFAULT) || c->Mpad != 16 || d % 32 || c->cfg.decoder_ffn_dim % 32 || !attn_qp_ok(probe) ||
+        !gemm_skinny_norm_ok(EPI_GELU_PACKED, 2, KT, 1, c->S_o, c->Mpad, c->batch)) return false;
+    p.role[WS_QKV] = {3 * d / 16, KT, c->S_qkv, 4};
+    p.role[WS_O] = p.role[WS_CO] = {d / 16, KT, c->S_o, 4};
+    p.role[WS_CQ] = {d / 16, KT, 1, 8};
+    p.role[WS_FC1] = {c->cfg.decoder_ffn_dim / 16, KT, 1, 8};
+    p.role[WS_FC2] = {d / 16, c->cfg.decoder_ffn_dim / 32, c->S_fc2, 4};
+    p.layers = c->step_layers.p; p.table = c->step_table.p; p.x0 = c->x.p; p.h0 = c->h.p; p.x_out = c->x.p;
+    p.self_k = c->self_k.p; p.self_v = c->self_v.p; p.cross_k = c->cross_k.p; p.cross_v = c->cross_v.p;
+    p.self_layer = (size_t)c->batch * c->Hd * c->Smax * c->D; p.cross_layer = (size_t)c->batch * c->Hd * c->Spad * c->D;
+    p.pos = c->pos_cur.p; p.active = c->active.p; p.exch = c->step_exch.p; p.sync = c->step_sync.p; p.fail = &c->scratch.p->c_fail; p.lock = c->step_lock;
+    const char* us = getenv("MIS_WHISPER_STEP_US");                        // (tests force the time-out)
+    p.limit = us ? 100ull * (unsigned long long)std::max(0, atoi(us)) : 5000000ull;       // 50 ms: a step takes a tenth to one
+    p.L = (int)c->dec.size(); p.d = d; p.ff = c->cfg.decoder_ffn_dim; p.H = c->Hd; p.rows = c->batch; p.Smax = c->Smax; p.Spad = c->Spad; p.cross_len = 1500;
+    p.eps = LN_EPS; p.scale = 1.0f / sqrtf((float)c->D);
+    return ws_plan(p, c->device);
+}
+// Whether a request takes it, and its buffers.  `alone`: no kernel of the request may wait for another block's.
+static bool step_begin(mis_whisper* c, bool alone) {
+    const char* e = getenv("MIS_WHISPER_STEP");                            // 0: the launch chain (parity tests, read per call)
+    WsParams p{};
+    if (alone || c->step_off || (e && atoi(e) == 0) || !step_params(c, p)) return false;
+    if (!c->step_layers.p) {
+        std::vector<WsLayer> t;
+        for (const DecLayer& l : c->dec)
+            t.push_back({{l.sqkv, l.so, l.cq, l.co, l.fc1, l.fc2}, {l.sbqkv, l.sbo, l.cbq, l.cbo, l.b1, l.b2}, {l.ln1w, l.ln2w, l.ln3w}, {l.ln1b, l.ln2b, l.ln3b}});
+        t.push_back({{}, {}, {c->dec_lnw}, {c->dec_lnb}});
+        c->step_layers.alloc(t.size());
+        HIP_CHECK(copy_now(c->step_layers.p, t.data(), t.size() * sizeof(WsLayer), hipMemcpyHostToDevice));
+    }
+    const std::vector<unsigned> table = ws_tables(p);
+    c->step_table.alloc(table.size());
+    HIP_CHECK(copy_now(c->step_table.p, table.data(), table.size() * 4, hipMemcpyHostToDevice));
+    c->step_lock = step_lock(c->device);
+    c->step_exch.alloc(ws_exch_bytes(p));
+    c->step_sync.alloc(SYNC_WORDS);
+    c->step_exch.zero(c->stream);                                          // (tags begin again)
+    c->step_sync.zero(c->stream);
+    return true;
+}
+static void enqueue_step(mis_whisper* c, const int32_t* ids) {
+    WsParams p{};
+    MIS_REQUIRE(step_params(c, p), MIS_ERR_GENERATION_FAILED, "internal: the plan of a decoder step changed under way");
+    if (ids)
+        launch_whisper_embed_ln(c->emb, c->dec_pos, ids, c->active.p, c->pos_cur.p, c->pos_next.p, c->dec[0].ln1w, c->dec[0].ln1b, c->h.p, c->x.p, c->d, c->V, c->cfg.max_target_positions,
+                                c->batch, c->Mpad, c->stream);
+    launch_whisper_step(p, c->stream);
+}
 static void enqueue_vocab(mis_whisper* c) {
     launch_gemm_skinny(EPI_BF16, 2, 1, c->emb_packed, c->x.p, c->logits.p, c->Vpad / 16, c->d / 32, 1, c->Vpad, c->Mpad, c->stream);
 }
@@ -695,7 +757,9 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
         // (one upload and no wait between the steps: a step's launches are queued while the one in front runs)
         HIP_CHECK(hipMemcpyAsync(c->prompt_rows.p, prompt_rows.data(), prompt_rows.size() * 4, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipMemcpyAsync(c->active.p, ones.data(), batch, hipMemcpyHostToDevice, s));
-        for (int j = 0; j < n_prompt; ++j) enqueue_decoder_step(c, c->prompt_rows.p + (size_t)j * batch);
+        const bool one_launch = step_begin(c, multi_launch_only);
+        auto layers = [&](const int32_t* ids) { if (one_launch) enqueue_step(c, ids); else enqueue_decoder_step(c, ids); };
+        for (int j = 0; j < n_prompt; ++j) layers(c->prompt_rows.p + (size_t)j * batch);
         // ---- decode loop
         c->tokens_out.alloc((size_t)batch * max_tokens);
         c->tokens_out.zero(s);
@@ -724,13 +788,13 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
             if (greedy_step_ok(q, c->d)) {
                 launch_greedy_step(q, GreedyStep{c->sup.p, c->bsup.p, sp->n_suppress, sp->n_begin_suppress, c->emb, c->dec_pos, c->dec[0].ln1w, c->dec[0].ln1b, c->pos_cur.p, c->pos_next.p,
                                                  c->h.p, c->x.p, c->d, c->cfg.max_target_positions, batch}, c->Mpad, s);
-                enqueue_decoder_step(c, nullptr);
+                layers(nullptr);
                 return;
             }
             launch_whisper_suppress(c->logits.p, c->Vpad, c->V, c->sup.p, sp->n_suppress, c->bsup.p, sp->n_begin_suppress, c->n_gen.p,
                                     c->active.p, batch, s);
             launch_sampler(q, batch, s);
-            enqueue_decoder_step(c, c->ids.p);
+            layers(c->ids.p);
     };
     hipGraphExec_t gexec = nullptr;
     const bool use_graph = getenv("MIS_NO_GRAPH") == nullptr;
@@ -775,7 +839,7 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     }
     if (gexec) (void)hipGraphExecDestroy(gexec);
     HIP_CHECK(hipGetLastError());
-    if (sampler_failed) sampler_note_failure(c->scratch.p, batch, s);
+    if (sampler_failed) { sampler_note_failure(c->scratch.p, batch, s); c->step_off = c->step_off || one_launch; }
     return !sampler_failed;
     };
     if (!attempt(c->shared_device)) {

@@ -1,0 +1,606 @@
+// whisper_step.hip - the decoder layers of a Whisper step in ONE launch, for as many rows as the compute units have room for.
+//
+// A step of the launch chain is eight launches a layer, each at its own end: Whisper-tiny's 34 launches of 3 - 10 us are 169 us for weights that stream in 11.  Here every block has ONE
+// task for all layers - a few column tiles of one matrix, or the self- or cross-attention of one (row, head) - and holds what the task needs of the NEXT layer in registers (its weight
+// tiles; a head's 384 KB of cached keys and values on eight waves) while the other seven tasks of this layer run.  So all streaming lies beside the chain of dependencies, and what is
+// left of that is eight hand-overs a layer.  These are granules as in lm_step.hip: eight bytes, two bfloat16 values and the tag that says whose they are; bounded polls; a lock a device.
+// A block polls one granule of the values in FRONT of its input, then all of its input: a poll of one granule of the input and then all of it is a round trip more.
+//
+// us a step with the output projection and the sampling (26), chain -> here: 384 columns, 4 layers, one row 169 -> 107, four 175 -> 119; 768, 12 layers 526 -> 301; 1280, 32 layers
+// 1523 -> 990.  What bounds it: the hand-overs, 0.7 - 1.4 us each, and the short programs between them (a norm 0.8, cross-attention 3, a few tiles' products and their sums 1 - 2).
+//
+// A row has the bits of the launch chain: K is cut and summed as there, and each norm's statistics are dealt and summed as in the kernel that held them (LN_* below).
+#include "whisper_step.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace {
+// MAX_BLOCKS: a block fills its compute unit's registers, and a few units stay for other handles' waiting k_step_lock
+constexpr int THREADS = 512, WAVES = 8, NF = 36, MAX_ROWS = 4, D = 64, CJ = 6, SJ = 2, LNG = 5, MAX_BLOCKS = 248;
+// attention: a strip of q | k | v a wave, a wave's scores, then probabilities (f32), their halves (bf16), their sums; the waves' partial results
+constexpr int ATT_SC = 3 * D * 2, ATT_PH = ATT_SC + CJ * 128, ATT_PL = ATT_PH + CJ * 64, ATT_PS = ATT_PL + CJ * 64, ATT_WAVE = ATT_PS + CJ * 16, ATT_LDS = WAVES * (ATT_WAVE + (D + 2) * 4);
+typedef unsigned long long u64;
+// (pointers out of a table in memory: without the address space their loads would be flat ones, which reads of LDS wait for)
+template <class T> using Global = const __attribute__((address_space(1))) T*;
+template <class T> __device__ __forceinline__ Global<T> global(const T* p) { return (Global<T>)(uintptr_t)p; }
+enum { LN_NONE, LN_GLUE, LN_SLICES, LN_WAVE };         // statistics as k_glue4, as k_attn_cross (slices of K a wave), as k_gemm_skinny_norm (a row a wave)
+enum { TO_T, TO_RESID, TO_GELU };
+
+struct Exch { unsigned q, at, h1, cq, ca, hb, act, h2, layer; };
+__host__ __device__ inline Exch exch_layout(int d, int ff, int rows) {
+    Exch e;
+    unsigned a = 0;
+    e.q = a; a += rows * 3 * d * 4;
+    e.at = a; a += rows * d * 4;
+    e.h1 = a; a += rows * d * 4;
+    e.cq = a; a += rows * d * 4;
+    e.ca = a; a += rows * d * 4;
+    e.hb = a; a += rows * d * 4;
+    e.act = a; a += rows * ff * 4;
+    e.h2 = a; a += rows * d * 4;
+    e.layer = a;
+    return e;
+}
+// x | what the columns without a row read (zeros) and write | partial sums | table of fragments | a norm's weights
+struct Lds { int none, part, tab, wb, total; };
+__host__ __device__ inline Lds lds_layout(int k_max, int rows, int units) {
+    Lds l;
+    int a = k_max * rows * 2;
+    l.none = a; a += 128;
+    l.part = a; a += units * rows * 64;
+    l.tab = a; a += WAVES * NF * 4;
+    l.wb = a; a += 2 * 256 * LNG * 2;
+    l.total = a > ATT_LDS ? a : ATT_LDS;
+    return l;
+}
+__device__ __forceinline__ void bar() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ void granule(unsigned char* p, uint32_t v, unsigned tag) {
+    __hip_atomic_store(reinterpret_cast<u64*>(p), (u64)v | (u64)tag << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float lo(uint32_t v) { return bf16_to_f32((bf16_t)(v & 0xffffu)); }
+__device__ __forceinline__ float hi(uint32_t v) { return bf16_to_f32((bf16_t)(v >> 16)); }
+__device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
+
+// The arguments, read again (scalar loads) from here on: kept in registers over the layer loop they are more than there are.
+typedef __attribute__((address_space(4))) const WsParams* ArgPtr;
+__device__ __forceinline__ const WsParams& args() {
+    ArgPtr a = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return *(const WsParams*)a;
+}
+
+__device__ __forceinline__ bool more_time(u64& t0, int lane) {
+    const WsParams& p = args();
+    const u64 now = wall_clock64();
+    if (t0 == 0) t0 = now;
+    if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(p.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) return false;
+    if (now - t0 < p.limit) return true;
+    if (lane == 0) __hip_atomic_store(p.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+}
+// `one`, the same for all lanes of the wave, until it carries `tag`
+__device__ __forceinline__ bool await(bool hasty, const unsigned char* one, unsigned tag, int lane) {
+    u64 t0 = 0;
+    for (int n = 0;; ++n) {
+        unsigned v = tag;
+        if (lane == 0) v = (unsigned)(__hip_atomic_load(reinterpret_cast<const u64*>(one), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32);
+        if ((unsigned)__builtin_amdgcn_readfirstlane(v) == tag) break;
+        if (((n & 63) == 63 || hasty) && !more_time(t0, lane)) return false;
+    }
+    asm volatile("" ::: "memory");
+    return true;
+}
+// N granules a lane, at(i) granule i's address, until all carry `tag`
+template <int N, class At>
+__device__ __forceinline__ bool gather(bool hasty, uint32_t (&out)[N], unsigned tag, int lane, At&& at) {
+    u64 t0 = 0;
+    for (int n = 0;; ++n) {
+        bool ok = true;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const u64 v = __hip_atomic_load(reinterpret_cast<const u64*>(at(i)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ok = ok && (unsigned)(v >> 32) == tag;
+            out[i] = (uint32_t)v;
+        }
+        if (__all(ok)) break;
+        if (((n & 63) == 63 || hasty) && !more_time(t0, lane)) return false;
+    }
+    asm volatile("" ::: "memory");
+    return true;
+}
+
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint2 load2(Global<bf16_t> p) { const u32x2 v = *(Global<u32x2>)p; return make_uint2(v[0], v[1]); }
+
+// ------------------------------------------------------------------------------------------------------------------ a matrix
+// A row's norm on one wave, from granules to xs.  `groups` of four columns a lane; the sums of their lanes are added as the chain's kernel added its waves (LN_WAVE: one sum).
+template <int KIND> __device__ __forceinline__ int norm_column(int K, int g, int lane) { return KIND == LN_SLICES ? 32 * ((K / 32 * g) / WAVES) + 4 * lane : 4 * (lane + 64 * g); }
+template <int KIND> __device__ __forceinline__ int norm_end(int K, int g) { return KIND == LN_SLICES ? 32 * ((K / 32 * (g + 1)) / WAVES) : min(K, 256 * (g + 1)); }
+__device__ __forceinline__ void norm_weights(bf16_t* wb, int K, Global<bf16_t> w, Global<bf16_t> b, int lane) {
+    for (int col = 4 * lane; col < K; col += 256) {
+        *reinterpret_cast<uint2*>(wb + col) = load2(w + col);
+        *reinterpret_cast<uint2*>(wb + K + col) = load2(b + col);
+    }
+}
+template <int KIND>
+__device__ __forceinline__ bool norm_row(bool hasty, const unsigned char* in, unsigned tag, bf16_t* row, const bf16_t* wb, int K, float eps, int lane) {
+    constexpr int G = KIND == LN_SLICES ? WAVES : LNG;
+    uint32_t v[2 * G];
+    if (!gather<2 * G>(hasty, v, tag, lane, [&](int i) {
+            const int col = norm_column<KIND>(K, i >> 1, lane);
+            return in + (size_t)(col < norm_end<KIND>(K, i >> 1) ? col : K - 4) * 4 + (i & 1) * 8;
+        })) return false;
+    float sum[G], sq[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const bool live = norm_column<KIND>(K, g, lane) < norm_end<KIND>(K, g);
+        float a = KIND == LN_WAVE && g > 0 ? sum[g - 1] : 0.0f;
+        a += live ? lo(v[2 * g]) : 0.0f; a += live ? hi(v[2 * g]) : 0.0f; a += live ? lo(v[2 * g + 1]) : 0.0f; a += live ? hi(v[2 * g + 1]) : 0.0f;
+        sum[g] = a;
+    }
+    auto total = [&](float (&part)[G]) {
+        if (KIND == LN_WAVE) return wave_sum_dpp(part[G - 1]);
+        float t = 0.0f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) part[g] = wave_sum_dpp(part[g]);
+#pragma unroll
+        for (int g = 0; g < G; ++g) t += part[g];
+        return t;
+    };
+    const float mean = total(sum) / (float)K;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const bool live = norm_column<KIND>(K, g, lane) < norm_end<KIND>(K, g);
+        const float h[4] = {lo(v[2 * g]), hi(v[2 * g]), lo(v[2 * g + 1]), hi(v[2 * g + 1])};
+        float a = KIND == LN_WAVE && g > 0 ? sq[g - 1] : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const float dl = h[e] - mean; a += live ? dl * dl : 0.0f; }
+        sq[g] = a;
+    }
+    const float rstd = 1.0f / sqrtf(total(sq) / (float)K + eps);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+        const int col = norm_column<KIND>(K, g, lane);
+        if (col < norm_end<KIND>(K, g)) {
+            const uint2 w = *reinterpret_cast<const uint2*>(wb + col), b = *reinterpret_cast<const uint2*>(wb + K + col);
+            const float h[4] = {lo(v[2 * g]), hi(v[2 * g]), lo(v[2 * g + 1]), hi(v[2 * g + 1])}, wv[4] = {lo(w.x), hi(w.x), lo(w.y), hi(w.y)}, bv[4] = {lo(b.x), hi(b.x), lo(b.y), hi(b.y)};
+            bf16_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = f32_to_bf16(fmaf((h[e] - mean) * rstd, wv[e], bv[e]));
+            *reinterpret_cast<uint2*>(row + col) = make_uint2((uint32_t)o[0] | ((uint32_t)o[1] << 16), (uint32_t)o[2] | ((uint32_t)o[3] << 16));
+        }
+    }
+    return true;
+}
+
+template <int R, int LN, int TO>
+__device__ __forceinline__ void matrix(unsigned char* smem, int block, int tid, unsigned near_at, unsigned in_at, unsigned out_at, unsigned res_at, unsigned exch_layer, unsigned tag) {
+    const WsParams& p = args();
+    const WsRole ro = p.role[R];
+    const bool hasty = p.limit == 0;
+    const int L = p.L;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int KT = ro.KT, K = KT * 32, P = ro.S * ro.ksb, tile0 = block * ro.per, nt = min(ro.per, ro.tiles - tile0), cols = ro.tiles * 16, rows = p.rows;
+    const Lds l = lds_layout(p.k_max, rows, p.units);
+    bf16_t* xs = reinterpret_cast<bf16_t*>(smem);
+    float* part = reinterpret_cast<float*>(smem + l.part);
+    unsigned* tab = reinterpret_cast<unsigned*>(smem + l.tab) + wave * NF;
+    if (tid < 32) reinterpret_cast<unsigned*>(smem + l.none)[tid] = 0;
+    for (int i = tid; i < p.units * rows * 16; i += THREADS) part[i] = 0.f;            // (a piece without a K-tile stays zero)
+    // this wave's fragments in the order of ws_table, those of tiles that the last block does not have left out: entry f in lane f; behind them the last one's weights times zero
+    unsigned ent = lane < NF ? p.table[(R * WAVES + wave) * NF + lane] : 0u;
+    const bool have = (ent >> 13 & 1u) && (int)(ent >> 8 & 15u) < nt;
+    const u64 all = __ballot(have);
+    const int n = __builtin_amdgcn_readfirstlane((int)__popcll(all));
+    if (have) tab[__popcll(all & ((1ull << lane) - 1ull))] = ent;
+    bar();
+    ent = n == 0 ? 0u : lane < n ? tab[lane] : tab[n - 1] & ~(3u << 12);
+    bf16x8_t w[NF];
+    auto request = [&](int li) {
+        const Global<bf16x8_t> base = (Global<bf16x8_t>)global(args().layers[li].w[R]) + (size_t)tile0 * KT * 64 + lane;
+#pragma unroll
+        for (int g = 0; g < NF / 4; ++g)
+            if (g * 4 < n) {
+#pragma unroll
+                for (int f = g * 4; f < g * 4 + 4; ++f) {
+                    const unsigned e = __builtin_amdgcn_readlane(ent, f);
+                    w[f] = __builtin_nontemporal_load(base + ((e >> 8 & 15u) * KT + (e & 255u)) * 64);
+                }
+            }
+        asm volatile("" ::: "memory");
+    };
+    request(0);
+    // the values that a thread sums: columns 2 c2, 2 c2 + 1 of tile t, row m
+    const int pairs = nt * 8, m = tid / pairs, rest = tid - m * pairs, t = rest >> 3, col = (tile0 + t) * 16 + (rest & 7) * 2;
+    const bool mine = tid < pairs * rows;
+    // the input of layer li into xs; false: stop
+    auto input = [&](const unsigned char* in, int id) {
+        const int total = rows * (K / 2);
+        auto some = [&](auto count, int b0) {
+            constexpr int N = decltype(count)::value;
+            if (b0 + wave * 64 >= total) return true;                       // (nothing for this wave)
+            uint32_t v[N];
+            if (!gather<N>(hasty, v, tag, lane, [&](int i) { return in + (size_t)min(b0 + id + i * THREADS, total - 1) * 8; })) return false;
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                if (b0 + id + i * THREADS < total) reinterpret_cast<uint32_t*>(xs)[b0 + id + i * THREADS] = v[i];
+            return true;
+        };
+        int b0 = 0;
+        for (; total - b0 > THREADS; b0 += 3 * THREADS)
+            if (!some(std::integral_constant<int, 3>{}, b0)) return false;
+        return b0 >= total || some(std::integral_constant<int, 1>{}, b0);
+    };
+    bf16_t* wb = reinterpret_cast<bf16_t*>(smem + l.wb);
+    // the input of a layer, from the values at `src`, into xs: false: stop
+    auto take = [&](int li, const unsigned char* src, int id) {
+        if constexpr (LN == LN_NONE) return input(src + in_at, id);
+        else {
+            if (wave >= rows) return true;
+            constexpr int which = LN == LN_GLUE ? 0 : LN == LN_SLICES ? 1 : 2;
+            const WsParams& p = args();
+            norm_weights(wb, K, global(p.layers[li].lnw[which]), global(p.layers[li].lnb[which]), id & 63);
+            return norm_row<LN>(hasty, src + in_at + (size_t)wave * K * 4, tag, xs + wave * K, wb, K, p.eps, id & 63);
+        }
+    };
+    if (R == WS_QKV)
+        for (int i = tid; i < rows * (K / 8); i += THREADS) {
+            const int r = i / (K / 8), k = (i - r * (K / 8)) * 8;
+            *reinterpret_cast<uint4*>(xs + r * K + k) = *reinterpret_cast<const uint4*>(p.x0 + xpk_index(r, k, 1));
+        }
+    for (int layer = 0; layer < L; ++layer) {
+        int li = layer, id = tid;
+        asm volatile("" : "+s"(li), "+v"(id));                             // (addresses kept over all layers are registers that the weights need)
+        const WsParams& p = args();
+        unsigned char* now = p.exch + (size_t)exch_layer * li;
+        // what the values in front of the input say is near, and what is there before it: bias, residual, the norm's weights
+        unsigned char* const src = R == WS_QKV ? now - exch_layer : now;
+        if ((R != WS_QKV || li > 0) && (LN == LN_NONE || wave < rows) && !await(hasty, src + near_at, tag, lane)) return;
+        const uint32_t bias = mine && p.layers[li].b[R] ? *(Global<uint32_t>)global(p.layers[li].b[R] + col) : 0u;
+        uint32_t hres[1] = {0};
+        bool good = true;
+        if (TO == TO_RESID && mine) {
+            if (R == WS_O && li == 0) hres[0] = *reinterpret_cast<const uint32_t*>(p.h0 + (size_t)m * p.d + col);
+            else {
+                const unsigned char* from = (R == WS_O ? now - exch_layer : now) + res_at + ((size_t)m * cols + col) * 4;
+                good = gather<1>(hasty, hres, tag, lane, [&](int) { return from; });
+            }
+        }
+        if (!__all(good)) return;
+        if ((R != WS_QKV || li > 0) && !take(li, src, id)) return;
+        bar();
+        {
+            const int xr = lane & 15, kg = lane >> 4;
+            const bool row = xr < rows;
+            const unsigned xstep = row ? 64 : 0, xbase = row ? xr * K * 2 + kg * 16 : l.none, ustep = row ? rows * 64 : 0, ubase = row ? l.part + xr * 64 + kg * 16 : l.none + 64 + kg * 16;
+            f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int g = 0; g < NF / 4; ++g)
+                if (g * 4 < n) {
+                    bf16x8_t x[4];
+#pragma unroll
+                    for (int f = 0; f < 4; ++f)
+                        x[f] = *reinterpret_cast<const bf16x8_t*>(smem + xbase + __umul24(__builtin_amdgcn_readlane(ent, g * 4 + f) & 255u, xstep));
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) {
+                        const unsigned e = __builtin_amdgcn_readlane(ent, g * 4 + f);
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[g * 4 + f], x[f], acc, 0, 0, 0);
+                        if (e & (1u << 12)) {
+                            *reinterpret_cast<f32x4_t*>(smem + ubase + __umul24(e >> 16, ustep)) = acc;
+                            acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                        }
+                    }
+                }
+        }
+        bar();
+        if (mine) {
+            constexpr int KSB = R == WS_CQ || R == WS_FC1 ? 8 : 4, G = 16 / KSB;
+            float a0 = 0.f, a1 = 0.f;
+            const float* q = part + (t * P * rows + m) * 16 + (rest & 7) * 2;
+            for (int s0 = 0; s0 < ro.S; s0 += G) {
+                float2 v[G][KSB];
+#pragma unroll
+                for (int g = 0; g < G; ++g)
+#pragma unroll
+                    for (int i = 0; i < KSB; ++i) v[g][i] = *reinterpret_cast<const float2*>(q + (min(s0 + g, ro.S - 1) * KSB + i) * rows * 16);
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    float b0 = v[g][0].x, b1 = v[g][0].y;
+#pragma unroll
+                    for (int i = 1; i < KSB; ++i) { b0 += v[g][i].x; b1 += v[g][i].y; }
+                    if (s0 + g == 0) { b0 += lo(bias); b1 += hi(bias); }
+                    if (s0 + g < ro.S) { a0 += b0; a1 += b1; }
+                }
+            }
+            if (TO == TO_RESID) { a0 = lo(hres[0]) + bf16_round_f32(a0); a1 = hi(hres[0]) + bf16_round_f32(a1); }
+            if (TO == TO_GELU) { a0 = gelu_erf(bf16_round_f32(a0)); a1 = gelu_erf(bf16_round_f32(a1)); }
+            granule(now + out_at + ((size_t)m * cols + col) * 4, (uint32_t)f32_to_bf16(a0) | (uint32_t)f32_to_bf16(a1) << 16, tag);
+        }
+        bar();                                                             // (the next weights are asked for behind the stores)
+        if (li + 1 < L) request(li + 1);
+    }
+    if (R == WS_QKV && block == 0) {                                       // behind the last layer: the decoder's norm
+        const unsigned char* src = args().exch + (size_t)exch_layer * (L - 1);
+        if ((wave < rows && !await(hasty, src + near_at, tag, lane)) || !take(L, src, tid)) return;
+        bar();
+        for (int i = tid; i < rows * (K / 8); i += THREADS) {
+            const int r = i / (K / 8), k = (i - r * (K / 8)) * 8;
+            *reinterpret_cast<uint4*>(args().x_out + xpk_index(r, k, 1)) = *reinterpret_cast<const uint4*>(xs + r * K + k);
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------------------------------ attention of a (row, head)
+// Eight waves, tiles wave, wave + 8, .. of 32 keys each (k_attn_decode's); NJ tiles a wave at most, all in registers before the query is there.  The products, the running maximum over the
+// tiles and the order of the sums are k_attn_cross's.
+template <int NJ, bool SELF>
+__device__ __forceinline__ void attention(unsigned char* smem, int item, int tid, unsigned near_at, unsigned q_at, unsigned out_at, unsigned exch_layer, unsigned tag) {
+    const WsParams& p = args();
+    const bool hasty = p.limit == 0;
+    const int L = p.L, d = p.d;
+    const float scale = p.scale;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g4 = lane >> 4, d0 = lane & 15;
+    const int b = item / p.H, h = item - b * p.H, S = SELF ? p.Smax : p.Spad;
+    unsigned char* own = smem + wave * ATT_WAVE;
+    bf16_t* strip = reinterpret_cast<bf16_t*>(own);
+    float *sc = reinterpret_cast<float*>(own + ATT_SC), *ps = reinterpret_cast<float*>(own + ATT_PS);
+    bf16_t *ph = reinterpret_cast<bf16_t*>(own + ATT_PH), *pl = reinterpret_cast<bf16_t*>(own + ATT_PL);
+    float* part = reinterpret_cast<float*>(smem + WAVES * ATT_WAVE);        // [WAVES][D + 2]
+    const int pos = SELF ? p.pos[b] : 0;
+    const bool live = p.active[b] != 0;
+    const int kv_len = SELF ? pos + 1 : p.cross_len, n_tiles = (kv_len + 31) >> 5;
+    const size_t head = ((size_t)b * p.H + h) * S * D;
+    bf16x8_t ka[NJ][2][2], va[NJ][4];
+    auto load = [&](int li) {
+        const WsParams& p = args();
+        const bf16x8_t* kb = reinterpret_cast<const bf16x8_t*>((SELF ? p.self_k + p.self_layer * li : p.cross_k + p.cross_layer * li) + head) + lane;
+        const bf16x8_t* vb = reinterpret_cast<const bf16x8_t*>((SELF ? p.self_v + p.self_layer * li : p.cross_v + p.cross_layer * li) + head) + lane;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int tile = min(wave + j * WAVES, n_tiles - 1);              // (a wave with fewer tiles: one that it does not use)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) ka[j][c >> 1][c & 1] = __builtin_nontemporal_load(kb + ((size_t)tile * 4 + c) * 64);
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) va[j][dt] = __builtin_nontemporal_load(vb + ((size_t)tile * 4 + dt) * 64);
+        }
+        asm volatile("" ::: "memory");
+    };
+    load(0);
+    for (int li = 0; li < L; ++li) {
+        const WsParams& p = args();
+        unsigned char* now = p.exch + (size_t)exch_layer * li;
+        constexpr int NG = SELF ? 2 : 1;
+        uint32_t v[NG];
+        if ((!SELF || li > 0) && !await(hasty, now - (SELF ? exch_layer : 0u) + near_at, tag, lane)) return;
+        const unsigned char* from = now + q_at + (size_t)b * (SELF ? 3 : 1) * d * 4 + h * D * 4;
+        // q | k | v of the head, 32 granules each; the cross-attention: q
+        if (!gather<NG>(hasty, v, tag, lane, [&](int i) {
+                const int g = min(lane + 64 * i, SELF ? 95 : 31);
+                return from + (size_t)(g >> 5) * d * 4 + (g & 31) * 8;
+            })) return;
+#pragma unroll
+        for (int i = 0; i < NG; ++i)
+            if (lane + 64 * i < (SELF ? 96 : 32)) reinterpret_cast<uint32_t*>(strip)[lane + 64 * i] = v[i];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        bf16x8_t qf[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(strip + c * 32 + g4 * 8);
+        if (SELF && live) {
+            // the new key, in the registers of the wave whose tile it is and in the cache
+            const int tile = pos >> 5, pr = pos & 31, prow = ((pr >> 3) << 2) | (pr & 3), half = (pr >> 2) & 1;
+            if ((tile & (WAVES - 1)) == wave) {
+                const int jn = tile / WAVES;
+                bf16x8_t* kc = reinterpret_cast<bf16x8_t*>(p.self_k + p.self_layer * li + head) + ((size_t)tile * 2 + half) * 2 * 64 + lane;
+                bf16_t* vc = p.self_v + p.self_layer * li + head;
+                if (d0 == prow) {
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const bf16x8_t kn = *reinterpret_cast<const bf16x8_t*>(strip + D + c * 32 + g4 * 8);
+                        kc[c * 64] = kn;
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+                            if (j == jn) { if (half) ka[j][1][c] = kn; else ka[j][0][c] = kn; }
+                    }
+                }
+                if (g4 == (pr >> 3)) {
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt) {
+                        const bf16_t vn = strip[2 * D + dt * 16 + d0];
+                        vc[(((size_t)tile * 4 + dt) * 64 + lane) * 8 + (pr & 7)] = vn;
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                            for (int e = 0; e < 8; ++e)
+                                if (j == jn && e == (pr & 7)) va[j][dt][e] = (short)vn;
+                    }
+                }
+            }
+        }
+        // Scores stand in all sixteen columns: through LDS a lane gets one key of every second tile, and gives the probabilities back (sixteen times the vector work otherwise:
+        // 4.9 us at six tiles a wave)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            f32x4_t S0 = (f32x4_t){0.f, 0.f, 0.f, 0.f}, S1 = S0;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][0][c], qf[c], S0, 0, 0, 0);
+                S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][1][c], qf[c], S1, 0, 0, 0);
+            }
+            if (d0 == 0) { *reinterpret_cast<f32x4_t*>(sc + j * 32 + g4 * 8) = S0; *reinterpret_cast<f32x4_t*>(sc + j * 32 + g4 * 8 + 4) = S1; }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (LDS operations of one wave execute in order)
+        float m_run = -INFINITY, l_run = 0.0f, alpha[NJ], x[NJ / 2], mx[NJ / 2];
+        const int up = lane >> 5;
+#pragma unroll
+        for (int i = 0; i < NJ / 2; ++i) {
+            const float v = sc[i * 64 + lane] * scale;
+            x[i] = (wave + (2 * i + up) * WAVES) * 32 + (lane & 31) < kv_len ? v : -INFINITY;
+            mx[i] = x[i];
+        }
+#pragma unroll
+        for (int k = 1; k < 32; k <<= 1)
+#pragma unroll
+            for (int i = 0; i < NJ / 2; ++i) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], k, 64));
+#pragma unroll
+        for (int i = 0; i < NJ / 2; ++i) {
+            const float m0 = fmaxf(m_run, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx[i]), 0)));
+            alpha[2 * i] = __expf(m_run - m0);
+            const bool two = wave + (2 * i + 1) * WAVES < n_tiles;         // (a group of five)
+            const float m1 = two ? fmaxf(m0, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx[i]), 32))) : m0;
+            alpha[2 * i + 1] = __expf(m0 - m1);
+            m_run = wave + 2 * i * WAVES < n_tiles ? m1 : m_run;
+            const float pe = __expf(x[i] - (up ? m1 : m0));
+            const bf16_t hb = f32_to_bf16(pe);
+            sc[i * 64 + lane] = pe;
+            ph[i * 64 + lane] = hb;
+            pl[i * 64 + lane] = f32_to_bf16(pe - bf16_to_f32(hb));
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (lane < NJ * 4) {
+            const f32x4_t a = *reinterpret_cast<const f32x4_t*>(sc + lane * 8), c = *reinterpret_cast<const f32x4_t*>(sc + lane * 8 + 4);
+            float psum = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) psum += e < 4 ? a[e & 3] : c[e & 3];
+            ps[lane] = psum;
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        f32x4_t O[4];
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) O[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            if (wave + j * WAVES < n_tiles) {
+                l_run = l_run * alpha[j] + ps[j * 4 + g4];
+                const bf16x8_t fh = *reinterpret_cast<const bf16x8_t*>(ph + j * 32 + g4 * 8), fl = *reinterpret_cast<const bf16x8_t*>(pl + j * 32 + g4 * 8);   // P in bf16 hi + lo parts
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) {
+                    f32x4_t o = O[dt];
+                    o[0] *= alpha[j];                                       // (row 0 of O is read, the others are copies without their factors)
+                    o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh, va[j][dt], o, 0, 0, 0);
+                    O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl, va[j][dt], o, 0, 0, 0);
+                }
+            }
+        l_run += __shfl_xor(l_run, 16, 64);
+        l_run += __shfl_xor(l_run, 32, 64);
+        if (g4 == 0) {
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) part[wave * (D + 2) + dt * 16 + d0] = O[dt][0];
+            if (d0 < 2) part[wave * (D + 2) + D + d0] = d0 ? l_run : m_run;
+        }
+        bar();
+        if (wave == 0) {
+            float M = -INFINITY, num = 0.0f, den = 0.0f;
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) M = fmaxf(M, part[w * (D + 2) + D]);
+#pragma unroll
+            for (int w = 0; w < WAVES; ++w) {
+                const float f = __expf(part[w * (D + 2) + D] - M);
+                num += f * part[w * (D + 2) + lane];
+                den += f * part[w * (D + 2) + D + 1];
+            }
+            const uint32_t o = live ? f32_to_bf16(num / den) : 0u, next = __shfl_xor(o, 1, 64);
+            if (!(lane & 1)) granule(now + out_at + ((size_t)b * d + h * D + lane) * 4, o | next << 16, tag);
+        }
+        bar();
+        if (li + 1 < L) load(li + 1);
+    }
+}
+
+__global__ void __launch_bounds__(THREADS, 2) k_whisper_step(WsParams) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int blk = blockIdx.x, tid = threadIdx.x;
+    const Exch ex = exch_layout(args().d, args().ff, args().rows);
+    const unsigned tag = args().sync[SYNC_TAG] + 1;
+    if (blk >= args().cross_first) attention<CJ, false>(smem, blk - args().cross_first, tid, ex.h1, ex.cq, ex.ca, ex.layer, tag);
+    else if (blk >= args().self_first) attention<SJ, true>(smem, blk - args().self_first, tid, ex.h2, ex.q, ex.at, ex.layer, tag);
+    else if (blk >= args().role[WS_FC2].first) matrix<WS_FC2, LN_NONE, TO_RESID>(smem, blk - args().role[WS_FC2].first, tid, ex.hb, ex.act, ex.h2, ex.hb, ex.layer, tag);
+    else if (blk >= args().role[WS_FC1].first) matrix<WS_FC1, LN_WAVE, TO_GELU>(smem, blk - args().role[WS_FC1].first, tid, ex.ca, ex.hb, ex.act, 0, ex.layer, tag);
+    else if (blk >= args().role[WS_CO].first) matrix<WS_CO, LN_NONE, TO_RESID>(smem, blk - args().role[WS_CO].first, tid, ex.cq, ex.ca, ex.hb, ex.h1, ex.layer, tag);
+    else if (blk >= args().role[WS_CQ].first) matrix<WS_CQ, LN_SLICES, TO_T>(smem, blk - args().role[WS_CQ].first, tid, ex.at, ex.h1, ex.cq, 0, ex.layer, tag);
+    else if (blk >= args().role[WS_O].first) matrix<WS_O, LN_NONE, TO_RESID>(smem, blk - args().role[WS_O].first, tid, ex.q, ex.at, ex.h1, ex.h2, ex.layer, tag);
+    else matrix<WS_QKV, LN_GLUE, TO_T>(smem, blk, tid, ex.act, ex.h2, ex.q, 0, ex.layer, tag);
+    if (blk == 0 && tid == 0) {
+        const WsParams& p = args();                               // (the block that ends last: it waits for the others' values)
+        p.sync[SYNC_TAG] = tag;
+        if (p.sync[SYNC_LOCKED]) {
+            p.sync[SYNC_LOCKED] = 0;
+            __hip_atomic_store(p.lock, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+int k_max(const WsParams& p) {
+    int k = 0;
+    for (const WsRole& r : p.role) k = std::max(k, r.KT * 32);
+    return k;
+}
+// Pieces to waves, the longest first, each to the wave with the least: fragments of the fullest wave; out: WAVES x NF entries of
+// K-tile | tile << 8 | last of its piece << 12 | 1 << 13 | piece << 16 (0: none)
+int ws_table(const WsRole& r, int per, unsigned* out) {
+    struct Piece { int unit, tile, k0, k1; };
+    std::vector<Piece> v;
+    const int P = r.S * r.ksb;
+    for (int u = 0; u < per * P; ++u) {
+        const int pc = u % P, ks = pc / r.ksb, w = pc % r.ksb, a = r.KT * ks / r.S, len = r.KT * (ks + 1) / r.S - a;
+        v.push_back({u, u / P, a + len * w / r.ksb, a + len * (w + 1) / r.ksb});
+    }
+    std::stable_sort(v.begin(), v.end(), [](const Piece& a, const Piece& b) { return a.k1 - a.k0 > b.k1 - b.k0; });
+    int n[WAVES] = {};
+    for (const Piece& c : v) {
+        const int w = (int)(std::min_element(n, n + WAVES) - n);
+        for (int k = c.k0; k < c.k1; ++k, ++n[w])
+            if (out && n[w] < NF) out[w * NF + n[w]] = (unsigned)k | (unsigned)c.tile << 8 | (k + 1 == c.k1 ? 1u << 12 : 0u) | 1u << 13 | (unsigned)c.unit << 16;
+    }
+    return *std::max_element(n, n + WAVES);
+}
+}
+
+size_t ws_exch_bytes(const WsParams& p) { return (size_t)exch_layout(p.d, p.ff, p.rows).layer * p.L; }
+
+bool ws_plan(WsParams& p, int device) {
+    if (p.rows < 1 || p.rows > MAX_ROWS || p.L < 1 || p.d % 64 || p.d > 256 * LNG || p.d != p.H * D || p.ff % 32 || p.Smax > 32 * WAVES * SJ || p.Smax % 32 ||
+        p.cross_len > 32 * WAVES * CJ || p.cross_len <= 32 * WAVES * (CJ - 1) || p.Spad < (p.cross_len + 31) / 32 * 32) return false;
+    for (WsRole& r : p.role) {
+        if (r.KT > 255 || r.S < 1 || r.S > 8 || ws_table(r, 1, nullptr) > NF) return false;
+        r.per = 1;
+    }
+    const int attn = 2 * p.rows * p.H;
+    for (;;) {                                                              // more tiles a block, where that makes the shortest block, until a compute unit has one block
+        int total = attn, best = -1, cost = 0;
+        for (int i = 0; i < WS_ROLES; ++i) {
+            WsRole& r = p.role[i];
+            r.blocks = (r.tiles + r.per - 1) / r.per;
+            total += r.blocks;
+            const int f = r.blocks > 1 ? ws_table(r, r.per + 1, nullptr) : NF + 1;
+            if (r.per < 8 && f <= NF && (best < 0 || f < cost)) { best = i; cost = f; }
+        }
+        if (total <= MAX_BLOCKS) break;
+        if (best < 0) return false;
+        ++p.role[best].per;
+    }
+    int at = 0;
+    p.units = 0;
+    for (WsRole& r : p.role) {
+        r.first = at; at += r.blocks;
+        p.units = std::max(p.units, r.per * r.S * r.ksb);
+        if (r.per * 8 * p.rows > THREADS) return false;
+    }
+    p.self_first = at; at += p.rows * p.H;
+    p.cross_first = at; at += p.rows * p.H;
+    p.blocks = at;
+    p.k_max = k_max(p);
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return false;
+    return p.blocks <= cus && lds_layout(p.k_max, p.rows, p.units).total <= 64 * 1024;
+}
+
+std::vector<unsigned> ws_tables(const WsParams& p) {
+    std::vector<unsigned> t(WS_ROLES * WAVES * NF, 0u);
+    for (int i = 0; i < WS_ROLES; ++i) ws_table(p.role[i], p.role[i].per, t.data() + i * WAVES * NF);
+    return t;
+}
+
+void launch_whisper_step(const WsParams& p, hipStream_t s) {
+    launch_step_lock(p.lock, p.sync, p.fail, s);
+    hipLaunchKernelGGL(k_whisper_step, dim3(p.blocks), dim3(THREADS), lds_layout(p.k_max, p.rows, p.units).total, s, p);
+}

@@ -1,0 +1,84 @@
+"""-m gpu: a Whisper decoder step's layers as one launch (csrc/whisper_step.hip): the bits of the launch chain - token ids, and the logits behind the caches it leaves - over widths, depth,
+rows, splits of K, positions past a wave's first tile of keys, rows that end, a launch that runs out of time, two handles at once."""
+import threading
+
+import numpy as np
+import pytest
+
+import mlx_audio_swift_amd as mas
+
+pytestmark = pytest.mark.gpu
+PROMPT = [690, 691, 692, 693]
+
+
+def model(d, layers, vocab=700):
+    cfg = mas.WhisperConfig(vocab_size=vocab, num_mel_bins=80, d_model=d, encoder_layers=1, encoder_attention_heads=d // 64, encoder_ffn_dim=d, decoder_layers=layers,
+                            decoder_attention_heads=d // 64, decoder_ffn_dim=4 * d)
+    return mas.WhisperModel.synthetic(cfg, seed=11)
+
+
+def run(m, rows, tokens, eot=699, seed=3):
+    rng = np.random.default_rng(seed)
+    wins = [(0.1 * rng.standard_normal(16000 * (1 + b))).astype(np.float32) for b in range(rows)]
+    ids = m.transcribe_windows(wins, PROMPT, mas.STTGenerateParameters(max_tokens=tokens, temperature=0.0, seed=5, eot_id=eot, timestamp_begin=695))
+    return ids, m.decoder_forward([5 + b for b in range(rows)])
+
+
+def same(a, b):
+    return a[0] == b[0] and np.array_equal(a[1], b[1]) and np.isfinite(a[1]).all()
+
+
+# one tile of columns a block and several; one, two, three and five slabs; the last block of a matrix with fewer tiles; 1280 columns at one row: every compute unit
+@pytest.mark.parametrize("d,layers,rows", [(128, 2, 1), (384, 4, 1), (384, 2, 3), (512, 2, 4), (768, 2, 2), (768, 3, 3), (1024, 2, 1), (1024, 1, 4), (1280, 2, 1)])
+def test_bits_of_the_launch_chain(monkeypatch, d, layers, rows):
+    m = model(d, layers)
+    monkeypatch.setenv("MIS_WHISPER_STEP", "0")
+    chain = run(m, rows, 36)
+    monkeypatch.delenv("MIS_WHISPER_STEP")
+    for _ in range(2):
+        assert same(run(m, rows, 36), chain)
+
+
+def test_positions_past_the_first_tiles(monkeypatch):
+    m = model(384, 2)
+    monkeypatch.setenv("MIS_WHISPER_STEP", "0")
+    chain = run(m, 2, 330)
+    monkeypatch.delenv("MIS_WHISPER_STEP")
+    assert same(run(m, 2, 330), chain)
+
+
+def test_a_row_alone_and_among_others():
+    m = model(384, 2)
+    ids, logits = run(m, 1, 20)
+    for rows in (2, 4, 6):                                                 # six: the launch chain
+        more, lm = run(m, rows, 20)
+        assert more[0] == ids[0] and np.array_equal(lm[0], logits[0])
+
+
+def test_a_row_that_ends(monkeypatch):
+    m = model(384, 2)
+    full = run(m, 2, 24)[0]
+    ends = [t for t in full[1][6:] if t not in full[0]][:1] or [full[1][6]]
+    monkeypatch.setenv("MIS_WHISPER_STEP", "0")
+    chain = run(m, 2, 24, eot=ends[0])[0]
+    monkeypatch.delenv("MIS_WHISPER_STEP")
+    assert run(m, 2, 24, eot=ends[0])[0] == chain and chain != full
+
+
+def test_out_of_time_runs_on_the_chain(monkeypatch):
+    m = model(384, 2)
+    want = run(m, 2, 20)
+    monkeypatch.setenv("MIS_WHISPER_STEP_US", "0")                         # the first poll in vain ends the launch
+    got = run(m, 2, 20)
+    monkeypatch.delenv("MIS_WHISPER_STEP_US")
+    assert same(got, want) and same(run(m, 2, 20), want)
+
+
+def test_two_handles_at_once():
+    ms = [model(384, 2), model(768, 2)]
+    want = [run(m, 2, 60) for m in ms]
+    got = [[], []]
+    ts = [threading.Thread(target=lambda i=i: got[i].extend(run(ms[i], 2, 60) for _ in range(3))) for i in range(2)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert all(same(g, want[i]) for i in range(2) for g in got[i])
