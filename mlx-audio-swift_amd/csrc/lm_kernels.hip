@@ -1724,7 +1724,7 @@ __global__ void __launch_bounds__(512) k_attn_decode(AttnParams p) {
                 c = bf16_round_f32(c); s = bf16_round_f32(s);
                 r1 = f32_to_bf16(bf16_round_f32(x1 * c) + bf16_round_f32(-x2 * s));
                 r2 = f32_to_bf16(bf16_round_f32(x2 * c) + bf16_round_f32(x1 * s));
-            } else { r1 = f32_to_bf16(fmaf(x1, c, -(x2 * s))); r2 = f32_to_bf16(fmaf(x1, s, x2 * c)); }
+            } else { r1 = f32_to_bf16(fmaf(x1, c, -(x2 * s))); r2 = f32_to_bf16(fmaf(x2, c, x1 * s)); }
         } else { r1 = f32_to_bf16(x1); r2 = f32_to_bf16(x2); }      // Whisper: learned positions, no rotary
         if (hh < G) { qs[hh * D + i] = r1; qs[hh * D + i + D / 2] = r2; }
         else {
@@ -2365,7 +2365,7 @@ __global__ void __launch_bounds__(512) k_attn_decode2(AttnParams p) {
                     const float x1 = x[c][e >> 2][e & 3], x2 = x[c + 2][e >> 2][e & 3];
                     const float cs = rc[c][e >> 2][e & 3], sn = rs[c][e >> 2][e & 3];
                     out[c][e] = (short)f32_to_bf16(fmaf(x1, cs, -(x2 * sn)));                 // (k_attn_decode rounds the other product of the second one)
-                    out[c + 2][e] = (short)f32_to_bf16(fmaf(x2, cs, x1 * sn));
+                    out[c + 2][e] = (short)f32_to_bf16(fmaf(x1, sn, x2 * cs));
                 }
         };
         bf16x8_t qf[4];

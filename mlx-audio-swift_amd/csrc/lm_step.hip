@@ -446,8 +446,8 @@ __device__ __forceinline__ bool attention(Ctx& c, const unsigned char* xq, unsig
                 const float x1 = x[k][e >> 2][e & 3], x2 = x[k + 2][e >> 2][e & 3];
                 const float cs = rc[k][e >> 2][e & 3], sn = rs[k][e >> 2][e & 3];
                 out[k][e] = (short)f32_to_bf16(fmaf(x1, cs, -(x2 * sn)));
-                const float a = p.schedule2 ? x1 * sn : x2 * cs;                              // the product that k_attn_decode2, or k_attn_decode, rounds
-                out[k + 2][e] = (short)f32_to_bf16(fmaf(p.schedule2 ? x2 : x1, p.schedule2 ? cs : sn, a));
+                const float a = p.schedule2 ? x2 * cs : x1 * sn;                              // the product that k_attn_decode2, or k_attn_decode, rounds
+                out[k + 2][e] = (short)f32_to_bf16(fmaf(p.schedule2 ? x1 : x2, p.schedule2 ? sn : cs, a));
             }
     };
     bf16x8_t qf[4];
