@@ -50,6 +50,7 @@ struct mis_whisper {
     DevBuf<float> qkv_part, part, e_buf, logits_f32;
     DevBuf<SamplerScratch> scratch;
     // a step's layers as one launch (whisper_step.hip)
+    WsParams step{};                       // the request's
     DevBuf<WsLayer> step_layers;
     DevBuf<unsigned char> step_exch;
     DevBuf<unsigned> step_sync, step_table;
@@ -645,15 +646,13 @@ static bool step_begin(mis_whisper* c, bool alone) {
     c->step_sync.alloc(SYNC_WORDS);
     c->step_exch.zero(c->stream);                                          // (tags begin again)
     c->step_sync.zero(c->stream);
-    return true;
+    return step_params(c, c->step);                                        // (with the buffers)
 }
 static void enqueue_step(mis_whisper* c, const int32_t* ids) {
-    WsParams p{};
-    MIS_REQUIRE(step_params(c, p), MIS_ERR_GENERATION_FAILED, "internal: the plan of a decoder step changed under way");
     if (ids)
         launch_whisper_embed_ln(c->emb, c->dec_pos, ids, c->active.p, c->pos_cur.p, c->pos_next.p, c->dec[0].ln1w, c->dec[0].ln1b, c->h.p, c->x.p, c->d, c->V, c->cfg.max_target_positions,
                                 c->batch, c->Mpad, c->stream);
-    launch_whisper_step(p, c->stream);
+    launch_whisper_step(c->step, c->stream);
 }
 static void enqueue_vocab(mis_whisper* c) {
     launch_gemm_skinny(EPI_BF16, 2, 1, c->emb_packed, c->x.p, c->logits.p, c->Vpad / 16, c->d / 32, 1, c->Vpad, c->Mpad, c->stream);

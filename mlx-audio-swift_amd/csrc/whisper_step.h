@@ -10,8 +10,11 @@ enum { WS_QKV, WS_O, WS_CQ, WS_CO, WS_FC1, WS_FC2, WS_ROLES };
 struct WsLayer { const bf16_t *w[WS_ROLES], *b[WS_ROLES], *lnw[3], *lnb[3]; };
 // column tiles of 16, K cut as the launch chain cuts it (slabs, then the waves of an item); `per` tiles a block, blocks [first, first + blocks)
 struct WsRole { int tiles, KT, S, ksb, per, first, blocks; };
+// what a block has for all layers: one matrix or attention; tiles of every matrix, or both attentions of a (row, head)
+enum { WS_ALL, WS_SHARED };
 struct WsParams {
     WsRole role[WS_ROLES];
+    int what;
     int self_first, cross_first, blocks;                                  // a block per (row, head)
     const WsLayer* layers;
     const unsigned* table;       // ws_tables

@@ -28,8 +28,9 @@ def same(a, b):
     return a[0] == b[0] and np.array_equal(a[1], b[1]) and np.isfinite(a[1]).all()
 
 
-# one tile of columns a block and several; one, two, three and five slabs; the last block of a matrix with fewer tiles; 1280 columns at one row: every compute unit
-@pytest.mark.parametrize("d,layers,rows", [(128, 2, 1), (384, 4, 1), (384, 2, 3), (512, 2, 4), (768, 2, 2), (768, 3, 3), (1024, 2, 1), (1024, 1, 4), (1280, 2, 1)])
+# one tile of columns a block and several; one, two, three and five slabs; the last block of a matrix with fewer tiles; 1280 columns at one row: every compute unit;
+# eight rows, a norm on each wave; blocks of all matrices (from 1024 columns or 768 and five rows on): one layer, few rows and many blocks, many rows and few blocks
+@pytest.mark.parametrize("d,layers,rows", [(384, 2, 5), (384, 4, 8), (768, 2, 8), (1024, 2, 6), (1280, 1, 4), (1280, 3, 3), (1280, 2, 5), (1280, 3, 8), (128, 2, 1), (384, 4, 1), (384, 2, 3), (512, 2, 4), (768, 2, 2), (768, 3, 3), (1024, 2, 1), (1024, 1, 4), (1280, 2, 1)])
 def test_bits_of_the_launch_chain(monkeypatch, d, layers, rows):
     m = model(d, layers)
     monkeypatch.setenv("MIS_WHISPER_STEP", "0")
@@ -40,45 +41,50 @@ def test_bits_of_the_launch_chain(monkeypatch, d, layers, rows):
 
 
 def test_positions_past_the_first_tiles(monkeypatch):
-    m = model(384, 2)
-    monkeypatch.setenv("MIS_WHISPER_STEP", "0")
-    chain = run(m, 2, 330)
-    monkeypatch.delenv("MIS_WHISPER_STEP")
-    assert same(run(m, 2, 330), chain)
+    for d, rows in ((384, 2), (1280, 4)):
+        m = model(d, 2)
+        monkeypatch.setenv("MIS_WHISPER_STEP", "0")
+        chain = run(m, rows, 330)
+        monkeypatch.delenv("MIS_WHISPER_STEP")
+        assert same(run(m, rows, 330), chain)
 
 
-def test_a_row_alone_and_among_others():
-    m = model(384, 2)
+@pytest.mark.parametrize("d,more_rows", [(384, (2, 4, 6, 9)), (1280, (2, 5))])    # nine: the launch chain
+def test_a_row_alone_and_among_others(d, more_rows):
+    m = model(d, 2)
     ids, logits = run(m, 1, 20)
-    for rows in (2, 4, 6):                                                 # six: the launch chain
+    for rows in more_rows:
         more, lm = run(m, rows, 20)
         assert more[0] == ids[0] and np.array_equal(lm[0], logits[0])
 
 
-def test_a_row_that_ends(monkeypatch):
-    m = model(384, 2)
-    full = run(m, 2, 24)[0]
+@pytest.mark.parametrize("d,rows", [(384, 2), (1280, 4)])
+def test_a_row_that_ends(monkeypatch, d, rows):
+    m = model(d, 2)
+    full = run(m, rows, 24)[0]
     ends = [t for t in full[1][6:] if t not in full[0]][:1] or [full[1][6]]
     monkeypatch.setenv("MIS_WHISPER_STEP", "0")
-    chain = run(m, 2, 24, eot=ends[0])[0]
+    chain = run(m, rows, 24, eot=ends[0])[0]
     monkeypatch.delenv("MIS_WHISPER_STEP")
-    assert run(m, 2, 24, eot=ends[0])[0] == chain and chain != full
+    assert run(m, rows, 24, eot=ends[0])[0] == chain and chain != full
 
 
-def test_out_of_time_runs_on_the_chain(monkeypatch):
-    m = model(384, 2)
-    want = run(m, 2, 20)
+@pytest.mark.parametrize("d,rows", [(384, 2), (1280, 4)])
+def test_out_of_time_runs_on_the_chain(monkeypatch, d, rows):
+    m = model(d, 2)
+    want = run(m, rows, 20)
     monkeypatch.setenv("MIS_WHISPER_STEP_US", "0")                         # the first poll in vain ends the launch
-    got = run(m, 2, 20)
+    got = run(m, rows, 20)
     monkeypatch.delenv("MIS_WHISPER_STEP_US")
-    assert same(got, want) and same(run(m, 2, 20), want)
+    assert same(got, want) and same(run(m, rows, 20), want)
 
 
-def test_two_handles_at_once():
-    ms = [model(384, 2), model(768, 2)]
-    want = [run(m, 2, 60) for m in ms]
+@pytest.mark.parametrize("d,rows", [(768, 2), (1280, 4)])
+def test_two_handles_at_once(d, rows):
+    ms, rows = [model(384, 2), model(d, 2)], [2, rows]
+    want = [run(m, r, 60) for m, r in zip(ms, rows)]
     got = [[], []]
-    ts = [threading.Thread(target=lambda i=i: got[i].extend(run(ms[i], 2, 60) for _ in range(3))) for i in range(2)]
+    ts = [threading.Thread(target=lambda i=i: got[i].extend(run(ms[i], rows[i], 60) for _ in range(3))) for i in range(2)]
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert all(same(g, want[i]) for i in range(2) for g in got[i])
