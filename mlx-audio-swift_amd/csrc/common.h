@@ -104,18 +104,26 @@ static inline hipError_t copy_now(void* dst, const void* src, size_t n, hipMemcp
 
 // Large copies between device memory and the caller's pageable memory, through a pinned ring with the host side spread over threads: one thread alone
 // writes fresh pages (allocated and cleared as they are touched) at a fifth of the link's rate.  Belongs to a handle (one call in flight); reserve()
-// where the handle is finalized.  Without a ring, for small copies and for device or pinned memory: one plain asynchronous copy.  Both wait for the copy.
+// where the handle is finalized.  Without a ring and for device or pinned memory: one plain asynchronous copy.  Both wait for the copy.
+// Small ones (up to SMALL together) go through the pinned memory by a kernel: a copy command waits on the host for the stream to drain (pageable memory) or changes to a copy engine
+// and back, 15 - 30 us each.  A SNAC encode's four results: 47 -> 9 us behind its last kernel.
 struct HostRing {
     static constexpr int SLOTS = 8;
-    static constexpr size_t SLOT = (size_t)2 << 20, MIN = (size_t)4 << 20;
-    PinnedBuf<uint8_t> buf;
+    static constexpr size_t SLOT = (size_t)2 << 20, MIN = (size_t)4 << 20, SMALL = (size_t)1 << 20, INPUT = (size_t)64 << 10;
+    static constexpr int PIECES = 8;
+    struct Piece { void* to; const void* from; size_t bytes; };
+    PinnedBuf<uint8_t> buf;                                                // SLOTS x SLOT for the large copies, or nothing; SMALL + INPUT for the small ones
+    size_t held = 0;
     hipEvent_t ev[SLOTS] = {};
     HostRing() {}
     HostRing(const HostRing&) = delete;
     HostRing& operator=(const HostRing&) = delete;
     ~HostRing();
-    void reserve();
+    void reserve(bool large = true);
     static bool pageable(const void* p);
+    // up to PIECES small copies at once; false: not small, or not between the device and pageable memory, and nothing done
+    bool out_small(const Piece* p, int n, hipStream_t s);                  // waits
+    bool in_small(const Piece* p, int n, hipStream_t s);                   // does not: once between two waits for the stream
     void out(void* host, const void* dev, size_t n, hipStream_t s);
     void in(void* dev, const void* host, size_t n, hipStream_t s);
 private:

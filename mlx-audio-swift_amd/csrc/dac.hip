@@ -40,6 +40,8 @@ struct mis_dac {
     DevBuf<float> buf[3];
     CodecPack pack;                      // split-bf16 weight fragments + activation scratch (codec_bf3.hip)
     DevBuf<int32_t> codes_dev;
+    DevBuf<float> wav;                   // a decode's samples (allocated on each call they were 40 us, and given back a wait for the device)
+    HostRing ring;
     // encoder (optional: built when the checkpoint carries encoder.* / in_proj tensors)
     bool has_encoder = false;
     int enc_dim = 0, hop = 1;
@@ -284,6 +286,7 @@ extern "C" mis_status mis_dac_finalize(mis_dac* c) {
     c->arena.alloc(arena.size());
     HIP_CHECK(hipMemcpy(c->arena.p, arena.data(), arena.size() * 4, hipMemcpyHostToDevice));
     c->raw.clear(); c->raw_shape.clear();
+    c->ring.reserve(false);
     c->finalized = true;
     MIS_API_END
 }
@@ -442,16 +445,15 @@ extern "C" mis_status mis_dac_decode_codes(mis_dac* c, const int32_t* codes, int
     MIS_REQUIRE(c && codes && wav_out && batch >= 1 && T >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
     const int64_t n = mis_dac_num_samples(c, T);
-    DevBuf<float> wav;
     codec_run(c->pack, [&] {
         int C; int64_t Tt;
         c->codes_dev.alloc((size_t)batch * c->cfg.n_codebooks * T);
-        HIP_CHECK(hipMemcpyAsync(c->codes_dev.p, codes, (size_t)batch * c->cfg.n_codebooks * T * 4, hipMemcpyDefault, c->stream));
-        wav.alloc((size_t)batch * n);
-        dac_run(c, c->codes_dev.p, batch, T, wav.p, n, 0, &C, &Tt);
+        const HostRing::Piece in{c->codes_dev.p, codes, (size_t)batch * c->cfg.n_codebooks * T * 4};
+        if (!c->ring.in_small(&in, 1, c->stream)) HIP_CHECK(hipMemcpyAsync(in.to, in.from, in.bytes, hipMemcpyDefault, c->stream));
+        c->wav.alloc((size_t)batch * n);
+        dac_run(c, c->codes_dev.p, batch, T, c->wav.p, n, 0, &C, &Tt);
     });
-    HIP_CHECK(hipMemcpyAsync(wav_out, wav.p, (size_t)batch * n * 4, hipMemcpyDefault, c->stream));
-    HIP_CHECK(hipStreamSynchronize(c->stream));
+    c->ring.out(wav_out, c->wav.p, (size_t)batch * n * 4, c->stream);
     MIS_API_END
 }
 extern "C" mis_status mis_dac_debug_tap(mis_dac* c, const int32_t* codes, int batch, int T, int block, float* out, int64_t capacity,

@@ -230,10 +230,58 @@ mis_dtype dtype_from_safetensors(const std::string& s) {
 HostRing::~HostRing() {
     for (auto& e : ev) if (e) (void)hipEventDestroy(e);
 }
-void HostRing::reserve() {
+void HostRing::reserve(bool large) {
     if (buf.p) return;
-    for (auto& e : ev) if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    buf.alloc(SLOTS * SLOT);
+    if (large) for (auto& e : ev) if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    const size_t n = (large ? SLOTS * SLOT : 0) + SMALL + INPUT;
+    buf.alloc(n);
+    held = n;
+}
+// block x, x + gridDim.x, ..: 16 bytes a thread; the last bytes one by one
+struct CopyPieces { HostRing::Piece p[HostRing::PIECES]; };
+static __global__ void __launch_bounds__(256) k_copy_pieces(CopyPieces c) {
+    const HostRing::Piece p = c.p[blockIdx.y];
+    const size_t units = p.bytes / 16, i0 = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = i0; i < units; i += (size_t)gridDim.x * 256) reinterpret_cast<uint4*>(p.to)[i] = reinterpret_cast<const uint4*>(p.from)[i];
+    if (i0 < p.bytes % 16) reinterpret_cast<uint8_t*>(p.to)[units * 16 + i0] = reinterpret_cast<const uint8_t*>(p.from)[units * 16 + i0];
+}
+static void copy_pieces(const CopyPieces& c, int n, hipStream_t s) {
+    size_t most = 0;
+    for (int i = 0; i < n; ++i) most = std::max(most, c.p[i].bytes);
+    hipLaunchKernelGGL(k_copy_pieces, dim3((unsigned)std::min<size_t>(64, (most / 16 + 255) / 256 + 1), n), dim3(256), 0, s, c);
+    HIP_CHECK(hipGetLastError());
+}
+bool HostRing::out_small(const Piece* p, int n, hipStream_t s) {
+    size_t total = 0;
+    if (!buf.p || n < 1 || n > PIECES) return false;
+    for (int i = 0; i < n; ++i) {
+        total += round_up(p[i].bytes, 16);
+        if (!p[i].bytes || total > SMALL || ((uintptr_t)p[i].from & 15) || !pageable(p[i].to)) return false;
+    }
+    CopyPieces c;
+    uint8_t* at = buf.p + held - INPUT - SMALL;
+    for (int i = 0; i < n; ++i) { c.p[i] = {at, p[i].from, p[i].bytes}; at += round_up(p[i].bytes, 16); }
+    copy_pieces(c, n, s);
+    HIP_CHECK(hipStreamSynchronize(s));
+    for (int i = 0; i < n; ++i) memcpy(p[i].to, c.p[i].to, p[i].bytes);
+    return true;
+}
+bool HostRing::in_small(const Piece* p, int n, hipStream_t s) {
+    size_t total = 0;
+    if (!buf.p || n < 1 || n > PIECES) return false;
+    for (int i = 0; i < n; ++i) {
+        total += round_up(p[i].bytes, 16);
+        if (!p[i].bytes || total > INPUT || ((uintptr_t)p[i].to & 15) || !pageable(p[i].from)) return false;
+    }
+    CopyPieces c;
+    uint8_t* at = buf.p + held - INPUT;
+    for (int i = 0; i < n; ++i) {
+        memcpy(at, p[i].from, p[i].bytes);
+        c.p[i] = {p[i].to, at, p[i].bytes};
+        at += round_up(p[i].bytes, 16);
+    }
+    copy_pieces(c, n, s);
+    return true;
 }
 bool HostRing::pageable(const void* p) {
     hipPointerAttribute_t a{};
@@ -242,13 +290,15 @@ bool HostRing::pageable(const void* p) {
 }
 void HostRing::out(void* host, const void* dev, size_t n, hipStream_t s) {
     if (n == 0) { HIP_CHECK(hipStreamSynchronize(s)); return; }
-    if (buf.p && n >= MIN && pageable(host)) { run((uint8_t*)host, (uint8_t*)const_cast<void*>(dev), n, true, s); return; }
+    const Piece p{host, dev, n};
+    if (n <= SMALL && out_small(&p, 1, s)) return;
+    if (ev[0] && buf.p && n >= MIN && pageable(host)) { run((uint8_t*)host, (uint8_t*)const_cast<void*>(dev), n, true, s); return; }
     HIP_CHECK(hipMemcpyAsync(host, dev, n, hipMemcpyDefault, s));
     HIP_CHECK(hipStreamSynchronize(s));
 }
 void HostRing::in(void* dev, const void* host, size_t n, hipStream_t s) {
     if (n == 0) return;
-    if (buf.p && n >= MIN && pageable(host)) { run((uint8_t*)const_cast<void*>(host), (uint8_t*)dev, n, false, s); return; }
+    if (ev[0] && buf.p && n >= MIN && pageable(host)) { run((uint8_t*)const_cast<void*>(host), (uint8_t*)dev, n, false, s); return; }
     HIP_CHECK(hipMemcpyAsync(dev, host, n, hipMemcpyDefault, s));
     HIP_CHECK(hipStreamSynchronize(s));
 }

@@ -1313,14 +1313,13 @@ static void snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_sa
     for (int i = 0; i < cf.n_codebooks; ++i) {
         MIS_REQUIRE(codes_out[i], MIS_ERR_INVALID_INPUT, "null argument");
         MIS_REQUIRE(T % cf.vq_strides[i] == 0, MIS_ERR_AUDIO_ENCODE, "internal: latent length not divisible by vq stride");
-        all_codes += (size_t)batch * (T / cf.vq_strides[i]);
+        all_codes += round_up((size_t)batch * (T / cf.vq_strides[i]), 4);
     }
     const bool one = cf.codebook_dim == 8;                                // one launch a level
     MIS_REQUIRE(cf.codebook_dim <= 64, MIS_ERR_INVALID_INPUT, "codebook_dim > 64 unsupported by the nearest-code kernel");
     if (!one) { c->vq_pool.alloc((size_t)batch * D * T); c->vq_ze.alloc((size_t)batch * cf.codebook_dim * T); }
     c->enc_codes.alloc(all_codes);
-    struct Result { void* to; const void* from; size_t bytes; };
-    std::vector<Result> results;
+    std::vector<HostRing::Piece> results;
     if (z_out) results.push_back({z_out, f1, (size_t)batch * D * T * 4});
     int32_t* codes = c->enc_codes.p;
     for (int i = 0; i < cf.n_codebooks; ++i) {
@@ -1346,22 +1345,12 @@ static void snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_sa
             if (!last) hipLaunchKernelGGL(k_vq_residual, dim3(cdiv(T, 256), D, batch), dim3(256), 0, s, f2, codes, table, D, (int)T, st);
         }
         results.push_back({codes_out[i], codes, (size_t)batch * Tm * 4});
-        codes += (size_t)batch * Tm;
+        codes += round_up((size_t)batch * Tm, 4);
     }
     HIP_CHECK(hipGetLastError());
-    // small results to pageable memory: side by side through the ring, one wait (copied one by one, each is a wait of its own)
-    size_t at = 0;
-    bool small = c->ring.buf.p != nullptr;
-    for (auto& r : results) { at += r.bytes; small = small && at < HostRing::MIN && HostRing::pageable(r.to); }
-    if (small) {
-        at = 0;
-        for (auto& r : results) { HIP_CHECK(hipMemcpyAsync(c->ring.buf.p + at, r.from, r.bytes, hipMemcpyDeviceToHost, s)); at += r.bytes; }
-        HIP_CHECK(hipStreamSynchronize(s));
-        at = 0;
-        for (auto& r : results) { memcpy(r.to, c->ring.buf.p + at, r.bytes); at += r.bytes; }
-    } else {
+    // one launch and one wait where they are small (copied one by one, each is a wait of its own)
+    if (!c->ring.out_small(results.data(), (int)results.size(), s))
         for (auto& r : results) c->ring.out(r.to, r.from, r.bytes, s);
-    }
     HIP_CHECK(hipGetLastError());
 }
 extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_samples, int32_t* const* codes_out, float* z_out) {
@@ -1622,16 +1611,19 @@ static void snac_stage_inputs(mis_snac* c, const int32_t* const* codes, int batc
     std::vector<size_t> offs(cf.n_codebooks);
     for (int i = 0; i < cf.n_codebooks; ++i) {
         offs[i] = total;
-        total += (size_t)batch * t_coarse * (cf.vq_strides[0] / cf.vq_strides[i]);
+        total += round_up((size_t)batch * t_coarse * (cf.vq_strides[0] / cf.vq_strides[i]), 4);
     }
     c->codes_ws.alloc(total);
+    std::vector<HostRing::Piece> from;
     dcodes.resize(cf.n_codebooks);
     for (int i = 0; i < cf.n_codebooks; ++i) {
         size_t n = (size_t)batch * t_coarse * (cf.vq_strides[0] / cf.vq_strides[i]);
         MIS_REQUIRE(codes[i], MIS_ERR_INVALID_INPUT, "codes[%d] is null", i);
-        HIP_CHECK(hipMemcpyAsync(c->codes_ws.p + offs[i], codes[i], n * sizeof(int32_t), hipMemcpyDefault, c->stream));
+        from.push_back({c->codes_ws.p + offs[i], codes[i], n * sizeof(int32_t)});
         dcodes[i] = c->codes_ws.p + offs[i];
     }
+    if (!c->ring.in_small(from.data(), (int)from.size(), c->stream))
+        for (auto& f : from) HIP_CHECK(hipMemcpyAsync(f.to, f.from, f.bytes, hipMemcpyDefault, c->stream));
     dnoise.clear();
     if (noise && cf.noise) {
         size_t tot = 0;
