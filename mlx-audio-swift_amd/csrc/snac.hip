@@ -410,17 +410,18 @@ __global__ void __launch_bounds__(256) k_snac_convt(GemmParams p) { snac_convt_b
 
 // ---- encoder kernels (Layers.swift:319-360, VQ.swift:47-120) ---------------------------------------------------------
 // first layer: conv k7 "same", 1 -> C
-// a thread owns a column and ENC_FIRST_CH channels: its seven samples are read once, the weights are scalar (one channel per thread: 29 -> 12.6 us for 48 x 151552)
+// a thread owns a column and ENC_FIRST_CH channels: its seven samples are read once, the weights are scalar (one channel per thread: 29 -> 12.6 us for 48 x 151552).  audio [batch][n]: what a
+// row is short of the T columns is zero (cleared in memory in front it was two launches, 20 us with what lies between them)
 #define ENC_FIRST_CH 16
 __global__ void __launch_bounds__(256) k_enc_first(const float* __restrict__ audio, float* __restrict__ y, const float* __restrict__ w /*[C][7]*/,
-                                                   const float* __restrict__ bias, int C, int T) {
+                                                   const float* __restrict__ bias, int C, int T, int n) {
     const int t = blockIdx.x * 256 + threadIdx.x, c0 = blockIdx.y * ENC_FIRST_CH, b = blockIdx.z;
-    const float* a = audio + (size_t)b * T;
+    const float* a = audio + (size_t)b * n;
     float v[7];
 #pragma unroll
-    for (int j = 0; j < 7; ++j) v[j] = a[min(max(t + j - 3, 0), T - 1)];
+    for (int j = 0; j < 7; ++j) v[j] = a[min(max(t + j - 3, 0), n - 1)];
 #pragma unroll
-    for (int j = 0; j < 7; ++j) v[j] = t + j - 3 >= 0 && t + j - 3 < T ? v[j] : 0.0f;
+    for (int j = 0; j < 7; ++j) v[j] = t + j - 3 >= 0 && t + j - 3 < n ? v[j] : 0.0f;
     if (t >= T) return;
     for (int c = c0; c < min(c0 + ENC_FIRST_CH, C); ++c) {
         float acc = bias[c];
@@ -1255,11 +1256,9 @@ static void snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_sa
     for (int i = 0; i < 3; ++i) c->enc_buf[i].alloc(cap);
     float *x = c->enc_buf[0].p, *f1 = c->enc_buf[1].p, *f2 = c->enc_buf[2].p;
     float* ain = f1;                                                      // (free until the first unit)
-    if (n_samples < Tp) HIP_CHECK(hipMemset2DAsync(ain + n_samples, (size_t)Tp * 4, 0, (size_t)(Tp - n_samples) * 4, batch, s));
-    if (batch == 1 || n_samples == Tp) HIP_CHECK(hipMemcpyAsync(ain, audio, (size_t)batch * n_samples * 4, hipMemcpyDefault, s));
-    else HIP_CHECK(hipMemcpy2DAsync(ain, (size_t)Tp * 4, audio, (size_t)n_samples * 4, (size_t)n_samples * 4, batch, hipMemcpyDefault, s));
+    HIP_CHECK(hipMemcpyAsync(ain, audio, (size_t)batch * n_samples * 4, hipMemcpyDefault, s));
     int64_t T = Tp;
-    hipLaunchKernelGGL(k_enc_first, dim3(cdiv(T, 256), cdiv(c->enc_dim, ENC_FIRST_CH), batch), dim3(256), 0, s, ain, x, W + c->enc_first.w, W + c->enc_first.b, c->enc_dim, (int)T);
+    hipLaunchKernelGGL(k_enc_first, dim3(cdiv(T, 256), cdiv(c->enc_dim, ENC_FIRST_CH), batch), dim3(256), 0, s, ain, x, W + c->enc_first.w, W + c->enc_first.b, c->enc_dim, (int)T, (int)n_samples);
     const int dils[3] = {1, 3, 9};
     for (auto& eb : c->enc_blocks) {
         for (int j = 0; j < 3; ++j) {
@@ -1384,7 +1383,7 @@ void launch_dw7(const float* X, float* Y, const float* w7, const float* bias, in
 
 // encoder pieces shared with the Descript DAC encoder (dac.hip)
 void launch_enc_first(const float* audio, float* y, const float* w, const float* bias, int batch, int C, int T, hipStream_t s) {
-    hipLaunchKernelGGL(k_enc_first, dim3(cdiv(T, 256), cdiv(C, ENC_FIRST_CH), batch), dim3(256), 0, s, audio, y, w, bias, C, T);
+    hipLaunchKernelGGL(k_enc_first, dim3(cdiv(T, 256), cdiv(C, ENC_FIRST_CH), batch), dim3(256), 0, s, audio, y, w, bias, C, T, T);
 }
 void launch_enc_phase_split(const float* x, float* y, const float* a, const float* ra, int batch, int C, int T, int stride, hipStream_t s) {
     hipLaunchKernelGGL(k_enc_phase_split, dim3(cdiv(T / stride + 1, 256), C, batch), dim3(256), 0, s, x, y, a, ra, C, T, stride, (stride + 1) / 2);
