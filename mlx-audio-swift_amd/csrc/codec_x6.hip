@@ -932,6 +932,141 @@ __global__ void __launch_bounds__(256, 3) k_x6_convt(GemmParams p, X6Noise nb, c
     x6_convt_body<MT, NOISE>(p, nb, p.X, p.Y, p.bias, p.alpha, p.ralpha, wp, nw);
 }
 
+// The same for few blocks (the same bits): 62 columns a block, a wave makes one phase of 32 of them, chunks of 32 channels, two of them requested ahead.  With a block a compute unit at most, the chain
+// of chunks is what there is to wait for: half as many, and none of them for its samples.  128 -> 64 channels
+// with the NoiseBlock, one row of 12288 columns: 29.3 -> 20.9 us; a decode of 1 x 12 groups 352 -> 344, of 1 x 4 326 -> 317.
+#define X6_CH 62
+template <int MT, bool NOISE>
+__device__ __forceinline__ void x6_convt_half_body(const GemmParams& p, const X6Noise& nb, const float* __restrict__ pX, float* __restrict__ pY, const float* __restrict__ pbias,
+                                                   const float* __restrict__ pa, const float* __restrict__ pra, const uint16_t* __restrict__ pwp, const uint16_t* __restrict__ pnw) {
+    constexpr int APC = 4 * MT * 192, NA = 2 * APC / 256, NN = MT * MT * 2 * 192;
+    __shared__ x6_u4 As[2 * APC];
+    __shared__ uint4 ts[3][4][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n0 = blockIdx.x * X6_CH, b = blockIdx.y, ph = wave >> 1, cb = (wave & 1) * 32;
+    const int q0 = p.pad / 2, dq = (1 + p.pad) / 2 - q0, t = n0 + q0 - 1 + lane;
+    const bool ok = t >= p.x_lo && t < p.Tin;
+    const float* xb = pX + ((size_t)b * p.Cin + wave * 8) * p.ldx + min(max(t, p.x_lo), p.Tin - 1);
+    f32x16_t acc[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
+    const x6_u4* wsrc = reinterpret_cast<const x6_u4*>(pwp) + tid;
+    const int chunks = p.Cin / 32;
+    float v[2][8];
+    x6_u4 wv[2][NA];
+    auto fetch = [&](int slot, int c) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[slot][j] = xb[(size_t)(c * 32 + j) * p.ldx];
+#pragma unroll
+        for (int i = 0; i < NA; ++i) wv[slot][i] = wsrc[(size_t)c * 2 * APC + i * 256];
+    };
+    fetch(0, 0);
+    fetch(1, min(1, chunks - 1));
+    auto chunk = [&](int slot, int c) {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int ch = c * 32 + wave * 8 + j;
+            x[j] = ok ? mis_snake(v[slot][j], pa[ch], pra[ch]) : 0.0f;
+        }
+        uint4 h, m, l;
+        x6_split<true>(x, h, m, l);
+        __syncthreads();                                                    // the previous chunk's products are done
+        ts[0][wave][lane] = h; ts[1][wave][lane] = m; ts[2][wave][lane] = l;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) As[tid + i * 256] = wv[slot][i];
+        if (c + 2 < chunks) fetch(slot, c + 2);
+        __syncthreads();
+        constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int tap = 0; tap < 2; ++tap) {
+                bf16x8_t bv[3], av[MT][3];
+                const int i = min(cb + (lane & 31) + 1 - tap + (ph ? dq : 0), 63);             // (past the end only for columns that are not stored)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) bv[q] = *reinterpret_cast<const bf16x8_t*>(&ts[q][2 * k + (lane >> 5)][i]);
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, As[k * APC + (((ph * 2 + tap) * MT + mi) * 3 + q) * 64 + lane]);
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int mi = 0; mi < MT; ++mi) acc[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[QB[q]], acc[mi], 0, 0, 0);
+            }
+    };
+    for (int c = 0; c < chunks; c += 2) {
+        chunk(0, c);
+        if (c + 1 < chunks) chunk(1, c + 1);
+    }
+    const int nl = cb + (lane & 31), n = n0 + nl, o = 2 * n + ph;
+    const bool in = nl < X6_CH && n < p.N && o < p.Tout, dup = n == 0 && p.dup_bias_n0;
+    const float* bp = pbias ? pbias : pX;
+    const int btop = pbias ? p.M - 1 : 0;
+    float nz = 0.0f;
+    if constexpr (NOISE) {
+        if (in && nb.noise) nz = nb.noise[(size_t)b * p.Tout + o];
+        else if (in && nb.rng) nz = codec_noise_value(nb.key, (uint64_t)(nb.row_offset + (nb.row_ids ? nb.row_ids[b] : b)), o);
+        __syncthreads();                                                    // the last chunk's products are done
+        for (int i = tid; i < NN; i += 256) As[i] = reinterpret_cast<const x6_u4*>(pnw)[i];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi) {
+        const int m0 = mi * 32 + 4 * (lane >> 5);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float bm = bp[min(m0 + (r & 3) + 8 * (r >> 2), btop)], bv = pbias ? bm : 0.0f;
+            acc[mi][r] += bv;
+            if (dup) acc[mi][r] += bv;
+        }
+    }
+    if constexpr (NOISE) {
+        f32x16_t w[MT];
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) w[mi][r] = 0.0f;
+        constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int ks = 0; ks < 2 * MT; ++ks) {
+            float x[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) x[r] = acc[ks / 2][ks % 2 * 8 + r];
+            bf16x8_t bv[3], av[MT][3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) bv[q] = __builtin_bit_cast(bf16x8_t, codec_tile_piece(x, q == 0));
+#pragma unroll
+            for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+                for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, As[((ks * MT + mi) * 3 + q) * 64 + lane]);
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int mi = 0; mi < MT; ++mi) w[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[QB[q]], w[mi], 0, 0, 0);
+        }
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mi][r] += nz * w[mi][r];
+    }
+    if (!in) return;
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int m = mi * 32 + 4 * (lane >> 5) + (r & 3) + 8 * (r >> 2);
+            if (m < p.M) pY[((size_t)b * p.M + m) * p.ldy + o] = acc[mi][r];
+        }
+}
+template <int MT, bool NOISE>
+__global__ void __launch_bounds__(256, 1) k_x6_convt_half(GemmParams p, X6Noise nb, const uint16_t* wp, const uint16_t* nw) {
+    x6_convt_half_body<MT, NOISE>(p, nb, p.X, p.Y, p.bias, p.alpha, p.ralpha, wp, nw);
+}
+
 bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s, const GemmParams* noise) {
     CodecPack* pack = p.pack ? p.pack : codec_x6_scope();
     if (!pack || codec_exact_f32() || p.s != 2 || p.K != 2 * p.Cin || p.M > 64 || p.M < 32 || p.Cin % 16 || !p.alpha) return false;
@@ -940,10 +1075,15 @@ bool launch_convt_x6(const GemmParams& p, int batch, hipStream_t s, const GemmPa
     const uint16_t* wp = pack->get_x6(p.AT, 4, p.Cin, p.M, s).wp;           // [phase][tap][Cin][M]
     const uint16_t* nw = noise ? pack->get_x6(noise->AT, 1, p.M, p.M, s).wp : nullptr;
     const X6Noise nb = noise ? X6Noise{noise->noise, noise->noise_rng, noise->noise_key, noise->row_ids, noise->row_offset} : X6Noise{};
-    const dim3 grid((p.N + X6_CT - 1) / X6_CT, batch);
-    if (p.M > 32 && noise) hipLaunchKernelGGL((k_x6_convt<2, true>), grid, dim3(256), 0, s, p, nb, wp, nw);
-    else if (p.M > 32) hipLaunchKernelGGL((k_x6_convt<2, false>), grid, dim3(256), 0, s, p, nb, wp, nw);
-    else if (noise) hipLaunchKernelGGL((k_x6_convt<1, true>), grid, dim3(256), 0, s, p, nb, wp, nw);
-    else hipLaunchKernelGGL((k_x6_convt<1, false>), grid, dim3(256), 0, s, p, nb, wp, nw);
+#define X6_GO(K, W) do { \
+        const dim3 grid((p.N + W - 1) / W, batch); \
+        if (p.M > 32 && noise) hipLaunchKernelGGL((K<2, true>), grid, dim3(256), 0, s, p, nb, wp, nw); \
+        else if (p.M > 32) hipLaunchKernelGGL((K<2, false>), grid, dim3(256), 0, s, p, nb, wp, nw); \
+        else if (noise) hipLaunchKernelGGL((K<1, true>), grid, dim3(256), 0, s, p, nb, wp, nw); \
+        else hipLaunchKernelGGL((K<1, false>), grid, dim3(256), 0, s, p, nb, wp, nw); } while (0)
+    // (while each has a compute unit of its own: a decode of 2 x 12 groups, 396 blocks, 427 either way)
+    if (p.Cin % 32 == 0 && (int64_t)((p.N + X6_CH - 1) / X6_CH) * batch <= 256) X6_GO(k_x6_convt_half, X6_CH);
+    else X6_GO(k_x6_convt, X6_CT);
+#undef X6_GO
     return true;
 }
