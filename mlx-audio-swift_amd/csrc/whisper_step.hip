@@ -11,9 +11,9 @@
 //    registers at a time - there are not enough compute units to hold a layer's weights and heads.
 //
 // us a step with the output projection and the sampling (26), chain -> here: 384 columns, 4 layers, one row 167 -> 106, eight 178 -> 128; 768, 12 layers, one 520 -> 300, five 559 -> 378,
-// eight 582 -> 413; 1024, 24 layers, one 1062 -> 583, eight 1227 -> 930; 1280, 32 layers, one 1500 -> 931, two 1526 -> 1015, eight 1737 -> 1553.  What bounds it: the hand-overs, about
+// eight 582 -> 415; 1024, 24 layers, one 1070 -> 577, eight 1230 -> 927; 1280, 32 layers, one 1503 -> 920, two 1526 -> 966, eight 1737 -> 1529.  What bounds it: the hand-overs, about
 // two us each with the polls, and the short programs between them (a norm 1 - 2, cross-attention 4, products and their sums 1 - 2); eight rows of 1280: 88 blocks for 46 MB of weights, and the
-// MLP's 20480 granules in four passes (6 us of a layer's 47; passes of 14 or 20 granules a thread are no faster, two launches a layer with a task a block 55).
+// MLP's 20480 granules in four passes (6 us of a layer's 46; passes of 14 or 20 granules a thread are no faster, two launches a layer with a task a block 55).
 //
 // A row has the bits of the launch chain: K is cut and summed as there, and each norm's statistics are dealt and summed as in the kernel that held them (LN_* below).
 #include "whisper_step.h"
@@ -126,12 +126,25 @@ __device__ __forceinline__ uint2 load2(Global<bf16_t> p) { const u32x2 v = *(Glo
 // A row's norm on one wave, from granules to xs.  `groups` of four columns a lane; the sums of their lanes are added as the chain's kernel added its waves (LN_WAVE: one sum).
 template <int KIND> __device__ __forceinline__ int norm_column(int K, int g, int lane) { return KIND == LN_SLICES ? 32 * ((K / 32 * g) / WAVES) + 4 * lane : 4 * (lane + 64 * g); }
 template <int KIND> __device__ __forceinline__ int norm_end(int K, int g) { return KIND == LN_SLICES ? 32 * ((K / 32 * (g + 1)) / WAVES) : min(K, 256 * (g + 1)); }
-__device__ __forceinline__ void norm_weights(bf16_t* wb, int K, Global<bf16_t> w, Global<bf16_t> b, int lane) {
-    for (int col = 4 * lane; col < K; col += 256) {
-        *reinterpret_cast<uint2*>(wb + col) = load2(w + col);
-        *reinterpret_cast<uint2*>(wb + K + col) = load2(b + col);
+// a norm's weights: asked for together, in front of the wait for its values (column by column behind it they were a round trip each: 1280 columns, 32 layers, two rows 1015 -> 966 us a step), into LDS behind it
+struct NormWeights {
+    uint2 w[LNG], b[LNG];
+    __device__ __forceinline__ void load(int K, Global<bf16_t> pw, Global<bf16_t> pb, int lane) {
+#pragma unroll
+        for (int g = 0; g < LNG; ++g) {
+            const unsigned col = min(4 * (lane + 64 * g), K - 4);
+            w[g] = load2(pw + col);
+            b[g] = load2(pb + col);
+        }
     }
-}
+    __device__ __forceinline__ void store(bf16_t* wb, int K, int lane) const {
+#pragma unroll
+        for (int g = 0; g < LNG; ++g) {
+            const int col = 4 * (lane + 64 * g);
+            if (col < K) { *reinterpret_cast<uint2*>(wb + col) = w[g]; *reinterpret_cast<uint2*>(wb + K + col) = b[g]; }
+        }
+    }
+};
 template <int KIND>
 __device__ __forceinline__ bool norm_row(bool hasty, const unsigned char* in, unsigned tag, bf16_t* row, const bf16_t* wb, int K, float eps, int lane) {
     constexpr int G = KIND == LN_SLICES ? WAVES : LNG;
@@ -222,17 +235,23 @@ struct Task {
             }
         asm volatile("" ::: "memory");
     }
+    __device__ __forceinline__ void weights(NormWeights& nw, int li, int lane, int wave) const {
+        if constexpr (LN != LN_NONE) {
+            constexpr int which = LN == LN_GLUE ? 0 : LN == LN_SLICES ? 1 : 2;
+            const WsParams& p = args();
+            if (wave < p.rows) nw.load(p.role[R].KT * 32, global(p.layers[li].lnw[which]), global(p.layers[li].lnb[which]), lane);
+        }
+    }
     // the input of a layer, from the values at `src`, into xs; false: stop
-    __device__ __forceinline__ bool take(unsigned char* smem, const Lds& l, int li, const unsigned char* src, unsigned tag, int id, int wave) const {
+    __device__ __forceinline__ bool take(unsigned char* smem, const Lds& l, const NormWeights& nw, const unsigned char* src, unsigned tag, int id, int wave) const {
         const WsParams& p = args();
         const int K = p.role[R].KT * 32, KP = K + XPAD, rows = p.rows, lane = id & 63;
         const bool hasty = p.limit == 0;
         bf16_t* xs = reinterpret_cast<bf16_t*>(smem);
         if constexpr (LN != LN_NONE) {
             if (wave >= rows) return true;
-            constexpr int which = LN == LN_GLUE ? 0 : LN == LN_SLICES ? 1 : 2;
             bf16_t* wb = reinterpret_cast<bf16_t*>(smem + l.wb);
-            norm_weights(wb, K, global(p.layers[li].lnw[which]), global(p.layers[li].lnb[which]), lane);
+            nw.store(wb, K, lane);
             return norm_row<LN>(hasty, src + (size_t)wave * K * 4, tag, xs + wave * KP, wb, K, p.eps, lane);
         }
         const int total = rows * (K / 2);
@@ -271,9 +290,11 @@ struct Task {
         unsigned char* now = p.exch + (size_t)exch_layer * li;
         // what the values in front of the input say is near, and what is there before it: bias, the norm's weights
         unsigned char* const src = R == WS_QKV ? now - exch_layer : now;
+        NormWeights nw;
+        if (R != WS_QKV || li > 0) weights(nw, li, lane, wave);
         if ((R != WS_QKV || li > 0) && at.near != at.in && (LN == LN_NONE || wave < rows) && !await(hasty, src + at.near, tag, lane)) return false;
         const uint32_t bias = mine && p.layers[li].b[R] ? *(Global<uint32_t>)global(p.layers[li].b[R] + col) : 0u;
-        if ((R != WS_QKV || li > 0) && !take(smem, l, li, src + at.in, tag, id, wave)) return false;
+        if ((R != WS_QKV || li > 0) && !take(smem, l, nw, src + at.in, tag, id, wave)) return false;
         // the residual: complete where the input, which is made of it, has come
         uint32_t hres = 0;
         if (TO == TO_RESID && mine) {
@@ -345,7 +366,9 @@ template <class T>
 __device__ __forceinline__ void last_rows(const T& qkv, unsigned char* smem, const Lds& l, int tid, int wave, const Edge& at, unsigned exch_layer, unsigned tag) {
     const WsParams& p = args();
     const unsigned char* src = p.exch + (size_t)exch_layer * (p.L - 1);
-    if ((wave < p.rows && !await(p.limit == 0, src + at.near, tag, tid & 63)) || !qkv.take(smem, l, p.L, src + at.in, tag, tid, wave)) return;
+    NormWeights nw;
+    qkv.weights(nw, p.L, tid & 63, wave);
+    if ((wave < p.rows && !await(p.limit == 0, src + at.near, tag, tid & 63)) || !qkv.take(smem, l, nw, src + at.in, tag, tid, wave)) return;
     bar();
     for (int i = tid; i < p.rows * (p.d / 8); i += THREADS) {
         const int r = i / (p.d / 8), k = (i - r * (p.d / 8)) * 8;
