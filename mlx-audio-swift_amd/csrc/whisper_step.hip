@@ -295,11 +295,12 @@ struct Task {
         if ((R != WS_QKV || li > 0) && at.near != at.in && (LN == LN_NONE || wave < rows) && !await(hasty, src + at.near, tag, lane)) return false;
         const uint32_t bias = mine && p.layers[li].b[R] ? *(Global<uint32_t>)global(p.layers[li].b[R] + col) : 0u;
         if ((R != WS_QKV || li > 0) && !take(smem, l, nw, src + at.in, tag, id, wave)) return false;
-        // the residual: complete where the input, which is made of it, has come
-        uint32_t hres = 0;
+        // the residual: there where the input, which is made of it, has come (its tag is looked at behind the products all the same)
+        const unsigned char* from = (R == WS_O ? now - exch_layer : now) + at.res + ((size_t)m * cols + col) * 4;
+        u64 res = (u64)tag << 32;
         if (TO == TO_RESID && mine) {
-            if (R == WS_O && li == 0) hres = *reinterpret_cast<const uint32_t*>(p.h0 + (size_t)m * p.d + col);
-            else hres = (uint32_t)__hip_atomic_load(reinterpret_cast<const u64*>((R == WS_O ? now - exch_layer : now) + at.res + ((size_t)m * cols + col) * 4), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (R == WS_O && li == 0) res |= *reinterpret_cast<const uint32_t*>(p.h0 + (size_t)m * p.d + col);
+            else res = __hip_atomic_load(reinterpret_cast<const u64*>(from), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         bar();
         {
@@ -326,6 +327,16 @@ struct Task {
                 }
         }
         bar();
+        uint32_t hres = (uint32_t)res;
+        if (TO == TO_RESID && !__all((unsigned)(res >> 32) == tag)) {
+            bool good = true;
+            if (mine && (R != WS_O || li > 0)) {
+                uint32_t v[1];
+                good = gather<1>(hasty, v, tag, lane, [&](int) { return from; });
+                hres = v[0];
+            }
+            if (!__all(good)) return false;
+        }
         if (mine) {
             constexpr int KSB = R == WS_CQ || R == WS_FC1 ? 8 : 4, G = 16 / KSB;
             float a0 = 0.f, a1 = 0.f;
