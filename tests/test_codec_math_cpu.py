@@ -1,5 +1,6 @@
 """CPU pins for two numerical building blocks of the codec kernels (no GPU, no library call):
- - mis_sin_sq (csrc/codec_kernels.h): the 12-instruction sin^2 of the Snake activations, restated operation by operation in float32
+ - sin^2 by multiples of pi and a polynomial for the sine, the form of the Snake activations that mis_snake (csrc/codec_kernels.h) took the place of: the measure
+   that tests/test_snake_cpu.py compares the kernels' form with
  - the split-bf16 contraction of csrc/codec_bf3.hip (x = xh + xl, three products, f32 accumulation) inside the SNAC oracle."""
 import numpy as np
 
@@ -9,7 +10,7 @@ F = np.float32
 
 
 def sin_sq_f32(y):
-    """mis_sin_sq, same constants and operation order; numpy float32 arithmetic (fma emulated in float64 and rounded once)."""
+    """sin^2 y in float32: y less a multiple of pi in two parts, a polynomial of degree eleven, squared (fma emulated in float64 and rounded once)."""
     y = np.asarray(y, F)
 
     def fma(a, b, c):

@@ -1,9 +1,14 @@
-"""mis_snake (csrc/codec_kernels.h) restated operation by operation in float32: its error against 64 bits, beside that of the form it took the place of, and its ends."""
+"""mis_snake (csrc/codec_kernels.h) restated operation by operation in float32, its coefficients read from there: its error against 64 bits, beside that of the form it took the place of, and its ends."""
+import pathlib
+import re
+
 import numpy as np
 import pytest
 
 F = np.float32
-C = [F(v) for v in (9.86960292, -32.4695811, 42.7253848, -30.0859532, 12.9907303, -3.27294594)]
+HEADER = pathlib.Path(__file__).resolve().parents[1] / "mlx-audio-swift_amd" / "csrc" / "codec_kernels.h"
+BODY = re.search(r"float mis_snake\(float x, float a, float ra\) \{(.*?)\n\}", HEADER.read_text(), re.S).group(1)
+C = [F(v) for v in reversed(re.findall(r"([-+]?\d\.\d+e[-+]\d+)f", BODY))]      # the highest degree stands first there
 
 
 def fma(a, b, c):
@@ -12,8 +17,7 @@ def fma(a, b, c):
 
 def snake(x, a, ra):
     """a = alpha / pi, rounded once."""
-    t = (a * x).astype(F)
-    f = (t - np.rint(t)).astype(F)
+    f = fma(a, x, -np.rint((a * x).astype(F)))
     s = (f * f).astype(F)
     p = fma(s, C[5], C[4])
     for k in C[3::-1]:
@@ -22,14 +26,23 @@ def snake(x, a, ra):
 
 
 def snake_by_sine(x, alpha, ra):
-    """alpha x reduced by multiples of pi, the square of a polynomial for the sine (mis_sin_sq, tests/test_codec_math_cpu.py)."""
+    """alpha x reduced by multiples of pi, the square of a polynomial for the sine (tests/test_codec_math_cpu.py)."""
     from test_codec_math_cpu import sin_sq_f32
     return fma(ra, sin_sq_f32((alpha * x).astype(F)), x)
 
 
-@pytest.mark.parametrize("scale,bound", [(0.3, 2.5e-8), (1.0, 7e-8), (3.0, 1.5e-7)])
+def test_body():
+    """The operations that snake() restates, in the kernel's words."""
+    lines = [re.sub(r"\s+", " ", l.strip()) for l in BODY.strip().splitlines()]
+    assert len(C) == 6 and len(lines) == 8
+    assert lines[0] == "const float f = fmaf(a, x, -rintf(a * x));" and lines[1] == "const float s = f * f;"
+    assert lines[2].startswith("float p = fmaf(s, ") and all(l.startswith("p = fmaf(s, p, ") for l in lines[3:7]) and lines[7] == "return fmaf(ra, p * s, x);"
+
+
+@pytest.mark.parametrize("scale,bound", [(0.3, 2.5e-8), (1.0, 5e-8), (3.0, 1.15e-7), (10.0, 3.5e-7), (30.0, 1.05e-6), (100.0, 3.5e-6)])
 def test_error_against_64_bits(scale, bound):
-    """Rounding of t = a x (2^-25 |alpha x|, and as much for a) times the slope of sin^2 / alpha, at most one, and that of the sum."""
+    """Rounding of a (at most 2^-24 |alpha x|, 2^-25.8 rms) times the slope of sin^2 / alpha, at most one, and that of the sum.  A product that is rounded before its
+    whole number is taken off has as much again: 1.06 times the form before at three, 1.15 from ten on."""
     r = np.random.default_rng(5)
     alpha = r.uniform(0.5, 2.0, 400_000).astype(F)
     x = (r.standard_normal(400_000) * scale).astype(F)
@@ -38,7 +51,7 @@ def test_error_against_64_bits(scale, bound):
     exact = x.astype(np.float64) + np.sin(alpha.astype(np.float64) * x.astype(np.float64)) ** 2 / (alpha.astype(np.float64) + 1e-9)
     rms = lambda y: float(np.sqrt(np.mean((y - exact) ** 2)))
     here, before = rms(snake(x, a, ra)), rms(snake_by_sine(x, alpha, ra))
-    assert here <= bound and here <= 1.15 * before, (here, before)
+    assert here <= bound and here <= 1.05 * before, (here, before)
 
 
 def test_ends():
