@@ -34,6 +34,8 @@ int32_t mis_debug_sampler_failures(void);
 /* tests: let the library's device buffers grow by at most `more` bytes from here on (negative: as far as the card's memory goes); returns the bytes they hold.
  * An allocation past it fails as one past the card's memory does. */
 int64_t mis_debug_device_limit(int64_t more);
+/* tests: how often this process has waited for results on their way to pageable memory (samples, codes, latents, logits) */
+int64_t mis_debug_result_waits(void);
 /* tests: for how many floats d in [1, 2^14) the reciprocal of the Whisper encoder's GELU is not 1 / d rounded to nearest (none) */
 mis_status mis_debug_gelu_rcp_misses(int device, int64_t* misses);
 

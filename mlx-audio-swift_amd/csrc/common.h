@@ -110,7 +110,7 @@ static inline hipError_t copy_now(void* dst, const void* src, size_t n, hipMemcp
 struct HostRing {
     static constexpr int SLOTS = 8;
     static constexpr size_t SLOT = (size_t)2 << 20, MIN = (size_t)4 << 20, SMALL = (size_t)1 << 20, INPUT = (size_t)64 << 10;
-    static constexpr int PIECES = 8;
+    static constexpr int PIECES = 9;                                       // (eight levels of codes and a latent)
     struct Piece { void* to; const void* from; size_t bytes; };
     PinnedBuf<uint8_t> buf;                                                // SLOTS x SLOT for the large copies, or nothing; SMALL + INPUT for the small ones
     size_t held = 0;
@@ -121,8 +121,9 @@ struct HostRing {
     ~HostRing();
     void reserve(bool large = true);
     static bool pageable(const void* p);
-    // up to PIECES small copies at once; false: not small, or not between the device and pageable memory, and nothing done
-    bool out_small(const Piece* p, int n, hipStream_t s);                  // waits
+    // up to PIECES copies at once; false: too large, or not between the device and pageable memory, and nothing done.
+    // Results: past SMALL and below MIN together by copy commands side by side into the slots; one wait either way
+    bool out_together(const Piece* p, int n, hipStream_t s);               // waits
     bool in_small(const Piece* p, int n, hipStream_t s);                   // does not: once between two waits for the stream
     void out(void* host, const void* dev, size_t n, hipStream_t s);
     void in(void* dev, const void* host, size_t n, hipStream_t s);

@@ -251,18 +251,30 @@ static void copy_pieces(const CopyPieces& c, int n, hipStream_t s) {
     hipLaunchKernelGGL(k_copy_pieces, dim3((unsigned)std::min<size_t>(64, (most / 16 + 255) / 256 + 1), n), dim3(256), 0, s, c);
     HIP_CHECK(hipGetLastError());
 }
-bool HostRing::out_small(const Piece* p, int n, hipStream_t s) {
+// waits for results on their way to the caller's memory (diagnostics, tests)
+static std::atomic<int64_t> g_result_waits{0};
+extern "C" int64_t mis_debug_result_waits(void) { return g_result_waits.load(); }
+static void wait_for_results(hipStream_t s) {
+    g_result_waits.fetch_add(1, std::memory_order_relaxed);
+    HIP_CHECK(hipStreamSynchronize(s));
+}
+bool HostRing::out_together(const Piece* p, int n, hipStream_t s) {
     size_t total = 0;
     if (!buf.p || n < 1 || n > PIECES) return false;
+    bool by_kernel = true;
     for (int i = 0; i < n; ++i) {
         total += round_up(p[i].bytes, 16);
-        if (!p[i].bytes || total > SMALL || ((uintptr_t)p[i].from & 15) || !pageable(p[i].to)) return false;
+        if (!p[i].bytes || total >= MIN || !pageable(p[i].to)) return false;
+        by_kernel = by_kernel && ((uintptr_t)p[i].from & 15) == 0;
     }
+    by_kernel = by_kernel && total <= SMALL;
+    if (!by_kernel && !ev[0]) return false;
     CopyPieces c;
-    uint8_t* at = buf.p + held - INPUT - SMALL;
+    uint8_t* at = by_kernel ? buf.p + held - INPUT - SMALL : buf.p;
     for (int i = 0; i < n; ++i) { c.p[i] = {at, p[i].from, p[i].bytes}; at += round_up(p[i].bytes, 16); }
-    copy_pieces(c, n, s);
-    HIP_CHECK(hipStreamSynchronize(s));
+    if (by_kernel) copy_pieces(c, n, s);
+    else for (int i = 0; i < n; ++i) HIP_CHECK(hipMemcpyAsync(c.p[i].to, c.p[i].from, c.p[i].bytes, hipMemcpyDeviceToHost, s));
+    wait_for_results(s);
     for (int i = 0; i < n; ++i) memcpy(p[i].to, c.p[i].to, p[i].bytes);
     return true;
 }
@@ -291,10 +303,10 @@ bool HostRing::pageable(const void* p) {
 void HostRing::out(void* host, const void* dev, size_t n, hipStream_t s) {
     if (n == 0) { HIP_CHECK(hipStreamSynchronize(s)); return; }
     const Piece p{host, dev, n};
-    if (n <= SMALL && out_small(&p, 1, s)) return;
+    if (n <= SMALL && ((uintptr_t)dev & 15) == 0 && out_together(&p, 1, s)) return;
     if (ev[0] && buf.p && n >= MIN && pageable(host)) { run((uint8_t*)host, (uint8_t*)const_cast<void*>(dev), n, true, s); return; }
     HIP_CHECK(hipMemcpyAsync(host, dev, n, hipMemcpyDefault, s));
-    HIP_CHECK(hipStreamSynchronize(s));
+    wait_for_results(s);
 }
 void HostRing::in(void* dev, const void* host, size_t n, hipStream_t s) {
     if (n == 0) return;

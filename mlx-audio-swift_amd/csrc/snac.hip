@@ -1347,8 +1347,8 @@ static void snac_encode(mis_snac* c, const float* audio, int batch, int64_t n_sa
         codes += round_up((size_t)batch * Tm, 4);
     }
     HIP_CHECK(hipGetLastError());
-    // one launch and one wait where they are small (copied one by one, each is a wait of its own)
-    if (!c->ring.out_small(results.data(), (int)results.size(), s))
+    // one wait below 4 MiB (copied one by one, each is a wait of its own)
+    if (!c->ring.out_together(results.data(), (int)results.size(), s))
         for (auto& r : results) c->ring.out(r.to, r.from, r.bytes, s);
     HIP_CHECK(hipGetLastError());
 }

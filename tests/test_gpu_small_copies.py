@@ -56,6 +56,19 @@ def test_snac_encode(snac, rows, samples):
     assert all(np.array_equal(c, o.cpu().numpy()) for c, o in zip(codes, out)) and np.array_equal(z, zo.cpu().numpy())
 
 
+# codes and latent of 0.1, 1.6, 2.8 MB: by a kernel, and side by side into the ring from 1 MiB on (one by one they were a wait each); 4.2 MB: one by one
+@pytest.mark.parametrize("rows,samples,waits", [(1, 30011, 1), (1, 800000, 1), (3, 470001, 1), (4, 522000, 4)])
+def test_results_of_an_encode_share_a_wait(snac, rows, samples, waits):
+    a = (0.1 * np.random.default_rng(samples).standard_normal((rows, samples))).astype(np.float32)
+    codes, z = snac.encode(a, return_latent=True)
+    total = z.nbytes + sum(c.nbytes for c in codes)
+    assert (total < 4 << 20) == (waits == 1)
+    before = _lib.lib().mis_debug_result_waits()
+    again, z2 = snac.encode(a, return_latent=True)
+    assert _lib.lib().mis_debug_result_waits() - before == waits
+    assert np.array_equal(z, z2) and all(np.array_equal(x, y) for x, y in zip(codes, again))
+
+
 @pytest.mark.parametrize("rows,frames", [(1, 1), (1, 30), (1, 251), (3, 250), (4, 400), (1, 1400)])
 def test_dac_decode(dac, rows, frames):
     rng = np.random.default_rng(frames)
