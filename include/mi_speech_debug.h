@@ -34,6 +34,12 @@ int32_t mis_debug_sampler_failures(void);
 /* tests: let the library's device buffers grow by at most `more` bytes from here on (negative: as far as the card's memory goes); returns the bytes they hold.
  * An allocation past it fails as one past the card's memory does. */
 int64_t mis_debug_device_limit(int64_t more);
+/* tests: decode steps of the handle's last request whose layers went as one launch (csrc/lm_step.hip, csrc/whisper_step.hip); the others took the launch chain */
+int32_t mis_debug_tts_step_launches(const mis_tts* c);
+int32_t mis_debug_whisper_step_launches(const mis_whisper* c);
+/* tests: which request may have its steps in one launch (DeviceCall, DeviceTurn: csrc/common.h), without a device.  op, of the calling thread: 0 / 1 a call on the device begins / ends,
+ * 2 takes the device (returns whether), 3 rests, 4 polls (returns whether it has the device), 5 gives it back, 6 waits as a call does whose kernels' blocks wait for each other */
+int32_t mis_debug_device_turn(int device, int op);
 /* tests: how often this process has waited for results on their way to pageable memory (samples, codes, latents, logits) */
 int64_t mis_debug_result_waits(void);
 /* tests: for how many floats d in [1, 2^14) the reciprocal of the Whisper encoder's GELU is not 1 / d rounded to nearest (none) */

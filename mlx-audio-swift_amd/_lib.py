@@ -299,6 +299,9 @@ DEBUG_SYMBOLS = {
     "mis_debug_device_cus": (C.c_int32, [C.c_int]),
     "mis_debug_sampler_failures": (C.c_int32, []),
     "mis_debug_codec_chain": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P, _P, _P, _P, _P, _P]),
+    "mis_debug_tts_step_launches": (C.c_int32, [_P]),
+    "mis_debug_whisper_step_launches": (C.c_int32, [_P]),
+    "mis_debug_device_turn": (C.c_int32, [C.c_int, C.c_int]),
     "mis_debug_result_waits": (C.c_int64, []),
     "mis_debug_device_limit": (C.c_int64, [C.c_int64]),
     "mis_debug_gelu_rcp_misses": (C.c_int, [C.c_int, C.POINTER(C.c_int64)]),

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <chrono>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdarg.h>
@@ -130,6 +131,38 @@ struct HostRing {
 private:
     void run(uint8_t* host, uint8_t* dev, size_t n, bool to_host, hipStream_t s);
 };
+
+// ---------------------------------------------------------------------------- calls on a device, and the device to oneself
+// An entry point that runs kernels holds a DeviceCall while it does.  A call that a thread makes inside another one of its own (an event callback) belongs to that one.
+struct DeviceCall {
+    const int device;
+    explicit DeviceCall(int device);
+    ~DeviceCall();
+    DeviceCall(const DeviceCall&) = delete;
+    DeviceCall& operator=(const DeviceCall&) = delete;
+};
+// Decode steps in one launch (lm_step.hip, whisper_step.hip) take every compute unit and wait until all of their blocks have one: beside another call's kernels they cost both more than the
+// launch chain does (two one-row requests 349 -> 400 ms, a 0.38 ms codec call 0.70), and beside kernels whose blocks wait for each other neither gets on.  So a request has its steps in
+// one launch while its call is the only one on the device in this process.
+class DeviceTurn {
+    int device = -1;
+    uint64_t seen = 0;                                                     // calls that had come when this one last looked
+    std::chrono::steady_clock::time_point since;                           // ... alone
+    bool held = false;
+public:
+    DeviceTurn() {}
+    DeviceTurn(const DeviceTurn&) = delete;
+    DeviceTurn& operator=(const DeviceTurn&) = delete;
+    ~DeviceTurn() { give(); }
+    bool take(int device);               // inside a DeviceCall; whether it is the only one
+    void rest();                         // with nothing of the request on the device, until at_poll: callbacks
+    bool at_poll();                      // whether the next steps have the device: no call has come; or none for QUIET
+    void give();
+    static constexpr int QUIET_MS = 50, SETTLE_MS = 500;
+};
+// In front of kernels whose blocks wait for each other (one-launch sampler, token engine, LSTM): until a request that has the device has seen this call at its next poll.  Bounded: past
+// SETTLE_MS the waits of both sides end by themselves, as they do beside another process.
+void device_settle(int device);
 
 // Between a wave's LDS writes and its other lanes' reads of them (and the other way round).  The hardware keeps one wave's LDS accesses in order; the fences
 // keep the compiler from moving them, which the barrier alone, no memory operation, does not promise.

@@ -129,6 +129,7 @@ extern "C" mis_status mis_dac_finalize(mis_dac* c) {
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized, MIS_ERR_INVALID_INPUT, "bad handle");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     const mis_dac_config& cf = c->cfg;
     const int64_t D = c->latent, cd = cf.codebook_dim, bins = cf.codebook_size, dd = cf.decoder_dim;
     std::vector<float> arena;
@@ -373,6 +374,7 @@ extern "C" mis_status mis_dac_encode(mis_dac* c, const float* audio, int batch, 
     MIS_REQUIRE(n_quantizers >= 0 && n_quantizers <= c->cfg.n_codebooks, MIS_ERR_INVALID_INPUT, "n_quantizers out of range");
     const int nq = n_quantizers ? n_quantizers : c->cfg.n_codebooks;
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     codec_run(c->pack, [&] { dac_encode(c, audio, batch, n_samples, nq, codes_out, z_out); });
     MIS_API_END
 }
@@ -444,6 +446,7 @@ extern "C" mis_status mis_dac_decode_codes(mis_dac* c, const int32_t* codes, int
     MIS_API_BEGIN
     MIS_REQUIRE(c && codes && wav_out && batch >= 1 && T >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     const int64_t n = mis_dac_num_samples(c, T);
     codec_run(c->pack, [&] {
         int C; int64_t Tt;
@@ -461,6 +464,7 @@ extern "C" mis_status mis_dac_debug_tap(mis_dac* c, const int32_t* codes, int ba
     MIS_API_BEGIN
     MIS_REQUIRE(c && codes && out && channels && length && block >= 0 && block < c->cfg.n_decoder_rates, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     DevBuf<float> wav;
     int C = 0; int64_t Tt = 0;
     const float* res = nullptr;

@@ -269,6 +269,7 @@ extern "C" mis_status mis_encodec_finalize(mis_encodec* c) {
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized, MIS_ERR_INVALID_INPUT, "bad handle");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     const mis_encodec_config& cf = c->cfg;
     std::vector<float> arena;
     auto push = [&](const std::vector<float>& v) { size_t o = arena.size(); arena.insert(arena.end(), v.begin(), v.end()); while (arena.size() & 3) arena.push_back(0.f); return o; };
@@ -401,6 +402,7 @@ static const float* encodec_run(mis_encodec* c, const int32_t* codes_dev, int nq
         MIS_REQUIRE(smem <= 64 * 1024 && NB <= 256, MIS_ERR_INVALID_INPUT, "LSTM width %d does not fit the persistent kernel", H);
         c->hstate.alloc((size_t)2 * batch * H);
         c->sync.alloc(2);
+        device_settle(c->device);
         const float* in = x;
         float* cur = y;
         for (size_t j = 0; j < c->lstm.size(); ++j) {
@@ -472,6 +474,7 @@ extern "C" mis_status mis_encodec_decode_frame(mis_encodec* c, const int32_t* co
     MIS_API_BEGIN
     MIS_REQUIRE(c && codes && wav_out && batch >= 1 && T >= 1 && n_q >= 1 && n_q <= c->n_q, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     const int64_t n = (int64_t)T * mis_encodec_hop_length(c) * c->cfg.audio_channels;
     c->codes_dev.alloc((size_t)batch * n_q * T);
@@ -494,6 +497,7 @@ extern "C" mis_status mis_encodec_debug_tap(mis_encodec* c, const int32_t* codes
     MIS_API_BEGIN
     MIS_REQUIRE(c && codes && out && channels && length && stage >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     c->codes_dev.alloc((size_t)batch * n_q * T);
     HIP_CHECK(hipMemcpyAsync(c->codes_dev.p, codes, (size_t)batch * n_q * T * 4, hipMemcpyDefault, s));

@@ -12,7 +12,10 @@
 #include <unistd.h>
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <fstream>
+#include <memory>
+#include <mutex>
 #include <sstream>
 #include <thread>
 
@@ -224,6 +227,98 @@ mis_dtype dtype_from_safetensors(const std::string& s) {
     if (s == "BF16") return MIS_BF16;
     if (s == "I32") return MIS_I32;
     throw MisError(MIS_ERR_INVALID_INPUT, "unsupported safetensors dtype " + s);
+}
+
+// ---------------------------------------------------------------------------- calls on a device
+namespace {
+struct DeviceUse {
+    std::mutex m;
+    std::condition_variable given;
+    int calls = 0;
+    uint64_t came = 0;
+    const DeviceTurn* holder = nullptr;
+    std::thread::id holder_thread;
+    bool resting = false;
+};
+constexpr int DEVICES = 64;                                                // (past them: no call is alone)
+DeviceUse g_use[DEVICES];
+thread_local int t_depth[DEVICES];
+bool known(int device) { return device >= 0 && device < DEVICES; }
+}
+DeviceCall::DeviceCall(int d) : device(d) {
+    if (!known(d) || t_depth[d]++) return;
+    std::lock_guard<std::mutex> g(g_use[d].m);
+    ++g_use[d].calls;
+    ++g_use[d].came;
+}
+DeviceCall::~DeviceCall() {
+    if (!known(device) || --t_depth[device]) return;
+    std::lock_guard<std::mutex> g(g_use[device].m);
+    --g_use[device].calls;
+}
+bool DeviceTurn::take(int d) {
+    give();
+    if (!known(d)) return false;
+    DeviceUse& u = g_use[d];
+    std::lock_guard<std::mutex> g(u.m);
+    device = d;
+    seen = u.came;
+    since = std::chrono::steady_clock::now();
+    if (u.calls != 1 || u.holder || !t_depth[d]) return false;
+    u.holder = this; u.holder_thread = std::this_thread::get_id(); u.resting = false;
+    return held = true;
+}
+void DeviceTurn::rest() {
+    if (!held) return;
+    DeviceUse& u = g_use[device];
+    { std::lock_guard<std::mutex> g(u.m); u.resting = true; }
+    u.given.notify_all();
+}
+bool DeviceTurn::at_poll() {
+    if (device < 0) return false;
+    DeviceUse& u = g_use[device];
+    std::lock_guard<std::mutex> g(u.m);
+    const auto now = std::chrono::steady_clock::now();
+    if (u.came != seen || u.calls != 1) {
+        seen = u.came;
+        since = now;
+        if (held) { u.holder = nullptr; held = false; u.given.notify_all(); }
+        return false;
+    }
+    if (!held && !u.holder && now - since >= std::chrono::milliseconds(QUIET_MS)) {
+        u.holder = this; u.holder_thread = std::this_thread::get_id();
+        held = true;
+    }
+    if (held) u.resting = false;
+    return held;
+}
+void DeviceTurn::give() {
+    if (!held) return;
+    DeviceUse& u = g_use[device];
+    std::lock_guard<std::mutex> g(u.m);
+    u.holder = nullptr;
+    held = false;
+    u.given.notify_all();
+}
+void device_settle(int d) {
+    if (!known(d)) return;
+    DeviceUse& u = g_use[d];
+    std::unique_lock<std::mutex> g(u.m);
+    const auto me = std::this_thread::get_id();
+    u.given.wait_for(g, std::chrono::milliseconds(DeviceTurn::SETTLE_MS), [&] { return !u.holder || u.resting || u.holder_thread == me; });
+}
+extern "C" int32_t mis_debug_device_turn(int device, int op) {
+    static thread_local std::vector<std::unique_ptr<DeviceCall>> calls;
+    static thread_local DeviceTurn turn;
+    switch (op) {
+        case 0: calls.emplace_back(new DeviceCall(device)); return 0;
+        case 1: if (!calls.empty()) calls.pop_back(); return 0;
+        case 2: return turn.take(device);
+        case 3: turn.rest(); return 0;
+        case 4: return turn.at_poll();
+        case 5: turn.give(); return 0;
+        default: device_settle(device); return 0;
+    }
 }
 
 // ---------------------------------------------------------------------------- large host copies

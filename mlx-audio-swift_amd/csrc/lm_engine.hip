@@ -82,10 +82,10 @@ struct mis_tts {
     DevBuf<SamplerScratch> samp_scratch;
     DevBuf<unsigned char> step_exch;             // decode steps in one launch (lm_step.hip): values handed between blocks, flags
     DevBuf<unsigned> step_sync;
-    unsigned* step_lock = nullptr;               // the device's, not this handle's
+    int step_count = 0;                          // decode steps of the last request that went as one launch
     bool step_off = false;                       // a launch has timed out: this handle stays on the launch chain
     HostRing ring;
-    hipGraphExec_t g_prefill = nullptr, g_decode = nullptr;
+    hipGraphExec_t g_prefill = nullptr, g_decode = nullptr, g_step = nullptr;   // g_step: a decode step whose layers are one launch
     bool shared_device = false;      // another replica's streams run on this device (group.hip): never a kernel that waits for co-resident blocks
     uint64_t graph_key = 0;
     bool use_graph = true;
@@ -397,6 +397,7 @@ extern "C" mis_status mis_tts_init_synthetic_quantized(mis_tts* c, uint64_t seed
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized && !c->blocks && (bits == 4 || bits == 8), MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     const int d = c->d, ff = c->ff, HD = c->H * c->D, KD = c->Hkv * c->D;
     const uint64_t base = seed * 100000ull;
@@ -443,6 +444,7 @@ extern "C" mis_status mis_tts_init_synthetic(mis_tts* c, uint64_t seed) {
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized, MIS_ERR_INVALID_INPUT, "bad handle");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     if (c->blocks) { c->blocks->init_synthetic(seed, s); return MIS_OK; }
     const int d = c->d, ff = c->ff, HD = c->H * c->D, KD = c->Hkv * c->D;
@@ -486,6 +488,7 @@ extern "C" mis_status mis_tts_finalize(mis_tts* c) {
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized, MIS_ERR_INVALID_INPUT, "bad handle");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     if (c->blocks) {
         c->blocks->finalize();
         c->staging.release(); c->raw_staging.release();
@@ -545,6 +548,7 @@ static int choose_split(int items, int KT, int ksb, const char* env, int s_max =
 static void destroy_graphs(mis_tts* c) {
     if (c->g_prefill) { (void)hipGraphExecDestroy(c->g_prefill); c->g_prefill = nullptr; }
     if (c->g_decode) { (void)hipGraphExecDestroy(c->g_decode); c->g_decode = nullptr; }
+    if (c->g_step) { (void)hipGraphExecDestroy(c->g_step); c->g_step = nullptr; }
 }
 
 static void build_rope_tables(mis_tts* c) {
@@ -799,7 +803,7 @@ static bool step_params(const mis_tts* c, StepParams& p) {
     p.norms = c->norms.p; p.kcache = c->kcache.p; p.vcache = c->vtcache.p;
     p.kv_layer = (size_t)c->batch * c->Hkv * c->Smax * c->D;
     p.pos = c->pos_cur.p; p.active = c->active.p; p.rope_cos = c->rope_cos.p; p.rope_sin = c->rope_sin.p;
-    p.exch = c->step_exch.p; p.sync = c->step_sync.p; p.lock = c->step_lock;
+    p.exch = c->step_exch.p; p.sync = c->step_sync.p;
     const char* us = getenv("MIS_LM_STEP_US");                             // (tests force the time-out)
     p.limit = us ? 100ull * (unsigned long long)std::max(0, atoi(us)) : 5000000ull;       // 50 ms: a step takes one to two
     p.L = c->L; p.d = c->d; p.H = c->H; p.Hkv = c->Hkv; p.Smax = c->Smax; p.rows = c->batch; p.Mpad = c->Mpad;
@@ -807,13 +811,12 @@ static bool step_params(const mis_tts* c, StepParams& p) {
     p.eps = c->cfg.rms_norm_eps; p.scale = 1.0f / sqrtf((float)c->D);
     return true;
 }
-// Whether a request takes it, and its buffers.  `alone`: no kernel of the request may wait for another block's (the second attempt behind a time-out, a device shared by replicas).
-static bool step_begin(mis_tts* c, bool alone) {
+// Whether a request may take it, and its buffers.  `apart`: no kernel of the request may wait for another block's (the second attempt behind a time-out, a device shared by replicas).
+static bool step_begin(mis_tts* c, bool apart) {
     const StepShape shape{c->L, c->d, c->ff, c->H, c->Hkv, c->D, c->batch};
     const char* e = getenv("MIS_LM_STEP");                                 // 0: the launch chain (parity tests, read per call)
     StepParams p{};
-    if (alone || c->step_off || (e && atoi(e) == 0) || !step_params(c, p) || !step_ok(shape, p, c->device)) return false;
-    c->step_lock = step_lock(c->device);
+    if (apart || c->step_off || (e && atoi(e) == 0) || !step_params(c, p) || !step_ok(shape, p, c->device)) return false;
     c->step_exch.alloc(step_exch_bytes(shape));
     c->step_sync.alloc(SYNC_WORDS);
     c->step_exch.zero(c->stream);                                          // (tags begin again)
@@ -1073,6 +1076,7 @@ extern "C" mis_status mis_lm_extend(mis_tts* c, const int32_t* rows, const int32
     MIS_REQUIRE(c->blocks, MIS_ERR_INVALID_INPUT, "mis_lm_extend serves models described layer by layer");
     MIS_REQUIRE(c->finalized && c->batch > 0, MIS_ERR_NOT_INITIALIZED, "call mis_lm_reset first");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     std::vector<PassEntry> entries;
     std::set<int32_t> seen;
@@ -1157,6 +1161,7 @@ extern "C" mis_status mis_lm_forward_hidden(mis_tts* c, const int32_t* ids, cons
     MIS_REQUIRE(c && ids, MIS_ERR_INVALID_INPUT, "null argument");
     MIS_REQUIRE(c->batch > 0, MIS_ERR_NOT_INITIALIZED, "call mis_lm_reset first");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     std::vector<uint8_t> act(c->batch, 1);
     if (active) {
@@ -1216,6 +1221,7 @@ extern "C" mis_status mis_lm_prefill(mis_tts* c, const int32_t* prompt_ids, cons
     MIS_REQUIRE(c && prompt_ids && prompt_lens && batch >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
     MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "model not finalized");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     std::vector<int32_t> lens(batch);
     HIP_CHECK(copy_now(lens.data(), prompt_lens, batch * 4, hipMemcpyDefault));
@@ -1290,6 +1296,7 @@ extern "C" mis_status mis_sample_logits(int device, const float* logits, int bat
     MIS_REQUIRE(logits && params && tokens_out && batch >= 1 && vocab >= 1, MIS_ERR_INVALID_INPUT, "bad argument");
     MIS_REQUIRE(ctx == 0 || (window && window_len), MIS_ERR_INVALID_INPUT, "window pointers required when ctx > 0");
     HIP_CHECK(hipSetDevice(device));
+    DeviceCall call(device);
     int Vpad = (int)round_up(vocab, 16);
     DevBuf<float> lf, eb;
     DevBuf<bf16_t> lb;
@@ -1327,6 +1334,7 @@ extern "C" mis_status mis_sample_logits(int device, const float* logits, int bat
     DevBuf<unsigned long long> dbg;
     const bool want_dbg = getenv("MIS_SAMP_DBG") != nullptr;        // diagnostics: phase stamps of block (0, 0) on stderr (tools/samp_phases.py)
     if (want_dbg) { dbg.alloc(48); dbg.zero(0); sp.dbg = dbg.p; }
+    device_settle(device);
     launch_sampler(sp, batch, 0);
     HIP_CHECK(hipGetLastError());
     if (want_dbg) {
@@ -1510,7 +1518,10 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         HIP_CHECK(hipMemcpyAsync(hid_count.p, ones_i.data(), batch * 4, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipStreamSynchronize(s));
     }
-    const bool one_launch = step_begin(c, multi_launch_only);
+    const bool one_launch = step_begin(c, multi_launch_only);           // where the device is this request's alone: `turn`
+    DeviceTurn turn;
+    bool by_step = false;
+    c->step_count = 0;
     sampler_resolve(sp, multi_launch_only);              // (environment switches read once per call; part of the graph key through sp)
     c->sp = sp;
     {   // the captured graphs bake in every pointer and scalar below: re-capture when any of them changes
@@ -1547,7 +1558,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
     auto decode_body = [&]() {
         enqueue_lm_head(c);
         launch_sampler(c->sp, batch, s);
-        if (one_launch) enqueue_step(c); else enqueue_layers(c);
+        if (by_step) enqueue_step(c); else enqueue_layers(c);
         collect(0);
     };
     auto capture = [&](hipGraphExec_t* exec, auto&& body) {
@@ -1582,7 +1593,8 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         HIP_CHECK(hipStreamSynchronize(s));
     }
     // ---- decode loop (:714-744)
-    if (c->use_graph && !c->g_decode) capture(&c->g_decode, decode_body);
+    by_step = one_launch && turn.take(c->device);
+    if (!by_step) device_settle(c->device);
     // (Several decode steps per graph launch were measured and removed: between two hipGraphLaunch calls of the one-step graph the
     // device idles for 8.2 us - profiles/r04/c1_gaps.json - and yet eight steps per graph are SLOWER, 2.1047 against 2.0953 ms per step
     // over five A/B runs, profiles/r04/c2_ab.json: a 1376-node graph costs more per node than its seven removed seams save.)
@@ -1596,10 +1608,13 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
     *done_host = 0;
     while (steps < max_tokens) {
         int chunk = std::min(poll, max_tokens - steps);
+        hipGraphExec_t& graph = by_step ? c->g_step : c->g_decode;
+        if (c->use_graph && !graph) capture(&graph, decode_body);
         for (int i = 0; i < chunk; ++i) {
-            if (c->use_graph) HIP_CHECK(hipGraphLaunch(c->g_decode, s)); else decode_body();
+            if (c->use_graph) HIP_CHECK(hipGraphLaunch(graph, s)); else decode_body();
         }
         steps += chunk;
+        if (by_step) c->step_count += chunk;
         HIP_CHECK(hipMemcpyAsync(done_host, c->done_count.p, 4, hipMemcpyDeviceToHost, s));
         sampler_fail_flags_async(c->samp_scratch.p, batch, fail_pin.p, s);
         if (cb) {
@@ -1613,10 +1628,11 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
             // k_samp_cluster).  The reference's loop cannot fail for lack of free compute units (LlamaTTS.swift:714-744): the caller
             // runs the request again on kernels that do not wait for each other.
             sampler_note_failure(c->samp_scratch.p, batch, s);
-            if (one_launch) c->step_off = true;
+            if (by_step) c->step_off = true;
             for (auto& e : ev) (void)hipEventDestroy(e);
             throw SamplerTimeout{};
         }
+        turn.rest();
         if (cb) {
             for (int b = 0; b < batch; ++b)
                 for (; emitted[b] < host_ngen[b]; ++emitted[b]) {
@@ -1627,7 +1643,9 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         }
         if (cancel && *cancel) { cancelled = true; break; }                    // Task.checkCancellation :715
         if (*done_host >= batch) break;
+        if (one_launch) by_step = turn.at_poll();
     }
+    turn.give();
     HIP_CHECK(hipEventRecord(ev[2], s));
     if (cancelled) {
         for (auto& e : ev) (void)hipEventDestroy(e);
@@ -1825,6 +1843,7 @@ static void run_generate(mis_tts* c, const int32_t* prompt_ids, const int32_t* p
                          const mis_gen_params* gp, const float* const* snac_noise, float* pcm_dev, int64_t pcm_stride,
                          bool want_tokens, mis_event_cb cb, void* user, const volatile int* cancel, GenOutputs& out,
                          HiddenMode* hm = nullptr) {
+    DeviceCall call(c ? c->device : -1);
     std::vector<int32_t> emitted(std::max(batch, 1), 0);
     const bool multi_first = c && c->shared_device;
     try {
@@ -1837,6 +1856,7 @@ static void run_generate(mis_tts* c, const int32_t* prompt_ids, const int32_t* p
                              true, emitted);
     }
 }
+extern "C" int32_t mis_debug_tts_step_launches(const mis_tts* c) { return c ? c->step_count : 0; }
 void tts_internal_set_shared_device(mis_tts* c, bool shared) { if (c) c->shared_device = shared; }
 bool tts_internal_shared_device(const mis_tts* c) { return c && c->shared_device; }
 
@@ -1998,6 +2018,7 @@ extern "C" mis_status mis_tts_time_gemm(mis_tts* c, int which, int batch, int it
     static const int attn_ctx = std::max(1, env_int("MIS_TIME_ATTN_CTX", 368));      // mean context of the C3 workload
     if (c->batch != batch || (which == 5 && c->Smax < attn_ctx + 1)) lm_reset(c, batch, which == 5 ? attn_ctx + 1 : 64);
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     const int d = c->d, HD = c->H * c->D, Mpad = c->Mpad;
     if (which == 5) {           // decode attention of every row at context attn_ctx (positions / active flags set once)

@@ -9,7 +9,7 @@ struct StepRole {
     size_t layer;                // bytes from a layer to the next
     int items, K_tiles, pieces, ksb, len;                // items: column tiles, or pairs of gate and up tiles
 };
-enum { SYNC_TAG = 0, SYNC_LOCKED = 1, SYNC_WORDS = 32 };
+enum { SYNC_TAG = 0, SYNC_WORDS = 32 };
 struct StepParams {
     StepRole qkv, o, gu, down;
     const bf16_t *x0, *h0;       // first layer: normalised rows (packed operand), residual stream [Mpad][d]
@@ -21,9 +21,8 @@ struct StepParams {
     const uint8_t* active;
     const float *rope_cos, *rope_sin;
     unsigned char* exch;         // values handed between blocks (step_exch_bytes): cleared, with sync, in front of a request
-    unsigned* sync;              // [SYNC_WORDS]: base of the next launch's tags; whether this handle holds `lock`
+    unsigned* sync;              // [SYNC_WORDS]: base of the next launch's tags
     unsigned* fail;              // sticky: a wait ran out of time (here or in the sampler)
-    unsigned* lock;              // step_lock(device)
     unsigned long long limit;    // ticks of the 100 MHz counter that a wait may take
     int L, d, H, Hkv, Smax, rows, Mpad;
     int schedule2;               // whose bits attention gives: k_attn_decode2's or (caches past 1024 positions) k_attn_decode's
@@ -34,7 +33,3 @@ size_t step_exch_bytes(const StepShape& s);
 // sizes that the launch takes (the device is asked too): otherwise the launch chain
 bool step_ok(const StepShape& s, const StepParams& p, int device);
 void launch_step(const StepParams& p, hipStream_t s);
-// A word per device, for all handles of the process: two launches that each hold part of the compute units and wait for the rest would both run out of time
-unsigned* step_lock(int device);
-// in front of a launch that needs the whole device; that launch gives it back (sync[SYNC_LOCKED])
-void launch_step_lock(unsigned* lock, unsigned* sync, unsigned* fail, hipStream_t s);

@@ -16,11 +16,8 @@
 //    it is there, then all of its own: every block polling all of a vector is as much traffic as the weights (46.3 against 47.5).  Every layer has granules of its own, so none is
 //    overwritten in a launch that reads it; tags grow over the launches of a request and the granules are cleared in front of it.
 //  * Polls end: out of time (StepParams::limit: another stream holds compute units), a block raises `fail`, which all others see, every wave leaves, and the request runs again on the launch
-//    chain.  A lock (k_step_lock) keeps two handles of a process from waiting for each other's compute units.
+//    chain.  Two launches that each hold part of the compute units would wait for each other: a request takes this path while its call is alone on the device (DeviceTurn, common.h).
 #include "lm_step.h"
-
-#include <map>
-#include <mutex>
 
 namespace {
 constexpr int CU = 256, MWAVES = 8, VWAVES = 4, THREADS = (MWAVES + VWAVES) * 64, VT = VWAVES * 64, MAX_ROWS = 2, TAB = 16, VIRT = 8, CPT = 3;
@@ -743,31 +740,12 @@ __global__ void __launch_bounds__(THREADS, 1) k_step_layers(StepParams p) {
         if (wave < MWAVES) matrix_role<RING>(c, wave);
         else vector_role(c, wave - MWAVES);
     }
-    if (cu == 0 && wave == MWAVES && lane == 0) {
-        const StepParams& p = args();
-        if (p.sync[SYNC_LOCKED]) {
-            p.sync[SYNC_LOCKED] = 0;
-            __hip_atomic_store(p.lock, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
 }
 int max_units(const StepParams& p) {
     const int uq = (p.qkv.items + CU - 1) / CU * p.qkv.pieces, ug = 2 * ((p.gu.items + CU - 1) / CU) * p.gu.pieces;
     return std::max(std::max(uq, ug), std::max(p.o.pieces, p.down.pieces));
 }
 int k_max(const StepParams& p) { return 32 * std::max(p.qkv.K_tiles, std::max(p.o.K_tiles, p.down.K_tiles)); }
-// Takes the device's lock; k_step_layers gives it back.  A launch of its own, of one wave in eight registers: it has to find room beside a resident block of k_step_layers (3 x 168
-// registers a SIMD), and leave it, where another handle's launch is yet to start - a wait in k_embed_rmsnorm's blocks would keep that launch from the unit that they wait on.
-constexpr unsigned long long LOCK_LIMIT = 5000000;                         // 50 ms
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_num_vgpr(8))) k_step_lock(unsigned* word, unsigned* sync, unsigned* fail, unsigned long long limit) {
-    if (threadIdx.x) return;
-    const unsigned long long t0 = wall_clock64();
-    while (!__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        if (!__hip_atomic_exchange(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) { sync[SYNC_LOCKED] = 1; return; }
-        if (wall_clock64() - t0 > limit) __hip_atomic_store(fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_sleep(20);
-    }
-}
 
 constexpr int LDS_MAX = 160 * 1024;
 int lds_bytes(const StepParams& p, int ring) { return lds_layout(ring, k_max(p), p.rows, p.H / p.Hkv, max_units(p)).total; }
@@ -799,24 +777,6 @@ bool step_ok(const StepShape& s, const StepParams& p, int device) {
 
 void launch_step(const StepParams& p, hipStream_t s) {
     const int ring = ring_of(p), lds = lds_bytes(p, ring);
-    launch_step_lock(p.lock, p.sync, p.fail, s);
     if (ring == 16) hipLaunchKernelGGL((k_step_layers<16>), dim3(CU), dim3(THREADS), lds, s, p);
     else hipLaunchKernelGGL((k_step_layers<12>), dim3(CU), dim3(THREADS), lds, s, p);
-}
-
-void launch_step_lock(unsigned* lock, unsigned* sync, unsigned* fail, hipStream_t s) { hipLaunchKernelGGL(k_step_lock, dim3(1), dim3(64), 0, s, lock, sync, fail, LOCK_LIMIT); }
-
-unsigned* step_lock(int device) {
-    static std::mutex m;
-    static std::map<int, unsigned*> words;
-    std::lock_guard<std::mutex> g(m);
-    unsigned*& w = words[device];
-    if (!w) {
-        unsigned* p = nullptr;
-        HIP_CHECK(hipMalloc((void**)&p, 128));
-        const unsigned zero[32] = {};
-        HIP_CHECK(copy_now(p, zero, sizeof(zero), hipMemcpyHostToDevice));
-        w = p;
-    }
-    return w;
 }

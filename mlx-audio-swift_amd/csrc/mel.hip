@@ -393,6 +393,7 @@ extern "C" mis_status mis_mel_spectrogram(int device, const mis_mel_config* cfg,
     if (batch == 0 || frames == 0) return MIS_OK;
     MIS_REQUIRE(pcm && out, MIS_ERR_INVALID_INPUT, "null pointer");
     HIP_CHECK(hipSetDevice(device));
+    DeviceCall call(device);
     DevBuf<float> din, dout;
     din.alloc((size_t)batch * n_samples);
     dout.alloc((size_t)batch * frames * cfg->n_mels);
@@ -411,6 +412,7 @@ extern "C" mis_status mis_whisper_encoder_features(int device, const float* pcm,
     if (batch == 0) return MIS_OK;
     MIS_REQUIRE(out && (stride == 0 || pcm), MIS_ERR_INVALID_INPUT, "null pointer");
     HIP_CHECK(hipSetDevice(device));
+    DeviceCall call(device);
     const int64_t W = 480000;                                   // WhisperConfig.swift:188-193
     mis_mel_config c{};
     c.sample_rate = 16000; c.n_fft = 400; c.hop_length = 160; c.n_mels = n_mels;
@@ -479,6 +481,7 @@ extern "C" int64_t mis_mel_stream_total_frames(const mis_mel_stream* h) { return
 
 static int64_t mel_stream_frames(mis_mel_stream* h, const std::vector<float>& signal, int64_t n_frames, float* out_host) {
     HIP_CHECK(hipSetDevice(h->device));
+    DeviceCall call(h->device);
     const mis_mel_config& c = h->cfg;
     MelPlan* pl = get_plan(h->device, c);
     hipStream_t s = h->stream;

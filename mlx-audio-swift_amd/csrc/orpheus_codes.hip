@@ -155,6 +155,7 @@ extern "C" mis_status mis_orpheus_deinterleave(int device, const int32_t* codes7
     MIS_REQUIRE(batch == 0 || groups == 0 || (codes7 && l0 && l1 && l2), MIS_ERR_INVALID_INPUT, "null pointer");
     if (batch == 0 || groups == 0) return MIS_OK;
     HIP_CHECK(hipSetDevice(device));
+    DeviceCall call(device);
     size_t n = (size_t)batch * groups;
     DevBuf<int32_t> din, d0, d1, d2;
     din.alloc(n * 7); d0.alloc(n); d1.alloc(n * 2); d2.alloc(n * 4);
@@ -187,6 +188,7 @@ static mis_status parse_output_host(int device, const int32_t* ids, const int32_
     if (batch == 0) return MIS_OK;
     MIS_REQUIRE(lens && n_codes_out && (stride == 0 || (ids && codes_out)), MIS_ERR_INVALID_INPUT, "null pointer");
     HIP_CHECK(hipSetDevice(device));
+    DeviceCall call(device);
     size_t n = (size_t)batch * (stride ? stride : 1);
     DevBuf<int32_t> din, dl, dout, dn;
     din.alloc(n); dl.alloc(batch); dout.alloc(n); dn.alloc(batch);

@@ -337,6 +337,7 @@ mis_status mis_q3dec_finalize(mis_q3dec* d) {
     MIS_API_BEGIN
     MIS_REQUIRE(!d->finalized, MIS_ERR_INVALID_INPUT, "already finalized");
     HIP_CHECK(hipSetDevice(d->device));
+    DeviceCall call(d->device);
     const mis_qwen3tts_config& cf = d->cfg;
     const int64_t Cd = cf.dec_codebook_dim, half = Cd / 2, bins = cf.dec_codebook_size, nq = cf.dec_num_quantizers,
                   nsem = cf.dec_num_semantic_quantizers, ld = cf.dec_latent_dim, hs = cf.dec_hidden_size, I = cf.dec_intermediate_size,
@@ -666,6 +667,7 @@ void q3dec_stream_begin(mis_q3dec* d, int batch, int cap_frames, int chunk_cap, 
     MIS_REQUIRE(d->finalized, MIS_ERR_NOT_INITIALIZED, "speech tokenizer not finalized");
     MIS_REQUIRE(batch >= 1 && cap_frames >= 1 && chunk_cap >= 1, MIS_ERR_INVALID_INPUT, "bad streaming session sizes");
     HIP_CHECK(hipSetDevice(d->device));
+    DeviceCall call(d->device);
     const mis_qwen3tts_config& cf = d->cfg;
     auto& st = d->st;
     st.open = true; st.dup_bias = dup_bias; st.batch = batch; st.cap_frames = cap_frames; st.pos = 0; st.steps = 0;
@@ -703,6 +705,7 @@ int q3dec_stream_pos(const mis_q3dec* d) { return d->st.open ? d->st.pos : -1; }
 // host entry used by mis_qwen3tts_decode / debug taps: codes host or device [B][nq][T]
 void q3dec_decode_host(mis_q3dec* d, const int32_t* codes, int batch, int T, float* out, int stop_after, int* outC, int64_t* outT, hipStream_t s) {
     HIP_CHECK(hipSetDevice(d->device));
+    DeviceCall call(d->device);
     const int nq = d->cfg.dec_num_quantizers;
     d->codes_dev.alloc((size_t)batch * nq * T);
     HIP_CHECK(hipMemcpyAsync(d->codes_dev.p, codes, (size_t)batch * nq * T * 4, hipMemcpyDefault, s));
@@ -719,6 +722,7 @@ void q3dec_decode_host(mis_q3dec* d, const int32_t* codes, int batch, int T, flo
 // streamingStep from host or device codes [B][nq][Tn] -> out (host or device) [B][Tn * samples_per_frame]
 void q3dec_stream_step_host(mis_q3dec* d, const int32_t* codes, int Tn, float* out, hipStream_t s) {
     HIP_CHECK(hipSetDevice(d->device));
+    DeviceCall call(d->device);
     const int nq = d->cfg.dec_num_quantizers, batch = d->st.batch;
     MIS_REQUIRE(d->st.open, MIS_ERR_NOT_INITIALIZED, "no streaming session is open");
     d->codes_dev.alloc((size_t)batch * nq * Tn);

@@ -288,6 +288,7 @@ static const std::vector<float>& rneed(mis_q3ref* r, const std::string& name, st
 void q3ref_finalize(mis_q3ref* r) {
     MIS_REQUIRE(!r->finalized, MIS_ERR_INVALID_INPUT, "already finalized");
     HIP_CHECK(hipSetDevice(r->device));
+    DeviceCall call(r->device);
     const mis_qwen3tts_reference_config& cf = r->cfg;
     std::vector<float> arena;
     auto push = [&](const std::vector<float>& v) { size_t o = arena.size(); arena.insert(arena.end(), v.begin(), v.end()); while (arena.size() & 3) arena.push_back(0.f); return o; };
@@ -486,6 +487,7 @@ void q3ref_speaker(mis_q3ref* r, const float* audio, int64_t n, int stage, float
     MIS_REQUIRE(r && r->finalized && r->has_spk, MIS_ERR_NOT_INITIALIZED, "this model has no speaker encoder (tts_model_type != base)");
     MIS_REQUIRE(audio && n >= 1, MIS_ERR_INVALID_INPUT, "empty reference audio");
     HIP_CHECK(hipSetDevice(r->device));
+    DeviceCall call(r->device);
     const mis_qwen3tts_reference_config& cf = r->cfg;
     hipStream_t s = r->s;
     mis_mel_config mc{};
@@ -559,6 +561,7 @@ void q3ref_encode(mis_q3ref* r, const float* audio, int64_t n, int stage, float*
     MIS_REQUIRE(r && r->finalized && r->has_enc, MIS_ERR_NOT_INITIALIZED, "this speech tokenizer has no encoder (encoder_config missing)");
     MIS_REQUIRE(audio && n >= 1 && n <= ((int64_t)1 << 25), MIS_ERR_INVALID_INPUT, "bad reference audio length (1 .. 2^25 samples)");
     HIP_CHECK(hipSetDevice(r->device));
+    DeviceCall call(r->device);
     const mis_qwen3tts_reference_config& cf = r->cfg;
     hipStream_t s = r->s;
     const float* W = r->arena.p;

@@ -383,6 +383,7 @@ extern "C" mis_status mis_qwen3tts_finalize(mis_qwen3tts* c) {
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized, MIS_ERR_INVALID_INPUT, "bad handle");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     std::vector<std::string> want = {"model.codec_embedding.weight", "codec_head.weight", "model.text_embedding.weight",
                                      "text_projection.linear_fc1.weight", "text_projection.linear_fc1.bias",
                                      "text_projection.linear_fc2.weight", "text_projection.linear_fc2.bias"};
@@ -443,6 +444,7 @@ void q3_generate_codes(mis_qwen3tts* c, const int32_t* text_ids, const int32_t* 
     MIS_REQUIRE(batch >= 1 && batch <= 64 && P >= 1 && Tt >= 0, MIS_ERR_INVALID_INPUT, "bad batch / prompt sizes");
     MIS_REQUIRE(gp->max_frames >= 1, MIS_ERR_INVALID_INPUT, "max_frames must be positive");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->s;
     const int G = c->G, d = c->d, max_frames = gp->max_frames;
     // ---- host prep: every distinct text position becomes a row of tproj
@@ -644,6 +646,7 @@ extern "C" mis_status mis_qwen3tts_sample_logits(int device, const float* logits
     MIS_API_BEGIN
     MIS_REQUIRE(logits && gp && tokens_out && batch >= 1 && vocab >= 1 && vocab <= 4096, MIS_ERR_INVALID_INPUT, "bad argument");
     HIP_CHECK(hipSetDevice(device));
+    DeviceCall call(device);
     const int Vpad = (int)round_up(vocab, 16), Mpad = (int)round_up(batch, 16);
     std::vector<bf16_t> lb((size_t)Mpad * Vpad, (bf16_t)0);
     for (int b = 0; b < batch; ++b) for (int i = 0; i < vocab; ++i) lb[(size_t)b * Vpad + i] = f32_to_bf16(logits[(size_t)b * vocab + i]);

@@ -1020,6 +1020,7 @@ extern "C" mis_status mis_snac_finalize(mis_snac* c) {
     MIS_REQUIRE(c, MIS_ERR_INVALID_INPUT, "null handle");
     MIS_REQUIRE(!c->finalized, MIS_ERR_INVALID_INPUT, "already finalized");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     const mis_snac_config& cf = c->cfg;
     const int64_t D = cf.latent_dim, CB = cf.codebook_size, CD = cf.codebook_dim;
     std::vector<float> arena;
@@ -1358,6 +1359,7 @@ extern "C" mis_status mis_snac_encode(mis_snac* c, const float* audio, int batch
     MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "SNAC model not finalized");
     MIS_REQUIRE(c->has_encoder, MIS_ERR_AUDIO_ENCODE, "this SNAC handle was loaded without encoder weights");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     codec_run(c->pack, [&] { snac_encode(c, audio, batch, n_samples, codes_out, z_out); });
     MIS_API_END
 }
@@ -1648,6 +1650,7 @@ extern "C" mis_status mis_snac_decode(mis_snac* c, const int32_t* const* codes, 
     if (batch == 0 || t_coarse == 0) return MIS_OK;       // empty input -> empty waveform
     MIS_REQUIRE(codes && pcm_out, MIS_ERR_INVALID_INPUT, "null pointer");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     std::vector<const int32_t*> dcodes;
     std::vector<const float*> dnoise;
     const int64_t N = mis_snac_num_samples(c, t_coarse);
@@ -1680,6 +1683,7 @@ extern "C" mis_status mis_snac_debug_tap(mis_snac* c, const char* name, float* o
     MIS_REQUIRE(c && name && out && channels && length, MIS_ERR_INVALID_INPUT, "null argument");
     MIS_REQUIRE(c->finalized && c->last_batch > 0, MIS_ERR_NOT_INITIALIZED, "no previous decode to tap");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     std::string n = name;
     int stop = -2;
     if (n == "zq") stop = 0;

@@ -263,6 +263,7 @@ extern "C" mis_status mis_soprano_finalize(mis_soprano* c) {
     mis_status st = mis_tts_finalize(c->lm);
     if (st != MIS_OK) return st;
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     const mis_soprano_config& cf = c->cfg;
     const int64_t C = cf.lm.hidden_size, d = cf.decoder_dim, inter = cf.decoder_intermediate_dim, nf = cf.n_fft, bins = nf / 2 + 1;
     const int64_t ik = cf.input_kernel, dk = cf.dw_kernel;
@@ -392,6 +393,7 @@ extern "C" mis_status mis_soprano_decode(mis_soprano* c, const float* hidden, in
     if (batch == 0 || n == 0) return MIS_OK;
     MIS_REQUIRE(hidden && audio_out, MIS_ERR_INVALID_INPUT, "null pointer");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = tts_stream(c->lm);
     const int C = c->cfg.lm.hidden_size;
     DevBuf<float> hd, ad;
@@ -414,6 +416,7 @@ static void soprano_generate_impl(mis_soprano* c, const int32_t* prompt_ids, con
     MIS_REQUIRE(c && prompt_ids && prompt_lens && params, MIS_ERR_INVALID_INPUT, "null argument");
     MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "Soprano model not finalized");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = tts_stream(c->lm);
     mis_gen_params gp = *params;
     gp.sampler_flavor = 1;

@@ -54,7 +54,7 @@ struct mis_whisper {
     DevBuf<WsLayer> step_layers;
     DevBuf<unsigned char> step_exch;
     DevBuf<unsigned> step_sync, step_table;
-    unsigned* step_lock = nullptr;       // the device's, not this handle's
+    int step_count = 0;                  // decode steps of the last request that went as one launch
     bool step_off = false;               // a launch ran out of time: the launch chain from then on
     // encoder workspace (a sub-batch of up to 8 windows), audio and features of a call: kept, they are the same size call after call
     DevBuf<bf16_t> e_col1, e_tight, e_h1, e_col2, e_h, e_x, e_qkv, e_att, e_ff, e_kc, e_vc, e_ckv;
@@ -204,6 +204,7 @@ extern "C" mis_status mis_whisper_finalize(mis_whisper* c) {
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized, MIS_ERR_INVALID_INPUT, "bad handle");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     const int64_t d = c->d, fe = c->cfg.encoder_ffn_dim, fd = c->cfg.decoder_ffn_dim, V = c->V, nm = c->nmel;
     const int Le = c->cfg.encoder_layers, Ld = c->cfg.decoder_layers;
@@ -321,6 +322,7 @@ extern "C" mis_status mis_whisper_init_synthetic(mis_whisper* c, uint64_t seed) 
     MIS_API_BEGIN
     MIS_REQUIRE(c && !c->finalized, MIS_ERR_INVALID_INPUT, "bad handle");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     uint64_t key = seed * 100000ull;
     const int64_t d = c->d, nm = c->nmel;
@@ -509,6 +511,7 @@ extern "C" mis_status mis_whisper_encode(mis_whisper* c, const float* features, 
     MIS_REQUIRE(c && features, MIS_ERR_INVALID_INPUT, "null argument");
     MIS_REQUIRE(batch >= 1 && batch <= 64, MIS_ERR_INVALID_INPUT, "batch per GPU must be 1..64");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     size_t n = (size_t)batch * 3000 * c->nmel;
     c->feats.alloc(n);
     whisper_in(c, c->feats.p, features, n * 4);
@@ -618,18 +621,18 @@ static bool step_params(const mis_whisper* c, WsParams& p) {
     p.layers = c->step_layers.p; p.table = c->step_table.p; p.x0 = c->x.p; p.h0 = c->h.p; p.x_out = c->x.p;
     p.self_k = c->self_k.p; p.self_v = c->self_v.p; p.cross_k = c->cross_k.p; p.cross_v = c->cross_v.p;
     p.self_layer = (size_t)c->batch * c->Hd * c->Smax * c->D; p.cross_layer = (size_t)c->batch * c->Hd * c->Spad * c->D;
-    p.pos = c->pos_cur.p; p.active = c->active.p; p.exch = c->step_exch.p; p.sync = c->step_sync.p; p.fail = &c->scratch.p->c_fail; p.lock = c->step_lock;
+    p.pos = c->pos_cur.p; p.active = c->active.p; p.exch = c->step_exch.p; p.sync = c->step_sync.p; p.fail = &c->scratch.p->c_fail;
     const char* us = getenv("MIS_WHISPER_STEP_US");                        // (tests force the time-out)
     p.limit = us ? 100ull * (unsigned long long)std::max(0, atoi(us)) : 5000000ull;       // 50 ms: a step takes a tenth to one
     p.L = (int)c->dec.size(); p.d = d; p.ff = c->cfg.decoder_ffn_dim; p.H = c->Hd; p.rows = c->batch; p.Smax = c->Smax; p.Spad = c->Spad; p.cross_len = 1500;
     p.eps = LN_EPS; p.scale = 1.0f / sqrtf((float)c->D);
     return ws_plan(p, c->device);
 }
-// Whether a request takes it, and its buffers.  `alone`: no kernel of the request may wait for another block's.
-static bool step_begin(mis_whisper* c, bool alone) {
+// Whether a request may take it, and its buffers.  `apart`: no kernel of the request may wait for another block's.
+static bool step_begin(mis_whisper* c, bool apart) {
     const char* e = getenv("MIS_WHISPER_STEP");                            // 0: the launch chain (parity tests, read per call)
     WsParams p{};
-    if (alone || c->step_off || (e && atoi(e) == 0) || !step_params(c, p)) return false;
+    if (apart || c->step_off || (e && atoi(e) == 0) || !step_params(c, p)) return false;
     if (!c->step_layers.p) {
         std::vector<WsLayer> t;
         for (const DecLayer& l : c->dec)
@@ -641,7 +644,6 @@ static bool step_begin(mis_whisper* c, bool alone) {
     const std::vector<unsigned> table = ws_tables(p);
     c->step_table.alloc(table.size());
     HIP_CHECK(copy_now(c->step_table.p, table.data(), table.size() * 4, hipMemcpyHostToDevice));
-    c->step_lock = step_lock(c->device);
     c->step_exch.alloc(ws_exch_bytes(p));
     c->step_sync.alloc(SYNC_WORDS);
     c->step_exch.zero(c->stream);                                          // (tags begin again)
@@ -678,6 +680,7 @@ extern "C" mis_status mis_whisper_decoder_forward(mis_whisper* c, const int32_t*
     MIS_REQUIRE(c && tokens, MIS_ERR_INVALID_INPUT, "null argument");
     MIS_REQUIRE(c->batch > 0, MIS_ERR_NOT_INITIALIZED, "encode first");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     std::vector<uint8_t> act(c->batch, 1);
     if (active) HIP_CHECK(copy_now(act.data(), active, c->batch, hipMemcpyDefault));
@@ -712,6 +715,7 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     MIS_REQUIRE(batch >= 1 && batch <= 64 && n_prompt >= 1 && stride >= 0, MIS_ERR_INVALID_INPUT, "bad sizes");
     MIS_REQUIRE(stride == 0 || pcm, MIS_ERR_INVALID_INPUT, "null audio");
     HIP_CHECK(hipSetDevice(c->device));
+    DeviceCall call(c->device);
     hipStream_t s = c->stream;
     // ---- features (WhisperAudio.encoderFeatures) on the device, then the encoder
     const int64_t W = 480000;
@@ -756,8 +760,12 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
         // (one upload and no wait between the steps: a step's launches are queued while the one in front runs)
         HIP_CHECK(hipMemcpyAsync(c->prompt_rows.p, prompt_rows.data(), prompt_rows.size() * 4, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipMemcpyAsync(c->active.p, ones.data(), batch, hipMemcpyHostToDevice, s));
-        const bool one_launch = step_begin(c, multi_launch_only);
-        auto layers = [&](const int32_t* ids) { if (one_launch) enqueue_step(c, ids); else enqueue_decoder_step(c, ids); };
+        const bool one_launch = step_begin(c, multi_launch_only);           // where the device is this request's alone: `turn`
+        DeviceTurn turn;
+        bool by_step = one_launch && turn.take(c->device);
+        c->step_count = 0;
+        if (!by_step) device_settle(c->device);
+        auto layers = [&](const int32_t* ids) { if (by_step) enqueue_step(c, ids); else enqueue_decoder_step(c, ids); };
         for (int j = 0; j < n_prompt; ++j) layers(c->prompt_rows.p + (size_t)j * batch);
         // ---- decode loop
         c->tokens_out.alloc((size_t)batch * max_tokens);
@@ -795,23 +803,27 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
             launch_sampler(q, batch, s);
             layers(c->ids.p);
     };
-    hipGraphExec_t gexec = nullptr;
+    hipGraphExec_t graphs[2] = {};                       // layers by launches, as one launch
+    auto drop_graphs = [&] { for (auto& g : graphs) if (g) { (void)hipGraphExecDestroy(g); g = nullptr; } };
     const bool use_graph = getenv("MIS_NO_GRAPH") == nullptr;
     try {
-        if (use_graph) {
+        auto capture = [&](hipGraphExec_t* exec) {
             hipGraph_t g = nullptr;
             HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             try { step_body(); } catch (...) { hipGraph_t dead = nullptr; (void)hipStreamEndCapture(s, &dead); if (dead) (void)hipGraphDestroy(dead); throw; }
             HIP_CHECK(hipStreamEndCapture(s, &g));
-            HIP_CHECK(hipGraphInstantiate(&gexec, g, nullptr, nullptr, 0));
+            HIP_CHECK(hipGraphInstantiate(exec, g, nullptr, nullptr, 0));
             HIP_CHECK(hipGraphDestroy(g));
-        }
+        };
         // stream form: the ids sampled since the last poll are announced in step order per row (the reference decodes them to a
         // text delta per step, WhisperModel.swift:242-254; detokenisation stays with the host); EOT is never announced (:238)
         std::vector<int32_t> h_ng(batch), h_tok;
         const int poll = on_event ? 3 : 7;
         for (int step = 0; step < max_tokens; ++step) {
-            if (use_graph) HIP_CHECK(hipGraphLaunch(gexec, s)); else step_body();
+            hipGraphExec_t& graph = graphs[by_step];
+            if (use_graph && !graph) capture(&graph);
+            if (use_graph) HIP_CHECK(hipGraphLaunch(graph, s)); else step_body();
+            c->step_count += by_step;
             if ((step & poll) == poll || step + 1 == max_tokens) {
                 HIP_CHECK(hipMemcpyAsync(done_host, c->done_count.p, 4, hipMemcpyDeviceToHost, s));
                 sampler_fail_flags_async(c->scratch.p, batch, fail_pin.p, s);
@@ -822,6 +834,7 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
                 }
                 HIP_CHECK(hipStreamSynchronize(s));
                 if (sampler_fail_flags_any(fail_pin.p, batch)) { sampler_failed = true; break; }
+                turn.rest();
                 if (on_event)
                     for (int b = 0; b < batch; ++b)
                         for (; emitted[b] < h_ng[b]; ++emitted[b]) {
@@ -830,15 +843,16 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
                         }
                 if (cancel_flag && *cancel_flag) throw MisError(MIS_ERR_CANCELLED, "transcription cancelled");
                 if (*done_host >= batch) break;
+                if (one_launch) by_step = turn.at_poll();
             }
         }
     } catch (...) {
-        if (gexec) (void)hipGraphExecDestroy(gexec);
+        drop_graphs();
         throw;
     }
-    if (gexec) (void)hipGraphExecDestroy(gexec);
+    drop_graphs();
     HIP_CHECK(hipGetLastError());
-    if (sampler_failed) { sampler_note_failure(c->scratch.p, batch, s); c->step_off = c->step_off || one_launch; }
+    if (sampler_failed) { sampler_note_failure(c->scratch.p, batch, s); c->step_off = c->step_off || by_step; }
     return !sampler_failed;
     };
     if (!attempt(c->shared_device)) {
@@ -868,6 +882,7 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     }
 }
 
+extern "C" int32_t mis_debug_whisper_step_launches(const mis_whisper* c) { return c ? c->step_count : 0; }
 int whisper_internal_device(const mis_whisper* c) { return c ? c->device : -1; }
 void whisper_internal_set_shared_device(mis_whisper* c, bool shared) { if (c) c->shared_device = shared; }
 

@@ -25,7 +25,7 @@ struct WsParams {
     const int* pos;
     const uint8_t* active;
     unsigned char* exch;         // values handed between blocks (ws_exch_bytes): cleared, with sync, in front of a request
-    unsigned *sync, *fail, *lock;                                         // as StepParams'
+    unsigned *sync, *fail;                                                // as StepParams'
     unsigned long long limit;
     int L, d, ff, H, rows, Smax, Spad, cross_len, units, k_max;
     float eps, scale;

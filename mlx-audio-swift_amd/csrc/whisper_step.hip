@@ -3,7 +3,7 @@
 // A step of the launch chain is eight launches a layer, each at its own end: Whisper-tiny's 34 launches of 3 - 10 us are 169 us for weights that stream in 11.  Here blocks stay for all
 // layers and hold what they need of the NEXT matrix or head in registers (weight tiles; a head's 384 KB of cached keys and values on eight waves) while others work.  So streaming lies
 // beside the chain of dependencies, and what is left of that is eight hand-overs a layer.  These are granules as in lm_step.hip: eight bytes, two bfloat16 values and the tag that says
-// whose they are; bounded polls; a lock a device.
+// whose they are; bounded polls; a request alone on the device.
 // A block polls one granule of the values in FRONT of its input, then all of its input: a poll of one granule of the input and then all of it is a round trip more.
 //
 //  * WS_ALL, small models: a block has ONE task, a few column tiles of one matrix, or the self- or cross-attention of one (row, head).
@@ -22,7 +22,7 @@
 #include <type_traits>
 
 namespace {
-// MAX_BLOCKS: a block fills its compute unit's registers, and a few units stay for other handles' waiting k_step_lock
+// MAX_BLOCKS: a block fills its compute unit's registers; with all 256 units 1280 columns at eight rows take 1474 us a step in place of 1536, but 768 at five 398 for 378, 1024 at one 601 for 577
 constexpr int THREADS = 512, WAVES = 8, XPAD = 8, NF = 36, MAX_ROWS = WAVES, D = 64, CJ = 6, SJ = 2, LNG = 5, MAX_BLOCKS = 248;
 // attention: a strip of q | k | v a wave, a wave's scores, then probabilities (f32), their halves (bf16), their sums; the waves' partial results
 constexpr int LDS_MAX = 160 * 1024;
@@ -689,10 +689,6 @@ __global__ void __launch_bounds__(THREADS, 2) k_whisper_step(WsParams) {
     if (blk == 0 && tid == 0) {
         const WsParams& p = args();                               // (the block that ends last: it waits for the others' values)
         p.sync[SYNC_TAG] = tag;
-        if (p.sync[SYNC_LOCKED]) {
-            p.sync[SYNC_LOCKED] = 0;
-            __hip_atomic_store(p.lock, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
     }
 }
 // Pieces to waves, the longest first, each to the wave with the least: fragments of the fullest wave; out: WAVES x NF entries of
@@ -805,7 +801,6 @@ std::vector<unsigned> ws_tables(const WsParams& p) {
 }
 
 void launch_whisper_step(const WsParams& p, hipStream_t s) {
-    launch_step_lock(p.lock, p.sync, p.fail, s);
     if (p.what == WS_SHARED) hipLaunchKernelGGL(k_whisper_step<WS_SHARED>, dim3(p.blocks), dim3(THREADS), lds_bytes(p), s, p);
     else hipLaunchKernelGGL(k_whisper_step<WS_ALL>, dim3(p.blocks), dim3(THREADS), lds_bytes(p), s, p);
 }

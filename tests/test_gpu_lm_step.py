@@ -1,5 +1,5 @@
 """-m gpu: the layers of a decode step as one launch (csrc/lm_step.hip): the bits of the launch chain - tokens, samples, and the logits behind the caches it leaves - over depth,
-rows, contexts at the edges of key tiles and of the chain's waves, a row that has ended, a launch that runs out of time, two handles at once."""
+rows, contexts at the edges of key tiles and of the chain's waves, a row that has ended, a launch that runs out of time, two handles at once.  Each test says which way the steps went."""
 import threading
 
 import numpy as np
@@ -33,6 +33,12 @@ def run(lm, rows, n, tokens):
     return [np.concatenate(pcm), np.concatenate(tok), lm.lm_forward([128258] * rows)]
 
 
+def launches(lm):
+    """Steps of the last request that went as one launch; requests of this process that ran out of time."""
+    lib = mas._lib.lib()
+    return lib.mis_debug_tts_step_launches(lm._h), lib.mis_debug_sampler_failures()
+
+
 def same(a, b):
     return all(np.array_equal(x, y) for x, y in zip(a, b)) and np.isfinite(a[2]).all()
 
@@ -46,24 +52,26 @@ def three():
 @pytest.mark.parametrize("rows,n", [(1, 26), (2, 26), (1, 245), (2, 245), (1, 1018)])
 def test_bits_of_the_launch_chain(monkeypatch, three, rows, n):
     monkeypatch.setenv("MIS_LM_STEP", "0")
-    chain = run(three, rows, n, 21)
+    chain, (none, late) = run(three, rows, n, 21), launches(three)
+    assert none == 0
     monkeypatch.delenv("MIS_LM_STEP")
     for _ in range(2):
-        assert same(run(three, rows, n, 21), chain)
+        assert same(run(three, rows, n, 21), chain) and launches(three) == (21, late)
 
 
 @pytest.mark.parametrize("layers", [1, 2])
 def test_depth(monkeypatch, layers):
     lm = model(layers)
     monkeypatch.setenv("MIS_LM_STEP", "0")
-    chain = run(lm, 2, 40, 70)                                             # more steps than one poll of the host's
+    chain, (_, late) = run(lm, 2, 40, 70), launches(lm)                    # more steps than one poll of the host's
     monkeypatch.delenv("MIS_LM_STEP")
-    assert same(run(lm, 2, 40, 70), chain)
+    assert same(run(lm, 2, 40, 70), chain) and launches(lm) == (70, late)
 
 
 def test_a_row_alone_and_among_others(three):
     """One row (here), two (here) and three (the chain) of the same batch."""
-    a, b, c = run(three, 1, 40, 14), run(three, 2, 40, 14), run(three, 3, 40, 14)
+    (a, na), (b, nb), (c, nc) = [(run(three, r, 40, 14), launches(three)[0]) for r in (1, 2, 3)]
+    assert (na, nb, nc) == (14, 14, 0)
     assert np.array_equal(a[1], b[1][:14]) and np.array_equal(b[1], c[1][:28]) and np.array_equal(a[2][0], b[2][0]) and np.array_equal(b[2], c[2][:2])
 
 
@@ -76,8 +84,9 @@ def test_a_row_that_has_ended(monkeypatch):
     monkeypatch.setenv("MIS_LM_STEP", "0")
     chain = lm.generate_batch(prompts(2, 40), gp, return_tokens=True)
     monkeypatch.delenv("MIS_LM_STEP")
+    late = launches(lm)[1]
     here = lm.generate_batch(prompts(2, 40), gp, return_tokens=True)
-    assert len(chain[1][1]) < len(chain[1][0])
+    assert launches(lm) == (28, late) and len(chain[1][1]) < len(chain[1][0])
     assert all(np.array_equal(x, y) for i in range(2) for x, y in zip(chain[i], here[i]))
 
 
@@ -85,17 +94,18 @@ def test_out_of_time_runs_on_the_chain(monkeypatch):
     """No time to wait at all: the first poll in vain ends every launch, the request runs again on the launch chain, and so do the handle's later ones."""
     lm = model(2)
     monkeypatch.setenv("MIS_LM_STEP", "0")
-    chain = run(lm, 1, 40, 14)
+    chain, (_, late) = run(lm, 1, 40, 14), launches(lm)
     monkeypatch.delenv("MIS_LM_STEP")
     monkeypatch.setenv("MIS_LM_STEP_US", "0")
-    assert same(run(lm, 1, 40, 14), chain)
+    assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (0, late + 1)
     monkeypatch.delenv("MIS_LM_STEP_US")
-    assert same(run(lm, 1, 40, 14), chain)
+    assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (0, late + 1)
 
 
 def test_two_handles_at_once(three):
     other = model(3)
-    want = run(three, 1, 40, 70)
+    want, (steps, late) = run(three, 1, 40, 70), launches(three)
+    assert steps == 70
     got = {}
 
     def work(name, lm):
@@ -105,4 +115,24 @@ def test_two_handles_at_once(three):
         t.start()
     for t in threads:
         t.join()
-    assert all(same(r, want) for k in "ab" for r in got[k])
+    assert all(same(r, want) for k in "ab" for r in got[k]) and launches(three)[1] == late        # neither waits for the other's compute units
+
+
+def test_another_call_beside_a_request(three):
+    """From the first poll behind another handle's call on, the launch chain, and the same tokens."""
+    cfg = mas.SNACConfig(**SMALL)
+    codec = mas.SNAC.from_weights(cfg, snac_synthetic_weights(cfg, seed=1))
+    codes = [np.zeros((1, k), np.int32) for k in (1, 2, 4)]
+    codec.decode(codes)
+    gp = mas.GenerateParameters(max_tokens=600, seed=5, temperature=0.8, frame_constrained=2)
+    want = three.generate_batch(prompts(1, 40), gp, return_tokens=True)[1][0]
+    steps, late = launches(three)
+    assert steps >= len(want) > 500
+    got = []
+    for e in three.generate_stream_batch(prompts(1, 40), gp):
+        if hasattr(e, "token"):
+            got.append(e.token)
+            if len(got) == 1:
+                codec.decode(codes)
+    here = launches(three)
+    assert np.array_equal(got, want) and 0 < here[0] < steps and here[1] == late

@@ -1,5 +1,5 @@
 """-m gpu: a Whisper decoder step's layers as one launch (csrc/whisper_step.hip): the bits of the launch chain - token ids, and the logits behind the caches it leaves - over widths, depth,
-rows, splits of K, positions past a wave's first tile of keys, rows that end, a launch that runs out of time, two handles at once."""
+rows, splits of K, positions past a wave's first tile of keys, rows that end, a launch that runs out of time, two handles at once.  Each test says which way the steps went."""
 import threading
 
 import numpy as np
@@ -24,6 +24,12 @@ def run(m, rows, tokens, eot=699, seed=3):
     return ids, m.decoder_forward([5 + b for b in range(rows)])
 
 
+def launches(m):
+    """Steps of the last request that went as one launch; requests of this process that ran out of time."""
+    lib = mas._lib.lib()
+    return lib.mis_debug_whisper_step_launches(m._h), lib.mis_debug_sampler_failures()
+
+
 def same(a, b):
     return a[0] == b[0] and np.array_equal(a[1], b[1]) and np.isfinite(a[1]).all()
 
@@ -34,27 +40,30 @@ def same(a, b):
 def test_bits_of_the_launch_chain(monkeypatch, d, layers, rows):
     m = model(d, layers)
     monkeypatch.setenv("MIS_WHISPER_STEP", "0")
-    chain = run(m, rows, 36)
+    chain, (none, late) = run(m, rows, 36), launches(m)
+    assert none == 0
     monkeypatch.delenv("MIS_WHISPER_STEP")
     for _ in range(2):
-        assert same(run(m, rows, 36), chain)
+        assert same(run(m, rows, 36), chain) and launches(m) == (36, late)
 
 
 def test_positions_past_the_first_tiles(monkeypatch):
     for d, rows in ((384, 2), (1280, 4)):
         m = model(d, 2)
         monkeypatch.setenv("MIS_WHISPER_STEP", "0")
-        chain = run(m, rows, 330)
+        chain, (_, late) = run(m, rows, 330), launches(m)
         monkeypatch.delenv("MIS_WHISPER_STEP")
-        assert same(run(m, rows, 330), chain)
+        assert same(run(m, rows, 330), chain) and launches(m) == (330, late)
 
 
 @pytest.mark.parametrize("d,more_rows", [(384, (2, 4, 6, 9)), (1280, (2, 5))])    # nine: the launch chain
 def test_a_row_alone_and_among_others(d, more_rows):
     m = model(d, 2)
     ids, logits = run(m, 1, 20)
+    assert launches(m)[0] == 20
     for rows in more_rows:
         more, lm = run(m, rows, 20)
+        assert launches(m)[0] == (20 if rows <= 8 else 0)
         assert more[0] == ids[0] and np.array_equal(lm[0], logits[0])
 
 
@@ -64,27 +73,52 @@ def test_a_row_that_ends(monkeypatch, d, rows):
     full = run(m, rows, 24)[0]
     ends = [t for t in full[1][6:] if t not in full[0]][:1] or [full[1][6]]
     monkeypatch.setenv("MIS_WHISPER_STEP", "0")
-    chain = run(m, rows, 24, eot=ends[0])[0]
+    chain, (_, late) = run(m, rows, 24, eot=ends[0])[0], launches(m)
     monkeypatch.delenv("MIS_WHISPER_STEP")
     assert run(m, rows, 24, eot=ends[0])[0] == chain and chain != full
+    steps, after = launches(m)
+    assert 0 < steps <= 24 and after == late
 
 
 @pytest.mark.parametrize("d,rows", [(384, 2), (1280, 4)])
 def test_out_of_time_runs_on_the_chain(monkeypatch, d, rows):
     m = model(d, 2)
-    want = run(m, rows, 20)
+    want, (steps, late) = run(m, rows, 20), launches(m)
+    assert steps == 20
     monkeypatch.setenv("MIS_WHISPER_STEP_US", "0")                         # the first poll in vain ends the launch
     got = run(m, rows, 20)
     monkeypatch.delenv("MIS_WHISPER_STEP_US")
-    assert same(got, want) and same(run(m, rows, 20), want)
+    assert same(got, want) and launches(m) == (0, late + 1)
+    assert same(run(m, rows, 20), want) and launches(m) == (0, late + 1)
 
 
 @pytest.mark.parametrize("d,rows", [(768, 2), (1280, 4)])
 def test_two_handles_at_once(d, rows):
     ms, rows = [model(384, 2), model(d, 2)], [2, rows]
     want = [run(m, r, 60) for m, r in zip(ms, rows)]
+    late = launches(ms[0])[1]
+    assert [launches(m)[0] for m in ms] == [60, 60]
     got = [[], []]
     ts = [threading.Thread(target=lambda i=i: got[i].extend(run(ms[i], rows[i], 60) for _ in range(3))) for i in range(2)]
     [t.start() for t in ts]
     [t.join() for t in ts]
-    assert all(same(g, want[i]) for i in range(2) for g in got[i])
+    assert all(same(g, want[i]) for i in range(2) for g in got[i]) and launches(ms[0])[1] == late        # neither waits for the other's compute units
+
+
+def test_another_call_beside_a_request():
+    """From the first poll behind another handle's call on, the launch chain, and the same tokens."""
+    m, other = model(384, 4), model(128, 1)
+    window, features = (0.1 * np.random.default_rng(3).standard_normal(16000)).astype(np.float32), np.zeros((1, 3000, 80), np.float32)
+    gp = mas.STTGenerateParameters(max_tokens=400, temperature=0.0, seed=5, eot_id=699, timestamp_begin=695)
+    other.encode(features)
+    want = m.transcribe_windows([window], PROMPT, gp)[0]
+    steps, late = launches(m)
+    assert steps >= len(want) > 300
+    got = []
+    for e in m.transcribe_windows_stream([window], PROMPT, gp):
+        if hasattr(e, "token"):
+            got.append(e.token)
+            if len(got) == 1:
+                other.encode(features)
+    here = launches(m)
+    assert got == list(want) and 0 < here[0] < steps and here[1] == late
