@@ -83,7 +83,7 @@ struct mis_tts {
     DevBuf<unsigned char> step_exch;             // decode steps in one launch (lm_step.hip): values handed between blocks, flags
     DevBuf<unsigned> step_sync;
     int step_count = 0;                          // decode steps of the last request that went as one launch
-    bool step_off = false;                       // a launch has timed out: this handle stays on the launch chain
+    StepPause step_pause;
     HostRing ring;
     hipGraphExec_t g_prefill = nullptr, g_decode = nullptr, g_step = nullptr;   // g_step: a decode step whose layers are one launch
     bool shared_device = false;      // another replica's streams run on this device (group.hip): never a kernel that waits for co-resident blocks
@@ -816,7 +816,7 @@ static bool step_begin(mis_tts* c, bool apart) {
     const StepShape shape{c->L, c->d, c->ff, c->H, c->Hkv, c->D, c->batch};
     const char* e = getenv("MIS_LM_STEP");                                 // 0: the launch chain (parity tests, read per call)
     StepParams p{};
-    if (apart || c->step_off || (e && atoi(e) == 0) || !step_params(c, p) || !step_ok(shape, p, c->device)) return false;
+    if (apart || (e && atoi(e) == 0) || !step_params(c, p) || !step_ok(shape, p, c->device) || !c->step_pause.due()) return false;
     c->step_exch.alloc(step_exch_bytes(shape));
     c->step_sync.alloc(SYNC_WORDS);
     c->step_exch.zero(c->stream);                                          // (tags begin again)
@@ -1628,7 +1628,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
             // k_samp_cluster).  The reference's loop cannot fail for lack of free compute units (LlamaTTS.swift:714-744): the caller
             // runs the request again on kernels that do not wait for each other.
             sampler_note_failure(c->samp_scratch.p, batch, s);
-            if (by_step) c->step_off = true;
+            if (by_step) step_was_late(c->step_sync.p, c->step_pause, "speech model");
             for (auto& e : ev) (void)hipEventDestroy(e);
             throw SamplerTimeout{};
         }
@@ -1646,6 +1646,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         if (one_launch) by_step = turn.at_poll();
     }
     turn.give();
+    if (c->step_count) c->step_pause.fine();
     HIP_CHECK(hipEventRecord(ev[2], s));
     if (cancelled) {
         for (auto& e : ev) (void)hipEventDestroy(e);

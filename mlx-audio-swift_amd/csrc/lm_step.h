@@ -9,7 +9,7 @@ struct StepRole {
     size_t layer;                // bytes from a layer to the next
     int items, K_tiles, pieces, ksb, len;                // items: column tiles, or pairs of gate and up tiles
 };
-enum { SYNC_TAG = 0, SYNC_WORDS = 32 };
+enum { SYNC_TAG = 0, SYNC_LATE = 1, SYNC_WORDS = 32 };
 struct StepParams {
     StepRole qkv, o, gu, down;
     const bf16_t *x0, *h0;       // first layer: normalised rows (packed operand), residual stream [Mpad][d]
@@ -21,7 +21,7 @@ struct StepParams {
     const uint8_t* active;
     const float *rope_cos, *rope_sin;
     unsigned char* exch;         // values handed between blocks (step_exch_bytes): cleared, with sync, in front of a request
-    unsigned* sync;              // [SYNC_WORDS]: base of the next launch's tags
+    unsigned* sync;              // [SYNC_WORDS]: base of the next launch's tags; whether a wait of a step ran out of time
     unsigned* fail;              // sticky: a wait ran out of time (here or in the sampler)
     unsigned long long limit;    // ticks of the 100 MHz counter that a wait may take
     int L, d, H, Hkv, Smax, rows, Mpad;
@@ -33,3 +33,13 @@ size_t step_exch_bytes(const StepShape& s);
 // sizes that the launch takes (the device is asked too): otherwise the launch chain
 bool step_ok(const StepShape& s, const StepParams& p, int device);
 void launch_step(const StepParams& p, hipStream_t s);
+// Steps that ran out of time: something that is no call of this process holds compute units (another process, another library's kernels).  The handle's next request stays on the launch
+// chain; the next two, four, .. up to 64 if it goes on; a request that gets through ends that.
+struct StepPause {
+    int skip = 0, next = 1;
+    bool due() { return skip == 0 || (--skip, false); }
+    void late() { skip = next; next = std::min(2 * next, 64); }
+    void fine() { next = 1; }
+};
+// behind a raised `fail`: whether it was a step's wait, on which `pause` then begins (one line to stderr); the launches have ended
+bool step_was_late(const unsigned* sync, StepPause& pause, const char* what);

@@ -19,6 +19,8 @@
 //    chain.  Two launches that each hold part of the compute units would wait for each other: a request takes this path while its call is alone on the device (DeviceTurn, common.h).
 #include "lm_step.h"
 
+#include <stdio.h>
+
 namespace {
 constexpr int CU = 256, MWAVES = 8, VWAVES = 4, THREADS = (MWAVES + VWAVES) * 64, VT = VWAVES * 64, MAX_ROWS = 2, TAB = 16, VIRT = 8, CPT = 3;
 constexpr int AHEAD = 3, FLIGHT = 3;
@@ -142,7 +144,10 @@ struct Ctx {
         if (t0 == 0) t0 = now;
         if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(p.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) return false;
         if (now - t0 < p.limit) return true;
-        if (lane == 0) __hip_atomic_store(p.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0) {
+            __hip_atomic_store(p.sync + SYNC_LATE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(p.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         return false;
     }
 };
@@ -779,4 +784,14 @@ void launch_step(const StepParams& p, hipStream_t s) {
     const int ring = ring_of(p), lds = lds_bytes(p, ring);
     if (ring == 16) hipLaunchKernelGGL((k_step_layers<16>), dim3(CU), dim3(THREADS), lds, s, p);
     else hipLaunchKernelGGL((k_step_layers<12>), dim3(CU), dim3(THREADS), lds, s, p);
+}
+
+bool step_was_late(const unsigned* sync, StepPause& pause, const char* what) {
+    unsigned late = 0;
+    HIP_CHECK(copy_now(&late, sync + SYNC_LATE, sizeof(late), hipMemcpyDeviceToHost));
+    if (!late) return false;
+    pause.late();
+    fprintf(stderr, "mi_speech: a %s step waited in vain for compute units (held from outside this library); its request runs again on the launch chain, and so do the handle's next %d\n", what,
+            pause.skip);
+    return true;
 }

@@ -55,7 +55,7 @@ struct mis_whisper {
     DevBuf<unsigned char> step_exch;
     DevBuf<unsigned> step_sync, step_table;
     int step_count = 0;                  // decode steps of the last request that went as one launch
-    bool step_off = false;               // a launch ran out of time: the launch chain from then on
+    StepPause step_pause;
     // encoder workspace (a sub-batch of up to 8 windows), audio and features of a call: kept, they are the same size call after call
     DevBuf<bf16_t> e_col1, e_tight, e_h1, e_col2, e_h, e_x, e_qkv, e_att, e_ff, e_kc, e_vc, e_ckv;
     DevBuf<float> pcm, padded, feats, enc_f32;
@@ -632,7 +632,7 @@ static bool step_params(const mis_whisper* c, WsParams& p) {
 static bool step_begin(mis_whisper* c, bool apart) {
     const char* e = getenv("MIS_WHISPER_STEP");                            // 0: the launch chain (parity tests, read per call)
     WsParams p{};
-    if (apart || c->step_off || (e && atoi(e) == 0) || !step_params(c, p)) return false;
+    if (apart || (e && atoi(e) == 0) || !step_params(c, p) || !c->step_pause.due()) return false;
     if (!c->step_layers.p) {
         std::vector<WsLayer> t;
         for (const DecLayer& l : c->dec)
@@ -852,7 +852,10 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     }
     drop_graphs();
     HIP_CHECK(hipGetLastError());
-    if (sampler_failed) { sampler_note_failure(c->scratch.p, batch, s); c->step_off = c->step_off || by_step; }
+    if (sampler_failed) {
+        sampler_note_failure(c->scratch.p, batch, s);
+        if (by_step) step_was_late(c->step_sync.p, c->step_pause, "Whisper");
+    } else if (c->step_count) c->step_pause.fine();
     return !sampler_failed;
     };
     if (!attempt(c->shared_device)) {

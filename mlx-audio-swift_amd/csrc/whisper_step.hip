@@ -85,7 +85,10 @@ __device__ __forceinline__ bool more_time(u64& t0, int lane) {
     if (t0 == 0) t0 = now;
     if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(p.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) return false;
     if (now - t0 < p.limit) return true;
-    if (lane == 0) __hip_atomic_store(p.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0) {
+        __hip_atomic_store(p.sync + SYNC_LATE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(p.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     return false;
 }
 // `one`, the same for all lanes of the wave, until it carries `tag`

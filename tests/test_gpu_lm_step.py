@@ -91,7 +91,7 @@ def test_a_row_that_has_ended(monkeypatch):
 
 
 def test_out_of_time_runs_on_the_chain(monkeypatch):
-    """No time to wait at all: the first poll in vain ends every launch, the request runs again on the launch chain, and so do the handle's later ones."""
+    """No time to wait at all: the first poll in vain ends every launch, the request runs again on the launch chain; the next request stays there, two after a second time-out in a row."""
     lm = model(2)
     monkeypatch.setenv("MIS_LM_STEP", "0")
     chain, (_, late) = run(lm, 1, 40, 14), launches(lm)
@@ -100,6 +100,27 @@ def test_out_of_time_runs_on_the_chain(monkeypatch):
     assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (0, late + 1)
     monkeypatch.delenv("MIS_LM_STEP_US")
     assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (0, late + 1)
+    monkeypatch.setenv("MIS_LM_STEP_US", "0")
+    assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (0, late + 2)
+    monkeypatch.delenv("MIS_LM_STEP_US")
+    for steps in (0, 0, 14, 14):
+        assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (steps, late + 2)
+    monkeypatch.setenv("MIS_LM_STEP_US", "0")                              # it got through in between: one request again
+    assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (0, late + 3)
+    monkeypatch.delenv("MIS_LM_STEP_US")
+    for steps in (0, 14):
+        assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (steps, late + 3)
+
+
+def test_a_time_out_of_the_sampler_is_not_the_steps(monkeypatch):
+    """A barrier of the one-launch sampler runs out of time: that request runs again, the next one has its steps in one launch."""
+    lm = model(2)
+    want, (steps, late) = run(lm, 1, 40, 14), launches(lm)
+    assert steps == 14
+    monkeypatch.setenv("MIS_SAMPLER_SPIN", "0")
+    assert same(run(lm, 1, 40, 14), want) and launches(lm) == (0, late + 1)
+    monkeypatch.delenv("MIS_SAMPLER_SPIN")
+    assert same(run(lm, 1, 40, 14), want) and launches(lm) == (14, late + 1)
 
 
 def test_two_handles_at_once(three):
