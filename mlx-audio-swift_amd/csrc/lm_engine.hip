@@ -811,14 +811,22 @@ static bool step_params(const mis_tts* c, StepParams& p) {
     p.eps = c->cfg.rms_norm_eps; p.scale = 1.0f / sqrtf((float)c->D);
     return true;
 }
-// Whether a request may take it, and its buffers.  `apart`: no kernel of the request may wait for another block's (the second attempt behind a time-out, a device shared by replicas).
+static void step_release(mis_tts* c) {
+    destroy_graphs(c);
+    c->graph_key = 0;
+    c->step_exch.release();
+    c->step_sync.release();
+}
+// Whether a request may take it, and its buffers (no room for them: it does not).  `apart`: no kernel of the request may wait for another block's (the second attempt behind a time-out, a device shared by replicas).
 static bool step_begin(mis_tts* c, bool apart) {
     const StepShape shape{c->L, c->d, c->ff, c->H, c->Hkv, c->D, c->batch};
     const char* e = getenv("MIS_LM_STEP");                                 // 0: the launch chain (parity tests, read per call)
     StepParams p{};
     if (apart || (e && atoi(e) == 0) || !step_params(c, p) || !step_ok(shape, p, c->device) || !c->step_pause.due()) return false;
-    c->step_exch.alloc(step_exch_bytes(shape));
-    c->step_sync.alloc(SYNC_WORDS);
+    try {
+        c->step_exch.alloc(step_exch_bytes(shape));
+        c->step_sync.alloc(SYNC_WORDS);
+    } catch (const MisNoMemory&) { step_release(c); return false; }
     c->step_exch.zero(c->stream);                                          // (tags begin again)
     c->step_sync.zero(c->stream);
     return true;
@@ -1428,7 +1436,7 @@ struct SamplerTimeout {};
 static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const int32_t* prompt_lens, int batch,
                                  const mis_gen_params* gp, const float* const* snac_noise, float* pcm_dev, int64_t pcm_stride,
                                  bool want_tokens, mis_event_cb cb, void* user, const volatile int* cancel, GenOutputs& out,
-                                 HiddenMode* hm, bool multi_launch_only, std::vector<int32_t>& emitted) {
+                                 HiddenMode* hm, bool multi_launch_only, bool no_step, std::vector<int32_t>& emitted) {
     MIS_REQUIRE(c && c->finalized, MIS_ERR_NOT_INITIALIZED, "model not initialized");
     const bool hidden_mode = hm && hm->on, collect_hidden = hidden_mode && hm->hidden;
     MIS_REQUIRE(!c->blocks || (hidden_mode && !collect_hidden), MIS_ERR_INVALID_INPUT, "this architecture generates tokens (mis_lm_generate)");
@@ -1518,7 +1526,7 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
         HIP_CHECK(hipMemcpyAsync(hid_count.p, ones_i.data(), batch * 4, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipStreamSynchronize(s));
     }
-    const bool one_launch = step_begin(c, multi_launch_only);           // where the device is this request's alone: `turn`
+    const bool one_launch = step_begin(c, multi_launch_only || no_step);           // where the device is this request's alone: `turn`
     DeviceTurn turn;
     bool by_step = false;
     c->step_count = 0;
@@ -1840,21 +1848,29 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
 // the step that needs that), the whole request once more on the multi-launch sampler - the request is deterministic, the second
 // attempt's tokens are the ones the first would have produced, and the callback continues behind what it has already been told.
 // A handle that shares its device with another replica's streams never takes the one-launch path in the first place.
+// Where it runs out of memory with the step's buffers held, it gives them back and runs once more on the launch chain.
 static void run_generate(mis_tts* c, const int32_t* prompt_ids, const int32_t* prompt_lens, int batch,
                          const mis_gen_params* gp, const float* const* snac_noise, float* pcm_dev, int64_t pcm_stride,
                          bool want_tokens, mis_event_cb cb, void* user, const volatile int* cancel, GenOutputs& out,
                          HiddenMode* hm = nullptr) {
     DeviceCall call(c ? c->device : -1);
     std::vector<int32_t> emitted(std::max(batch, 1), 0);
-    const bool multi_first = c && c->shared_device;
-    try {
-        run_generate_attempt(c, prompt_ids, prompt_lens, batch, gp, snac_noise, pcm_dev, pcm_stride, want_tokens, cb, user, cancel, out, hm,
-                             multi_first, emitted);
-    } catch (const SamplerTimeout&) {
-        MIS_REQUIRE(!multi_first, MIS_ERR_GENERATION_FAILED, "sampler: time-out flag raised on the multi-launch path");   // (cannot happen: nothing spins there)
+    bool apart = c && c->shared_device, no_step = false;
+    for (;;) {
+        try {
+            run_generate_attempt(c, prompt_ids, prompt_lens, batch, gp, snac_noise, pcm_dev, pcm_stride, want_tokens, cb, user, cancel, out, hm,
+                                 apart, no_step, emitted);
+            return;
+        } catch (const SamplerTimeout&) {
+            MIS_REQUIRE(!apart, MIS_ERR_GENERATION_FAILED, "sampler: time-out flag raised on the multi-launch path");   // (cannot happen: nothing spins there)
+            apart = true;
+        } catch (const MisNoMemory&) {
+            if (!c || !c->step_exch.p) throw;
+            HIP_CHECK(hipStreamSynchronize(c->stream));
+            step_release(c);
+            no_step = true;
+        }
         out = GenOutputs{};
-        run_generate_attempt(c, prompt_ids, prompt_lens, batch, gp, snac_noise, pcm_dev, pcm_stride, want_tokens, cb, user, cancel, out, hm,
-                             true, emitted);
     }
 }
 extern "C" int32_t mis_debug_tts_step_launches(const mis_tts* c) { return c ? c->step_count : 0; }

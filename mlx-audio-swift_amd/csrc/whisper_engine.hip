@@ -628,24 +628,30 @@ static bool step_params(const mis_whisper* c, WsParams& p) {
     p.eps = LN_EPS; p.scale = 1.0f / sqrtf((float)c->D);
     return ws_plan(p, c->device);
 }
-// Whether a request may take it, and its buffers.  `apart`: no kernel of the request may wait for another block's.
+static void step_release(mis_whisper* c) {
+    c->step_layers.release(); c->step_table.release(); c->step_exch.release(); c->step_sync.release();
+}
+// Whether a request may take it, and its buffers (no room for them: it does not).  `apart`: no kernel of the request may wait for another block's.
 static bool step_begin(mis_whisper* c, bool apart) {
     const char* e = getenv("MIS_WHISPER_STEP");                            // 0: the launch chain (parity tests, read per call)
     WsParams p{};
     if (apart || (e && atoi(e) == 0) || !step_params(c, p) || !c->step_pause.due()) return false;
-    if (!c->step_layers.p) {
+    const std::vector<unsigned> table = ws_tables(p);
+    const bool new_layers = !c->step_layers.p;
+    try {
+        c->step_layers.alloc(c->dec.size() + 1);
+        c->step_table.alloc(table.size());
+        c->step_exch.alloc(ws_exch_bytes(p));
+        c->step_sync.alloc(SYNC_WORDS);
+    } catch (const MisNoMemory&) { step_release(c); return false; }
+    if (new_layers) {
         std::vector<WsLayer> t;
         for (const DecLayer& l : c->dec)
             t.push_back({{l.sqkv, l.so, l.cq, l.co, l.fc1, l.fc2}, {l.sbqkv, l.sbo, l.cbq, l.cbo, l.b1, l.b2}, {l.ln1w, l.ln2w, l.ln3w}, {l.ln1b, l.ln2b, l.ln3b}});
         t.push_back({{}, {}, {c->dec_lnw}, {c->dec_lnb}});
-        c->step_layers.alloc(t.size());
         HIP_CHECK(copy_now(c->step_layers.p, t.data(), t.size() * sizeof(WsLayer), hipMemcpyHostToDevice));
     }
-    const std::vector<unsigned> table = ws_tables(p);
-    c->step_table.alloc(table.size());
     HIP_CHECK(copy_now(c->step_table.p, table.data(), table.size() * 4, hipMemcpyHostToDevice));
-    c->step_exch.alloc(ws_exch_bytes(p));
-    c->step_sync.alloc(SYNC_WORDS);
     c->step_exch.zero(c->stream);                                          // (tags begin again)
     c->step_sync.zero(c->stream);
     return step_params(c, c->step);                                        // (with the buffers)
@@ -706,10 +712,11 @@ extern "C" mis_status mis_whisper_decoder_forward(mis_whisper* c, const int32_t*
 
 // transcribeChunk for a batch of <= 30 s windows (WhisperModel.swift:186-282): mel -> encoder -> prompt prefill ->
 // greedy / temperature loop with the suppress masks, until EOT or max_tokens.  Token ids only; text stays host side.
-static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_t* lens, int batch, int64_t stride,
+// `emitted`: ids already announced to the callback, a row each (kept across a second attempt)
+static void whisper_generate_once(mis_whisper* c, const float* pcm, const int64_t* lens, int batch, int64_t stride,
                                   const int32_t* prompt_ids, int n_prompt, const mis_stt_params* sp,
                                   int32_t** tokens_out, int64_t* tokens_stride, int32_t* n_tokens, mis_event_cb on_event, void* user,
-                                  const volatile int* cancel_flag) {
+                                  const volatile int* cancel_flag, bool no_step, std::vector<int32_t>& emitted) {
     MIS_REQUIRE(c && prompt_ids && sp, MIS_ERR_INVALID_INPUT, "null argument");
     MIS_REQUIRE(c->finalized, MIS_ERR_NOT_INITIALIZED, "model not finalized");
     MIS_REQUIRE(batch >= 1 && batch <= 64 && n_prompt >= 1 && stride >= 0, MIS_ERR_INVALID_INPUT, "bad sizes");
@@ -751,7 +758,6 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     for (size_t i = 0; i < prompt_rows.size(); ++i) prompt_rows[i] = prompt[i / batch];
     c->prompt_rows.alloc(prompt_rows.size());
     for (int j = 0; j < n_prompt; ++j) MIS_REQUIRE(prompt[j] >= 0 && prompt[j] < c->V, MIS_ERR_INVALID_INPUT, "prompt token outside the vocabulary");
-    std::vector<int32_t> emitted(batch, 0);              // ids already announced to the callback (kept across a second attempt)
     // One attempt of prompt prefill + decode loop on the encoder output already in place.  Returns false when a row barrier of the
     // one-launch sampler timed out (its blocks were not co-resident: another stream holds compute units) - seen at the poll, before any
     // id of that poll interval is announced; the caller resets the decoder state and runs the attempt again on the multi-launch
@@ -760,7 +766,7 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
         // (one upload and no wait between the steps: a step's launches are queued while the one in front runs)
         HIP_CHECK(hipMemcpyAsync(c->prompt_rows.p, prompt_rows.data(), prompt_rows.size() * 4, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipMemcpyAsync(c->active.p, ones.data(), batch, hipMemcpyHostToDevice, s));
-        const bool one_launch = step_begin(c, multi_launch_only);           // where the device is this request's alone: `turn`
+        const bool one_launch = step_begin(c, multi_launch_only || no_step);           // where the device is this request's alone: `turn`
         DeviceTurn turn;
         bool by_step = one_launch && turn.take(c->device);
         c->step_count = 0;
@@ -885,6 +891,21 @@ static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_
     }
 }
 
+// Where it runs out of memory with the step's buffers held, it gives them back and runs once more on the launch chain (deterministic, as behind a time-out).
+static void whisper_generate_impl(mis_whisper* c, const float* pcm, const int64_t* lens, int batch, int64_t stride,
+                                  const int32_t* prompt_ids, int n_prompt, const mis_stt_params* sp,
+                                  int32_t** tokens_out, int64_t* tokens_stride, int32_t* n_tokens, mis_event_cb on_event, void* user,
+                                  const volatile int* cancel_flag) {
+    std::vector<int32_t> emitted(std::min(std::max(batch, 1), 64), 0);
+    auto once = [&](bool no_step) {
+        whisper_generate_once(c, pcm, lens, batch, stride, prompt_ids, n_prompt, sp, tokens_out, tokens_stride, n_tokens, on_event, user, cancel_flag, no_step, emitted);
+    };
+    try { once(false); return; }
+    catch (const MisNoMemory&) { if (!c->step_exch.p) throw; }
+    HIP_CHECK(hipStreamSynchronize(c->stream));
+    step_release(c);
+    once(true);
+}
 extern "C" int32_t mis_debug_whisper_step_launches(const mis_whisper* c) { return c ? c->step_count : 0; }
 int whisper_internal_device(const mis_whisper* c) { return c ? c->device : -1; }
 void whisper_internal_set_shared_device(mis_whisper* c, bool shared) { if (c) c->shared_device = shared; }

@@ -28,9 +28,13 @@ def prompts(rows, n):
     return [np.concatenate([[128259], r.integers(0, 128000, n - 4 - 3 * b), [128009, 128260, 128257]]).astype(np.int32) for b in range(rows)]
 
 
-def run(lm, rows, n, tokens):
+def generate(lm, rows, n, tokens):
     pcm, tok = lm.generate_batch(prompts(rows, n), mas.GenerateParameters(max_tokens=tokens, seed=5, temperature=0.8, frame_constrained=2), return_tokens=True)
-    return [np.concatenate(pcm), np.concatenate(tok), lm.lm_forward([128258] * rows)]
+    return [np.concatenate(pcm), np.concatenate(tok)]
+
+
+def run(lm, rows, n, tokens):
+    return generate(lm, rows, n, tokens) + [lm.lm_forward([128258] * rows)]
 
 
 def launches(lm):
@@ -121,6 +125,46 @@ def test_a_time_out_of_the_sampler_is_not_the_steps(monkeypatch):
     assert same(run(lm, 1, 40, 14), want) and launches(lm) == (0, late + 1)
     monkeypatch.delenv("MIS_SAMPLER_SPIN")
     assert same(run(lm, 1, 40, 14), want) and launches(lm) == (14, late + 1)
+
+
+def least(make, call):
+    """Bytes past a new handle's that two requests of the launch chain get by with, to 64 KiB."""
+    held = mas._lib.lib().mis_debug_device_limit
+    h = make()
+    before = held(-1)
+    call(h)
+    more = held(-1) - before
+    while True:
+        h = make()
+        held(more)
+        try:
+            call(h), call(h)
+            return more
+        except mas.generation.AudioGenerationError:
+            more += 1 << 16
+        finally:
+            held(-1)
+
+
+def test_no_room_for_the_step(monkeypatch):
+    """Where the launch chain has room and the values handed between blocks (180 KiB here) have none, or none is left behind them, a request takes the chain."""
+    make, call = lambda: model(2), lambda lm: generate(lm, 1, 40, 14)
+    monkeypatch.setenv("MIS_LM_STEP", "0")
+    chain, more = run(make(), 1, 40, 14), least(make, call)
+    monkeypatch.delenv("MIS_LM_STEP")
+    held = mas._lib.lib().mis_debug_device_limit
+    for extra, steps in ((0, 0), (100 << 10, 0), (1 << 20, 14)):
+        lm = make()
+        late = launches(lm)[1]
+        held(more + extra)
+        try:
+            for _ in range(2):
+                got = call(lm)
+                assert launches(lm)[0] == steps
+                assert all(np.array_equal(x, y) for x, y in zip(got, chain))
+        finally:
+            held(-1)
+        assert same(run(lm, 1, 40, 14), chain) and launches(lm) == (14, late)
 
 
 def test_two_handles_at_once(three):

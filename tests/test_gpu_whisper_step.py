@@ -17,11 +17,14 @@ def model(d, layers, vocab=700):
     return mas.WhisperModel.synthetic(cfg, seed=11)
 
 
-def run(m, rows, tokens, eot=699, seed=3):
+def transcribe(m, rows, tokens, eot=699, seed=3):
     rng = np.random.default_rng(seed)
     wins = [(0.1 * rng.standard_normal(16000 * (1 + b))).astype(np.float32) for b in range(rows)]
-    ids = m.transcribe_windows(wins, PROMPT, mas.STTGenerateParameters(max_tokens=tokens, temperature=0.0, seed=5, eot_id=eot, timestamp_begin=695))
-    return ids, m.decoder_forward([5 + b for b in range(rows)])
+    return m.transcribe_windows(wins, PROMPT, mas.STTGenerateParameters(max_tokens=tokens, temperature=0.0, seed=5, eot_id=eot, timestamp_begin=695))
+
+
+def run(m, rows, tokens, eot=699, seed=3):
+    return transcribe(m, rows, tokens, eot, seed), m.decoder_forward([5 + b for b in range(rows)])
 
 
 def launches(m):
@@ -91,6 +94,46 @@ def test_out_of_time_runs_on_the_chain(monkeypatch, d, rows):
     assert same(got, want) and launches(m) == (0, late + 1)
     for steps in (0, 20):                                                  # the next request stays on the launch chain
         assert same(run(m, rows, 20), want) and launches(m) == (steps, late + 1)
+
+
+def least(make, call):
+    """Bytes past a new handle's that two requests of the launch chain get by with, to 64 KiB."""
+    held = mas._lib.lib().mis_debug_device_limit
+    h = make()
+    before = held(-1)
+    call(h)
+    more = held(-1) - before
+    while True:
+        h = make()
+        held(more)
+        try:
+            call(h), call(h)
+            return more
+        except mas.generation.AudioGenerationError:
+            more += 1 << 16
+        finally:
+            held(-1)
+
+
+def test_no_room_for_the_step(monkeypatch):
+    """Where the launch chain has room and the values handed between blocks (1 MiB here) have none, or none is left behind them, a request takes the chain."""
+    make, call = lambda: model(1280, 2), lambda m: transcribe(m, 8, 20)
+    monkeypatch.setenv("MIS_WHISPER_STEP", "0")
+    chain, more = run(make(), 8, 20), least(make, call)
+    monkeypatch.delenv("MIS_WHISPER_STEP")
+    held = mas._lib.lib().mis_debug_device_limit
+    for extra, room in ((0, False), (1 << 19, False), (8 << 20, True)):
+        m = make()
+        late, steps = launches(m)[1], []
+        held(more + extra)
+        try:
+            for _ in range(2):                                             # (the second one's encoder beside what the first one keeps)
+                assert call(m) == chain[0]
+                steps.append(launches(m)[0])
+            assert steps == [20, 20] if room else 0 in steps
+        finally:
+            held(-1)
+        assert same(run(m, 8, 20), chain) and launches(m) == (20, late)
 
 
 @pytest.mark.parametrize("d,rows", [(768, 2), (1280, 4)])
