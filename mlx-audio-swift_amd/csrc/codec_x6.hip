@@ -777,6 +777,38 @@ struct X6Noise { const float* noise; int rng; uint64_t key; const int32_t* row_i
 // NOISE: the NoiseBlock behind it, y = x + noise (W x), on the registers: a wave holds all rows of its columns, lanes l and l + 32 trade halves of x's planes, which
 // makes them fragments, and W takes the place of the last chunk's weights (fragments [Cin / 16][MT][plane], the size of a chunk's).  As a launch of its own, in f32, it read and
 // wrote the tensor: 16 us for one row of 24576 columns, 0.90 ms for 32 of 196608; here 3 us and 0.19 ms.
+// x += nz (W x), x a phase's rows of a wave's columns.  SERIAL: a step's fragments at a time (where all of them do not fit the registers)
+template <int MT, bool SERIAL>
+__device__ __forceinline__ void x6_noise_block(f32x16_t (&acc)[MT], float nz, const x6_u4* As, int lane) {
+    f32x16_t w[MT];
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) w[mi][r] = 0.0f;
+    constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int ks = 0; ks < 2 * MT; ++ks) {
+        float x[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) x[r] = acc[ks / 2][ks % 2 * 8 + r];
+        bf16x8_t bv[3], av[MT][3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) bv[q] = __builtin_bit_cast(bf16x8_t, codec_tile_piece(x, q == 0));
+#pragma unroll
+        for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, As[((ks * MT + mi) * 3 + q) * 64 + lane]);
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int mi = 0; mi < MT; ++mi) w[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[QB[q]], w[mi], 0, 0, 0);
+        if constexpr (SERIAL) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int mi = 0; mi < MT; ++mi)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[mi][r] += nz * w[mi][r];
+}
 #define X6_CT 126
 template <int MT, bool NOISE>
 __device__ __forceinline__ void x6_convt_body(const GemmParams& p, const X6Noise& nb, const float* __restrict__ pX, float* __restrict__ pY, const float* __restrict__ pbias,
@@ -882,36 +914,7 @@ __device__ __forceinline__ void x6_convt_body(const GemmParams& p, const X6Noise
     }
     if constexpr (NOISE) {
 #pragma unroll
-        for (int ph = 0; ph < 2; ++ph) {
-            f32x16_t w[MT];
-#pragma unroll
-            for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) w[mi][r] = 0.0f;
-            constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-            for (int ks = 0; ks < 2 * MT; ++ks) {
-                float x[8];
-#pragma unroll
-                for (int r = 0; r < 8; ++r) x[r] = acc[ph][ks / 2][ks % 2 * 8 + r];
-                bf16x8_t bv[3], av[MT][3];
-#pragma unroll
-                for (int q = 0; q < 3; ++q) bv[q] = __builtin_bit_cast(bf16x8_t, codec_tile_piece(x, q == 0));
-#pragma unroll
-                for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, As[((ks * MT + mi) * 3 + q) * 64 + lane]);
-#pragma unroll
-                for (int q = 0; q < 6; ++q)
-#pragma unroll
-                    for (int mi = 0; mi < MT; ++mi) w[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[QB[q]], w[mi], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);                          // (a step's fragments at a time: all of them do not fit the registers)
-            }
-#pragma unroll
-            for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[ph][mi][r] += nz[ph] * w[mi][r];
-        }
+        for (int ph = 0; ph < 2; ++ph) x6_noise_block<MT, true>(acc[ph], nz[ph], As, lane);
         if (!in) return;
     }
     int hi = lane >> 5;                                                     // (opaque: the rows' addresses are not to be computed ahead)
@@ -1024,35 +1027,7 @@ __device__ __forceinline__ void x6_convt_half_body(const GemmParams& p, const X6
             if (dup) acc[mi][r] += bv;
         }
     }
-    if constexpr (NOISE) {
-        f32x16_t w[MT];
-#pragma unroll
-        for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) w[mi][r] = 0.0f;
-        constexpr int QA[6] = {2, 0, 1, 1, 0, 0}, QB[6] = {0, 2, 1, 0, 1, 0};
-#pragma unroll
-        for (int ks = 0; ks < 2 * MT; ++ks) {
-            float x[8];
-#pragma unroll
-            for (int r = 0; r < 8; ++r) x[r] = acc[ks / 2][ks % 2 * 8 + r];
-            bf16x8_t bv[3], av[MT][3];
-#pragma unroll
-            for (int q = 0; q < 3; ++q) bv[q] = __builtin_bit_cast(bf16x8_t, codec_tile_piece(x, q == 0));
-#pragma unroll
-            for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-                for (int q = 0; q < 3; ++q) av[mi][q] = __builtin_bit_cast(bf16x8_t, As[((ks * MT + mi) * 3 + q) * 64 + lane]);
-#pragma unroll
-            for (int q = 0; q < 6; ++q)
-#pragma unroll
-                for (int mi = 0; mi < MT; ++mi) w[mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[mi][QA[q]], bv[QB[q]], w[mi], 0, 0, 0);
-        }
-#pragma unroll
-        for (int mi = 0; mi < MT; ++mi)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mi][r] += nz * w[mi][r];
-    }
+    if constexpr (NOISE) x6_noise_block<MT, false>(acc, nz, As, lane);
     if (!in) return;
 #pragma unroll
     for (int mi = 0; mi < MT; ++mi)
