@@ -17,7 +17,7 @@
 //    overwritten in a launch that reads it; tags grow over the launches of a request and the granules are cleared in front of it.
 //  * Polls end: out of time (StepParams::limit: another stream holds compute units), a block raises `fail`, which all others see, every wave leaves, and the request runs again on the launch
 //    chain.  Two launches that each hold part of the compute units would wait for each other: a request takes this path while its call is alone on the device (DeviceTurn, common.h).
-#include "lm_step.h"
+#include "step_granules.h"
 
 #include <stdio.h>
 
@@ -60,22 +60,11 @@ __host__ __device__ inline Lds lds_layout(int ring, int k_max, int rows, int G, 
 typedef __attribute__((address_space(3))) unsigned LdsWord;             // (a generic pointer to them would be polled by flat loads, which wait for every load in flight)
 __device__ __forceinline__ unsigned lds_word(int at) { return *(volatile LdsWord*)(uintptr_t)at; }
 enum { W_VEC = 0, W_GO = 1, W_STOP = 3 };
-__device__ __forceinline__ void bar() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ void arrive(int at, int lane) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (lane == 0) __hip_atomic_fetch_add((LdsWord*)(uintptr_t)at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-typedef unsigned long long u64;
-// two values and the tag that says whose they are: one store, no flag, nothing to wait for
-__device__ __forceinline__ void granule(unsigned char* p, uint32_t v, unsigned tag) { __hip_atomic_store(reinterpret_cast<u64*>(p), (u64)v | (u64)tag << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
-// The arguments, read again (scalar loads) from here on: kept in registers over the layer loop they are more than there are.
-typedef __attribute__((address_space(4))) const StepParams* ArgPtr;
-__device__ __forceinline__ const StepParams& args() {
-    ArgPtr a = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(a));
-    return *(const StepParams*)a;
-}
+__device__ __forceinline__ const StepParams& args() { return step_args<StepParams>(); }
 
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
@@ -112,7 +101,7 @@ struct Ctx {
     // N pairs of granules (four columns each) per lane, at(i) the address of pair i, until each carries `want`; out: the four values
     template <int N, class At>
     __device__ __forceinline__ bool pairs(uint2 (&out)[N], unsigned want, At&& at) const {
-        unsigned long long t0 = 0;
+        u64 t0 = 0;
         // one granule of the wave first: all of them at every poll, from every block, are as much traffic as the weights
         if (!first(reinterpret_cast<const unsigned*>(at(0)) + 1, want, t0)) return false;
         for (int n = 0;; ++n) {
@@ -128,7 +117,7 @@ struct Ctx {
             if (((n & 63) == 63 || hasty) && !more_time(t0)) return false;
         }
     }
-    __device__ __forceinline__ bool first(const unsigned* tag_word, unsigned want, unsigned long long& t0) const {
+    __device__ __forceinline__ bool first(const unsigned* tag_word, unsigned want, u64& t0) const {
         const unsigned long long a = (unsigned long long)tag_word;
         const unsigned* one = (const unsigned*)((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)a) | (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((unsigned)(a >> 32)) << 32);
         for (int n = 0;; ++n) {
@@ -138,18 +127,7 @@ struct Ctx {
             if (((n & 63) == 63 || hasty) && !more_time(t0)) return false;
         }
     }
-    __device__ __forceinline__ bool more_time(unsigned long long& t0) const {
-        const StepParams& p = args();
-        const unsigned long long now = wall_clock64();
-        if (t0 == 0) t0 = now;
-        if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(p.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) return false;
-        if (now - t0 < p.limit) return true;
-        if (lane == 0) {
-            __hip_atomic_store(p.sync + SYNC_LATE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(p.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        return false;
-    }
+    __device__ __forceinline__ bool more_time(u64& t0) const { return ::more_time<StepParams>(t0, lane); }
 };
 
 // ------------------------------------------------------------------------------------------------------------------ matrix waves
@@ -329,8 +307,6 @@ __device__ __forceinline__ void matrix_role(const Ctx& c, int wave) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------ vector waves
-__device__ __forceinline__ float bf_lo(uint32_t v) { return bf16_to_f32((bf16_t)(v & 0xffffu)); }
-__device__ __forceinline__ float bf_hi(uint32_t v) { return bf16_to_f32((bf16_t)(v >> 16)); }
 __device__ __forceinline__ uint32_t bf_pack(float a, float b) { return (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16); }
 
 // residual stream of one edge -> RMSNorm (k_glue_cpt's columns, sums and rounding) -> sink(row, first of four columns, values)

@@ -17,6 +17,7 @@
 //
 // A row has the bits of the launch chain: K is cut and summed as there, and each norm's statistics are dealt and summed as in the kernel that held them (LN_* below).
 #include "whisper_step.h"
+#include "step_granules.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -29,7 +30,6 @@ constexpr int LDS_MAX = 160 * 1024;
 // WS_SHARED: fragments a wave holds of q | k | v, in whose registers the three square matrices come (two of SH_O, one of SH_CQ), and of the MLP's matrices
 constexpr int SH_O = 6, SH_CQ = 5, SH_Q = 2 * SH_O + SH_CQ, SH_F = 24;
 constexpr int ATT_SC = 3 * D * 2, ATT_PH = ATT_SC + CJ * 128, ATT_PL = ATT_PH + CJ * 64, ATT_PS = ATT_PL + CJ * 64, ATT_WAVE = ATT_PS + CJ * 16, ATT_LDS = WAVES * (ATT_WAVE + (D + 2) * 4);
-typedef unsigned long long u64;
 // (pointers out of a table in memory: without the address space their loads would be flat ones, which reads of LDS wait for)
 template <class T> using Global = const __attribute__((address_space(1))) T*;
 template <class T> __device__ __forceinline__ Global<T> global(const T* p) { return (Global<T>)(uintptr_t)p; }
@@ -63,34 +63,9 @@ __host__ __device__ inline Lds lds_layout(int k_max, int rows, int units) {
     l.total = a > ATT_LDS ? a : ATT_LDS;
     return l;
 }
-__device__ __forceinline__ void bar() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-__device__ __forceinline__ void granule(unsigned char* p, uint32_t v, unsigned tag) {
-    __hip_atomic_store(reinterpret_cast<u64*>(p), (u64)v | (u64)tag << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float lo(uint32_t v) { return bf16_to_f32((bf16_t)(v & 0xffffu)); }
-__device__ __forceinline__ float hi(uint32_t v) { return bf16_to_f32((bf16_t)(v >> 16)); }
 __device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
-// The arguments, read again (scalar loads) from here on: kept in registers over the layer loop they are more than there are.
-typedef __attribute__((address_space(4))) const WsParams* ArgPtr;
-__device__ __forceinline__ const WsParams& args() {
-    ArgPtr a = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(a));
-    return *(const WsParams*)a;
-}
-
-__device__ __forceinline__ bool more_time(u64& t0, int lane) {
-    const WsParams& p = args();
-    const u64 now = wall_clock64();
-    if (t0 == 0) t0 = now;
-    if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(p.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) return false;
-    if (now - t0 < p.limit) return true;
-    if (lane == 0) {
-        __hip_atomic_store(p.sync + SYNC_LATE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(p.fail, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    return false;
-}
+__device__ __forceinline__ const WsParams& args() { return step_args<WsParams>(); }
 // `one`, the same for all lanes of the wave, until it carries `tag`
 __device__ __forceinline__ bool await(bool hasty, const unsigned char* one, unsigned tag, int lane) {
     u64 t0 = 0;
@@ -98,7 +73,7 @@ __device__ __forceinline__ bool await(bool hasty, const unsigned char* one, unsi
         unsigned v = tag;
         if (lane == 0) v = (unsigned)(__hip_atomic_load(reinterpret_cast<const u64*>(one), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32);
         if ((unsigned)__builtin_amdgcn_readfirstlane(v) == tag) break;
-        if (((n & 63) == 63 || hasty) && !more_time(t0, lane)) return false;
+        if (((n & 63) == 63 || hasty) && !more_time<WsParams>(t0, lane)) return false;
     }
     asm volatile("" ::: "memory");
     return true;
@@ -116,7 +91,7 @@ __device__ __forceinline__ bool gather(bool hasty, uint32_t (&out)[N], unsigned 
             out[i] = (uint32_t)v;
         }
         if (__all(ok)) break;
-        if (((n & 63) == 63 || hasty) && !more_time(t0, lane)) return false;
+        if (((n & 63) == 63 || hasty) && !more_time<WsParams>(t0, lane)) return false;
     }
     asm volatile("" ::: "memory");
     return true;
@@ -161,7 +136,7 @@ __device__ __forceinline__ bool norm_row(bool hasty, const unsigned char* in, un
     for (int g = 0; g < G; ++g) {
         const bool live = norm_column<KIND>(K, g, lane) < norm_end<KIND>(K, g);
         float a = KIND == LN_WAVE && g > 0 ? sum[g - 1] : 0.0f;
-        a += live ? lo(v[2 * g]) : 0.0f; a += live ? hi(v[2 * g]) : 0.0f; a += live ? lo(v[2 * g + 1]) : 0.0f; a += live ? hi(v[2 * g + 1]) : 0.0f;
+        a += live ? bf_lo(v[2 * g]) : 0.0f; a += live ? bf_hi(v[2 * g]) : 0.0f; a += live ? bf_lo(v[2 * g + 1]) : 0.0f; a += live ? bf_hi(v[2 * g + 1]) : 0.0f;
         sum[g] = a;
     }
     auto total = [&](float (&part)[G]) {
@@ -177,7 +152,7 @@ __device__ __forceinline__ bool norm_row(bool hasty, const unsigned char* in, un
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         const bool live = norm_column<KIND>(K, g, lane) < norm_end<KIND>(K, g);
-        const float h[4] = {lo(v[2 * g]), hi(v[2 * g]), lo(v[2 * g + 1]), hi(v[2 * g + 1])};
+        const float h[4] = {bf_lo(v[2 * g]), bf_hi(v[2 * g]), bf_lo(v[2 * g + 1]), bf_hi(v[2 * g + 1])};
         float a = KIND == LN_WAVE && g > 0 ? sq[g - 1] : 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) { const float dl = h[e] - mean; a += live ? dl * dl : 0.0f; }
@@ -189,7 +164,7 @@ __device__ __forceinline__ bool norm_row(bool hasty, const unsigned char* in, un
         const int col = norm_column<KIND>(K, g, lane);
         if (col < norm_end<KIND>(K, g)) {
             const uint2 w = *reinterpret_cast<const uint2*>(wb + col), b = *reinterpret_cast<const uint2*>(wb + K + col);
-            const float h[4] = {lo(v[2 * g]), hi(v[2 * g]), lo(v[2 * g + 1]), hi(v[2 * g + 1])}, wv[4] = {lo(w.x), hi(w.x), lo(w.y), hi(w.y)}, bv[4] = {lo(b.x), hi(b.x), lo(b.y), hi(b.y)};
+            const float h[4] = {bf_lo(v[2 * g]), bf_hi(v[2 * g]), bf_lo(v[2 * g + 1]), bf_hi(v[2 * g + 1])}, wv[4] = {bf_lo(w.x), bf_hi(w.x), bf_lo(w.y), bf_hi(w.y)}, bv[4] = {bf_lo(b.x), bf_hi(b.x), bf_lo(b.y), bf_hi(b.y)};
             bf16_t o[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = f32_to_bf16(fmaf((h[e] - mean) * rstd, wv[e], bv[e]));
@@ -355,11 +330,11 @@ struct Task {
                     float b0 = v[g][0].x, b1 = v[g][0].y;
 #pragma unroll
                     for (int i = 1; i < KSB; ++i) { b0 += v[g][i].x; b1 += v[g][i].y; }
-                    if (s0 + g == 0) { b0 += lo(bias); b1 += hi(bias); }
+                    if (s0 + g == 0) { b0 += bf_lo(bias); b1 += bf_hi(bias); }
                     if (s0 + g < ro.S) { a0 += b0; a1 += b1; }
                 }
             }
-            if (TO == TO_RESID) { a0 = lo(hres) + bf16_round_f32(a0); a1 = hi(hres) + bf16_round_f32(a1); }
+            if (TO == TO_RESID) { a0 = bf_lo(hres) + bf16_round_f32(a0); a1 = bf_hi(hres) + bf16_round_f32(a1); }
             if (TO == TO_GELU) { a0 = gelu_erf(bf16_round_f32(a0)); a1 = gelu_erf(bf16_round_f32(a1)); }
             granule(now + at.out + ((size_t)m * cols + col) * 4, (uint32_t)f32_to_bf16(a0) | (uint32_t)f32_to_bf16(a1) << 16, tag);
         }
@@ -507,139 +482,139 @@ __device__ __forceinline__ bool attend(unsigned char* smem, const Head<SELF>& hd
     bf16_t *ph = reinterpret_cast<bf16_t*>(own + ATT_PH), *pl = reinterpret_cast<bf16_t*>(own + ATT_PL);
     float* part = reinterpret_cast<float*>(smem + WAVES * ATT_WAVE);        // [WAVES][D + 2]
     unsigned char* now = p.exch + (size_t)exch_layer * li;
-            constexpr int NG = SELF ? 2 : 1;
-            uint32_t v[NG];
-        if ((!SELF || li > 0) && !await(hasty, now - (SELF ? exch_layer : 0u) + near_at, tag, lane)) return false;
-            const unsigned char* from = now + q_at + (size_t)b * (SELF ? 3 : 1) * d * 4 + h * D * 4;
-            // q | k | v of the head, 32 granules each; the cross-attention: q
-            if (!gather<NG>(hasty, v, tag, lane, [&](int i) {
-                    const int g = min(lane + 64 * i, SELF ? 95 : 31);
-                    return from + (size_t)(g >> 5) * d * 4 + (g & 31) * 8;
-                })) return false;
-    #pragma unroll
-            for (int i = 0; i < NG; ++i)
-                if (lane + 64 * i < (SELF ? 96 : 32)) reinterpret_cast<uint32_t*>(strip)[lane + 64 * i] = v[i];
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            bf16x8_t qf[2];
-    #pragma unroll
-            for (int c = 0; c < 2; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(strip + c * 32 + g4 * 8);
-            if (SELF && live) {
-                // the new key, in the registers of the wave whose tile it is and in the cache
-                const int tile = pos >> 5, pr = pos & 31, prow = ((pr >> 3) << 2) | (pr & 3), half = (pr >> 2) & 1;
-                if ((tile & (WAVES - 1)) == wave) {
-                    const int jn = tile / WAVES;
-                    bf16x8_t* kc = reinterpret_cast<bf16x8_t*>(p.self_k + p.self_layer * li + head) + ((size_t)tile * 2 + half) * 2 * 64 + lane;
-                    bf16_t* vc = p.self_v + p.self_layer * li + head;
-                    if (d0 == prow) {
-    #pragma unroll
-                        for (int c = 0; c < 2; ++c) {
-                            const bf16x8_t kn = *reinterpret_cast<const bf16x8_t*>(strip + D + c * 32 + g4 * 8);
-                            kc[c * 64] = kn;
-    #pragma unroll
-                            for (int j = 0; j < NJ; ++j)
-                                if (j == jn) { if (half) ka[j][1][c] = kn; else ka[j][0][c] = kn; }
-                        }
-                    }
-                    if (g4 == (pr >> 3)) {
-    #pragma unroll
-                        for (int dt = 0; dt < 4; ++dt) {
-                            const bf16_t vn = strip[2 * D + dt * 16 + d0];
-                            vc[(((size_t)tile * 4 + dt) * 64 + lane) * 8 + (pr & 7)] = vn;
-    #pragma unroll
-                            for (int j = 0; j < NJ; ++j)
-    #pragma unroll
-                                for (int e = 0; e < 8; ++e)
-                                    if (j == jn && e == (pr & 7)) va[j][dt][e] = (short)vn;
-                        }
-                    }
-                }
-            }
-            // Scores stand in all sixteen columns: through LDS a lane gets one key of every second tile, and gives the probabilities back (sixteen times the vector work otherwise:
-            // 4.9 us at six tiles a wave)
-    #pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                f32x4_t S0 = (f32x4_t){0.f, 0.f, 0.f, 0.f}, S1 = S0;
-    #pragma unroll
+    constexpr int NG = SELF ? 2 : 1;
+    uint32_t v[NG];
+    if ((!SELF || li > 0) && !await(hasty, now - (SELF ? exch_layer : 0u) + near_at, tag, lane)) return false;
+    const unsigned char* from = now + q_at + (size_t)b * (SELF ? 3 : 1) * d * 4 + h * D * 4;
+    // q | k | v of the head, 32 granules each; the cross-attention: q
+    if (!gather<NG>(hasty, v, tag, lane, [&](int i) {
+            const int g = min(lane + 64 * i, SELF ? 95 : 31);
+            return from + (size_t)(g >> 5) * d * 4 + (g & 31) * 8;
+        })) return false;
+#pragma unroll
+    for (int i = 0; i < NG; ++i)
+        if (lane + 64 * i < (SELF ? 96 : 32)) reinterpret_cast<uint32_t*>(strip)[lane + 64 * i] = v[i];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bf16x8_t qf[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) qf[c] = *reinterpret_cast<const bf16x8_t*>(strip + c * 32 + g4 * 8);
+    if (SELF && live) {
+        // the new key, in the registers of the wave whose tile it is and in the cache
+        const int tile = pos >> 5, pr = pos & 31, prow = ((pr >> 3) << 2) | (pr & 3), half = (pr >> 2) & 1;
+        if ((tile & (WAVES - 1)) == wave) {
+            const int jn = tile / WAVES;
+            bf16x8_t* kc = reinterpret_cast<bf16x8_t*>(p.self_k + p.self_layer * li + head) + ((size_t)tile * 2 + half) * 2 * 64 + lane;
+            bf16_t* vc = p.self_v + p.self_layer * li + head;
+            if (d0 == prow) {
+#pragma unroll
                 for (int c = 0; c < 2; ++c) {
-                    S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][0][c], qf[c], S0, 0, 0, 0);
-                    S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][1][c], qf[c], S1, 0, 0, 0);
+                    const bf16x8_t kn = *reinterpret_cast<const bf16x8_t*>(strip + D + c * 32 + g4 * 8);
+                    kc[c * 64] = kn;
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+                        if (j == jn) { if (half) ka[j][1][c] = kn; else ka[j][0][c] = kn; }
                 }
-                if (d0 == 0) { *reinterpret_cast<f32x4_t*>(sc + j * 32 + g4 * 8) = S0; *reinterpret_cast<f32x4_t*>(sc + j * 32 + g4 * 8 + 4) = S1; }
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (LDS operations of one wave execute in order)
-            float m_run = -INFINITY, l_run = 0.0f, alpha[NJ], x[NJ / 2], mx[NJ / 2];
-            const int up = lane >> 5;
-    #pragma unroll
-            for (int i = 0; i < NJ / 2; ++i) {
-                const float v = sc[i * 64 + lane] * scale;
-                x[i] = (wave + (2 * i + up) * WAVES) * 32 + (lane & 31) < kv_len ? v : -INFINITY;
-                mx[i] = x[i];
-            }
-    #pragma unroll
-            for (int k = 1; k < 32; k <<= 1)
-    #pragma unroll
-                for (int i = 0; i < NJ / 2; ++i) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], k, 64));
-    #pragma unroll
-            for (int i = 0; i < NJ / 2; ++i) {
-                const float m0 = fmaxf(m_run, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx[i]), 0)));
-                alpha[2 * i] = __expf(m_run - m0);
-                const bool two = wave + (2 * i + 1) * WAVES < n_tiles;         // (a group of five)
-                const float m1 = two ? fmaxf(m0, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx[i]), 32))) : m0;
-                alpha[2 * i + 1] = __expf(m0 - m1);
-                m_run = wave + 2 * i * WAVES < n_tiles ? m1 : m_run;
-                const float pe = __expf(x[i] - (up ? m1 : m0));
-                const bf16_t hb = f32_to_bf16(pe);
-                sc[i * 64 + lane] = pe;
-                ph[i * 64 + lane] = hb;
-                pl[i * 64 + lane] = f32_to_bf16(pe - bf16_to_f32(hb));
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            if (lane < NJ * 4) {
-                const f32x4_t a = *reinterpret_cast<const f32x4_t*>(sc + lane * 8), c = *reinterpret_cast<const f32x4_t*>(sc + lane * 8 + 4);
-                float psum = 0.0f;
-    #pragma unroll
-                for (int e = 0; e < 8; ++e) psum += e < 4 ? a[e & 3] : c[e & 3];
-                ps[lane] = psum;
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            f32x4_t O[4];
-    #pragma unroll
-            for (int dt = 0; dt < 4; ++dt) O[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    #pragma unroll
-            for (int j = 0; j < NJ; ++j)
-                if (wave + j * WAVES < n_tiles) {
-                    l_run = l_run * alpha[j] + ps[j * 4 + g4];
-                    const bf16x8_t fh = *reinterpret_cast<const bf16x8_t*>(ph + j * 32 + g4 * 8), fl = *reinterpret_cast<const bf16x8_t*>(pl + j * 32 + g4 * 8);   // P in bf16 hi + lo parts
-    #pragma unroll
-                    for (int dt = 0; dt < 4; ++dt) {
-                        f32x4_t o = O[dt];
-                        o[0] *= alpha[j];                                       // (row 0 of O is read, the others are copies without their factors)
-                        o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh, va[j][dt], o, 0, 0, 0);
-                        O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl, va[j][dt], o, 0, 0, 0);
-                    }
+            if (g4 == (pr >> 3)) {
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) {
+                    const bf16_t vn = strip[2 * D + dt * 16 + d0];
+                    vc[(((size_t)tile * 4 + dt) * 64 + lane) * 8 + (pr & 7)] = vn;
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            if (j == jn && e == (pr & 7)) va[j][dt][e] = (short)vn;
                 }
-            l_run += __shfl_xor(l_run, 16, 64);
-            l_run += __shfl_xor(l_run, 32, 64);
-            if (g4 == 0) {
-    #pragma unroll
-                for (int dt = 0; dt < 4; ++dt) part[wave * (D + 2) + dt * 16 + d0] = O[dt][0];
-                if (d0 < 2) part[wave * (D + 2) + D + d0] = d0 ? l_run : m_run;
             }
-            bar();
-            if (wave == 0) {
-                float M = -INFINITY, num = 0.0f, den = 0.0f;
-    #pragma unroll
-                for (int w = 0; w < WAVES; ++w) M = fmaxf(M, part[w * (D + 2) + D]);
-    #pragma unroll
-                for (int w = 0; w < WAVES; ++w) {
-                    const float f = __expf(part[w * (D + 2) + D] - M);
-                    num += f * part[w * (D + 2) + lane];
-                    den += f * part[w * (D + 2) + D + 1];
-                }
-                const uint32_t o = live ? f32_to_bf16(num / den) : 0u, next = __shfl_xor(o, 1, 64);
-                if (!(lane & 1)) granule(now + out_at + ((size_t)b * d + h * D + lane) * 4, o | next << 16, tag);
+        }
+    }
+    // Scores stand in all sixteen columns: through LDS a lane gets one key of every second tile, and gives the probabilities back (sixteen times the vector work otherwise:
+    // 4.9 us at six tiles a wave)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        f32x4_t S0 = (f32x4_t){0.f, 0.f, 0.f, 0.f}, S1 = S0;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            S0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][0][c], qf[c], S0, 0, 0, 0);
+            S1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[j][1][c], qf[c], S1, 0, 0, 0);
+        }
+        if (d0 == 0) { *reinterpret_cast<f32x4_t*>(sc + j * 32 + g4 * 8) = S0; *reinterpret_cast<f32x4_t*>(sc + j * 32 + g4 * 8 + 4) = S1; }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (LDS operations of one wave execute in order)
+    float m_run = -INFINITY, l_run = 0.0f, alpha[NJ], x[NJ / 2], mx[NJ / 2];
+    const int up = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < NJ / 2; ++i) {
+        const float v = sc[i * 64 + lane] * scale;
+        x[i] = (wave + (2 * i + up) * WAVES) * 32 + (lane & 31) < kv_len ? v : -INFINITY;
+        mx[i] = x[i];
+    }
+#pragma unroll
+    for (int k = 1; k < 32; k <<= 1)
+#pragma unroll
+        for (int i = 0; i < NJ / 2; ++i) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], k, 64));
+#pragma unroll
+    for (int i = 0; i < NJ / 2; ++i) {
+        const float m0 = fmaxf(m_run, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx[i]), 0)));
+        alpha[2 * i] = __expf(m_run - m0);
+        const bool two = wave + (2 * i + 1) * WAVES < n_tiles;         // (a group of five)
+        const float m1 = two ? fmaxf(m0, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mx[i]), 32))) : m0;
+        alpha[2 * i + 1] = __expf(m0 - m1);
+        m_run = wave + 2 * i * WAVES < n_tiles ? m1 : m_run;
+        const float pe = __expf(x[i] - (up ? m1 : m0));
+        const bf16_t hb = f32_to_bf16(pe);
+        sc[i * 64 + lane] = pe;
+        ph[i * 64 + lane] = hb;
+        pl[i * 64 + lane] = f32_to_bf16(pe - bf16_to_f32(hb));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (lane < NJ * 4) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(sc + lane * 8), c = *reinterpret_cast<const f32x4_t*>(sc + lane * 8 + 4);
+        float psum = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) psum += e < 4 ? a[e & 3] : c[e & 3];
+        ps[lane] = psum;
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    f32x4_t O[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) O[dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+        if (wave + j * WAVES < n_tiles) {
+            l_run = l_run * alpha[j] + ps[j * 4 + g4];
+            const bf16x8_t fh = *reinterpret_cast<const bf16x8_t*>(ph + j * 32 + g4 * 8), fl = *reinterpret_cast<const bf16x8_t*>(pl + j * 32 + g4 * 8);   // P in bf16 hi + lo parts
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                f32x4_t o = O[dt];
+                o[0] *= alpha[j];                                       // (row 0 of O is read, the others are copies without their factors)
+                o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh, va[j][dt], o, 0, 0, 0);
+                O[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl, va[j][dt], o, 0, 0, 0);
             }
-            bar();
+        }
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    if (g4 == 0) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) part[wave * (D + 2) + dt * 16 + d0] = O[dt][0];
+        if (d0 < 2) part[wave * (D + 2) + D + d0] = d0 ? l_run : m_run;
+    }
+    bar();
+    if (wave == 0) {
+        float M = -INFINITY, num = 0.0f, den = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) M = fmaxf(M, part[w * (D + 2) + D]);
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float f = __expf(part[w * (D + 2) + D] - M);
+            num += f * part[w * (D + 2) + lane];
+            den += f * part[w * (D + 2) + D + 1];
+        }
+        const uint32_t o = live ? f32_to_bf16(num / den) : 0u, next = __shfl_xor(o, 1, 64);
+        if (!(lane & 1)) granule(now + out_at + ((size_t)b * d + h * D + lane) * 4, o | next << 16, tag);
+    }
+    bar();
     return true;
 }
 template <int NJ, bool SELF>
