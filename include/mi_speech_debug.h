@@ -28,7 +28,7 @@ int32_t mis_debug_choose_split(int32_t items, int32_t k_tiles, int32_t waves_per
 mis_status mis_debug_occupy_cus(int device, int blocks, int threads, double seconds);
 mis_status mis_debug_occupy_wait(void);
 int32_t mis_debug_device_cus(int device);            /* compute units of a device (0 when it does not exist) */
-/* diagnostics / tests: launches of the one-launch sampler that reported a timed-out row barrier in this process so far */
+/* diagnostics / tests: requests and sampler calls of this process so far that a kernel whose blocks wait for each other (one-launch sampler, decode step in one launch) ended by a time-out */
 int32_t mis_debug_sampler_failures(void);
 
 /* tests: let the library's device buffers grow by at most `more` bytes from here on (negative: as far as the card's memory goes); returns the bytes they hold.

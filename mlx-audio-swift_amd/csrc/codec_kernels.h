@@ -8,7 +8,7 @@ enum { GEMM_PLAIN = 0, GEMM_RESID = 1, GEMM_NOISE = 2, GEMM_CONVT = 3, GEMM_GELU
 // Snake, x + sin^2(alpha x) ra, with the factor as `a` = alpha / pi (snake_alpha below, rounded once when the weights are laid out): f = a x less its nearest
 // whole number, rounded once (fmaf: the rounding of the product alone, kept in the difference, is 1.15 times the error from |alpha x| = ten on), and sin^2(pi f),
 // |f| <= 1/2, is f^2 times a polynomial of degree five in f^2 (least maximum, found by reweighted least squares; 5.9e-9 before rounding).  Eleven VALU instructions:
-// the product alpha x reduced by multiples of pi and the square of a polynomial for the sine were fourteen, in kernels that issue VALU in 60 - 90 % of their cycles.
+// the product alpha x reduced by multiples of pi and the square of a polynomial for the sine were fourteen, in kernels that then issued VALU in 60 - 90 % of their cycles (50 - 80 now).
 // Off 64 bits by 4.5e-8 (rms) where |alpha x| is about one, 1.01e-7 at three, 3.15e-7 at ten, 3.11e-6 at a hundred: rounding of a.  The form before: 5.1e-8, 1.08e-7,
 // 3.15e-7, 3.10e-6.
 __device__ __forceinline__ float mis_snake(float x, float a, float ra) {

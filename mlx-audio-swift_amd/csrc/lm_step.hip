@@ -15,6 +15,7 @@
 //    it.  Nothing is waited for behind the store and there is no flag (with lines of values, a flag behind their acknowledgement and a gather: 59 us).  A wave polls one granule until
 //    it is there, then all of its own: every block polling all of a vector is as much traffic as the weights (46.3 against 47.5).  Every layer has granules of its own, so none is
 //    overwritten in a launch that reads it; tags grow over the launches of a request and the granules are cleared in front of it.
+//  * Registers: 168 for each of twelve waves, of which 37 spill (112 bytes a lane).
 //  * Polls end: out of time (StepParams::limit: another stream holds compute units), a block raises `fail`, which all others see, every wave leaves, and the request runs again on the launch
 //    chain.  Two launches that each hold part of the compute units would wait for each other: a request takes this path while its call is alone on the device (DeviceTurn, common.h).
 #include "step_granules.h"

@@ -15,6 +15,8 @@
 // two us each with the polls, and the short programs between them (a norm 1 - 2, cross-attention 4, products and their sums 1 - 2); eight rows of 1280: 88 blocks for 46 MB of weights, and the
 // MLP's 20480 granules in four passes (6 us of a layer's 46; passes of 14 or 20 granules a thread are no faster, two launches a layer with a task a block 55).
 //
+// Registers: 255 of WS_ALL; WS_SHARED 256, of which 8 spill (20 bytes a lane).
+//
 // A row has the bits of the launch chain: K is cut and summed as there, and each norm's statistics are dealt and summed as in the kernel that held them (LN_* below).
 #include "whisper_step.h"
 #include "step_granules.h"
