@@ -1603,6 +1603,9 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
     // ---- decode loop (:714-744)
     by_step = one_launch && turn.take(c->device);
     if (!by_step) device_settle(c->device);
+    // (captured here alone: a request that changes its way at a poll does so beside another call, whose use of the legacy stream would invalidate a capture.  It then launches its steps one by
+    // one where the handle has no graph of them yet: 4 launches, or the chain's, which the host queues in half of a step's time)
+    if (hipGraphExec_t& first = by_step ? c->g_step : c->g_decode; c->use_graph && !first) capture(&first, decode_body);
     // (Several decode steps per graph launch were measured and removed: between two hipGraphLaunch calls of the one-step graph the
     // device idles for 8.2 us - profiles/r04/c1_gaps.json - and yet eight steps per graph are SLOWER, 2.1047 against 2.0953 ms per step
     // over five A/B runs, profiles/r04/c2_ab.json: a 1376-node graph costs more per node than its seven removed seams save.)
@@ -1616,10 +1619,9 @@ static void run_generate_attempt(mis_tts* c, const int32_t* prompt_ids, const in
     *done_host = 0;
     while (steps < max_tokens) {
         int chunk = std::min(poll, max_tokens - steps);
-        hipGraphExec_t& graph = by_step ? c->g_step : c->g_decode;
-        if (c->use_graph && !graph) capture(&graph, decode_body);
+        const hipGraphExec_t graph = c->use_graph ? by_step ? c->g_step : c->g_decode : nullptr;
         for (int i = 0; i < chunk; ++i) {
-            if (c->use_graph) HIP_CHECK(hipGraphLaunch(graph, s)); else decode_body();
+            if (graph) HIP_CHECK(hipGraphLaunch(graph, s)); else decode_body();
         }
         steps += chunk;
         if (by_step) c->step_count += chunk;

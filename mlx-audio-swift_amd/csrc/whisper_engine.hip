@@ -809,26 +809,24 @@ static void whisper_generate_once(mis_whisper* c, const float* pcm, const int64_
             launch_sampler(q, batch, s);
             layers(c->ids.p);
     };
-    hipGraphExec_t graphs[2] = {};                       // layers by launches, as one launch
-    auto drop_graphs = [&] { for (auto& g : graphs) if (g) { (void)hipGraphExecDestroy(g); g = nullptr; } };
+    hipGraphExec_t gexec = nullptr;                      // a step of the way that the request begins with; one that changes at a poll launches its steps one by one (capture: lm_engine.hip)
+    const bool captured_step = by_step;
     const bool use_graph = getenv("MIS_NO_GRAPH") == nullptr;
     try {
-        auto capture = [&](hipGraphExec_t* exec) {
+        if (use_graph) {
             hipGraph_t g = nullptr;
             HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
             try { step_body(); } catch (...) { hipGraph_t dead = nullptr; (void)hipStreamEndCapture(s, &dead); if (dead) (void)hipGraphDestroy(dead); throw; }
             HIP_CHECK(hipStreamEndCapture(s, &g));
-            HIP_CHECK(hipGraphInstantiate(exec, g, nullptr, nullptr, 0));
+            HIP_CHECK(hipGraphInstantiate(&gexec, g, nullptr, nullptr, 0));
             HIP_CHECK(hipGraphDestroy(g));
-        };
+        }
         // stream form: the ids sampled since the last poll are announced in step order per row (the reference decodes them to a
         // text delta per step, WhisperModel.swift:242-254; detokenisation stays with the host); EOT is never announced (:238)
         std::vector<int32_t> h_ng(batch), h_tok;
         const int poll = on_event ? 3 : 7;
         for (int step = 0; step < max_tokens; ++step) {
-            hipGraphExec_t& graph = graphs[by_step];
-            if (use_graph && !graph) capture(&graph);
-            if (use_graph) HIP_CHECK(hipGraphLaunch(graph, s)); else step_body();
+            if (use_graph && by_step == captured_step) HIP_CHECK(hipGraphLaunch(gexec, s)); else step_body();
             c->step_count += by_step;
             if ((step & poll) == poll || step + 1 == max_tokens) {
                 HIP_CHECK(hipMemcpyAsync(done_host, c->done_count.p, 4, hipMemcpyDeviceToHost, s));
@@ -853,10 +851,10 @@ static void whisper_generate_once(mis_whisper* c, const float* pcm, const int64_
             }
         }
     } catch (...) {
-        drop_graphs();
+        if (gexec) (void)hipGraphExecDestroy(gexec);
         throw;
     }
-    drop_graphs();
+    if (gexec) (void)hipGraphExecDestroy(gexec);
     HIP_CHECK(hipGetLastError());
     if (sampler_failed) {
         sampler_note_failure(c->scratch.p, batch, s);

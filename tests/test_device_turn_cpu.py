@@ -51,9 +51,11 @@ def test_alone_until_another_call_comes(two):
     assert a(TAKE) == 1 and a(POLL) == 1
     b(ENTER)
     assert b(TAKE) == 0
-    assert a(POLL) == 0 and a(POLL) == 0 and b(POLL) == 0                  # neither, beside each other
-    b(LEAVE)
+    assert a(POLL) == 0 and b(POLL) == 0                                   # neither, beside each other
+    t = time.perf_counter()
     assert a(POLL) == 0
+    b(LEAVE)
+    assert a(POLL) == 0 or time.perf_counter() - t >= QUIET
     time.sleep(QUIET + 0.02)
     assert a(POLL) == 1                                                    # alone for a while
     a(GIVE), a(LEAVE)
@@ -69,9 +71,10 @@ def test_a_call_that_has_gone_again(two):
     assert a(TAKE) == 1
     for _ in range(3):
         b(ENTER), b(LEAVE)
+        t = time.perf_counter()
         assert a(POLL) == 0
         time.sleep(0.6 * QUIET)
-    assert a(POLL) == 0
+    assert a(POLL) == 0 or time.perf_counter() - t >= QUIET
     time.sleep(QUIET)
     assert a(POLL) == 1
     a(GIVE), a(LEAVE)

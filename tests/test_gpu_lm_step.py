@@ -183,13 +183,24 @@ def test_two_handles_at_once(three):
     assert all(same(r, want) for k in "ab" for r in got[k]) and launches(three)[1] == late        # neither waits for the other's compute units
 
 
-def test_another_call_beside_a_request(three):
+@pytest.mark.parametrize("graph", [True, False])                          # the handle has a graph of the chain's steps, or none yet
+@pytest.mark.parametrize("other", ["codec", "sampler"])                   # the sampler's blocks wait for each other, its copies go over the legacy stream
+def test_another_call_beside_a_request(monkeypatch, three, graph, other):
     """From the first poll behind another handle's call on, the launch chain, and the same tokens."""
     cfg = mas.SNACConfig(**SMALL)
     codec = mas.SNAC.from_weights(cfg, snac_synthetic_weights(cfg, seed=1))
-    codes = [np.zeros((1, k), np.int32) for k in (1, 2, 4)]
-    codec.decode(codes)
+    codes, logits = [np.zeros((1, k), np.int32) for k in (1, 2, 4)], np.random.default_rng(0).standard_normal((8, 30000)).astype(np.float32)
+    calls = dict(codec=lambda: codec.decode(codes),
+                 sampler=lambda: mas.tts.sample_logits(logits, np.zeros((8, 0), np.int32), np.zeros(8, np.int32), mas.GenerateParameters(temperature=0.8, top_p=0.9), 0))
+    calls[other]()
     gp = mas.GenerateParameters(max_tokens=600, seed=5, temperature=0.8, frame_constrained=2)
+    if not graph:
+        three.generate_batch(prompts(1, 41), gp)                           # (another prompt length: the graphs of the one before go)
+    else:
+        monkeypatch.setenv("MIS_LM_STEP", "0")
+        for _ in three.generate_stream_batch(prompts(1, 40), gp):
+            pass
+        monkeypatch.delenv("MIS_LM_STEP")
     want = three.generate_batch(prompts(1, 40), gp, return_tokens=True)[1][0]
     steps, late = launches(three)
     assert steps >= len(want) > 500
@@ -198,6 +209,6 @@ def test_another_call_beside_a_request(three):
         if hasattr(e, "token"):
             got.append(e.token)
             if len(got) == 1:
-                codec.decode(codes)
+                calls[other]()
     here = launches(three)
     assert np.array_equal(got, want) and 0 < here[0] < steps and here[1] == late
